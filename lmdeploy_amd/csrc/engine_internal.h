@@ -143,6 +143,7 @@ struct LayeredModel {
     std::vector<LmLayer> layers;
     DenseWeight          head;
     DenseWeight          loop_in;               // [width][2 width]: the mix of stream and embedding output at the start of a loop pass
+    StreamScratch        scratch;               // slices of k of the few-row products
     float*               loop_step = nullptr;   // [loop_times][width]
     void*                embed      = nullptr;  // [vocab][width] bf16 | fp32
     float*               final_norm = nullptr;

@@ -66,6 +66,7 @@
 //            two batched products -> weighted sum + gated shared expert
 //   x       += N2b y (+ x0 where the next run opens a later pass of a loop), h = N1 of the next layer                 one launch (launch_block_close)
 #include "engine_internal.h"
+#include "gemm_stream.h"
 
 namespace tmk {
 
@@ -837,6 +838,12 @@ int layered_init_synthetic(tm_engine* e, uint64_t seed)
     return 0;
 }
 
+static std::vector<DenseWeight*> dense_weights(LmLayer& L)
+{
+    return {&L.qkv, &L.up, &L.out, &L.wo, &L.gu, &L.down, &L.uk, &L.uv, &L.w2, &L.router, &L.sh_up, &L.sh_down, &L.wo_r, &L.a2, &L.g2, &L.uq,
+            &L.side_gate, &L.side_proj, &L.sh_gu};
+}
+
 template<class T>
 static int lm_alloc(T** p, size_t n, hipStream_t st)
 {
@@ -1048,6 +1055,15 @@ int layered_start(tm_engine* e)
     if (lm.state_slot_floats > 0) {
         TM_TRY(lm_alloc(&lm.d_state, ((size_t)B + 1) * lm.state_slot_floats, st));
     }
+    TM_TRY(lm_alloc((char**)&lm.scratch.slabs, kStreamWsBytes, st));
+    TM_TRY(lm_alloc(&lm.scratch.tickets, (size_t)kStreamTickets, st));
+    lm.scratch.bytes = kStreamWsBytes, lm.scratch.count = kStreamTickets;
+    for (LmLayer& L : lm.layers) {
+        for (DenseWeight* d : dense_weights(L)) {
+            d->scratch = &lm.scratch;
+        }
+    }
+    lm.head.scratch = lm.loop_in.scratch = &lm.scratch;
     TM_TRY(lm_alloc(&lm.d_res, T * m.width, st));
     TM_TRY(lm_alloc((char**)&lm.d_h1, T * lm.ldw * lm.elem, st));
     TM_TRY(lm_alloc((char**)&lm.d_h2, T * lm.ldw * lm.elem, st));
@@ -1123,11 +1139,9 @@ void layered_free(tm_engine* e)
     for (size_t i = 0; i < lm.layers.size(); ++i) {
         LmLayer& L = lm.layers[i];
         if (L.src == (int)i) {
-            dense_weight_free(L.qkv), dense_weight_free(L.up), dense_weight_free(L.out);
-            dense_weight_free(L.wo), dense_weight_free(L.gu), dense_weight_free(L.down), dense_weight_free(L.uk), dense_weight_free(L.uv);
-            dense_weight_free(L.w2), dense_weight_free(L.router), dense_weight_free(L.sh_up), dense_weight_free(L.sh_down);
-            dense_weight_free(L.wo_r), dense_weight_free(L.a2), dense_weight_free(L.g2);
-            dense_weight_free(L.uq), dense_weight_free(L.side_gate), dense_weight_free(L.side_proj), dense_weight_free(L.sh_gu);
+            for (DenseWeight* d : dense_weights(L)) {
+                dense_weight_free(*d);
+            }
             for (float* p : {L.norm1, L.norm2, L.sink, L.r1, L.r2, L.rg1_b, L.rg2_b, L.c_norm, L.inv_freq, L.norm1_b, L.norm2_b, L.proj_bias,
                              L.q_w, L.k_w, L.mix_norm, L.w0, L.act_par, L.decay_d, L.conv_w, L.lambda, L.dist_tab, L.talk, L.zero_sink, L.join_l,
                              L.join_r, L.a_log, L.dt_bias, L.r_norm, L.cq_norm, L.f_bias, L.f_low, L.side_w, L.dwa, L.norm1b, L.norm2b, L.mu, L.bonus, L.correction}) {
@@ -1154,7 +1168,7 @@ void layered_free(tm_engine* e)
     }
     for (void* p : {(void*)lm.embed, (void*)lm.final_norm, (void*)lm.d_res, lm.d_h1, lm.d_h2, lm.d_qkv, lm.d_cat, lm.d_hn, (void*)lm.d_logits_f32,
                     (void*)lm.d_row_seq, (void*)lm.d_row_pos, (void*)lm.d_iota, (void*)lm.d_want, (void*)lm.d_seq_slot, (void*)lm.d_step_ids,
-                    (void*)lm.d_step_cu_q, (void*)lm.d_step_k_len, (void*)lm.d_attn_ws}) {
+                    (void*)lm.d_step_cu_q, (void*)lm.d_step_k_len, (void*)lm.d_attn_ws, (void*)lm.scratch.slabs, (void*)lm.scratch.tickets}) {
         if (p) {
             (void)hipFree(p);
         }

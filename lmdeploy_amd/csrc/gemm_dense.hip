@@ -1,16 +1,12 @@
 // Dense linears with unquantised weights: y = x . W^T for W stored [N][K] (the checkpoint's own orientation), in two number formats.
 //
-//   bf16 : weights and activations bfloat16, fp32 accumulation on the matrix cores (v_mfma_f32_16x16x32_bf16).  Both operands are
-//          K-contiguous, so a lane's MFMA fragment (row = lane % 16, eight consecutive k at (lane / 16) * 8) is ONE 16-byte load.
-//            * skinny kernel (M <= 32, the decode step): a wave owns 16 or 32 output columns, the four waves of a workgroup split K
-//              and merge through LDS; weights stream straight from HBM into the fragments, one 256-wide chunk ahead of the MFMAs.
-//            * tiled kernel (M > 32, prefill): 128 x 128 x 32 workgroup tiles staged in LDS (padded rows, no bank conflicts on the
-//              16-byte fragment reads), 2 x 2 waves of 64 x 64, next tile prefetched into registers under the MFMAs.
-//   fp32 : true 32-bit FMA arithmetic (no matrix-core shortcut, no reduced-precision mode), 64 x 64 x 16 LDS tiles, 4 x 4 per thread.
+//   bf16 : weights and activations bfloat16, fp32 accumulation on the matrix cores (v_mfma_f32_16x16x32_bf16).
+//   fp32 : weights and activations fp32, multiplied and added in 32 bits (v_mfma_f32_16x16x4_f32).
 //
-// Weights are kept as zero-padded images of Np x Kp elements (Np % 128 == 0, Kp % 32 == 0; bf16: in MFMA fragment order, see
-// dense_frag_index; fp32: [Np][Kp]): no bounds test in any inner loop.  Activation rows
-// have a leading dimension >= Kp; what lies in their pad columns only has to be finite, it meets zero weights.
+// The kernels are gemm_stream.h's: the weight stream for up to 64 rows (a decode step), tiles staged in LDS for more (prompts).
+// Weights are kept as zero-padded images of Np x Kp elements in fragment order (Np % 128 == 0, Kp % 32 == 0; dense_frag_index): no bounds
+// test in any inner loop.  Activation rows have a leading dimension >= Kp; what lies in their pad columns only has to be finite, it
+// meets zero weights.
 //
 // The epilogue is chosen per call (DenseEpilogue): plain store, relu(x)^2 (the squared-ReLU feed-forward), accumulate into the fp32
 // residual stream with a multiplier (resid += alpha * acc: the output projection of a residual block closes the block in the GEMM),
@@ -24,427 +20,231 @@
 // A launch may also have SEGMENTS (DenseCall::n_seg): ranges of output columns that read x at columns of their own -- the projections of
 // several inputs derived from one token (each its own mix of the token and its predecessor) as one product of any widths.
 #include "tm_kernels.h"
+#include "gemm_stream.h"
+#include <algorithm>
 
 namespace tmk {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-
-// EPI >= 0: the epilogue is known at compile time (a kernel with many outputs per thread must not carry every epilogue per output: the
-// unroller gives up and the accumulators land in scratch memory); -1: the call's own
-template<class T, int EPI = -1>
-__device__ __forceinline__ void dense_epilogue(void* y, int ldy, int m, int n, float acc, const DenseCall& c)
-{
-    const size_t i   = (size_t)m * ldy + n;
-    const int    epi = EPI >= 0 ? EPI : c.epi;
-    if (epi == kDenseStore) {
-        ((T*)y)[i] = (T)acc;
-    }
-    else if (epi == kDenseRelu2) {
-        const float r = fmaxf(acc, 0.f);
-        ((T*)y)[i]    = (T)(r * r);
-    }
-    else if (epi == kDenseResidAdd) {
-        const float v  = ((float*)y)[i] + c.alpha * acc;
-        ((float*)y)[i] = v;
-        if (c.y2) {
-            ((T*)c.y2)[(size_t)m * c.ldy2 + n] = (T)v;
-        }
-    }
-    else if (epi == kDenseScaleF32) {
-        ((float*)y)[i] = c.alpha * acc;
-    }
-    else if (epi == kDenseBiasF32) {
-        ((float*)y)[i] = acc + c.bias[n];
-    }
-    else if (epi == kDenseXielu) {
-        const float a = c.act_par[0], b = c.act_par[1];
-        ((T*)y)[i]    = (T)(acc > 0.f ? fmaf(a * acc, acc, 0.5f * acc) : fmaf(b, expm1f(acc) - acc, 0.5f * acc));
-    }
-    else if (epi == kDenseActTable) {
-        const int id = min(max(c.ids[m], 0), c.table_rows - 1);
-        ((T*)y)[i]   = (T)(act_apply(c.act, acc) * (float)((const __bf16*)c.table)[(size_t)id * c.ld_table + c.table_col + n]);
-    }
-    else {  // kDenseResidGate
-        const float z = c.gate[(size_t)m * c.ldg + n] + c.gate_bias[n];
-        ((float*)y)[i] += acc / (1.f + expf(-z));
-    }
-}
-
-// gate / up pair of a gated feed-forward
-__device__ __forceinline__ float dense_gated(const DenseCall& c, float g, float u)
+// gate / up pairs of a gated feed-forward (the branch on the activation is outside the loop: N independent chains)
+template<int N>
+__device__ __forceinline__ void dense_gated(const DenseCall& c, const float (&g)[N], const float (&u)[N], float (&r)[N])
 {
     if (c.act == kActClamped) {
-        g = fminf(g, c.act_limit);
-        u = fminf(fmaxf(u, -c.act_limit), c.act_limit);
-        return g / (1.f + expf(-c.act_alpha * g)) * (u + 1.f);
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            const float gc = fminf(g[e], c.act_limit), uc = fminf(fmaxf(u[e], -c.act_limit), c.act_limit);
+            r[e]           = gc / (1.f + expf(-c.act_alpha * gc)) * (uc + 1.f);
+        }
     }
-    return act_apply(c.act, g) * u;
+    else if (c.act == kActGeluTanh) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            r[e] = act_apply(kActGeluTanh, g[e]) * u[e];
+        }
+    }
+    else if (c.act == kActSilu) {
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            r[e] = act_apply(kActSilu, g[e]) * u[e];
+        }
+    }
+    else {
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+            r[e] = act_apply(c.act, g[e]) * u[e];
+        }
+    }
 }
 
-// the item of a batched launch: where its operands start, and its row count (<= 0: nothing to do)
+// where an item of a batched launch starts (bytes), and its row count (<= 0: nothing to do)
 struct DenseItem {
-    size_t x_off, w_off;
-    int    row_base, col_base, M;
+    int64_t x_off, w_off;
+    int     row_base, col_base, M;
 };
-__device__ __forceinline__ DenseItem dense_item(const DenseCall& c, int g, int M, int ldx, int n0)
+
+// N consecutive elements of a row, as one store where the row allows it (`vec`: rows and columns aligned to the vector)
+template<class O, int N>
+__device__ __forceinline__ void store_run(O* y, size_t i, const float (&v)[N], bool vec, int left)
 {
-    DenseItem it{(size_t)g * c.x_col_stride, (size_t)g * c.w_stride, 0, g * c.y_col_stride, M};
+    typedef O run_t __attribute__((ext_vector_type(N)));
+    if (vec && left >= N) {
+        run_t o;
 #pragma unroll
-    for (int s = 1; s < kDenseMaxSeg; ++s) {  // (the segment of this workgroup's columns)
-        it.x_off += s < c.n_seg && n0 >= c.seg_n0[s] ? c.x_col_stride : 0;
-    }
-    if (c.row_offsets) {
-        it.row_base = c.row_offsets[g];
-        it.x_off += (size_t)it.row_base * ldx;
-        it.M = c.row_offsets[g + 1] - it.row_base;
-    }
-    return it;
-}
-
-// ---- bf16, M <= 32 ------------------------------------------------------------------------------------------------------------
-// grid = ceil(N / (16 * NT)) workgroups of 4, 8 or 16 waves (narrow outputs with a long K: more waves split K so that the device still
-// holds enough of them to cover the HBM latency).  A wave owns NT tiles of 16 output columns x MT tiles of 16 rows and every fourth
-// k-chunk (eight 32-k MFMA steps with one column tile, four with two); an activation fragment serves the NT
-// column tiles, a weight fragment the MT row tiles.  The weight stream is what comes from HBM, so it runs one chunk AHEAD in a second
-// register buffer: the loads of chunk c + 1 are in flight under the activation reads (L2 hits) and MFMAs of chunk c.  The waves'
-// partial sums meet in LDS.
-
-template<int MT, int NT, int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void dense_skinny_bf16_kernel(const __bf16* __restrict__ x, int ldx, const __bf16* __restrict__ w, int Kp,
-                                                                void* __restrict__ y, int ldy, int M, int N, DenseCall call)
-{
-    __shared__ float red[WAVES][MT * NT][64][4];
-    const DenseItem it = dense_item(call, blockIdx.y, M, ldx, blockIdx.x * 16 * NT);
-    const int       row_base = it.row_base, col_base = it.col_base;
-    M = it.M, x += it.x_off, w += it.w_off;
-    if (M <= 0) {
+        for (int e = 0; e < N; ++e) {
+            o[e] = (O)v[e];
+        }
+        *(run_t*)(y + i) = o;
         return;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n0   = blockIdx.x * 16 * NT;
-    const int r    = lane & 15, kc = (lane >> 4) * 8;
-    const __bf16* wp[NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) {
-        // fragment order: block (tile, k / 32) at ((tile * Kp / 32 + k / 32) * 64 + lane) * 8 -- k advances by 16 elements per k.
-        // Tiles up to Np / 16 exist (zero): no column test in the loop
-        wp[j] = w + ((size_t)(n0 / 16 + j) * (Kp >> 5) * 64 + lane) * 8;
+    for (int e = 0; e < N; ++e) {
+        if (e < left) {
+            y[i + e] = (O)v[e];
+        }
     }
-    const __bf16* xp[MT];
-    bool          xin[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        xin[t] = t * 16 + r < M;
-        xp[t]  = x + (size_t)(xin[t] ? t * 16 + r : 0) * ldx + kc;
+}
+
+// Epilogues on four consecutive columns n .. n + 3 of row m.  EPI >= 0: known at compile time (a kernel with many outputs per thread must not
+// carry every epilogue per output: the unroller gives up and the accumulators land in scratch memory); -1: the call's own
+template<class T, int EPI>
+struct DenseEpi {
+    DenseCall c;
+    int       vec;  // rows of y (and of the operands read beside it) start at multiples of 16 bytes
+
+    static constexpr bool kPairs = EPI == kDenseGatedAct && sizeof(T) == 2;
+    __device__ __forceinline__ const int* row_offsets() const
+    {
+        return c.row_offsets;
     }
-    floatx4 acc[MT][NT];
+    __device__ __forceinline__ int items() const
+    {
+        return c.count;
+    }
+    __device__ __forceinline__ DenseItem item(int g, int M, int n0) const
+    {
+        DenseItem it{(int64_t)g * c.x_col_stride, (int64_t)g * (int64_t)c.w_stride, 0, g * c.y_col_stride, M};
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
+        for (int s = 1; s < kDenseMaxSeg; ++s) {  // (the segment of this workgroup's columns)
+            it.x_off += s < c.n_seg && n0 >= c.seg_n0[s] ? c.x_col_stride : 0;
+        }
+        if (c.row_offsets) {
+            it.row_base = c.row_offsets[g];
+            it.x_off += (int64_t)it.row_base * c.ldx;
+            it.M = c.row_offsets[g + 1] - it.row_base;
+        }
+        it.x_off *= sizeof(T), it.w_off *= sizeof(T);
+        return it;
+    }
+    // acc[j]: columns n + 16 j .. + 3
+    template<int NT>
+    __device__ __forceinline__ void rows(const StreamArgs& a, const DenseItem& it, int m, int n, const floatx4 (&acc)[NT]) const
+    {
+        const int epi = EPI >= 0 ? EPI : c.epi;
+        m += it.row_base;
+        if (epi == kDenseGatedAct) {
+            if constexpr (sizeof(T) == 4) {  // the four columns are gate, gate, up, up of two outputs
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const int   o    = (n + 16 * j) >> 1;
+                    const float g[2] = {acc[j][0], acc[j][1]}, u[2] = {acc[j][2], acc[j][3]};
+                    float       r[2];
+                    dense_gated(c, g, u, r);
+                    store_run<T, 2>((T*)a.y, (size_t)m * a.ldy + it.col_base + o, r, vec, c.n_out - o);
+                }
+            }
+            else if constexpr (NT % 2 == 0) {  // tiles 2 j, 2 j + 1 of the image are the gate / up halves of output tile j
+#pragma unroll
+                for (int j = 0; j < NT; j += 2) {
+                    const int n16 = n & ~15, o = (n16 >> 1) + (n & 15) + 8 * j;
+                    const float g[4] = {acc[j][0], acc[j][1], acc[j][2], acc[j][3]}, u[4] = {acc[j + 1][0], acc[j + 1][1], acc[j + 1][2], acc[j + 1][3]};
+                    float       r[4];
+                    dense_gated(c, g, u, r);
+                    store_run<T, 4>((T*)a.y, (size_t)m * a.ldy + it.col_base + o, r, vec, c.n_out - o);
+                }
+            }
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            acc[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+            one(a, it, m, n + 16 * j, acc[j], epi);
         }
     }
-    // MFMA steps per chunk: two chunk buffers of KS x NT fragments must leave room for three to four waves per SIMD
-    constexpr int kSkinnyKS = NT == 1 ? 8 : 4;
-    const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-    bf16x8       wa[kSkinnyKS][NT], wb[kSkinnyKS][NT];
-    auto fetch = [&](bf16x8 (&buf)[kSkinnyKS][NT], int k0) {
-#pragma unroll
-        for (int kk = 0; kk < kSkinnyKS; ++kk) {
-            const int k = k0 + kk * 32;
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                const bf16x8 v = *(const bf16x8*)(wp[j] + (size_t)min(k, Kp - 32) * 16);  // (k / 32) blocks of 512 elements; loads are
-                buf[kk][j]     = k < Kp ? v : zero;                                        // unconditional so that all stay in flight
-            }
+    __device__ __forceinline__ void one(const StreamArgs& a, const DenseItem& it, int m, int n, floatx4 acc, int epi) const
+    {
+        const int left = a.N - n;
+        if (left <= 0) {
+            return;
         }
-    };
-    auto compute = [&](const bf16x8 (&buf)[kSkinnyKS][NT], int k0) {
+        const size_t i = (size_t)m * a.ldy + it.col_base + n;
+        float        r[4];
+        if (epi == kDenseStore || epi == kDenseRelu2 || epi == kDenseXielu || epi == kDenseActTable) {
+            if (epi == kDenseXielu) {
+                const float p = c.act_par[0], q = c.act_par[1];
 #pragma unroll
-        for (int kk = 0; kk < kSkinnyKS; ++kk) {
-            const int k = k0 + kk * 32;
-            if (k < Kp) {
-                bf16x8 a[MT];
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const bf16x8 v = *(const bf16x8*)(xp[t] + k);  // (rows beyond M read row 0)
-                    a[t]           = xin[t] ? v : zero;
-                }
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) {
-                        acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], buf[kk][j], acc[t][j], 0, 0, 0);
-                    }
+                for (int e = 0; e < 4; ++e) {
+                    const float z = acc[e];
+                    r[e]          = z > 0.f ? fmaf(p * z, z, 0.5f * z) : fmaf(q, expm1f(z) - z, 0.5f * z);
                 }
             }
-        }
-    };
-    constexpr int kChunk = kSkinnyKS * 32, kStride = WAVES * kChunk;  // the waves interleave their chunks
-    int k0 = wave * kChunk;
-    if (k0 < Kp) {
-        fetch(wa, k0);
-    }
-    for (; k0 < Kp; k0 += 2 * kStride) {
-        const int k1 = k0 + kStride, k2 = k1 + kStride;
-        if (k1 < Kp) {
-            fetch(wb, k1);
-        }
-        compute(wa, k0);
-        if (k2 < Kp) {
-            fetch(wa, k2);
-        }
-        if (k1 < Kp) {
-            compute(wb, k1);
-        }
-    }
+            else if (epi == kDenseActTable) {
+                const int     id  = min(max(c.ids[m], 0), c.table_rows - 1);
+                const __bf16* row = (const __bf16*)c.table + (size_t)id * c.ld_table + c.table_col + n;
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                red[wave][t * NT + j][lane][i] = acc[t][j][i];
-            }
-        }
-    }
-    __syncthreads();
-    if (call.epi == kDenseGatedAct) {  // column tiles 2 j, 2 j + 1 of the image are the gate / up halves of output tile j
-        if constexpr (NT == 2) {
-            for (int idx = threadIdx.x; idx < MT * 256; idx += WAVES * 64) {
-                const int t = idx >> 8, l = (idx >> 2) & 63, i = idx & 3;
-                float     g = 0.f, u = 0.f;
-#pragma unroll
-                for (int wv = 0; wv < WAVES; wv += 4) {
-                    g += (red[wv][t * 2][l][i] + red[wv + 1][t * 2][l][i]) + (red[wv + 2][t * 2][l][i] + red[wv + 3][t * 2][l][i]);
-                    u += (red[wv][t * 2 + 1][l][i] + red[wv + 1][t * 2 + 1][l][i]) + (red[wv + 2][t * 2 + 1][l][i] + red[wv + 3][t * 2 + 1][l][i]);
-                }
-                const int m = t * 16 + (l >> 4) * 4 + i, n = (n0 >> 1) + (l & 15);
-                if (m < M && n < call.n_out) {
-                    ((__bf16*)y)[(size_t)(row_base + m) * ldy + col_base + n] = (__bf16)dense_gated(call, g, u);
+                for (int e = 0; e < 4; ++e) {
+                    r[e] = e < left ? act_apply(c.act, acc[e]) * (float)row[e] : 0.f;
                 }
             }
-        }
-        return;
-    }
-    for (int idx = threadIdx.x; idx < MT * NT * 256; idx += WAVES * 64) {
-        const int tj = idx >> 8, l = (idx >> 2) & 63, i = idx & 3;
-        float     s  = 0.f;
+            else {
 #pragma unroll
-        for (int wv = 0; wv < WAVES; wv += 4) {  // fixed order: the result does not depend on which wave finished first
-            s += (red[wv][tj][l][i] + red[wv + 1][tj][l][i]) + (red[wv + 2][tj][l][i] + red[wv + 3][tj][l][i]);
-        }
-        // C fragment: column = lane % 16, rows (lane / 16) * 4 + i
-        const int m = (tj / NT) * 16 + (l >> 4) * 4 + i, n = n0 + (tj % NT) * 16 + (l & 15);
-        if (m < M && n < N) {
-            dense_epilogue<__bf16>(y, ldy, row_base + m, col_base + n, s, call);
-        }
-    }
-}
-
-// ---- bf16, tiled ----------------------------------------------------------------------------------------------------------------
-constexpr int kTN = 128, kTK = 32, kLdsRow = kTK + 8;  // 80-byte LDS rows: 16-byte fragment reads of 16 rows hit all banks once
-// TM: rows of a workgroup tile, 128, or 64 | 32 where 128-row tiles of a narrow output would leave CUs without work
-
-template<int EPI, int TM>
-__global__ __launch_bounds__(256) void dense_tiled_bf16_kernel(const __bf16* __restrict__ x, int ldx, const __bf16* __restrict__ w, int Kp,
-                                                               void* __restrict__ y, int ldy, int M, int N, DenseCall call)
-{
-    constexpr int RI = TM / 32;  // 16-row tiles per wave
-    __shared__ __attribute__((aligned(16))) __bf16 sa[2][TM * kLdsRow];
-    __shared__ __attribute__((aligned(16))) __bf16 sb[2][kTN * kLdsRow];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * kTN;
-    const DenseItem it = dense_item(call, blockIdx.z, M, ldx, n0);
-    const int       row_base = it.row_base, col_base = it.col_base;
-    M = it.M, x += it.x_off, w += it.w_off;
-    if (m0 >= M) {  // the whole workgroup: an item with fewer rows than the launch's largest
-        return;
-    }
-    const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * 64;
-    // staging: 128 rows x 32 k = 512 16-byte vectors per operand, two per thread: vector v -> row v / 4, k chunk (v % 4) * 8 (TM = 64: one
-    // activation vector per thread, TM = 32: one for the first half of the threads)
-    const int  sr0 = tid >> 2, sr1 = sr0 + 64, sk = (tid & 3) * 8;
-    const bool a0 = sr0 < TM && m0 + sr0 < M, a1 = TM > 64 && m0 + sr1 < M;
-    const __bf16* ap0 = x + (size_t)(a0 ? m0 + sr0 : 0) * ldx + sk;
-    const __bf16* ap1 = x + (size_t)(a1 ? m0 + sr1 : 0) * ldx + sk;
-    // weights come in fragment order: vector v of a 128 x 32 tile = lane v % 64 of 16-row tile v / 64; it lands in the LDS row of that lane
-    const int bt0 = tid >> 6, bt1 = bt0 + 4, bl = tid & 63;
-    const int br0 = bt0 * 16 + (bl & 15), br1 = bt1 * 16 + (bl & 15), bk = (bl >> 4) * 8;
-    const __bf16* bp0 = w + ((size_t)(n0 / 16 + bt0) * (Kp >> 5) * 64 + bl) * 8;
-    const __bf16* bp1 = w + ((size_t)(n0 / 16 + bt1) * (Kp >> 5) * 64 + bl) * 8;
-    const bf16x8  zero = {0, 0, 0, 0, 0, 0, 0, 0};
-    bf16x8        ra0, ra1, rb0, rb1;
-    auto fetch = [&](int k) {
-        const bf16x8 v0 = *(const bf16x8*)(ap0 + k);  // unconditional (rows beyond M read row 0)
-        ra0 = a0 ? v0 : zero;
-        if constexpr (TM > 64) {
-            const bf16x8 v1 = *(const bf16x8*)(ap1 + k);
-            ra1 = a1 ? v1 : zero;
-        }
-        rb0 = *(const bf16x8*)(bp0 + (size_t)k * 16);
-        rb1 = *(const bf16x8*)(bp1 + (size_t)k * 16);
-    };
-    auto stash = [&](int buf) {
-        if (TM >= 64 || sr0 < TM) {
-            *(bf16x8*)(&sa[buf][sr0 * kLdsRow + sk]) = ra0;
-        }
-        if constexpr (TM > 64) {
-            *(bf16x8*)(&sa[buf][sr1 * kLdsRow + sk]) = ra1;
-        }
-        *(bf16x8*)(&sb[buf][br0 * kLdsRow + bk]) = rb0;
-        *(bf16x8*)(&sb[buf][br1 * kLdsRow + bk]) = rb1;
-    };
-    floatx4 acc[RI][4];
-#pragma unroll
-    for (int i = 0; i < RI; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    const int fr = lane & 15, fk = (lane >> 4) * 8;
-    fetch(0);
-    stash(0);
-    __syncthreads();
-    const int steps = Kp / kTK;
-    for (int s = 0; s < steps; ++s) {
-        const int buf = s & 1;
-        if (s + 1 < steps) {
-            fetch((s + 1) * kTK);
-        }
-        bf16x8 fa[RI], fb[4];
-#pragma unroll
-        for (int i = 0; i < RI; ++i) {
-            fa[i] = *(const bf16x8*)(&sa[buf][(wm + i * 16 + fr) * kLdsRow + fk]);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            fb[i] = *(const bf16x8*)(&sb[buf][(wn + i * 16 + fr) * kLdsRow + fk]);
-        }
-#pragma unroll
-        for (int i = 0; i < RI; ++i) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-            }
-        }
-        if (s + 1 < steps) {
-            stash(buf ^ 1);  // the other buffer: its readers finished before the barrier that ended step s - 1
-        }
-        __syncthreads();
-    }
-    if constexpr (EPI == kDenseGatedAct) {
-#pragma unroll
-        for (int i = 0; i < RI; ++i) {
-#pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int m = m0 + wm + i * 16 + (lane >> 4) * 4 + q, n = ((n0 + wn) >> 1) + (j >> 1) * 16 + (lane & 15);
-                    if (m < M && n < call.n_out) {
-                        ((__bf16*)y)[(size_t)(row_base + m) * ldy + col_base + n] = (__bf16)dense_gated(call, acc[i][j][q], acc[i][j + 1][q]);
-                    }
+                for (int e = 0; e < 4; ++e) {
+                    const float z = epi == kDenseRelu2 ? fmaxf(acc[e], 0.f) : acc[e];
+                    r[e]          = epi == kDenseRelu2 ? z * z : z;
                 }
             }
+            store_run<T, 4>((T*)a.y, i, r, vec, left);
+            return;
         }
-        return;
-    }
+        float* y = (float*)a.y;
+        if (epi == kDenseScaleF32 || epi == kDenseBiasF32) {
 #pragma unroll
-    for (int i = 0; i < RI; ++i) {
+            for (int e = 0; e < 4; ++e) {
+                r[e] = epi == kDenseScaleF32 ? c.alpha * acc[e] : acc[e] + (e < left ? c.bias[n + e] : 0.f);
+            }
+            store_run<float, 4>(y, i, r, vec, left);
+            return;
+        }
+        // the residual stream is read and written
+        floatx4 old = {0.f, 0.f, 0.f, 0.f}, g = old;
+        if (vec && left >= 4) {
+            old = *(const floatx4*)(y + i);
+        }
+        else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int m = m0 + wm + i * 16 + (lane >> 4) * 4 + q, n = n0 + wn + j * 16 + (lane & 15);
-                if (m < M && n < N) {
-                    dense_epilogue<__bf16, EPI>(y, ldy, row_base + m, col_base + n, acc[i][j][q], call);
-                }
+            for (int e = 0; e < 4; ++e) {
+                old[e] = e < left ? y[i + e] : 0.f;
             }
         }
-    }
-}
-
-// ---- fp32 -------------------------------------------------------------------------------------------------------------------------
-// 64 x 64 x 16 tiles, 256 threads, 4 x 4 outputs per thread; operands transposed into LDS ([k][row]) so that a thread's four rows /
-// columns are one 16-byte read.  fmaf in k order: the result of a row does not depend on what shares its tile.
-template<int EPI>
-__global__ __launch_bounds__(256) void dense_f32_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w, int Kp,
-                                                        void* __restrict__ y, int ldy, int M, int N, DenseCall call)
-{
-    __shared__ __attribute__((aligned(16))) float sa[16][64 + 4];
-    __shared__ __attribute__((aligned(16))) float sb[16][64 + 4];
-    const int tid = threadIdx.x;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    const DenseItem it = dense_item(call, blockIdx.z, M, ldx, n0);
-    const int       row_base = it.row_base, col_base = it.col_base;
-    M = it.M, x += it.x_off, w += it.w_off;
-    if (m0 >= M) {
-        return;
-    }
-    const int tr = (tid >> 4) * 4, tc = (tid & 15) * 4;
-    const int lr = tid >> 2, lk = (tid & 3) * 4;  // staging: row lr (0..63), k chunk lk (0, 4, 8, 12)
-    const bool   ain = m0 + lr < M;
-    const float* ap  = x + (size_t)(ain ? m0 + lr : 0) * ldx + lk;
-    const float* bp  = w + (size_t)(n0 + lr) * Kp + lk;
-    float        acc[4][4] = {};
-    for (int k = 0; k < Kp; k += 16) {
-        const floatx4 va = ain ? *(const floatx4*)(ap + k) : floatx4{0.f, 0.f, 0.f, 0.f};
-        const floatx4 vb = *(const floatx4*)(bp + k);
-        __syncthreads();
+        if (epi == kDenseResidAdd) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            sa[lk + i][lr] = va[i];
-            sb[lk + i][lr] = vb[i];
+            for (int e = 0; e < 4; ++e) {
+                r[e] = old[e] + c.alpha * acc[e];
+            }
+            store_run<float, 4>(y, i, r, vec, left);
+            if (c.y2) {
+                store_run<T, 4>((T*)c.y2, (size_t)m * c.ldy2 + n, r, vec, left);
+            }
+            return;
         }
-        __syncthreads();
+        // kDenseResidGate
+        const float* gp = c.gate + (size_t)m * c.ldg + n;
+        if (vec && left >= 4) {
+            g = *(const floatx4*)gp;
+        }
+        else {
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            const floatx4 a = *(const floatx4*)(&sa[kk][tr]);
-            const floatx4 b = *(const floatx4*)(&sb[kk][tc]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-                }
+            for (int e = 0; e < 4; ++e) {
+                g[e] = e < left ? gp[e] : 0.f;
             }
         }
-    }
-    if constexpr (EPI == kDenseGatedAct) {  // a thread's columns are gate, gate, up, up of two outputs
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const int m = m0 + tr + i, n = ((n0 + tc) >> 1) + j;
-                if (m < M && n < call.n_out) {
-                    ((float*)y)[(size_t)(row_base + m) * ldy + col_base + n] = dense_gated(call, acc[i][j], acc[i][j + 2]);
-                }
-            }
+        for (int e = 0; e < 4; ++e) {
+            const float z = g[e] + (e < left ? c.gate_bias[n + e] : 0.f);
+            r[e]          = old[e] + acc[e] / (1.f + expf(-z));
         }
-        return;
+        store_run<float, 4>(y, i, r, vec, left);
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int m = m0 + tr + i, n = n0 + tc + j;
-            if (m < M && n < N) {
-                dense_epilogue<float, EPI>(y, ldy, row_base + m, col_base + n, acc[i][j], call);
-            }
-        }
-    }
-}
+};
 
 // ---- weight images ----------------------------------------------------------------------------------------------------------------
 // src: bf16 [rows][cols] (checkpoint bytes) -> dst[(row0 + r) * Kp + col0 + c], T = bf16 (copy) or float (exact widening)
-// bf16 images are stored in FRAGMENT ORDER: the 16 rows x 32 k block (n / 16, k / 32) is one contiguous KB laid out as the 64 lanes of
-// its MFMA fragment (lane = (k % 32) / 8 * 16 + n % 16, eight k each), blocks of one 16-row tile consecutive along k -- a wave's fragment
+// Images are stored in FRAGMENT ORDER: the 16 rows x 64 bytes block (n / 16, k / step) is one contiguous KB laid out as the 64 lanes of
+// its MFMA fragment (16 bytes each: lane = piece * 16 + n % 16), blocks of one 16-row tile consecutive along k -- a wave's fragment
 // load is one contiguous KB and a workgroup streams whole contiguous runs of HBM instead of 64-byte pieces of 16 rows
+template<class T>
 __host__ __device__ inline size_t dense_frag_index(int n, int k, int Kp)
 {
-    return ((((size_t)(n >> 4) * (Kp >> 5) + (k >> 5)) * 64 + ((k & 31) >> 3) * 16 + (n & 15)) << 3) + (k & 7);
+    constexpr int E = 16 / sizeof(T), S = 4 * E;  // elements of a 16-byte piece, of a step
+    return (((size_t)(n >> 4) * (Kp / S) + k / S) * 64 + (k % S) / E * 16 + (n & 15)) * E + k % E;
 }
 
 template<class T>
@@ -459,12 +259,7 @@ __global__ void dense_place_kernel(T* __restrict__ dst, int Kp, int row0, int co
         if (half) {
             n = dense_pair_row(n, half - 1, sizeof(T) == 4);
         }
-        if constexpr (sizeof(T) == 2) {
-            dst[dense_frag_index(n, k, Kp)] = (T)(float)src[i];
-        }
-        else {
-            dst[(size_t)n * Kp + k] = (T)(float)src[i];
-        }
+        dst[dense_frag_index<T>(n, k, Kp)] = (T)(float)src[i];
     }
 }
 
@@ -512,6 +307,60 @@ void dense_weight_free(DenseWeight& d)
     d.w = nullptr;
 }
 
+// The lines between the kernels are a model of one CU's time in microseconds, fitted to measurements of this file's kernels (graph replays, weights from HBM).
+//   tile kernels: (tiles of the fullest CU) x (steps x time of a step with the CU full + prologue and results), at least one tile alone.  16-bit, 8192
+//     rows, (K, N) = (4096, 21504): 256 x 256 1155 us (1.25 PFLOP/s), 256 x 128 1281, 128 x 128 1520, 64 x 64 2714; (2048, 256) with 8000 rows: 46,
+//     33, 23, 20 us; (2048, 2048) with 2600 rows: 50, 36, 35, 48 us
+//   skinny kernel: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; 25 GB/s a CU, a line of x (from L2) at 0.7 of the
+//     price of a line of weights.  32 rows bf16, (25600, 4096): one slice 119 us, four 46, eight 45; (4096, 6144): one 23, three 19, four 18;
+//     (4096, 21504): one 40, two 42; nine items of (2048, 2816): one 21, three 31; three rows fp32, (8448, 2048): one 75, eight 21; pairs, four
+//     rows, (2048, 11264): one 17, two 23
+//   narrow kernel: eight rows bf16, (2048, 2048): 6.5 us against 7.3 with four slices; three rows fp32, (768, 2048): 6.1 against 7.8, (2048, 2048): 11.2
+//     against 9.8; without scratch (25600, 4096) with 32 rows: 76 against 120
+StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets)
+{
+    struct Tile {
+        int    rows, cols;
+        double full16, alone16, full32, alone32, fixed;
+    };
+    static const Tile kTiles[] = {{256, 256, 0.83, 0.83, 1e9, 1e9, 8.0}, {256, 128, 0.46, 0.55, 1.75, 1.75, 5.0}, {128, 128, 0.283, 0.40, 0.90, 0.95, 3.0},
+                                  {64, 64, 0.125, 0.25, 0.24, 0.32, 1.0}};
+    StreamPlan        best{};
+    double            cost = 1e30;
+    for (int k = 0; k < 4; ++k) {
+        const Tile&   t     = kTiles[k];
+        const int64_t rt    = own_rows ? rows / t.rows + items : (int64_t)((rows + t.rows - 1) / t.rows) * items;
+        const int64_t n     = (rt * ((cols + t.cols - 1) / t.cols) + 255) / 256;
+        const double  full  = elem == 4 ? t.full32 : t.full16, alone = elem == 4 ? t.alone32 : t.alone16;
+        const double  fixed = k == 0 && pairs ? 22.0 : t.fixed;  // (an activation per output, and no other workgroup on the CU meanwhile)
+        const double  c     = std::max(n * (full * steps + fixed), alone * steps + fixed);
+        if (c < cost) {
+            cost = c, best.tile = k;
+        }
+    }
+    if (own_rows ? rows > 64 : rows > 256) {  // (an item's rows are one block of the skinny kernel)
+        return best;
+    }
+    const int    mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, rb = (rows + 16 * mt - 1) / (16 * mt), wg_cols = pairs ? 128 : 64;
+    const int    groups = (cols + wg_cols - 1) / wg_cols * items * rb;
+    const double step   = 64.0 * (wg_cols + 0.7 * std::min(rows, 16 * mt)) / 25e3;
+    int          sp     = groups >= (pairs ? 80 : 200) ? 1 : (256 + groups - 1) / groups;  // about one workgroup a CU
+    sp          = std::max(1, std::min({sp, steps / 16, 16}));
+    best.narrow = groups < 200 && !pairs && rows <= 16 && steps <= 64;  // short sums: the way through memory costs more than it gives
+    if (best.narrow) {
+        sp = 1;
+    }
+    if (sp > 1 && ((size_t)groups * sp * mt * 16 * wg_cols * 4 > ws_bytes || groups > tickets)) {
+        sp = 1, best.narrow = true;
+    }
+    const int    ss = ((steps + sp - 1) / sp + 7) / 8 * 8;
+    const double c  = std::max(1.0, groups * sp / 256.0) * ss * step + 3.0;
+    if (rows <= 64 || c < cost) {
+        best.skinny = true, best.mt = mt, best.splits = (steps + ss - 1) / ss, best.split_steps = ss, best.row_blocks = rb;
+    }
+    return best;
+}
+
 int launch_dense_linear(const DenseWeight& d, const void* x, int ldx, void* y, int ldy, int M, int epi, float alpha, hipStream_t st)
 {
     DenseCall c;
@@ -534,6 +383,104 @@ int launch_dense_linear(const DenseWeight& d, const void* x, int ldx, void* y, i
         case kDenseActTable: LAUNCH(kDenseActTable); break;  \
     }
 
+template<class T, int MT, int NT, int CW, int KP>
+static int launch_dense_skinny(const StreamArgs& a, const DenseCall& call, int vec, dim3 grid, hipStream_t st)
+{
+    stream_skinny_kernel<T, DenseEpi<T, -1>, MT, NT, CW, KP><<<grid, CW * KP * 64, 0, st>>>(a, DenseEpi<T, -1>{call, vec});
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+template<class T, int MT, int NT>
+static int launch_dense_narrow(const StreamArgs& a, const DenseCall& call, int vec, int items, hipStream_t st)
+{
+    constexpr int W = MT * NT <= 2 ? 16 : 8;
+    stream_narrow_kernel<T, DenseEpi<T, -1>, MT, NT, W><<<dim3((a.tiles + NT - 1) / NT, items * a.row_blocks), W * 64, 0, st>>>(a, DenseEpi<T, -1>{call, vec});
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+static dim3 stream_tile_grid(const StreamArgs& a, int bm, int bn, const DenseCall& call)
+{
+    const unsigned tns = (a.tiles * 16 + bn - 1) / bn;
+    return call.row_offsets ? dim3((a.M / bm + call.count) * tns) : dim3((a.M + bm - 1) / bm * tns, call.count);
+}
+
+template<class T, int EPI, int BM, int BN, int WM, int WN>
+static int launch_dense_tile(const StreamArgs& a, const DenseCall& call, int vec, hipStream_t st)
+{
+    constexpr int lds = 3 * (BM + BN) * 64;
+    const auto    k   = stream_tile_kernel<T, DenseEpi<T, EPI>, BM, BN, WM, WN>;
+    if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {
+        return rc;
+    }
+    k<<<stream_tile_grid(a, BM, BN, call), 256, lds, st>>>(a, DenseEpi<T, EPI>{call, vec});
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+template<class T, int EPI>
+static int launch_dense_tile256(const StreamArgs& a, const DenseCall& call, int vec, hipStream_t st)
+{
+    constexpr int lds = 3 * 512 * 64;
+    const auto    k   = stream_tile256_kernel<T, DenseEpi<T, EPI>>;
+    if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {
+        return rc;
+    }
+    k<<<stream_tile_grid(a, 256, 256, call), 256, lds, st>>>(a, DenseEpi<T, EPI>{call, vec});
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+template<class T>
+static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void* y, int ldy, int M, const DenseCall& call, hipStream_t st)
+{
+    const int  epi = call.epi, G = call.count;
+    StreamArgs a{};
+    a.x = (const char*)x, a.ldx = (int64_t)ldx * sizeof(T);
+    a.w = (const char*)d.w, a.steps = (int)(d.Kp * sizeof(T) / 64), a.tiles = d.Np / 16;
+    a.w_tile = (int64_t)a.steps * 1024, a.w_quad = 4096;
+    a.y = y, a.ldy = ldy, a.M = M, a.N = d.N;
+    const bool f32_out = epi == kDenseResidAdd || epi == kDenseScaleF32 || epi == kDenseBiasF32 || epi == kDenseResidGate;
+    const int  align   = f32_out || sizeof(T) == 4 ? 4 : 8;  // elements of 16 bytes
+    const int  vec     = ldy % align == 0 && (uintptr_t)y % 16 == 0 && call.y_col_stride % align == 0
+                    && (!call.y2 || (call.ldy2 % 8 == 0 && (uintptr_t)call.y2 % 16 == 0))
+                    && (epi != kDenseResidGate || (call.ldg % 4 == 0 && (uintptr_t)call.gate % 16 == 0));
+    const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2, d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0);
+    if (p.skinny) {
+        const bool pairs = epi == kDenseGatedAct && sizeof(T) == 2;
+        a.split_steps    = p.split_steps;
+        a.row_blocks     = p.row_blocks;
+        a.slabs          = p.splits > 1 ? d.scratch->slabs : nullptr;
+        a.tickets        = p.splits > 1 ? d.scratch->tickets : nullptr;
+        const dim3 grid((unsigned)((a.tiles + (pairs ? 7 : 3)) / (pairs ? 8 : 4)), G * p.row_blocks, p.splits);
+#define TM_SKINNY(MT_, NT_, CW_, KP_)                                                    \
+    if (p.mt == MT_ && pairs == (NT_ == 2)) {                                            \
+        if (p.narrow) {                                                                  \
+            return launch_dense_narrow<T, MT_, NT_>(a, call, vec, G, st);                \
+        }                                                                                \
+        return launch_dense_skinny<T, MT_, NT_, CW_, KP_>(a, call, vec, grid, st);       \
+    }
+        TM_STREAM_SHAPES(TM_SKINNY)
+        if constexpr (sizeof(T) == 2) {
+            TM_STREAM_SHAPES_PAIRS(TM_SKINNY)
+        }
+#undef TM_SKINNY
+    }
+#define TM_TILE(EPI_)                                                                    \
+    if constexpr (sizeof(T) == 2 && EPI_ != kDenseActTable) {                            \
+        if (p.tile == 0) {                                                               \
+            return launch_dense_tile256<T, EPI_>(a, call, vec, st);                      \
+        }                                                                                \
+    }                                                                                    \
+    return p.tile <= 1 ? launch_dense_tile<T, EPI_, 256, 128, 2, 2>(a, call, vec, st) :  \
+           p.tile == 2 ? launch_dense_tile<T, EPI_, 128, 128, 2, 2>(a, call, vec, st) :  \
+                         launch_dense_tile<T, EPI_, 64, 64, 2, 2>(a, call, vec, st)
+    TM_EPI_SWITCH(TM_TILE)
+#undef TM_TILE
+    return 0;
+}
+
 int launch_dense_call(const DenseWeight& d, const void* x, int ldx, void* y, int ldy, int M, DenseCall call, hipStream_t st)
 {
     const int epi = call.epi;
@@ -551,88 +498,21 @@ int launch_dense_call(const DenseWeight& d, const void* x, int ldx, void* y, int
     TM_REQUIRE(call.n_seg >= 0 && call.n_seg <= kDenseMaxSeg && (call.n_seg == 0 || (call.count == 1 && call.seg_n0[0] == 0 && ldx >= d.Kp + (call.n_seg - 1) * call.x_col_stride)),
                "dense linear: segments");
     for (int s = 1; s < call.n_seg; ++s) {
-        TM_REQUIRE(call.seg_n0[s] % kTN == 0 && call.seg_n0[s] > call.seg_n0[s - 1] && call.seg_n0[s] < d.N, "dense linear: segment borders");
+        TM_REQUIRE(call.seg_n0[s] % 128 == 0 && call.seg_n0[s] > call.seg_n0[s - 1] && call.seg_n0[s] < d.N, "dense linear: segment borders");
     }
     TM_REQUIRE(call.act != kActClamped || epi == kDenseGatedAct, "dense linear: the clamped activation takes a gate / up pair");
     if (M == 0) {
         return 0;
     }
     call.w_stride = (size_t)d.Np * d.Kp;
-    const int G   = call.count;
+    call.ldx      = ldx;
     if (d.dtype == kDenseF32) {
         TM_REQUIRE(ldx % 4 == 0, "dense linear (fp32): rows must be 16-byte aligned");
         TM_REQUIRE(call.x_col_stride % 4 == 0, "dense linear (fp32): items must be 16-byte aligned");
-#define TM_F32(EPI_) \
-    dense_f32_kernel<EPI_><<<dim3(d.Np / 64, (M + 63) / 64, G), 256, 0, st>>>((const float*)x, ldx, (const float*)d.w, d.Kp, y, ldy, M, d.N, call)
-        TM_EPI_SWITCH(TM_F32)
-#undef TM_F32
+        return launch_dense_typed<float>(d, x, ldx, y, ldy, M, call, st);
     }
-    else {
-        TM_REQUIRE(ldx % 8 == 0 && call.x_col_stride % 8 == 0, "dense linear (bf16): rows and items must be 16-byte aligned");
-        if (M <= 32) {
-            // two column tiles per wave where that still leaves >= 512 workgroups (two per CU): wide outputs amortise the activation reads
-            const int nt     = (d.N >= 512 * 32 || epi == kDenseGatedAct) ? 2 : 1;  // (a gate / up pair is two adjacent tiles of one wave)
-            const int wgs    = (d.N + 16 * nt - 1) / (16 * nt);
-            const int chunk  = (nt == 1 ? 8 : 4) * 32;
-            int       waves  = 4;  // ... and more waves per workgroup while the device holds fewer than 16 per CU and K has a chunk for each
-            while (waves < (nt == 1 ? 16 : 8) && wgs * G * waves < 256 * 16 && d.Kp >= chunk * 2 * waves) {
-                waves *= 2;
-            }
-#define TM_SKINNY(MT_, NT_, W_)                                                                                                     \
-    dense_skinny_bf16_kernel<MT_, NT_, W_><<<dim3(wgs, G), W_ * 64, 0, st>>>((const __bf16*)x, ldx, (const __bf16*)d.w, d.Kp, y, ldy, M, d.N, call)
-#define TM_SKINNY_W(MT_, NT_)                     \
-    if (waves == 16 && NT_ == 1) {                \
-        TM_SKINNY(MT_, 1, 16);                    \
-    }                                             \
-    else if (waves >= 8) {                        \
-        TM_SKINNY(MT_, NT_, 8);                   \
-    }                                             \
-    else {                                        \
-        TM_SKINNY(MT_, NT_, 4);                   \
-    }
-            if (M <= 16) {
-                if (nt == 2) {
-                    TM_SKINNY_W(1, 2)
-                }
-                else {
-                    TM_SKINNY_W(1, 1)
-                }
-            }
-            else {
-                if (nt == 2) {
-                    TM_SKINNY_W(2, 2)
-                }
-                else {
-                    TM_SKINNY_W(2, 1)
-                }
-            }
-#undef TM_SKINNY_W
-#undef TM_SKINNY
-        }
-        else {
-#define TM_TILED_ROWS(EPI_, TM_)                                                                                                              \
-    dense_tiled_bf16_kernel<EPI_, TM_><<<dim3(d.Np / kTN, (M + TM_ - 1) / TM_, G), 256, 0, st>>>((const __bf16*)x, ldx, (const __bf16*)d.w, d.Kp, y, \
-                                                                                                 ldy, M, d.N, call)
-#define TM_TILED(EPI_)                   \
-    if (rows == 32) {                    \
-        TM_TILED_ROWS(EPI_, 32);         \
-    }                                    \
-    else if (rows == 64) {               \
-        TM_TILED_ROWS(EPI_, 64);         \
-    }                                    \
-    else {                               \
-        TM_TILED_ROWS(EPI_, 128);        \
-    }
-            // (the k order of a row's sums is the same in all of them: the choice never shows in a result)
-            const int64_t wgs  = (int64_t)(d.Np / kTN) * ((M + 127) / 128) * G;
-            const int     rows = call.row_offsets || wgs >= 256 ? 128 : wgs >= 192 ? 64 : 32;
-            TM_EPI_SWITCH(TM_TILED)
-#undef TM_TILED
-#undef TM_TILED_ROWS
-        }
-    }
-    TM_HIP_CHECK(hipGetLastError());
-    return 0;
+    TM_REQUIRE(ldx % 8 == 0 && call.x_col_stride % 8 == 0, "dense linear (bf16): rows and items must be 16-byte aligned");
+    return launch_dense_typed<__bf16>(d, x, ldx, y, ldy, M, call, st);
 }
 
 }  // namespace tmk

@@ -1,0 +1,736 @@
+// Building blocks of the unquantised products y = x . W^T (gemm_dense.hip: bf16 and fp32 checkpoint weights; gemm_w4a16.hip: the fp16
+// linears of the Llama family), one set for the three number formats.
+//
+// Weight image: 16 output columns x 64 bytes of k are one contiguous KB in MFMA fragment order, lane l holds column l % 16 and the 16 bytes at
+// (l / 16) * 16 of that column's 64 -- eight k of a 16-bit format (v_mfma_f32_16x16x32), four of fp32 (four v_mfma_f32_16x16x4, which
+// multiply and add in full 32 bits).  A "step" below is such a 64-byte range of k.  Rows of x are read in the same 64 bytes a step, so
+// everything that moves data counts in bytes and is the same code for every format.
+//
+// The weight is the MFMA's A operand: a lane's four results are four CONSECUTIVE output columns of one row of x, so results leave in
+// 8- or 16-byte stores, and a gate / up pair of a feed-forward is in one lane.
+#pragma once
+#include "tm_common.h"
+#include <type_traits>
+
+namespace tmk {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float  floatx16 __attribute__((ext_vector_type(16)));
+
+template<class T>
+struct StreamOp;
+template<>
+struct StreamOp<__bf16> {
+    static __device__ __forceinline__ floatx4 mma(u32x4 a, u32x4 b, floatx4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(bit_cast<bf16x8>(a), bit_cast<bf16x8>(b), c, 0, 0, 0);
+    }
+};
+template<>
+struct StreamOp<half_t> {
+    static __device__ __forceinline__ floatx4 mma(u32x4 a, u32x4 b, floatx4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(bit_cast<half8_t>(a), bit_cast<half8_t>(b), c, 0, 0, 0);
+    }
+};
+template<>
+struct StreamOp<float> {
+    static __device__ __forceinline__ floatx4 mma(u32x4 a, u32x4 b, floatx4 c)
+    {
+        const floatx4 fa = bit_cast<floatx4>(a), fb = bit_cast<floatx4>(b);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], c, 0, 0, 0);
+        }
+        return c;
+    }
+};
+
+struct StreamArgs {
+    const char* x;       // rows of ldx bytes, 16-byte aligned
+    int64_t     ldx;
+    const char* w;       // image of the first item
+    int64_t     w_tile;  // bytes from one 16-column tile to the next ...
+    int64_t     w_quad;  // ... and from four steps to the next four (the four are contiguous)
+    int         tiles;   // 16-column tiles the image holds
+    int         steps;   // steps of k
+    int         split_steps;  // skinny kernel: steps of one slice of k (grid z), a multiple of 8
+    int         row_blocks;   // skinny kernel: blocks of 16 MT rows (grid y = item * row_blocks + block)
+    void*       y;
+    int         ldy, M, N;
+    float*      slabs;        // skinny kernel, several slices: their partial sums, [item][column group][slice][16 rows x ...]
+    unsigned*   tickets;      // ... and an arrival counter per (item, column group), zero between launches
+};
+
+// ---- few rows: the weight stream ---------------------------------------------------------------------------------------------------
+// What bounds it: a CU keeps about 440 cache lines in flight whatever their source, so a line of x that comes from L2 costs nearly what a
+// line of weights costs.  One workgroup therefore covers CW x NT column tiles with ONE copy of its rows of x in LDS (double buffered, eight
+// steps at a time), and few columns are spread over the CUs by cutting k instead of the column group: KP waves share a column
+// tile inside the workgroup and meet in LDS, grid z slices of k meet in the last workgroup of a column group to arrive, which adds the
+// slices in slice order (the sum never depends on the order of arrival; no workgroup waits for another).
+// Weights run one chunk of eight steps ahead of the MFMAs in a second register buffer; all loads are unconditional (clamped).
+// 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 46 us = 4.5 TB/s, (4096, 21504) 40 us = 4.4 TB/s (with every wave reading x for itself, no
+// slices: 76 and 50); three rows fp32, (8448, 2048): 21 us = 3.3 TB/s (64 x 64 tiles: 331).
+template<class T, class Epi, int MT, int NT, int CW, int KP>
+__global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a, Epi epi)
+{
+    constexpr int kThreads = CW * KP * 64, kChunk = 8;
+    constexpr int kXVecs  = KP * MT * kChunk * 64;                          // 16-byte pieces of one x stage
+    constexpr int kXPer   = (kXVecs + kThreads - 1) / kThreads;             // ... per thread (kXVecs is a multiple of kThreads or of 64)
+    constexpr int kRed    = KP > 1 ? (KP - 1) * CW * MT * NT * 64 * 16 : 0;  // the other k-phases' sums
+    constexpr int kXBytes = 2 * kXVecs * 16;
+    __shared__ __attribute__((aligned(16))) char smem[kXBytes > kRed ? kXBytes : kRed];
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int cw = wave % CW, ph = wave / CW;
+    const int tile0 = (blockIdx.x * CW + cw) * NT;
+    const int  mb   = blockIdx.y % a.row_blocks * (MT * 16);
+    const auto item = epi.item(blockIdx.y / a.row_blocks, a.M, blockIdx.x * CW * NT * 16);
+    const int  M    = min(item.M - mb, MT * 16);
+    if (M <= 0) {
+        return;
+    }
+    const char* x = a.x + item.x_off + mb * a.ldx;
+    const char* w = a.w + item.w_off + lane * 16;
+    const int   s0 = blockIdx.z * a.split_steps, s1 = min(a.steps, s0 + a.split_steps);
+    const char* wp[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        wp[j] = w + (int64_t)min(tile0 + j, a.tiles - 1) * a.w_tile;
+    }
+    u32x4 wa[kChunk][NT], wb[kChunk][NT], xr[kXPer];
+    auto  fetch = [&](u32x4(&buf)[kChunk][NT], int base) {
+#pragma unroll
+        for (int kk = 0; kk < kChunk; ++kk) {
+            const int s = min(base + kk, a.steps - 1);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                buf[kk][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + (s >> 2) * a.w_quad + (s & 3) * 1024));
+            }
+        }
+    };
+    // x stage: [phase][row tile][pair of steps] blocks of 16 rows x 128 bytes, 16-byte piece c of row r at r * 128 + ((c ^ (r & 7)) * 16): a
+    // fragment read meets every bank once, a row's 128 bytes are one line of memory
+    auto fetch_x = [&](int base) {
+#pragma unroll
+        for (int i = 0; i < kXPer; ++i) {
+            const int v = tid + i * kThreads;
+            const int c = v & 7, r = (v >> 3) & 15, blk = v >> 7;
+            const int pair = blk & 3, rt = (blk >> 2) % MT, p = (blk >> 2) / MT;
+            const int row = min(rt * 16 + r, M - 1);
+            const int64_t col = min((int64_t)(base + p * kChunk + pair * 2) * 64 + c * 16, (int64_t)a.steps * 64 - 16);
+            xr[i] = *(const u32x4*)(x + row * a.ldx + col);
+        }
+    };
+    auto stash_x = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < kXPer; ++i) {
+            const int v = tid + i * kThreads;
+            if (kXVecs % kThreads == 0 || v < kXVecs) {
+                const int c = v & 7, r = (v >> 3) & 15, blk = v >> 7;
+                *(u32x4*)(smem + buf * kXVecs * 16 + blk * 2048 + r * 128 + ((c ^ (r & 7)) << 4)) = xr[i];
+            }
+        }
+    };
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            acc[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    const int   fr = lane & 15, fc = lane >> 4;
+    const char* xf = smem + ph * (MT * 4 * 2048) + fr * 128;
+    auto        one = [&](const u32x4(&buf)[kChunk][NT], int xbuf, int kk) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const u32x4 b = *(const u32x4*)(xf + xbuf * kXVecs * 16 + (t * 4 + (kk >> 1)) * 2048 + ((((kk & 1) * 4 + fc) ^ (fr & 7)) << 4));
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                acc[t][j] = StreamOp<T>::mma(buf[kk][j], b, acc[t][j]);
+            }
+        }
+    };
+    auto compute = [&](const u32x4(&buf)[kChunk][NT], int xbuf, int base) {
+        if (base + kChunk <= s1) {
+#pragma unroll
+            for (int kk = 0; kk < kChunk; ++kk) {
+                one(buf, xbuf, kk);
+            }
+        }
+        else {
+#pragma unroll
+            for (int kk = 0; kk < kChunk; ++kk) {
+                if (base + kk < s1) {
+                    one(buf, xbuf, kk);
+                }
+            }
+        }
+    };
+    constexpr int kStride = KP * kChunk;
+    fetch(wa, s0 + ph * kChunk);
+    fetch_x(s0);
+    stash_x(0);
+    __syncthreads();
+    int buf = 0;
+    for (int base = s0; base < s1; base += 2 * kStride) {
+        fetch(wb, base + kStride + ph * kChunk);
+        fetch_x(base + kStride);
+        compute(wa, buf, base + ph * kChunk);
+        stash_x(buf ^ 1);  // its readers finished before the last barrier
+        __syncthreads();
+        fetch(wa, base + 2 * kStride + ph * kChunk);
+        fetch_x(base + 2 * kStride);
+        compute(wb, buf ^ 1, base + kStride + ph * kChunk);
+        stash_x(buf);
+        __syncthreads();
+    }
+    if constexpr (KP > 1) {  // (the last barrier freed the x buffers)
+        floatx4* red = (floatx4*)smem;
+        if (ph > 0) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    red[(((ph - 1) * CW + cw) * MT * NT + t * NT + j) * 64 + lane] = acc[t][j];
+                }
+            }
+        }
+        __syncthreads();
+        if (ph == 0) {
+#pragma unroll
+            for (int p = 1; p < KP; ++p) {  // fixed order
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) {
+                        acc[t][j] += red[(((p - 1) * CW + cw) * MT * NT + t * NT + j) * 64 + lane];
+                    }
+                }
+            }
+        }
+    }
+    if (gridDim.z > 1) {
+        // 16-byte pieces in accumulator order, written through to memory (sc1) and drained before the counter moves; the last workgroup reads
+        // them past its L1 (sc1)
+        constexpr int64_t kTileFloats = (int64_t)CW * MT * NT * 256;
+        const int         group = blockIdx.y * gridDim.x + blockIdx.x;
+        float*            mine  = a.slabs + ((int64_t)group * gridDim.z) * kTileFloats;
+        const auto        rs    = __builtin_amdgcn_make_buffer_rsrc((void*)mine, 0, (int)(gridDim.z * kTileFloats * 4), 0x00020000);
+        if (ph == 0) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                if (t * 16 < M) {
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) {
+                        const int at = ((cw * MT + t) * NT + j) * 1024 + lane * 16;
+                        __builtin_amdgcn_raw_buffer_store_b128(bit_cast<u32x4>(acc[t][j]), rs, at, (int)(blockIdx.z * kTileFloats * 4), /*sc1*/ 16);
+                    }
+                }
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        unsigned* last = (unsigned*)smem;  // (every reader of the x buffers and of `red` has passed a barrier)
+        if (tid == 0) {
+            *last = __hip_atomic_fetch_add(a.tickets + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (*last != gridDim.z - 1) {
+            return;
+        }
+        if (tid == 0) {
+            __hip_atomic_store(a.tickets + group, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (ph > 0) {
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            if (t * 16 < M) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const int at = ((cw * MT + t) * NT + j) * 1024 + lane * 16;
+                    acc[t][j]    = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+                    for (int z = 0; z < (int)gridDim.z; ++z) {
+                        acc[t][j] += bit_cast<floatx4>(__builtin_amdgcn_raw_buffer_load_b128(rs, at, (int)(z * kTileFloats * 4), /*sc1*/ 16));
+                    }
+                }
+            }
+        }
+    }
+    if (KP > 1 && ph > 0) {
+        return;
+    }
+    // results: row m = t * 16 + lane % 16, columns tile * 16 + (lane / 16) * 4 + 0 .. 3
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int m = t * 16 + fr;
+        if (m < M) {
+            epi.template rows<NT>(a, item, mb + m, tile0 * 16 + fc * 4, acc[t]);
+        }
+    }
+}
+
+// The same without slices across workgroups, for callers that bring no scratch and few columns: a workgroup owns NT column tiles, its W waves take chunks of
+// eight steps in turn, each reading its own rows of x, and meet in LDS in wave order.
+template<class T, class Epi, int MT, int NT, int W>
+__global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi epi)
+{
+    constexpr int kChunk = 8 / NT;
+    __shared__ __attribute__((aligned(16))) floatx4 red[W][MT * NT][64];
+    const int  lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int  mb   = blockIdx.y % a.row_blocks * (MT * 16), tile0 = blockIdx.x * NT;
+    const auto item = epi.item(blockIdx.y / a.row_blocks, a.M, tile0 * 16);
+    const int  M    = min(item.M - mb, MT * 16);
+    if (M <= 0) {
+        return;
+    }
+    const int   fr = lane & 15, fc = lane >> 4;
+    const char* xp[MT];
+    const char* wp[NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        xp[t] = a.x + item.x_off + (int64_t)(mb + min(t * 16 + fr, M - 1)) * a.ldx + fc * 16;
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        wp[j] = a.w + item.w_off + (int64_t)min(tile0 + j, a.tiles - 1) * a.w_tile + lane * 16;
+    }
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            acc[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    u32x4 wa[kChunk][NT], wb[kChunk][NT];
+    auto  fetch = [&](u32x4(&buf)[kChunk][NT], int base) {
+#pragma unroll
+        for (int kk = 0; kk < kChunk; ++kk) {
+            const int s = min(base + kk, a.steps - 1);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                buf[kk][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + (s >> 2) * a.w_quad + (s & 3) * 1024));
+            }
+        }
+    };
+    auto compute = [&](const u32x4(&buf)[kChunk][NT], int base) {
+#pragma unroll
+        for (int kk = 0; kk < kChunk; ++kk) {
+            if (base + kk < a.steps) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const u32x4 b = *(const u32x4*)(xp[t] + (int64_t)(base + kk) * 64);
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) {
+                        acc[t][j] = StreamOp<T>::mma(buf[kk][j], b, acc[t][j]);
+                    }
+                }
+            }
+        }
+    };
+    constexpr int kStride = W * kChunk;
+    int           base    = wave * kChunk;
+    fetch(wa, base);
+    for (; base < a.steps; base += 2 * kStride) {
+        fetch(wb, base + kStride);
+        compute(wa, base);
+        fetch(wa, base + 2 * kStride);
+        compute(wb, base + kStride);
+    }
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            red[wave][t * NT + j][lane] = acc[t][j];
+        }
+    }
+    __syncthreads();
+    if (wave < MT) {  // wave t: row tile t
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            floatx4 s = red[0][wave * NT + j][lane];
+            for (int v = 1; v < W; ++v) {
+                s += red[v][wave * NT + j][lane];
+            }
+            acc[0][j] = s;
+        }
+        const int m = wave * 16 + fr;
+        if (m < M) {
+            epi.template rows<NT>(a, item, mb + m, tile0 * 16 + fc * 4, acc[0]);
+        }
+    }
+}
+
+// ---- many rows: tiles staged in LDS by DMA -------------------------------------------------------------------------------------------
+// Workgroup tile BM x BN, 4 waves of (BM / WM) x (BN / WN) outputs, one step of k (64 bytes a row) per stage, three stages in LDS.  The fragments of
+// step s + 1 are read into a second register set under the MFMAs of step s, so the stage of step s is free when step s begins: the DMA of stage s + 3
+// is issued there and has two steps to land.  One barrier a step.  Weight blocks are lane-linear in memory and in LDS; a row of x is four
+// 16-byte pieces, piece c of row r at c ^ ((r >> 1) & 3) (the swizzle is on the DMA's source address): fragment reads meet every bank once.
+__device__ __forceinline__ void stream_dma16(__amdgpu_buffer_rsrc_t rs, int voff, int soff, unsigned lds)
+{
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %1, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(voff), "s"(lds), "s"(rs), "s"(soff)
+                 : "memory");
+}
+
+// Which tile a workgroup owns.  XCD-aware order: workgroup i runs on XCD i % 8; each XCD gets a contiguous eighth of the tiles, walked in bands of
+// BAND row tiles, so that what its CUs hold at a time shares operands in its L2.  Items with rows of their own (row_offsets): the row tiles of all
+// items are one list, at most rows / BM + items long, so no workgroups stand idle for the rows an item does not have.
+struct StreamTile {
+    int tm, tn, item;  // item < 0: past the end of the list
+};
+template<int BM, int BN, int BAND>
+__device__ __forceinline__ StreamTile stream_tile_of(const StreamArgs& a, const int* row_offsets, int items)
+{
+    const int tms = row_offsets ? a.M / BM + items : (a.M + BM - 1) / BM, tns = (a.tiles * 16 + BN - 1) / BN, total = tms * tns;
+    const int i = blockIdx.x, q = total >> 3, rem = total & 7, xcd = i & 7;
+    const int lin  = xcd * q + min(xcd, rem) + (i >> 3);
+    const int band = lin / (BAND * tns), in = lin - band * BAND * tns, h = min(BAND, tms - band * BAND);
+    StreamTile t{band * BAND + in % h, in / h, (int)blockIdx.y};
+    if (row_offsets) {
+        const int lane = threadIdx.x & 63;
+        t.item         = -1;
+        for (int base = 0; base < items; base += 64) {
+            const int g   = base + lane;
+            const int n   = g < items ? (row_offsets[g + 1] - row_offsets[g] + BM - 1) / BM : 0;
+            int       sum = n;  // inclusive
+#pragma unroll
+            for (int d = 1; d < 64; d *= 2) {
+                const int up = __shfl_up(sum, d);
+                sum += lane >= d ? up : 0;
+            }
+            const uint64_t past = __ballot(t.tm < sum);
+            if (past) {
+                const int f = __builtin_ctzll(past);
+                t.item      = base + f;
+                t.tm -= __builtin_amdgcn_readlane(sum - n, f);
+                break;
+            }
+            t.tm -= __builtin_amdgcn_readlane(sum, 63);
+        }
+        t.item = __builtin_amdgcn_readfirstlane(t.item);
+        t.tm   = __builtin_amdgcn_readfirstlane(t.tm);
+    }
+    return t;
+}
+
+template<class T, class Epi, int BM, int BN, int WM, int WN>
+__global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_kernel(StreamArgs a, Epi epi)
+{
+    static_assert(WM * WN == 4, "four waves");
+    constexpr int MI = BM / WM / 16, NI = BN / WN / 16;
+    constexpr int kXB = BM * 64, kWB = BN * 64, kStage = kXB + kWB, kBufs = 3;
+    constexpr int kXP = BM / 16 / 4, kWP = BN / 16 / 4;  // DMA pieces of one KB per wave and stage
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const StreamTile t = stream_tile_of<BM, BN, 8>(a, epi.row_offsets(), epi.items());
+    if (t.item < 0) {
+        return;
+    }
+    const int  m0 = t.tm * BM, n0 = t.tn * BN;
+    const auto item = epi.item(t.item, a.M, n0);
+    const int  Mloc = min(item.M - m0, BM);
+    if (Mloc <= 0) {  // an item with fewer rows than the launch's largest
+        return;
+    }
+    const auto rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + item.x_off + m0 * a.ldx), 0, (int)((Mloc - 1) * a.ldx + (int64_t)a.steps * 64), 0x00020000);
+    const int64_t w_left = (int64_t)(a.tiles - (n0 >> 4)) * a.w_tile + (a.w_quad > 4096 ? (int64_t)((a.steps - 1) >> 2) * a.w_quad : 0);
+    const auto rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + item.w_off + (int64_t)(n0 >> 4) * a.w_tile), 0, (int)min(w_left, (int64_t)0xffffffff), 0x00020000);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
+    int            xoff[kXP];
+#pragma unroll
+    for (int r = 0; r < kXP; ++r) {
+        const int row = 16 * (kXP * wave + r) + (lane >> 2);
+        xoff[r]       = (int)(min(row, Mloc - 1) * a.ldx) + ((lane & 3) ^ ((row >> 1) & 3)) * 16;
+    }
+    int woff[kWP];
+#pragma unroll
+    for (int r = 0; r < kWP; ++r) {
+        woff[r] = (int)(min(kWP * wave + r, a.tiles - 1 - (n0 >> 4)) * a.w_tile) + lane * 16;
+    }
+    auto dma = [&](int s, int buf) {
+        const int      ws  = (int)((s >> 2) * a.w_quad) + (s & 3) * 1024;
+        const unsigned dst = lds0 + buf * kStage;
+#pragma unroll
+        for (int r = 0; r < kXP; ++r) {
+            stream_dma16(rs_x, xoff[r], s * 64, dst + (kXP * wave + r) * 1024);
+        }
+#pragma unroll
+        for (int r = 0; r < kWP; ++r) {
+            stream_dma16(rs_w, woff[r], ws, dst + kXB + (kWP * wave + r) * 1024);
+        }
+    };
+    floatx4 acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    const int wm = wave / WN, wn = wave % WN;
+    const int fr = lane & 15, fc = lane >> 4;
+    const int xf = (wm * (BM / WM) + fr) * 64 + ((fc ^ ((fr >> 1) & 3)) << 4);
+    const int wf = kXB + wn * NI * 1024 + lane * 16;
+    const int steps = a.steps;
+    u32x4     fx[2][MI], fw[2][NI];
+    auto      read = [&](int q, int buf) {
+        const char* st = smem + buf * kStage;
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            fw[q][j] = *(const u32x4*)(st + wf + j * 1024);
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            fx[q][i] = *(const u32x4*)(st + xf + i * 1024);
+        }
+    };
+    constexpr int kPieces = kXP + kWP;
+    // no branch inside a step (the reads and MFMAs of one block are interleaved): past the end the DMA fetches the last stage again, into
+    // buffers that are not read any more
+    dma(0, 0);
+    dma(min(1, steps - 1), 1);
+    dma(min(2, steps - 1), 2);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPieces) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0);
+    int  buf  = 0;  // stage of step s
+    auto step = [&](auto Q, int s) {
+        constexpr int q   = decltype(Q)::value;
+        const int     nxt = buf == 2 ? 0 : buf + 1;
+        // this wave's fragments of step s are in registers and its pieces of stage s + 1 have landed; then everybody's
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPieces) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        dma(min(s + 3, steps - 1), buf);
+        read(q ^ 1, nxt);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+                acc[i][j] = StreamOp<T>::mma(fw[q][j], fx[q][i], acc[i][j]);
+            }
+        }
+#pragma unroll
+        for (int g = 0; g < MI + NI; ++g) {  // the next step's fragment reads go between the MFMAs
+            __builtin_amdgcn_sched_group_barrier(0x008, MI * NI / (MI + NI) * (sizeof(T) == 4 ? 4 : 1), 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        }
+        buf = nxt;
+    };
+    for (int s = 0; s < steps; s += 2) {
+        step(std::integral_constant<int, 0>{}, s);
+        if (s + 1 < steps) {
+            step(std::integral_constant<int, 1>{}, s + 1);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the DMA writes this workgroup's LDS)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int m = m0 + wm * (BM / WM) + i * 16 + fr;
+        if (m < item.M) {
+            epi.template rows<NI>(a, item, m, n0 + wn * NI * 16 + fc * 4, acc[i]);
+        }
+    }
+}
+
+// ---- many rows of a 16-bit format: 256 x 256 tiles -----------------------------------------------------------------------------------
+// 4 waves of 128 x 128 outputs (v_mfma_f32_32x32x16, 256 accumulator registers, one wave per SIMD): a step moves 32 KB into a CU and 64 KB out of its LDS per
+// 1024 cycles of matrix work, where the 256 x 128 tiles above move 48 and 96.  bf16, 8192 rows, MI355X: (K, N) = (4096, 21504) 1155 us = 1.25 PFLOP/s, (25600, 4096) 1370 us =
+// 1.25 PFLOP/s (the library's best on a square of 8192: 1.38; power holds the clock); 256 x 128 tiles 1281 and 1670 us, the 128 x 128 x 32 tiles through
+// registers that stood here before 1827 and 2447.
+// The MFMAs are asm so that the accumulators are accumulation registers and nothing else (left to the register allocator, it spills fragments); they
+// and the fragment reads stay in the order written.
+template<class T>
+__device__ __forceinline__ void stream_mma32(floatx16& c, const u32x4& a, const u32x4& b)
+{
+    if constexpr (std::is_same<T, __bf16>::value) {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
+    else {
+        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    }
+}
+
+template<class T, class Epi>
+__global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Epi epi)
+{
+    constexpr int BM = 256, BN = 256, kXB = BM * 64, kStage = kXB + BN * 64;
+    constexpr int kXP = 4, kWP = 4, kPieces = 8;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const StreamTile t = stream_tile_of<BM, BN, 4>(a, epi.row_offsets(), epi.items());
+    if (t.item < 0) {
+        return;
+    }
+    const int  m0 = t.tm * BM, n0 = t.tn * BN;
+    const auto item = epi.item(t.item, a.M, n0);
+    const int  Mloc = min(item.M - m0, BM);
+    if (Mloc <= 0) {
+        return;
+    }
+    const auto rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + item.x_off + m0 * a.ldx), 0, (int)((Mloc - 1) * a.ldx + (int64_t)a.steps * 64), 0x00020000);
+    const int64_t w_left = (int64_t)(a.tiles - (n0 >> 4)) * a.w_tile + (a.w_quad > 4096 ? (int64_t)((a.steps - 1) >> 2) * a.w_quad : 0);
+    const auto rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + item.w_off + (int64_t)(n0 >> 4) * a.w_tile), 0, (int)min(w_left, (int64_t)0xffffffff), 0x00020000);
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
+    int            xoff[kXP], woff[kWP];
+#pragma unroll
+    for (int r = 0; r < kXP; ++r) {
+        const int row = 16 * (kXP * wave + r) + (lane >> 2);
+        xoff[r]       = (int)(min(row, Mloc - 1) * a.ldx) + ((lane & 3) ^ ((row >> 1) & 3)) * 16;
+        woff[r]       = (int)(min(kWP * wave + r, a.tiles - 1 - (n0 >> 4)) * a.w_tile) + lane * 16;
+    }
+    auto dma_piece = [&](int s, int buf, int n) {
+        const unsigned dst = lds0 + buf * kStage + (4 * wave + (n & 3)) * 1024;
+        if (n < 4) {
+            stream_dma16(rs_x, xoff[n], s * 64, dst);
+        }
+        else {
+            stream_dma16(rs_w, woff[n - 4], (int)((s >> 2) * a.w_quad) + (s & 3) * 1024, dst + kXB);
+        }
+    };
+    auto dma = [&](int s, int buf) {
+#pragma unroll
+        for (int n = 0; n < kPieces; ++n) {
+            dma_piece(s, buf, n);
+        }
+    };
+    floatx16 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc[i][j][r] = 0.f;
+            }
+        }
+    }
+    const int wm = wave >> 1, wn = wave & 1;
+    const int l31 = lane & 31, half = lane >> 5;
+    // x: row r at r * 64, piece (2 j + half) ^ ((r >> 1) & 3); j = 1 flips bit 1 of the piece
+    const int xf = (wm * 128 + l31) * 64 + ((half ^ ((l31 >> 1) & 3)) << 4);
+    const int wf = kXB + (wn * 8 + (l31 >> 4)) * 1024 + (half * 16 + (l31 & 15)) * 16;
+    // 16 k are a half step; the fragments of the next half step are read under the MFMAs of this one.  The barrier sits in the middle of a step: the
+    // second half's fragments are in registers there, so the step's own stage is free for the DMA of stage s + 3
+    u32x4     fx[2][4], fw[2][4];
+    const int steps = a.steps;
+    auto      read  = [&](int j, const char* st, int n) {
+        if (n < 4) {
+            fw[j][n] = *(const u32x4*)(st + wf + n * 2048 + j * 512);
+        }
+        else {
+            fx[j][n - 4] = *(const u32x4*)(st + (xf ^ (j * 32)) + (n - 4) * 2048);
+        }
+    };
+    dma(0, 0);
+    dma(min(1, steps - 1), 1);
+    dma(min(2, steps - 1), 2);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPieces) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+        read(0, smem, n);
+    }
+    int buf = 0;
+    for (int s = 0; s < steps; ++s) {
+        const int   nxt = buf == 2 ? 0 : buf + 1;
+        const char* st  = smem + buf * kStage;
+#pragma unroll
+        for (int n = 0; n < 16; ++n) {
+            if (n % 2 == 0) {
+                read(1, st, n >> 1);
+            }
+            stream_mma32<T>(acc[n >> 2][n & 3], fw[0][n & 3], fx[0][n >> 2]);
+        }
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPieces) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        st = smem + nxt * kStage;
+#pragma unroll
+        for (int n = 0; n < 16; ++n) {
+            if (n % 2 == 0) {
+                read(0, st, n >> 1);
+            }
+            else {
+                dma_piece(min(s + 3, steps - 1), buf, n >> 1);
+            }
+            stream_mma32<T>(acc[n >> 2][n & 3], fw[1][n & 3], fx[1][n >> 2]);
+        }
+        buf = nxt;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the DMA writes this workgroup's LDS)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {  // (the last results are sixteen passes behind their issue)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            asm volatile("s_nop 7" : "+a"(acc[i][c]));
+        }
+    }
+    // A lane's results are four columns each of 32 rows apart; through the wave's own 16 KB of LDS they leave as whole runs of a row (512 bytes of fp32): 32
+    // rows at a time, piece p (four columns) of row r at p ^ r
+    __builtin_amdgcn_s_barrier();  // every wave is through with the stages
+    asm volatile("" ::: "memory");
+    floatx4* const sw = (floatx4*)(smem + wave * 16384);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int n = 0; n < 16; ++n) {  // columns 32 c + 8 g + 4 half + 0 .. 3
+            const int c = n >> 2, g = n & 3;
+            sw[l31 * 32 + ((8 * c + 2 * g + half) ^ l31)] = floatx4{acc[i][c][4 * g], acc[i][c][4 * g + 1], acc[i][c][4 * g + 2], acc[i][c][4 * g + 3]};
+        }
+        __builtin_amdgcn_wave_barrier();
+        const int mb = m0 + wm * 128 + i * 32, nb = n0 + wn * 128;
+        if constexpr (Epi::kPairs) {  // gate and up are 16 columns (four pieces) apart: a lane has both
+#pragma unroll
+            for (int n = 0; n < 8; ++n) {
+                const int     r = n * 4 + (lane >> 4), p = ((lane & 15) >> 2) * 8 + (lane & 3);
+                const floatx4 v[2] = {sw[r * 32 + (p ^ r)], sw[r * 32 + ((p + 4) ^ r)]};
+                if (mb + r < item.M) {
+                    epi.template rows<2>(a, item, mb + r, nb + p * 4, v);
+                }
+            }
+        }
+        else {
+#pragma unroll
+            for (int n = 0; n < 16; ++n) {
+                const int     r = n * 2 + half;
+                const floatx4 v[1] = {sw[r * 32 + (l31 ^ r)]};
+                if (mb + r < item.M) {
+                    epi.template rows<1>(a, item, mb + r, nb + l31 * 4, v);
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// ---- which kernel, which shape -------------------------------------------------------------------------------------------------------
+// (row tiles, column tiles a wave, column waves, k-phases) of the skinny kernels that exist: 64 columns a workgroup of four waves, and 128 columns where
+// a wave needs a pair of column tiles.  Of 15 shapes (column groups of 64 and 128, one to four k-phases) these were the fastest or within 3 %
+// everywhere (K 768 ... 25600, N 256 ... 32000, 3 ... 64 rows); the number of slices of k matters more.
+#define TM_STREAM_SHAPES(X) X(1, 1, 4, 1) X(2, 1, 4, 1) X(4, 1, 4, 1)
+#define TM_STREAM_SHAPES_PAIRS(X) X(1, 2, 4, 2) X(2, 2, 4, 2) X(4, 2, 4, 1)
+
+struct StreamPlan {
+    bool skinny, narrow;  // narrow: few columns and nothing to meet in across workgroups
+    int  mt, splits, split_steps, row_blocks;  // skinny kernel
+    int  tile;                                 // 0: 256 x 256 (16-bit formats), 1: 256 x 128, 2: 128 x 128, 3: 64 x 64
+};
+// steps of k, image columns, rows, items (own_rows: each with rows of its own, `rows` in total), bytes of an element; pairs: a wave needs two
+// column tiles; ws_bytes / tickets: what slices of k may use (0: no slices)
+StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets);
+constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
+constexpr int    kStreamTickets = 4096;
+
+}  // namespace tmk

@@ -370,12 +370,21 @@ inline int dense_pair_rows(int n_out)  // rows of a paired image for n_out outpu
     return (n_out + 15) / 16 * 32;
 }
 constexpr int kDenseMaxSeg = 8;
+// What slices of k of few-row products meet in (gemm_stream.h): scratch and zeroed arrival counters, which every launch leaves at zero.  One
+// per stream of launches -- an engine's; without it a product runs unsliced
+struct StreamScratch {
+    float*    slabs   = nullptr;
+    size_t    bytes   = 0;
+    unsigned* tickets = nullptr;
+    int       count   = 0;
+};
 struct DenseWeight {
-    int    K = 0, N = 0, Kp = 0, Np = 0;  // Kp = K rounded up to 32, Np = N rounded up to 128: zero-padded image [Np][Kp]
+    int    K = 0, N = 0, Kp = 0, Np = 0;  // Kp = K rounded up to 32, Np = N rounded up to 128: zero-padded image of Np x Kp elements
     int    dtype = kDenseBf16;
     int    count = 1;                     // images of the same size behind each other (heads, experts)
     void*  w     = nullptr;
     size_t bytes = 0;
+    const StreamScratch* scratch = nullptr;  // set by an engine for its own weights
 };
 // one launch: the epilogue with its operands, and the items of a batched launch
 struct DenseCall {
@@ -400,6 +409,7 @@ struct DenseCall {
     int          x_col_stride = 0, y_col_stride = 0;
     const int*   row_offsets = nullptr; // ... and, when set, the rows [row_offsets[g], row_offsets[g + 1]) of x and y (device, [count + 1])
     size_t       w_stride = 0;          // (set by the launcher)
+    int          ldx = 0;               // (set by the launcher)
 };
 int  dense_weight_alloc(DenseWeight& d, int K, int N, int dtype, hipStream_t st, int count = 1);
 // rows x cols bf16 block (checkpoint orientation [out][in]) -> image rows [row0, row0 + rows), columns [col0, col0 + cols):

@@ -1,0 +1,95 @@
+"""GPU tests of the unquantised products (gemm_stream.h) where their kernels can go wrong: row counts around the tile heights, columns around
+the tile widths, one to three steps of k and odd counts of them, every kernel of the dispatch; slices of k that meet across workgroups; items whose
+row tiles are one list.  Bounds: a sum of K products in fp32 in any order is within K 2^-24 sum|x w| of the exact one, a bf16 result adds 2^-8 |y|."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from lmdeploy_amd import _ffi
+from tests import febivik_oracle as fo
+from tests import layered_oracle as lo
+from tests.gpu_helpers import release_all, st
+from tests.test_gpu_febivik import engine, model_folder
+from tests.test_gpu_febivik import rel_err as rel_err_febivik
+from tests.test_gpu_layered import _layer, engine_for, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _release():
+    yield
+    release_all()
+
+
+def check(got, ref, size, K, bf16):
+    bound = K * 2.0 ** -24 * size + (2.0 ** -8 if bf16 else 2.0 ** -22) * ref.abs() + 1e-30
+    assert bool(((got.double() - ref).abs() <= bound).all())
+
+
+@pytest.mark.parametrize('dtype', [0, 1])
+@pytest.mark.parametrize('K,N,rows', [
+    (32, 130, (1, 63, 64, 65, 127, 256, 257)),      # one step, a ragged last column tile
+    (96, 4100, (2, 16, 17, 129, 1500)),             # three steps; 256 x 128 tiles with a ragged edge on both sides
+    (1056, 2304, (3, 33, 300, 2100)),               # 33 steps, 256 x 256 tiles
+    (2080, 2048, (5, 48, 255)),
+    (200, 512, (70, 511, 513)),
+])
+def test_products_at_the_edges_of_tiles(tm, cuda, dtype, K, N, rows):
+    g = torch.Generator('cuda').manual_seed(K + N)
+    w = torch.randn(N, K, generator=g, device='cuda').bfloat16()
+    h = C.c_void_p()
+    _ffi.check(tm.tm_dense_create(C.byref(h), K, N, dtype, w.data_ptr(), st()))
+    T = torch.bfloat16 if dtype == 0 else torch.float32
+    ldx = (K + 31) // 32 * 32 + 32
+    for M in rows:
+        x = torch.full((M, ldx), 5.0, device='cuda', dtype=T)
+        x[:, :K] = torch.randn(M, K, generator=g, device='cuda').to(T)
+        ref, size = x[:, :K].double() @ w.double().t(), x[:, :K].double().abs() @ w.double().abs().t()
+        for ldy in (N, N + 5, (N + 7) // 8 * 8 + 8):      # rows that start on 16 bytes and rows that do not
+            y = torch.full((M + 1, ldy), -3.0, device='cuda', dtype=T)
+            _ffi.check(tm.tm_dense_forward(h, x.data_ptr(), ldx, y.data_ptr(), ldy, M, 0, 1.0, st()))
+            check(y[:M, :N], ref, size, K, dtype == 0)
+            assert bool((y[M] == -3.0).all()) and bool((y[:M, N:] == -3.0).all())      # nothing is written beyond
+        y = torch.randn(M, N, generator=g, device='cuda')
+        old = y.double()
+        _ffi.check(tm.tm_dense_forward(h, x.data_ptr(), ldx, y.data_ptr(), N, M, 2, 0.25, st()))
+        check(y, old + 0.25 * ref, 0.25 * size + old.abs(), K, False)
+    _ffi.check(tm.tm_dense_destroy(h))
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('rows', [3, 20, 40, 64])
+def test_slices_of_k_meet_in_any_order(cuda, dtype, rows):
+    """decode steps of an engine, whose products may be cut along k: widths and feed-forwards of 33 and 130 (bf16) and 66 and 260 (fp32) steps,
+    one, two and four row tiles; the same step again gives the same bits (slices are added in their own order)"""
+    cfg = lo.make_config(1056, 203, [_layer(heads=8, kv_heads=2, dim=32, vdim=32, ff=4160), _layer(heads=8, kv_heads=2, dim=32, vdim=32, ff=2080)], mult=0.4)
+    w = lo.make_weights(cfg, 5)
+    eng = engine_for(cfg, w, dtype, max_batch_size=64, cache_blocks=70)
+    rng = np.random.default_rng(rows)
+    toks = rng.integers(0, cfg['vocab'], (rows, 3))
+    outs = []
+    for _ in range(3):
+        s = [eng.open_session() for _ in range(rows)]
+        outs.append([eng.step_tokens([(s[i], [int(toks[i, k])], [0]) for i in range(rows)]) for k in range(3)])
+        for i in s:
+            eng.close_session(i)
+    assert all(np.array_equal(a, b) for o in outs[1:] for a, b in zip(o, outs[0]))
+    got = np.stack(outs[0], 1)
+    for i in range(0, rows, 7):
+        assert rel_err(got[i], lo.forward(cfg, w, toks[i].tolist())[0]) <= (3e-5 if dtype == 'float32' else 4e-2)
+    eng.close()
+
+
+def test_row_tiles_of_many_items(cuda, tmp_path):
+    """prompts through 70 experts (more items than a wave has lanes), most of them with a few rows, some with none"""
+    cfg = fo.make_config(64, 97, [fo.attention_layer(2, 1, 8, 8, 0.3, 16, 1, 4, mlp=fo.moe(70, 2, 24, 1.5, 8))])
+    toks = np.random.default_rng(1).integers(0, 97, 300).tolist()
+    folder, w = model_folder(tmp_path, cfg, 3)
+    eng = engine(folder, 'float32')
+    s = eng.open_session()
+    got = eng.step_tokens([(s, toks, list(range(300)))])
+    assert rel_err_febivik(got, fo.forward(cfg, w, toks)) <= 3e-5
+    eng.close()
