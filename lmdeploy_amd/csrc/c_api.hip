@@ -297,10 +297,12 @@ int tm_linear_forward(const tm_linear* w, const void* x, int ldx, void* y, int l
         cfg.nt = nt;
     }
     if (splits > 0) {
-        cfg.splits = splits;
+        cfg.splits     = splits;
+        cfg.f16_stream = false;  // (its slices are its own)
     }
     if (nt > 0 || (waves > 0 && !(waves & 0x200))) {
-        cfg.d32_shape = -1;  // an explicit tiling of the general kernel
+        cfg.d32_shape  = -1;  // an explicit tiling of the general kernel
+        cfg.f16_stream = false;
         if (splits <= 0) {
             cfg.splits = gemm_pick_config_general(w->w, M).splits;
         }
@@ -354,7 +356,8 @@ int tm_linear_residual_norm(const tm_linear* w, const void* x, int ldx, void* y,
         cfg.d32_shape = shape;
     }
     if (splits > 0) {
-        cfg.splits = splits;
+        cfg.splits     = splits;
+        cfg.f16_stream = false;  // (its slices are its own)
     }
     TM_REQUIRE(cfg.splits <= 16, "splits <= 16");
     // slabs (or, with one slice, the fp16 product parked at the end of the workspace) + the reduce-norm kernel

@@ -479,6 +479,7 @@ int tm_engine_start(tm_engine* e)
         // tiles (every weight unit read by four row blocks), the 128-row tile with 10 slices + the fused reduce-norm wins w2 by 4 us
         e->fold_max_rows = fm ? std::min(kFoldMaxRows, std::max(1, atoi(fm))) : 64;
         TM_TRY(dmalloc(&e->d_tickets, ntk));
+        e->n_tickets = (int)ntk;
         TM_HIP_CHECK(hipMemset(e->d_tickets, 0, ntk * sizeof(unsigned)));
         // Default 0 since round 6: the folded layer is a departure from the reference's rounding sequence (one fp16 rounding
         // of the normalised activations instead of two) and a default-on departure has to pay more than box noise -- four interleaved runs per arm

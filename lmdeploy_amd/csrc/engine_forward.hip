@@ -142,7 +142,8 @@ static int linear_plain(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, 
     if (gemm_workspace_bytes(M, l.w.N, cfg.splits) > e->gemm_ws_bytes) {
         cfg.splits = 1;
     }
-    cfg.tickets = e->d_tickets;
+    cfg.tickets      = e->d_tickets;
+    cfg.ticket_count = e->n_tickets;
     return launch_linear(l.w, x, ldx, y, ldy, M, gated, cfg, e->d_gemm_ws, false, nullptr, e->stream);
 }
 

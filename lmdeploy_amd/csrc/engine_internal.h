@@ -279,6 +279,7 @@ struct tm_engine {
     // RMSNorm folded into the decode GEMMs (NormFold, tm_kernels.h): per-tile sums of squares [hidden / 64][64] and the split-K
     // arrival counters of the producing GEMM; TM_FOLD_NORM=0 keeps the reduce-norm launches
     float*    d_ss      = nullptr;
+    int       n_tickets = 0;
     unsigned* d_tickets = nullptr;
     int       fold_max_rows = 64;  // rows of a forward up to which the folded layer runs (TM_FOLD_MAX_M: 64 | 128)
     int       fold_norm = 0;  // bit 0: wo -> w1w3, bit 1: w2 -> the next layer's w_qkv

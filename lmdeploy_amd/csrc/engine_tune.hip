@@ -332,8 +332,10 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
         if (nc == 0) {
             continue;
         }
-        const GemmConfig heur = gemm_pick_config_general(w0, M);
-        auto same = [](const GemmConfig& a, const GemmConfig& b) { return a.nt == b.nt && a.splits == b.splits; };
+        GemmConfig heur = gemm_pick_config(w0, M);
+        heur.tickets      = e->d_tickets;
+        heur.ticket_count = e->n_tickets;
+        auto same = [](const GemmConfig& a, const GemmConfig& b) { return a.nt == b.nt && a.splits == b.splits && a.f16_stream == b.f16_stream; };
         bool has = false;
         for (int i = 0; i < nc; ++i) {
             has = has || same(cand[i], heur);
@@ -384,7 +386,8 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
         if (!(best < 0.93f * t_heur)) {
             bc = heur;
         }
-        const int v[4] = {bc.nt, bc.splits, bc.waves, bc.kphases < 1 ? 1 : bc.kphases};
+        // (fp16: gemm_kernel has one k-phase; an entry with two says that the dispatch's own kernels, gemm_f16.hip, were the fastest)
+        const int v[4] = {bc.nt, bc.f16_stream ? 1 : bc.splits, bc.waves, bc.f16_stream ? 2 : w0.type == 1 || bc.kphases < 1 ? 1 : bc.kphases};
         gen_table_set(kGenDense + w0.type, w0.role, w0.K, w0.N, Mb, v);
         if (verbose) {
             fprintf(stderr, "[tm tune] %-7s K=%d N=%d M=%d -> general nt %d splits %d (%.2f us; heuristic %.2f us)\n", r.name, w0.K, w0.N, M, bc.nt,

@@ -350,7 +350,7 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     if (best.narrow) {
         sp = 1;
     }
-    if (sp > 1 && ((size_t)groups * sp * mt * 16 * wg_cols * 4 > ws_bytes || groups > tickets)) {
+    if (sp > 1 && ((size_t)items * sp * rows * cols * 4 > ws_bytes || groups > tickets)) {
         sp = 1, best.narrow = true;
     }
     const int    ss = ((steps + sp - 1) / sp + 7) / 8 * 8;

@@ -1,0 +1,149 @@
+// fp16 linears of the Llama family (w_qkv / wo / w1w3 / w2 of an unquantised checkpoint, lm_head) on the kernels of gemm_stream.h: the weight stream for
+// decode-sized forwards, tiles by DMA for prompts.
+//
+// Replaces: LlamaLinear::Forward -> gemm::Gemm::Run for fp16 weights (src/turbomind/models/llama/LlamaLinear.cu:140-216), the gated-SiLU epilogue
+// (kernels/gemm/epilogue.h:159-176,428-446).  Same arithmetic as gemm_kernel<WT = 1> (gemm_w4a16.hip): fp32 accumulation, one rounding of the result;
+// the image is the one linear_weight_prepare_f16 makes ([k / 128][n / 16][4] blocks of one KB).
+//
+// Weights from HBM, MI355X, here | gemm_kernel: 8 rows (2048, 4096) 7.2 | 13.0 us, (8192, 2048) 14.1 | 43.7, (2048, 16384) gated 15.7 | 17.2; 64 rows (14336,
+// 4096) 33 | 101; 2664 rows (2048, 16384) gated 215 | 501; 8192 rows (4096, 28672) gated 1702 | 5390 us (1.13 PFLOP/s), (14336, 4096) 810 | 2159 (1.19).
+#include "gemm_stream.h"
+#include "tm_kernels.h"
+#include <algorithm>
+
+namespace tmk {
+
+struct F16Item {
+    int64_t x_off, w_off;
+    int     M;
+};
+
+struct F16Epi {
+    int gated;  // columns alternate (gate_j, up_j): out[m][j] = silu(acc[m][2 j]) * acc[m][2 j + 1]
+    int vec;    // rows of y start on 8 bytes
+
+    static constexpr bool kPairs = false;
+    __device__ __forceinline__ const int* row_offsets() const
+    {
+        return nullptr;
+    }
+    __device__ __forceinline__ int items() const
+    {
+        return 1;
+    }
+    __device__ __forceinline__ F16Item item(int, int M, int) const
+    {
+        return {0, 0, M};
+    }
+    template<int NT>
+    __device__ __forceinline__ void rows(const StreamArgs& a, const F16Item&, int m, int n, const floatx4 (&acc)[NT]) const
+    {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int c = n + 16 * j;
+            if (c >= a.N) {  // (N is a multiple of 16)
+                continue;
+            }
+            const floatx4 v = acc[j];
+            if (gated) {
+                const float s0 = v[0] / (1.0f + __builtin_expf(-v[0]));
+                const float s1 = v[2] / (1.0f + __builtin_expf(-v[2]));
+                half_t*     y  = (half_t*)a.y + (size_t)m * a.ldy + (c >> 1);
+                if (vec) {
+                    *(half2_t*)y = half2_t{(half_t)(s0 * v[1]), (half_t)(s1 * v[3])};
+                }
+                else {
+                    y[0] = (half_t)(s0 * v[1]), y[1] = (half_t)(s1 * v[3]);
+                }
+            }
+            else {
+                half_t* y = (half_t*)a.y + (size_t)m * a.ldy + c;
+                if (vec) {
+                    *(half4_t*)y = half4_t{(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
+                }
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        y[e] = (half_t)v[e];
+                    }
+                }
+            }
+        }
+    }
+};
+
+// 17 ... 64 rows of a wide output stay on gemm_kernel, whose 128-column workgroups read x half as often where all of them are busy anyway: (K, N) =
+// (4096, 28672) 64 rows 44 us against 53, 32 rows 40 against 42; (4096, 128256) 64 rows 191 against 216, 16 rows 169 against 165; (4096, 14336) 64
+// rows 37 against 32; (14336, 4096) 64 rows 101 against 33.  (Workgroups of 128 columns in the stream kernel: 52, 42, 215, 166, 43, 44 us.)
+bool f16_stream_supported(const LinearWeight& w, int M)
+{
+    return w.type == 1 && w.packed && (size_t)w.K * w.N * 2 < ((size_t)1 << 31)  // (byte offsets inside the image are 32 bits)
+           && !(M > 16 && M <= 64 && w.N >= 24576);
+}
+
+int f16_stream_splits(const LinearWeight& w, int M)
+{
+    const StreamPlan p = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, ~(size_t)0, 1 << 30);
+    return p.skinny ? p.splits : 1;
+}
+
+template<int MT>
+static int launch_skinny(const StreamArgs& a, const F16Epi& epi, int splits, bool narrow, hipStream_t st)
+{
+    if (narrow) {
+        constexpr int W = MT <= 2 ? 16 : 8;
+        stream_narrow_kernel<half_t, F16Epi, MT, 1, W><<<dim3(a.tiles, a.row_blocks), W * 64, 0, st>>>(a, epi);
+    }
+    else {
+        stream_skinny_kernel<half_t, F16Epi, MT, 1, 4, 1><<<dim3((a.tiles + 3) / 4, a.row_blocks, splits), 256, 0, st>>>(a, epi);
+    }
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+template<class K>
+static int launch_tiles(K kernel, const StreamArgs& a, const F16Epi& epi, int bm, int bn, hipStream_t st)
+{
+    const int lds = 3 * (bm + bn) * 64;
+    if (const int rc = ensure_dynamic_lds((const void*)kernel, lds)) {
+        return rc;
+    }
+    kernel<<<dim3((unsigned)((a.M + bm - 1) / bm) * (unsigned)((a.tiles * 16 + bn - 1) / bn)), 256, lds, st>>>(a, epi);
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// splits: slices of k the caller's workspace holds slabs for (1: none).  With slices, fp32 slabs [slices][M][N] are left in the workspace and *slabs says
+// how many (defer, or no arrival counters), or they meet inside the launch (tickets)
+int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int splits, float* workspace,
+                      unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st)
+{
+    TM_REQUIRE(f16_stream_supported(w, M), "fp16 linear: image");
+    const bool       slice = splits > 1 && workspace;
+    const StreamPlan p     = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, slice ? ~(size_t)0 : 0, slice ? 1 << 30 : 0);
+    StreamArgs       a{};
+    a.x = (const char*)x, a.ldx = (int64_t)ldx * 2;
+    a.w = (const char*)w.packed, a.tiles = w.N / 16, a.steps = w.K / 32;
+    a.w_tile = 4096, a.w_quad = (int64_t)a.tiles * 4096;
+    a.y = y, a.ldy = ldy, a.M = M, a.N = w.N;
+    const F16Epi epi{gated ? 1 : 0, gated ? (ldy % 2 == 0 && (uintptr_t)y % 4 == 0) : (ldy % 4 == 0 && (uintptr_t)y % 8 == 0)};
+    *slabs = 1;
+    if (p.skinny) {
+        TM_REQUIRE(p.splits <= std::max(1, splits), "fp16 linear: slices of k");
+        a.split_steps = p.split_steps;
+        a.row_blocks  = p.row_blocks;
+        if (p.splits > 1) {
+            a.slabs   = workspace;
+            a.tickets = defer || (a.tiles + 3) / 4 * p.row_blocks > ticket_count ? nullptr : tickets;
+            *slabs    = a.tickets ? 1 : p.splits;
+        }
+        return p.mt == 1 ? launch_skinny<1>(a, epi, p.splits, p.narrow, st) : p.mt == 2 ? launch_skinny<2>(a, epi, p.splits, p.narrow, st) :
+                                                                                        launch_skinny<4>(a, epi, p.splits, p.narrow, st);
+    }
+    return p.tile == 0 ? launch_tiles(stream_tile256_kernel<half_t, F16Epi>, a, epi, 256, 256, st) :
+           p.tile == 1 ? launch_tiles(stream_tile_kernel<half_t, F16Epi, 256, 128, 2, 2>, a, epi, 256, 128, st) :
+           p.tile == 2 ? launch_tiles(stream_tile_kernel<half_t, F16Epi, 128, 128, 2, 2>, a, epi, 128, 128, st) :
+                         launch_tiles(stream_tile_kernel<half_t, F16Epi, 64, 64, 2, 2>, a, epi, 64, 64, st);
+}
+
+}  // namespace tmk

@@ -58,8 +58,8 @@ struct StreamArgs {
     int         row_blocks;   // skinny kernel: blocks of 16 MT rows (grid y = item * row_blocks + block)
     void*       y;
     int         ldy, M, N;
-    float*      slabs;        // skinny kernel, several slices: their partial sums, [item][column group][slice][16 rows x ...]
-    unsigned*   tickets;      // ... and an arrival counter per (item, column group), zero between launches
+    float*      slabs;        // skinny kernel, several slices: their partial sums, [item][slice][M][16 tiles]
+    unsigned*   tickets;      // ... and an arrival counter per (column group, row block, item), zero between launches (nullptr: the slabs are the result)
 };
 
 // ---- few rows: the weight stream ---------------------------------------------------------------------------------------------------
@@ -212,36 +212,41 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
         }
     }
     if (gridDim.z > 1) {
-        // 16-byte pieces in accumulator order, written through to memory (sc1) and drained before the counter moves; the last workgroup reads
-        // them past its L1 (sc1)
-        constexpr int64_t kTileFloats = (int64_t)CW * MT * NT * 256;
-        const int         group = blockIdx.y * gridDim.x + blockIdx.x;
-        float*            mine  = a.slabs + ((int64_t)group * gridDim.z) * kTileFloats;
-        const auto        rs    = __builtin_amdgcn_make_buffer_rsrc((void*)mine, 0, (int)(gridDim.z * kTileFloats * 4), 0x00020000);
+        // slabs [item][slice][row][column] of all the columns the image holds.  Without counters they are the result; else they are written through to
+        // memory (sc1) and drained before the counter moves, and the last workgroup reads them past its L1 (sc1)
+        const int     ld   = a.tiles * 16, n = tile0 * 16 + fc * 4;
+        const int64_t rows = (int64_t)a.M * ld * 4;  // bytes of one slice
+        const auto    rs   = __builtin_amdgcn_make_buffer_rsrc((void*)((char*)a.slabs + blockIdx.y / a.row_blocks * gridDim.z * rows), 0, (int)(gridDim.z * rows), 0x00020000);
         if (ph == 0) {
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                if (t * 16 < M) {
+                if (t * 16 + fr < M) {
 #pragma unroll
                     for (int j = 0; j < NT; ++j) {
-                        const int at = ((cw * MT + t) * NT + j) * 1024 + lane * 16;
-                        __builtin_amdgcn_raw_buffer_store_b128(bit_cast<u32x4>(acc[t][j]), rs, at, (int)(blockIdx.z * kTileFloats * 4), /*sc1*/ 16);
+                        const int at = ((mb + t * 16 + fr) * ld + n + 16 * j) * 4;
+                        if (n + 16 * j < ld) {
+                            __builtin_amdgcn_raw_buffer_store_b128(bit_cast<u32x4>(acc[t][j]), rs, at, (int)(blockIdx.z * rows), /*sc1*/ 16);
+                        }
                     }
                 }
             }
         }
+        if (!a.tickets) {
+            return;
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         unsigned* last = (unsigned*)smem;  // (every reader of the x buffers and of `red` has passed a barrier)
+        unsigned* mine = a.tickets + blockIdx.y * gridDim.x + blockIdx.x;
         if (tid == 0) {
-            *last = __hip_atomic_fetch_add(a.tickets + group, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            *last = __hip_atomic_fetch_add(mine, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
         if (*last != gridDim.z - 1) {
             return;
         }
         if (tid == 0) {
-            __hip_atomic_store(a.tickets + group, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         if (ph > 0) {
             return;
@@ -251,11 +256,11 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
             if (t * 16 < M) {
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
-                    const int at = ((cw * MT + t) * NT + j) * 1024 + lane * 16;
+                    const int at = ((mb + min(t * 16 + fr, M - 1)) * ld + min(n + 16 * j, ld - 4)) * 4;
                     acc[t][j]    = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
                     for (int z = 0; z < (int)gridDim.z; ++z) {
-                        acc[t][j] += bit_cast<floatx4>(__builtin_amdgcn_raw_buffer_load_b128(rs, at, (int)(z * kTileFloats * 4), /*sc1*/ 16));
+                        acc[t][j] += bit_cast<floatx4>(__builtin_amdgcn_raw_buffer_load_b128(rs, at, (int)(z * rows), /*sc1*/ 16));
                     }
                 }
             }

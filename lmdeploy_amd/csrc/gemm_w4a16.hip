@@ -944,7 +944,14 @@ GemmConfig gemm_pick_config(const LinearWeight& w, int M)
         cfg.kphases = 1;
         return cfg;
     }
-    return gemm_pick_config_general(w, M);
+    GemmConfig cfg = gemm_pick_config_general(w, M);
+    int        tv[4];
+    static const bool forced = getenv("TM_GEMM_NT") || getenv("TM_GEMM_SPLITS") || getenv("TM_GEMM_WAVES") || getenv("TM_GEMM_KPHASES");
+    if (f16_stream_supported(w, M) && !forced && (!gen_table_get(kGenDense + w.type, w.role, w.K, w.N, dec32_m_bucket(M), tv) || tv[3] == 2)) {
+        cfg.f16_stream = true;
+        cfg.splits     = f16_stream_splits(w, M);
+    }
+    return cfg;
 }
 
 GemmConfig gemm_pick_config_general(const LinearWeight& w, int M)
@@ -1183,6 +1190,22 @@ int launch_linear(const LinearWeight& w,
         return 0;
     }
     TM_REQUIRE(w.packed != nullptr, "this linear holds only the decode kernels' image (prepared p32_only)");
+    if (cfg.f16_stream) {
+        int n = 1;
+        if (const int rc = launch_f16_stream(w, x, ldx, y, ldy, M, gated_silu, cfg.splits, workspace, cfg.tickets, cfg.ticket_count, defer_reduce, &n, st)) {
+            return rc;
+        }
+        if (n > 1 && !defer_reduce) {
+            if (const int rc = launch_splitk_reduce(y, ldy, workspace, n, M, w.N, gated_silu, st)) {
+                return rc;
+            }
+            n = 1;
+        }
+        if (slabs) {
+            *slabs = n;
+        }
+        return 0;
+    }
     int nt    = cfg.nt;
     int waves = cfg.waves == 16 ? 16 : (cfg.waves == 8 ? 8 : 4);
     int wk    = cfg.kphases == 2 || waves == 16 ? 2 : 1;

@@ -134,7 +134,9 @@ struct GemmConfig {
     int kphases; // split-K inside the workgroup: 1 or 2 (8 waves only)
     int kstage;  // max k-blocks per barrier (0 = auto: 4)
     int d32_shape = -1;  // >= 0: a P32 kernel (gemm_decode.hip / gemm_decode_lc.hip / gemm_prefill.hip) with this workgroup shape
-    unsigned* tickets = nullptr;  // arrival counters (zero between launches) of the kShapeMerge shapes: >= ceil(N / 64) * ceil(M / 32) words
+    unsigned* tickets = nullptr;  // arrival counters (zero between launches) of the kShapeMerge shapes and of f16_stream: >= ceil(N / 64) * ceil(M / 32) words
+    int       ticket_count = 0;   // (f16_stream: how many there are)
+    bool      f16_stream = false; // the kernels of gemm_f16.hip
 };
 // (shape 10 was "dequantise + the vendor library's fp16 GEMM" in round 3: removed -- no vendor GEMM on any path of this library)
 constexpr int kShapePre256     = 12;   // gemm_prefill.hip: 256 x 256 tiles, weights dequantised once per workgroup tile through LDS (M > 64)
@@ -173,6 +175,12 @@ GemmConfig gemm_pick_config_general(const LinearWeight& w, int M);  // ... the t
 // `defer_reduce`, a reduce kernel writes y.
 int launch_linear(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated_silu,
                   GemmConfig cfg, float* workspace, bool defer_reduce, int* slabs, hipStream_t st);
+
+// ---- gemm_f16.hip: fp16 linears on the kernels of gemm_stream.h ---------------------------------------------------
+bool f16_stream_supported(const LinearWeight& w, int M);
+int  f16_stream_splits(const LinearWeight& w, int M);
+int  launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int splits, float* workspace,
+                       unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st);
 
 // ---- gemm_decode.hip: W4A16 decode GEMM (M <= 64), 32x32x16 MFMA, 16 waves per CU ------------------------------
 size_t p32_bytes(int K, int N);

@@ -93,3 +93,37 @@ def test_row_tiles_of_many_items(cuda, tmp_path):
     got = eng.step_tokens([(s, toks, list(range(300)))])
     assert rel_err_febivik(got, fo.forward(cfg, w, toks)) <= 3e-5
     eng.close()
+
+
+@pytest.mark.parametrize('K,N,gated,rows', [
+    (128, 16, 0, (1, 17, 65, 300)),                   # one column tile
+    (256, 4128, 1, (1, 16, 33, 64, 129)),             # a ragged last column group, gated
+    (2048, 2080, 0, (8, 16, 31, 64, 200, 257, 1100)),  # slices of k that meet in a reduce launch; tiles of every height
+    (4096, 544, 0, (3, 20, 64)),
+    (1024, 24576, 1, (16, 17, 64)),                   # both sides of the line to the general kernel
+    (512, 9216, 1, (513, 2111)),
+])
+def test_f16_linears_at_the_edges(tm, cuda, K, N, gated, rows):
+    g = torch.Generator('cuda').manual_seed(K + N)
+    w = (torch.randn(K, N, generator=g, device='cuda') / K ** 0.5).half()
+    h = C.c_void_p()
+    _ffi.check(tm.tm_linear_create(C.byref(h), K, N, 1, 128))
+    _ffi.check(tm.tm_linear_prepare(h, w.data_ptr(), None, None, st()))
+    No = N // 2 if gated else N
+    for M in rows:
+        ldx = K + 8
+        x = torch.randn(M, ldx, generator=g, device='cuda').half()
+        ref, size = x[:, :K].double() @ w.double(), x[:, :K].double().abs() @ w.double().abs()
+        err = K * 2.0 ** -24 * size
+        if gated:       # d silu <= 1.1 d; the product of two values with errors; exp and division within a few fp32 ulps
+            s, u = torch.nn.functional.silu(ref[:, 0::2]), ref[:, 1::2]
+            err = 1.1 * err[:, 0::2] * (u.abs() + err[:, 1::2]) + s.abs() * err[:, 1::2] + 2.0 ** -20 * (s * u).abs()
+            ref = s * u
+        bound = err + 2.0 ** -11 * (ref.abs() + err) + 2.0 ** -24      # one rounding to fp16, subnormal results included
+        ws = torch.zeros(tm.tm_linear_workspace(h, M) // 4 + 4, device='cuda')
+        for work, ldy in ((ws.data_ptr(), No), (None, No + 3), (ws.data_ptr(), No + 8)):
+            y = torch.full((M + 1, ldy), -3.0, device='cuda', dtype=torch.half)
+            _ffi.check(tm.tm_linear_forward(h, x.data_ptr(), ldx, y.data_ptr(), ldy, M, gated, 0, 0, 0, work, st()))
+            assert bool(((y[:M, :No].double() - ref).abs() <= bound).all()), (M, ldy)
+            assert bool((y[M] == -3.0).all()) and bool((y[:M, No:] == -3.0).all())
+    _ffi.check(tm.tm_linear_destroy(h))
