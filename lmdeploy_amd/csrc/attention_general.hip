@@ -23,10 +23,12 @@
 //   * tile kernel: bf16 prefill on the matrix cores -- 64 query rows of one sequence x one query head per workgroup, four waves of 16
 //                  rows; S^T = K Q^T and O^T += V^T P^T as v_mfma_f32_16x16x32_bf16 with every operand a 16-byte load straight from the
 //                  cache (keys [token][channel], values stored transposed [channel][token]); online soft-max in fp32; no LDS, no barrier.
+//   * staged kernel: the tile kernel's products over cache blocks that a workgroup brings into LDS once (head sizes of 64 ... 256).
 //   * decode kernel: the same products with the query HEADS of one key head as the 16 rows (one row per sequence): a workgroup per
 //                  (sequence, key head, key split), its four waves take every fourth cache block and merge at the end.
 // Cache block layout per layer: keys [kv_heads][64][dim], then values [kv_heads][vdim][64].
 #include "tm_kernels.h"
+#include "gemm_stream.h"  // stream_dma16
 #include <stdlib.h>
 
 #define TM_TRY_RC(expr)      \
@@ -38,8 +40,6 @@
     } while (0)
 
 namespace tmk {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ float ga_wave_max(float v)
 {
@@ -746,6 +746,302 @@ bool general_attention_tiles_ok(const GeneralAttnParams& p)
            && p.cu_q && p.k_len && p.nseq >= 1 && p.max_q_len >= 1 && p.splits == 1 && p.q_heads % p.kv_heads == 0;
 }
 
+// ---- prefill over staged blocks -------------------------------------------------------------------------------------------------------
+// Workgroup = W waves of RT tiles of 16 query rows of one sequence x one query head.  A cache block's keys and values are brought into LDS once per
+// workgroup by DMA (no registers), double buffered, one barrier per block; the fragments come from there.  What bounds the kernel is the soft-max
+// arithmetic (per score three transcendentals with a cap, one without, at quarter rate) beside about as many cycles of MFMA, so what matters is that two waves
+// share a SIMD and run out of phase: under 256 registers a wave, 64 KB of LDS for 128 / 128 heads (two workgroups of four waves), one workgroup of eight
+// waves for key size 256, one row tile a wave there (two spill: 640 us where one takes 271).
+// MI355X, 4 x 2048 rows: 32 / 8 heads of 128 / 128 273 us = 0.50 PFLOP/s (8000 rows: 0.72; attn_tiles_kernel, which reads fragments straight from the
+// cache with one wave a SIMD: 1126 us), 16 / 1 heads of 256 / 192 271 us (1055), 16 / 8 heads of 64 / 128 with a cap 139 us (465), 40 x 100 rows of 32 / 8
+// heads of 128 / 128 61 us (136).
+// Serves the sizes of staged_shape(); attn_tiles_kernel serves the rest (sizes that do not fill the pieces of a DMA or the 16-channel tiles).
+typedef unsigned ga_u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float ga_max_groups(float v)  // over the four lane groups (lanes l ^ 16, l ^ 32)
+{
+    unsigned       b = bit_cast<unsigned>(v);
+    const ga_u32x2 r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+    b                = bit_cast<unsigned>(fmaxf(bit_cast<float>((unsigned)r[0]), bit_cast<float>((unsigned)r[1])));
+    const ga_u32x2 q = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return fmaxf(bit_cast<float>((unsigned)q[0]), bit_cast<float>((unsigned)q[1]));
+}
+
+// 16-byte piece of a key row (2 D bytes) that holds channels 8 c .. 8 c + 7: fragment reads are served in groups of 16 lanes (eight rows each of two
+// neighbouring pieces), whose pieces fall on 16 different slots of 256 bytes
+template<int DS>
+__device__ __forceinline__ int ga_key_swizzle(int row)
+{
+    return DS == 2 ? (row & 2) | ((row & 8) >> 1) : (row & 8) | ((row & 3) << 1);
+}
+
+template<int DS, int VT, int RT, bool MASK>
+__device__ __forceinline__ void ga_staged_step(const bf16x8 (&qf)[RT][DS], const char* __restrict__ kt_lds, const char* __restrict__ vt_lds, const int (&limit)[RT],
+                                               const int (&lower)[RT], int keep_rel, const float (&qscale)[RT], float cap, float inv_cap, bool bias, float r1,
+                                               float r2, float (&m)[RT], float (&l)[RT], floatx4 (&o)[RT][VT], const float* __restrict__ tab, int tab_len)
+{
+    const int lane = threadIdx.x & 63, lr = lane & 15, lg = lane >> 4;
+    floatx4   sc[RT][4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            sc[rt][kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        const int   row = (kt >> 1) * 32 + (lr >> 2) * 8 + (kt & 1) * 4 + (lr & 3);
+        const char* kr  = kt_lds + row * (DS * 64);
+        const int   sw  = ga_key_swizzle<DS>(row);
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) {
+            const bf16x8 kf = *(const bf16x8*)(kr + (((ds * 4 + lg) ^ sw) << 4));
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                sc[rt][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][ds], sc[rt][kt], 0, 0, 0);
+            }
+        }
+    }
+    bf16x8      pf[RT][2];
+    const float cap2 = cap * kLog2e;
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const float k1 = cap > 0.f ? qscale[rt] * inv_cap * (2.f * kLog2e) : qscale[rt] * kLog2e;
+        // (one loop per modifier, the branch outside: a branch per score would leave every score in a block of its own)
+        auto each = [&](auto f) {
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    sc[rt][kt][r] = f(sc[rt][kt][r], (kt >> 1) * 32 + lg * 8 + (kt & 1) * 4 + r);
+                }
+            }
+        };
+        if (cap > 0.f) {
+            each([&](float v, int) { return fmaf(__builtin_amdgcn_rcpf(fast_exp2(v * k1) + 1.f), -2.f * cap2, cap2); });
+        }
+        else {
+            each([&](float v, int) { return v * k1; });
+        }
+        if (bias) {  // (a key ahead of the row gives the logarithm of a number that may be negative: the mask below discards it)
+            each([&](float v, int key) { return fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, (float)(limit[rt] - key), 1.f)), v); });
+        }
+        if (tab) {  // (a key ahead of the row reads entry 0 and is masked below)
+            each([&](float v, int key) { return fmaf(tab[min(max(limit[rt] - key, 0), tab_len - 1)], kLog2e, v); });
+        }
+        if (MASK) {
+            each([&](float v, int key) { return (key <= limit[rt] && (key >= lower[rt] || key < keep_rel)) ? v : -1e30f; });
+        }
+        float bmax = -1e30f;
+        each([&](float v, int) {
+            bmax = fmaxf(bmax, v);
+            return v;
+        });
+        const float m_new = fmaxf(m[rt], ga_max_groups(bmax));
+        const float m_ref = fmaxf(m_new, -1e29f);  // a row that has seen no key yet (its chunk starts behind this block): every weight is 0
+        float       sum   = 0.f;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float e = fast_exp2(sc[rt][kt][r] - m_ref);  // a masked score is -1e30: 2^(-1e30 - m) = 0
+                sum += e;
+                pf[rt][kt >> 1][(kt & 1) * 4 + r] = (__bf16)e;
+            }
+        }
+        if (__any(m_new != m[rt])) {  // (after the first blocks a row's maximum rarely moves)
+            const float alpha = fast_exp2(m[rt] - m_new);
+            l[rt] *= alpha;
+#pragma unroll
+            for (int t = 0; t < VT; ++t) {
+                o[rt][t] *= alpha;
+            }
+        }
+        l[rt] += sum;  // the lane's own sixteen keys: the lane groups meet at the end
+        m[rt] = m_new;
+    }
+    const char* vr = vt_lds + lr * 128;
+#pragma unroll
+    for (int t = 0; t < VT; ++t) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const bf16x8 vf = *(const bf16x8*)(vr + t * 2048 + (((ks * 4 + lg) ^ (lr & 7)) << 4));
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                o[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf[rt][ks], o[rt][t], 0, 0, 0);
+            }
+        }
+    }
+}
+
+template<int DS, int VT, int RT, int W>
+__global__ __launch_bounds__(W * 64, 2) void attn_staged_kernel(GeneralAttnParams p, int tiles_per_seq)
+{
+    constexpr int kKeyBytes = 64 * DS * 64, kBytes = kKeyBytes + VT * 16 * 128, kPieces = DS * 4 + VT * 2;  // of one block; DMA pieces of 1 KB
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // workgroup i runs on XCD i % 8: consecutive heads (they share a key head) on one XCD; the longest rows of a sequence first
+    int       i = blockIdx.x, h;
+    const int H = p.q_heads;
+    if (H % 8 == 0) {
+        h = (i % 8) * (H / 8) + (i / 8) % (H / 8);
+    }
+    else {
+        h = i % H;
+    }
+    i /= H;
+    const int s = i % p.nseq, ti = tiles_per_seq - 1 - i / p.nseq;
+    const int row_base = p.cu_q[s] - p.cu_q[0];
+    const int q_len    = p.cu_q[s + 1] - p.cu_q[s];
+    const int wg0      = ti * (W * RT * 16);  // the workgroup's first row inside the sequence's portion
+    if (wg0 >= q_len) {
+        return;
+    }
+    const int  row0   = wg0 + wave * (RT * 16);
+    const bool active = row0 < q_len;  // (an inactive wave still stages and meets the barriers)
+    const int  D = p.dim, V = p.vdim;
+    const int  g = h / (H / p.kv_heads);
+    const int  pos0 = p.k_len[s] - q_len;
+    const int  lr = lane & 15, lg = lane >> 4;
+    // (a scalar load, one block ahead: a vector load would be waited for together with the DMA in flight)
+    typedef const __attribute__((address_space(4))) uint64_t ga_table;
+    ga_table*   table = (ga_table*)(p.block_ptrs + (size_t)__builtin_amdgcn_readfirstlane(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride);
+    const float cap = p.softcap, inv_cap = cap > 0.f ? 1.f / cap : 0.f;
+    const bool  bias = p.dist_r1 != nullptr;
+    const float     r1 = bias ? p.dist_r1[h] : 0.f, r2 = bias ? p.dist_r2[h] : 0.f;
+    const float*    tab = p.dist_table ? p.dist_table + (size_t)h * p.dist_table_len : nullptr;
+    bf16x8     qf[RT][DS];
+    float      qscale[RT], m[RT], l[RT] = {};
+    int        pos[RT], first[RT];
+    bool       q_ok[RT];
+    floatx4    o[RT][VT];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int qi = row0 + rt * 16 + lr;
+        q_ok[rt]     = qi < q_len;
+        pos[rt]      = pos0 + qi;
+        first[rt]    = ga_first_key(p, pos[rt]);
+        const __bf16* q = (const __bf16*)p.q + (size_t)(row_base + min(qi, q_len - 1)) * p.ldq + (size_t)h * D;
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) {
+            qf[rt][ds] = *(const bf16x8*)(q + ds * 32 + lg * 8);
+        }
+        qscale[rt] = p.scale * ga_query_temp(p, pos[rt]);
+        m[rt]      = -1e30f;
+#pragma unroll
+        for (int t = 0; t < VT; ++t) {
+            o[rt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    // this wave's rows see keys up to last_w; those of the workgroup up to last
+    const int last_w = pos0 + min(q_len, row0 + RT * 16) - 1, last = pos0 + min(q_len, wg0 + W * RT * 16) - 1;
+    const int lo_w = ga_first_key(p, pos0 + min(row0, q_len - 1)), hi_w = ga_first_key(p, last_w);
+    const int lo = ga_first_key(p, pos0 + wg0), keep = ga_keep(p);
+    const int bf = __builtin_amdgcn_readfirstlane(lo / 64), nk = __builtin_amdgcn_readfirstlane(ga_keep_blocks(p, lo, bf, 64));
+    const int n  = __builtin_amdgcn_readfirstlane(nk + last / 64 + 1 - bf);
+    // DMA: lane L of a piece fetches the 16 bytes that belong into slot L.  Piece k of the keys: 1024 / 2 D rows, of the values: 8 channels
+    constexpr int  kRowsPer = 1024 / (DS * 64);
+    const unsigned lds0     = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
+    const int      vsrc     = (lane >> 3) * 128 + (((lane & 7) ^ ((lane >> 3) & 7)) << 4);
+    const int64_t  khead = p.layer_offset + (int64_t)ga_key_head(p, g) * kKeyBytes, vhead = p.layer_offset + p.v_offset + (int64_t)ga_value_head(p, g) * V * 128;
+    uint64_t next = table[ga_block_at(0, nk, bf)];
+    auto stage = [&](int bi, int buf) {
+        const char* base = (const char*)next;
+        next             = table[ga_block_at(min(bi + 1, n - 1), nk, bf)];
+        const auto     rk   = __builtin_amdgcn_make_buffer_rsrc((void*)(base + khead), 0, kKeyBytes, 0x00020000);
+        const auto     rv   = __builtin_amdgcn_make_buffer_rsrc((void*)(base + vhead), 0, VT * 2048, 0x00020000);
+        const unsigned dst  = lds0 + buf * kBytes;
+#pragma unroll
+        for (int r = 0; r < (kPieces + W - 1) / W; ++r) {
+            const int pc = r * W + wave;
+            if (pc < DS * 4) {
+                const int row = pc * kRowsPer + lane / (DS * 4), c = lane % (DS * 4);
+                stream_dma16(rk, row * (DS * 64) + ((c ^ ga_key_swizzle<DS>(row)) << 4), 0, dst + pc * 1024);
+            }
+            else if (pc < kPieces) {
+                stream_dma16(rv, vsrc, (pc - DS * 4) * 1024, dst + pc * 1024);
+            }
+        }
+    };
+    stage(0, 0);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    for (int bi = 0; bi < n; ++bi) {
+        const int buf = bi & 1, b = ga_block_at(bi, nk, bf);
+        if (bi + 1 < n) {
+            stage(bi + 1, buf ^ 1);  // every wave is past the barrier behind its reads of that buffer
+        }
+        const char *kt = smem + buf * kBytes, *vt = kt + kKeyBytes;
+        if (active && b * 64 <= last_w && (b * 64 + 63 >= lo_w || b * 64 < keep)) {
+            int limit[RT], lower[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                limit[rt] = q_ok[rt] ? pos[rt] - b * 64 : -1;
+                lower[rt] = first[rt] - b * 64;
+            }
+            const bool whole = b * 64 + 63 <= pos0 + row0 && b * 64 >= hi_w;  // every row of the wave sees the whole block
+#define TM_STAGED(MASK_) \
+    ga_staged_step<DS, VT, RT, MASK_>(qf, kt, vt, limit, lower, MASK_ ? keep - b * 64 : 0, qscale, cap, inv_cap, bias, r1, r2, m, l, o, tab, p.dist_table_len)
+            if (whole) {
+                TM_STAGED(false);
+            }
+            else {
+                TM_STAGED(true);
+            }
+#undef TM_STAGED
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of the next block have landed ...
+        __syncthreads();                                  // ... everybody's have, and everybody is done reading this one
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        float sum = l[rt];
+        sum += __shfl_xor(sum, 16);
+        sum += __shfl_xor(sum, 32);
+        if (!q_ok[rt]) {
+            continue;
+        }
+        float inv;
+        if (p.sink) {  // m is in the log2 domain
+            const float sk = p.sink[h] * kLog2e, mf = fmaxf(m[rt], sk), a = fast_exp2(m[rt] - mf);
+            inv            = a / (sum * a + fast_exp2(sk - mf));
+        }
+        else {
+            inv = 1.f / sum;
+        }
+        const int t0 = row_base + row0 + rt * 16 + lr;
+        inv *= ga_out_gate(p, t0, h);
+#pragma unroll
+        for (int t = 0; t < VT; ++t) {  // lane holds O[row lr][channel t * 16 + lg * 4 + r]
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                ga_store<__bf16>(p, t0, h, t * 16 + lg * 4 + r, o[rt][t][r] * inv);
+            }
+        }
+    }
+}
+
+template<int DS, int VT, int RT, int W>
+static int launch_staged(const GeneralAttnParams& p, hipStream_t st)
+{
+    constexpr int lds = 2 * (64 * DS * 64 + VT * 16 * 128);
+    const auto    k   = attn_staged_kernel<DS, VT, RT, W>;
+    TM_TRY_RC(ensure_dynamic_lds((const void*)k, lds));
+    const int tiles = (p.max_q_len + W * RT * 16 - 1) / (W * RT * 16);
+    k<<<(unsigned)(p.nseq * tiles) * (unsigned)p.q_heads, W * 64, lds, st>>>(p, tiles);
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// key / value sizes of the staged kernel (0: none)
+static int staged_shape(const GeneralAttnParams& p)
+{
+    static const int kShapes[][2] = {{64, 64}, {64, 128}, {128, 128}, {256, 128}, {256, 192}, {256, 256}};
+    for (int i = 0; i < 6; ++i) {
+        if (p.dim == kShapes[i][0] && p.vdim == kShapes[i][1]) {
+            return i + 1;
+        }
+    }
+    return 0;
+}
+
 // row tiles per wave of the prefill kernel (64 * RT query rows per workgroup): as many as the register file holds without scratch --
 // every key / value fragment a wave loads then serves 16 * RT query rows.  (Key sizes up to 256 with value sizes up to 192 -- the latent
 // space of latent attention -- still hold two: 256 VGPRs + 184 AGPRs.)
@@ -816,6 +1112,15 @@ int launch_general_attention_tiles(const GeneralAttnParams& p, hipStream_t st)
     TM_REQUIRE(general_attention_tiles_ok(p), "attention tile kernel: bf16, 64-token blocks, dim and vdim multiples of 8 up to 256, sequence description");
     if (p.rows == 0) {
         return 0;
+    }
+    switch (staged_shape(p)) {
+        case 1: return launch_staged<2, 4, 2, 4>(p, st);
+        case 2: return launch_staged<2, 8, 2, 4>(p, st);
+        case 3: return launch_staged<4, 8, 2, 4>(p, st);
+        case 4: return launch_staged<8, 8, 1, 8>(p, st);
+        case 5: return launch_staged<8, 12, 1, 8>(p, st);
+        case 6: return launch_staged<8, 16, 1, 8>(p, st);
+        default: break;
     }
     const int ds = (p.dim + 31) / 32, vt = (p.vdim + 15) / 16;
     const int rows = kTileRows * tile_rt(ds <= 4 ? ds : (ds <= 6 ? 6 : 8), vt <= 1 ? 1 : (vt + 1) / 2 * 2);  // the instantiation launch_mfma picks
