@@ -10,20 +10,17 @@
 // directly the B operand of the second contraction O^T = V^T P^T -- no LDS round trip, no cross-lane shuffle for P.
 // The k-slot <-> key mapping of that second MFMA is (g, e) -> key 4g+e (e<4) / 16+4g+(e-4) (e>=4), which is
 // why V is kept transposed: a lane fetches its 8 keys of one head-dim row with one 16-byte read.
-// One wave = 16 query rows of G query heads that share a kv head (GQA): every K / V fragment feeds G MFMAs.
-// Softmax state is per lane and head.  Key order inside a 32-key step is permuted so that a lane's 8 probabilities
+// Softmax state is per lane.  Key order inside a 32-key step is permuted so that a lane's 8 probabilities
 // belong to 8 CONSECUTIVE keys: score tile A row 4g+r <-> key 8g+r, tile B row 4g+r <-> key 8g+4+r.
 //
-// K / V^T tiles go through LDS (round 3).  The four waves of a workgroup (64 query rows) need the SAME keys; rounds 1-2 read the
-// fragments straight from L2 per wave (16 KB per wave and 32-key step, 4 x redundant inside a workgroup).  Now a stage = 64 keys
-// (K 16 KB + V^T 16 KB) is brought in ONCE per workgroup by LDS-DMA (buffer_load ... lds: no staging registers -- accumulators
-// and Q fragments already take ~200), double buffered, one barrier per stage; the XOR swizzle that makes the 16-byte fragment
-// reads bank-conflict free sits on the DMA's source addresses (the DMA writes lane L to slot L of its 1 KB piece).
-// Measured (8 x 1024 prompt tokens of Llama-3-8B per launch, rocprofv3 kernel trace): 282 -> 252 us; 235 us = 0.29 PFLOP/s with
-// the conflict-free swizzle (ksw) and the leaner softmax below (profiles/r03_pmc_prefill_attention.txt).  What
-// bounds it now is the softmax's VALU issue, not memory: per 32-key step and wave 64 MFMAs (1024 matrix-pipe cycles) stand
-// against ~500 VALU slots (32 v_exp_f32 at quarter rate alone are 512 cycles), and the two waves of a SIMD share one VALU.
-// Prefill attention is 8 % of a prefill chunk (the GEMMs are 82 %), so this is where the kernel was left.
+// A workgroup is 128 query rows of one sequence and head, four waves of two 16-row tiles; a stage = 64 keys (K 16 KB + V^T 16 KB) comes in ONCE per
+// workgroup by LDS-DMA (buffer_load ... lds: no staging registers), double buffered, one barrier per stage; the XOR swizzles that make the 16-byte
+// fragment reads bank-conflict free sit on the DMA's source addresses (the DMA writes lane L to slot L of its 1 KB piece).  What bounds it is the
+// softmax's VALU issue (v_exp_f32 at quarter rate) beside about as many matrix-pipe cycles: two waves share a SIMD, out of phase, under 256 registers
+// each; a lane keeps its own partial row sum (the lane groups meet once, at the end) and the accumulators are rescaled only when a row's maximum moved.
+// MI355X, Llama-3-8B heads (32 / 8), rocprofv3: 8192 rows of two sequences of ~8000 621 us a launch (~0.85 PFLOP/s), 8 x ~1024 rows 137 us.  (Sixteen rows of four query heads
+// a wave, the form that stood here, spilled: 1236 and 237 us.)
+#include "gemm_stream.h"  // stream_dma16
 #include "tm_common.h"
 #include "tm_kernels.h"
 
@@ -68,48 +65,134 @@ __device__ __forceinline__ float sum_xor16_xor32(float v)
 // or is a clean -inf (masked score -> exp2(-inf) = 0), and the "-inf so far" selects around each exp disappear.
 constexpr float kMinScore = -1.0e30f;
 
-template<int G>
-__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(PrefillAttnParams p)
-{
-    constexpr int D     = 128;
-    constexpr int KS    = 64;           // keys per stage
-    constexpr int KTILE = KS * D * 2;   // bytes of a K tile (and of a V^T tile)
-    constexpr int STG   = 2 * KTILE;
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int b     = blockIdx.z;
-    const int hq0   = blockIdx.y * G;
-    const int lane  = threadIdx.x & 63;
-    const int wave  = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i16   = lane & 15;
-    const int g     = lane >> 4;
+constexpr int kRowTiles = 2, kRowsWave = 16 * kRowTiles, kRowsGroup = 4 * kRowsWave;
 
+template<bool MASK>
+__device__ __forceinline__ void prefill_step(const half8_t (&qf)[kRowTiles][4], const char* __restrict__ kt, const char* __restrict__ vt,
+                                             const int (&limit)[kRowTiles], float sc, float (&m)[kRowTiles], float (&l)[kRowTiles],
+                                             floatx4 (&O)[kRowTiles][8])
+{
+    const int lane = threadIdx.x & 63, i16 = lane & 15, g = lane >> 4;
+    floatx4   s[kRowTiles][4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {  // score tile t, row i16: key 32 (t / 2) + 8 (i16 / 4) + 4 (t % 2) + i16 % 4 of the stage
+#pragma unroll
+        for (int rt = 0; rt < kRowTiles; ++rt) {
+            s[rt][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        const int   row = (t >> 1) * 32 + (i16 >> 2) * 8 + (t & 1) * 4 + (i16 & 3);
+        const char* kr  = kt + row * 256;
+        const int   sw  = ksw(row);
+#pragma unroll
+        for (int dd = 0; dd < 4; ++dd) {
+            const half8_t kf = *(const half8_t*)(kr + (((4 * dd + g) ^ sw) << 4));
+#pragma unroll
+            for (int rt = 0; rt < kRowTiles; ++rt) {
+                s[rt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qf[rt][dd], s[rt][t], 0, 0, 0);
+            }
+        }
+    }
+    half8_t pf[kRowTiles][2];
+#pragma unroll
+    for (int rt = 0; rt < kRowTiles; ++rt) {
+        // lane holds S[key 32 (t / 2) + 8 g + 4 (t % 2) + r][q = i16]
+        float tmax = kMinScore;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (MASK) {
+                    s[rt][t][r] = (t >> 1) * 32 + 8 * g + (t & 1) * 4 + r <= limit[rt] ? s[rt][t][r] : -INFINITY;
+                }
+                tmax = fmaxf(tmax, s[rt][t][r]);
+            }
+        }
+        tmax             = max_xor32(max_xor16(tmax));
+        const float mnew = fmaxf(m[rt], tmax);  // finite (kMinScore at least)
+        const float ms   = mnew * sc;
+        float       psum = 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float pv = fast_exp2(__builtin_fmaf(s[rt][t][r], sc, -ms));  // masked score: exp2(-inf) = 0
+                psum += pv;
+                pf[rt][t >> 1][(t & 1) * 4 + r] = (half_t)pv;
+            }
+        }
+        if (__any(mnew != m[rt])) {
+            const float alpha = fast_exp2((m[rt] - mnew) * sc);
+            l[rt] *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+                O[rt][dt] *= alpha;
+            }
+        }
+        l[rt] += psum;
+        m[rt] = mnew;
+    }
+    // O^T += V^T P^T: one 16-byte V^T fragment (8 consecutive keys of one head-dim row) feeds both row tiles
+    const char* vr = vt + i16 * 128;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const half8_t vf = *(const half8_t*)(vr + dt * 2048 + (((4 * ks + g) ^ (i16 & 7)) << 4));
+#pragma unroll
+            for (int rt = 0; rt < kRowTiles; ++rt) {
+                O[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[rt][ks], O[rt][dt], 0, 0, 0);
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(PrefillAttnParams p, int tiles)
+{
+    constexpr int D = 128, KS = 64, KTILE = KS * D * 2, STG = 2 * KTILE;  // keys per stage; bytes of a K tile (and of a V^T tile)
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i16 = lane & 15, g = lane >> 4;
+    // workgroup i runs on XCD i % 8: the query heads of a kv head on one XCD where the head count allows it; the longest row blocks of every sequence first
+    // (longest-processing-time order: the short ones fill the tail)
+    int       i = blockIdx.x, hq;
+    const int H = p.q_heads;
+    if (H % 8 == 0) {
+        hq = (i % 8) * (H / 8) + (i / 8) % (H / 8);
+    }
+    else {
+        hq = i % H;
+    }
+    i /= H;
+    const int b = i % p.batch, bx = tiles - 1 - i / p.batch;
     const int q_beg = p.cu_q_len[b];
     const int qlen  = p.cu_q_len[b + 1] - q_beg;
     const int klen  = p.k_len[b];
     const int hist  = klen - qlen;
-    // causal: query block bx walks bx + 1 stages (+ history).  The dispatcher hands out workgroups in blockIdx order, so the
-    // LONGEST blocks of every (head group, sequence) go first and the short ones fill the tail (longest-processing-time order)
-    const int bx = (int)gridDim.x - 1 - (int)blockIdx.x;
-    if (bx * 64 >= qlen) {
+    if (bx * kRowsGroup >= qlen) {
         return;  // workgroup-uniform
     }
-    const int  q0     = bx * 64 + wave * 16;
+    const int  q0     = bx * kRowsGroup + wave * kRowsWave;
     const bool active = q0 < qlen;  // wave-uniform; an inactive wave still stages tiles and meets the barriers
-    const int  group  = p.q_heads / p.kv_heads;
-    const int  kvh    = hq0 / group;
+    const int  kvh    = hq / (H / p.kv_heads);
 
-    // Q^T fragments (B operand): lane (j = query row, g) holds Q[q0+j][32*dd + 8g .. +8) of head hq0 + h
-    const int     qrow = min(q0 + i16, qlen - 1);
-    const half_t* qptr = p.q + (size_t)(q_beg + qrow) * p.q_stride + (size_t)hq0 * D;
-    half8_t       qf[G][4];
+    // Q^T fragments (B operand): lane (j = query row, g) holds Q[row j][32*dd + 8g .. +8)
+    half8_t qf[kRowTiles][4];
+    floatx4 O[kRowTiles][8];
+    float   m[kRowTiles], l[kRowTiles];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
+    for (int rt = 0; rt < kRowTiles; ++rt) {
+        const half_t* qptr = p.q + (size_t)(q_beg + min(q0 + rt * 16 + i16, qlen - 1)) * p.q_stride + (size_t)hq * D;
 #pragma unroll
         for (int dd = 0; dd < 4; ++dd) {
-            qf[h][dd] = *(const half8_t*)(qptr + h * D + dd * 32 + g * 8);
+            qf[rt][dd] = *(const half8_t*)(qptr + dd * 32 + g * 8);
+        }
+        m[rt] = kMinScore;
+        l[rt] = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) {
+            O[rt][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
     }
-
     // the sequence's region of the scratch is 64-key aligned, its V^T tail is zero-filled (flatten_kv_kernel): a 64-key stage
     // never leaves the region; K rows past klen may hold stale data, their scores are masked below
     const half_t* kbase    = p.k + ((size_t)kvh * p.k_stride + p.cu_k_off[b]) * D;
@@ -129,36 +212,13 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(PrefillAttnPa
     auto stage_in = [&](int ks, int buf) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            unsigned       keep;
             const unsigned dk = lds0 + buf * STG + (4 * r + wave) * 1024;
-            const unsigned dv = dk + KTILE;
-            const int      sk = ks * D * 2 + r * 16 * 256, sv = ks * 2 + r * 32 * p.k_stride * 2;
-            asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\t"
-                         "buffer_load_dwordx4 %1, %2, %4 offen lds\n\t"
-                         "s_mov_b32 m0, %5\n\ts_nop 0\n\t"
-                         "buffer_load_dwordx4 %6, %7, %8 offen lds\n\ts_mov_b32 m0, %0"
-                         : "=&s"(keep)
-                         : "v"(kdo), "s"(rs_k), "s"(dk), "s"(sk), "s"(dv), "v"(vdo), "s"(rs_v), "s"(sv)
-                         : "memory");
+            stream_dma16(rs_k, kdo, ks * D * 2 + r * 16 * 256, dk);
+            stream_dma16(rs_v, vdo, ks * 2 + r * 32 * p.k_stride * 2, dk + KTILE);
         }
     };
-
-    floatx4 O[G][8];
-    float   m[G], l[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-        m[h] = kMinScore;
-        l[h] = 0.f;
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-            O[h][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    const float sc      = p.scale_log2;
-    const int   qpos    = hist + q0 + i16;                              // absolute position of this lane's query row
-    const int   kend_w  = active ? min(klen, hist + q0 + 16) : 0;       // keys visible to the last row of this wave
-    const int   kend_wg = min(klen, hist + bx * 64 + 64);               // ... of this workgroup
-    const int   krow    = 8 * (i16 >> 2) + (i16 & 3);                   // key (within the 32-key step) of score-tile-A row i16; tile B: +4
+    const int kend_w  = active ? min(klen, hist + q0 + kRowsWave) : 0;      // keys visible to the last row of this wave
+    const int kend_wg = min(klen, hist + (bx + 1) * kRowsGroup);            // ... of this workgroup
 
     stage_in(0, 0);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -168,110 +228,36 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(PrefillAttnPa
         if (ks0 + KS < kend_wg) {
             stage_in(ks0 + KS, buf ^ 1);  // every wave is past the barrier behind its reads of that buffer
         }
-        const char* kt = smem + buf * STG;
-        const char* vt = kt + KTILE;
-#pragma nounroll
-        for (int sub = 0; sub < 2; ++sub) {
-            const int ks = ks0 + 32 * sub;
-            if (ks >= kend_w) {  // wave-uniform: causal end of this wave (or an inactive wave)
-                continue;
+        const char *kt = smem + buf * STG, *vt = kt + KTILE;
+        if (ks0 < kend_w) {  // wave-uniform: causal end of this wave (or an inactive wave)
+            int limit[kRowTiles];  // last visible key of the lane's rows in this stage (rows past the portion: none)
+#pragma unroll
+            for (int rt = 0; rt < kRowTiles; ++rt) {
+                const int r = q0 + rt * 16 + i16;
+                limit[rt]   = r < qlen ? hist + r - ks0 : -1;
             }
-            half8_t ka[4], kb[4];
-            {
-                const int ra = 32 * sub + krow, rb = ra + 4;
-#pragma unroll
-                for (int dd = 0; dd < 4; ++dd) {
-                    ka[dd] = *(const half8_t*)(kt + ra * 256 + (((4 * dd + g) ^ ksw(ra)) << 4));
-                    kb[dd] = *(const half8_t*)(kt + rb * 256 + (((4 * dd + g) ^ ksw(rb)) << 4));
-                }
+            // the whole stage lies at or below the diagonal for every row of the wave: no masking needed (all but the last stages)
+            if (ks0 + KS - 1 <= hist + q0 && q0 + kRowsWave <= qlen) {
+                prefill_step<false>(qf, kt, vt, limit, p.scale_log2, m, l, O);
             }
-            // the whole 32-key step lies at or below the diagonal for every row of the wave and inside the context:
-            // no masking needed (wave-uniform; true for all but the last one or two steps)
-            const bool full = ks + 32 <= klen && ks + 31 <= hist + q0;
-            half8_t    pf[G];
-            floatx4    sa_[G], sb_[G];
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                floatx4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int dd = 0; dd < 4; ++dd) {
-                    sa = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka[dd], qf[h][dd], sa, 0, 0, 0);
-                    sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[dd], qf[h][dd], sb, 0, 0, 0);
-                }
-                sa_[h] = sa;
-                sb_[h] = sb;
-            }
-            // one head at a time, its rescale decided right there: the branch per head keeps the four chains from being
-            // interleaved -- measured: ONE basic block for all heads (scheduler free to overlap the chains) needs 45 spilled
-            // registers and runs 284 us against 239..261 us this way
-#pragma unroll
-            for (int h = 0; h < G; ++h) {
-                const floatx4 sa = sa_[h], sb = sb_[h];
-                // lane holds S[key = ks + 8g + r][q] in sa[r] and S[key = ks + 8g + 4 + r][q] in sb[r]
-                float s[8];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    s[r]     = sa[r];
-                    s[4 + r] = sb[r];
-                }
-                if (!full) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) {
-                        const int t = ks + 8 * g + e;
-                        s[e]        = (t < klen && t <= qpos) ? s[e] : -INFINITY;
-                    }
-                }
-                float tmax = s[0];
-#pragma unroll
-                for (int e = 1; e < 8; ++e) {
-                    tmax = fmaxf(tmax, s[e]);
-                }
-                tmax              = max_xor32(max_xor16(tmax));
-                const float mnew  = fmaxf(m[h], tmax);  // finite (kMinScore at least)
-                const float alpha = fast_exp2((m[h] - mnew) * sc);
-                float       psum  = 0.f;
-                const float ms    = mnew * sc;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const float pv = fast_exp2(__builtin_fmaf(s[e], sc, -ms));  // masked score: exp2(-inf) = 0
-                    psum += pv;
-                    pf[h][e] = (half_t)pv;
-                }
-                l[h] = l[h] * alpha + psum;
-                if (__builtin_amdgcn_readfirstlane((int)__any(mnew != m[h]))) {  // wave-uniform: did any row's max move?
-#pragma unroll
-                    for (int dt = 0; dt < 8; ++dt) {
-                        O[h][dt] *= alpha;
-                    }
-                }
-                m[h] = mnew;
-            }
-            // ---- O^T += V^T P^T: one 16-byte V^T fragment (8 consecutive keys of one head-dim row) feeds G MFMAs ----
-            // (fragments fetched here, not above the softmax: 32 more live registers there would spill at G = 4)
-            const char* vrow = vt + i16 * 128 + (((4 * sub + g) ^ (i16 & 7)) << 4);  // row dt*16 + i16: same swizzle term for every dt
-#pragma unroll
-            for (int dt = 0; dt < 8; ++dt) {
-                const half8_t vf = *(const half8_t*)(vrow + dt * 16 * 128);
-#pragma unroll
-                for (int h = 0; h < G; ++h) {
-                    O[h][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf[h], O[h][dt], 0, 0, 0);
-                }
+            else {
+                prefill_step<true>(qf, kt, vt, limit, p.scale_log2, m, l, O);
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's pieces of the next stage have landed ...
         __syncthreads();                                  // ... everybody's have, and everybody is done reading this one
     }
-
-    if (active && q0 + i16 < qlen) {
 #pragma unroll
-        for (int h = 0; h < G; ++h) {
-            const float lh = sum_xor16_xor32(l[h]);
-            half_t*     optr = p.out + (size_t)(q_beg + q0 + i16) * p.q_heads * D + (size_t)(hq0 + h) * D;
+    for (int rt = 0; rt < kRowTiles; ++rt) {
+        const float lh = sum_xor16_xor32(l[rt]);
+        const int   r  = q0 + rt * 16 + i16;
+        if (r < qlen) {
+            half_t*     optr = p.out + (size_t)(q_beg + r) * p.q_heads * D + (size_t)hq * D;
             const float inv  = 1.0f / lh;
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) {
-                half4_t o = {(half_t)(O[h][dt][0] * inv), (half_t)(O[h][dt][1] * inv), (half_t)(O[h][dt][2] * inv),
-                             (half_t)(O[h][dt][3] * inv)};
+                half4_t o = {(half_t)(O[rt][dt][0] * inv), (half_t)(O[rt][dt][1] * inv), (half_t)(O[rt][dt][2] * inv),
+                             (half_t)(O[rt][dt][3] * inv)};
                 *(half4_t*)(optr + dt * 16 + g * 4) = o;
             }
         }
@@ -285,25 +271,12 @@ int launch_prefill_attention(const PrefillAttnParams& p, hipStream_t st)
     if (p.batch == 0 || p.max_q_len == 0) {
         return 0;
     }
-    const int group = p.q_heads / p.kv_heads;
-    const int G     = group % 4 == 0 ? 4 : (group % 2 == 0 ? 2 : 1);  // query heads per wave (share one kv head); G = 4 spills ~25
-                                                                       // registers at two workgroups per CU -- measured equal to G = 2
-    dim3      grid((p.max_q_len + 63) / 64, p.q_heads / G, p.batch);
     constexpr int lds = 2 * 2 * 64 * 128 * 2;  // two stages of (K tile + V^T tile)
-    const void* const k = G == 4 ? (const void*)prefill_attention_kernel<4> :
-                          G == 2 ? (const void*)prefill_attention_kernel<2> : (const void*)prefill_attention_kernel<1>;
-    if (const int rc = ensure_dynamic_lds(k, lds)) {
+    if (const int rc = ensure_dynamic_lds((const void*)prefill_attention_kernel, lds)) {
         return rc;
     }
-    if (G == 4) {
-        prefill_attention_kernel<4><<<grid, 256, lds, st>>>(p);
-    }
-    else if (G == 2) {
-        prefill_attention_kernel<2><<<grid, 256, lds, st>>>(p);
-    }
-    else {
-        prefill_attention_kernel<1><<<grid, 256, lds, st>>>(p);
-    }
+    const int tiles = (p.max_q_len + kRowsGroup - 1) / kRowsGroup;
+    prefill_attention_kernel<<<(unsigned)(tiles * p.batch) * (unsigned)p.q_heads, 256, lds, st>>>(p, tiles);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }
