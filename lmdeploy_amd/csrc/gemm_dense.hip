@@ -312,11 +312,11 @@ void dense_weight_free(DenseWeight& d)
 //     rows, (K, N) = (4096, 21504): 256 x 256 1155 us (1.25 PFLOP/s), 256 x 128 1281, 128 x 128 1520, 64 x 64 2714; (2048, 256) with 8000 rows: 46,
 //     33, 23, 20 us; (2048, 2048) with 2600 rows: 50, 36, 35, 48 us
 //   skinny kernel: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; 25 GB/s a CU, a line of x (from L2) at 0.7 of the
-//     price of a line of weights.  32 rows bf16, (25600, 4096): one slice 119 us, four 46, eight 45; (4096, 6144): one 23, three 19, four 18;
+//     price of a line of weights.  32 rows bf16, (25600, 4096): one slice 119 us, four 46, eight 45; (4096, 6144): one 23, three 19, four 18 (slices of equal length);
 //     (4096, 21504): one 40, two 42; nine items of (2048, 2816): one 21, three 31; three rows fp32, (8448, 2048): one 75, eight 21; pairs, four
 //     rows, (2048, 11264): one 17, two 23
-//   narrow kernel: eight rows bf16, (2048, 2048): 6.5 us against 7.3 with four slices; three rows fp32, (768, 2048): 6.1 against 7.8, (2048, 2048): 11.2
-//     against 9.8; without scratch (25600, 4096) with 32 rows: 76 against 120
+//   narrow kernel: eight rows bf16, (2048, 2048): 6.5 us against 7.5 with four slices, (2048, 4096): 8.3 against 8.9, (2048, 6144): 12.5 against 10.5, (2048,
+//     10240): 18.3 against 13.0 unsliced; three rows fp32, (768, 2048): 6.1 against 7.9, (2048, 2048): 10.8 against 9.6; without scratch (25600, 4096) with 32 rows: 76 against 120
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets)
 {
     struct Tile {
@@ -346,7 +346,13 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     const double step   = 64.0 * (wg_cols + 0.7 * std::min(rows, 16 * mt)) / 25e3;
     int          sp     = groups >= (pairs ? 80 : 200) ? 1 : (256 + groups - 1) / groups;  // about one workgroup a CU
     sp          = std::max(1, std::min({sp, steps / 16, 16}));
-    best.narrow = groups < 200 && !pairs && rows <= 16 && steps <= 64;  // short sums: the way through memory costs more than it gives
+    for (int more = sp; sp > 1 && more < 2 * sp && more <= 16; ++more) {  // slices of equal length
+        if (steps % (8 * more) == 0) {
+            sp = more;
+            break;
+        }
+    }
+    best.narrow = groups <= 64 && !pairs && rows <= 16 && steps <= 64;  // short sums: the way through memory costs more than it gives
     if (best.narrow) {
         sp = 1;
     }
