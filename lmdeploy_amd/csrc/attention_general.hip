@@ -29,6 +29,7 @@
 // Cache block layout per layer: keys [kv_heads][64][dim], then values [kv_heads][vdim][64].
 #include "tm_kernels.h"
 #include "gemm_stream.h"  // stream_dma16
+#include <algorithm>
 #include <stdlib.h>
 
 #define TM_TRY_RC(expr)      \
@@ -126,6 +127,18 @@ __device__ __forceinline__ int ga_block_at(int bi, int nk, int bf)
     return bi < nk ? bi : bf + (bi - nk);
 }
 
+// blocks of a key split of a row that visits nvis blocks, and the splits it needs then (at least one): the others leave at once, and a row of one split
+// is finished by it
+__device__ __forceinline__ int ga_split_len(const GeneralAttnParams& p, int nvis)
+{
+    return max((nvis + p.splits - 1) / p.splits, p.split_blocks);
+}
+__device__ __forceinline__ int ga_split_count(const GeneralAttnParams& p, int nvis)
+{
+    const int per = ga_split_len(p, nvis);
+    return max((nvis + per - 1) / per, 1);
+}
+
 // where head h of an output row starts: heads side by side unless the caller spaces them (a batched product reads them at a stride)
 __device__ __forceinline__ size_t ga_out_head(const GeneralAttnParams& p, int h)
 {
@@ -160,6 +173,21 @@ __device__ __forceinline__ void ga_store(const GeneralAttnParams& p, int t, int 
     }
 }
 
+// four channels from v on (the hardware stores 8 and 16 bytes at any element's address)
+typedef float ga_floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
+template<class T>
+__device__ __forceinline__ void ga_store4(const GeneralAttnParams& p, int t, int h, int v, floatx4 val)
+{
+    typedef T    T4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+    const size_t at = (size_t)t * p.ldo + ga_out_head(p, h) + v;
+    if (p.out_f32) {
+        *(ga_floatx4_any*)((float*)p.out + at) = val;
+    }
+    else {
+        *(T4*)((T*)p.out + at) = T4{(T)val[0], (T)val[1], (T)val[2], (T)val[3]};
+    }
+}
+
 // grid (rows, ceil(q_heads / 4), splits), 256 threads: wave w -> head blockIdx.y * 4 + w
 template<class T, int VC>
 __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
@@ -182,8 +210,11 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
     const int   nkeys = pos + 1, nblk = (nkeys + p.block_len - 1) / p.block_len;
     const int   first = ga_first_key(p, pos), bf = first / p.block_len;  // the first key of the visible range and its block
     const int   keep = ga_keep(p), nk = ga_keep_blocks(p, first, bf, p.block_len), nvis = nk + nblk - bf;
-    const int   per = (nvis + p.splits - 1) / p.splits;
+    const int   per = ga_split_len(p, nvis), nsplit = ga_split_count(p, nvis);
     const int   i0 = sp * per, i1 = min(nvis, i0 + per);
+    if (sp >= nsplit) {
+        return;
+    }
     const float r1 = p.dist_r1 ? p.dist_r1[h] : 0.f, r2 = p.dist_r1 ? p.dist_r2[h] : 0.f;
     float m = -1e30f, l = 0.f, o[VC];
 #pragma unroll
@@ -238,7 +269,7 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
             }
         }
     }
-    if (p.splits == 1) {
+    if (nsplit == 1) {
         float inv;
         if (p.sink) {
             const float sk = p.sink[h], mf = fmaxf(m, sk), a = __expf(m - mf);
@@ -277,10 +308,15 @@ template<class T, int VC>
 __global__ __launch_bounds__(64) void attn_rows_merge_kernel(GeneralAttnParams p)
 {
     const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, V = p.vdim;
+    const int pos = p.row_pos[t], first = ga_first_key(p, pos), bf = first / p.block_len;
+    const int nsplit = ga_split_count(p, ga_keep_blocks(p, first, bf, p.block_len) + (pos + p.block_len) / p.block_len - bf);
+    if (nsplit == 1) {
+        return;
+    }
     const float* pm = p.partial_ml + ((size_t)t * p.q_heads + h) * p.splits * 2;
     const float* po = p.partial_o + ((size_t)t * p.q_heads + h) * p.splits * V;
     float        mf = p.sink ? p.sink[h] : -1e30f;
-    for (int s = 0; s < p.splits; ++s) {
+    for (int s = 0; s < nsplit; ++s) {
         mf = fmaxf(mf, pm[s * 2]);
     }
     float l = p.sink ? __expf(p.sink[h] - mf) : 0.f;
@@ -289,7 +325,8 @@ __global__ __launch_bounds__(64) void attn_rows_merge_kernel(GeneralAttnParams p
     for (int c = 0; c < VC; ++c) {
         o[c] = 0.f;
     }
-    for (int s = 0; s < p.splits; ++s) {
+#pragma unroll 4
+    for (int s = 0; s < nsplit; ++s) {
         const float a = __expf(pm[s * 2] - mf);
         l += a * pm[s * 2 + 1];
 #pragma unroll
@@ -620,7 +657,7 @@ template<int DS, int VT>
 __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, int chunks)
 {
     __shared__ float ml_s[4][16][2];
-    __shared__ float o_s[3][16][VT * 16];
+    __shared__ float o_s[3][16][VT * 16 + 4];  // + 4: the sixteen rows start in different banks
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = blockIdx.x, g = blockIdx.y / chunks, chunk = blockIdx.y % chunks, sp = blockIdx.z;
     const int D = p.dim, V = p.vdim, group = p.q_heads / p.kv_heads;
@@ -654,8 +691,11 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
     const float* tab = p.dist_table ? p.dist_table + (size_t)h * p.dist_table_len : nullptr;
     const int first = ga_first_key(p, pos), bf = first / 64;
     const int keep = ga_keep(p), nk = ga_keep_blocks(p, first, bf, 64);
-    const int nvis = nk + pos / 64 + 1 - bf, per = (nvis + p.splits - 1) / p.splits;
+    const int nvis = nk + pos / 64 + 1 - bf, per = ga_split_len(p, nvis), nsplit = ga_split_count(p, nvis);
     const int i0 = sp * per, i1 = min(nvis, i0 + per);
+    if (sp >= nsplit) {
+        return;
+    }
     for (int bi = i0 + wave; bi < i1; bi += 4) {
         const int   b    = ga_block_at(bi, nk, bf);
         const char* base = (const char*)table[b] + p.layer_offset;
@@ -677,10 +717,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
     if (wave > 0) {
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                o_s[wave - 1][lr][v * 16 + lg * 4 + r] = o[v][r] * a;
-            }
+            *(floatx4*)&o_s[wave - 1][lr][v * 16 + lg * 4] = o[v] * a;
         }
     }
     __syncthreads();
@@ -694,13 +731,10 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
     }
 #pragma unroll
     for (int v = 0; v < VT; ++v) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int c = v * 16 + lg * 4 + r;
-            o[v][r]     = o[v][r] * a + ((o_s[0][lr][c] + o_s[1][lr][c]) + o_s[2][lr][c]);
-        }
+        const int c = v * 16 + lg * 4;
+        o[v]        = o[v] * a + ((*(const floatx4*)&o_s[0][lr][c] + *(const floatx4*)&o_s[1][lr][c]) + *(const floatx4*)&o_s[2][lr][c]);
     }
-    if (p.splits == 1) {
+    if (nsplit == 1) {
         float inv;
         if (p.sink) {
             const float sk = p.sink[h], m2 = fmaxf(mf, sk), a2 = __expf(mf - m2);
@@ -712,12 +746,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
         inv *= ga_out_gate(p, t, h);
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int c = v * 16 + lg * 4 + r;
-                if (c < V) {
-                    ga_store<__bf16>(p, t, h, c, o[v][r] * inv);
-                }
+            const int c = v * 16 + lg * 4;
+            if (c < V) {
+                ga_store4<__bf16>(p, t, h, c, o[v] * inv);
             }
         }
         return;
@@ -726,12 +757,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
     float* pm = p.partial_ml + (((size_t)t * p.q_heads + h) * p.splits + sp) * 2;
 #pragma unroll
     for (int v = 0; v < VT; ++v) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int c = v * 16 + lg * 4 + r;
-            if (c < V) {
-                po[c] = o[v][r];
-            }
+        const int c = v * 16 + lg * 4;
+        if (c < V) {
+            *(ga_floatx4_any*)(po + c) = o[v];
         }
     }
     if (lg == 0) {
@@ -1098,10 +1126,15 @@ int launch_general_attention_decode(const GeneralAttnParams& p, hipStream_t st)
     if (p.rows == 0) {
         return 0;
     }
-    const int chunks = (p.q_heads / p.kv_heads + 15) / 16;
-    TM_TRY_RC(launch_mfma(p, chunks, dim3(p.rows, p.kv_heads * chunks, p.splits), st, true));
+    // A workgroup takes four blocks at the time of one, so splits below four blocks only pay while the launch leaves compute units idle: 256 workgroups
+    // without splits (64 * 4) are enough.  32 rows of 32 / 8 heads of 128, ~150 tokens, 8 splits: 13.2 + 5.0 us (kernel + merge) with splits of one block,
+    // 9.4 + 2.4 with splits of at least four (eight: the same); 21.9 + 7.9 when the splits without a block ran to the end as well
+    const int         chunks = (p.q_heads / p.kv_heads + 15) / 16, base = p.rows * p.kv_heads * chunks;
+    GeneralAttnParams a      = p;
+    a.split_blocks           = std::min(4, std::max(1, base / 64));
+    TM_TRY_RC(launch_mfma(a, chunks, dim3(p.rows, p.kv_heads * chunks, p.splits), st, true));
     if (p.splits > 1) {
-        launch_rows_merge<__bf16>(p, st);
+        launch_rows_merge<__bf16>(a, st);
         TM_HIP_CHECK(hipGetLastError());
     }
     return 0;

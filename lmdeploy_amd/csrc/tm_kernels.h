@@ -461,7 +461,8 @@ struct GeneralAttnParams {
     const float*    dist_table = nullptr;  // [q_heads][dist_table_len] or nullptr: score += dist_table[head][min(position - key position, len - 1)]
     int             dist_table_len = 0;
     int             out_f32 = 0;           // != 0: the output rows are fp32 whatever the cache's element type
-    int             splits = 1;
+    int             splits = 1;            // most workgroups that share the keys of a row; a row uses as many as it has blocks for
+    int             split_blocks = 1;      // least cache blocks of a split
     float*          partial_o = nullptr;   // [rows][q_heads][splits][vdim]
     float*          partial_ml = nullptr;  // [rows][q_heads][splits][2]
     // tile kernel only: the sequences of the launch
