@@ -1560,15 +1560,12 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
     else {
         const int k = s.top, E = s.experts;
         TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_dense_linear(L.router, lm.d_h1, lm.ldw, lm.d_proj, lm.ldproj, M, kDenseScaleF32, 1.f, st)));
-        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_topk_softmax(lm.d_topk_ids, lm.d_topk_w, lm.d_proj, lm.ldproj, M, E, k, s.router_scale, st)));
-        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_route(lm.d_offsets, lm.d_f2n, lm.d_en2f, lm.d_topk_ids, M, E, k, st)));
-        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_gather(lm.d_moe_x, lm.ldw, lm.d_h1, lm.ldw, lm.elem, lm.d_topk_w, lm.d_en2f, M, W, k, false, st)));
-        int rows = M * k;
-        if (L.shared_fused) {  // the shared expert: item E of the batched products over a copy of all rows behind the routed ones
-            TM_HIP_CHECK(hipMemcpyAsync((char*)lm.d_moe_x + (size_t)rows * lm.ldw * lm.elem, lm.d_h1, (size_t)M * lm.ldw * lm.elem, hipMemcpyDeviceToDevice, st));
-            TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_extend_offsets(lm.d_offsets, E, M, st)));
-            rows += M;
-        }
+        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_softmax_route(lm.d_topk_ids, lm.d_topk_w, lm.d_offsets, lm.d_f2n, lm.d_en2f, lm.d_proj, lm.ldproj, M, E,
+                                                                k, s.router_scale, st)));
+        // the shared expert: item E of the batched products over a copy of all rows behind the routed ones
+        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_gather(lm.d_moe_x, lm.ldw, lm.d_h1, lm.ldw, lm.elem, lm.d_topk_w, lm.d_en2f, M, W, k, false, st,
+                                                         L.shared_fused ? lm.d_offsets : nullptr, E)));
+        const int rows = M * (k + (L.shared_fused ? 1 : 0));
         DenseCall c;
         c.epi         = kDenseRelu2;
         c.count       = E + (L.shared_fused ? 1 : 0);

@@ -26,7 +26,23 @@ namespace tmk {
 constexpr int kMaxExperts = 64;
 constexpr int kMaxTopK    = 8;
 
-// one 256-thread workgroup per token; Wg fp16 [H][E] (input-major like every other weight)
+// the largest v of a wave, the lower index on a tie (i = INT_MAX: no candidate); every lane ends up with lane 0's choice
+__device__ __forceinline__ void wave_argmax(float& v, int& i)
+{
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const float ov = __shfl_xor(v, d);
+        const int   oi = __shfl_xor(i, d);
+        if (oi != 0x7fffffff && (i == 0x7fffffff || ov > v || (ov == v && oi < i))) {
+            v = ov, i = oi;
+        }
+    }
+}
+
+// One 256-thread workgroup per token; Wg fp16 [H][E] (input-major like every other weight).  V experts share a pass over the token (V = 8: E a multiple of
+// eight, 16-byte loads of Wg), so the row is read E / V times and every load is independent of the last; one wave picks the experts.  Bound by that
+// chain: H = 4096, 8 experts: 24.6 us with a pass per expert and one thread picking, 8.5 us so.
+template<int V>
 __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_ids,      // [T][k]
                                                        float* __restrict__ topk_w,      // [T][k]
                                                        float* __restrict__ logits_out,  // [T][E] or nullptr
@@ -39,67 +55,160 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_id
                                                        int norm_topk,
                                                        float routed_scale)
 {
+    typedef half_t HV __attribute__((ext_vector_type(V)));
     __shared__ float part[4][kMaxExperts];
-    __shared__ float logit[kMaxExperts];
     const int        t    = blockIdx.x;
     const int        lane = threadIdx.x & 63;
     const int        wave = threadIdx.x >> 6;
     const half_t*    xr   = x + (size_t)t * ldx;
-    for (int e = 0; e < E; ++e) {
-        float acc = 0.f;
+    for (int e = 0; e < E; e += V) {
+        float acc[V];
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            acc[i] = 0.f;
+        }
+#pragma unroll 8
         for (int h = threadIdx.x; h < H; h += 256) {
-            acc = __builtin_fmaf((float)xr[h], (float)wg[(size_t)h * E + e], acc);
+            const float xv = (float)xr[h];
+            const HV    wv = *(const HV*)(wg + (size_t)h * E + e);
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                acc[i] = __builtin_fmaf(xv, (float)wv[i], acc[i]);
+            }
         }
-        acc = group_sum<64>(acc);
-        if (lane == 0) {
-            part[wave][e] = acc;
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            acc[i] = group_sum<64>(acc[i]);
+            if (lane == 0) {
+                part[wave][e + i] = acc[i];
+            }
         }
     }
     __syncthreads();
-    if (threadIdx.x < E) {
-        logit[threadIdx.x] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
-        if (logits_out) {
-            logits_out[(size_t)t * E + threadIdx.x] = logit[threadIdx.x];
-        }
+    if (wave > 0) {
+        return;
+    }
+    const bool  in    = lane < E;  // lane = expert
+    const float logit = in ? (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]) : -INFINITY;
+    if (in && logits_out) {
+        logits_out[(size_t)t * E + lane] = logit;
+    }
+    const float mx    = group_max<64>(logit);
+    bool        taken = !in;
+    int         id    = 0;       // lane j < k: choice j
+    float       val   = 0.f, denom = 0.f;
+    for (int j = 0; j < k; ++j) {
+        float v = logit;
+        int   i = taken ? 0x7fffffff : lane;
+        wave_argmax(v, i);
+        i     = __builtin_amdgcn_readfirstlane(i);
+        v     = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+        taken = taken || lane == i;
+        id    = lane == j ? i : id;
+        val   = lane == j ? v : val;
+        denom += __builtin_expf(v - mx);
+    }
+    if (!norm_topk) {
+        denom = group_sum<64>(in ? __builtin_expf(logit - mx) : 0.f);
+    }
+    if (lane < k) {
+        topk_ids[(size_t)t * k + lane] = id;
+        topk_w[(size_t)t * k + lane]   = __builtin_expf(val - mx) * (1.0f / denom) * routed_scale;
+    }
+}
+
+// Routing tables of up to kRouteTokens tokens and kRouteExperts experts in one workgroup: an expert's tokens are a 64-bit mask in LDS, a pair's place the
+// expert's first row (a wave's scan over the experts) plus the tokens ahead of it in the mask -- no pass over the experts.  PICK: the experts are first
+// chosen here, one wave per token, as moe_topk_softmax_kernel does (expert e on lane e % 64).  A chain of latencies: 8 tokens, 8 experts, 2 a token take
+// 4.8 us, the two kernels for any size 5.7 + 9.5.
+constexpr int kRouteTokens = 64, kRouteExperts = 256;
+template<bool PICK>
+__global__ __launch_bounds__(1024) void moe_route_masks_kernel(int* __restrict__ offsets, int* __restrict__ f2n, int* __restrict__ en2f, int* topk_ids,
+                                                               float* __restrict__ w, const float* __restrict__ logits, int ld, int T, int E, int k,
+                                                               float scale)
+{
+    constexpr int NE = kRouteExperts / 64;
+    __shared__ unsigned long long mask[kRouteExperts];
+    __shared__ int                first[kRouteExperts];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid < kRouteExperts) {
+        mask[tid] = 0;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int      ids[kMaxTopK];
-        float    val[kMaxTopK];
-        uint64_t taken = 0;
-        float    mx    = -INFINITY;
-        for (int e = 0; e < E; ++e) {
-            mx = fmaxf(mx, logit[e]);
-        }
-        for (int j = 0; j < k; ++j) {
-            int   best = -1;
-            float bv   = -INFINITY;
-            for (int e = 0; e < E; ++e) {
-                if (!((taken >> e) & 1) && (best < 0 || logit[e] > bv)) {
-                    best = e;
-                    bv   = logit[e];
+    if constexpr (PICK) {
+        for (int t = wave; t < T; t += 16) {
+            float z[NE], mx = -INFINITY, den = 0.f;
+            bool  taken[NE];
+#pragma unroll
+            for (int q = 0; q < NE; ++q) {
+                const int e = q * 64 + lane;
+                taken[q]    = e >= E;
+                z[q]        = e < E ? logits[(size_t)t * ld + e] : -INFINITY;
+                mx          = fmaxf(mx, z[q]);
+            }
+            mx = group_max<64>(mx);
+#pragma unroll
+            for (int q = 0; q < NE; ++q) {
+                den += taken[q] ? 0.f : expf(z[q] - mx);
+            }
+            den = group_sum<64>(den);
+            for (int j = 0; j < k; ++j) {
+                float v = 0.f;
+                int   i = 0x7fffffff;
+#pragma unroll
+                for (int q = 0; q < NE; ++q) {
+                    if (!taken[q] && (i == 0x7fffffff || z[q] > v)) {
+                        v = z[q], i = q * 64 + lane;
+                    }
+                }
+                wave_argmax(v, i);
+                i = __builtin_amdgcn_readfirstlane(i);
+#pragma unroll
+                for (int q = 0; q < NE; ++q) {
+                    taken[q] = taken[q] || q * 64 + lane == i;
+                }
+                if (lane == 0) {
+                    topk_ids[(size_t)t * k + j] = i;
+                    w[(size_t)t * k + j]        = scale * (expf(v - mx) / den);
+                    atomicOr(&mask[i], 1ull << t);
                 }
             }
-            taken |= 1ull << best;
-            ids[j] = best;
-            val[j] = bv;
         }
-        float denom = 0.f;
-        if (norm_topk) {
-            for (int j = 0; j < k; ++j) {
-                denom += __builtin_expf(val[j] - mx);
-            }
+    }
+    else {
+        for (int p = tid; p < T * k; p += 1024) {
+            atomicOr(&mask[topk_ids[p]], 1ull << (p / k));
         }
-        else {
-            for (int e = 0; e < E; ++e) {
-                denom += __builtin_expf(logit[e] - mx);
-            }
+    }
+    __syncthreads();
+    if (wave == 0) {
+        int n[NE], sum = 0;
+#pragma unroll
+        for (int q = 0; q < NE; ++q) {
+            n[q] = __popcll(mask[lane * NE + q]);
+            sum += n[q];
         }
-        const float inv = 1.0f / denom;
-        for (int j = 0; j < k; ++j) {
-            topk_ids[(size_t)t * k + j] = ids[j];
-            topk_w[(size_t)t * k + j]   = __builtin_expf(val[j] - mx) * inv * routed_scale;
+        int x = sum;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int y = __shfl_up(x, d);
+            x += lane >= d ? y : 0;
         }
+        x -= sum;
+#pragma unroll
+        for (int q = 0; q < NE; ++q) {
+            first[lane * NE + q] = x;
+            x += n[q];
+        }
+    }
+    __syncthreads();
+    if (tid <= E) {
+        offsets[tid] = tid < E ? first[tid] : T * k;
+    }
+    for (int p = tid; p < T * k; p += 1024) {
+        const int t = p / k, e = topk_ids[p], f = first[e] + __popcll(mask[e] & ((1ull << t) - 1));
+        f2n[f]                          = t;
+        en2f[(size_t)(p - t * k) * T + t] = f;
     }
 }
 
@@ -198,14 +307,24 @@ int launch_moe_gate(int* topk_ids, float* topk_w, float* logits_out, const half_
     if (T == 0) {
         return 0;
     }
-    moe_gate_kernel<<<T, 256, 0, st>>>(topk_ids, topk_w, logits_out, x, ldx, wg, H, E, k, norm_topk ? 1 : 0, routed_scale);
+    if (E % 8 == 0 && (uintptr_t)wg % 16 == 0) {
+        moe_gate_kernel<8><<<T, 256, 0, st>>>(topk_ids, topk_w, logits_out, x, ldx, wg, H, E, k, norm_topk ? 1 : 0, routed_scale);
+    }
+    else {
+        moe_gate_kernel<1><<<T, 256, 0, st>>>(topk_ids, topk_w, logits_out, x, ldx, wg, H, E, k, norm_topk ? 1 : 0, routed_scale);
+    }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }
 
 int launch_moe_route(int* offsets, int* f2n, int* en2f, const int* topk_ids, int T, int E, int k, hipStream_t st)
 {
-    moe_route_kernel<<<1, 1024, 0, st>>>(offsets, f2n, en2f, topk_ids, T, E, k);
+    if (T <= kRouteTokens && E <= kRouteExperts) {
+        moe_route_masks_kernel<false><<<1, 1024, 0, st>>>(offsets, f2n, en2f, (int*)topk_ids, nullptr, nullptr, 0, T, E, k, 0.f);
+    }
+    else {
+        moe_route_kernel<<<1, 1024, 0, st>>>(offsets, f2n, en2f, topk_ids, T, E, k);
+    }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }
@@ -413,31 +532,25 @@ __global__ void moe_topk_softmax_kernel(int* __restrict__ ids, float* __restrict
     }
 }
 
-int launch_moe_topk_softmax(int* ids, float* w, const float* logits, int ld, int T, int E, int k, float scale, hipStream_t st)
+int launch_moe_softmax_route(int* ids, float* w, int* offsets, int* f2n, int* en2f, const float* logits, int ld, int T, int E, int k, float scale,
+                             hipStream_t st)
 {
     TM_REQUIRE(ids && w && logits && E >= 1 && k >= 1 && k <= E && ld >= E, "moe top-k: operands");
     if (T == 0) {
+        return launch_moe_route(offsets, f2n, en2f, ids, T, E, k, st);
+    }
+    if (T <= kRouteTokens && E <= kRouteExperts) {
+        moe_route_masks_kernel<true><<<1, 1024, 0, st>>>(offsets, f2n, en2f, ids, w, logits, ld, T, E, k, scale);
+        TM_HIP_CHECK(hipGetLastError());
         return 0;
     }
     moe_topk_softmax_kernel<<<(T + 63) / 64, 64, 0, st>>>(ids, w, logits, ld, T, E, k, scale);
     TM_HIP_CHECK(hipGetLastError());
-    return 0;
+    return launch_moe_route(offsets, f2n, en2f, ids, T, E, k, st);
 }
 
 // Grouped router, one wave per token (four tokens per workgroup): the choice scores of a token lie in LDS, the lanes share the searches.
 constexpr int kGroupedMaxExperts = 1024, kGroupedMaxGroups = 256;
-
-__device__ __forceinline__ void wave_argmax(float& v, int& i)  // the largest v, the lower index on a tie (i = INT_MAX: no candidate)
-{
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const float ov = __shfl_xor(v, d);
-        const int   oi = __shfl_xor(i, d);
-        if (oi != 0x7fffffff && (i == 0x7fffffff || ov > v || (ov == v && oi < i))) {
-            v = ov, i = oi;
-        }
-    }
-}
 
 __global__ __launch_bounds__(256) void moe_topk_grouped_kernel(int* __restrict__ ids, float* __restrict__ w, const float* __restrict__ logits, int ld,
                                                                const float* __restrict__ corr, int T, int E, int groups, int keep, int k, int renorm)
@@ -535,27 +648,49 @@ int launch_moe_topk_grouped(int* ids, float* w, const float* logits, int ld, con
     return 0;
 }
 
-// rows sorted by expert: xs[en2f[j][t]] = (scale ? w[t][j] : 1) * x[t] -- the weight on the expert's INPUT
-template<class T>
+// rows sorted by expert: xs[en2f[j][t]] = (scale ? w[t][j] : 1) * x[t] -- the weight on the expert's INPUT; V neighbouring channels a thread
+template<class T, int V>
 __global__ __launch_bounds__(256) void moe_gather_kernel(T* __restrict__ xs, int lds, const T* __restrict__ x, int ldx, const float* __restrict__ w,
                                                          const int* __restrict__ en2f, int Tn, int H, int k, int scale, int* __restrict__ shared_offsets,
                                                          int E)
 {
+    typedef T TV __attribute__((ext_vector_type(V)));
     const int kk = k + (shared_offsets ? 1 : 0);
     const int t = blockIdx.x / kk, j = blockIdx.x % kk;
     if (j == k) {  // the copy behind the routed rows
         if (t == 0 && threadIdx.x == 0) {
             shared_offsets[E + 1] = Tn * kk;
         }
-        for (int i = threadIdx.x; i < H; i += 256) {
-            xs[((size_t)Tn * k + t) * lds + i] = x[(size_t)t * ldx + i];
+        for (int i = threadIdx.x * V; i < H; i += 256 * V) {
+            *(TV*)(xs + ((size_t)Tn * k + t) * lds + i) = *(const TV*)(x + (size_t)t * ldx + i);
         }
         return;
     }
     const int f = en2f[(size_t)j * Tn + t];
     const float a = scale ? w[(size_t)t * k + j] : 1.f;
-    for (int i = threadIdx.x; i < H; i += 256) {
-        xs[(size_t)f * lds + i] = (T)(a * (float)x[(size_t)t * ldx + i]);
+    for (int i = threadIdx.x * V; i < H; i += 256 * V) {
+        TV v = *(const TV*)(x + (size_t)t * ldx + i);
+        if (scale) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                v[e] = (T)(a * (float)v[e]);
+            }
+        }
+        *(TV*)(xs + (size_t)f * lds + i) = v;
+    }
+}
+
+template<class T>
+static void launch_moe_gather_t(T* xs, int lds, const T* x, int ldx, const float* w, const int* en2f, int Tn, int H, int k, bool scale, int* shared_offsets,
+                                int E, hipStream_t st)
+{
+    constexpr int V = 16 / sizeof(T);
+    const int     wgs = Tn * (k + (shared_offsets ? 1 : 0));
+    if (H % V == 0 && lds % V == 0 && ldx % V == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)xs % 16 == 0) {
+        moe_gather_kernel<T, V><<<wgs, 256, 0, st>>>(xs, lds, x, ldx, w, en2f, Tn, H, k, scale, shared_offsets, E);
+    }
+    else {
+        moe_gather_kernel<T, 1><<<wgs, 256, 0, st>>>(xs, lds, x, ldx, w, en2f, Tn, H, k, scale, shared_offsets, E);
     }
 }
 
@@ -566,12 +701,11 @@ int launch_moe_gather(void* xs, int lds, const void* x, int ldx, int elem_bytes,
     if (T == 0) {
         return 0;
     }
-    const int wgs = T * (k + (shared_offsets ? 1 : 0));
     if (elem_bytes == 2) {
-        moe_gather_kernel<__bf16><<<wgs, 256, 0, st>>>((__bf16*)xs, lds, (const __bf16*)x, ldx, w, en2f, T, H, k, scale, shared_offsets, E);
+        launch_moe_gather_t((__bf16*)xs, lds, (const __bf16*)x, ldx, w, en2f, T, H, k, scale, shared_offsets, E, st);
     }
     else {
-        moe_gather_kernel<float><<<wgs, 256, 0, st>>>((float*)xs, lds, (const float*)x, ldx, w, en2f, T, H, k, scale, shared_offsets, E);
+        launch_moe_gather_t((float*)xs, lds, (const float*)x, ldx, w, en2f, T, H, k, scale, shared_offsets, E, st);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
@@ -591,9 +725,15 @@ __global__ void moe_combine_f32_kernel(float* __restrict__ resid, const float* _
     }
     const int t = (int)(i / H), c = (int)(i % H);
     VF        s = 0.f;
-    for (int j = 0; j < k; ++j) {
-        const VF v = *(const VF*)(y + (size_t)en2f[(size_t)j * Tn + t] * H + c);
-        s += weighted ? w[(size_t)t * k + j] * v : v;
+    for (int j = 0; j < k; j += 2) {  // two rows in flight
+        const int   j1 = min(j + 1, k - 1);
+        const int   f0 = en2f[(size_t)j * Tn + t], f1 = en2f[(size_t)j1 * Tn + t];
+        const float w0 = weighted ? w[(size_t)t * k + j] : 1.f, w1 = weighted ? w[(size_t)t * k + j1] : 1.f;
+        const VF    v0 = *(const VF*)(y + (size_t)f0 * H + c), v1 = *(const VF*)(y + (size_t)f1 * H + c);
+        s += w0 * v0;
+        if (j + 1 < k) {
+            s += w1 * v1;
+        }
     }
     if (gate) {
 #pragma unroll
@@ -623,19 +763,6 @@ int launch_moe_combine_f32(float* resid, const float* y, const float* w, const i
     else {
         moe_combine_f32_kernel<1><<<(total + 255) / 256, 256, 0, st>>>(resid, y, w, en2f, gate, ldg, gate_bias, T, H, k, weighted, overwrite, add, add_gate, ld_add_gate);
     }
-    TM_HIP_CHECK(hipGetLastError());
-    return 0;
-}
-
-__global__ void moe_extend_offsets_kernel(int* offsets, int n, int extra)
-{
-    offsets[n + 1] = offsets[n] + extra;
-}
-
-int launch_moe_extend_offsets(int* offsets, int n, int extra, hipStream_t st)
-{
-    TM_REQUIRE(offsets && n >= 0 && extra >= 0, "moe offsets: operands");
-    moe_extend_offsets_kernel<<<1, 1, 0, st>>>(offsets, n, extra);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }

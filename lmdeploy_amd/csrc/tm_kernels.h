@@ -546,8 +546,9 @@ int launch_latent_prep(const float* proj, int ld, const LatentPrep& a, const Gen
 int launch_concat2(void* out, int ldo, int out_elem_bytes, const float* a, const float* b, int M, int H, hipStream_t st);
 // mixture of experts on the fp32 stream: sigmoid router top-k from fp32 logits; gather (optionally scaled) rows in expert order; gated sum
 int launch_moe_topk_sigmoid(int* ids, float* w, const float* logits, int ld, int T, int E, int k, hipStream_t st);
-// soft-max over all E logits; the k largest scores win (ties: the lower index); w = scale * score (not renormalised)
-int launch_moe_topk_softmax(int* ids, float* w, const float* logits, int ld, int T, int E, int k, float scale, hipStream_t st);
+// soft-max over all E logits; the k largest scores win (ties: the lower index); w = scale * score (not renormalised); and the routing tables
+int launch_moe_softmax_route(int* ids, float* w, int* offsets, int* f2n, int* en2f, const float* logits, int ld, int T, int E, int k, float scale,
+                             hipStream_t st);
 // scores s = sigmoid(logit); experts are ordered by s + correction[e] (nullptr: by s) and come from the `keep` best of `groups` equal groups of
 // neighbours, a group counting the sum of its two best (ties: the lower index); w = the chosen s, divided by their sum + 1e-20 with renorm
 int launch_moe_topk_grouped(int* ids, float* w, const float* logits, int ld, const float* correction, int T, int E, int groups, int keep, int k,
@@ -560,8 +561,6 @@ int launch_moe_combine_f32(float* resid, const float* y, const float* w, const i
                            int H, int k, bool weighted, hipStream_t st, bool overwrite = false /* resid = sum instead of resid += sum */,
                            const float* add = nullptr /* overwrite: resid = add + sum ([T][H]) */,
                            const float* add_gate = nullptr /* ... add[t] times sigmoid(add_gate[t * ld_add_gate]) */, int ld_add_gate = 0);
-// offsets[n + 1] = offsets[n] + extra: one more item behind the n items of a routing table (rows that every token sends)
-int launch_moe_extend_offsets(int* offsets, int n, int extra, hipStream_t st);
 // layer norm with bias on the fp32 stream.  launch_layernorm_f32: y[m] = LN(x[rows ? rows[m] : m]) (bf16 | fp32 [M][ldy]);
 // launch_layernorm_add_f32: x[m] += LN(r[m]), and the updated row also goes to h [M][ldh] in the activation type (the next sublayer's
 // GEMM operand).  LN(v) = (v - mean) / sqrt(mean((v - mean)^2) + eps) * w + b, two passes over the row in fp32
