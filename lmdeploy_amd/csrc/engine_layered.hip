@@ -931,6 +931,9 @@ int layered_start(tm_engine* e)
             lm.blocks_floats = std::max(lm.blocks_floats, parallel ? decay_workspace_floats((int)T, B, L.spec.r_heads, L.spec.r_dim)
                                                                    : decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim));
         }
+        if (L.post && L.spec.mixer == TM_MIXER_LIGHTNING) {
+            lm.blocks_floats = std::max(lm.blocks_floats, decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim));
+        }
         if (L.post || L.both) {
             max_cat  = std::max(max_cat, L.wo.Kp);
             max_proj = std::max(max_proj, std::max(L.qkv.N, L.spec.experts + 1));
@@ -1011,12 +1014,14 @@ int layered_start(tm_engine* e)
             TM_TRY(lm_alloc(&lm.d_gate2, T * lm.ldmix, st));
         }
     }
+    if (lm.blocks_floats > 0) {
+        TM_TRY(lm_alloc(&lm.d_blocks, lm.blocks_floats, st));
+    }
     if (lm.has_both) {
         lm.ldmix  = std::max(4, (max_mix + 3) / 4 * 4);
         lm.ldlora = std::max(32, max_lora);
         TM_TRY(lm_alloc(&lm.d_y, T * m.width, st));
         TM_TRY(lm_alloc(&lm.d_mixo, T * lm.ldmix, st));
-        TM_TRY(lm_alloc(&lm.d_blocks, lm.blocks_floats, st));
         if (lm.ldmixin > 0) {
             TM_TRY(lm_alloc((char**)&lm.d_mix, T * lm.ldmixin * lm.elem, st));
             TM_TRY(lm_alloc(&lm.d_hf, T * m.width, st));
@@ -1035,9 +1040,6 @@ int layered_start(tm_engine* e)
         if (max_mix > 0) {
             lm.ldmix = (max_mix + 3) / 4 * 4;
             TM_TRY(lm_alloc(&lm.d_mixo, T * lm.ldmix, st));
-        }
-        if (lm.blocks_floats > 0) {
-            TM_TRY(lm_alloc(&lm.d_blocks, lm.blocks_floats, st));
         }
         if (lm.ldcq > 0) {
             TM_TRY(lm_alloc((char**)&lm.d_cq, T * lm.ldcq * lm.elem, st));
@@ -1540,6 +1542,7 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
             sp.decay_w = lm.d_wdec + (size_t)P.row0 * lm.ldmix, sp.ld_w = lm.ldmix;
             sp.unit    = lm.d_aux + (size_t)P.row0 * lm.ldmix, sp.ld_u = lm.ldmix;
             sp.out     = lm.d_mixo + (size_t)P.row0 * lm.ldmix, sp.ldo = lm.ldmix;
+            sp.rows = P.rows, sp.blocks = lm.d_blocks, sp.blocks_floats = lm.blocks_floats;
             TM_PROF(P_ATTN, TM_TRY(launch_state_mix(sp, delta ? kStateDelta : kStateLinear, st)));
         }
         TM_PROF(P_ATTN, TM_TRY(launch_gated_group_norm(lm.d_cat, lm.ldcat, lm.elem, lm.d_mixo, lm.ldmix, L.mix_norm, lm.d_proj + L.c_g, lm.ldproj, M,

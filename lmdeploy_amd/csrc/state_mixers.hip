@@ -24,12 +24,8 @@
 // vectors (q, k, and w, a u, u for the delta rule), loaded TB tokens at a time: the next stage's global loads are issued before the
 // current stage's tokens are walked and land in the other LDS buffer afterwards, so their latency hides under the recurrence.  A slab is
 // stored as the wave holds it, [ii][column of the pair][lane]: loading and storing it are fully coalesced.
-// The delta rule walks its tokens one by one (two dependent reductions per token).  Linear attention with its scalar decay takes a whole
-// stage of T <= TB tokens at once, which replaces T dependent steps by independent sums:
-//   o_t = decay^(t+1) S0^T q_t + sum_{j <= t} decay^(t-j) (q_t . k_j) v_j          S_T = decay^T S0 + sum_j decay^(T-1-j) k_j v_j^T
-// -- the pair products (q_t . k_j) decay^(t-j) are formed once per workgroup (one thread per pair) and shared by all columns.
-// The forget-gate mixer, retention and the bonus recurrence take this kernel for decoded tokens; their prompt portions run in chunks on the
-// matrix cores (below).
+// The delta rule walks its tokens one by one (two dependent reductions per token); the other mixers take this kernel for decoded tokens, their prompt
+// portions run in chunks on the matrix cores (below).
 // One kernel serves prompt portions (many rows per sequence) and decoded tokens (one row, TB = 1): the state traffic of a decode step,
 // 2 * dim * vdim * 4 bytes per head, is what bounds it.
 #include "tm_kernels.h"
@@ -75,7 +71,7 @@ size_t state_mix_floats(int heads, int dim, int vdim)
     return (size_t)heads * ((vdim + wcols - 1) / wcols) * ((dim + 7) / 8) * 64 * kStateNC;
 }
 
-// grid (nseq, heads, ceil(vdim / 64)), 256 threads, dynamic LDS = 2 * tb * (NV * dim + 64) floats (+ TB * TB for linear attention); NV = 2 ... 5
+// grid (nseq, heads, ceil(vdim / 64)), 256 threads, dynamic LDS = 2 * tb * (NV * dim + 64) floats; NV = 2 ... 5
 // staged vectors per token, tb = min(TB, max_q_len) tokens per stage, TB: as many as keep the buffers under 64 KB.
 // EXACT: dim == 8 * DQ -- every LDS stride is a compile-time constant and the per-token vectors are read 16 bytes at a time
 template<int DQ, int KIND, int TB, bool EXACT>
@@ -87,7 +83,6 @@ __global__ __launch_bounds__(256) void state_mix_kernel(StateMixParams p)
     constexpr int NV = state_vectors(KIND), CW = kStateCW, NC = kStateNC, RG = 64 / CW, WV = CW * NC, WC = 4 * WV;
     constexpr int PER  = (TB * DQ * RG + 255) / 256;  // staged elements per vector and thread (dim <= DQ * RG)
     constexpr int VPER = (TB * WC + 255) / 256;
-    static_assert(TB * TB <= 256, "one thread per token pair");
     const int s = blockIdx.x, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int D = EXACT ? DQ * RG : p.dim, V = p.vdim, dq = EXACT ? DQ : (D + RG - 1) / RG, ncb = (V + WV - 1) / WV;
     const int Dp = dq * RG;  // staged vectors are padded to the row groups' share (zeros behind dim)
@@ -188,20 +183,6 @@ __global__ __launch_bounds__(256) void state_mix_kernel(StateMixParams p)
             }
         }
     };
-    // linear attention: powers of the decay, and this thread's pair (t, j) of the stage's token-by-token products
-    float     pwr[TB + 1], pair_pow = 1.f;
-    const int pt = threadIdx.x / TB, pj = threadIdx.x % TB;
-    float*    Pm = lds_all + 2 * stage;  // [TB][TB] (q_t . k_j) decay^(t - j), zero where j > t or t is not in the stage
-    if constexpr (LINEAR) {
-        pwr[0] = 1.f;
-#pragma unroll
-        for (int n = 1; n <= TB; ++n) {
-            pwr[n] = pwr[n - 1] * decay;
-        }
-        for (int n = 0; pt < TB && n < pt - pj; ++n) {
-            pair_pow *= decay;
-        }
-    }
     auto reduce_rg = [&](float a) {
         a += __shfl_xor(a, 8);
         a += __shfl_xor(a, 16);
@@ -228,178 +209,56 @@ __global__ __launch_bounds__(256) void state_mix_kernel(StateMixParams p)
         }
         const float* lds = lds_all + buf * stage;
         const float* sv  = lds + (size_t)tb * NV * Dp + wave * WV + c * NC;  // the lane's columns of token t at sv[t * WC + n]
-        if constexpr (LINEAR) {
-            if (threadIdx.x < TB * TB) {
-                float dot = 0.f;
-                if (pt < nt && pj <= pt) {
-                    const float* qt = lds + (size_t)(pt * NV + 0) * Dp;
-                    const float* kj = lds + (size_t)(pj * NV + 1) * Dp;
-                    // (every thread starts at another channel: the threads of a wave read different LDS banks)
-                    if constexpr (EXACT) {
-                        for (int d4 = 0; d4 < Dp / 4; ++d4) {
-                            const int     i = ((d4 + pj) % (Dp / 4)) * 4;
-                            const floatx4 a = *(const floatx4*)(qt + i), b = *(const floatx4*)(kj + i);
-                            dot = fmaf(a[0], b[0], fmaf(a[1], b[1], fmaf(a[2], b[2], fmaf(a[3], b[3], dot))));
-                        }
-                    }
-                    else {
-                        for (int d = 0; d < Dp; ++d) {
-                            const int i = (d + pj) % Dp;
-                            dot         = fmaf(qt[i], kj[i], dot);
-                        }
-                    }
-                    dot *= pair_pow;
-                }
-                Pm[pt * TB + pj] = dot;
+        for (int t = 0; wave_on && t < nt; ++t) {
+            const float* q  = lds + (size_t)(t * NV + 0) * Dp + rg * dq;
+            const float* k  = lds + (size_t)(t * NV + 1) * Dp + rg * dq;
+            const float* w  = lds + (size_t)(t * NV + (LINEAR || RETAIN ? 0 : 2)) * Dp + rg * dq;
+            const float* au = lds + (size_t)(t * NV + (DELTA || BONUS ? 3 : 0)) * Dp + rg * dq;  // a u, or bonus times key
+            const float* u  = lds + (size_t)(t * NV + (DELTA ? 4 : 0)) * Dp + rg * dq;
+            float        v[NC], us[NC], acc[NC];
+#pragma unroll
+            for (int n = 0; n < NC; ++n) {
+                v[n]  = sv[t * WC + n];
+                us[n] = acc[n] = 0.f;
             }
-            __syncthreads();
-            if (wave_on) {
-                float acc[TB][NC];
-#pragma unroll
-                for (int t = 0; t < TB; ++t) {  // what the old state answers to every query of the stage
-#pragma unroll
-                    for (int n = 0; n < NC; ++n) {
-                        acc[t][n] = 0.f;
-                    }
-                    if (t < nt) {
-                        const float* q = lds + (size_t)(t * NV + 0) * Dp + rg * dq;
-#pragma unroll
-                        for (int ii = 0; ii < DQ; ++ii) {
-                            if (EXACT || ii < dq) {
-                                const float qv = q[ii];
-#pragma unroll
-                                for (int n = 0; n < NC; ++n) {
-                                    acc[t][n] = fmaf(S[ii][n], qv, acc[t][n]);
-                                }
-                            }
-                        }
-#pragma unroll
-                        for (int n = 0; n < NC; ++n) {
-                            acc[t][n] *= pwr[t + 1];
-                        }
-                    }
-                }
-#pragma unroll
-                for (int m = 0; m < (TB + RG - 1) / RG; ++m) {  // the stage's own tokens: row group rg adds tokens rg, rg + 8, ...
-                    const int jt = rg + RG * m;
-                    if (jt < TB) {
-                        float vj[NC];
-#pragma unroll
-                        for (int n = 0; n < NC; ++n) {
-                            vj[n] = jt < nt ? sv[jt * WC + n] : 0.f;
-                        }
-#pragma unroll
-                        for (int t = 0; t < TB; ++t) {
-                            const float pw = Pm[t * TB + jt];
-#pragma unroll
-                            for (int n = 0; n < NC; ++n) {
-                                acc[t][n] = fmaf(pw, vj[n], acc[t][n]);
-                            }
-                        }
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < TB; ++t) {
-                    if (t < nt) {
-                        float o[NC];
-#pragma unroll
-                        for (int n = 0; n < NC; ++n) {
-                            o[n] = reduce_rg(acc[t][n]);
-                        }
-                        if ((t & (RG - 1)) == rg) {
-                            store_out(t0 + t, o);
-                        }
-                    }
-                }
-                float dn = 1.f;
-#pragma unroll
-                for (int t = 0; t < TB; ++t) {
-                    dn *= t < nt ? decay : 1.f;
-                }
+            if constexpr (DELTA) {
 #pragma unroll
                 for (int ii = 0; ii < DQ; ++ii) {
-#pragma unroll
-                    for (int n = 0; n < NC; ++n) {
-                        S[ii][n] *= dn;
-                    }
-                }
-                float wgt = 1.f;  // decay^(nt - 1 - token)
-#pragma unroll
-                for (int t = TB - 1; t >= 0; --t) {
-                    if (t < nt) {
-                        const float* k = lds + (size_t)(t * NV + 1) * Dp + rg * dq;
-                        float        wv[NC];
+                    if (EXACT || ii < dq) {  // (rows behind dim meet staged zeros and stay zero)
+                        const float uv = u[ii];
 #pragma unroll
                         for (int n = 0; n < NC; ++n) {
-                            wv[n] = wgt * sv[t * WC + n];
-                        }
-#pragma unroll
-                        for (int ii = 0; ii < DQ; ++ii) {
-                            if (EXACT || ii < dq) {
-                                const float kv = k[ii];
-#pragma unroll
-                                for (int n = 0; n < NC; ++n) {
-                                    S[ii][n] = fmaf(kv, wv[n], S[ii][n]);
-                                }
-                            }
-                        }
-                        wgt *= decay;
-                    }
-                }
-            }
-        }
-        else {
-            for (int t = 0; wave_on && t < nt; ++t) {
-                const float* q  = lds + (size_t)(t * NV + 0) * Dp + rg * dq;
-                const float* k  = lds + (size_t)(t * NV + 1) * Dp + rg * dq;
-                const float* w  = lds + (size_t)(t * NV + (RETAIN ? 0 : 2)) * Dp + rg * dq;
-                const float* au = lds + (size_t)(t * NV + (DELTA || BONUS ? 3 : 0)) * Dp + rg * dq;  // a u, or bonus times key
-                const float* u  = lds + (size_t)(t * NV + (DELTA ? 4 : 0)) * Dp + rg * dq;
-                float        v[NC], us[NC], acc[NC];
-#pragma unroll
-                for (int n = 0; n < NC; ++n) {
-                    v[n]  = sv[t * WC + n];
-                    us[n] = acc[n] = 0.f;
-                }
-                if constexpr (DELTA) {
-#pragma unroll
-                    for (int ii = 0; ii < DQ; ++ii) {
-                        if (EXACT || ii < dq) {  // (rows behind dim meet staged zeros and stay zero)
-                            const float uv = u[ii];
-#pragma unroll
-                            for (int n = 0; n < NC; ++n) {
-                                us[n] = fmaf(uv, S[ii][n], us[n]);
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int n = 0; n < NC; ++n) {
-                        us[n] = reduce_rg(us[n]);
-                    }
-                }
-#pragma unroll
-                for (int ii = 0; ii < DQ; ++ii) {
-                    if (EXACT || ii < dq) {
-                        const float wv = RETAIN ? decay : w[ii], av = au[ii], kv = k[ii], qv = q[ii];
-#pragma unroll
-                        for (int n = 0; n < NC; ++n) {
-                            if constexpr (BONUS) {
-                                acc[n]   = fmaf(fmaf(av, v[n], S[ii][n]), qv, acc[n]);
-                                S[ii][n] = fmaf(wv, S[ii][n], kv * v[n]);
-                                continue;
-                            }
-                            S[ii][n] = fmaf(wv, S[ii][n], DELTA ? fmaf(-av, us[n], kv * v[n]) : kv * v[n]);
-                            acc[n]   = fmaf(S[ii][n], qv, acc[n]);
+                            us[n] = fmaf(uv, S[ii][n], us[n]);
                         }
                     }
                 }
 #pragma unroll
                 for (int n = 0; n < NC; ++n) {
-                    acc[n] = reduce_rg(acc[n]);
+                    us[n] = reduce_rg(us[n]);
                 }
-                if (rg == (t & (RG - 1))) {
-                    store_out(t0 + t, acc);
+            }
+#pragma unroll
+            for (int ii = 0; ii < DQ; ++ii) {
+                if (EXACT || ii < dq) {
+                    const float wv = LINEAR || RETAIN ? decay : w[ii], av = au[ii], kv = k[ii], qv = q[ii];
+#pragma unroll
+                    for (int n = 0; n < NC; ++n) {
+                        if constexpr (BONUS) {
+                            acc[n]   = fmaf(fmaf(av, v[n], S[ii][n]), qv, acc[n]);
+                            S[ii][n] = fmaf(wv, S[ii][n], kv * v[n]);
+                            continue;
+                        }
+                        S[ii][n] = fmaf(wv, S[ii][n], DELTA ? fmaf(-av, us[n], kv * v[n]) : kv * v[n]);
+                        acc[n]   = fmaf(S[ii][n], qv, acc[n]);
+                    }
                 }
+            }
+#pragma unroll
+            for (int n = 0; n < NC; ++n) {
+                acc[n] = reduce_rg(acc[n]);
+            }
+            if (rg == (t & (RG - 1))) {
+                store_out(t0 + t, acc);
             }
         }
         if (more) {
@@ -424,8 +283,8 @@ template<int KIND>
 static void launch_state_dq(const StateMixParams& p, dim3 grid, hipStream_t st)
 {
     const int  dp  = (p.dim + 7) / 8 * 8;
-    constexpr bool DELTA = KIND == kStateDelta, LINEAR = KIND == kStateLinear, CHUNKS = !DELTA && !LINEAR;
-    auto       lds = [&](int tb) { return (2 * (size_t)tb * (state_vectors(KIND) * dp + 4 * kStateCW * kStateNC) + (LINEAR ? tb * tb : 0)) * sizeof(float); };
+    constexpr bool DELTA = KIND == kStateDelta;
+    auto       lds = [&](int tb) { return 2 * (size_t)tb * (state_vectors(KIND) * dp + 4 * kStateCW * kStateNC) * sizeof(float); };
     const bool one = p.max_q_len == 1;  // decoded tokens: one token per stage
 #define TM_STATE_LAUNCH_TB(DQ_, TB_)                                                     \
     if (p.dim == 8 * DQ_) {                                                              \
@@ -435,7 +294,7 @@ static void launch_state_dq(const StateMixParams& p, dim3 grid, hipStream_t st)
         state_mix_kernel<DQ_, KIND, TB_, false><<<grid, 256, lds(TB_), st>>>(p);        \
     }
 #define TM_STATE_LAUNCH(DQ_, TB_)                                             \
-    if constexpr (CHUNKS) { /* one token: portions take chunks */              \
+    if constexpr (!DELTA) { /* one token: portions take chunks */              \
         TM_STATE_LAUNCH_TB(DQ_, 1)                                            \
     }                                                                         \
     else if (one) {                                                           \
@@ -452,17 +311,19 @@ static void launch_state_dq(const StateMixParams& p, dim3 grid, hipStream_t st)
         TM_STATE_LAUNCH(8, 16)
     }
     else if (dq <= 16) {
-        TM_STATE_LAUNCH(16, (DELTA ? 8 : 16))
+        TM_STATE_LAUNCH(16, 8)
     }
     else {
-        TM_STATE_LAUNCH(32, (DELTA ? 4 : 8))
+        TM_STATE_LAUNCH(32, 4)
     }
 #undef TM_STATE_LAUNCH
 #undef TM_STATE_LAUNCH_TB
 }
 
 // ---- linear attention with decays over prompt portions: chunks of 16 tokens on the fp32 matrix cores -------------------------------------
-// Serves the forget-gate mixer (k = 1 - f), retention (f = the head's decay, q and k rotated as they are loaded) and the bonus recurrence.
+// Serves the forget-gate mixer (k = 1 - f), lightning attention (f = the head's decay; silu on q, k and v as they are loaded), retention (f = the head's
+// decay, q and k rotated as they are loaded) and the bonus recurrence.
+// 8 prompts of ~1000 tokens, 16 heads of 128 / 128, lightning: 84 + 186 us a layer; on the vector units (16 tokens at a time in LDS) 790.
 // Per chunk, head and key channel d, with t, j counting tokens of the chunk and P(a..b) = prod of f_s[d] for a <= s <= b:
 //   o_t = sum_d q_t P(0..t) S0[d] + sum_{j <= t} A[t][j] v_j,    A[t][j] = sum_d q_t k_j P(j+1..t)
 //   S   = P(0..15) S0 + sum_j k_j P(j+1..15) v_j^T
@@ -529,6 +390,11 @@ __global__ __launch_bounds__(256) void decay_blocks_kernel(StateMixParams p, int
                 const Rotation ro(p, p.k_len[s] - q_len + t0 + t, d);
                 q = ro(pr + p.c_q);
                 k = ro(pr + p.c_k) * p.k_mult;
+                f = p.decay_h[h];
+            }
+            else if constexpr (KIND == kStateLinear) {
+                q = sm_silu(pr[p.c_q]);
+                k = sm_silu(pr[p.c_k]);
                 f = p.decay_h[h];
             }
             else {
@@ -617,8 +483,8 @@ __global__ __launch_bounds__(256) void decay_blocks_kernel(StateMixParams p, int
     }
 }
 
-// grid (nseq, heads, ceil(vdim / 64)), 256 threads: wave -> 16 value columns
-template<int DR>
+// grid (nseq, heads, ceil(vdim / 64)), 256 threads: wave -> 16 value columns; SILU: on the values
+template<int DR, bool SILU>
 __global__ __launch_bounds__(256) void decay_chunks_kernel(StateMixParams p)
 {
     constexpr int NC = kStateNC, WV = kStateCW * kStateNC;
@@ -664,7 +530,13 @@ __global__ __launch_bounds__(256) void decay_chunks_kernel(StateMixParams p)
             o.v[e]      = p.proj[(size_t)(row0 + t) * p.ld + p.c_v + h * V + min(col, V - 1)];
         }
     };
-    auto step = [&](const Operands& o, int t0) {
+    auto step = [&](Operands& o, int t0) {
+        if constexpr (SILU) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o.v[e] = sm_silu(o.v[e]);
+            }
+        }
         floatx4 y0 = {0.f, 0.f, 0.f, 0.f}, y1 = y0;
 #pragma unroll
         for (int r = 0; r < DR; r += 2) {
@@ -745,7 +617,7 @@ static int launch_decay_chunks(const StateMixParams& p, hipStream_t st)
 #define TM_CHUNKS(DR_)                                                  \
     case DR_:                                                           \
         decay_blocks_kernel<DR_, KIND><<<gb, 256, 0, st>>>(p, chunks); \
-        decay_chunks_kernel<DR_><<<gc, 256, 0, st>>>(p);               \
+        decay_chunks_kernel<DR_, KIND == kStateLinear><<<gc, 256, 0, st>>>(p); \
         break;
     switch (decay_tiles(p.dim)) {
         TM_CHUNKS(2)
@@ -771,6 +643,9 @@ int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
     }
     TM_REQUIRE(kind != kStateRetention || (p.rot_dims >= 0 && p.rot_dims % 2 == 0 && p.rot_dims <= p.dim && (p.rot_dims == 0 || p.inv_freq)),
                "state mixer: rotation");
+    if (p.max_q_len > 1 && kind == kStateLinear) {
+        return launch_decay_chunks<kStateLinear>(p, st);
+    }
     if (p.max_q_len > 1 && kind == kStateForget) {
         return launch_decay_chunks<kStateForget>(p, st);
     }
