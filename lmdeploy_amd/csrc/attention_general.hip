@@ -75,6 +75,7 @@ __device__ __forceinline__ float ga_dot(const T* __restrict__ k, const float* __
     float acc = 0.f;
     if constexpr (sizeof(T) == 2) {
         if ((D & 7) == 0) {
+#pragma unroll 8
             for (int d = 0; d < D; d += 8) {
                 const bf16x8 v = *(const bf16x8*)(k + d);
 #pragma unroll
@@ -87,6 +88,7 @@ __device__ __forceinline__ float ga_dot(const T* __restrict__ k, const float* __
     }
     else {
         if ((D & 3) == 0) {
+#pragma unroll 8
             for (int d = 0; d < D; d += 4) {
                 const floatx4 v = *(const floatx4*)(k + d);
 #pragma unroll
@@ -188,10 +190,12 @@ __device__ __forceinline__ void ga_store4(const GeneralAttnParams& p, int t, int
     }
 }
 
-// grid (rows, ceil(q_heads / 4), splits), 256 threads: wave w -> head blockIdx.y * 4 + w
+// grid (rows, ceil(q_heads / 4), splits), 256 threads: wave w -> head blockIdx.y * 4 + w.  A chain of dependent loads bounds it at a few rows: eight pieces
+// of a key and four keys of a value channel are in flight at a time (3 rows of 16 heads over ~190 latent entries in fp32: 55 us with one of each, 31 so)
 template<class T, int VC>
 __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
 {
+    typedef T T4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
     __shared__ float qs[4][kGaMaxDim];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = blockIdx.x, h = blockIdx.y * 4 + wave, sp = blockIdx.z;
@@ -256,8 +260,9 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
                 o[c] *= alpha;
             }
             const int cnt = min(64, n - j0);
-            for (int jj = klo > 0 ? 0 : max(0, jlo - j0); jj < cnt; ++jj) {
-                const float w  = __shfl(pj, jj);
+            auto      wt  = [&](int jj) { return bit_cast<float>(__builtin_amdgcn_readlane(bit_cast<int>(pj), jj)); };
+            auto      one = [&](int jj) {
+                const float w  = wt(jj);
                 const T*    vr = vb + (j0 + jj);
 #pragma unroll
                 for (int c = 0; c < VC; ++c) {
@@ -266,6 +271,26 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
                         o[c] = fmaf(w, (float)vr[(size_t)v * p.block_len], o[c]);
                     }
                 }
+            };
+            int jj = klo > 0 ? 0 : max(0, jlo - j0);
+            for (; jj < cnt && (jj & 3); ++jj) {
+                one(jj);
+            }
+#pragma unroll 2
+            for (; jj + 4 <= cnt; jj += 4) {  // four keys of a channel a load
+                const float w0 = wt(jj), w1 = wt(jj + 1), w2 = wt(jj + 2), w3 = wt(jj + 3);
+                const T*    vr = vb + (j0 + jj);
+#pragma unroll
+                for (int c = 0; c < VC; ++c) {
+                    const int v = lane + 64 * c;
+                    if (v < V) {
+                        const T4 x = *(const T4*)(vr + (size_t)v * p.block_len);
+                        o[c]       = fmaf(w3, (float)x[3], fmaf(w2, (float)x[2], fmaf(w1, (float)x[1], fmaf(w0, (float)x[0], o[c]))));
+                    }
+                }
+            }
+            for (; jj < cnt; ++jj) {
+                one(jj);
             }
         }
     }
