@@ -323,7 +323,7 @@ static void launch_state_dq(const StateMixParams& p, dim3 grid, hipStream_t st)
 // ---- linear attention with decays over prompt portions: chunks of 16 tokens on the fp32 matrix cores -------------------------------------
 // Serves the forget-gate mixer (k = 1 - f), lightning attention (f = the head's decay; silu on q, k and v as they are loaded), retention (f = the head's
 // decay, q and k rotated as they are loaded) and the bonus recurrence.
-// 8 prompts of ~1000 tokens, 16 heads of 128 / 128, lightning: 84 + 186 us a layer; on the vector units (16 tokens at a time in LDS) 790.
+// 8 prompts of ~1000 tokens, 16 heads of 128 / 128, lightning: 84 + 190 us a layer; on the vector units (16 tokens at a time in LDS) 790.
 // Per chunk, head and key channel d, with t, j counting tokens of the chunk and P(a..b) = prod of f_s[d] for a <= s <= b:
 //   o_t = sum_d q_t P(0..t) S0[d] + sum_{j <= t} A[t][j] v_j,    A[t][j] = sum_d q_t k_j P(j+1..t)
 //   S   = P(0..15) S0 + sum_j k_j P(j+1..15) v_j^T
@@ -537,18 +537,21 @@ __global__ __launch_bounds__(256) void decay_chunks_kernel(StateMixParams p)
                 o.v[e] = sm_silu(o.v[e]);
             }
         }
-        floatx4 y0 = {0.f, 0.f, 0.f, 0.f}, y1 = y0;
+        floatx4 y[4], ya = {0.f, 0.f, 0.f, 0.f};  // short chains of sums: independent products for the matrix core and less rounding
 #pragma unroll
-        for (int r = 0; r < DR; r += 2) {
+        for (int i = 0; i < 4; ++i) {
+            y[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                y0 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[r][i], S[r][i], y0, 0, 0, 0);
-                y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[r + 1][i], S[r + 1][i], y1, 0, 0, 0);
+                y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[r][i], S[r][i], y[i], 0, 0, 0);
             }
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            y1 = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[e], o.v[e], y1, 0, 0, 0);
+            ya = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[e], o.v[e], ya, 0, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < DR; ++r) {
@@ -565,7 +568,7 @@ __global__ __launch_bounds__(256) void decay_chunks_kernel(StateMixParams p)
         for (int i = 0; i < 4; ++i) {
             const int t = t0 + g * 4 + i;
             if (t < q_len && col < V) {
-                p.out[(size_t)(row0 + t) * p.ldo + h * V + col] = y0[i] + y1[i];
+                p.out[(size_t)(row0 + t) * p.ldo + h * V + col] = ((y[0][i] + y[1][i]) + (y[2][i] + y[3][i])) + ya[i];
             }
         }
     };
