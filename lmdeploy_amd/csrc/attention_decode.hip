@@ -21,6 +21,7 @@
 //   * grid = (kv_heads * head_chunks, batch, splits) -> 512..2048 workgroups for the metric shape.
 #include "tm_common.h"
 #include "tm_kernels.h"
+#include "decode_merge.h"
 #include <stdlib.h>
 
 namespace tmk {
@@ -111,9 +112,13 @@ __global__ __launch_bounds__(256, 2) void decode_attention_kernel(DecodeAttnPara
 
     const int ctx        = p.k_len[b];
     const int tiles      = (ctx + TILE - 1) / TILE;
-    const int per_split  = (tiles + p.splits - 1) / p.splits;
+    const int per_split  = max((tiles + p.splits - 1) / p.splits, p.split_tiles);
     const int tile_begin = split * per_split;
     const int tile_end   = min(tile_begin + per_split, tiles);
+    const int nsplit     = max((tiles + per_split - 1) / per_split, 1);  // splits with keys: the others leave at once
+    if (split >= nsplit) {
+        return;
+    }
 
     // ---- queries: q[h][E dims of chunk c] as half2 pairs, kept in registers ------------------
     half2_t qv[HPW][E / 2];
@@ -284,6 +289,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_kernel(DecodeAttnPara
     // ---- reduce over the token lanes of the wave, then over the 4 waves through LDS -------------
     __shared__ float sm_o[4][HPW][D];
     __shared__ float sm_ml[4][HPW][2];
+    __shared__ unsigned sm_last;
 #pragma unroll
     for (int h = 0; h < HPW; ++h) {
         lsum[h] = group_sum<64>(lsum[h]);
@@ -321,40 +327,35 @@ __global__ __launch_bounds__(256, 2) void decode_attention_kernel(DecodeAttnPara
             l += wt * sm_ml[w][h][1];
         }
         const int hq = head0 + h;
-        if (p.splits == 1) {
+        if (nsplit == 1) {
             p.out[(size_t)b * p.q_heads * D + (size_t)hq * D + d] = (half_t)(o / l);
         }
         else {
-            const size_t slot                 = ((size_t)b * p.q_heads + hq) * p.splits + split;
-            p.partial_o[slot * D + d]         = o;
+            const size_t slot = ((size_t)b * p.q_heads + hq) * p.splits + split;
+            agent_store(p.partial_o + slot * D + d, o);
             if (d == 0) {
-                p.partial_ml[slot * 2]     = ms;
-                p.partial_ml[slot * 2 + 1] = l;
+                agent_store(p.partial_ml + slot * 2, ms);
+                agent_store(p.partial_ml + slot * 2 + 1, l);
             }
         }
     }
+    if (nsplit == 1 || !p.tickets || !ticket_last_workgroup(p.tickets + (size_t)b * p.q_heads + head0, nsplit, &sm_last)) {
+        return;
+    }
+    for (int idx = threadIdx.x; idx < HPW * D; idx += 256) {
+        const int h = idx / D;
+        decode_merge(p, b, head0 + h, idx - h * D, nsplit);
+    }
 }
 
-// split-K merge: one 128-thread workgroup per (sequence, query head)
+// split-K merge as a launch of its own, for callers without tickets: one 128-thread workgroup per (sequence, query head)
 __global__ __launch_bounds__(128) void decode_reduce_kernel(DecodeAttnParams p)
 {
-    constexpr int D    = 128;
-    const int     hq   = blockIdx.x;
-    const int     b    = blockIdx.y;
-    const int     d    = threadIdx.x;
-    const size_t  slot = ((size_t)b * p.q_heads + hq) * p.splits;
-    float         ms   = -INFINITY;
-    for (int s = 0; s < p.splits; ++s) {
-        ms = fmaxf(ms, p.partial_ml[(slot + s) * 2]);
+    const int b = blockIdx.y, tiles = (p.k_len[b] + p.tile_len - 1) / p.tile_len;
+    const int per = max((tiles + p.splits - 1) / p.splits, p.split_tiles), nsplit = (tiles + per - 1) / per;
+    if (nsplit > 1) {
+        decode_merge(p, b, blockIdx.x, threadIdx.x, nsplit);
     }
-    float o = 0.f, l = 0.f;
-    for (int s = 0; s < p.splits; ++s) {
-        const float mw = p.partial_ml[(slot + s) * 2];
-        const float wt = (mw == -INFINITY) ? 0.f : fast_exp2((mw - ms) * p.scale_log2);
-        o += wt * p.partial_o[(slot + s) * D + d];
-        l += wt * p.partial_ml[(slot + s) * 2 + 1];
-    }
-    p.out[(size_t)b * p.q_heads * D + (size_t)hq * D + d] = (half_t)(o / l);
 }
 
 size_t decode_attention_workspace_bytes(int batch, int q_heads, int head_dim, int splits)
@@ -362,10 +363,19 @@ size_t decode_attention_workspace_bytes(int batch, int q_heads, int head_dim, in
     return (size_t)batch * q_heads * splits * (head_dim + 2) * sizeof(float);
 }
 
-template<int BITS>
-static int launch_bits(const DecodeAttnParams& p, hipStream_t st)
+int launch_decode_reduce(const DecodeAttnParams& p, hipStream_t st)
 {
-    const int group = p.q_heads / p.cache.layout.kv_heads;
+    if (p.splits > 1 && !p.tickets) {
+        decode_reduce_kernel<<<dim3(p.q_heads, p.batch), 128, 0, st>>>(p);
+        TM_HIP_CHECK(hipGetLastError());
+    }
+    return 0;
+}
+
+template<int BITS>
+static int launch_bits(const DecodeAttnParams& p_in, hipStream_t st)
+{
+    const int group = p_in.q_heads / p_in.cache.layout.kv_heads;
     int       hpw   = 1;
     for (int cand = 4; cand >= 1; --cand) {
         if (group % cand == 0) {
@@ -373,8 +383,12 @@ static int launch_bits(const DecodeAttnParams& p, hipStream_t st)
             break;
         }
     }
-    const int chunks = group / hpw;
-    dim3      grid(p.cache.layout.kv_heads * chunks, p.batch, p.splits);
+    const int        chunks = group / hpw;
+    DecodeAttnParams p      = p_in;
+    dim3             grid(p.cache.layout.kv_heads * chunks, p.batch, p.splits);
+    p.tile_len           = KvTraits<BITS>::TILE;
+    p.split_tiles        = decode_split_tiles(grid.x * grid.y);
+    p.tickets            = p.ticket_count >= p.batch * p.q_heads ? p.tickets : nullptr;
     switch (hpw) {
         case 4:
             decode_attention_kernel<BITS, 4><<<grid, 256, 0, st>>>(p, chunks);
@@ -389,11 +403,7 @@ static int launch_bits(const DecodeAttnParams& p, hipStream_t st)
             decode_attention_kernel<BITS, 1><<<grid, 256, 0, st>>>(p, chunks);
     }
     TM_HIP_CHECK(hipGetLastError());
-    if (p.splits > 1) {
-        decode_reduce_kernel<<<dim3(p.q_heads, p.batch), 128, 0, st>>>(p);
-        TM_HIP_CHECK(hipGetLastError());
-    }
-    return 0;
+    return launch_decode_reduce(p, st);
 }
 
 int launch_decode_attention(const DecodeAttnParams& p, hipStream_t st)
@@ -418,16 +428,7 @@ int launch_decode_attention(const DecodeAttnParams& p, hipStream_t st)
             if (valu && !fused) {
                 return launch_bits<8>(p, st);
             }
-            DecodeAttnParams pt = p;
-            int rc = launch_decode_attention_i8_mfma(pt, st);
-            if (rc) {
-                return rc;
-            }
-            if (p.splits > 1) {
-                decode_reduce_kernel<<<dim3(p.q_heads, p.batch), 128, 0, st>>>(p);
-                TM_HIP_CHECK(hipGetLastError());
-            }
-            return 0;
+            return launch_decode_attention_i8_mfma(p, st);
         }
         case 4: {
             // int4 KV: the same MFMA kernel, nibbles expanded to bytes on the way into LDS (TM_ATTN_VALU=1: VALU kernel)
@@ -435,16 +436,7 @@ int launch_decode_attention(const DecodeAttnParams& p, hipStream_t st)
             if (valu4 && !fused) {
                 return launch_bits<4>(p, st);
             }
-            DecodeAttnParams pt = p;
-            int rc = launch_decode_attention_i8_mfma(pt, st);
-            if (rc) {
-                return rc;
-            }
-            if (p.splits > 1) {
-                decode_reduce_kernel<<<dim3(p.q_heads, p.batch), 128, 0, st>>>(p);
-                TM_HIP_CHECK(hipGetLastError());
-            }
-            return 0;
+            return launch_decode_attention_i8_mfma(p, st);
         }
     }
     TM_REQUIRE(false, "kv bits in {16,8,4}");

@@ -28,6 +28,7 @@
 // transpose-read simply addresses those rows.
 #include "tm_common.h"
 #include "tm_kernels.h"
+#include "decode_merge.h"
 #include <type_traits>
 
 namespace tmk {
@@ -148,7 +149,8 @@ __device__ __forceinline__ void expand_u4x32(u32x4 w, u32x4& a, u32x4& b)
 // BITS = 8: the cache bytes are the codes.  BITS = 4: the block is half as large in HBM; the nibbles are expanded to
 // one byte per code when the block is written to the wave's LDS image, everything after that is the int8 path
 // (scales / zeros are per token either way, quantization.h:316-366).
-template<bool FUSED, int BITS>
+// SPLIT: the keys are shared by p.splits workgroups; without, neither the divisions nor the merge are in the kernel
+template<bool FUSED, int BITS, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(DecodeAttnParams p, int head_chunks, int hpw)
 {
     static_assert(BITS == 8 || BITS == 4, "int8 / int4 KV");
@@ -199,9 +201,12 @@ __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(Decode
 
     const int ctx        = *(const CONST_AS int*)(p.k_len + b);
     const int tiles      = (ctx + 63) >> 6;
-    const int per_split  = (tiles + p.splits - 1) / p.splits;
-    const int tile_begin = split * per_split;
-    const int tile_end   = min(tile_begin + per_split, tiles);
+    const int per_split  = SPLIT ? max((tiles + p.splits - 1) / p.splits, p.split_tiles) : tiles;
+    const int tile_begin = SPLIT ? split * per_split : 0;
+    const int tile_end   = SPLIT ? min(tile_begin + per_split, tiles) : tiles;
+    if (SPLIT && split > 0 && tile_begin >= tiles) {
+        return;  // a split without keys
+    }
 
     // ---- q^T fragments (B operand of S^T = K q^T): lane (head = i16, g) holds q[head][32dd + 8g .. +8) -----------
     half8_t    qf[4];
@@ -561,6 +566,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(Decode
     }
     __syncthreads();
 
+    const int nsplit = SPLIT ? max((tiles + per_split - 1) / per_split, 1) : 1;
     for (int idx = threadIdx.x; idx < hpw * D; idx += 256) {
         const int h = idx / D;
         const int d = idx - h * D;
@@ -578,15 +584,23 @@ __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(Decode
             l += wt * sm_ml[(w * 16 + h) * 2 + 1];
         }
         const int hq = head0 + h;
-        if (p.splits == 1) {
+        if (nsplit == 1) {
             p.out[(size_t)b * p.q_heads * D + (size_t)hq * D + d] = (half_t)(o / l);
         }
         else {
-            const size_t slot         = ((size_t)b * p.q_heads + hq) * p.splits + split;
-            p.partial_o[slot * D + d] = o;
+            const size_t slot = ((size_t)b * p.q_heads + hq) * p.splits + split;
+            agent_store(p.partial_o + slot * D + d, o);
             if (d == 0) {
-                p.partial_ml[slot * 2]     = ms;
-                p.partial_ml[slot * 2 + 1] = l;
+                agent_store(p.partial_ml + slot * 2, ms);
+                agent_store(p.partial_ml + slot * 2 + 1, l);
+            }
+        }
+    }
+    if (nsplit > 1 && p.tickets) {  // (the flag's word lies behind the merge buffers)
+        if (ticket_last_workgroup(p.tickets + (size_t)b * p.q_heads + head0, nsplit, (unsigned*)(smem + 4 * 16 * D * 4 + 4 * 16 * 2 * 4))) {
+            for (int idx = threadIdx.x; idx < hpw * D; idx += 256) {
+                const int h = idx / D;
+                decode_merge(p, b, head0 + h, idx - h * D, nsplit);
             }
         }
     }
@@ -615,37 +629,32 @@ int launch_decode_attention_i8_mfma(const DecodeAttnParams& p_in, hipStream_t st
     // against this kernel's 34.4 at ctx 1040 -- four waves per CU issue the per-block arithmetic more slowly than eight
     // (profiles/r05_attention_pair_kernel.txt).
     dim3      grid(p.cache.layout.kv_heads * chunks, p.batch, p.splits);
+    p.tile_len    = 64;
+    p.split_tiles = decode_split_tiles(grid.x * grid.y);
+    p.tickets     = p.ticket_count >= p.batch * p.q_heads ? p.tickets : nullptr;
     p.dbg = gemm_trace_for((size_t)grid.x * grid.y * grid.z, "attn", grid.x, grid.y, grid.z);
     // 4 wave-private images (+ 4 KB q exchange for the fused prologue); the merge buffers overlay the images
     static_assert(4 * kWaveLds + 4096 > 4 * 16 * 128 * 4 + 4 * 16 * 2 * 4, "merge buffers must fit");
     const int lds = 4 * kWaveLds + 4096;
-    const void* const k = (p.qkv_slabs || p.qkv_f16) ?
-                              (p.cache.layout.bits == 4 ? (const void*)decode_attention_i8_mfma_kernel<true, 4> :
-                                                          (const void*)decode_attention_i8_mfma_kernel<true, 8>) :
-                              (p.cache.layout.bits == 4 ? (const void*)decode_attention_i8_mfma_kernel<false, 4> :
-                                                          (const void*)decode_attention_i8_mfma_kernel<false, 8>);
-    if (const int rc = ensure_dynamic_lds(k, lds)) {
+    const bool fused = p.qkv_slabs || p.qkv_f16;
+    TM_REQUIRE(!fused || (p.qkv_n % 8 == 0 && (p.qkv_splits == 0) == (p.qkv_slabs == nullptr)), "fused qkv input");
+    auto launch = [&](auto FUSED, auto BITS, auto SPLIT) {
+        constexpr auto k = decode_attention_i8_mfma_kernel<decltype(FUSED)::value, decltype(BITS)::value, decltype(SPLIT)::value>;
+        if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {
+            return rc;
+        }
+        k<<<grid, 256, lds, st>>>(p, chunks, hpw);
+        return 0;
+    };
+    auto by_split = [&](auto FUSED, auto BITS) { return p.splits > 1 ? launch(FUSED, BITS, std::true_type{}) : launch(FUSED, BITS, std::false_type{}); };
+    auto by_bits  = [&](auto FUSED) {
+        return p.cache.layout.bits == 4 ? by_split(FUSED, std::integral_constant<int, 4>{}) : by_split(FUSED, std::integral_constant<int, 8>{});
+    };
+    if (const int rc = fused ? by_bits(std::true_type{}) : by_bits(std::false_type{})) {
         return rc;
     }
-    if (p.qkv_slabs || p.qkv_f16) {
-        TM_REQUIRE(p.qkv_n % 8 == 0 && (p.qkv_splits == 0) == (p.qkv_slabs == nullptr), "fused qkv input");
-        if (p.cache.layout.bits == 4) {
-            decode_attention_i8_mfma_kernel<true, 4><<<grid, 256, lds, st>>>(p, chunks, hpw);
-        }
-        else {
-            decode_attention_i8_mfma_kernel<true, 8><<<grid, 256, lds, st>>>(p, chunks, hpw);
-        }
-    }
-    else {
-        if (p.cache.layout.bits == 4) {
-            decode_attention_i8_mfma_kernel<false, 4><<<grid, 256, lds, st>>>(p, chunks, hpw);
-        }
-        else {
-            decode_attention_i8_mfma_kernel<false, 8><<<grid, 256, lds, st>>>(p, chunks, hpw);
-        }
-    }
     TM_HIP_CHECK(hipGetLastError());
-    return 0;
+    return launch_decode_reduce(p, st);
 }
 
 }  // namespace tmk

@@ -28,6 +28,7 @@
 //                  (sequence, key head, key split), its four waves take every fourth cache block and merge at the end.
 // Cache block layout per layer: keys [kv_heads][64][dim], then values [kv_heads][vdim][64].
 #include "tm_kernels.h"
+#include "decode_merge.h"
 #include "gemm_stream.h"  // stream_dma16
 #include <algorithm>
 #include <stdlib.h>
@@ -190,6 +191,32 @@ __device__ __forceinline__ void ga_store4(const GeneralAttnParams& p, int t, int
     }
 }
 
+// C channels of head h of row t from the results of its key splits (+ the sink): channel(c), those below vdim
+template<class T, int C, class Channel>
+__device__ __forceinline__ void ga_merge(const GeneralAttnParams& p, int t, int h, int nsplit, Channel&& channel)
+{
+    const size_t slot = ((size_t)t * p.q_heads + h) * p.splits;
+    float        m = p.sink ? p.sink[h] : -1e30f, l = p.sink ? 1.f : 0.f, o[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        o[c] = 0.f;
+    }
+    merge_splits<C <= 4 ? 8 : 2>(p.partial_ml + slot * 2, [&](int s, int c) { return p.partial_o + (slot + s) * p.vdim + min(channel(c), p.vdim - 1); },
+                                 nsplit, 1.4426950408889634f, m, l, o);
+    const float inv = ga_out_gate(p, t, h) / l;
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        if (channel(c) < p.vdim) {
+            ga_store<T>(p, t, h, channel(c), o[c] * inv);
+        }
+    }
+}
+template<class T, int VC>
+__device__ __forceinline__ void ga_merge_row(const GeneralAttnParams& p, int t, int h, int nsplit)  // all channels, by one wave
+{
+    ga_merge<T, VC>(p, t, h, nsplit, [](int c) { return (int)(threadIdx.x & 63) + 64 * c; });
+}
+
 // grid (rows, ceil(q_heads / 4), splits), 256 threads: wave w -> head blockIdx.y * 4 + w.  A chain of dependent loads bounds it at a few rows: eight pieces
 // of a key and four keys of a value channel are in flight at a time (3 rows of 16 heads over ~190 latent entries in fp32: 55 us with one of each, 31 so)
 template<class T, int VC>
@@ -319,56 +346,26 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
     for (int c = 0; c < VC; ++c) {
         const int v = lane + 64 * c;
         if (v < V) {
-            po[v] = o[c];
+            agent_store(po + v, o[c]);
         }
     }
     if (lane == 0) {
-        pm[0] = m;
-        pm[1] = l;
+        agent_store(pm, m);
+        agent_store(pm + 1, l);
+    }
+    if (p.tickets && ticket_last_wave(p.tickets + (size_t)t * p.q_heads + h, nsplit)) {
+        ga_merge_row<T, VC>(p, t, h, nsplit);
     }
 }
 
-// merge of the key splits (+ the sink): grid (rows, q_heads), 64 threads
+// merge of the key splits as a launch of its own, for callers without tickets: grid (rows, q_heads), 64 threads
 template<class T, int VC>
 __global__ __launch_bounds__(64) void attn_rows_merge_kernel(GeneralAttnParams p)
 {
-    const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x, V = p.vdim;
-    const int pos = p.row_pos[t], first = ga_first_key(p, pos), bf = first / p.block_len;
+    const int pos = p.row_pos[blockIdx.x], first = ga_first_key(p, pos), bf = first / p.block_len;
     const int nsplit = ga_split_count(p, ga_keep_blocks(p, first, bf, p.block_len) + (pos + p.block_len) / p.block_len - bf);
-    if (nsplit == 1) {
-        return;
-    }
-    const float* pm = p.partial_ml + ((size_t)t * p.q_heads + h) * p.splits * 2;
-    const float* po = p.partial_o + ((size_t)t * p.q_heads + h) * p.splits * V;
-    float        mf = p.sink ? p.sink[h] : -1e30f;
-    for (int s = 0; s < nsplit; ++s) {
-        mf = fmaxf(mf, pm[s * 2]);
-    }
-    float l = p.sink ? __expf(p.sink[h] - mf) : 0.f;
-    float o[VC];
-#pragma unroll
-    for (int c = 0; c < VC; ++c) {
-        o[c] = 0.f;
-    }
-#pragma unroll 4
-    for (int s = 0; s < nsplit; ++s) {
-        const float a = __expf(pm[s * 2] - mf);
-        l += a * pm[s * 2 + 1];
-#pragma unroll
-        for (int c = 0; c < VC; ++c) {
-            const int v = lane + 64 * c;
-            if (v < V) {
-                o[c] = fmaf(a, po[(size_t)s * V + v], o[c]);
-            }
-        }
-    }
-    const float inv = ga_out_gate(p, t, h) / l;
-#pragma unroll
-    for (int c = 0; c < VC; ++c) {
-        const int v = lane + 64 * c;
-        if (v < V) {
-            ga_store<T>(p, t, h, v, o[c] * inv);
-        }
+    if (nsplit > 1) {
+        ga_merge_row<T, VC>(p, blockIdx.x, blockIdx.y, nsplit);
     }
 }
 
@@ -399,8 +396,15 @@ size_t general_attention_workspace_bytes(int rows, int q_heads, int vdim, int sp
     return (size_t)rows * q_heads * splits * (vdim + 2) * sizeof(float);
 }
 
-int launch_general_attention_rows(const GeneralAttnParams& p, hipStream_t st)
+static unsigned* ga_tickets(const GeneralAttnParams& p)  // one per (row, head), or the splits' results are merged by a launch of their own
 {
+    return p.ticket_count >= p.rows * p.q_heads ? p.tickets : nullptr;
+}
+
+int launch_general_attention_rows(const GeneralAttnParams& p_in, hipStream_t st)
+{
+    GeneralAttnParams p = p_in;
+    p.tickets           = ga_tickets(p_in);
     TM_REQUIRE(p.rows >= 0 && p.q_heads >= 1 && p.kv_heads >= 1 && p.q_heads % p.kv_heads == 0, "attention: head counts");
     TM_REQUIRE(p.dim >= 1 && p.dim <= kGaMaxDim && p.vdim >= 1 && p.vdim <= kGaMaxDim, "attention: 1 <= dim, vdim <= 1024");
     TM_REQUIRE(p.chunk >= 0 && (!p.dist_r1 || p.dist_r2) && (!p.out_gate || p.ld_gate >= p.q_heads), "attention: chunk / distance penalty / gate");
@@ -420,7 +424,7 @@ int launch_general_attention_rows(const GeneralAttnParams& p, hipStream_t st)
         launch_rows<float>(p, grid, st);
     }
     TM_HIP_CHECK(hipGetLastError());
-    if (p.splits > 1) {
+    if (p.splits > 1 && !p.tickets) {
         if (p.elem_bytes == 2) {
             launch_rows_merge<__bf16>(p, st);
         }
@@ -681,7 +685,8 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(GeneralAttnParams p, in
 template<int DS, int VT>
 __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, int chunks)
 {
-    __shared__ float ml_s[4][16][2];
+    __shared__ float    ml_s[4][16][2];
+    __shared__ unsigned last_s;
     __shared__ float o_s[3][16][VT * 16 + 4];  // + 4: the sixteen rows start in different banks
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = blockIdx.x, g = blockIdx.y / chunks, chunk = blockIdx.y % chunks, sp = blockIdx.z;
@@ -746,50 +751,65 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
         }
     }
     __syncthreads();
-    if (wave > 0 || !h_ok) {
-        return;
-    }
-    float lt = 0.f;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-        lt += ml_s[w][lr][1] * __expf(ml_s[w][lr][0] - mf);
-    }
-#pragma unroll
-    for (int v = 0; v < VT; ++v) {
-        const int c = v * 16 + lg * 4;
-        o[v]        = o[v] * a + ((*(const floatx4*)&o_s[0][lr][c] + *(const floatx4*)&o_s[1][lr][c]) + *(const floatx4*)&o_s[2][lr][c]);
-    }
-    if (nsplit == 1) {
-        float inv;
-        if (p.sink) {
-            const float sk = p.sink[h], m2 = fmaxf(mf, sk), a2 = __expf(mf - m2);
-            inv            = a2 / (lt * a2 + __expf(sk - m2));
+    const int nheads = min(16, group - chunk * 16);
+    if (wave > 0) {
+        if (nsplit == 1 || !p.tickets) {
+            return;
         }
-        else {
-            inv = 1.f / lt;
+    }
+    else {
+        float lt = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            lt += ml_s[w][lr][1] * __expf(ml_s[w][lr][0] - mf);
         }
-        inv *= ga_out_gate(p, t, h);
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
             const int c = v * 16 + lg * 4;
-            if (c < V) {
-                ga_store4<__bf16>(p, t, h, c, o[v] * inv);
+            o[v]        = o[v] * a + ((*(const floatx4*)&o_s[0][lr][c] + *(const floatx4*)&o_s[1][lr][c]) + *(const floatx4*)&o_s[2][lr][c]);
+        }
+        if (nsplit == 1) {
+            float inv;
+            if (p.sink) {
+                const float sk = p.sink[h], m2 = fmaxf(mf, sk), a2 = __expf(mf - m2);
+                inv            = a2 / (lt * a2 + __expf(sk - m2));
+            }
+            else {
+                inv = 1.f / lt;
+            }
+            inv *= ga_out_gate(p, t, h);
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+                const int c = v * 16 + lg * 4;
+                if (h_ok && c < V) {
+                    ga_store4<__bf16>(p, t, h, c, o[v] * inv);
+                }
+            }
+            return;
+        }
+        float* po = p.partial_o + (((size_t)t * p.q_heads + h) * p.splits + sp) * V;
+        float* pm = p.partial_ml + (((size_t)t * p.q_heads + h) * p.splits + sp) * 2;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            const int c = v * 16 + lg * 4;
+            if (h_ok && c < V) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    agent_store(po + c + r, o[v][r]);
+                }
             }
         }
-        return;
-    }
-    float* po = p.partial_o + (((size_t)t * p.q_heads + h) * p.splits + sp) * V;
-    float* pm = p.partial_ml + (((size_t)t * p.q_heads + h) * p.splits + sp) * 2;
-#pragma unroll
-    for (int v = 0; v < VT; ++v) {
-        const int c = v * 16 + lg * 4;
-        if (c < V) {
-            *(ga_floatx4_any*)(po + c) = o[v];
+        if (h_ok && lg == 0) {
+            agent_store(pm, mf);
+            agent_store(pm + 1, lt);
         }
     }
-    if (lg == 0) {
-        pm[0] = mf;
-        pm[1] = lt;
+    if (p.tickets && ticket_last_workgroup(p.tickets + (size_t)t * p.q_heads + g * group + chunk * 16, nsplit, &last_s)) {
+        const int pieces = V / 4;
+        for (int i = threadIdx.x; i < nheads * pieces; i += 256) {
+            const int head = i / pieces, c0 = (i - head * pieces) * 4;
+            ga_merge<__bf16, 4>(p, t, g * group + chunk * 16 + head, nsplit, [=](int c) { return c0 + c; });
+        }
     }
 }
 
@@ -1152,13 +1172,14 @@ int launch_general_attention_decode(const GeneralAttnParams& p, hipStream_t st)
         return 0;
     }
     // A workgroup takes four blocks at the time of one, so splits below four blocks only pay while the launch leaves compute units idle: 256 workgroups
-    // without splits (64 * 4) are enough.  32 rows of 32 / 8 heads of 128, ~150 tokens, 8 splits: 13.2 + 5.0 us (kernel + merge) with splits of one block,
-    // 9.4 + 2.4 with splits of at least four (eight: the same); 21.9 + 7.9 when the splits without a block ran to the end as well
+    // without splits (64 * 4) are enough.  32 rows of 32 / 8 heads of 128, ~150 tokens, 8 splits: 13.2 us with splits of one block, 9.4 with at least four
+    // (eight: the same), 21.9 when the splits without a block ran to the end as well; a merge launch took 4.6 more
     const int         chunks = (p.q_heads / p.kv_heads + 15) / 16, base = p.rows * p.kv_heads * chunks;
     GeneralAttnParams a      = p;
+    a.tickets                = ga_tickets(p);
     a.split_blocks           = std::min(4, std::max(1, base / 64));
     TM_TRY_RC(launch_mfma(a, chunks, dim3(p.rows, p.kv_heads * chunks, p.splits), st, true));
-    if (p.splits > 1) {
+    if (p.splits > 1 && !a.tickets) {
         launch_rows_merge<__bf16>(a, st);
         TM_HIP_CHECK(hipGetLastError());
     }

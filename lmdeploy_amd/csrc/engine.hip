@@ -530,6 +530,8 @@ int tm_engine_start(tm_engine* e)
     }
     const int max_splits = 16;
     TM_HIP_CHECK(hipMalloc((void**)&e->d_attn_ws, decode_attention_workspace_bytes(B, e->q_heads, e->D, max_splits)));
+    TM_TRY(dmalloc(&e->d_attn_tickets, (size_t)B * e->q_heads));
+    TM_HIP_CHECK(hipMemset(e->d_attn_tickets, 0, (size_t)B * e->q_heads * sizeof(unsigned)));
 
     // KV pool
     int64_t blocks = c.cache_blocks;
@@ -748,7 +750,7 @@ int tm_engine_destroy(tm_engine* e)
         }
     }
     void* bufs[] = {e->pool, e->d_block_ptrs, e->d_cu_block_nums, e->d_resid, e->d_x, e->d_qkv, e->d_attn, e->d_act,
-                    e->d_tmp, e->d_logits, e->d_last, e->d_gemm_ws, e->d_attn_ws, e->d_kflat, e->d_vflat, e->d_rope,
+                    e->d_tmp, e->d_logits, e->d_last, e->d_gemm_ws, e->d_attn_ws, e->d_attn_tickets, e->d_kflat, e->d_vflat, e->d_rope,
                     e->d_ids, e->d_k_len, e->d_cu_q, e->d_cu_q_b, e->d_cu_koff, e->d_rows, e->d_generated, e->d_step,
                     e->d_prefill_ids, e->d_argmax_val, e->d_cand, e->d_cand_all, e->d_next_ids, e->d_ss, e->d_tickets};
     for (void* p : bufs) {

@@ -530,6 +530,8 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
             p.splits         = e->decode_splits;
             p.partial_o      = e->d_attn_ws;
             p.partial_ml     = e->d_attn_ws + (size_t)nd * e->q_heads * e->decode_splits * e->D;
+            p.tickets        = e->d_attn_tickets;
+            p.ticket_count   = nd * e->q_heads;
             p.cache          = cvd;
             TM_PROF(P_ATTN, TM_TRY(launch_decode_attention(p, dst)));
             if (dst != st) {
@@ -556,6 +558,8 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
             p.splits     = e->decode_splits;
             p.partial_o  = e->d_attn_ws;
             p.partial_ml = e->d_attn_ws + (size_t)nseq * e->q_heads * e->decode_splits * e->D;
+            p.tickets    = e->d_attn_tickets;
+            p.ticket_count = nseq * e->q_heads;
             p.cache      = cv;
             TM_PROF(P_ATTN, TM_TRY(launch_decode_attention(p, st)));
         }

@@ -185,6 +185,8 @@ struct LayeredModel {
     int *                d_row_seq = nullptr, *d_row_pos = nullptr, *d_iota = nullptr, *d_want = nullptr, *d_seq_slot = nullptr;
     int *                d_step_ids = nullptr, *d_step_cu_q = nullptr, *d_step_k_len = nullptr;
     float*               d_attn_ws = nullptr;
+    unsigned*            d_attn_tickets = nullptr;  // [max rows][max heads], zero between launches
+    int                  n_attn_tickets = 0;
     size_t               attn_ws_bytes = 0;
     int                  decode_splits = 1;
     int                  debug_layers  = -1;  // >= 0: the forward stops behind this many layers (parity tests read the residual stream)
@@ -285,7 +287,8 @@ struct tm_engine {
     int       fold_norm = 0;  // bit 0: wo -> w1w3, bit 1: w2 -> the next layer's w_qkv
     unsigned  h_mark = 0;             // host copy of the native communicator's give-up mark (device_marks_fetch)
     bool      comm_failed = false;    // a give-up mark was seen: the ranks' call sequences may have diverged (sticky, see device_marks_check)
-    float*  d_attn_ws = nullptr;
+    float*    d_attn_ws = nullptr;
+    unsigned* d_attn_tickets = nullptr;  // [B][q_heads], zero between launches (the decode attention's own: it may run beside a prefill)
     half_t *d_kflat = nullptr, *d_vflat = nullptr;
     int     kflat_stride = 0;
     half2_t* d_rope = nullptr;

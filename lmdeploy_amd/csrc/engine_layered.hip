@@ -1087,6 +1087,8 @@ int layered_start(tm_engine* e)
     lm.decode_splits = std::min(8, std::max(1, e->max_blocks_per_seq / 4));
     lm.attn_ws_bytes = general_attention_workspace_bytes(B, max_heads, max_vdim, lm.decode_splits);
     TM_HIP_CHECK(hipMalloc((void**)&lm.d_attn_ws, lm.attn_ws_bytes));
+    lm.n_attn_tickets = (int)B * max_heads;
+    TM_TRY(lm_alloc(&lm.d_attn_tickets, (size_t)lm.n_attn_tickets, st));
 
     // the engine's batch state (same fields as every other model family)
     TM_TRY(lm_alloc(&e->d_logits, (size_t)B * e->vocab_local, st));
@@ -1170,7 +1172,7 @@ void layered_free(tm_engine* e)
     }
     for (void* p : {(void*)lm.embed, (void*)lm.final_norm, (void*)lm.d_res, lm.d_h1, lm.d_h2, lm.d_qkv, lm.d_cat, lm.d_hn, (void*)lm.d_logits_f32,
                     (void*)lm.d_row_seq, (void*)lm.d_row_pos, (void*)lm.d_iota, (void*)lm.d_want, (void*)lm.d_seq_slot, (void*)lm.d_step_ids,
-                    (void*)lm.d_step_cu_q, (void*)lm.d_step_k_len, (void*)lm.d_attn_ws, (void*)lm.scratch.slabs, (void*)lm.scratch.tickets}) {
+                    (void*)lm.d_step_cu_q, (void*)lm.d_step_k_len, (void*)lm.d_attn_ws, (void*)lm.d_attn_tickets, (void*)lm.scratch.slabs, (void*)lm.scratch.tickets}) {
         if (p) {
             (void)hipFree(p);
         }
@@ -1262,6 +1264,7 @@ static int run_attention_parts(tm_engine* e, const LmLayer& L, const LmPart* par
             p.splits     = lm.decode_splits;
             p.partial_o  = lm.d_attn_ws;
             p.partial_ml = lm.d_attn_ws + (size_t)P.rows * L.a_heads * p.splits * L.a_vdim;
+            p.tickets    = lm.d_attn_tickets, p.ticket_count = lm.n_attn_tickets;
         }
         TM_PROF(P_ATTN, TM_TRY(launch_general_attention(p, !P.decode, e->stream)));
     }
@@ -1513,6 +1516,7 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
                 p.splits     = lm.decode_splits;
                 p.partial_o  = lm.d_attn_ws;
                 p.partial_ml = lm.d_attn_ws + (size_t)P.rows * H * p.splits * L.a_vdim;
+                p.tickets    = lm.d_attn_tickets, p.ticket_count = lm.n_attn_tickets;
             }
             TM_PROF(P_ATTN, TM_TRY(launch_general_attention(p, !P.decode, st)));
         }
@@ -1919,6 +1923,7 @@ static int layered_layers(tm_engine* e, const int* d_ids, int M, const LmPart* p
                 p.splits     = lm.decode_splits;
                 p.partial_o  = lm.d_attn_ws;
                 p.partial_ml = lm.d_attn_ws + (size_t)P.rows * s.heads * p.splits * s.vdim;
+                p.tickets    = lm.d_attn_tickets, p.ticket_count = lm.n_attn_tickets;
             }
             TM_PROF(P_ATTN, TM_TRY(launch_general_attention(p, !P.decode, st)));
         }

@@ -130,4 +130,45 @@ __device__ __forceinline__ float fast_exp2(float x)
     return __builtin_amdgcn_exp2f(x);  // v_exp_f32 (no denormal range handling needed here)
 }
 
+// ---- results of several workgroups met in one launch ----
+// Partial results are written through to the device's memory (agent_store), drained, and counted in a ticket that is zero between launches; who arrives last
+// reads them past its caches (agent_load) and finishes.  No workgroup waits for another.
+__device__ __forceinline__ void agent_store(float* p, float v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float agent_load(const float* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// of n arrivals: is this the last one (which also clears the ticket)?  One lane calls it after the stores are drained
+__device__ __forceinline__ bool ticket_last(unsigned* ticket, int n)
+{
+    const bool last = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (unsigned)n;
+    if (last) {
+        __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return last;
+}
+// the same for a wave (the lanes that are active; lane 0 is one of them) and for a whole workgroup (flag: one word of LDS)
+__device__ __forceinline__ bool ticket_last_wave(unsigned* ticket, int n)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    int last = 0;
+    if ((threadIdx.x & 63) == 0) {
+        last = ticket_last(ticket, n);
+    }
+    return __builtin_amdgcn_readfirstlane(last) != 0;
+}
+__device__ __forceinline__ bool ticket_last_workgroup(unsigned* ticket, int n, unsigned* flag)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        *flag = ticket_last(ticket, n);
+    }
+    __syncthreads();
+    return *flag != 0;
+}
+
 }  // namespace tmk

@@ -68,6 +68,10 @@ struct DecodeAttnParams {
     float*        partial_o;   // [B][q_heads][splits][D]
     float*        partial_ml;  // [B][q_heads][splits][2]
     KvCacheView   cache;
+    unsigned*     tickets      = nullptr;  // zero between launches; with ticket_count >= B * q_heads of them the splits meet inside the launch
+    int           ticket_count = 0;
+    int           split_tiles  = 1;        // least tiles of a split, tokens of a tile (set by the launch)
+    int           tile_len     = 64;
     // Fused prologue (int8 MFMA kernel only): q/k/v of the new token are taken straight from the qkv GEMM output --
     // `qkv_splits` fp32 split-K slabs [qkv_splits][B][qkv_n] (or the fp16 [B][qkv_n] result when qkv_splits == 0) --
     // rotated, and K/V are quantised + stored by the attention kernel itself (the reference decode kernel does the
@@ -463,6 +467,8 @@ struct GeneralAttnParams {
     int             out_f32 = 0;           // != 0: the output rows are fp32 whatever the cache's element type
     int             splits = 1;            // most workgroups that share the keys of a row; a row uses as many as it has blocks for
     int             split_blocks = 1;      // least cache blocks of a split
+    unsigned*       tickets = nullptr;     // zero between launches; with ticket_count >= rows * q_heads of them the splits meet inside the launch
+    int             ticket_count = 0;
     float*          partial_o = nullptr;   // [rows][q_heads][splits][vdim]
     float*          partial_ml = nullptr;  // [rows][q_heads][splits][2]
     // tile kernel only: the sequences of the launch
