@@ -22,8 +22,8 @@
 //     row scale sx (a lane owns ONE row of the D tile) times the even / odd column scale;
 //   * CG column groups x WK k-phases per workgroup, partial tiles of the k-phases summed through LDS, whole-row stores
 //     (fp16, gated SiLU, fp32 split-K slabs) -- as in gemm_decode.hip;
-//   * grouped: grid.z = expert x row block; device-side row segments (`seg`), x rows gathered through `row_idx`, per-expert
-//     weight pointers; a block without rows exits before its first barrier.
+//   * grouped: device-side row segments (`seg`), x rows gathered through `row_idx`, per-expert weight pointers; tiles of 32, 64 or 128
+//     rows, only row blocks that hold rows, those of a column tile side by side.
 #include "tm_common.h"
 #include "tm_kernels.h"
 #include <algorithm>
@@ -149,7 +149,7 @@ struct Fp8Params {
     const void* const* groups;  // ... or device [experts] unit pointers (grouped)
     const int*     seg;         // grouped: device [experts + 1] flat-row offsets
     const int*     row_idx;     // grouped: x / sx row of flat row f (nullptr: f)
-    int            zper;        // grouped: row blocks per expert
+    int            experts, ct8, one_block;  // grouped: at most 64 experts; column tiles over eight; no expert has more rows than a block
     half_t*        y;
     int            ldy;
     float*         partial;
@@ -193,20 +193,47 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_fp8_kernel(Fp8Params p)
     const int l31  = lane & 31;
     const int half = lane >> 5;
 
-    // rows of this workgroup
-    int         m0 = blockIdx.z * ROWS, row0 = 0, Mloc = min(ROWS, p.M - m0);
+    // rows and columns of this workgroup
+    int         m0 = blockIdx.z * ROWS, row0 = 0, Mloc = min(ROWS, p.M - m0), ct = blockIdx.x;
     const void* wbase = p.wp;
     if constexpr (GRP) {
-        const int e = blockIdx.z / p.zper;
-        m0          = (blockIdx.z - e * p.zper) * ROWS;
-        row0        = p.seg[e];
-        Mloc        = min(ROWS, p.seg[e + 1] - row0 - m0);
-        wbase       = p.groups[e];
-        if (Mloc <= 0) {
-            return;  // whole workgroup, before any barrier
+        // One-dimensional grid over (expert, column tile, row block) with only the row blocks that hold rows, the row blocks of a column tile on
+        // consecutive turns of one XCD (workgroups are dealt to the eight in turn): its second-level cache serves a weight unit to all of them.  (Empty
+        // blocks in between would leave the shader engines they fall on idle: up to 1.9 times slower.)
+        const int turn = blockIdx.x >> 3;
+        int       e, n_e = 1, in_e;
+        if (p.one_block) {  // decode: no expert has more rows than a block
+            e    = turn / p.ct8;
+            in_e = turn - e * p.ct8;
         }
+        else {
+            const int ln = threadIdx.x & 63, nb = ln < p.experts ? (p.seg[ln + 1] - p.seg[ln] + ROWS - 1) / ROWS : 0;
+            int       upto = nb;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(upto, d);
+                upto += ln >= d ? o : 0;
+            }
+            e = __popcll(__ballot(upto * p.ct8 <= turn));  // experts whose workgroups come before this turn
+            if (e >= p.experts) {
+                return;  // whole workgroup, before any barrier
+            }
+            n_e  = __builtin_amdgcn_readlane(nb, e);
+            in_e = turn - (__builtin_amdgcn_readlane(upto, e) - n_e) * p.ct8;
+        }
+        ct = in_e / n_e * 8 + (blockIdx.x & 7);
+        if (ct * CG >= p.ncg) {
+            return;
+        }
+        m0   = in_e % n_e * ROWS;
+        row0 = p.seg[e];
+        Mloc        = min(ROWS, p.seg[e + 1] - row0 - m0);
+        if (Mloc <= 0) {
+            return;
+        }
+        wbase       = p.groups[e];
     }
-    const int cg  = blockIdx.x * CG + cgl;
+    const int cg  = ct * CG + cgl;
     const int cgc = min(cg, p.ncg - 1);
     const int kb0 = blockIdx.y * p.kb_per_split;
     const int nkb = min(p.kb_per_split, p.KB - kb0);
@@ -379,7 +406,7 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_fp8_kernel(Fp8Params p)
         }
         __syncthreads();
         constexpr int NE    = ROWS * C4;
-        const int     ncol0 = blockIdx.x * CG * 32;
+        const int     ncol0 = ct * CG * 32;
 #pragma unroll
         for (int e0 = 0; e0 < NE; e0 += T) {
             const int e = e0 + tid;
@@ -497,10 +524,10 @@ int launch_linear_fp8(const LinearWeight& w, const uint8_t* xq, const float* sx,
 // grouped: flat rows seg[e] .. seg[e+1] of expert e, x / sx row of flat row f = row_idx ? row_idx[f] : f; m_hint = expected rows
 // per expert (tile height), m_cap = upper bound
 int launch_linear_fp8_grouped(const LinearWeight& proto, const void* d_groups, int E, const uint8_t* xq, const float* sx, int ldsx,
-                              int x_rows, half_t* y, int ldy, int m_cap, int m_hint, bool gated_silu, const int* seg,
+                              int x_rows, half_t* y, int ldy, int m_cap, int total_rows, int m_hint, bool gated_silu, const int* seg,
                               const int* row_idx, hipStream_t st)
 {
-    TM_REQUIRE(proto.type == 2 && proto.N % 32 == 0 && proto.K % 128 == 0, "grouped fp8 MFMA linear: e4m3 experts, N % 32 == 0");
+    TM_REQUIRE(E <= 64 && proto.type == 2 && proto.N % 32 == 0 && proto.K % 128 == 0, "grouped fp8 MFMA linear: e4m3 experts, N % 32 == 0");
     if (m_cap == 0 || E == 0) {
         return 0;
     }
@@ -512,14 +539,17 @@ int launch_linear_fp8_grouped(const LinearWeight& proto, const void* d_groups, i
     const int want = std::min(m_cap, std::max(1, 2 * m_hint));
     int       tv[4];
     const bool measured = gen_table_get(kGenGrouped + 2, 0, proto.K, proto.N, dec32_m_bucket(m_cap), tv);  // tm_engine_tune_gemm
-    if (measured ? tv[0] == 32 : want <= 32) {
-        p.zper = (m_cap + 31) / 32;
-        dim3 grid((p.ncg + 3) / 4, 1, E * p.zper);
-        return launch_fp8_one<1, 4, 4, true>(p, grid, st);
-    }
-    p.zper = (m_cap + 63) / 64;
-    dim3 grid((p.ncg + 3) / 4, 1, E * p.zper);
-    return launch_fp8_one<2, 4, 2, true>(p, grid, st);
+    // Rows of a tile, by the expected rows of an expert: a weight unit costs a workgroup the same for 128 rows as for 32, but rows that are not there cost as
+    // much as those that are.  Mixtral-sized experts (4096 x 14336, 8, top 2), us a layer with 32 / 64 / 128 rows: 16 expected 259 / 302 / 427, 48: 398 / 326
+    // / 428, 64: 469 / 478 / 430, 100: 612 / 522 / 447, 128: 735 / 641 / 697, 256: 1304 / 1088 / 1013, 1024: 4915 / 3857 / 3264 (0.88 PFLOP/s; 64 rows with
+    // the row blocks of a column tile far apart: 4868)
+    const int rows = measured ? tv[0] : want <= 32 ? 32 : m_hint < 56 ? 64 : 128;
+    p.experts      = E;
+    p.ct8          = ((p.ncg + 3) / 4 + 7) / 8;
+    p.one_block    = m_cap <= rows;
+    const dim3 grid(p.ct8 * 8 * (p.one_block ? E : std::min(E * ((m_cap + rows - 1) / rows), total_rows / rows + E)));
+    return rows == 32 ? launch_fp8_one<1, 4, 4, true>(p, grid, st) :
+           rows == 64 ? launch_fp8_one<2, 4, 2, true>(p, grid, st) : launch_fp8_one<4, 4, 2, true>(p, grid, st);
 }
 
 }  // namespace tmk

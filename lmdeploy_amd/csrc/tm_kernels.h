@@ -203,7 +203,7 @@ int    dec32_m_bucket(int M);  // table key of a forward with M rows: M itself u
 // Measured dispatch of everything that is NOT a P32 kernel (reference: gemm.cu:92-224 caches every problem the
 // warm-up of turbomind.cc:363-487 meets, not only the dense u4 ones).  One table, key (kind, role, K, N, M bucket):
 //   kind kGenDense + type   : gemm_kernel of a dense linear (fp16 lm_head, e4m3 weight-only, u4 with N % 32 != 0) -> {nt, splits, waves, kphases}
-//   kind kGenGrouped + type : row-tile height of the grouped expert GEMMs (u4: 16 / 32 / 64 rows, fp8 MFMA: 32 / 64) -> {rows, 0, 0, 0}
+//   kind kGenGrouped + type : row-tile height of the grouped expert GEMMs (u4: 16 / 32 / 64 rows, fp8 MFMA: 32 / 64; larger prompts without an entry take 128) -> {rows, 0, 0, 0}
 // Text form (same file as the P32 table): `G kind role K N M a b c d`.  role 5 = lm_head; grouped entries use role 0.
 constexpr int kGenDense   = 16;
 constexpr int kGenGrouped = 32;
@@ -248,7 +248,7 @@ int    launch_quant_fp8_rows(uint8_t* xq, float* sx, const half_t* x, int ldx, i
 int    launch_linear_fp8(const LinearWeight& w, const uint8_t* xq, const float* sx, int ldsx, half_t* y, int ldy, int M, bool gated_silu,
                          int splits, float* workspace, int* slabs_out, hipStream_t st);
 int    launch_linear_fp8_grouped(const LinearWeight& proto, const void* d_groups, int E, const uint8_t* xq, const float* sx, int ldsx,
-                                 int x_rows, half_t* y, int ldy, int m_cap, int m_hint, bool gated_silu, const int* seg,
+                                 int x_rows, half_t* y, int ldy, int m_cap, int total_rows, int m_hint, bool gated_silu, const int* seg,
                                  const int* row_idx, hipStream_t st);
 
 // ---- comm_p2p.hip: fused one-shot all-reduce + residual + RMSNorm over peer-mapped buffers (TM_COMM=native) ------------
