@@ -1588,6 +1588,26 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
         *splits_out = env_splits > 0 ? env_splits : sp;
         return;
     }
+    // Up to 32 rows: a narrow projection's 128-column tiles are too few and their slices too many, 64-column tiles (shape 3) with slices of at least eight
+    // k-blocks are faster up to N = 5120 whatever K, and beyond while K is short.  Kernel + consumer, us a layer, 128-column tiles / this (K x N, rows):
+    // 4096 x 4096, 1: 10.6 / 9.6, 32: 12.1 / 10.0; 14336 x 4096, 1: 15.1 / 13.5, 16: 17.4 / 14.5; 4096 x 6144, 1: 10.8 / 10.1, 32: 12.1 / 10.4; 8192 x 2048,
+    // 1: 15.5 / 13.9; 13824 x 5120, 8: 20.7 / 19.7; 6144 x 8192, 8: 16.3 / 15.5.  Not taken: 6144 x 6144, 8: 16.7 / 16.9; 16384 x 6144, 1: 23.2 / 25.0;
+    // 28672 x 8192, 1: 33.5 / 36.6; 8192 x 8192, 1: 18.9 / 19.1; 512 x 4096, 32: 12.4 / 12.7 (8: 12.0 / 10.9)
+    if (rowhalf && env_shape < 0 && M <= 32 && ncg >= 8 && ncg <= 256 && (KB >= 8 || M <= 16)) {
+        const int tiles = (ncg + 1) / 2;
+        int       sp    = 1;
+        for (int s2 = 2; s2 <= 16 && tiles * s2 <= 256; ++s2) {
+            const int per = ((KB + s2 - 1) / s2 + 3) / 4 * 4;
+            if ((KB + per - 1) / per == s2 && per >= 8) {
+                sp = s2;
+            }
+        }
+        if (ncg <= 160 || KB <= 32 || (KB <= 48 && tiles * sp >= 224)) {
+            *shape_out  = 3;
+            *splits_out = env_splits > 0 ? env_splits : sp;
+            return;
+        }
+    }
     int cgn, S;
     dec32_shape_dims(shape, &cgn, &S);
     const int col_wgs = (ncg + cgn - 1) / cgn * ((M + 127) / 128);
