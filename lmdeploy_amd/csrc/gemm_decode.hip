@@ -1529,12 +1529,12 @@ int dec32_candidates(const LinearWeight& w, int M, int (*out)[2], int cap)
 
 // Tiling for the decode GEMM: `shape` (see launch_dec32_shape) and the split-K count.  One workgroup per CU (128 KB of
 // LDS): take the widest split that keeps <= 256 workgroups and >= one stage (4 k-blocks) per slice.
-void dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out)
+void dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool folded)
 {
-    dec32_pick_ex(w, M, shape_out, splits_out, true);
+    dec32_pick_ex(w, M, shape_out, splits_out, true, folded);
 }
 
-void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table)
+void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table, bool folded)
 {
     const int ncg = w.N / 32;
     const int KB  = w.K / 128;
@@ -1585,6 +1585,25 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
             }
         }
         *shape_out  = nshape;
+        *splits_out = env_splits > 0 ? env_splits : sp;
+        return;
+    }
+    // 65 .. 256 rows of a small product: row blocks of 32 with 64-column tiles (shape 6) keep more compute units busy than tiles of 128 rows that need slices of
+    // k, until re-reading the weights for every row block costs more.  us a layer with the consumer, 128 rows: 4096 x 6144 28.2 -> 20.2, 4096 x 4096 25.2 ->
+    // 17.5, 14336 x 4096 38.0 -> 34.0, 2048 x 16384 30.7 -> 25.3, 8192 x 2048 26.1 -> 18.0, 512 x 4096 18.1 -> 12.1; 256 rows: 4096 x 4096 29.8 -> 24.3, 8192 x 2048
+    // 28.3 -> 24.8, 1024 x 8192 25.9 -> 22.0.  Not taken, 128 rows: 13824 x 5120 39.1 / 52.0, 8192 x 10240 40.7 / 47.8; 256 rows: 8192 x 3072 31.5 / 36.2, 6144 x 6144
+    // 37.4 / 42.5, 14336 x 4096 46.6 / 56.2.  (Products with a folded norm keep tiles of their own at these row counts.)
+    const size_t rb = (M + 31) / 32, kn = (size_t)w.K * w.N;
+    if (rowhalf && env_shape < 0 && !folded && M > 64 && M <= 256 && ncg >= 8 && (rb <= 4 ? kn <= 60000000 : kn * rb <= 140000000)) {
+        const int tiles = (ncg + 1) / 2 * (int)rb;
+        int       sp    = 1;
+        for (int s2 = 2; s2 <= 16 && tiles * s2 <= 256; ++s2) {
+            const int per = ((KB + s2 - 1) / s2 + 3) / 4 * 4;
+            if ((KB + per - 1) / per == s2 && per >= 8) {
+                sp = s2;
+            }
+        }
+        *shape_out  = 6;
         *splits_out = env_splits > 0 ? env_splits : sp;
         return;
     }

@@ -1,5 +1,6 @@
-"""GPU test of the tiling rule for W4 products of up to 32 rows (64-column tiles, gemm_decode.hip): sizes on both sides of its lines in columns and k, k-block
-counts that leave a short last slice, the fewest and the most rows, through the entry point that picks the tiling itself, against the oracle."""
+"""GPU test of the tiling rules for W4 products of up to 32 and of 65 to 256 rows (64-column tiles, gemm_decode.hip): sizes on both sides of their lines in
+columns, k and rows, k-block counts that leave a short last slice, the fewest and the most rows, through the entry point that picks the tiling itself, against
+the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -19,7 +20,7 @@ def _release():
 
 @pytest.mark.parametrize('K,N', [(128, 256), (896, 288), (1024, 224), (1152, 256), (2048, 1056), (4096, 5120), (4096, 5152), (4224, 5152), (6144, 7168),
                                  (6272, 7168), (13824, 512)])
-@pytest.mark.parametrize('M', [1, 16, 17, 32])
+@pytest.mark.parametrize('M', [1, 16, 17, 32, 65, 96, 128, 129, 250, 256])
 def test_picked_tiling(tm, cuda, K, N, M):
     rng = np.random.default_rng(K + N + M)
     h, _ = _make_linear(tm, rng, K, N)
