@@ -377,9 +377,9 @@ static int fold_tile_pick(const tm_linear* w, int M, int* shape, int* splits, bo
 {
     int sh = *shape, sp = *splits;
     if (sh < 0) {
-        dec32_pick(w->w, M, &sh, &sp, true);
+        dec32_pick(w->w, M, &sh, &sp);
         if (!dec32_fold_shape_m(sh, M, producer)) {
-            dec32_pick_ex(w->w, M, &sh, &sp, false, true);
+            dec32_pick_ex(w->w, M, &sh, &sp, false);
         }
         if (!dec32_fold_shape_m(sh, M, producer)) {
             sh = M <= 64 ? 0 : (producer ? 7 : 4);

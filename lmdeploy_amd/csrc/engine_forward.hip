@@ -274,9 +274,9 @@ static int forward_layers_two_microbatches(tm_engine* e, int M, int nseq, int ma
 // the tiling of a folded launch: the measured / heuristic pick when its kernel carries the folded epilogue, else the heuristic's
 static void fold_tiling(tm_engine* e, const LinearWeight& w, int M, int* shape, int* splits, bool producer)
 {
-    dec32_pick(w, M, shape, splits, true);
+    dec32_pick(w, M, shape, splits);
     if (!dec32_fold_shape_m(*shape, M, producer)) {
-        dec32_pick_ex(w, M, shape, splits, false, true);
+        dec32_pick_ex(w, M, shape, splits, false);
     }
     if (!dec32_fold_shape_m(*shape, M, producer)) {
         // M <= 64: the 128-column tile over the whole k range; above (batch 128): the same tile on 32-row blocks for a producer, the 128-row

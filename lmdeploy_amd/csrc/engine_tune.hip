@@ -68,7 +68,12 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
         if (dec32_table_get(w0.K, w0.N, M, &hs, &hp, r.which + 1)) {
             continue;  // imported / tuned already
         }
-        dec32_pick_ex(w0, M, &hs, &hp, false);
+        if (e->fold_norm != 0 && M <= e->fold_max_rows) {
+            dec32_pick_ex(w0, M, &hs, &hp, false);
+        }
+        else {
+            dec32_pick_plain(w0, M, &hs, &hp, false);
+        }
         int       cand[96][2];
         int       nc = dec32_candidates(w0, M, cand, 95);
         bool      has = false;

@@ -1529,12 +1529,12 @@ int dec32_candidates(const LinearWeight& w, int M, int (*out)[2], int cap)
 
 // Tiling for the decode GEMM: `shape` (see launch_dec32_shape) and the split-K count.  One workgroup per CU (128 KB of
 // LDS): take the widest split that keeps <= 256 workgroups and >= one stage (4 k-blocks) per slice.
-void dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool folded)
+void dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out)
 {
-    dec32_pick_ex(w, M, shape_out, splits_out, true, folded);
+    dec32_pick_ex(w, M, shape_out, splits_out, true);
 }
 
-void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table, bool folded)
+void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table)
 {
     const int ncg = w.N / 32;
     const int KB  = w.K / 128;
@@ -1588,13 +1588,45 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
         *splits_out = env_splits > 0 ? env_splits : sp;
         return;
     }
+    int cgn, S;
+    dec32_shape_dims(shape, &cgn, &S);
+    const int col_wgs = (ncg + cgn - 1) / cgn * ((M + 127) / 128);
+    int       splits  = 1;
+    static const int min_kb = env_int2("TM_D32_MIN_KB", 4);
+    for (int s = 2; s <= 16; ++s) {  // the engine's slab workspace holds 16 splits
+        int per = (KB + s - 1) / s;
+        per     = (per + S - 1) / S * S;
+        const int eff = (KB + per - 1) / per;  // splits after rounding the slice to whole stages
+        if (eff != s) {
+            continue;
+        }
+        if (col_wgs * s <= 256 && per >= (M > 64 ? 8 : min_kb) && (M <= 256 || s <= 4)) {
+            splits = s;  // (prefill-sized forwards: slabs of MBs per slice -- never more than 4)
+        }
+    }
+    splits      = env_splits > 0 ? env_splits : splits;
+    *shape_out  = shape;
+    *splits_out = splits < 1 ? 1 : (splits > KB ? KB : splits);
+}
+
+// Tiling of a product without a folded norm: the measured table, then the lines below for few rows, then the rule above (which the folded launches keep:
+// their residual sums are formed in its slices' order)
+void dec32_pick_plain(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table)
+{
+    const int        ncg = w.N / 32, KB = w.K / 128;
+    static const int env_shape  = env_int2("TM_D32_SHAPE", -1);
+    static const int env_splits = env_int2("TM_D32_SPLITS", 0);
+    static const int rowhalf    = env_int2("TM_D32_ROWHALF", 1);
+    if (use_table && dec32_table_get(w.K, w.N, dec32_m_bucket(M), shape_out, splits_out, w.role)) {
+        return;
+    }
     // 65 .. 256 rows of a small product: row blocks of 32 with 64-column tiles (shape 6) keep more compute units busy than tiles of 128 rows that need slices of
     // k, until re-reading the weights for every row block costs more.  us a layer with the consumer, 128 rows: 4096 x 6144 28.2 -> 20.2, 4096 x 4096 25.2 ->
     // 17.5, 14336 x 4096 38.0 -> 34.0, 2048 x 16384 30.7 -> 25.3, 8192 x 2048 26.1 -> 18.0, 512 x 4096 18.1 -> 12.1; 256 rows: 4096 x 4096 29.8 -> 24.3, 8192 x 2048
     // 28.3 -> 24.8, 1024 x 8192 25.9 -> 22.0.  Not taken, 128 rows: 13824 x 5120 39.1 / 52.0, 8192 x 10240 40.7 / 47.8; 256 rows: 8192 x 3072 31.5 / 36.2, 6144 x 6144
-    // 37.4 / 42.5, 14336 x 4096 46.6 / 56.2.  (Products with a folded norm keep tiles of their own at these row counts.)
+    // 37.4 / 42.5, 14336 x 4096 46.6 / 56.2.
     const size_t rb = (M + 31) / 32, kn = (size_t)w.K * w.N;
-    if (rowhalf && env_shape < 0 && !folded && M > 64 && M <= 256 && ncg >= 8 && (rb <= 4 ? kn <= 60000000 : kn * rb <= 140000000)) {
+    if (rowhalf && env_shape < 0 && M > 64 && M <= 256 && ncg >= 8 && (rb <= 4 ? kn <= 60000000 : kn * rb <= 140000000)) {
         const int tiles = (ncg + 1) / 2 * (int)rb;
         int       sp    = 1;
         for (int s2 = 2; s2 <= 16 && tiles * s2 <= 256; ++s2) {
@@ -1627,25 +1659,7 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
             return;
         }
     }
-    int cgn, S;
-    dec32_shape_dims(shape, &cgn, &S);
-    const int col_wgs = (ncg + cgn - 1) / cgn * ((M + 127) / 128);
-    int       splits  = 1;
-    static const int min_kb = env_int2("TM_D32_MIN_KB", 4);
-    for (int s = 2; s <= 16; ++s) {  // the engine's slab workspace holds 16 splits
-        int per = (KB + s - 1) / s;
-        per     = (per + S - 1) / S * S;
-        const int eff = (KB + per - 1) / per;  // splits after rounding the slice to whole stages
-        if (eff != s) {
-            continue;
-        }
-        if (col_wgs * s <= 256 && per >= (M > 64 ? 8 : min_kb) && (M <= 256 || s <= 4)) {
-            splits = s;  // (prefill-sized forwards: slabs of MBs per slice -- never more than 4)
-        }
-    }
-    splits      = env_splits > 0 ? env_splits : splits;
-    *shape_out  = shape;
-    *splits_out = splits < 1 ? 1 : (splits > KB ? KB : splits);
+    dec32_pick_ex(w, M, shape_out, splits_out, false);
 }
 
 // y / slabs as launch_linear: *slabs_out = number of fp32 slabs written into `workspace` (1 = direct epilogue)

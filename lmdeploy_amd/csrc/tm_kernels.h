@@ -190,8 +190,9 @@ int  launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* 
 size_t p32_bytes(int K, int N);
 int    launch_repack_p32(void* out, const int32_t* qweight, const half_t* scales, const half_t* zeros, int K, int N, hipStream_t st);
 bool   dec32_supported(const LinearWeight& w, int M);
-void   dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool folded = false);  // measured table first, then the heuristic
-void   dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table, bool folded = false);
+void   dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out);  // measured table first, then the heuristic
+void   dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table);
+void   dec32_pick_plain(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table);  // ... of a product without a folded norm
 // measured dispatch table of the decode linears: key (K, N, M <= 64) -> (shape, splits)
 void   dec32_table_set(int K, int N, int M, int shape, int splits, int role = 0);
 bool   dec32_table_get(int K, int N, int M, int* shape, int* splits, int role = 0);  // the role's entry, else the role-0 entry
