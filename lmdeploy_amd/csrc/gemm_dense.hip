@@ -22,6 +22,7 @@
 #include "tm_kernels.h"
 #include "gemm_stream.h"
 #include <algorithm>
+#include <numeric>
 
 namespace tmk {
 
@@ -104,7 +105,7 @@ struct DenseEpi {
     {
         DenseItem it{(int64_t)g * c.x_col_stride, (int64_t)g * (int64_t)c.w_stride, 0, g * c.y_col_stride, M};
 #pragma unroll
-        for (int s = 1; s < kDenseMaxSeg; ++s) {  // (the segment of this workgroup's columns)
+        for (int s = 1; s < kDenseMaxSeg; ++s) {  // (the segment of this workgroup's columns: the plan takes no tile that holds a border)
             it.x_off += s < c.n_seg && n0 >= c.seg_n0[s] ? c.x_col_stride : 0;
         }
         if (c.row_offsets) {
@@ -317,7 +318,7 @@ void dense_weight_free(DenseWeight& d)
 //     rows, (2048, 11264): one 17, two 23
 //   narrow kernel: eight rows bf16, (2048, 2048): 6.5 us against 7.5 with four slices, (2048, 4096): 8.3 against 8.9, (2048, 6144): 12.5 against 10.5, (2048,
 //     10240): 18.3 against 13.0 unsliced; three rows fp32, (768, 2048): 6.1 against 7.9, (2048, 2048): 10.8 against 9.6; without scratch (25600, 4096) with 32 rows: 76 against 120
-StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets)
+StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border)
 {
     struct Tile {
         int    rows, cols;
@@ -329,6 +330,9 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     double            cost = 1e30;
     for (int k = 0; k < 4; ++k) {
         const Tile&   t     = kTiles[k];
+        if (border % t.cols) {  // a workgroup reads x at one place
+            continue;
+        }
         const int64_t rt    = own_rows ? rows / t.rows + items : (int64_t)((rows + t.rows - 1) / t.rows) * items;
         const int64_t n     = (rt * ((cols + t.cols - 1) / t.cols) + 255) / 256;
         const double  full  = elem == 4 ? t.full32 : t.full16, alone = elem == 4 ? t.alone32 : t.alone16;
@@ -452,7 +456,12 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
     const int  vec     = ldy % align == 0 && (uintptr_t)y % 16 == 0 && call.y_col_stride % align == 0
                     && (!call.y2 || (call.ldy2 % 8 == 0 && (uintptr_t)call.y2 % 16 == 0))
                     && (epi != kDenseResidGate || (call.ldg % 4 == 0 && (uintptr_t)call.gate % 16 == 0));
-    const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2, d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0);
+    int border = 0;  // the segments begin at multiples of this many columns
+    for (int s = 1; s < call.n_seg; ++s) {
+        border = std::gcd(border, call.seg_n0[s]);
+    }
+    const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2,
+                                     d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border);
     if (p.skinny) {
         const bool pairs = epi == kDenseGatedAct && sizeof(T) == 2;
         a.split_steps    = p.split_steps;

@@ -733,8 +733,9 @@ struct StreamPlan {
     int  tile;                                 // 0: 256 x 256 (16-bit formats), 1: 256 x 128, 2: 128 x 128, 3: 64 x 64
 };
 // steps of k, image columns, rows, items (own_rows: each with rows of its own, `rows` in total), bytes of an element; pairs: a wave needs two
-// column tiles; ws_bytes / tickets: what slices of k may use (0: no slices)
-StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets);
+// column tiles; ws_bytes / tickets: what slices of k may use (0: no slices); border: x is read elsewhere from multiples of this many columns on (a
+// multiple of 128; 0: nowhere)
+StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0);
 constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
 constexpr int    kStreamTickets = 4096;
 

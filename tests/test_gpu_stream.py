@@ -10,10 +10,13 @@ import torch
 from lmdeploy_amd import _ffi
 from tests import febivik_oracle as fo
 from tests import layered_oracle as lo
+from tests import roravik_oracle as ro
 from tests.gpu_helpers import release_all, st
 from tests.test_gpu_febivik import engine, model_folder
 from tests.test_gpu_febivik import rel_err as rel_err_febivik
 from tests.test_gpu_layered import _layer, engine_for, rel_err
+from tests.test_gpu_roravik import engine as roravik_engine
+from tests.test_gpu_roravik import model_folder as roravik_folder
 
 pytestmark = pytest.mark.gpu
 
@@ -127,3 +130,29 @@ def test_f16_linears_at_the_edges(tm, cuda, K, N, gated, rows):
             assert bool(((y[:M, :No].double() - ref).abs() <= bound).all()), (M, ldy)
             assert bool((y[M] == -3.0).all()) and bool((y[:M, No:] == -3.0).all())
     _ffi.check(tm.tm_linear_destroy(h))
+
+
+def stream_errs(eng, toks, trail):
+    """rms error of every row of the residual stream behind the first layer of a prompt taken in one forward, relative to the stream's size"""
+    eng.stop_after(1)
+    s = eng.open_session()
+    eng.step_tokens([(s, toks, [])])
+    d = eng.fetch_residual(len(toks)) - trail[0]
+    eng.close_session(s)
+    return np.sqrt((d ** 2).mean(-1)) / np.sqrt((trail[0] ** 2).mean())
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('rows', [2048, 3000])
+def test_segments_that_begin_at_odd_multiples_of_128(cuda, tmp_path, dtype, rows):
+    """the projections of a parallel pair of mixers are one product whose columns read six inputs of a row: borders at 2048, 2688, 3328, 3968 and 4608, of
+    which 2688 and 3968 lie in the middle of 256 columns, at row counts where a product of one input takes 256-column tiles.  bf16 rounds the mixed rows, the
+    queries, keys, values and weights of the window, the joined heads and the matrices' inputs, 2^-9 each, and a norm behind the sum scales a small
+    row up: within 4e-2 of the stream's size; a projection of the wrong input is 0.3 off in every row"""
+    cfg = ro.make_config(128, 97, [ro.parallel_layer(8, 4, 128, 128, 64, 5, 128)])
+    toks = np.random.default_rng(rows).integers(0, 97, rows).tolist()
+    folder, w = roravik_folder(tmp_path, cfg, 3)
+    eng = roravik_engine(folder, dtype, max_batch_size=1, session_len=3072, cache_blocks=64, max_prefill_token_num=3072)
+    errs = stream_errs(eng, toks, ro.forward(cfg, w, toks, True)[1])
+    eng.close()
+    assert errs.max() <= (3e-5 if dtype == 'float32' else 4e-2), np.sort(errs)[-5:]
