@@ -61,6 +61,11 @@ struct StreamArgs {
     float*      slabs;        // skinny kernel, several slices: their partial sums, [item][slice][M][16 tiles]
     unsigned*   tickets;      // ... and an arrival counter per (column group, row block, item), zero between launches (nullptr: the slabs are the result)
 };
+// from the first block of a column tile to the end of the image's last block
+__device__ __forceinline__ int64_t stream_weight_bytes(const StreamArgs& a, int tile)
+{
+    return (int64_t)(a.tiles - 1 - tile) * a.w_tile + (int64_t)((a.steps - 1) >> 2) * a.w_quad + ((a.steps - 1) & 3) * 1024 + 1024;
+}
 
 // ---- few rows: the weight stream ---------------------------------------------------------------------------------------------------
 // What bounds it: a CU keeps about 440 cache lines in flight whatever their source, so a line of x that comes from L2 costs nearly what a
@@ -447,7 +452,7 @@ __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_k
         return;
     }
     const auto rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + item.x_off + m0 * a.ldx), 0, (int)((Mloc - 1) * a.ldx + (int64_t)a.steps * 64), 0x00020000);
-    const int64_t w_left = (int64_t)(a.tiles - (n0 >> 4)) * a.w_tile + (a.w_quad > 4096 ? (int64_t)((a.steps - 1) >> 2) * a.w_quad : 0);
+    const int64_t w_left = stream_weight_bytes(a, n0 >> 4);
     const auto rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + item.w_off + (int64_t)(n0 >> 4) * a.w_tile), 0, (int)min(w_left, (int64_t)0xffffffff), 0x00020000);
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
     int            xoff[kXP];
@@ -584,7 +589,7 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
         return;
     }
     const auto rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + item.x_off + m0 * a.ldx), 0, (int)((Mloc - 1) * a.ldx + (int64_t)a.steps * 64), 0x00020000);
-    const int64_t w_left = (int64_t)(a.tiles - (n0 >> 4)) * a.w_tile + (a.w_quad > 4096 ? (int64_t)((a.steps - 1) >> 2) * a.w_quad : 0);
+    const int64_t w_left = stream_weight_bytes(a, n0 >> 4);
     const auto rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + item.w_off + (int64_t)(n0 >> 4) * a.w_tile), 0, (int)min(w_left, (int64_t)0xffffffff), 0x00020000);
     const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
     int            xoff[kXP], woff[kWP];

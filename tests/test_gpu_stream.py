@@ -100,6 +100,8 @@ def test_row_tiles_of_many_items(cuda, tmp_path):
 
 @pytest.mark.parametrize('K,N,gated,rows', [
     (128, 16, 0, (1, 17, 65, 300)),                   # one column tile
+    (256, 16, 0, (17, 65, 300)),                      # ... and more than one block of 128 k
+    (2048, 16, 0, (1, 65, 300)),
     (256, 4128, 1, (1, 16, 33, 64, 129)),             # a ragged last column group, gated
     (2048, 2080, 0, (8, 16, 31, 64, 200, 257, 1100)),  # slices of k that meet in a reduce launch; tiles of every height
     (4096, 544, 0, (3, 20, 64)),
