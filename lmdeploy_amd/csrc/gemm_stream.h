@@ -174,23 +174,36 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
         }
     };
     constexpr int kStride = KP * kChunk;
-    fetch(wa, s0 + ph * kChunk);
+    const int     first   = ph * kChunk;  // of this k-phase in a stage
+    fetch(wa, s0 + first);
     fetch_x(s0);
     stash_x(0);
     __syncthreads();
-    int buf = 0;
-    for (int base = s0; base < s1; base += 2 * kStride) {
-        fetch(wb, base + kStride + ph * kChunk);
+    int base = s0;
+    for (; base + 2 * kStride < s1; base += 2 * kStride) {  // three stages lie ahead
+        fetch(wb, base + kStride + first);
         fetch_x(base + kStride);
-        compute(wa, buf, base + ph * kChunk);
-        stash_x(buf ^ 1);  // its readers finished before the last barrier
+        compute(wa, 0, base + first);
+        stash_x(1);  // its readers finished before the last barrier
         __syncthreads();
-        fetch(wa, base + 2 * kStride + ph * kChunk);
+        fetch(wa, base + 2 * kStride + first);
         fetch_x(base + 2 * kStride);
-        compute(wb, buf ^ 1, base + kStride + ph * kChunk);
-        stash_x(buf);
+        compute(wb, 1, base + kStride + first);
+        stash_x(0);
         __syncthreads();
     }
+    if (base + kStride < s1) {  // the last two stages, or the last: nothing is fetched that is not used
+        fetch(wb, base + kStride + first);
+        fetch_x(base + kStride);
+        compute(wa, 0, base + first);
+        stash_x(1);
+        __syncthreads();
+        compute(wb, 1, base + kStride + first);
+    }
+    else {
+        compute(wa, 0, base + first);
+    }
+    __syncthreads();
     if constexpr (KP > 1) {  // (the last barrier freed the x buffers)
         floatx4* red = (floatx4*)smem;
         if (ph > 0) {
@@ -345,12 +358,22 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
     };
     constexpr int kStride = W * kChunk;
     int           base    = wave * kChunk;
-    fetch(wa, base);
-    for (; base < a.steps; base += 2 * kStride) {
-        fetch(wb, base + kStride);
-        compute(wa, base);
-        fetch(wa, base + 2 * kStride);
-        compute(wb, base + kStride);
+    if (base < a.steps) {
+        fetch(wa, base);
+        for (; base + 2 * kStride < a.steps; base += 2 * kStride) {
+            fetch(wb, base + kStride);
+            compute(wa, base);
+            fetch(wa, base + 2 * kStride);
+            compute(wb, base + kStride);
+        }
+        if (base + kStride < a.steps) {  // the last two chunks, or the last: nothing is fetched that is not used
+            fetch(wb, base + kStride);
+            compute(wa, base);
+            compute(wb, base + kStride);
+        }
+        else {
+            compute(wa, base);
+        }
     }
 #pragma unroll
     for (int t = 0; t < MT; ++t) {

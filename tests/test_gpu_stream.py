@@ -39,6 +39,7 @@ def check(got, ref, size, K, bf16):
     (1056, 2304, (3, 33, 300, 2100)),               # 33 steps, 256 x 256 tiles
     (2080, 2048, (5, 48, 255)),
     (200, 512, (70, 511, 513)),
+    (9000, 130, (2, 20, 40)),                       # waves that take several chunks of a long k, up to a ragged end
 ])
 def test_products_at_the_edges_of_tiles(tm, cuda, dtype, K, N, rows):
     g = torch.Generator('cuda').manual_seed(K + N)
@@ -82,6 +83,27 @@ def test_slices_of_k_meet_in_any_order(cuda, dtype, rows):
     assert all(np.array_equal(a, b) for o in outs[1:] for a, b in zip(o, outs[0]))
     got = np.stack(outs[0], 1)
     for i in range(0, rows, 7):
+        assert rel_err(got[i], lo.forward(cfg, w, toks[i].tolist())[0]) <= (3e-5 if dtype == 'float32' else 4e-2)
+    eng.close()
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('rows,ff', [(3, 8320), (20, 8320), (65, 4160), (100, 4160), (250, 4160)])
+def test_slices_of_k_of_long_sums_and_of_several_row_blocks(cuda, dtype, rows, ff):
+    """the same for sums that are cut whatever the format, and for two to four blocks of 64 rows: counters and slabs of every (column group, block)"""
+    cfg = lo.make_config(1056, 203, [_layer(heads=8, kv_heads=2, dim=32, vdim=32, ff=ff)], mult=0.4)
+    w = lo.make_weights(cfg, 6)
+    eng = engine_for(cfg, w, dtype, max_batch_size=256, cache_blocks=260)
+    toks = np.random.default_rng(rows).integers(0, cfg['vocab'], (rows, 2))
+    outs = []
+    for _ in range(3):
+        s = [eng.open_session() for _ in range(rows)]
+        outs.append([eng.step_tokens([(s[i], [int(toks[i, k])], [0]) for i in range(rows)]) for k in range(2)])
+        for i in s:
+            eng.close_session(i)
+    assert all(np.array_equal(a, b) for o in outs[1:] for a, b in zip(o, outs[0]))
+    got = np.stack(outs[0], 1)
+    for i in [0, 1, rows // 2, rows - 1] + list(range(0, rows, 13)):
         assert rel_err(got[i], lo.forward(cfg, w, toks[i].tolist())[0]) <= (3e-5 if dtype == 'float32' else 4e-2)
     eng.close()
 
