@@ -316,8 +316,11 @@ void dense_weight_free(DenseWeight& d)
 //     price of a line of weights.  32 rows bf16, (25600, 4096): one slice 119 us, four 46, eight 45; (4096, 6144): one 23, three 19, four 18 (slices of equal length);
 //     (4096, 21504): one 40, two 42; nine items of (2048, 2816): one 21, three 31; three rows fp32, (8448, 2048): one 75, eight 21; pairs, four
 //     rows, (2048, 11264): one 17, two 23
-//   narrow kernel: eight rows bf16, (2048, 2048): 6.5 us against 7.5 with four slices, (2048, 4096): 8.3 against 8.9, (2048, 6144): 12.5 against 10.5, (2048,
-//     10240): 18.3 against 13.0 unsliced; three rows fp32, (768, 2048): 6.1 against 7.9, (2048, 2048): 10.8 against 9.6; without scratch (25600, 4096) with 32 rows: 76 against 120
+//   narrow kernel, up to 32 rows of one item: 16 columns a workgroup, a line of x at 0.6 of the price of a line of weights; the way through memory costs
+//     slices about 4.5 us more.  Narrow | slices, bf16: 8 rows (2048, 2048) 5.0 | 6.6 us, (4096, 4096) 9.4 | 11.8, (25600, 4096) 38.7 | 40.0, (2048, 8448)
+//     11.8 | 11.3, (4096, 12288) 24.2 | 21.8; 16 rows (14336, 4096) 28.0 | 25.2; 32 rows (768, 768) 4.2 | 6.0 (one slice), (2048, 2048) 7.4 | 8.2, (4096,
+//     4096) 14.2 | 13.3, (25600, 4096) 68 | 44; fp32, 4 rows: (2048, 2048) 8.0 | 9.2, (2048, 4096) 9.8 | 12.1, (2048, 6144) 15.5 | 14.3, (4096, 3072) 15.8
+//     | 13.9, (25600, 4096) 76.2 | 76.3
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border)
 {
     struct Tile {
@@ -356,7 +359,14 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
             break;
         }
     }
-    best.narrow = groups <= 64 && !pairs && rows <= 16 && steps <= 64;  // short sums: the way through memory costs more than it gives
+    if (items == 1 && !pairs && rows <= 32 && groups < 200) {
+        const int    wgs = (cols + 15) / 16, len = ((steps + sp - 1) / sp + 7) / 8 * 8;
+        const double slices = std::max(1.0, groups * sp / 256.0) * len * step + (sp > 1 ? 7.0 : 2.5);
+        best.narrow = (elem == 4 ? wgs <= 256 && steps <= 128 : wgs <= 512) && (wgs + 255) / 256 * (steps * 64.0 * (16 + 0.6 * rows) / 25e3) + 2.5 < slices;
+    }
+    else {
+        best.narrow = groups <= 64 && !pairs && rows <= 16 && steps <= 64;  // short sums: the way through memory costs more than it gives
+    }
     if (best.narrow) {
         sp = 1;
     }
@@ -404,8 +414,13 @@ static int launch_dense_skinny(const StreamArgs& a, const DenseCall& call, int v
 template<class T, int MT, int NT>
 static int launch_dense_narrow(const StreamArgs& a, const DenseCall& call, int vec, int items, hipStream_t st)
 {
-    constexpr int W = MT * NT <= 2 ? 16 : 8;
-    stream_narrow_kernel<T, DenseEpi<T, -1>, MT, NT, W><<<dim3((a.tiles + NT - 1) / NT, items * a.row_blocks), W * 64, 0, st>>>(a, DenseEpi<T, -1>{call, vec});
+    const dim3 grid((a.tiles + NT - 1) / NT, items * a.row_blocks);
+    if (MT * NT <= 2 && stream_narrow_waves(a) == 16) {
+        stream_narrow_kernel<T, DenseEpi<T, -1>, MT, NT, MT * NT <= 2 ? 16 : 8><<<grid, 1024, 0, st>>>(a, DenseEpi<T, -1>{call, vec});
+    }
+    else {
+        stream_narrow_kernel<T, DenseEpi<T, -1>, MT, NT, 8><<<grid, 512, 0, st>>>(a, DenseEpi<T, -1>{call, vec});
+    }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }

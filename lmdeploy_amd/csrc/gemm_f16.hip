@@ -91,8 +91,12 @@ template<int MT>
 static int launch_skinny(const StreamArgs& a, const F16Epi& epi, int splits, bool narrow, hipStream_t st)
 {
     if (narrow) {
-        constexpr int W = MT <= 2 ? 16 : 8;
-        stream_narrow_kernel<half_t, F16Epi, MT, 1, W><<<dim3(a.tiles, a.row_blocks), W * 64, 0, st>>>(a, epi);
+        if (MT <= 2 && stream_narrow_waves(a) == 16) {
+            stream_narrow_kernel<half_t, F16Epi, MT, 1, MT <= 2 ? 16 : 8><<<dim3(a.tiles, a.row_blocks), 1024, 0, st>>>(a, epi);
+        }
+        else {
+            stream_narrow_kernel<half_t, F16Epi, MT, 1, 8><<<dim3(a.tiles, a.row_blocks), 512, 0, st>>>(a, epi);
+        }
     }
     else {
         stream_skinny_kernel<half_t, F16Epi, MT, 1, 4, 1><<<dim3((a.tiles + 3) / 4, a.row_blocks, splits), 256, 0, st>>>(a, epi);

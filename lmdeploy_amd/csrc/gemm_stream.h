@@ -764,6 +764,12 @@ struct StreamPlan {
 // column tiles; ws_bytes / tickets: what slices of k may use (0: no slices); border: x is read elsewhere from multiples of this many columns on (a
 // multiple of 128; 0: nowhere)
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0);
+// waves of the narrow kernel (row tiles x column tiles <= 2): eight where sixteen would have nothing to do, or would keep a second workgroup off the CU
+inline int stream_narrow_waves(const StreamArgs& a)
+{
+    return a.steps <= 64 || a.tiles > 256 ? 8 : 16;
+}
+
 constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
 constexpr int    kStreamTickets = 4096;
 
