@@ -327,8 +327,8 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
         int    rows, cols;
         double full16, alone16, full32, alone32, fixed;
     };
-    static const Tile kTiles[] = {{256, 256, 0.83, 0.83, 1e9, 1e9, 8.0}, {256, 128, 0.46, 0.55, 1.75, 1.75, 5.0}, {128, 128, 0.283, 0.40, 0.90, 0.95, 3.0},
-                                  {64, 64, 0.125, 0.25, 0.24, 0.32, 1.0}};
+    static const Tile kTiles[] = {{256, 256, 0.83, 0.83, 1e9, 1e9, 8.0}, {256, 128, 0.46, 0.55, 1.75, 1.75, 5.0}, {128, 128, 0.283, 0.30, 0.90, 0.95, 3.0},
+                                  {64, 64, 0.125, 0.15, 0.24, 0.32, 1.0}};
     StreamPlan        best{};
     double            cost = 1e30;
     for (int k = 0; k < 4; ++k) {
@@ -434,7 +434,7 @@ static dim3 stream_tile_grid(const StreamArgs& a, int bm, int bn, const DenseCal
 template<class T, int EPI, int BM, int BN, int WM, int WN>
 static int launch_dense_tile(const StreamArgs& a, const DenseCall& call, int vec, hipStream_t st)
 {
-    constexpr int lds = 3 * (BM + BN) * 64;
+    constexpr int lds = stream_tile_bufs(BM, BN) * (BM + BN) * 64;
     const auto    k   = stream_tile_kernel<T, DenseEpi<T, EPI>, BM, BN, WM, WN>;
     if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {
         return rc;

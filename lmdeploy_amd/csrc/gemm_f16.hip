@@ -72,13 +72,19 @@ struct F16Epi {
     }
 };
 
-// 17 ... 64 rows of a wide output stay on gemm_kernel, whose 128-column workgroups read x half as often where all of them are busy anyway: (K, N) =
-// (4096, 28672) 64 rows 44 us against 53, 32 rows 40 against 42; (4096, 128256) 64 rows 191 against 216, 16 rows 169 against 165; (4096, 14336) 64
-// rows 37 against 32; (14336, 4096) 64 rows 101 against 33.  (Workgroups of 128 columns in the stream kernel: 52, 42, 215, 166, 43, 44 us.)
+// Where gemm_kernel is still the better one: its workgroups of 64 rows x 128 columns take the weights straight into registers and read x half as often as 64
+// columns do, so it wins where about one round of them keeps the CUs busy.  us, gemm_kernel | here, weights from HBM:
+//   up to 16 rows, 192 ... 256 workgroups: (K, N) = (4096, 28672) gated 36.4 | 39.6, (5120, 27648) gated 43.3 | 48, (4096, 32000) 40.4 | 42.2; not (4096,
+//     14336) 29.6 | 28.1, (2048, 92544) 59 | 58
+//   17 ... 64 rows, from 112 on: (2048, 16384) gated, 32 rows 17.0 | 18.6, (4096, 14336) 48 rows 33 | 35, (4096, 128256) 64 rows 191 | 216; not (4096,
+//     8192) gated 0.71 - 0.79 of its time here, (14336, 4096) 64 rows 98 | 35
+//   more rows, one round of them where 64 x 64 tiles take two: (2048, 16384) gated, 128 rows 20.9 | 26, (4096, 6144) 192 rows 30 | 42, (4096, 4096) 320 rows 29 |
+//     39, (14336, 4096) 320 rows 92 | 130; not where one round of tiles is enough, (4096, 4096) 256 rows 29 | 23, nor where it takes two, 640 rows 58 | 45
 bool f16_stream_supported(const LinearWeight& w, int M)
 {
-    return w.type == 1 && w.packed && (size_t)w.K * w.N * 2 < ((size_t)1 << 31)  // (byte offsets inside the image are 32 bits)
-           && !(M > 16 && M <= 64 && w.N >= 24576);
+    const int  rb = (M + 63) / 64, t64 = (w.N + 63) / 64 * rb, t128 = (w.N + 127) / 128 * rb;
+    const bool general = M <= 16 ? t128 >= 192 && t128 <= 256 : M <= 64 ? t128 >= 112 : t64 > 256 && t128 <= 256;
+    return w.type == 1 && w.packed && (size_t)w.K * w.N * 2 < ((size_t)1 << 31) && !general;  // (byte offsets inside the image are 32 bits)
 }
 
 int f16_stream_splits(const LinearWeight& w, int M)
@@ -108,7 +114,7 @@ static int launch_skinny(const StreamArgs& a, const F16Epi& epi, int splits, boo
 template<class K>
 static int launch_tiles(K kernel, const StreamArgs& a, const F16Epi& epi, int bm, int bn, hipStream_t st)
 {
-    const int lds = 3 * (bm + bn) * 64;
+    const int lds = stream_tile_bufs(bm, bn) * (bm + bn) * 64;
     if (const int rc = ensure_dynamic_lds((const void*)kernel, lds)) {
         return rc;
     }

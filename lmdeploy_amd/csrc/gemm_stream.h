@@ -400,9 +400,9 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
 }
 
 // ---- many rows: tiles staged in LDS by DMA -------------------------------------------------------------------------------------------
-// Workgroup tile BM x BN, 4 waves of (BM / WM) x (BN / WN) outputs, one step of k (64 bytes a row) per stage, three stages in LDS.  The fragments of
-// step s + 1 are read into a second register set under the MFMAs of step s, so the stage of step s is free when step s begins: the DMA of stage s + 3
-// is issued there and has two steps to land.  One barrier a step.  Weight blocks are lane-linear in memory and in LDS; a row of x is four
+// Workgroup tile BM x BN, 4 waves of (BM / WM) x (BN / WN) outputs, one step of k (64 bytes a row) per stage, B = three to six stages in LDS.  The fragments of
+// step s + 1 are read into a second register set under the MFMAs of step s, so the stage of step s is free when step s begins: the DMA of stage s + B
+// is issued there and has B - 1 steps to land.  One barrier a step.  Weight blocks are lane-linear in memory and in LDS; a row of x is four
 // 16-byte pieces, piece c of row r at c ^ ((r >> 1) & 3) (the swizzle is on the DMA's source address): fragment reads meet every bank once.
 __device__ __forceinline__ void stream_dma16(__amdgpu_buffer_rsrc_t rs, int voff, int soff, unsigned lds)
 {
@@ -455,12 +455,20 @@ __device__ __forceinline__ StreamTile stream_tile_of(const StreamArgs& a, const 
     return t;
 }
 
+// Stages of a tile in LDS.  The small tiles are what a few hundred rows of a narrow product get, about one workgroup a CU: only the bytes in flight hide the
+// way to memory.  fp16, weights from HBM, 200 rows of (4096, 4096) in 64 x 64 tiles: three stages 38 us, four 28, six 19.9, eight 18.6 (300 rows, two tiles on
+// some CUs: 41, 37, 37, 38); 400 rows of (5120, 5120) in 128 x 128 tiles: three 57, four 44
+constexpr int stream_tile_bufs(int bm, int bn)
+{
+    return bm == 64 && bn == 64 ? 6 : bm == 128 && bn == 128 ? 4 : 3;
+}
+
 template<class T, class Epi, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_kernel(StreamArgs a, Epi epi)
 {
     static_assert(WM * WN == 4, "four waves");
     constexpr int MI = BM / WM / 16, NI = BN / WN / 16;
-    constexpr int kXB = BM * 64, kWB = BN * 64, kStage = kXB + kWB, kBufs = 3;
+    constexpr int kXB = BM * 64, kWB = BN * 64, kStage = kXB + kWB, kBufs = stream_tile_bufs(BM, BN);
     constexpr int kXP = BM / 16 / 4, kWP = BN / 16 / 4;  // DMA pieces of one KB per wave and stage
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -529,22 +537,23 @@ __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_k
     constexpr int kPieces = kXP + kWP;
     // no branch inside a step (the reads and MFMAs of one block are interleaved): past the end the DMA fetches the last stage again, into
     // buffers that are not read any more
-    dma(0, 0);
-    dma(min(1, steps - 1), 1);
-    dma(min(2, steps - 1), 2);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPieces) : "memory");
+#pragma unroll
+    for (int b = 0; b < kBufs; ++b) {
+        dma(min(b, steps - 1), b);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kBufs - 1) * kPieces) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     read(0, 0);
     int  buf  = 0;  // stage of step s
     auto step = [&](auto Q, int s) {
         constexpr int q   = decltype(Q)::value;
-        const int     nxt = buf == 2 ? 0 : buf + 1;
+        const int     nxt = buf == kBufs - 1 ? 0 : buf + 1;
         // this wave's fragments of step s are in registers and its pieces of stage s + 1 have landed; then everybody's
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPieces) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kBufs - 2) * kPieces) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        dma(min(s + 3, steps - 1), buf);
+        dma(min(s + kBufs, steps - 1), buf);
         read(q ^ 1, nxt);
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
@@ -755,6 +764,12 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
 #define TM_STREAM_SHAPES(X) X(1, 1, 4, 1) X(2, 1, 4, 1) X(4, 1, 4, 1)
 #define TM_STREAM_SHAPES_PAIRS(X) X(1, 2, 4, 2) X(2, 2, 4, 2) X(4, 2, 4, 1)
 
+// waves of the narrow kernel (row tiles x column tiles <= 2): eight where sixteen would have nothing to do, or would keep a second workgroup off the CU
+inline int stream_narrow_waves(const StreamArgs& a)
+{
+    return a.steps <= 64 || a.tiles > 256 ? 8 : 16;
+}
+
 struct StreamPlan {
     bool skinny, narrow;  // narrow: few columns and nothing to meet in across workgroups
     int  mt, splits, split_steps, row_blocks;  // skinny kernel
@@ -764,12 +779,6 @@ struct StreamPlan {
 // column tiles; ws_bytes / tickets: what slices of k may use (0: no slices); border: x is read elsewhere from multiples of this many columns on (a
 // multiple of 128; 0: nowhere)
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0);
-// waves of the narrow kernel (row tiles x column tiles <= 2): eight where sixteen would have nothing to do, or would keep a second workgroup off the CU
-inline int stream_narrow_waves(const StreamArgs& a)
-{
-    return a.steps <= 64 || a.tiles > 256 ? 8 : 16;
-}
-
 constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
 constexpr int    kStreamTickets = 4096;
 

@@ -129,6 +129,9 @@ def test_row_tiles_of_many_items(cuda, tmp_path):
     (4096, 544, 0, (3, 20, 64)),
     (1024, 24576, 1, (16, 17, 64)),                   # both sides of the line to the general kernel
     (512, 9216, 1, (513, 2111)),
+    (128, 4096, 0, (256, 257, 512, 513)),             # ... and of the lines at one round of 64 x 64 tiles, or of the general kernel's 64 x 128
+    (128, 14336, 0, (16, 17, 64, 65, 128, 129)),
+    (128, 32784, 0, (15, 17)),                        # ... and where that has just more than one round for a few rows
 ])
 def test_f16_linears_at_the_edges(tm, cuda, K, N, gated, rows):
     g = torch.Generator('cuda').manual_seed(K + N)
