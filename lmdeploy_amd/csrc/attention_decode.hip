@@ -112,12 +112,15 @@ __global__ __launch_bounds__(256, 2) void decode_attention_kernel(DecodeAttnPara
 
     const int ctx        = p.k_len[b];
     const int tiles      = (ctx + TILE - 1) / TILE;
-    const int per_split  = max((tiles + p.splits - 1) / p.splits, p.split_tiles);
-    const int tile_begin = split * per_split;
-    const int tile_end   = min(tile_begin + per_split, tiles);
-    const int nsplit     = max((tiles + per_split - 1) / per_split, 1);  // splits with keys: the others leave at once
-    if (split >= nsplit) {
-        return;
+    int tile_begin = 0, tile_end = tiles, nsplit = 1;  // nsplit: splits with keys, the others leave at once
+    if (p.splits > 1) {                                // (no divisions ahead of the first load without splits)
+        const int per = max((tiles + p.splits - 1) / p.splits, p.split_tiles);
+        tile_begin    = split * per;
+        tile_end      = min(tile_begin + per, tiles);
+        nsplit        = max((tiles + per - 1) / per, 1);
+        if (split >= nsplit) {
+            return;
+        }
     }
 
     // ---- queries: q[h][E dims of chunk c] as half2 pairs, kept in registers ------------------
