@@ -868,8 +868,8 @@ static bool gen_entry_valid(int kind, int role, int K, int N, int M, const int v
     if (kind == kGenGrouped) {  // u4 experts: 16 / 32 / 64-row tiles (decode batches only)
         return (v[0] == 16 || v[0] == 32 || v[0] == 64) && M <= 64;
     }
-    if (kind == kGenGrouped + 2) {  // e4m3 experts on the fp8 matrix cores: 32 / 64-row tiles
-        return v[0] == 32 || v[0] == 64;
+    if (kind == kGenGrouped + 2) {  // e4m3 experts on the fp8 matrix cores
+        return v[0] == 32 || v[0] == 64 || v[0] == 128;
     }
     return false;
 }
@@ -925,8 +925,8 @@ int gen_grouped_candidates(const LinearWeight& proto, int m_cap, int* rows_out, 
         }
     }
     else if (proto.type == 2) {
-        for (int r : {32, 64}) {
-            if (n < cap && (r == 32 || m_cap > 32)) {
+        for (int r : {32, 64, 128}) {
+            if (n < cap && (r == 32 || r / 2 < m_cap)) {
                 rows_out[n++] = r;
             }
         }

@@ -51,3 +51,28 @@ def test_row_tiles(tm, cuda, T, skew):
     err, ref = np.abs(host(out).astype(np.float32) - ref.astype(np.float32)), np.abs(ref.astype(np.float32))
     assert (err <= 4e-3 + 2.0**-6 * ref).all(), err.max()
     _ffi.check(tm.tm_moe_destroy(h))
+
+
+def test_tiles_of_the_measured_dispatch(tm, cuda, tmp_path):
+    """a table line decides the tile: 32, 64 and 128 rows give the same result, whatever the rule would take for these 100 tokens"""
+    rng = np.random.default_rng(5)
+    T, H, I, E, k = 100, 256, 384, 4, 2
+    x = rng.standard_normal((T, H)).astype(f16)
+    h, experts, gate = _ffi.C.c_void_p(), [], (rng.standard_normal((H, E)) * 0.2).astype(f16)
+    _ffi.check(tm.tm_moe_create(_ffi.C.byref(h), H, I, E, k, 2, 1, 1.0))
+    _ffi.check(tm.tm_moe_set_gate(h, dev(gate).data_ptr(), st()))
+    for e in range(E):
+        w1, w3 = ((rng.standard_normal((H, I)) * (0.1 / math.sqrt(H))).astype(f16) for _ in range(2))
+        (q1, s1), (q3, s3), (q2, s2) = (o.fp8_quantize_blockwise(w) for w in (w1, w3, (rng.standard_normal((I, H)) * (0.1 / math.sqrt(I))).astype(f16)))
+        q13, s13 = o.interleave_w1w3(q1, q3), np.concatenate([s1, s3], axis=1)
+        experts.append(((q13, s13), (q2, s2)))
+        _ffi.check(tm.tm_moe_set_expert(h, e, dev(q13).data_ptr(), dev(s13).data_ptr(), None, dev(q2).data_ptr(), dev(s2).data_ptr(), None, st()))
+    ref = o.moe_ffn_fp8(x, gate, experts, k)[0].astype(np.float32)
+    ws, table = torch.zeros(tm.tm_moe_workspace(h, T), dtype=torch.uint8, device='cuda'), tmp_path / 't.txt'
+    for rows in (32, 64, 128):
+        table.write_text(f'G 34 0 {H} {2 * I} {T} {rows} 0 0 0\nG 34 0 {I} {H} {T} {rows} 0 0 0\n')
+        _ffi.check(tm.tm_gemm_import(str(table).encode()))
+        out = torch.zeros((T, H), dtype=torch.float16, device='cuda')
+        _ffi.check(tm.tm_moe_forward(h, out.data_ptr(), dev(x).data_ptr(), T, ws.data_ptr(), None, None, st()))
+        assert (np.abs(host(out).astype(np.float32) - ref) <= 4e-3 + 2.0**-6 * np.abs(ref)).all()
+    _ffi.check(tm.tm_moe_destroy(h))
