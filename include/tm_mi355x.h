@@ -307,6 +307,8 @@ int     tm_debug_trace_arena(void* dev_buf, int64_t capacity_workgroups);
 int64_t tm_debug_trace_records(char* host_out, int64_t cap);
 /* Host-only: the (workgroup shape, split-K) the decode GEMM dispatch picks for a W4A16 linear of K x N at M rows --
  * use_table bit 0: the measured table first (tm_engine_tune_gemm / tm_gemm_import), then the heuristic; clear: heuristic only;
+ * bit 1: of a launch without a folded norm (tm_linear_forward, and the engine unless TM_FOLD_NORM asks for folded norms); clear: the heuristic of
+ * the folded launches, which differs up to 32 rows of narrow and for 65 .. 256 rows of small projections;
  * bits 8 .. 11: the linear's role -- 0 any, 1 w_qkv, 2 wo, 3 w1w3, 4 w2 (the table is keyed (role, K, N, M): the tuner times each
  * role with its own consumer kernel; an entry of role 0, e.g. an imported line without a role column, serves every role).
  * Shapes: 0..3 decode tiles (M <= 64), 4 / 5 the 128-row tiles (M > 64), 6..9 shapes 3, 0, 2, 1 on 32-row blocks

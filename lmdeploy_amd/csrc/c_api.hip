@@ -980,7 +980,7 @@ int tm_debug_pick_tiling(int K, int N, int M, int use_table, int* shape, int* sp
     w.N    = N;
     w.role = (use_table >> 8) & 0xf;  // 0 any, 1 w_qkv, 2 wo, 3 w1w3, 4 w2: the measured table is keyed (role, K, N, M)
     TM_REQUIRE(w.role <= 4, "role 0 .. 4 in bits 8 .. 11 of use_table");
-    dec32_pick_ex(w, M, shape, splits, (use_table & 1) != 0);
+    (use_table & 2 ? dec32_pick_plain : dec32_pick_ex)(w, M, shape, splits, (use_table & 1) != 0);
     return 0;
 }
 

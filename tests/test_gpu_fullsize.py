@@ -120,9 +120,11 @@ def test_w4a16_every_tuner_candidate_full_size(tm, cuda, K, N, gated, M):
     x_d = dev(x)
     cands = _candidates(tm, K, N, M)
     assert len(cands) >= (8 if M <= 256 else 2), cands
-    hs, hp = _ffi.C.c_int(0), _ffi.C.c_int(0)
-    _ffi.check(tm.tm_debug_pick_tiling(K, N, M, 0, _ffi.C.byref(hs), _ffi.C.byref(hp)))
-    for shape, splits in cands + [(hs.value, hp.value)]:
+    for rule in (0, 2):                                  # the heuristic's picks with and without a folded norm
+        hs, hp = _ffi.C.c_int(0), _ffi.C.c_int(0)
+        _ffi.check(tm.tm_debug_pick_tiling(K, N, M, rule, _ffi.C.byref(hs), _ffi.C.byref(hp)))
+        cands.append((hs.value, hp.value))
+    for shape, splits in cands:
         y = torch.zeros((M, N // 2 if gated else N), dtype=torch.float16, device='cuda')
         _ffi.check(tm.tm_linear_forward(h, x_d.data_ptr(), K, y.data_ptr(), y.shape[1], M, gated, 0, splits, 0x200 | shape, ws.data_ptr(), st()))
         err = np.abs(host(y).astype(np.float32) - ref)

@@ -61,6 +61,19 @@ def test_dispatch_table_is_keyed_by_role(tmp_path):
         _pick(lib, K, N, M, table=1, role=5)
 
 
+def test_reported_tiling_of_launches_without_a_folded_norm():
+    """bit 1 of use_table (and Engine.pick_tiling) report the tiling that plain launches take: 64-column tiles for up to 32 rows of narrow projections, row
+    blocks of 32 for 65 .. 256 rows of small ones, and between those the heuristic that both kinds of launch share"""
+    from lmdeploy_amd.turbomind.engine import Engine
+    lib = _ffi.load()
+    assert _pick(lib, 4096, 6144, 8, 2)[0] == 3 and _pick(lib, 4096, 4096, 32, 2)[0] == 3 and _pick(lib, 14336, 4096, 1, 2)[0] == 3
+    assert _pick(lib, 4096, 4096, 128, 2)[0] == 6 and _pick(lib, 4096, 4096, 256, 2)[0] == 6 and _pick(lib, 14336, 4096, 65, 2)[0] == 6
+    for K, N, M in ((4096, 6144, 33), (4096, 28672, 64), (4096, 28672, 8), (16384, 6144, 1), (13824, 5120, 128), (4096, 28672, 8192)):
+        assert _pick(lib, K, N, M, 2) == _pick(lib, K, N, M, 0), (K, N, M)
+    assert Engine.pick_tiling(4096, 6144, 8, use_table=False) == _pick(lib, 4096, 6144, 8, 2)
+    assert Engine.pick_tiling(4096, 6144, 8, use_table=False, folded=True) == _pick(lib, 4096, 6144, 8, 0)
+
+
 def test_decode_gemm_heuristic_equals_the_measured_winners(tmp_path):
     """dec32_pick (host code): on the Llama-3-8B decode shapes the heuristic picks what the start-up tuner measured as
     fastest on MI355X (profiles/r02_gemm_tune_measurements.txt); wide / tiny linears and other batch sizes keep the older
