@@ -8,10 +8,13 @@ import pytest
 import torch
 
 from lmdeploy_amd import _ffi
+from tests import bedenex_oracle as bo
 from tests import febivik_oracle as fo
 from tests import layered_oracle as lo
 from tests import roravik_oracle as ro
 from tests.gpu_helpers import release_all, st
+from tests.test_gpu_bedenex import engine as bedenex_engine
+from tests.test_gpu_bedenex import model_folder as bedenex_folder
 from tests.test_gpu_febivik import engine, model_folder
 from tests.test_gpu_febivik import rel_err as rel_err_febivik
 from tests.test_gpu_layered import _layer, engine_for, rel_err
@@ -170,16 +173,44 @@ def stream_errs(eng, toks, trail):
 
 
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
-@pytest.mark.parametrize('rows', [2048, 3000])
-def test_segments_that_begin_at_odd_multiples_of_128(cuda, tmp_path, dtype, rows):
+@pytest.mark.parametrize('rows,right_heads', [(2048, 5), (3000, 5), (3000, 4)])
+def test_segments_that_begin_at_odd_multiples_of_128(cuda, tmp_path, dtype, rows, right_heads):
     """the projections of a parallel pair of mixers are one product whose columns read six inputs of a row: borders at 2048, 2688, 3328, 3968 and 4608, of
-    which 2688 and 3968 lie in the middle of 256 columns, at row counts where a product of one input takes 256-column tiles.  bf16 rounds the mixed rows, the
+    which 2688 and 3968 lie in the middle of 256 columns (four heads: all at multiples of 256), at row counts where a product of one input takes
+    256-column tiles.  bf16 rounds the mixed rows, the
     queries, keys, values and weights of the window, the joined heads and the matrices' inputs, 2^-9 each, and a norm behind the sum scales a small
     row up: within 4e-2 of the stream's size; a projection of the wrong input is 0.3 off in every row"""
-    cfg = ro.make_config(128, 97, [ro.parallel_layer(8, 4, 128, 128, 64, 5, 128)])
+    cfg = ro.make_config(128, 97, [ro.parallel_layer(8, 4, 128, 128, 64, right_heads, 128)])
     toks = np.random.default_rng(rows).integers(0, 97, rows).tolist()
     folder, w = roravik_folder(tmp_path, cfg, 3)
     eng = roravik_engine(folder, dtype, max_batch_size=1, session_len=3072, cache_blocks=64, max_prefill_token_num=3072)
     errs = stream_errs(eng, toks, ro.forward(cfg, w, toks, True)[1])
     eng.close()
     assert errs.max() <= (3e-5 if dtype == 'float32' else 4e-2), np.sort(errs)[-5:]
+
+
+def _wide_models():
+    """one-layer models and row counts at which the products named take 256 x 256 tiles (plan of the bf16 kernels), ragged in rows"""
+    ret = dict(heads=2, dim=16, vdim=16, decay=[0.8, 0.99])
+    light = dict(heads=2, dim=16, vdim=16, decay=[0.8, 0.99])
+    return {
+        'gate and up in one tile': (ro, roravik_folder, roravik_engine, ro.make_config(4608, 97, [ro.retention_layer(**ret, mlp=ro.dense(4096))]), 2000),
+        'gate and up, row tiles of items': (ro, roravik_folder, roravik_engine,
+                                            ro.make_config(4608, 97, [ro.retention_layer(**ret, mlp=ro.moe(2, 2, 2048, 1, 1, 2048))]), 1000),
+        'row tiles of items': (fo, model_folder, engine, fo.make_config(512, 97, [fo.lightning_layer(**light, mlp=fo.moe(2, 2, 2048))]), 2990),
+        'activation with two numbers': (fo, model_folder, engine, fo.make_config(512, 97, [fo.lightning_layer(**light, mlp=fo.dense(4096))]), 3000),
+        'heads as items, gated sum into the stream': (bo, bedenex_folder, bedenex_engine,
+                                                      bo.make_config(2816, 97, [bo.latent_layer(8, 128, 16, 64, 512, 0.05)]), 3000),
+    }
+
+
+@pytest.mark.parametrize('name', list(_wide_models()))
+def test_epilogues_of_256_column_tiles(cuda, tmp_path, name):
+    oracle, folder, build, cfg, rows = _wide_models()[name]
+    toks = np.random.default_rng(rows).integers(0, 97, rows).tolist()
+    path, w = folder(tmp_path, cfg, 3)
+    eng = build(path, 'bfloat16', max_batch_size=1, session_len=3072, cache_blocks=64, max_prefill_token_num=3072)
+    errs = stream_errs(eng, toks, oracle.forward(cfg, w, toks, True)[1])
+    eng.close()
+    # roundings to bf16 (2^-9) of the normed rows, heads, activations and their products' inputs; a column from a wrong place is off by its own size
+    assert errs.max() <= 4e-2, np.sort(errs)[-5:]
