@@ -311,7 +311,7 @@ void dense_weight_free(DenseWeight& d)
 // The lines between the kernels are a model of one CU's time in microseconds, fitted to measurements of this file's kernels (graph replays, weights from HBM).
 //   tile kernels: (tiles of the fullest CU) x (steps x time of a step with the CU full + prologue and results), at least one tile alone.  16-bit, 8192
 //     rows, (K, N) = (4096, 21504): 256 x 256 1155 us (1.25 PFLOP/s), 256 x 128 1281, 128 x 128 1520, 64 x 64 2714; (2048, 256) with 8000 rows: 46,
-//     33, 23, 20 us; (2048, 2048) with 2600 rows: 50, 36, 35, 48 us
+//     33, 23, 20 us; (2048, 2048) with 2600 rows: 50, 36, 35, 48 us; fp16 (5120, 5120) with 400 rows: -, 74, 44, 57, (4096, 4096) with 200: -, 69, 38, 20
 //   skinny kernel: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; 25 GB/s a CU, a line of x (from L2) at 0.7 of the
 //     price of a line of weights.  32 rows bf16, (25600, 4096): one slice 119 us, four 46, eight 45; (4096, 6144): one 23, three 19, four 18 (slices of equal length);
 //     (4096, 21504): one 40, two 42; nine items of (2048, 2816): one 21, three 31; three rows fp32, (8448, 2048): one 75, eight 21; pairs, four

@@ -1,4 +1,4 @@
-// Building blocks of the unquantised products y = x . W^T (gemm_dense.hip: bf16 and fp32 checkpoint weights; gemm_w4a16.hip: the fp16
+// Building blocks of the unquantised products y = x . W^T (gemm_dense.hip: bf16 and fp32 checkpoint weights; gemm_f16.hip: the fp16
 // linears of the Llama family), one set for the three number formats.
 //
 // Weight image: 16 output columns x 64 bytes of k are one contiguous KB in MFMA fragment order, lane l holds column l % 16 and the 16 bytes at
@@ -73,9 +73,10 @@ __device__ __forceinline__ int64_t stream_weight_bytes(const StreamArgs& a, int 
 // steps at a time), and few columns are spread over the CUs by cutting k instead of the column group: KP waves share a column
 // tile inside the workgroup and meet in LDS, grid z slices of k meet in the last workgroup of a column group to arrive, which adds the
 // slices in slice order (the sum never depends on the order of arrival; no workgroup waits for another).
-// Weights run one chunk of eight steps ahead of the MFMAs in a second register buffer; all loads are unconditional (clamped).
-// 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 46 us = 4.5 TB/s, (4096, 21504) 40 us = 4.4 TB/s (with every wave reading x for itself, no
-// slices: 76 and 50); three rows fp32, (8448, 2048): 21 us = 3.3 TB/s (64 x 64 tiles: 331).
+// Weights run one chunk of eight steps ahead of the MFMAs in a second register buffer; all loads of a stage are unconditional (clamped).
+// 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 43 us = 4.8 TB/s, (4096, 21504) 38 us = 4.6 TB/s (with every wave reading x for itself, no
+// slices: 76 and 50); four rows fp32, (8448, 2048): 18 us = 3.8 TB/s (64 x 64 tiles: 331).  The loop fetches without a branch: with one around the
+// loads the two above take 52 and 42.  Its last two stages stand behind it and fetch nothing beyond the slice: 8 rows bf16 of (8448, 2048) 15.1 -> 11.8.
 template<class T, class Epi, int MT, int NT, int CW, int KP>
 __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a, Epi epi)
 {
@@ -297,8 +298,8 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
     }
 }
 
-// The same without slices across workgroups, for callers that bring no scratch and few columns: a workgroup owns NT column tiles, its W waves take chunks of
-// eight steps in turn, each reading its own rows of x, and meet in LDS in wave order.
+// The same without slices across workgroups, for callers that bring no scratch and where slices cost more than they give (stream_plan): a workgroup owns NT
+// column tiles, its W waves take chunks of eight steps in turn, each reading its own rows of x, and meet in LDS in wave order.
 template<class T, class Epi, int MT, int NT, int W>
 __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi epi)
 {
@@ -771,7 +772,7 @@ inline int stream_narrow_waves(const StreamArgs& a)
 }
 
 struct StreamPlan {
-    bool skinny, narrow;  // narrow: few columns and nothing to meet in across workgroups
+    bool skinny, narrow;  // narrow: no slices across workgroups
     int  mt, splits, split_steps, row_blocks;  // skinny kernel
     int  tile;                                 // 0: 256 x 256 (16-bit formats), 1: 256 x 128, 2: 128 x 128, 3: 64 x 64
 };
