@@ -23,6 +23,7 @@
 #include "tm_kernels.h"
 #include "decode_merge.h"
 #include <stdlib.h>
+#include <type_traits>
 
 namespace tmk {
 
@@ -84,7 +85,8 @@ __device__ __forceinline__ void dequant_chunk(const uint32_t (&raw)[KvTraits<BIT
     }
 }
 
-template<int BITS, int HPW>
+// SPLIT: the keys are shared by p.splits workgroups; without, neither the divisions nor the merge are in the kernel
+template<int BITS, int HPW, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void decode_attention_kernel(DecodeAttnParams p, int head_chunks)
 {
     using Tr                 = KvTraits<BITS>;
@@ -113,7 +115,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_kernel(DecodeAttnPara
     const int ctx        = p.k_len[b];
     const int tiles      = (ctx + TILE - 1) / TILE;
     int tile_begin = 0, tile_end = tiles, nsplit = 1;  // nsplit: splits with keys, the others leave at once
-    if (p.splits > 1) {                                // (no divisions ahead of the first load without splits)
+    if (SPLIT) {
         const int per = max((tiles + p.splits - 1) / p.splits, p.split_tiles);
         tile_begin    = split * per;
         tile_end      = min(tile_begin + per, tiles);
@@ -342,7 +344,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_kernel(DecodeAttnPara
             }
         }
     }
-    if (nsplit == 1 || !p.tickets || !ticket_last_workgroup(p.tickets + (size_t)b * p.q_heads + head0, nsplit, &sm_last)) {
+    if (!SPLIT || nsplit == 1 || !p.tickets || !ticket_last_workgroup(p.tickets + (size_t)b * p.q_heads + head0, nsplit, &sm_last)) {
         return;
     }
     for (int idx = threadIdx.x; idx < HPW * D; idx += 256) {
@@ -392,18 +394,19 @@ static int launch_bits(const DecodeAttnParams& p_in, hipStream_t st)
     p.tile_len           = KvTraits<BITS>::TILE;
     p.split_tiles        = decode_split_tiles(grid.x * grid.y);
     p.tickets            = p.ticket_count >= p.batch * p.q_heads ? p.tickets : nullptr;
+    auto launch = [&](auto HPW) {
+        if (p.splits > 1) {
+            decode_attention_kernel<BITS, decltype(HPW)::value, true><<<grid, 256, 0, st>>>(p, chunks);
+        }
+        else {
+            decode_attention_kernel<BITS, decltype(HPW)::value, false><<<grid, 256, 0, st>>>(p, chunks);
+        }
+    };
     switch (hpw) {
-        case 4:
-            decode_attention_kernel<BITS, 4><<<grid, 256, 0, st>>>(p, chunks);
-            break;
-        case 3:
-            decode_attention_kernel<BITS, 3><<<grid, 256, 0, st>>>(p, chunks);
-            break;
-        case 2:
-            decode_attention_kernel<BITS, 2><<<grid, 256, 0, st>>>(p, chunks);
-            break;
-        default:
-            decode_attention_kernel<BITS, 1><<<grid, 256, 0, st>>>(p, chunks);
+        case 4: launch(std::integral_constant<int, 4>{}); break;
+        case 3: launch(std::integral_constant<int, 3>{}); break;
+        case 2: launch(std::integral_constant<int, 2>{}); break;
+        default: launch(std::integral_constant<int, 1>{});
     }
     TM_HIP_CHECK(hipGetLastError());
     return launch_decode_reduce(p, st);
