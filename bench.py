@@ -9,7 +9,7 @@
 A "step" = one decode iteration of the whole batch (64 tokens).  Rank 0 prints ONE JSON line.
 `value` = batch * K / t, where t brackets exactly K steps (graph replays) with barrier + device sync on both
 sides, max over ranks.  Inputs (weights, KV cache of the prefilled prompts) are resident in HBM.
-`roofline` is for the kernel family that takes the most TIME of a step -- at the driver command's context the four W4A16
+`roofline` is for the kernel family that takes the most TIME of a step -- at 20 steps behind the prompts the four W4A16
 decode GEMMs of a layer (algorithmic weight bytes of the layer / the sum of their mean launch durations), else the paged decode
 attention (algorithmic KV bytes per launch / mean launch duration); the other one follows as `attention_roofline` /
 `gemm_family_roofline`, the whole step as `step_roofline`.  Durations are IN-GRAPH: a rocprofv3 --kernel-trace child run of this
@@ -29,13 +29,13 @@ sys.path.insert(0, ROOT)
 
 LLAMA3_8B = dict(hidden=4096, layers=32, q_heads=32, kv_heads=8, head_dim=128, inter=14336, vocab=128256,
                  rms_eps=1e-5)
-# BASELINE.json configs 3 / 4 (parity-test cases; `--model` lets the same harness time them)
+# further models (parity-test cases; `--model` lets the same harness time them)
 INTERNLM2_20B = dict(hidden=6144, layers=48, q_heads=48, kv_heads=8, head_dim=128, inter=16384, vocab=92544, rms_eps=1e-5)
 LLAMA3_70B = dict(hidden=8192, layers=80, q_heads=64, kv_heads=8, head_dim=128, inter=28672, vocab=128256, rms_eps=1e-5)
-# config 5: Mixtral-8x7B, fp8 block-scaled weights, 8 experts / top-2 (TP = 2 in BASELINE.json; --emulate-tp 2 = one rank)
+# Mixtral-8x7B, fp8 block-scaled weights, 8 experts / top-2 (meant for TP = 2; --emulate-tp 2 = one rank)
 MIXTRAL_8X7B = dict(hidden=4096, layers=32, q_heads=32, kv_heads=8, head_dim=128, inter=14336, vocab=32000, rms_eps=1e-5,
                     moe_experts=8, moe_top_k=2, weight_type=2)
-# config 1: the reference's own CPU-runnable case -- `--cpu-config0` times it on the host cores, no GPU involved
+# the reference's own CPU-runnable case -- `--cpu-config0` times it on the host cores, no GPU involved
 INTERNLM2_1_8B = dict(hidden=2048, layers=24, q_heads=16, kv_heads=8, head_dim=128, inter=8192, vocab=92544, rms_eps=1e-5)
 MODELS = {'llama3_8b': LLAMA3_8B, 'internlm2_20b': INTERNLM2_20B, 'llama3_70b': LLAMA3_70B, 'mixtral_8x7b': MIXTRAL_8X7B}
 HBM_PEAK_GBPS = 8000.0     # MI355X HBM3E spec (/opt/skills/guides/MI355X_MICROARCH.md); 6290 measured copy
@@ -55,7 +55,7 @@ class _Cfg:
 
 
 def algorithmic_bytes(m, batch, ctx, kv_bits, tp):
-    """SURVEY 8(d): bytes(step) = W_q + W_sz + W_head + B*ctx*kv_bytes_per_token (per rank: / tp)."""
+    """bytes(step) = W_q + W_sz + W_head + B*ctx*kv_bytes_per_token (per rank: / tp)."""
     H, D = m['hidden'], m['head_dim']
     P = m['layers'] * (H * (m['q_heads'] + 2 * m['kv_heads']) * D + m['q_heads'] * D * H + 3 * H * m['inter'])
     w = 0.5 * P + 4.0 * P / 128 + 2.0 * H * m['vocab']
@@ -146,7 +146,7 @@ def measure_attention_traffic(args, ctx_prof):
 
 
 def gemm_family_bytes(m, tp=1):
-    """SURVEY 8(d): algorithmic bytes of the four W4A16 decode linears of ONE layer -- K * N / 2 + K * N / 32 each (u4 codes + fp16 scale /
+    """algorithmic bytes of the four W4A16 decode linears of ONE layer -- K * N / 2 + K * N / 32 each (u4 codes + fp16 scale /
     zero per 128 x 1 group), per rank.  Returns ({role: bytes}, total)."""
     H, D = m['hidden'], m['head_dim']
     hq, hkv, inter = m['q_heads'] // tp, max(1, m['kv_heads'] // tp), m['inter'] // tp
@@ -168,7 +168,7 @@ def measure_in_graph_durations(args, table_text, ctx_target, layers, batch):
     """Mean IN-GRAPH launch durations of the decode kernels, measured NOW: a child run of this script under `rocprofv3 --kernel-trace`
     (tracing only, no counters) with hipGraph replays, the parent's GEMM dispatch table imported (same tilings, no tuning launches) and a
     prompt length that puts the mean context of its replayed steps at `ctx_target`.  The eager HIP-event numbers (`kernel_ms_per_step`)
-    time a slower path than the one `value` is measured on (VERDICT r05); these are the launches of the timed path itself.
+    time a slower path than the one `value` is measured on; these are the launches of the timed path itself.
     Returns ({'w_qkv' | 'wo' | 'w1w3' | 'w2' | 'attention' | 'lm_head': mean us per launch}, description) or (None, reason)."""
     import glob
     import shutil
@@ -227,7 +227,7 @@ def run_canary(args, rank, world, timeout_s=240, extra_env=None):
     """Multi-GPU runs only: before THIS process touches the device for real, a child copy of the bench (its own rendezvous port) pushes a
     2-layer model of the same width through every collective code path the real run will take with the CURRENT switches -- RCCL bring-up,
     the native communicator + its self-test, a prefill forward large enough for the side-stream micro-batch schedule, graph-captured decode
-    steps -- under a hard time limit.  No multi-rank collective of this engine has ever crossed xGMI before the driver's scaling run,
+    steps -- under a hard time limit.  No multi-rank collective of this engine has ever crossed xGMI before the first scaling run,
     and a hang inside a collective cannot be recovered in-process: the canary turns "hang -> no record at all" into "fall back to the most
     conservative switches and measure".  Returns True when the child exited 0 within the limit."""
     import subprocess
@@ -307,8 +307,8 @@ def emit_json(obj):
 
 
 def main():
-    # multi-process GPU work on this pool needs dmabuf IPC (RCCL's P2P setup fails with the legacy mode:
-    # "hipIpcGetMemHandle: invalid argument"); already exported on the driver's boxes, kept here for hand launches
+    # multi-process GPU work needs dmabuf IPC (RCCL's P2P setup fails with the legacy mode:
+    # "hipIpcGetMemHandle: invalid argument"); kept here for hand launches
     os.environ.setdefault('HSA_ENABLE_IPC_MODE_LEGACY', '0')
     ap = argparse.ArgumentParser()
     ap.add_argument('--gpus', type=int, default=1)
@@ -336,7 +336,7 @@ def main():
                          'TTFT of B simultaneous prompts is quantised by it: sequences get their first token when THEIR chunk is done')
     ap.add_argument('--decode-splits', type=int, default=0, help='split-KV count of the decode attention (0: the engine\'s heuristic)')
     ap.add_argument('--emulate-tp', type=int, default=0,
-                    help='SURVEY 8(e) on a 1-GPU box: run ONE rank\'s shard of a TP=N job (heads / inter / vocab divided by N, '
+                    help='on one GPU: run ONE rank\'s shard of a TP=N job (heads / inter / vocab divided by N, '
                          'collectives through a 1-rank RCCL communicator): per-rank kernel time only, labelled as such')
     ap.add_argument('--layered', action='store_true',
                     help='instead of the headline workload: prefill and decode throughput of a layer-list model (Fokonex blocks, bf16) at the layer '
@@ -348,7 +348,7 @@ def main():
                          'febivik (beside the Bedenex blocks at equal size), mededra (beside the Febivik blocks at equal size), sanozen (beside the '
                          'Bedenex blocks at equal size) or roravik (beside the Febivik blocks at equal size)')
     ap.add_argument('--cpu-config0', action='store_true',
-                    help='BASELINE.json configs[0] only: InternLM2-1.8B fp16 greedy decode on the host cores (oracle/cpu_baseline.py::run_config0, the '
+                    help='InternLM2-1.8B only: fp16 greedy decode on the host cores (oracle/cpu_baseline.py::run_config0, the '
                          'torch-CPU port of the reference\'s default-backend ops); prints its own JSON line; no GPU is touched')
     ap.add_argument('--layered-one', action='store_true', help='with --layered: run the design itself only, not the model beside it (kernel traces)')
     args = ap.parse_args()
@@ -412,7 +412,7 @@ def main():
         dist.init_process_group('gloo', rank=rank, world_size=world)   # control plane only; data plane = RCCL in C++
         # the canary (run_canary): every rank's child forms its own group; ANY failure -> all ranks take the conservative switches together
         if not os.environ.get('TM_BENCH_CANARY') and os.environ.get('TM_BENCH_NO_CANARY', '0') == '0' \
-                and (ranks_per_device == 1 or os.environ.get('TM_BENCH_CANARY_SHARED', '0') == '1'):     # (the latter: mechanism test on a 1-GPU box)
+                and (ranks_per_device == 1 or os.environ.get('TM_BENCH_CANARY_SHARED', '0') == '1'):     # (the latter: mechanism test on one GPU)
             ok = run_canary(args, rank, world)
             oks = [None] * world
             dist.all_gather_object(oks, bool(ok))
@@ -445,7 +445,7 @@ def main():
                      vocab=model['vocab'] // emu)
         os.environ['TM_FORCE_COMM'] = '1'      # the rank's collective code path, through a 1-rank communicator
         # a 1-rank exchange takes no time, so splitting the prefill forwards to hide it would only add launches: the emulation reports the
-        # rank's kernel time unsplit, unless the run asks for the exchange stand-in (TM_EMULATE_AR_GBPS: the overlap experiment, DESIGN 6)
+        # rank's kernel time unsplit, unless the run asks for the exchange stand-in (TM_EMULATE_AR_GBPS: the overlap experiment)
         os.environ.setdefault('TM_COMM_STREAM', '1' if float(os.environ.get('TM_EMULATE_AR_GBPS', '0') or 0) > 0 else '0')
     K, W, B, S = args.steps, args.warmup, args.batch, args.prompt_len
     P = args.profile_steps
@@ -465,7 +465,7 @@ def main():
             out = [None] * world
             dist.all_gather_object(out, h)
             return out
-        # default (round 6): RCCL for the prefill-sized forwards + the native fused all-reduce + residual + RMSNorm for the decode-sized
+        # default: RCCL for the prefill-sized forwards + the native fused all-reduce + residual + RMSNorm for the decode-sized
         # ones, taken only when its bring-up self-test passes on every rank; TM_COMM=rccl keeps RCCL alone, TM_COMM=native drops RCCL
         mode = os.environ.get('TM_COMM', 'hybrid')
         want_native = mode == 'native'
@@ -583,7 +583,7 @@ def main():
     # ---- per-kernel durations: HIP events on the engine stream, eager steps right after the timed region ----
     prof = eng.profile_decode(P) if P > 0 else {}
     ctx_prof = S + 1 + W + K + (P - 1) / 2.0
-    # ---- the rest of the 1k-out window (SURVEY 8d: 64 x 1024 generated tokens, steady state without the first steps):
+    # ---- the rest of the 1k-out window (64 x 1024 generated tokens, steady state without the first steps):
     # the timed K steps sit at the CHEAP end of the run (shortest contexts), so also report the rate over everything
     # from the first timed step to the 1024th generated token (the P eager profile steps advance the context but are
     # not part of either time)
@@ -718,7 +718,7 @@ def main():
                 a2 = per_launch_bytes / (ing['attention'] * 1e-6) / 1e9
                 attn_obj.update(achieved=round(a2, 1), frac=round(a2 / HBM_PEAK_GBPS, 4), us_per_launch=round(ing['attention'], 2),
                                 timing=ing_src, us_per_launch_eager=round(per_launch_s * 1e6, 2))
-            # `roofline` = the kernel (family) that takes the most time of a step: at the driver command's context
+            # `roofline` = the kernel (family) that takes the most time of a step: at 20 steps behind the prompts
             # the four W4A16 decode GEMMs of a layer; the attention and the whole step follow as named extras
             gemm_roles = ('w_qkv', 'wo', 'w1w3', 'w2')
             if ing and all(r in ing for r in gemm_roles):
@@ -756,7 +756,7 @@ def main():
                                     'peak': HBM_PEAK_GBPS, 'unit': 'GB/s',
                                     'frac': round(wbytes / (gemm_ms / 1e3) / 1e9 / HBM_PEAK_GBPS, 4),
                                     'bytes_per_step': int(wbytes)}
-            # matrix-pipe view of the same four GEMMs (north_star: "MFMA utilisation for the dequant-GEMM against gfx950 peak"):
+            # matrix-pipe view of the same four GEMMs (MFMA utilisation of the dequant-GEMM against gfx950 peak):
             # 2 * B * (quantised linear parameters) flop per step over their time, against the dense fp16 peak of 2.5 PFLOP/s
             lin_params = model['layers'] * (H_ * (hq_l + 2 * hkv_l) * D_ + hq_l * D_ * H_ + 3 * H_ * I_l) if not model.get('moe_experts') else 0
             if lin_params:
@@ -775,7 +775,7 @@ def main():
                                                 'ratio': round(gemm_traffic['bytes_per_layer'] / alg, 4), 'launches': gemm_traffic['launches'],
                                                 'source': 'FETCH_SIZE x 1024 x 2 of the M <= 64 GEMM dispatches in the child PMC pass'}
         if full is not None:
-            out['value_1k_out'] = full['value']      # the metric-faithful rate: all 1024 generated tokens of the batch (SURVEY 8d)
+            out['value_1k_out'] = full['value']      # the metric-faithful rate: all 1024 generated tokens of the batch
             out['value_full_run'] = full
             out['value_full_run']['step_roofline_frac'] = round(
                 algorithmic_bytes(model, B, (full['ctx_first'] + full['ctx_last']) / 2.0, kv_bits, tp)[0] / (full['ms_per_step'] / 1e3) / 1e9

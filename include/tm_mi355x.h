@@ -184,18 +184,17 @@ int    tm_linear_forward(const tm_linear* w, const void* x, int ldx, void* y, in
                          int nt, int splits, int waves, void* workspace, tm_stream_t st);
 /* tm_linear_dequant_f16: the fp16 image [N][K] of the weights, bit for bit the operand the W4A16 kernels build on chip
  * (w = h(fma(h(q), s, h(-z*s))), kernels/gemm/transform.h:34-74) -- what the reference's own tests call quant_vs_dequant
- * (tests/turbomind/linear/fixture.py:404-507).  (Round 3 also exported tm_f16_library_available / tm_linear_build_f16_image:
- * prefill-sized forwards through a vendor fp16 GEMM on that image -- removed in round 4, every GEMM of this library is its own.) */
+ * (tests/turbomind/linear/fixture.py:404-507).
+ * (Every GEMM of this library is its own: there is no path through a vendor fp16 GEMM on that image.) */
 int    tm_linear_dequant_f16(const tm_linear* w, void* out_nk, tm_stream_t st);
 /* Row-parallel linear closed by residual + RMSNorm -- wo / w2 of a decoder layer at the decode batch: LlamaLinear::Forward
  * followed by invokeResidualBiasRMSNorm (src/turbomind/models/llama/unified_decoder.cc:149,226; kernels/norm/rms_norm.cu:286-362):
  *   resid += fp16(x . W);  y = RMSNorm(resid) * norm_w.
  * The GEMM (fp32 split-K slabs when it splits), then the reduce-norm kernel.
- * shape: decode tile 0..3 / 6..9 / 11, -1 = dispatch; splits: 0 = dispatch.  workspace >= tm_linear_workspace(w, M) + M * N * 2 bytes.
- * (Round 3's in-launch consumer behind a `fused` flag was removed in round 4; its two dead parameters left the signature in round 5.) */
+ * shape: decode tile 0..3 / 6..9 / 11, -1 = dispatch; splits: 0 = dispatch.  workspace >= tm_linear_workspace(w, M) + M * N * 2 bytes. */
 int    tm_linear_residual_norm(const tm_linear* w, const void* x, int ldx, void* y, void* resid, const void* norm_w, float eps, int M,
                                int shape, int splits, void* workspace, tm_stream_t st);
-/* The same pair of operators with the RMSNorm FOLDED into the two GEMMs around it (round 5; the engine's decode step at tp = 1):
+/* The same pair of operators with the RMSNorm FOLDED into the two GEMMs around it (the engine's decode step at tp = 1):
  *   RMSNorm(r) . W2 = inv[m] * sum_k (r[m,k] g[k]) W2[k,n],   inv[m] = 1 / sqrt(sum_k r[m,k]^2 / H + eps)
  * tm_linear_fold_produce -- the row-parallel linear (wo / w2): resid += fp16(x . W) in the GEMM's own epilogue (bit-identical to
  *   tm_linear_residual_norm's residual stream, split-K included: the last-arriving slice of a column tile sums the slices' fp32 slabs in
@@ -278,7 +277,7 @@ int tm_p2p_allgather(void* const* segs, int tp, int me, void* state, int rows, i
  * [256 B flags | one-shot tile 0 | tile 1 (rows x H each) | in2 | out2 (rows2 x H each)], M <= rows2; shares `state` and the call
  * sequence with the one-shot calls (it advances the epoch by two). */
 size_t tm_p2p_segment_bytes2(int rows, int rows2, int H);
-/* One-shot form whose workgroups do not wait for each other (round 6): one workgroup owns a token row end to end -- its own call counter
+/* One-shot form whose workgroups do not wait for each other: one workgroup owns a token row end to end -- its own call counter
  * (state[4 + row]), write-through system-scope stores of its partial row, ONE flag word per (sender, row) in every peer's segment, system-
  * scope loads of the peers' rows -- no tickets, no shared epoch, no residency requirement, no L2 write-back / invalidate on the path; same
  * arithmetic and bits as tm_p2p_allreduce_norm.  Segments of tm_p2p_segment_bytes_rows(rows, rows2, H) bytes = the two-shot layout followed
@@ -295,7 +294,7 @@ int tm_p2p_allreduce_norm_2shot(void* const* segs, int tp, int me, void* state, 
  * entry, loop entry, loop exit, exit, ...) of every GEMM / decode-attention workgroup launched afterwards; launches of more
  * than 8192 workgroups are not traced; NULL switches it off. */
 int tm_debug_set_gemm_trace(void* dev_buf);
-/* Arena form of the same trace (round 5, tools/fixed_cost_table.py): every traced launch (decode GEMMs, decode attention, the
+/* Arena form of the same trace (tools/fixed_cost_table.py): every traced launch (decode GEMMs, decode attention, the
  * norm kernels) is given ITS OWN region of `dev_buf` (capacity_workgroups x 8 uint64), in launch order -- so the launches of a
  * captured hipGraph keep distinct regions and one replay leaves the stamps of every kernel of the decode step.  Slots per
  * workgroup: 0 entry, 5 prologue loads issued, 1 activations landed (first stage barrier), 6 wave 0's first weight unit landed,
@@ -397,7 +396,7 @@ int tm_engine_comm_native_drop(tm_engine* e);
  * tm_engine_weight_copy : host -> device staging copy; byte size must match exactly. */
 int64_t tm_engine_weight_bytes(tm_engine* e, const char* name);
 int     tm_engine_weight_copy(tm_engine* e, const char* name, const void* host_src, int64_t bytes);
-/* Device-side synthetic init (random weights with the real shapes, SURVEY 8d): N(0,1)*0.1/sqrt(K) fp16
+/* Device-side synthetic init (random weights with the real shapes): N(0,1)*0.1/sqrt(K) fp16
  * master -> group-128 asymmetric u4; norms 1+0.02N; embeddings 0.02N.  For benchmarks without checkpoints. */
 int     tm_engine_init_synthetic(tm_engine* e, uint64_t seed);
 /* ModelRoot::prepare(): repack every linear, free staging */
@@ -736,7 +735,7 @@ int tm_sched_session_grow(struct tm_sched* s, int64_t session, int tokens);
 int tm_sched_session_close(struct tm_sched* s, int64_t session);
 
 /* ----------------------------------------------------------------------------------------------
- * Continuous batching (SURVEY 8f-1).  Replaces ModelRequest.forward / cancel + the engine thread's
+ * Continuous batching.  Replaces ModelRequest.forward / cancel + the engine thread's
  * schedule-forward-update loop (bind.cpp:743-793, engine/engine.cc:434-470,770-870, model_request.cc:36-135):
  * requests are queued, admitted in arrival order when a batch slot and enough KV blocks (prompt + max_new_tokens,
  * 64-token blocks) are free, prefilled (chunked, <= max_prefill_token_num prompt tokens per step) and then decoded
@@ -788,8 +787,8 @@ int tm_engine_wait(tm_engine* e, int64_t req_id, int have_tokens, int timeout_ms
 /* The scheduler by itself (host-only bookkeeping: queue, slots, block accounting) -- what the engine embeds,
  * exported so that its policy is testable without a GPU (engine/scheduler.cc:1018-1078 at the level used here). */
 /* Host-only, exported for the CPU tests like the scheduler below: where a tensor-parallel prefill forward of nseq sequences (row offsets
- * cu_q[0 .. nseq], cu_q[0] = 0) splits into the two micro-batches whose all-reduces overlap the other one's kernels (DESIGN.md 6;
- * no reference counterpart: the reference hides the exchange in a fused kernel, comm/cuda_ipc/fused_allreduce.cu:406-500).
+ * cu_q[0 .. nseq], cu_q[0] = 0) splits into the two micro-batches whose all-reduces overlap the other one's kernels
+ * (no reference counterpart: the reference hides the exchange in a fused kernel, comm/cuda_ipc/fused_allreduce.cu:406-500).
  * *seqs_a = sequences of the first micro-batch, *rows_a = its rows; 0 / 0: no usable boundary (fewer than two sequences, or the smaller side
  * below min_rows / 2 rows) -- the engine then splits the row-wise part of every layer by rows instead. */
 int tm_prefill_split(const int* cu_q, int nseq, int min_rows, int* seqs_a, int* rows_a);

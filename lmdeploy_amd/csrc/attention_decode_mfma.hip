@@ -12,8 +12,8 @@
 // so the MFMAs contract the RAW integer codes -- turned into fp16 with ONE v_perm per two codes and no arithmetic at
 // all: the byte b becomes the fp16 SUBNORMAL 0x00bb = b * 2^-24, which the matrix core multiplies exactly; the factor
 // 2^24 is folded into the K scale and into the final O -- and the scales touch 4 values per lane per tile instead of
-// 256.  (Round 1 used 0x64bb = 1024 + b and removed 1024 * sum_t (P s_t) at the end: the full-size parity test of
-// round 2 found the cancellation -- O ~ 1031 * sum P against a signal of ~7 * sum P for int4 -- costing up to 9e-3
+// 256.  (0x64bb = 1024 + b with 1024 * sum_t (P s_t) removed at the end was tried first: the full-size parity test
+// found the cancellation -- O ~ 1031 * sum P against a signal of ~7 * sum P for int4 -- costing up to 9e-3
 // absolute on 3 of 2048 (sequence, head) pairs at ctx ~1.6k; the subnormal form has no bias and is also cheaper.)  This is NOT the reference's rounding sequence
 // (no per-element fp16 rounding of k^ / v^): results agree with it to ~1e-3 relative, inside the stated tolerance
 // (reference Compare thresholds rtol 1e-2 / atol 1e-4, kernels/attention/test_utils.h:12-14).
@@ -61,7 +61,7 @@ struct QkvRaw {
     floatx4 a0[4], a1[4];
 };
 
-// Branch-free (round 5): fp16 input and slab input issue the same 8 loads (fp16: eight times the same 16 bytes).  A branch around the loads
+// Branch-free: fp16 input and slab input issue the same 8 loads (fp16: eight times the same 16 bytes).  A branch around the loads
 // makes the loaded registers phi values, the compiler copies them (v_mov) where the branches meet -- and a copy waits for the load: the
 // cache-block loads behind it were issued one memory round trip late (seen in the ISA).  Address space 1 spelled out for the same reason
 // as in load_tile.
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(Decode
     constexpr int D = 128;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // every kernel argument of the prologue in ONE batch of scalar loads: hipcc otherwise fetches late-used fields behind branches
-    // -- five dependent s_load round trips in front of the first cache-block load (seen in the ISA, round 5)
+    // -- five dependent s_load round trips in front of the first cache-block load (seen in the ISA)
     asm volatile("" ::"s"(p.q), "s"(p.q_stride), "s"(p.out), "s"(p.k_len), "s"(p.batch), "s"(p.q_heads), "s"(p.scale_log2), "s"(p.splits),
                  "s"(p.partial_o), "s"(p.partial_ml), "s"(p.cache.block_ptrs), "s"(p.cache.cu_block_nums), "s"(p.cache.block_stride),
                  "s"(p.cache.layer_offset), "s"(p.cache.layout.kv_heads), "s"(p.cache.layout.head_dim), "s"(p.cache.layout.block_len),
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(Decode
 
     // Context length and block pointers are SCALAR loads (constant address space spelled out: the table and k_len are read-only during the
     // launch): a few hundred ns each through the scalar cache instead of a VMEM round trip, and no vector load whose result the block
-    // loop would have to wait for with vmcnt(0).  Round 4 kept 64 pointers in a VGPR (v_readlane per block) and re-fetched the window
+    // loop would have to wait for with vmcnt(0).  Before, 64 pointers lay in a VGPR (v_readlane per block), the window re-fetched
     // with a vector load; the pointer of the NEXT block to prefetch is now loaded one iteration ahead (ptr_next below).
     const int       bstride = p.cache.block_stride;
     const uint64_t* blocks  = p.cache.block_ptrs
@@ -243,10 +243,10 @@ __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(Decode
             // int8: token (lane/8 + 8r), 16-byte chunk lane%8 of its 128 bytes; int4: token (lane/4 + 16r), chunk lane%4 of 64
             const int row = BITS == 8 ? (lane >> 3) + 8 * r : (lane >> 2) + 16 * r;
             const int off = BITS == 8 ? min(row, last) * 128 + (lane & 7) * 16 : min(row, last) * 64 + (lane & 3) * 16;
-            // non-temporal: every cache byte is read ONCE per launch by ONE workgroup -- measured (round 3, call 8;
-            // profiles/r03_attention_nontemporal_loads.txt) 32.4 -> 30.3 us at ctx 1040, 43.3 -> 39.5 us at ctx 1536
-            // address space 1 spelled out: a pointer read from the block table is "generic" to the compiler, the loads were FLAT ones
-            // (both counters, waited for with vmcnt(0) lgkmcnt(0)) until round 5
+            // non-temporal: every cache byte is read ONCE per launch by ONE workgroup -- measured
+            // (profiles/r03_attention_nontemporal_loads.txt) 32.4 -> 30.3 us at ctx 1040, 43.3 -> 39.5 us at ctx 1536
+            // address space 1 spelled out: a pointer read from the block table is "generic" to the compiler, the loads would be FLAT ones
+            // (both counters, waited for with vmcnt(0) lgkmcnt(0))
             kreg[r]       = __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(base + koff + off));
             vreg[r]       = __builtin_nontemporal_load((const GLOBAL_AS u32x4*)(base + voff + off));
         }
@@ -293,12 +293,12 @@ __global__ __launch_bounds__(256, 2) void decode_attention_i8_mfma_kernel(Decode
     // pointers of this wave's first and second block (scalar loads; the clamp keeps the address valid when the wave has fewer blocks)
     // block tiles - 1 always exists for ctx >= 1 (the contract: tm_decode_attention* require k_len >= 1; the engine parks free slots on a
     // dummy block with k_len = 1).  The outer max keeps the index at 0 for a k_len = 0 entry all the same: its first block-table entry is
-    // read (and must be a mapped block), never blocks[-1] (ADVICE r05)
+    // read (and must be a mapped block), never blocks[-1]
     auto        in_range = [&](int t) { return max(min(max(t, tile_begin), tiles - 1), 0); };
     const char* ptr_cur  = block_ptr(in_range(tile));
     const char* ptr_next = block_ptr(in_range(tile - 4));
     if constexpr (FUSED) {
-        // One fixed order, no branch around a load (round 5): q slice, the new token's K / V slice (every wave loads one, the owner uses
+        // One fixed order, no branch around a load: q slice, the new token's K / V slice (every wave loads one, the owner uses
         // it), the RoPE rows, then the first cache block -- all in flight together, waited for one by one with exact counts.  Before, each
         // of these waited for the one in front of it (k_len -> pointer window -> qkv slabs -> cache block: four VMEM round trips).
         const int     pos   = min(ctx - 1, p.max_pos - 1);
@@ -625,7 +625,7 @@ int launch_decode_attention_i8_mfma(const DecodeAttnParams& p_in, hipStream_t st
     }
     const int chunks = group / hpw;
     // A variant with TWO kv heads per workgroup (one workgroup per CU, 9 / 8 / 8 / 9 blocks per wave instead of 5 / 4 / 4 / 4, one or two
-    // blocks in flight per wave) was built and measured in round 5 and is in the history (commit eff45b9): parity-green, 38.2-41.4 us
+    // blocks in flight per wave) was built and measured: parity-green, 38.2-41.4 us
     // against this kernel's 34.4 at ctx 1040 -- four waves per CU issue the per-block arithmetic more slowly than eight
     // (profiles/r05_attention_pair_kernel.txt).
     dim3      grid(p.cache.layout.kv_heads * chunks, p.batch, p.splits);

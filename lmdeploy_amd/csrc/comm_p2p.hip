@@ -62,7 +62,7 @@ struct P2pParams {
     int             n;
     size_t          dst_stride;
     uint64_t        timeout;  // bound of a peer wait in 100 MHz ticks (p2p_timeout_ticks)
-    // row-flag form (p2p_allreduce_norm_rows_kernel, round 6): its own two tiles and one flag word per (sender, row) in every segment
+    // row-flag form (p2p_allreduce_norm_rows_kernel): its own two tiles and one flag word per (sender, row) in every segment
     half_t*         rdata[8];
     uint32_t*       rflags[8];  // [8 senders][rows_cap]
     int             rows_cap;
@@ -70,7 +70,7 @@ struct P2pParams {
 
 // Wait bound of a peer flag, in ticks of the 100 MHz realtime counter.  TM_P2P_TIMEOUT_MS, default 30 s (read once): RCCL has no
 // bound at all, and ranks are host-driven one by one -- graph capture, a first-use code load or a descheduled host thread on ONE
-// rank must not end the job (ADVICE r03: the former bound was ~1 s of polling).  On expiry: state[3] = the epoch, the engine
+// rank must not end the job (the former bound was ~1 s of polling).  On expiry: state[3] = the epoch, the engine
 // fails the step and refuses further work (engine_comm.hip: device_marks_check).
 static std::atomic<uint64_t> g_p2p_timeout_cap{0};  // > 0: upper bound of the wait while a bring-up self-test runs (tm_engine_comm_native_selftest)
 void p2p_timeout_cap_ms(long ms)
@@ -97,9 +97,9 @@ static uint64_t p2p_timeout_ticks_base()
 
 // steps 1 + 2; the caller's writes into its own segment buffer precede (a __syncthreads in between).  `phase` = how many syncs of
 // THIS launch came before: the entry tickets (state[1]) run monotonically through a launch -- sync k publishes at ticket
-// (k + 1) * gridDim.x - 1 -- and are reset by p2p_exit only, when every workgroup is past its last sync (ADVICE r03: a reset
+// (k + 1) * gridDim.x - 1 -- and are reset by p2p_exit only, when every workgroup is past its last sync (a reset
 // between two syncs of one launch could wipe an early ticket of the second).
-// WT (round 6, the one-shot kernel): the payload went out through WRITE-THROUGH system-scope stores (sc0 sc1) and the consumer reads the
+// WT (the one-shot kernel): the payload went out through WRITE-THROUGH system-scope stores (sc0 sc1) and the consumer reads the
 // peers' rows with system-scope loads -- the drained stores are the publish, no L2 write-back (release fence, 1.7 .. 6.5 us) and no
 // cache invalidate (acquire fence, ~1.7 us) on the path of a decode-sized exchange (MI355X_MICROARCH.md, valid forms: "{sc0 sc1 stores and
 // loads both sides}"; price list: handoff-flag, drained write-through payload vs plain + release).
@@ -107,8 +107,8 @@ template<bool WT = false>
 __device__ __forceinline__ void p2p_publish_and_wait(const P2pParams& p, uint32_t epoch, uint32_t phase = 0)
 {
     const int tid = threadIdx.x;
-    // every storing wave drains its own stores before the one release below can cover them (cdna_hip_programming.md Guideline
-    // 16 pitfall 14: "only lane 0 drained" is stale under load)
+    // every storing wave drains its own stores before the one release below can cover them (with only lane 0 drained, rows are
+    // stale under load)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
@@ -174,8 +174,8 @@ __global__ __launch_bounds__(512) void p2p_allreduce_norm_kernel(P2pParams p)
     size_t    off[NV];
     bool      ok[NV];
     // ---- 0. own partial row -> own segment; the loads that do not depend on the peers are issued here as well -------------
-    // The row leaves through write-through system-scope stores (16 bytes, `sc0 sc1`; the asm ends with s_nop 1: cdna_hip_programming.md 5.7
-    // item 1): once a wave's vmcnt is 0 its part of the row is in memory, where the peers' system-scope loads find it -- no L2 write-back.
+    // The row leaves through write-through system-scope stores (16 bytes, `sc0 sc1`; the asm ends with s_nop 1, see
+    // gemm_decode_common.h): once a wave's vmcnt is 0 its part of the row is in memory, where the peers' system-scope loads find it -- no L2 write-back.
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int vi = tid + i * blockDim.x;
@@ -251,10 +251,10 @@ __global__ __launch_bounds__(512) void p2p_allreduce_norm_kernel(P2pParams p)
     p2p_exit(p, epoch);
 }
 
-// ---- one-shot form WITHOUT any coupling between the workgroups of a launch (round 6) -----------------------------------------------
+// ---- one-shot form WITHOUT any coupling between the workgroups of a launch -----------------------------------------------
 // The kernel above pays, per exchange, a local fan-in (every workgroup's ticket -> the last one publishes the call's epoch), a fan-out
 // (every workgroup polls that one flag) and an exit fan-in (the epoch word): three device-scope round trips on the critical path of a
-// 64-row decode exchange whatever the peers do (8 us per launch with ONE rank, profiles/r06_tp_default_*).  Here a workgroup owns one
+// 64-row decode exchange whatever the peers do (8 us per launch with ONE rank, measured).  Here a workgroup owns one
 // token row END TO END: it reads the row's call counter (state[4 + row], a local word only it touches), pushes its partial row into its
 // own segment with write-through system-scope stores, drains, stores the counter value into flag [me][row] of every peer's segment,
 // polls flags [q][row] of its own segment, sums the peers' rows (system-scope loads) in rank order, normalises, and writes the counter

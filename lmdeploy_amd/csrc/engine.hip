@@ -313,7 +313,7 @@ int tm_engine_init_synthetic(tm_engine* e, uint64_t seed)
             TM_HIP_CHECK(hipMalloc((void**)&master, n * 2));
             master_elems = n;
         }
-        // TM_SYNTH_WEIGHT_SCALE (diagnostics only: `0` = all-zero linear weights, the low-toggle arm of the power experiment in DESIGN 3.8)
+        // TM_SYNTH_WEIGHT_SCALE (diagnostics only: `0` = all-zero linear weights, the low-toggle arm of a power experiment)
         static const float wscale = [] {
             const char* v = getenv("TM_SYNTH_WEIGHT_SCALE");
             return v ? (float)atof(v) : 1.0f;
@@ -474,16 +474,16 @@ int tm_engine_start(tm_engine* e)
         // arrival counters: one per (column tile, row block) of the widest decode linear at its narrowest tile (64 columns, 32 rows)
         const size_t ntk = (size_t)(std::max(std::max(e->qkv_n, 2 * e->inter), e->hidden) + 63) / 64 * (kFoldMaxRows / 32);
         const char* fm   = getenv("TM_FOLD_MAX_M");
-        // default 64: at batch 128 (BASELINE config 3) the folded layer is parity-green but measured SLOWER than the reduce-norm launches it
+        // default 64: at batch 128 the folded layer is parity-green but measured SLOWER than the reduce-norm launches it
         // removes (InternLM2-20B: 10.83 .. 10.91 vs 10.43 ms per step, profiles/r06_fold128_*): its producers are limited to the 32-row-block
         // tiles (every weight unit read by four row blocks), the 128-row tile with 10 slices + the fused reduce-norm wins w2 by 4 us
         e->fold_max_rows = fm ? std::min(kFoldMaxRows, std::max(1, atoi(fm))) : 64;
         TM_TRY(dmalloc(&e->d_tickets, ntk));
         e->n_tickets = (int)ntk;
         TM_HIP_CHECK(hipMemset(e->d_tickets, 0, ntk * sizeof(unsigned)));
-        // Default 0 since round 6: the folded layer is a departure from the reference's rounding sequence (one fp16 rounding
+        // Default 0: the folded layer is a departure from the reference's rounding sequence (one fp16 rounding
         // of the normalised activations instead of two) and a default-on departure has to pay more than box noise -- four interleaved runs per arm
-        // on one box: 19 278.6 (fold 3) vs 19 283.5 tok/s (fold 0) on the driver command, 17 632.6 vs 17 619.5 over the 1k-out run
+        // on one box: 19 278.6 (fold 3) vs 19 283.5 tok/s (fold 0) over bench.py's 20 steps, 17 632.6 vs 17 619.5 over the 1k-out run
         // (profiles/r06_fold_ab.txt).  TM_FOLD_NORM=3 runs it (bit 0: wo -> w1w3, bit 1: w2 -> w_qkv); every test of it stays.
         const char* fold = getenv("TM_FOLD_NORM");
         e->fold_norm     = (!e->use_comm && m.weight_type == 0 && m.moe_experts == 0 && e->hidden % 64 == 0) ? (fold ? atoi(fold) & 3 : 0) : 0;
@@ -598,7 +598,7 @@ int tm_engine_fetch(tm_engine* e, int* host_out, int* n_generated)
         e->steps_valid = e->steps_fetched;  // the mark was first seen now: what an earlier, clean fetch reported is known to be valid
     }
     // after a communicator give-up *n_generated = the columns known to be valid (the step count of the last clean fetch): the
-    // caller can keep those and must discard the rest; the status says so (ADVICE r04)
+    // caller can keep those and must discard the rest; the status says so
     *n_generated = rc ? (e->steps_valid < 0 ? 0 : e->steps_valid) : e->steps_done;
     if (!rc) {
         e->steps_fetched = e->steps_done;

@@ -7,7 +7,7 @@ namespace tmk {
 // Stand-in for the duration of an exchange, for the ONE-rank emulation of a tensor-parallel rank only (TM_FORCE_COMM=1 / `bench.py
 // --emulate-tp N`: the communicator has one rank, its all-reduce is the identity and takes no time).  TM_EMULATE_AR_GBPS = g > 0: every
 // all-reduce of a prefill-sized forward is followed, on the stream it was enqueued on, by one idle workgroup that waits
-// 10 us + bytes / g -- what an all-reduce with algorithm bandwidth g GB/s would hold that stream for.  It lets a 1-GPU box show what the
+// 10 us + bytes / g -- what an all-reduce with algorithm bandwidth g GB/s would hold that stream for.  It lets one GPU show what the
 // two-row-half choreography hides and what it leaves exposed (profiles/r05_prefill_overlap_emulated_exchange.txt); it moves no data, is
 // never armed with more than one rank, and is not a scaling result.
 __global__ void exchange_standin_kernel(unsigned ticks)
@@ -30,7 +30,7 @@ static int exchange_standin(tm_engine* e, size_t bytes, hipStream_t st)
 
 // fp16 sum of the row-parallel partial outputs over the TP group (comm/nccl/nccl.cu:356-398 calls ncclAllReduce on the
 // compute stream).  Decode-sized forwards always take this form: a decode layer is one dependent chain, a collective between two
-// of its kernels has nothing to run beside (round 2 measured a side stream with and without a weight prefetch under it:
+// of its kernels has nothing to run beside (measured: a side stream with and without a weight prefetch under it:
 // profiles/r02_comm_stream_arms.txt).  Prefill-sized forwards overlap for real: allreduce_rows_side below.
 static int allreduce_hidden(tm_engine* e, half_t* buf, int M)
 {

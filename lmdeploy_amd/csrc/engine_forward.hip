@@ -304,7 +304,7 @@ static int linear_fold_consume(tm_engine* e, LinearSlots& l, const half_t* x, in
     const bool mrg = dec32_is_merge_shape(shape);  // split-K merged in the launch: no slab leaves it, whoever consumes
     // a split-K consumer nobody takes slabs from (w1w3; w_qkv without the fused attention prologue): the slices' slabs already carry the row
     // factor (it is applied to the accumulators before ANY epilogue, and a sum of scaled slices is the scaled sum), so the plain reduce launch
-    // finishes them -- what the 128-row tile needs at batch 128, where one slice per column tile leaves half the CUs idle (round 6)
+    // finishes them -- what the 128-row tile needs at batch 128, where one slice per column tile leaves half the CUs idle
     const bool reduce_after = !slabs_ok && !mrg && splits > 1 && M > 64;
     if (!slabs_ok && !mrg && !reduce_after) {
         splits = 1;
@@ -803,7 +803,7 @@ void setup_decode(tm_engine* e, int batch)
         const int wgs = e->kv_heads * (group / hpw) * batch;
         splits        = 1;
         // (the 256-workgroup target is what was measured: full decode batches; small batches -- typically long contexts per sequence --
-        // keep the deeper split, ADVICE r04)
+        // keep the deeper split)
         while (wgs * splits < (mfma && batch >= 32 ? 256 : 512) && splits < 16) {
             splits *= 2;
         }

@@ -222,7 +222,7 @@ struct tm_engine {
     // TM_COMM_STREAM (default 1): the all-reduces of PREFILL-sized tensor-parallel forwards run on their own stream under the other
     // row half's GEMMs (engine_comm.hip: allreduce_rows_side; engine_forward.hip: forward_tail_two_halves).  Decode-sized forwards
     // keep every collective on the engine stream: a decode layer is one dependent chain, a side stream had nothing to run beside it
-    // (profiles/r02_comm_stream_arms.txt; the fork / join arm of rounds 2-4 is gone)
+    // (profiles/r02_comm_stream_arms.txt)
     hipStream_t  comm_stream = nullptr;
     std::vector<hipEvent_t> pipe_events;      // (ready, done) pairs of the side-stream all-reduces of ONE forward
     size_t       pipe_events_used = 0;
@@ -251,7 +251,7 @@ struct tm_engine {
     bool         comm_overlap = false;   // TM_COMM_STREAM != 0 and an RCCL communicator: prefill all-reduces on comm_stream
     bool         graph_comm_failed = false;  // capturing the RCCL calls failed once: stay eager
     bool         use_comm = false;  // collectives on the data path: tp > 1 (or TM_FORCE_COMM=1: single-rank communicator,
-                                    // exercises the RCCL code path on a 1-GPU box)
+                                    // exercises the RCCL code path on one GPU)
     std::map<std::string, Slot> slots;
     std::unique_ptr<tmk::LayeredModel> lm;   // set: a layer-list model (tm_engine_create_layered); `layers` below stays empty
     std::vector<Layer>          layers;

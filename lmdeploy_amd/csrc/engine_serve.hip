@@ -16,7 +16,7 @@ __global__ void park_slot_kernel(int* active, int* k_len, uint64_t* block_row, i
 extern "C" {
 
 // ------------------------------------------------------------------------------------------------------------------
-// Continuous batching (SURVEY 8f-1): request queue + slot scheduler (scheduler.h) on top of the same forward().
+// Continuous batching: request queue + slot scheduler (scheduler.h) on top of the same forward().
 // Every decode step runs all max_batch_size slots (one graph); a free slot is parked on a scratch block with
 // k_len = 1 and its token is ignored.  A scheduler step = admit waiting requests (prefill, chunked) + one decode step
 // for everything that is running (prefill-priority, like the reference's default when new requests arrive).

@@ -207,7 +207,7 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
         // keep the heuristic unless the measurement clearly beats it.  7 %: run-to-run spread of a candidate is +-3 % (the same tiling
         // measured 18.35 / 18.72 / 19.13 us in three starts on one box), and the chain here is not the model (the same kernel back
         // to back, its activations hot in L2): with a 3 % bar w2 of Llama-3-8B once flipped from (3, 4) to (6, 2) -- 12 % slower in
-        // the model (gpurun_out/profile_r03c: 0.61 vs 0.54 ms per step)
+        // the model (0.61 vs 0.54 ms per step)
         if (!(best < 0.93f * heur)) {
             bs = hs;
             bp = hp;
@@ -226,7 +226,7 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// The same for everything that is not a P32 kernel (VERDICT r03 item 7): the dense linears gemm_kernel serves (e4m3 weight-only
+// The same for everything that is not a P32 kernel: the dense linears gemm_kernel serves (e4m3 weight-only
 // w_qkv / wo / w1w3 / w2, the fp16 lm_head) and the grouped expert GEMMs (row-tile height; u4 through gemm_kernel<GRP>, e4m3 on
 // the fp8 matrix cores).  Same method: one hipGraph per candidate over the model's own weights, min of 5 replays, a measured
 // winner replaces the heuristic only when it is >= 7 % faster.  Results enter gen_table (tm_kernels.h) and travel in the same

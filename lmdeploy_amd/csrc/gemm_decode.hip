@@ -5,7 +5,7 @@
 //           kernels/gemm/transform.h:34-74, gated-SiLU epilogue kernels/gemm/epilogue.h:159-176.
 // Arithmetic is the one of gemm_w4a16.hip: w = h(fma(h(q), s, h(-z*s))), fp32 MFMA accumulation, one rounding to fp16.
 //
-// Why a second kernel (round-1 measurements): with 8 waves per CU moving in lockstep through one barrier
+// Why a second kernel (measured): with 8 waves per CU moving in lockstep through one barrier
 // per k-block, the per-CU costs of a 16-column x 128-k weight tile ADD UP -- HBM 109 clk (at 10 B/clk/CU), MFMA 64,
 // x fragments out of LDS 64, dequant VALU 26..52, x staging -- to ~290 clk, which is what was measured (0.19 of the
 // HBM roofline).  This kernel is built so that they overlap instead:
@@ -170,14 +170,14 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_dec32_kernel(Dec32Params p)
 
     const int tid  = threadIdx.x;
     const int wgid = (blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
-    // (Round 5 measured an XCD-aware re-deal of split-K grids -- one slice's workgroups on 8 / slices XCDs, so that each L2 pulls only its
+    // (An XCD-aware re-deal of split-K grids was measured -- one slice's workgroups on 8 / slices XCDs, so that each L2 pulls only its
     // slice's columns of x: FETCH 1.40 -> 1.28 x the weight bytes and the step 1.8 % SLOWER, because the plain mapping below keeps the
     // slices of one column tile on ONE XCD, blockIdx.x % 8, which is what the slab merge wants.  Removed;
     // profiles/r05_fold_modes_and_xcd_placement_ab.txt.)
     const int bx = blockIdx.x, by = blockIdx.y;
     // every kernel argument the prologue needs, fetched by ONE batch of scalar loads at entry: left to itself hipcc sinks the loads
     // of late-used fields behind branches -- three dependent s_load round trips on the way to the first HBM request (seen in the ISA;
-    // round 5, profiles/r05_fixed_cost_by_launch.txt: "issue" 0.41 us per launch)
+    // profiles/r05_fixed_cost_by_launch.txt: "issue" 0.41 us per launch)
     asm volatile("" ::"s"(p.x), "s"(p.wp), "s"(p.y), "s"(p.partial), "s"(p.ldx), "s"(p.ldy), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.KB),
                  "s"(p.ncg), "s"(p.kb_per_split), "s"(p.epilogue), "s"(p.wt), "s"(p.dbg));
     asm volatile("" ::"s"(p.ss_in), "s"(p.ss_tiles), "s"(p.ss_inv_h), "s"(p.ss_eps), "s"(p.resid), "s"(p.norm_w), "s"(p.ss_out), "s"(p.tickets));
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_dec32_kernel(Dec32Params p)
 
     u32x4    ring[PF][2];
     uint32_t sring[PF];
-    // ---- L2 prefetch of the weight stream (ABL 0x4000 / 0x8000: one / two stages beyond the ring; round 6) ----------------------------
+    // ---- L2 prefetch of the weight stream (ABL 0x4000 / 0x8000: one / two stages beyond the ring) ----------------------------
     // The ring holds PF k-blocks per wave: a unit is requested UNR stages before its first use, and VMEM returns in order -- one late HBM
     // line holds up every younger load of the wave at its next counted wait, and the stage barrier passes the stall to the other 15
     // waves.  One more instruction per refill touches the unit the wave will request a stage (two) LATER: lane i reads 4 bytes of the
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_dec32_kernel(Dec32Params p)
                 }
                 // Not behind the last stage: nobody would read it, and the refills that the counted wait below relies on
                 // are dead code there (hipcc drops them in the remainder stage), so that DMA could still be landing when the
-                // epilogue lays the reduction image over the stage buffers (seen as flaky rows 96..127 of row blocks, r02).
+                // epilogue lays the reduction image over the stage buffers (seen as flaky rows 96..127 of row blocks).
                 if (t + 1 < nst) {  // uniform
                     D32_DMA_X(phys(t + 1), buf ^ 1);
                 }
@@ -1022,7 +1022,7 @@ __global__ __launch_bounds__(512) void gemm_pre64_kernel(Dec32Params p)
             // the issue port for 4, so ~4 VALU ops fit behind each one: a1(j) is built behind the four MFMAs that use a0(j),
             // a0(j+1) behind the four that use a1(j).  Back-to-back "dequant block, then MFMA block" (the first version of
             // this kernel, and what hipcc emits on its own) measured additive: loop 102 us = 55 us of MFMA + 42 us of
-            // everything else (profiles/r02_pre64_phase_traces.txt).
+            // everything else.
             // experiments (TM_D32_ABL, results are garbage; profiles/r04_gemm_experiments_session2.txt): 8 = the raw codes as fp16
             // subnormals on the matrix pipe instead of the dequantised operand, 16 = the accumulators rescaled once per k-block
             // (what a per-group scale applied on the accumulator side would cost)
@@ -1195,7 +1195,7 @@ static int launch_dec32_shape(const Dec32Params& p, dim3 grid, int shape, hipStr
     static const int abl = env_int2("TM_D32_ABL", -1);
 #endif
     // TM_D32_L2PF = 1 / 2 (TM_EXPERIMENTS builds): the weight stream's L2 prefetch one / two stages beyond the ring (ABL 0x4000 / 0x8000; shapes 0, 3 and
-    // their 32-row forms).  Measured negative in round 6 (profiles/r06_l2pf_*: parity-green, w1w3's loop 14.9 -> 16.1 us, driver line -1.5 .. -2 %):
+    // their 32-row forms).  Measured negative (profiles/r06_l2pf_*: parity-green, w1w3's loop 14.9 -> 16.1 us, tokens/s -1.5 .. -2 %):
     // the loop does not wait for late weight lines -- one more request per 2 KB of weights in the CU's load path costs more than it hides.
 #ifdef TM_EXPERIMENTS
     static const int l2pf = env_int2("TM_D32_L2PF", 0);
@@ -1478,7 +1478,7 @@ int dec32_candidates(const LinearWeight& w, int M, int (*out)[2], int cap)
         }
     }
     if (M <= 64) {
-        // in-launch merged split-K (kShapeMerge + shape, round 6): 2 .. 4 slices of the <= 64-row tiles.  The last arriver of a tile reads
+        // in-launch merged split-K (kShapeMerge + shape): 2 .. 4 slices of the <= 64-row tiles.  The last arriver of a tile reads
         // (slices - 1) x 64 x columns x 4 bytes on its critical path -- beyond 4 slices that is longer than the reduce launch it replaces
         const int base = n;
         for (int i = 0; i < base; ++i) {
@@ -1552,7 +1552,7 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
         // 512-column tile with two weight fragments per x-fragment read (TM_PRE64_MIN_M: first M that takes it)
         static const int pre64_from = env_int2("TM_PRE64_MIN_M", 257);
         // The 128 x 512 tile only when it alone puts ~one workgroup on most CUs; otherwise the 128 x 256 tile with at most 4
-        // split-K slices (round 3, measured by the tuner at the Llama-3-8B shapes, us per layer incl. the consumer --
+        // split-K slices (measured by the tuner at the Llama-3-8B shapes, us per layer incl. the consumer --
         // M = 512: w_qkv 49.3 -> 36.5, wo 44.9 -> 28.5, w2 74.2 -> 54.2; M = 1024: 66.8 -> 48.1, 61.4 -> 41.5, 105.5 -> 92.6;
         // M = 2048: wo 81.6 -> 61.2; from M = 4096 the wide tile wins everywhere: profiles/r03_gemm_tune_prefill_classes.txt)
         const int wgs5 = (ncg + 15) / 16 * ((M + 127) / 128);
@@ -1569,7 +1569,7 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
     // wo 14.3 -> 10.5 us, w2 18.6 -> 17.1 us, w_qkv 12.2 -> 9.8 us; profiles/r02_gemm_tune_measurements.txt); with
     // TM_GEMM_TUNE=1 the engine measures instead of trusting this rule.  The two row halves of a shape-6 column tile are
     // gridDim.x * gridDim.y workgroups apart -- the same XCD when that is a multiple of 8: the second reader hits L2.
-    // Round 4: the same rule holds for the TP-shard shapes (one rank of TP = 2 / 8 of Llama-3-8B / -70B: N = 768 .. 8192, K = 512 ..
+    // The same rule holds for the TP-shard shapes (one rank of TP = 2 / 8 of Llama-3-8B / -70B: N = 768 .. 8192, K = 512 ..
     // 8192, ragged k-block counts) -- the tuner picks shape 6 for every one of them (profiles/r04_gemm_experiments_session2.txt,
     // call23: w2 1792 x 4096 6.2 us against 10.6 for the old fall-back, w_qkv 4096 x 768 7.7 against 10.8) -- with slices of at
     // least 16 k-blocks: below that a slab boundary costs more than the workgroups it adds.
@@ -1698,7 +1698,7 @@ int launch_linear_dec32(const LinearWeight& w, const half_t* x, int ldx, half_t*
         TM_REQUIRE(!merge || (nf && nf->tickets && (M <= 64 || (M <= kFoldMaxRows && shape >= 6 && shape <= 9))),
                    "merged split-K: arrival counters (NormFold::tickets), M <= 64 (32-row-block tiles: <= 128)");
     }
-    // folded RMSNorm: M <= 64 on every <= 64-row decode tile; 64 < M <= kFoldMaxRows (round 6, BASELINE config 3 = batch 128) on the 32-row-block
+    // folded RMSNorm: M <= 64 on every <= 64-row decode tile; 64 < M <= kFoldMaxRows (batch 128) on the 32-row-block
     // tiles 6..9 (producer and consumer: one ticket / one row of sums per (column tile, row block)) and, consumer only, on the 128-row tile 4
     TM_REQUIRE(!nf || !(produce || consume)
                    || (M <= 64 ? dec32_fold_shape(shape) : (M <= kFoldMaxRows && ((shape >= 6 && shape <= 9) || (shape == 4 && !produce)))),

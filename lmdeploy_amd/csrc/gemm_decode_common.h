@@ -25,7 +25,7 @@ struct Dec32Params {
                              // release writes them back (the kernel boundary then waits for MBs of fp32 slabs)
     uint64_t*     dbg;       // optional [workgroups][8] s_memrealtime stamps (tm_debug_set_gemm_trace): start, loop, epilogue, end,
                              // hw id, -, -, after the k-phase reduction barrier
-    // ---- RMSNorm folded into the neighbouring decode GEMMs (round 5; gemm_dec32_kernel only) ------------------------------
+    // ---- RMSNorm folded into the neighbouring decode GEMMs (gemm_dec32_kernel only) ------------------------------
     // y = RMSNorm(r) . W = inv[m] * sum_k (r[m,k] g[k]) W[k,n]: the GEMM that PRODUCES r (epilogue 3) adds its fp16 output to
     // the residual stream (bit-exact: r = h(r + h(acc)), rms_norm.cu:286-362), writes xg = h(f32(r) * f32(g)) as the next
     // GEMM's activations and, per column tile, the partial row sums of f32(r)^2; the GEMM that CONSUMES xg multiplies its fp32
@@ -39,10 +39,10 @@ struct Dec32Params {
     int           ss_tiles;
     float         ss_inv_h;  // 1 / H of the norm
     float         ss_eps;
-    // ---- split-K merged INSIDE the launch for the fp16 / gated-SiLU epilogues (round 6; shapes kShapeMerge + 0..3 / 6..9): the slices
+    // ---- split-K merged INSIDE the launch for the fp16 / gated-SiLU epilogues (shapes kShapeMerge + 0..3 / 6..9): the slices
     // park their fp32 tiles write-through and take a ticket exactly as epilogue 3 does; the last arriver of a column tile sums the
     // slices in slice order from zero (the bits of splitk_reduce_kernel) and runs the epilogue.  No slab leaves the launch, no reduce
-    // launch follows: what a 256-column tile with a 2-way cross-CU k-split needs for the gated w1w3 (VERDICT r05 item 1a).
+    // launch follows: what a 256-column tile with a 2-way cross-CU k-split needs for the gated w1w3.
     int           merge;     // 1: epilogues 0 / 1 with gridDim.y > 1 merge in the launch (tickets != nullptr)
 };
 constexpr int kDec32NormLds = 32 * 64 * 4 + 512;  // consumer scratch behind the stage buffers / reduction image: [parts][rows] sums + inv[rows]
@@ -60,8 +60,8 @@ __device__ __forceinline__ floatx4 load_agent(const float* src)
 }
 
 // The 16-byte asm stores END WITH `s_nop 1`: hipcc neither counts nor pads an asm statement, and a VALU write to the store's data
-// registers within two wait states of a > 64-bit store corrupts what the store reads (cdna_hip_programming.md 5.7 item 1).  Round 6 found
-// it the hard way: the merged split-K park loop put `v_or_b32 v6, ...` one instruction behind `global_store_dwordx4 v[2:3], v[6:9]` --
+// registers within two wait states of a > 64-bit store corrupts what the store reads.
+// Found the hard way: the merged split-K park loop put `v_or_b32 v6, ...` one instruction behind `global_store_dwordx4 v[2:3], v[6:9]` --
 // dword 0 of lanes 12..15 of every 16-lane row arrived in the slab as 0.0 on some launches (tools/r06_dbg_merge.py).
 __device__ __forceinline__ void store_wt(floatx4* dst, floatx4 v, int mode = 1)
 {

@@ -5,7 +5,7 @@
 //           kernels/gemm/transform.h:34-74, gated-SiLU epilogue kernels/gemm/epilogue.h:159-176.
 // w = h(fma(h(q), s, h(-z*s))) per element (bit-identical to the reference's operand), fp32 MFMA accumulation, one rounding.
 //
-// Structure (round 4).  gemm_dec32_kernel lets every wave issue BOTH its weight-ring refills and its share of the activation
+// Structure.  gemm_dec32_kernel lets every wave issue BOTH its weight-ring refills and its share of the activation
 // DMA; VMEM returns in order, so the wait that covers a wave's activation pieces also retires every older weight load.  Here
 // the two streams live in different waves (different vmcnt queues) and a wave's tile is twice as wide:
 //   * 4 LOADER waves bring the activations of a stage (WK k-blocks x ROWS rows) into LDS by DMA (buffer_load ... lds),

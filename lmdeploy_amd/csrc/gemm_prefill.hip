@@ -4,7 +4,7 @@
 //           kernels/gemm/kernel/sm80_16816_4.cu:18-61), dequant kernels/gemm/transform.h:34-74, gated-SiLU epilogue
 //           kernels/gemm/epilogue.h:159-176.  Same operand as every other W4A16 kernel here: w = h(fma(h(q), s, h(-z*s))).
 //
-// Why (round 3 / 4 measurements): a compute-bound MFMA kernel on real data is POWER-limited (~1.6 GHz instead of
+// Why (measured): a compute-bound MFMA kernel on real data is POWER-limited (~1.6 GHz instead of
 // 2.4), and in gemm_pre64_kernel every wave dequantises its own 64 columns for 128 rows -- 13 packed VALU ops per 4 MFMAs, each
 // of them power the matrix pipe does not get (1.10 .. 1.24 PF/s against 1.42 .. 1.49 of a plain fp16 library GEMM).  Here a
 // 64-deep k-slice of 256 columns is dequantised once per workgroup (4 dwords = 52 VALU ops per thread and stage, 1.6 per MFMA)
@@ -90,8 +90,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_pre256_kernel(Dec32Params p)
                      : "memory");                                                                                 \
     }
     // half unit of stage st (k-block st / 2, half st & 1) of this wave's staging column group -> registers.  Inline asm: beside
-    // the LDS-DMA (invisible to hipcc's waitcnt pass) a compiler-counted load would be waited for with the wrong count
-    // (cdna_hip_programming.md 5.7); every load of the loop is retired by the ONE hand-written vmcnt(0) at the end of a stage.
+    // the LDS-DMA (invisible to hipcc's waitcnt pass) a compiler-counted load would be waited for with the wrong count;
+    // every load of the loop is retired by the ONE hand-written vmcnt(0) at the end of a stage.
     u32x4    wq[SG], wn[SG];
     uint32_t wsz[SG], wszn[SG];
 #define P256_LOAD_W(st, q_, sz_)                                                                                  \

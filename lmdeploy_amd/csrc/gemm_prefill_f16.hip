@@ -6,11 +6,11 @@
 //           load by dequant_p32_f16_kernel (bit for bit: tests/test_gpu_fullsize.py::test_w4a16_dequantised_image_full_size), so results
 //           are those of the fused tiles to the accumulation order.
 //
-// Why (rounds 3-6): a compute-bound MFMA kernel on real data is POWER-limited on this chip (~1.6 GHz instead of 2.4).  The fused tiles
+// Why: a compute-bound MFMA kernel on real data is POWER-limited on this chip (~1.6 GHz instead of 2.4).  The fused tiles
 // spend part of that budget on the dequantisation -- gemm_pre64_kernel: 14 packed VALU ops per 4 MFMAs in every wave; gemm_pre256_kernel:
 // 52 per thread and stage plus the LDS write pass -- and reach 1.10 .. 1.20 PF/s where a plain fp16 x fp16 GEMM reaches 1.4 .. 1.5
-// (round 3 measured the vendor library on the same image; cdna_hip_programming.md quotes 1.32 .. 1.47 PF/s on random data for its own
-// 256 x 256 LDS-DMA template).  MI355X has 288 GB of HBM: the fp16 image of an 8 B-parameter model is 14 GB.  The decode path keeps
+// (the vendor library on the same image, random data; 1.32 .. 1.47 PF/s are quoted for 256 x 256 tiles by
+// LDS DMA).  MI355X has 288 GB of HBM: the fp16 image of an 8 B-parameter model is 14 GB.  The decode path keeps
 // streaming the 4-bit image (bandwidth); prefill-sized forwards contract the fp16 image (matrix pipe), with NO VALU work in the main loop:
 //   stage = 64 k: x image 256 rows x 128 B (32 KB) + w image 256 columns x 128 B (32 KB), both row-major with the 16-byte chunks
 //   XOR-swizzled by (row >> 1) & 7 on the SOURCE address of the DMA (the LDS image is lane-linear), double buffered (128 KB);

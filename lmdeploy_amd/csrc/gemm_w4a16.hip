@@ -825,7 +825,7 @@ bool gen_table_get(int kind, int role, int K, int N, int M, int v[4])
     return true;
 }
 
-// the start-up tuner's candidate row tile of the grouped expert GEMMs: an override of THIS thread only (ADVICE r04: a transient entry
+// the start-up tuner's candidate row tile of the grouped expert GEMMs: an override of THIS thread only (a transient entry
 // in the process-wide table was picked up by other engines / rank threads launching MoE forwards during the timing window)
 static thread_local int tl_grouped_rows = 0;
 void gen_grouped_rows_override(int rows)
@@ -887,8 +887,8 @@ bool gen_table_import_line(const char* line)
 
 // every tiling of gemm_kernel worth timing for a dense linear that the P32 kernels do not serve.  fp16 (lm_head): 64- or
 // 128-column workgroups; e4m3 weight-only: one or two tiles per wave; both with the split-K counts that keep >= 8 k-blocks per
-// slice and whose slabs fit the workspace.  (u4 linears of this kernel -- N % 32 != 0 -- keep the heuristic: no model of
-// BASELINE.json has one.)
+// slice and whose slabs fit the workspace.  (u4 linears of this kernel -- N % 32 != 0 -- keep the heuristic: no benchmarked
+// model has one.)
 int gen_dense_candidates(const LinearWeight& w, int M, size_t workspace_bytes, GemmConfig* out, int cap)
 {
     if ((w.type != 1 && w.type != 2) || M > 256) {
@@ -956,7 +956,7 @@ GemmConfig gemm_pick_config(const LinearWeight& w, int M)
 
 GemmConfig gemm_pick_config_general(const LinearWeight& w, int M)
 {
-    // Heuristic (measured on MI355X with tools/tune_gemm.py, see DESIGN.md): the decode GEMMs are latency /
+    // Heuristic (measured on MI355X with tools/tune_gemm.py): the decode GEMMs are latency /
     // issue bound, so aim at ~256 workgroups of 8 waves.  TM_GEMM_NT / _SPLITS / _WAVES / _KPHASES override.
     GemmConfig cfg{};
     const int  ntiles = w.N / 16;
@@ -968,7 +968,7 @@ GemmConfig gemm_pick_config_general(const LinearWeight& w, int M)
         cfg.splits  = tv[1];
         cfg.waves   = tv[2];
         cfg.kphases = tv[3];
-        // the documented TM_GEMM_* overrides apply to measured entries as well (ADVICE r04: they silently stopped working once a
+        // the documented TM_GEMM_* overrides apply to measured entries as well (they silently stopped working once a
         // `G` line existed)
         cfg.nt      = env_int("TM_GEMM_NT", cfg.nt);
         cfg.splits  = env_int("TM_GEMM_SPLITS", cfg.splits);
@@ -1080,7 +1080,7 @@ static int launch_u4_nt1(const GemmParams& p, dim3 grid, int ks, hipStream_t st)
       if (ks == 4) {
 #ifdef TM_EXPERIMENTS  // timing-ablation instantiations (results are garbage by design): not in the shipped library
         if constexpr (MT == 4) {
-            switch (env_int("TM_GEMM_ABL", 0)) {  // ablation timing experiments (round 1)
+            switch (env_int("TM_GEMM_ABL", 0)) {  // ablation timing experiments
                 case 1: return launch_one<0, MT, 1, WN, WK, 4, 2, 1>(p, grid, st);
                 case 2: return launch_one<0, MT, 1, WN, WK, 4, 2, 2>(p, grid, st);
                 case 4: return launch_one<0, MT, 1, WN, WK, 4, 2, 4>(p, grid, st);
@@ -1267,7 +1267,7 @@ int launch_linear(const LinearWeight& w,
     p.dbg      = nullptr;  // set below, once the grid is known
     // k-blocks per grid.y slice: whole iterations of ks*wk k-blocks, for every slice including the last one.
     // ks (k-blocks per barrier) = the largest of {4, 2, 1} (capped by cfg.kstage) that divides the slice.
-    // measured (round 1 ablations): more k-blocks per barrier does NOT pay (the loop is issue-bound, not
+    // measured: more k-blocks per barrier does NOT pay (the loop is issue-bound, not
     // barrier-bound), so the default is 1; TM_GEMM_KSTAGE=2|4 keeps the experiment reachable.
     int ks_cap = cfg.kstage > 0 ? cfg.kstage : 1;
     if (w.type != 0 || (waves == 4 && nt == 4) || waves == 16) {

@@ -4,8 +4,8 @@
 // (src/turbomind/engine/engine.cc:434-470,770-870) and Scheduler::Schedule (engine/scheduler.cc:1018-1078):
 //   * requests are admitted in arrival order (the reference sorts by unique_id, scheduler.cc:1076-1078);
 //   * a request is admitted when a batch slot is free and the block pool can hold prompt + max_new_tokens
-//     (blocks of 64 tokens, all reserved at admission: no preemption / eviction, no prefix cache -- SURVEY 8f-1
-//     names the prefix-free variant);
+//     (blocks of 64 tokens, all reserved at admission: no preemption / eviction, no prefix
+//     cache);
 //   * the prefill token budget of one scheduler step is max_prefill_token_num (ForwardTokenResource,
 //     engine.cc:462-464); at least one waiting request is admitted per step if it fits at all;
 //   * a sequence finishes on EOS (unless ignore_eos), at max_new_tokens, or when cancelled; its slot and blocks are

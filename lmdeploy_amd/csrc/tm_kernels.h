@@ -142,16 +142,16 @@ struct GemmConfig {
     int       ticket_count = 0;   // (f16_stream: how many there are)
     bool      f16_stream = false; // the kernels of gemm_f16.hip
 };
-// (shape 10 was "dequantise + the vendor library's fp16 GEMM" in round 3: removed -- no vendor GEMM on any path of this library)
+// (shape 10, once "dequantise + the vendor library's fp16 GEMM", does not exist -- no vendor GEMM on any path of this library)
 constexpr int kShapePre256     = 12;   // gemm_prefill.hip: 256 x 256 tiles, weights dequantised once per workgroup tile through LDS (M > 64)
 constexpr int kShapeF16        = 13;   // gemm_prefill_f16.hip: 256 x 256 tiles over the resident fp16 image, both operands by LDS-DMA (M > 64; LinearWeight::image16)
 constexpr int kShapeLC         = 11;   // gemm_decode_lc.hip: 8 consumer + 4 loader waves, 128 columns x M <= 64 rows per workgroup
-// kShapeMerge + s (s = 0..3, 6..9; round 6): the decode tile s whose split-K slices are merged INSIDE the launch by the last-arriving
+// kShapeMerge + s (s = 0..3, 6..9): the decode tile s whose split-K slices are merged INSIDE the launch by the last-arriving
 // slice of each column tile, for the fp16 / gated-SiLU epilogues (the folded-norm producers, epilogue 3, always merge that way): a
 // gated w1w3 can then split K across CUs (256-column tiles, half the activation bytes per CU) without slabs leaving the launch.
 // Needs arrival counters: NormFold::tickets (engine) / the tail of the workspace (tm_linear_forward).
 constexpr int kShapeMerge      = 16;
-// 256 columns x 2 k-phases x 16 waves on 2-k-block stages (gemm_dec32_kernel<MH, 8, 2, 2, 2>; round 6): the 256-column decode tile that does not
+// 256 columns x 2 k-phases x 16 waves on 2-k-block stages (gemm_dec32_kernel<MH, 8, 2, 2, 2>): the 256-column decode tile that does not
 // spill (shape 1 = the same wave layout on 4-k-block stages with a 4-deep ring: 60 B / lane of scratch at the 128-register cap)
 constexpr int kShapeWide2      = 10;
 inline bool dec32_is_merge_shape(int shape)
@@ -201,7 +201,7 @@ int    dec32_table_export(const char* path);
 int    dec32_table_import(const char* path);
 int    dec32_candidates(const LinearWeight& w, int M, int (*out)[2], int cap);
 int    dec32_m_bucket(int M);  // table key of a forward with M rows: M itself up to 256, then 512, 1024, ... 8192
-// Measured dispatch of everything that is NOT a P32 kernel (VERDICT r03 item 7; reference: gemm.cu:92-224 caches every problem the
+// Measured dispatch of everything that is NOT a P32 kernel (reference: gemm.cu:92-224 caches every problem the
 // warm-up of turbomind.cc:363-487 meets, not only the dense u4 ones).  One table, key (kind, role, K, N, M bucket):
 //   kind kGenDense + type   : gemm_kernel of a dense linear (fp16 lm_head, e4m3 weight-only, u4 with N % 32 != 0) -> {nt, splits, waves, kphases}
 //   kind kGenGrouped + type : row-tile height of the grouped expert GEMMs (u4: 16 / 32 / 64 rows, fp8 MFMA: 32 / 64 / 128) -> {rows, 0, 0, 0}
@@ -217,7 +217,7 @@ int    gen_table_export_lines(FILE* f);      // appends the G lines; returns the
 bool   gen_table_import_line(const char* line);  // a `G ...` line; false = not valid (ignored)
 int    gen_dense_candidates(const LinearWeight& w, int M, size_t workspace_bytes, GemmConfig* out, int cap);
 int    gen_grouped_candidates(const LinearWeight& proto, int m_cap, int* rows_out, int cap);
-// RMSNorm folded into the neighbouring decode GEMMs (round 5; gemm_decode_common.h has the arithmetic).  One struct, two roles:
+// RMSNorm folded into the neighbouring decode GEMMs (gemm_decode_common.h has the arithmetic).  One struct, two roles:
 //   producer (resid != nullptr): the row-parallel GEMM (wo / w2) adds its fp16 output to the residual stream in its own epilogue
 //     (split-K: the last-arriving slice of a column tile sums the slices' slabs in slice order), writes y = h(f32(r) * f32(g)) and
 //     ss_out[tile][m] = partial sum of f32(r)^2 over the tile's columns; tiles_out = column tiles written (set by the launcher)
@@ -234,7 +234,7 @@ struct NormFold {
     unsigned*     tickets = nullptr;
     int           tiles_out = 0;
 };
-constexpr int kFoldMaxRows = 128;  // rows of a forward whose RMSNorms fold into the decode GEMMs (round 6: BASELINE config 3 runs batch 128)
+constexpr int kFoldMaxRows = 128;  // rows of a forward whose RMSNorms fold into the decode GEMMs (for batch 128)
 bool   dec32_fold_shape_m(int shape, int M, bool producer);  // can (shape, M) run as a folded producer / consumer?
 bool   dec32_fold_shape(int shape);  // shapes whose kernel carries the folded-norm epilogue / prologue (0..3, 6..9)
 int    launch_linear_dec32(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated_silu, int shape,
@@ -328,9 +328,9 @@ int launch_moe_combine(half_t* out, int ldo, const half_t* y, int ldy, const flo
 extern uint64_t* g_gemm_dbg;  // gemm_w4a16.hip: optional per-workgroup timing stamps (tm_debug_set_gemm_trace)
 // The trace buffer holds kTraceMaxWorkgroups x 8 stamps; a launch with more workgroups is not traced.  (The only unbounded
 // device write the library had: a trace buffer sized for one kernel left set while a larger grid ran -- the probable origin of
-// the one-off "memory access fault" of a round-2 diagnostic script; tests/test_gpu_fullsize.py::..._with_canaries is clean.)
+// the one-off "memory access fault" of a diagnostic script; tests/test_gpu_fullsize.py::..._with_canaries is clean.)
 constexpr size_t kTraceMaxWorkgroups = 8192;
-// Arena mode (tm_debug_trace_arena, round 5): every traced launch gets ITS OWN region of a caller-sized buffer, handed out in
+// Arena mode (tm_debug_trace_arena): every traced launch gets ITS OWN region of a caller-sized buffer, handed out in
 // launch order, and a host-side record (tag, grid, offset) -- so that the launches of a captured hipGraph keep distinct regions
 // and one replay leaves the stamps of every kernel of the step (tools/fixed_cost_table.py).  Allocation happens on the host at
 // launch / capture time; launches that no longer fit are not traced.

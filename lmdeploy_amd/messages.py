@@ -2,7 +2,7 @@
 
 Reference: QuantPolicy (lmdeploy/messages.py:20-27), GenerationConfig (:35-205), TurbomindEngineConfig (:208-367),
 ResponseType / Response (:553-602).  Fields that the MI355X engine does not implement raise NotImplementedError when
-set to a non-default value -- loudly, instead of being silently ignored (SURVEY 8b).
+set to a non-default value -- loudly, instead of being silently ignored.
 """
 from __future__ import annotations
 

@@ -2,7 +2,7 @@
 
 Reference: lmdeploy/api.py:15-82 (pipeline), lmdeploy/pipeline.py:33-183,317-327 (Pipeline.infer / __call__ /
 stream_infer / close).  The reference routes through AsyncEngine + its continuous-batching scheduler; here up to
-`max_batch_size` prompts run as one static batch (chunked prefill + decode, the configuration BASELINE.json's metric is
+`max_batch_size` prompts run as one static batch (chunked prefill + decode, the configuration the headline metric is
 quoted on), more prompts -- and every stream_infer call -- go through the engine's scheduler (tm_engine_submit / step /
 poll: requests leave the batch when they stop, waiting ones take their slots).
 """
@@ -107,7 +107,7 @@ class Pipeline:
         self._group = None
         if cfg.tp > 1:
             rows = cfg.max_batch_size or 64
-            # ranks that share a device (a 1-GPU box driving tp = 2 for bring-up): RCCL refuses duplicate devices -> native P2P communicator
+            # ranks that share a device (one GPU driving tp = 2 for bring-up): RCCL refuses duplicate devices -> native P2P communicator
             want_rccl = len(set(devices[r % len(devices)] for r in range(cfg.tp))) == cfg.tp
             want_native = cfg.communicator in ('native', 'cuda-ipc')    # the reference's names for its in-house communicator
             if comm_unique_id is not None:              # expert path: the caller launched one process per GPU and broadcast the id
@@ -144,7 +144,7 @@ class Pipeline:
                 self._group.wait_ready()
                 self.engine = tp_group.TpEngine(self.engine, self._group, self._comm_backend)
         except BaseException:      # weights / tokenizer / start / a worker that failed to come up: the workers (and their GPU memory) must not
-            if self._group is not None:     # outlive the failed constructor (ADVICE r05)
+            if self._group is not None:     # outlive the failed constructor
                 self._group.close()
             raise
 

@@ -205,7 +205,7 @@ class Engine:
         _ffi.check(self._lib.tm_engine_sync(self._h))
 
     def fetch(self) -> np.ndarray:
-        """tokens generated so far, [batch, steps].  After a communicator give-up (terminal) the native call hands over
+        """tokens generated so far, [batch, steps].  After a communicator give-up (terminal: the group has to be rebuilt) the native call hands over
         the columns known to be valid together with its error status: they travel on the raised TmError as `.partial_tokens`."""
         out = np.zeros((self.batch, self.max_new), np.int32)
         n = C.c_int(0)

@@ -37,7 +37,7 @@ RANK0_READS = ('poll', 'poll_logprobs', 'fetch', 'fetch_logprobs', 'fetch_logits
                'overlapped_steps', 'pick_tiling', 'pick_general', 'export_gemm_table', 'stream', 'cfg', 'batch', 'max_new', 'PROF_CATEGORIES')
 # everything else of Engine either runs a forward or changes engine state on ONE rank (serve_start / serve_stop / wait: the engine thread;
 # profile_decode; init_synthetic / load_weights / start / comm_*: construction): rank 0 alone would enter collectives the workers never
-# join (RCCL: hangs without bound; native communicator: its 30 s give-up, terminal) -- refused loudly (ADVICE r05)
+# join (RCCL: hangs without bound; native communicator: its 30 s give-up, terminal) -- refused loudly
 _TIMEOUT_S = float(os.environ.get('TM_TP_GROUP_TIMEOUT_S', '600'))
 
 
@@ -47,10 +47,10 @@ def _setup_comm(eng: Engine, want_rccl: bool, uid: bytes, all_gather, rows: int,
     want_native (`TurbomindEngineConfig.communicator` = 'native' / 'cuda-ipc', the reference's names for its own in-house communicator,
     src/turbomind/comm/device_comm.cc:14-30): the native communicator serves the decode-sized forwards -- one fused launch per
     exchange, as the reference's AllreduceResidualBiasRMSnorm -- and RCCL, where it came up on every rank, keeps the prefill-sized
-    ones (side-stream overlap, DESIGN 6)."""
+    ones (side-stream overlap)."""
     # the switches that decide HOW MANY collectives a forward issues are read by every rank from its own environment (engine_comm.hip:
     # TM_COMM_STREAM / TM_PIPE_MIN_ROWS / TM_PIPE_MICROBATCH select the two-micro-batch prefill schedule): a mismatch would change the
-    # collective sequence on one rank only and deadlock the group -- compare them before any communicator exists (ADVICE r05)
+    # collective sequence on one rank only and deadlock the group -- compare them before any communicator exists
     knobs = tuple(os.environ.get(k, '') for k in ('TM_COMM_STREAM', 'TM_PIPE_MIN_ROWS', 'TM_PIPE_MICROBATCH', 'TM_COMM', 'TM_GRAPH_COMM',
                                                   'TM_FOLD_NORM', 'TM_P2P_DECODE_ROWS'))
     seen = all_gather(knobs)
@@ -66,7 +66,7 @@ def _setup_comm(eng: Engine, want_rccl: bool, uid: bytes, all_gather, rows: int,
             ok = False
     oks = all_gather(ok)
     if want_rccl and all(oks):
-        # The DEFAULT arrangement (round 6): RCCL serves the prefill-sized forwards (side-stream overlap), the native
+        # The DEFAULT arrangement: RCCL serves the prefill-sized forwards (side-stream overlap), the native
         # communicator the decode-sized ones -- wo / w2 -> ONE fused all-reduce + residual + RMSNorm launch per exchange, as the
         # reference's AllreduceResidualBiasRMSnorm (fused_allreduce.cu:406-500, unified_decoder.cc:278-285,328-335) -- provided its bring-up
         # self-test passes on EVERY rank (the hop between devices is what no single-GPU test covers); else RCCL + the norm launch.
@@ -260,7 +260,7 @@ class TpEngine:
                 out = attr(*args, **kwargs)
             except BaseException as e:      # noqa: BLE001 -- ANY failure of rank 0's own call (a ValueError from argument conversion as well as
                 err, out = e, None          # a TmError): the workers ran the call and queued a reply each -- drain them, or every later call
-            try:                            # reads the previous call's replies and the ranks drift apart (ADVICE r05)
+            try:                            # reads the previous call's replies and the ranks drift apart
                 replies = self._link.collect()
             except BaseException:           # noqa: BLE001 -- a worker died / timed out: rank 0's own error is the more useful one
                 if err is not None:
