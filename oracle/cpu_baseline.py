@@ -1,7 +1,7 @@
 """CPU baseline for bench.py's `cpu_baseline` leg (TEST / MEASUREMENT INFRASTRUCTURE, never the product path).
 
 kind = "port": the reference has no CPU backend (`PytorchEngineConfig.device_type` in {cuda, ascend, maca, camb},
-lmdeploy/messages.py:531) and `/root/reference` does not exist on the GPU box, so this is a torch-CPU port of the
+lmdeploy/messages.py:531), so this is a torch-CPU port of the
 reference PyTorchEngine's pure-torch "default" op backend, restated from:
   * W4A16:   lmdeploy/pytorch/backends/default/awq_modules.py:37-46,58-81  ((q - z) * s in fp16, then matmul)
   * RMSNorm: lmdeploy/pytorch/backends/default/norm.py:14-28
@@ -64,8 +64,8 @@ def physical_cores() -> int:
 
 def run(model: dict, batch: int, ctx: int, sample_layers: int = 2, seed: int = 0, threads: int | None = None,
         passes: int = 3, budget_s: float = 25.0) -> dict:
-    # one thread per PHYSICAL core: the contraction is fp32 FMA-bound, SMT siblings only add contention (round 2 ran
-    # os.cpu_count() = 256 logical CPUs of a 128-core host and measured the oversubscribed rate)
+    # one thread per PHYSICAL core: the contraction is fp32 FMA-bound, SMT siblings only add contention (os.cpu_count() =
+    # 256 logical CPUs of a 128-core host give an oversubscribed rate)
     threads = threads or physical_cores()
     torch.set_num_threads(threads)
     g = torch.Generator().manual_seed(seed)
@@ -135,8 +135,8 @@ def run(model: dict, batch: int, ctx: int, sample_layers: int = 2, seed: int = 0
     step_s = t_layer * model['layers'] + t_head
     return dict(value=batch / step_s, unit='tokens/s', cores=threads, logical_cpus=os.cpu_count(), kind='port',
                 pinned_by='tests/test_oracle.py::test_cpu_baseline_port_matches_reference_golden_vectors (golden vectors generated by '
-                          'importing the reference\'s pytorch/backends/default functions; /root/reference does not exist on the GPU box, '
-                          'so the reference functions themselves cannot be the timed baseline)',
+                          'importing the reference\'s pytorch/backends/default functions, which are not '
+                          'there when this is timed)',
                 sample=(f'{sample_layers} of {model["layers"]} decoder layers + lm_head, one decode step, batch {batch}, '
                         f'ctx {ctx}, int8 KV; 1 warm-up + {len(per_layer)} timed passes (median {t_layer:.2f} s / layer, '
                         f'{t_head:.2f} s head); fp32 contraction on CPU; extrapolated to {model["layers"]} layers'))
@@ -144,7 +144,7 @@ def run(model: dict, batch: int, ctx: int, sample_layers: int = 2, seed: int = 0
 
 def run_config0(model: dict, batch: int = 1, ctx: int = 1024, steps: int = 4, seed: int = 0, threads: int | None = None,
                 budget_s: float = 25.0) -> dict:
-    """BASELINE.json configs[0]: InternLM2-1.8B, fp16 weights, fp16 KV, greedy decode on the host cores (the reference's own
+    """InternLM2-1.8B, fp16 weights, fp16 KV, greedy decode on the host cores (the reference's own
     CPU-runnable case is its PyTorch engine's default op backend: pytorch/backends/default/{norm,activation,apply_rotary_emb}.py --
     plain torch ops; there is no quantised linear and no KV quantisation in it).  The WHOLE model runs (24 layers: no
     extrapolation): one untimed warm-up step, then up to `steps` timed decode steps of `batch` sequences at context `ctx` within

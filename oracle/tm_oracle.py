@@ -11,7 +11,7 @@ even to fp16".  fp16 add/sub/mul are evaluated in float32 and rounded once
 (innocuous double rounding: 24 >= 2*11+2); fp16 fma is evaluated exactly in
 float64 and rounded once.
 
-Pinning status (see DESIGN.md "Oracle"):
+Pinning status:
   * AWQ unpack / dequant formula ......... pinned against the reference's own
     Python (`lmdeploy/pytorch/backends/default/awq_modules.py:12-46`,
     `lmdeploy/turbomind/weight_format.py:47-74,236-247`) via tests/golden.
@@ -681,7 +681,7 @@ class ModelConfig:
     group: int = 128
     kv_bits: int = 8
     block_len: int = 64
-    # BASELINE config 5: fp8 block-scaled weights, mixture-of-experts FFN (0 experts = dense)
+    # fp8 block-scaled weights, mixture-of-experts FFN (0 experts = dense)
     weight_format: str = 'u4'          # 'u4' (AWQ g128) | 'fp8' (e4m3, 128x128 block scales)
     moe_experts: int = 0
     moe_top_k: int = 0
@@ -703,7 +703,7 @@ LLAMA3_70B = dict(hidden=8192, layers=80, q_heads=64, kv_heads=8, head_dim=128, 
 
 
 def make_synthetic_weights(cfg: ModelConfig, seed: int = 0, quantized: bool = True):
-    """Random weights with real shapes (SURVEY 8d): fp16 master N(0,1)*0.1/sqrt(K), group-128
+    """Random weights with real shapes: fp16 master N(0,1)*0.1/sqrt(K), group-128
     asymmetric u4 quantisation; norms 1+0.02 N; embeddings N(0,0.02).
     Layout = the boundary ("TM") layout: q [K,N] u4 as uint8, scales/zeros fp16 [K/g,N];
     w_qkv = [Q|K|V] fused along N (Q/K columns already in interleaved-RoPE order);
