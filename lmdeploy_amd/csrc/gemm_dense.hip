@@ -447,7 +447,7 @@ static int launch_dense_tile(const StreamArgs& a, const DenseCall& call, int vec
 template<class T, int EPI>
 static int launch_dense_tile256(const StreamArgs& a, const DenseCall& call, int vec, hipStream_t st)
 {
-    constexpr int lds = 3 * 512 * 64;
+    constexpr int lds = stream_tile_bufs(256, 256) * 512 * 64;
     const auto    k   = stream_tile256_kernel<T, DenseEpi<T, EPI>>;
     if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {
         return rc;

@@ -15,7 +15,6 @@
 namespace tmk {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float  floatx16 __attribute__((ext_vector_type(16)));
 
 template<class T>
 struct StreamOp;
@@ -461,7 +460,7 @@ __device__ __forceinline__ StreamTile stream_tile_of(const StreamArgs& a, const 
 // some CUs: 41, 37, 37, 38); 400 rows of (5120, 5120) in 128 x 128 tiles: three 57, four 44
 constexpr int stream_tile_bufs(int bm, int bn)
 {
-    return bm == 64 && bn == 64 ? 6 : bm == 128 && bn == 128 ? 4 : 3;
+    return bm == 64 && bn == 64 ? 6 : bm == 128 && bn == 128 || bm == 256 && bn == 256 ? 4 : 3;
 }
 
 template<class T, class Epi, int BM, int BN, int WM, int WN>
@@ -587,27 +586,28 @@ __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_k
 }
 
 // ---- many rows of a 16-bit format: 256 x 256 tiles -----------------------------------------------------------------------------------
-// 4 waves of 128 x 128 outputs (v_mfma_f32_32x32x16, 256 accumulator registers, one wave per SIMD): a step moves 32 KB into a CU and 64 KB out of its LDS per
-// 1024 cycles of matrix work, where the 256 x 128 tiles above move 48 and 96.  bf16, 8192 rows, MI355X: (K, N) = (4096, 21504) 1155 us = 1.25 PFLOP/s, (25600, 4096) 1370 us =
-// 1.25 PFLOP/s (the library's best on a square of 8192: 1.38; power holds the clock); 256 x 128 tiles 1281 and 1670 us, the 128 x 128 x 32 tiles through
-// registers that stood here before 1827 and 2447.
+// 4 waves of 128 x 128 outputs (v_mfma_f32_16x16x32, 256 accumulator registers, one wave per SIMD): a step moves 32 KB into a CU and 64 KB out of its LDS per
+// 1024 cycles of matrix work, where the 256 x 128 tiles above move 48 and 96.  Power holds the clock, and what a multiply-add costs depends on the
+// instruction: from registers alone, on normal operands, 16x16x32 reaches 1.98 PFLOP/s on this card and 32x32x16 1.72 (2.40 and 2.43 on zeros); neighbours in
+// the order of issue share an operand, which is another 1 %.  bf16, 8192 rows, MI355X: (K, N) = (4096, 21504) 1162 us, (25600, 4096) 1280 us =
+// 1.34 PFLOP/s, (8448, 2048) 212; with 32x32x16 1225, 1374 and 230, 256 x 128 tiles 1281 and 1670 (first two).
 // The MFMAs are asm so that the accumulators are accumulation registers and nothing else (left to the register allocator, it spills fragments); they
 // and the fragment reads stay in the order written.
 template<class T>
-__device__ __forceinline__ void stream_mma32(floatx16& c, const u32x4& a, const u32x4& b)
+__device__ __forceinline__ void stream_mma_acc(floatx4& c, const u32x4& a, const u32x4& b)
 {
     if constexpr (std::is_same<T, __bf16>::value) {
-        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     }
     else {
-        asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
     }
 }
 
 template<class T, class Epi>
 __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Epi epi)
 {
-    constexpr int BM = 256, BN = 256, kXB = BM * 64, kStage = kXB + BN * 64;
+    constexpr int BM = 256, BN = 256, kXB = BM * 64, kStage = kXB + BN * 64, kBufs = stream_tile_bufs(BM, BN);
     constexpr int kXP = 4, kWP = 4, kPieces = 8;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -641,96 +641,96 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
             stream_dma16(rs_w, woff[n - 4], (int)((s >> 2) * a.w_quad) + (s & 3) * 1024, dst + kXB);
         }
     };
-    auto dma = [&](int s, int buf) {
+    floatx4 acc[8][8];
 #pragma unroll
-        for (int n = 0; n < kPieces; ++n) {
-            dma_piece(s, buf, n);
-        }
-    };
-    floatx16 acc[4][4];
+    for (int i = 0; i < 8; ++i) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                acc[i][j][r] = 0.f;
-            }
+        for (int j = 0; j < 8; ++j) {
+            acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
     }
     const int wm = wave >> 1, wn = wave & 1;
-    const int l31 = lane & 31, half = lane >> 5;
-    // x: row r at r * 64, piece (2 j + half) ^ ((r >> 1) & 3); j = 1 flips bit 1 of the piece
-    const int xf = (wm * 128 + l31) * 64 + ((half ^ ((l31 >> 1) & 3)) << 4);
-    const int wf = kXB + (wn * 8 + (l31 >> 4)) * 1024 + (half * 16 + (l31 & 15)) * 16;
-    // 16 k are a half step; the fragments of the next half step are read under the MFMAs of this one.  The barrier sits in the middle of a step: the
-    // second half's fragments are in registers there, so the step's own stage is free for the DMA of stage s + 3
-    u32x4     fx[2][4], fw[2][4];
+    const int fr = lane & 15, fc = lane >> 4;
+    // x: row r at r * 64, piece c at c ^ ((r >> 1) & 3)
+    const int xf = (wm * 128 + fr) * 64 + ((fc ^ ((fr >> 1) & 3)) << 4);
+    const int wf = kXB + wn * 8192 + lane * 16;
+    // The fragments of step s + 1 are read under the MFMAs of step s, so the step's own stage is free behind its barrier: the DMA of stage s + kBufs goes there
+    u32x4     fx[2][8], fw[2][8];
     const int steps = a.steps;
-    auto      read  = [&](int j, const char* st, int n) {
-        if (n < 4) {
-            fw[j][n] = *(const u32x4*)(st + wf + n * 2048 + j * 512);
+    auto      read  = [&](auto Q, const char* st, int n) {
+        constexpr int q = decltype(Q)::value;
+        if (n < 8) {
+            fw[q][n] = *(const u32x4*)(st + wf + n * 1024);
         }
         else {
-            fx[j][n - 4] = *(const u32x4*)(st + (xf ^ (j * 32)) + (n - 4) * 2048);
+            fx[q][n - 8] = *(const u32x4*)(st + xf + (n - 8) * 1024);
         }
     };
-    dma(0, 0);
-    dma(min(1, steps - 1), 1);
-    dma(min(2, steps - 1), 2);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kPieces) : "memory");
+#pragma unroll
+    for (int b = 0; b < kBufs; ++b) {
+#pragma unroll
+        for (int n = 0; n < kPieces; ++n) {
+            dma_piece(min(b, steps - 1), b, n);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kBufs - 1) * kPieces) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int n = 0; n < 8; ++n) {
-        read(0, smem, n);
+    for (int n = 0; n < 16; ++n) {
+        read(std::integral_constant<int, 0>{}, smem, n);
     }
-    int buf = 0;
-    for (int s = 0; s < steps; ++s) {
-        const int   nxt = buf == 2 ? 0 : buf + 1;
-        const char* st  = smem + buf * kStage;
-#pragma unroll
-        for (int n = 0; n < 16; ++n) {
-            if (n % 2 == 0) {
-                read(1, st, n >> 1);
-            }
-            stream_mma32<T>(acc[n >> 2][n & 3], fw[0][n & 3], fx[0][n >> 2]);
-        }
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kPieces) : "memory");
+    int  buf  = 0;  // stage of step s
+    auto step = [&](auto Q, int s) {
+        constexpr int q   = decltype(Q)::value;
+        const int     nxt = buf == kBufs - 1 ? 0 : buf + 1;
+        // this wave's fragments of step s are in registers and its pieces of stage s + 1 have landed; then everybody's
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kBufs - 2) * kPieces) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        st = smem + nxt * kStage;
+        const char* st = smem + nxt * kStage;
+        const int   sd = min(s + kBufs, steps - 1);
 #pragma unroll
-        for (int n = 0; n < 16; ++n) {
-            if (n % 2 == 0) {
-                read(0, st, n >> 1);
+        for (int n = 0; n < 64; ++n) {
+            if (n % 3 == 0 && n < 48) {
+                read(std::integral_constant<int, q ^ 1>{}, st, n / 3);
             }
-            else {
-                dma_piece(min(s + 3, steps - 1), buf, n >> 1);
+            if (n % 8 == 4) {
+                dma_piece(sd, buf, n >> 3);
             }
-            stream_mma32<T>(acc[n >> 2][n & 3], fw[1][n & 3], fx[1][n >> 2]);
+            const int i = n >> 3, j = i & 1 ? 7 - (n & 7) : n & 7;
+            stream_mma_acc<T>(acc[i][j], fw[q][j], fx[q][i]);
         }
         buf = nxt;
+    };
+    int s = 0;
+    for (; s + 1 < steps; s += 2) {
+        step(std::integral_constant<int, 0>{}, s);
+        step(std::integral_constant<int, 1>{}, s + 1);
+    }
+    if (s < steps) {
+        step(std::integral_constant<int, 0>{}, s);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the DMA writes this workgroup's LDS)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {  // (the last results are sixteen passes behind their issue)
+    for (int i = 0; i < 8; ++i) {  // (the last results are passes behind their issue)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (int c = 0; c < 8; ++c) {
             asm volatile("s_nop 7" : "+a"(acc[i][c]));
         }
     }
-    // A lane's results are four columns each of 32 rows apart; through the wave's own 16 KB of LDS they leave as whole runs of a row (512 bytes of fp32): 32
+    // A lane's results are four columns each of 16 rows apart; through the wave's own 16 KB of LDS they leave as whole runs of a row (512 bytes of fp32): 32
     // rows at a time, piece p (four columns) of row r at p ^ r
     __builtin_amdgcn_s_barrier();  // every wave is through with the stages
     asm volatile("" ::: "memory");
     floatx4* const sw = (floatx4*)(smem + wave * 16384);
+    const int      l31 = lane & 31, half = lane >> 5;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int n = 0; n < 16; ++n) {  // columns 32 c + 8 g + 4 half + 0 .. 3
-            const int c = n >> 2, g = n & 3;
-            sw[l31 * 32 + ((8 * c + 2 * g + half) ^ l31)] = floatx4{acc[i][c][4 * g], acc[i][c][4 * g + 1], acc[i][c][4 * g + 2], acc[i][c][4 * g + 3]};
+        for (int n = 0; n < 16; ++n) {  // row 16 (n / 8) + fr, columns 16 (n % 8) + 4 fc + 0 .. 3
+            const int r = (n >> 3) * 16 + fr;
+            sw[r * 32 + ((4 * (n & 7) + fc) ^ r)] = acc[2 * i + (n >> 3)][n & 7];
         }
         __builtin_amdgcn_wave_barrier();
         const int mb = m0 + wm * 128 + i * 32, nb = n0 + wn * 128;
