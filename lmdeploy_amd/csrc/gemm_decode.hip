@@ -1205,7 +1205,7 @@ static int launch_dec32_shape(const Dec32Params& p, dim3 grid, int shape, hipStr
     if constexpr (MH == 4) {
         // row blocks of 128 rows x 256 columns, 8 waves of 32 columns over the whole k slice (M > 64): every dequantised
         // weight fragment feeds 4 MFMAs, every x fragment read from LDS feeds 32 columns
-        if (shape == 5) {  // 128 x 512 tile, two weight fragments per x-fragment read (gemm_pre64_kernel)
+        if (shape == 5) {  // largest prefill tile, where 128 x 512 is the cheaper one (launch_linear_dec32): two weight fragments per x-fragment read
 #ifdef TM_EXPERIMENTS
             if (abl == 2) return launch_pre64_one<2>(p, grid, st);  // timing: no MFMA
             if (abl == 8) return launch_pre64_one<8>(p, grid, st);  // timing: raw codes on the matrix pipe
@@ -1527,6 +1527,27 @@ int dec32_candidates(const LinearWeight& w, int M, int (*out)[2], int cap)
     return n;
 }
 
+// Prefill tiles: what a product costs in rounds of one 256 x 256 tile a CU.  A round that is not full costs 0.7 + 0.3 of its share: power, not the number of
+// busy CUs, bounds a full one.  Measured, us (128 x 256 / 128 x 512 / 256 x 256 tiles): full rounds (4096, 4096) 4096 rows 136 / 127 / 112, (14336, 4096) 4096
+// rows 427 / 403 / 365, (4096, 28672) 8192 rows 1902 / 1757 / 1630; partial ones (4096, 6144) 1280 rows 65 / 87 / 87, 2604 rows 131 / 124 / 188, 5300
+// rows 260 / 246 / 218; (4096, 28672) 640 rows 183 / 203 / 207, 768 rows 191 / 209 / 209, 1000 rows 254 / 232 / 222; (5120, 13824) 1972 rows 309 / 291 / 254;
+// (14336, 4096) 2048 rows 215 / 269 / 270, 2604 rows 356 / 318 / 293.  The lines taken, before (128 x 512 from 192 of its tiles on) and now: (4096, 28672) 640 rows 199 ->
+// 179, 1972 rows 444 -> 416, 8192 rows 1636 -> 1494, (4096, 6144) 1536 rows 109 -> 96, (14336, 4096) 2604 rows 341 -> 292, (5120, 13824) 1280 rows 247 -> 207
+static double tile_rounds(int tiles)
+{
+    const int rest = tiles % 256;
+    return tiles / 256 + (rest ? 0.7 + 0.3 * rest / 256 : 0.0);
+}
+static double prefill_cost_512(int ncg, int M)
+{
+    return 1.1 * tile_rounds((ncg + 15) / 16 * ((M + 127) / 128));
+}
+static double prefill_cost_256(int ncg, int M)
+{
+    const int blocks = (M + 255) / 256;  // (a last row block that is nearly empty costs the smaller tiles less: 257 rows 112 / 108 / 116)
+    return (10 * M < 7 * 256 * blocks ? 1.1 : 1.0) * tile_rounds((ncg + 7) / 8 * blocks);
+}
+
 // Tiling for the decode GEMM: `shape` (see launch_dec32_shape) and the split-K count.  One workgroup per CU (128 KB of
 // LDS): take the widest split that keeps <= 256 workgroups and >= one stage (4 k-blocks) per slice.
 void dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out)
@@ -1548,15 +1569,13 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
         shape = 0;
     }
     if (M > 64) {
-        // M <= 256 (batch-128 decode, small admissions): 256-column tiles keep more workgroups alive; beyond that the
-        // 512-column tile with two weight fragments per x-fragment read (TM_PRE64_MIN_M: first M that takes it)
+        // M <= 256 (batch-128 decode, small admissions): 256-column tiles of 128 rows keep more workgroups alive; beyond that the largest prefill tile
+        // (shape 5) where its rounds cost less (TM_PRE64_MIN_M: first M that may take it).  With fewer tiles than CUs the 128 x 256 tile takes at most 4
+        // slices of k (measured by the tuner at the Llama-3-8B shapes, us per layer incl. the consumer -- M = 512: w_qkv 49.3 -> 36.5, wo 44.9 -> 28.5,
+        // w2 74.2 -> 54.2; M = 1024: 66.8 -> 48.1, 61.4 -> 41.5, 105.5 -> 92.6)
         static const int pre64_from = env_int2("TM_PRE64_MIN_M", 257);
-        // The 128 x 512 tile only when it alone puts ~one workgroup on most CUs; otherwise the 128 x 256 tile with at most 4
-        // split-K slices (measured by the tuner at the Llama-3-8B shapes, us per layer incl. the consumer --
-        // M = 512: w_qkv 49.3 -> 36.5, wo 44.9 -> 28.5, w2 74.2 -> 54.2; M = 1024: 66.8 -> 48.1, 61.4 -> 41.5, 105.5 -> 92.6;
-        // M = 2048: wo 81.6 -> 61.2; from M = 4096 the wide tile wins everywhere: profiles/r03_gemm_tune_prefill_classes.txt)
-        const int wgs5 = (ncg + 15) / 16 * ((M + 127) / 128);
-        shape          = (M >= pre64_from && w.N >= 512 && wgs5 >= 192) ? 5 : 4;
+        const double     c4 = 0.59 * tile_rounds((ncg + 7) / 8 * ((M + 127) / 128));
+        shape               = (M >= pre64_from && w.N >= 512 && std::min(prefill_cost_512(ncg, M), prefill_cost_256(ncg, M)) < c4) ? 5 : 4;
     }
     // Narrow projections at a full decode batch (33 .. 64 rows, N <= 8192: w_qkv, wo, w2 of an 8B model): 64-column tiles
     // with as little split-K as still gives ~256 workgroups.  Split-K costs more at the kernel boundary than it buys inside
@@ -1708,6 +1727,9 @@ int launch_linear_dec32(const LinearWeight& w, const half_t* x, int ldx, half_t*
     TM_REQUIRE(w.packed32 != nullptr && w.N % 32 == 0, "decode GEMM: P32 layout missing");
     if (shape == kShapeF16 && (w.image16 == nullptr || M <= 64)) {
         shape = kShapePre256;  // a table entry for a linear without the fp16 image (operator-level handle, TM_PREFILL_F16_IMAGE=0): the fused 256 x 256 tile
+    }
+    if (shape == 5 && splits <= 1 && prefill_cost_256(w.N / 32, M) <= prefill_cost_512(w.N / 32, M)) {
+        shape = kShapePre256;
     }
     TM_REQUIRE(M >= 1 && shape >= 0 && (shape <= 9 || shape == kShapeWide2 || shape == kShapeLC || shape == kShapePre256 || shape == kShapeF16)
                    && (shape >= 6 || (M <= 64) == (shape < 4)) && (shape != kShapeLC || M <= 64) && (shape != kShapePre256 || M > 64)

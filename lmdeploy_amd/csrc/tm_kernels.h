@@ -143,7 +143,7 @@ struct GemmConfig {
     bool      f16_stream = false; // the kernels of gemm_f16.hip
 };
 // (shape 10, once "dequantise + the vendor library's fp16 GEMM", does not exist -- no vendor GEMM on any path of this library)
-constexpr int kShapePre256     = 12;   // gemm_prefill.hip: 256 x 256 tiles, weights dequantised once per workgroup tile through LDS (M > 64)
+constexpr int kShapePre256     = 12;   // gemm_prefill.hip: 256 x 256 tiles, each weight dequantised once per workgroup tile (M > 64)
 constexpr int kShapeF16        = 13;   // gemm_prefill_f16.hip: 256 x 256 tiles over the resident fp16 image, both operands by LDS-DMA (M > 64; LinearWeight::image16)
 constexpr int kShapeLC         = 11;   // gemm_decode_lc.hip: 8 consumer + 4 loader waves, 128 columns x M <= 64 rows per workgroup
 // kShapeMerge + s (s = 0..3, 6..9): the decode tile s whose split-K slices are merged INSIDE the launch by the last-arriving
