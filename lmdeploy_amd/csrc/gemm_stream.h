@@ -72,10 +72,12 @@ __device__ __forceinline__ int64_t stream_weight_bytes(const StreamArgs& a, int 
 // steps at a time), and few columns are spread over the CUs by cutting k instead of the column group: KP waves share a column
 // tile inside the workgroup and meet in LDS, grid z slices of k meet in the last workgroup of a column group to arrive, which adds the
 // slices in slice order (the sum never depends on the order of arrival; no workgroup waits for another).
-// Weights run one chunk of eight steps ahead of the MFMAs in a second register buffer; all loads of a stage are unconditional (clamped).
-// 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 43 us = 4.8 TB/s, (4096, 21504) 38 us = 4.6 TB/s (with every wave reading x for itself, no
-// slices: 76 and 50); four rows fp32, (8448, 2048): 18 us = 3.8 TB/s (64 x 64 tiles: 331).  The loop fetches without a branch: with one around the
-// loads the two above take 52 and 42.  Its last two stages stand behind it and fetch nothing beyond the slice: 8 rows bf16 of (8448, 2048) 15.1 -> 11.8.
+// Weights run one chunk of eight steps ahead of the MFMAs in a second register buffer; all loads of a stage are unconditional (clamped).  Loads return in
+// order, so a stage's x is asked for ahead of its weights: the wait for x then leaves the weights in flight (the other way round every stage drained the
+// queue: 8 rows fp16 of (2048, 16384) 14.6 us, now 11.9 = 5.6 TB/s; bf16 of (2048, 8448) 12.0, 9.9; 3 rows fp32 of (2048, 8448) 19.9, 16.5).
+// 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 38 us = 5.5 TB/s, (4096, 21504) 39 us = 4.5 TB/s (with every wave reading x for itself, no
+// slices: 76 and 50).  The loop fetches without a branch: with one around the
+// loads the two above took 52 and 42.  Its last two stages stand behind it and fetch nothing beyond the slice: 8 rows bf16 of (8448, 2048) then took 15.1 -> 11.8.
 template<class T, class Epi, int MT, int NT, int CW, int KP>
 __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a, Epi epi)
 {
@@ -175,26 +177,28 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
     };
     constexpr int kStride = KP * kChunk;
     const int     first   = ph * kChunk;  // of this k-phase in a stage
-    fetch(wa, s0 + first);
-    fetch_x(s0);
+    auto load = [&](u32x4(&buf)[kChunk][NT], int at) {
+        fetch_x(at);
+        asm volatile("" ::: "memory");
+        fetch(buf, at + first);
+        asm volatile("" ::: "memory");
+    };
+    load(wa, s0);
     stash_x(0);
     __syncthreads();
     int base = s0;
     for (; base + 2 * kStride < s1; base += 2 * kStride) {  // three stages lie ahead
-        fetch(wb, base + kStride + first);
-        fetch_x(base + kStride);
+        load(wb, base + kStride);
         compute(wa, 0, base + first);
         stash_x(1);  // its readers finished before the last barrier
         __syncthreads();
-        fetch(wa, base + 2 * kStride + first);
-        fetch_x(base + 2 * kStride);
+        load(wa, base + 2 * kStride);
         compute(wb, 1, base + kStride + first);
         stash_x(0);
         __syncthreads();
     }
     if (base + kStride < s1) {  // the last two stages, or the last: nothing is fetched that is not used
-        fetch(wb, base + kStride + first);
-        fetch_x(base + kStride);
+        load(wb, base + kStride);
         compute(wa, 0, base + first);
         stash_x(1);
         __syncthreads();
@@ -298,11 +302,11 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
 }
 
 // The same without slices across workgroups, for callers that bring no scratch and where slices cost more than they give (stream_plan): a workgroup owns NT
-// column tiles, its W waves take chunks of eight steps in turn, each reading its own rows of x, and meet in LDS in wave order.
+// column tiles, its W waves take chunks of steps in turn, each reading its own rows of x, and meet in LDS in wave order.
 template<class T, class Epi, int MT, int NT, int W>
 __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi epi)
 {
-    constexpr int kChunk = 8 / NT;
+    constexpr int kChunk = MT * NT > 1 ? 4 : 8;
     __shared__ __attribute__((aligned(16))) floatx4 red[W][MT * NT][64];
     const int  lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int  mb   = blockIdx.y % a.row_blocks * (MT * 16), tile0 = blockIdx.x * NT;
@@ -330,8 +334,19 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
             acc[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    u32x4 wa[kChunk][NT], wb[kChunk][NT];
-    auto  fetch = [&](u32x4(&buf)[kChunk][NT], int base) {
+    // x of a chunk leaves with its weights, ahead of them: loads return in order, and a load of x where it is used would wait for the next
+    // chunk's weights (fp16, 8 rows: (2048, 4096) 5.9 -> 5.4 us, (2048, 2048) 5.1 -> 4.8; fp32, 3 rows, (2048, 2048) 8.5 -> 8.0)
+    u32x4 wa[kChunk][NT], wb[kChunk][NT], xa[kChunk][MT], xb[kChunk][MT];
+    auto  fetch = [&](u32x4(&buf)[kChunk][NT], u32x4(&xbuf)[kChunk][MT], int base) {
+#pragma unroll
+        for (int kk = 0; kk < kChunk; ++kk) {
+            const int s = min(base + kk, a.steps - 1);
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                xbuf[kk][t] = *(const u32x4*)(xp[t] + (int64_t)s * 64);
+            }
+        }
+        asm volatile("" ::: "memory");
 #pragma unroll
         for (int kk = 0; kk < kChunk; ++kk) {
             const int s = min(base + kk, a.steps - 1);
@@ -340,17 +355,17 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
                 buf[kk][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + (s >> 2) * a.w_quad + (s & 3) * 1024));
             }
         }
+        asm volatile("" ::: "memory");
     };
-    auto compute = [&](const u32x4(&buf)[kChunk][NT], int base) {
+    auto compute = [&](const u32x4(&buf)[kChunk][NT], const u32x4(&xbuf)[kChunk][MT], int base) {
 #pragma unroll
         for (int kk = 0; kk < kChunk; ++kk) {
             if (base + kk < a.steps) {
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
-                    const u32x4 b = *(const u32x4*)(xp[t] + (int64_t)(base + kk) * 64);
 #pragma unroll
                     for (int j = 0; j < NT; ++j) {
-                        acc[t][j] = StreamOp<T>::mma(buf[kk][j], b, acc[t][j]);
+                        acc[t][j] = StreamOp<T>::mma(buf[kk][j], xbuf[kk][t], acc[t][j]);
                     }
                 }
             }
@@ -359,20 +374,20 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
     constexpr int kStride = W * kChunk;
     int           base    = wave * kChunk;
     if (base < a.steps) {
-        fetch(wa, base);
+        fetch(wa, xa, base);
         for (; base + 2 * kStride < a.steps; base += 2 * kStride) {
-            fetch(wb, base + kStride);
-            compute(wa, base);
-            fetch(wa, base + 2 * kStride);
-            compute(wb, base + kStride);
+            fetch(wb, xb, base + kStride);
+            compute(wa, xa, base);
+            fetch(wa, xa, base + 2 * kStride);
+            compute(wb, xb, base + kStride);
         }
         if (base + kStride < a.steps) {  // the last two chunks, or the last: nothing is fetched that is not used
-            fetch(wb, base + kStride);
-            compute(wa, base);
-            compute(wb, base + kStride);
+            fetch(wb, xb, base + kStride);
+            compute(wa, xa, base);
+            compute(wb, xb, base + kStride);
         }
         else {
-            compute(wa, base);
+            compute(wa, xa, base);
         }
     }
 #pragma unroll
