@@ -312,16 +312,30 @@ void dense_weight_free(DenseWeight& d)
 //   tile kernels: (tiles of the fullest CU) x (steps x time of a step with the CU full + prologue and results), at least one tile alone.  16-bit, 8192
 //     rows, (K, N) = (4096, 21504): 256 x 256 1155 us (1.25 PFLOP/s), 256 x 128 1281, 128 x 128 1520, 64 x 64 2714; (2048, 256) with 8000 rows: 46,
 //     33, 23, 20 us; (2048, 2048) with 2600 rows: 50, 36, 35, 48 us; fp16 (5120, 5120) with 400 rows: -, 74, 44, 57, (4096, 4096) with 200: -, 69, 38, 20
-//   skinny kernel: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; 25 GB/s a CU, a line of x (from L2) at 0.7 of the
-//     price of a line of weights.  32 rows bf16, (25600, 4096): one slice 119 us, four 46, eight 45; (4096, 6144): one 23, three 19, four 18 (slices of equal length);
-//     (4096, 21504): one 40, two 42; nine items of (2048, 2816): one 21, three 31; three rows fp32, (8448, 2048): one 75, eight 21; pairs, four
-//     rows, (2048, 11264): one 17, two 23
-//   narrow kernel, up to 32 rows of one item: 16 columns a workgroup, a line of x at 0.6 of the price of a line of weights; the way through memory costs
-//     slices about 4.5 us more.  Narrow | slices, bf16: 8 rows (2048, 2048) 5.0 | 6.6 us, (4096, 4096) 9.4 | 11.8, (25600, 4096) 38.7 | 40.0, (2048, 8448)
-//     11.8 | 11.3, (4096, 12288) 24.2 | 21.8; 16 rows (14336, 4096) 28.0 | 25.2; 32 rows (768, 768) 4.2 | 6.0 (one slice), (2048, 2048) 7.4 | 8.2, (4096,
-//     4096) 14.2 | 13.3, (25600, 4096) 68 | 44; fp32, 4 rows: (2048, 2048) 8.0 | 9.2, (2048, 4096) 9.8 | 12.1, (2048, 6144) 15.5 | 14.3, (4096, 3072) 15.8
-//     | 13.9, (25600, 4096) 76.2 | 76.3
-StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border)
+//   few rows of one item (few_rows_cost): what the workgroups of the fullest CU stream, at 32 - 33 GB/s of weights a CU with a line of x (from L2) at a fraction
+//     of the price of a line of weights; 6.1 TB/s for all of them; a workgroup's chain of steps; for slices the way through memory.  Of 184 sizes
+//     (K 768 ... 25600, N 768 ... 32000, 1 ... 64 rows, bf16 and fp32, 64 and 96 columns a workgroup, 1 ... 16 slices and the narrow kernel) what it takes is on
+//     average 0.8 % and at most 10 % slower than the best.  us, bf16: (4096, 21504) 32 rows, 64 columns 38.9 (two workgroups on some CUs), 96 columns 30.1; (25600,
+//     4096) 32 rows, one slice 95, four 36, eight 39; (4096, 6144) 32 rows, 96 columns four slices 14.8, 64 columns four 15.8, one 18.6; (2048, 2048) 8
+//     rows, narrow 5.1, four slices 6.3, one 7.9; (14336, 4096) 16 rows, narrow 27.3, four slices 21.6; fp32, 3 rows: (8448, 2048) narrow 19.9, eight slices
+//     15.3; (4096, 4096) narrow 13.8, four slices 16.2
+//   items, pairs: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; nine items of (2048, 2816): one 21, three 31; pairs, four rows,
+//     (2048, 11264): one 17, two 23
+// us; cw: column tiles a workgroup (0: narrow kernel), ss: steps of one of sp slices
+static double few_rows_cost(int steps, int cols, int rows, int elem, int cw, int sp, int ss)
+{
+    const int    mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, wgs = cw ? (cols / 16 + cw - 1) / cw * sp : cols / 16;
+    const double per_cu = wgs <= 1024 ? (wgs + 255) / 256 : wgs / 256.0;
+    const double all    = cols * 64e-6 * steps / 6.1;
+    if (cw == 0) {
+        return 2.4 + std::max(all, per_cu * steps * 64 * (16 + 0.82 * rows) / 33e3);
+    }
+    const double chain = ss * (0.018 + 0.037 * mt * (elem == 4 ? 2.6 : 1.0)), mfma = elem == 4 ? per_cu * ss * cw * mt * 0.026 : 0.0;  // (fp32: the matrix unit too)
+    return 2.6 + std::max({all, per_cu * ss * 64 * (cw * 16 + 0.26 * rows) / 32e3, chain, mfma}) + (sp > 1 ? 2.4 + 0.66 * sp * rows * cols * 4e-6 : 0.0);
+}
+
+StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border,
+                       bool k_major)
 {
     struct Tile {
         int    rows, cols;
@@ -348,10 +362,34 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     if (own_rows ? rows > 64 : rows > 256) {  // (an item's rows are one block of the skinny kernel)
         return best;
     }
-    const int    mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, rb = (rows + 16 * mt - 1) / (16 * mt), wg_cols = pairs ? 128 : 64;
-    const int    groups = (cols + wg_cols - 1) / wg_cols * items * rb;
-    const double step   = 64.0 * (wg_cols + 0.7 * std::min(rows, 16 * mt)) / 25e3;
-    int          sp     = groups >= (pairs ? 80 : 200) ? 1 : (256 + groups - 1) / groups;  // about one workgroup a CU
+    const int mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, rb = (rows + 16 * mt - 1) / (16 * mt);
+    best.mt = mt, best.row_blocks = rb, best.cw = pairs ? 8 : 4, best.splits = 1, best.split_steps = (steps + 7) / 8 * 8;
+    if (items == 1 && !pairs && rows <= 64) {
+        // (the waves of a narrow workgroup read pieces of 4 KB that lie far apart in a k-major image: fp16 (2048, 16384) 8 rows, narrow 14.6, 64 columns 11.9,
+        // (2048, 4096) 48 rows 10.2 and 9.4)
+        double least = k_major && cols > (rows > 32 ? 2048 : 8192) ? 1e30 : few_rows_cost(steps, cols, rows, elem, 0, 1, 0);
+        best.skinny = best.narrow = true;
+        for (int cw : {4, 6}) {
+            const int groups = (cols / 16 + cw - 1) / cw;
+            if (border % (16 * cw)) {
+                continue;
+            }
+            for (int sp = 1; sp <= 16 && (sp == 1 || steps / sp >= 16); ++sp) {
+                const int ss = ((steps + sp - 1) / sp + 7) / 8 * 8;
+                if ((steps + ss - 1) / ss != sp || (sp > 1 && ((size_t)sp * rows * cols * 4 > ws_bytes || groups > tickets))) {
+                    continue;
+                }
+                const double c = few_rows_cost(steps, cols, rows, elem, cw, sp, ss);
+                if (c < least) {
+                    least = c, best.narrow = false, best.cw = cw, best.splits = sp, best.split_steps = ss;
+                }
+            }
+        }
+        return best;
+    }
+    const int    wg_cols = pairs ? 128 : 64, groups = (cols + wg_cols - 1) / wg_cols * items * rb;
+    const double step = 64.0 * (wg_cols + 0.7 * std::min(rows, 16 * mt)) / 25e3;
+    int          sp   = groups >= (pairs ? 80 : 200) ? 1 : (256 + groups - 1) / groups;  // about one workgroup a CU
     sp          = std::max(1, std::min({sp, steps / 16, 16}));
     for (int more = sp; sp > 1 && more < 2 * sp && more <= 16; ++more) {  // slices of equal length
         if (steps % (8 * more) == 0) {
@@ -359,14 +397,7 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
             break;
         }
     }
-    if (items == 1 && !pairs && rows <= 32 && groups < 200) {
-        const int    wgs = (cols + 15) / 16, len = ((steps + sp - 1) / sp + 7) / 8 * 8;
-        const double slices = std::max(1.0, groups * sp / 256.0) * len * step + (sp > 1 ? 7.0 : 2.5);
-        best.narrow = (elem == 4 ? wgs <= 256 && steps <= 128 : wgs <= 512) && (wgs + 255) / 256 * (steps * 64.0 * (16 + 0.6 * rows) / 25e3) + 2.5 < slices;
-    }
-    else {
-        best.narrow = groups <= 64 && !pairs && rows <= 16 && steps <= 64;  // short sums: the way through memory costs more than it gives
-    }
+    best.narrow = groups <= 64 && !pairs && rows <= 16 && steps <= 64;  // short sums: the way through memory costs more than it gives
     if (best.narrow) {
         sp = 1;
     }
@@ -376,7 +407,7 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     const int    ss = ((steps + sp - 1) / sp + 7) / 8 * 8;
     const double c  = std::max(1.0, groups * sp / 256.0) * ss * step + 3.0;
     if (rows <= 64 || c < cost) {
-        best.skinny = true, best.mt = mt, best.splits = (steps + ss - 1) / ss, best.split_steps = ss, best.row_blocks = rb;
+        best.skinny = true, best.splits = (steps + ss - 1) / ss, best.split_steps = ss;
     }
     return best;
 }
@@ -478,14 +509,13 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
     const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2,
                                      d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border);
     if (p.skinny) {
-        const bool pairs = epi == kDenseGatedAct && sizeof(T) == 2;
-        a.split_steps    = p.split_steps;
-        a.row_blocks     = p.row_blocks;
-        a.slabs          = p.splits > 1 ? d.scratch->slabs : nullptr;
-        a.tickets        = p.splits > 1 ? d.scratch->tickets : nullptr;
-        const dim3 grid((unsigned)((a.tiles + (pairs ? 7 : 3)) / (pairs ? 8 : 4)), G * p.row_blocks, p.splits);
+        a.split_steps = p.split_steps;
+        a.row_blocks  = p.row_blocks;
+        a.slabs       = p.splits > 1 ? d.scratch->slabs : nullptr;
+        a.tickets     = p.splits > 1 ? d.scratch->tickets : nullptr;
+        const dim3 grid((unsigned)((a.tiles + p.cw - 1) / p.cw), G * p.row_blocks, p.splits);
 #define TM_SKINNY(MT_, NT_, CW_, KP_)                                                    \
-    if (p.mt == MT_ && pairs == (NT_ == 2)) {                                            \
+    if (p.mt == MT_ && p.cw == CW_ * NT_) {                                              \
         if (p.narrow) {                                                                  \
             return launch_dense_narrow<T, MT_, NT_>(a, call, vec, G, st);                \
         }                                                                                \

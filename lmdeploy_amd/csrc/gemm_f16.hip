@@ -74,29 +74,30 @@ struct F16Epi {
 
 // Where gemm_kernel is still the better one: its workgroups of 64 rows x 128 columns take the weights straight into registers and read x half as often as 64
 // columns do, so it wins where about one round of them keeps the CUs busy.  us, gemm_kernel | here, weights from HBM:
-//   up to 16 rows, 192 ... 256 workgroups: (K, N) = (4096, 28672) gated 36.4 | 39.6, (5120, 27648) gated 43.3 | 48, (4096, 32000) 40.4 | 42.2; not (4096,
-//     14336) 29.6 | 28.1, (2048, 92544) 59 | 58
-//   17 ... 64 rows, from 112 on: (2048, 16384) gated, 32 rows 17.0 | 18.6, (4096, 14336) 48 rows 33 | 35, (4096, 128256) 64 rows 191 | 216; not (4096,
-//     8192) gated 0.71 - 0.79 of its time here, (14336, 4096) 64 rows 98 | 35
+//   up to 64 rows, 193 ... 256 workgroups: (K, N) = (4096, 28672) gated 8 rows 35.4 | 34.7, 32 rows 35.5 | 38.5, 64 rows 40 | 44, (5120, 27648) gated 8 rows
+//     43.6 | 44.1, 64 rows 48 | 55, (4096, 32000) 64 rows 42 | 47; not (4096, 24576) 32 rows 34 | 32, (4096, 20480) 64 rows 37 | 31, (2048, 16384) gated 21 | 15,
+//     nor (4096, 36864) 32 rows 65 | 55, (4096, 8192) gated 27 | 16
+//   41 ... 64 rows of very wide outputs: (4096, 128256) 64 rows 186 | 197, 48 rows 179 | 183, (2048, 92544) 64 rows 72 | 74; not 32 rows 171 | 167
 //   more rows, one round of them where 64 x 64 tiles take two: (2048, 16384) gated, 128 rows 20.9 | 26, (4096, 6144) 192 rows 30 | 42, (4096, 4096) 320 rows 29 |
 //     39, (14336, 4096) 320 rows 92 | 130; not where one round of tiles is enough, (4096, 4096) 256 rows 29 | 23, nor where it takes two, 640 rows 58 | 45
 bool f16_stream_supported(const LinearWeight& w, int M)
 {
     const int  rb = (M + 63) / 64, t64 = (w.N + 63) / 64 * rb, t128 = (w.N + 127) / 128 * rb;
-    const bool general = M <= 16 ? t128 >= 192 && t128 <= 256 : M <= 64 ? t128 >= 112 : t64 > 256 && t128 <= 256;
+    const bool general = M <= 64 ? (t128 > 192 && t128 <= 256) || (M > 40 && t128 > 448) : t64 > 256 && t128 <= 256;
     return w.type == 1 && w.packed && (size_t)w.K * w.N * 2 < ((size_t)1 << 31) && !general;  // (byte offsets inside the image are 32 bits)
 }
 
 int f16_stream_splits(const LinearWeight& w, int M)
 {
-    const StreamPlan p = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, ~(size_t)0, 1 << 30);
+    const StreamPlan p = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, ~(size_t)0, 1 << 30, 0, true);
     return p.skinny ? p.splits : 1;
 }
 
 template<int MT>
-static int launch_skinny(const StreamArgs& a, const F16Epi& epi, int splits, bool narrow, hipStream_t st)
+static int launch_skinny(const StreamArgs& a, const F16Epi& epi, const StreamPlan& p, hipStream_t st)
 {
-    if (narrow) {
+    const dim3 grid((a.tiles + p.cw - 1) / p.cw, a.row_blocks, p.splits);
+    if (p.narrow) {
         if (MT <= 2 && stream_narrow_waves(a) == 16) {
             stream_narrow_kernel<half_t, F16Epi, MT, 1, MT <= 2 ? 16 : 8><<<dim3(a.tiles, a.row_blocks), 1024, 0, st>>>(a, epi);
         }
@@ -104,8 +105,11 @@ static int launch_skinny(const StreamArgs& a, const F16Epi& epi, int splits, boo
             stream_narrow_kernel<half_t, F16Epi, MT, 1, 8><<<dim3(a.tiles, a.row_blocks), 512, 0, st>>>(a, epi);
         }
     }
+    else if (p.cw == 6) {
+        stream_skinny_kernel<half_t, F16Epi, MT, 1, 6, 1><<<grid, 384, 0, st>>>(a, epi);
+    }
     else {
-        stream_skinny_kernel<half_t, F16Epi, MT, 1, 4, 1><<<dim3((a.tiles + 3) / 4, a.row_blocks, splits), 256, 0, st>>>(a, epi);
+        stream_skinny_kernel<half_t, F16Epi, MT, 1, 4, 1><<<grid, 256, 0, st>>>(a, epi);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
@@ -130,7 +134,7 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
 {
     TM_REQUIRE(f16_stream_supported(w, M), "fp16 linear: image");
     const bool       slice = splits > 1 && workspace;
-    const StreamPlan p     = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, slice ? ~(size_t)0 : 0, slice ? 1 << 30 : 0);
+    const StreamPlan p     = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, slice ? ~(size_t)0 : 0, slice ? 1 << 30 : 0, 0, true);
     StreamArgs       a{};
     a.x = (const char*)x, a.ldx = (int64_t)ldx * 2;
     a.w = (const char*)w.packed, a.tiles = w.N / 16, a.steps = w.K / 32;
@@ -144,11 +148,10 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
         a.row_blocks  = p.row_blocks;
         if (p.splits > 1) {
             a.slabs   = workspace;
-            a.tickets = defer || (a.tiles + 3) / 4 * p.row_blocks > ticket_count ? nullptr : tickets;
+            a.tickets = defer || (a.tiles + p.cw - 1) / p.cw * p.row_blocks > ticket_count ? nullptr : tickets;
             *slabs    = a.tickets ? 1 : p.splits;
         }
-        return p.mt == 1 ? launch_skinny<1>(a, epi, p.splits, p.narrow, st) : p.mt == 2 ? launch_skinny<2>(a, epi, p.splits, p.narrow, st) :
-                                                                                        launch_skinny<4>(a, epi, p.splits, p.narrow, st);
+        return p.mt == 1 ? launch_skinny<1>(a, epi, p, st) : p.mt == 2 ? launch_skinny<2>(a, epi, p, st) : launch_skinny<4>(a, epi, p, st);
     }
     return p.tile == 0 ? launch_tiles(stream_tile256_kernel<half_t, F16Epi>, a, epi, 256, 256, st) :
            p.tile == 1 ? launch_tiles(stream_tile_kernel<half_t, F16Epi, 256, 128, 2, 2>, a, epi, 256, 128, st) :

@@ -774,10 +774,9 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
 }
 
 // ---- which kernel, which shape -------------------------------------------------------------------------------------------------------
-// (row tiles, column tiles a wave, column waves, k-phases) of the skinny kernels that exist: 64 columns a workgroup of four waves, and 128 columns where
-// a wave needs a pair of column tiles.  Of 15 shapes (column groups of 64 and 128, one to four k-phases) these were the fastest or within 3 %
-// everywhere (K 768 ... 25600, N 256 ... 32000, 3 ... 64 rows); the number of slices of k matters more.
-#define TM_STREAM_SHAPES(X) X(1, 1, 4, 1) X(2, 1, 4, 1) X(4, 1, 4, 1)
+// (row tiles, column tiles a wave, column waves, k-phases) of the skinny kernels that exist: 64 columns a workgroup of four waves, 96 of six where those
+// fill the CUs more evenly, and 128 columns where a wave needs a pair of column tiles.  Eight waves (128 columns) gave 1 - 2 % at two of 184 sizes, k-phases nothing.
+#define TM_STREAM_SHAPES(X) X(1, 1, 4, 1) X(2, 1, 4, 1) X(4, 1, 4, 1) X(1, 1, 6, 1) X(2, 1, 6, 1) X(4, 1, 6, 1)
 #define TM_STREAM_SHAPES_PAIRS(X) X(1, 2, 4, 2) X(2, 2, 4, 2) X(4, 2, 4, 1)
 
 // waves of the narrow kernel (row tiles x column tiles <= 2): eight where sixteen would have nothing to do, or would keep a second workgroup off the CU
@@ -788,13 +787,14 @@ inline int stream_narrow_waves(const StreamArgs& a)
 
 struct StreamPlan {
     bool skinny, narrow;  // narrow: no slices across workgroups
-    int  mt, splits, split_steps, row_blocks;  // skinny kernel
+    int  mt, cw, splits, split_steps, row_blocks;  // skinny kernel (cw: column tiles a workgroup)
     int  tile;                                 // 0: 256 x 256 (16-bit formats), 1: 256 x 128, 2: 128 x 128, 3: 64 x 64
 };
 // steps of k, image columns, rows, items (own_rows: each with rows of its own, `rows` in total), bytes of an element; pairs: a wave needs two
 // column tiles; ws_bytes / tickets: what slices of k may use (0: no slices); border: x is read elsewhere from multiples of this many columns on (a
-// multiple of 128; 0: nowhere)
-StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0);
+// multiple of 128; 0: nowhere); k_major: the image holds four steps of every column tile before the next four
+StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0,
+                       bool k_major = false);
 constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
 constexpr int    kStreamTickets = 4096;
 
