@@ -5,15 +5,7 @@
 
 namespace tmk {
 
-__global__ void advance_kernel(int* k_len, int batch)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b < batch) {
-        k_len[b] += 1;
-    }
-}
-
-// continuous batching: only slots that hold a running sequence advance
+// continuous batching, a decode step that rides on a prompt forward: only slots that hold a running sequence advance
 __global__ void advance_active_kernel(int* k_len, const int* active, int batch)
 {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
@@ -22,27 +14,11 @@ __global__ void advance_active_kernel(int* k_len, const int* active, int batch)
     }
 }
 
-// continuous batching: a finished / cancelled slot goes back to the scratch block (no host memory involved: the launch needs
-// no synchronisation, so it can queue up behind a decode step that is still running)
-int launch_advance_active(int* k_len, const int* active, int n, hipStream_t st)
+static int launch_advance_active(int* k_len, const int* active, int n, hipStream_t st)
 {
     advance_active_kernel<<<(n + 63) / 64, 64, 0, st>>>(k_len, active, n);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
-}
-
-// ids -> generated[b][step]; step++ (single thread does the counter after everybody read it)
-__global__ void record_kernel(const int* ids, int* generated, int* step_counter, int batch, int max_new)
-{
-    const int b    = blockIdx.x * blockDim.x + threadIdx.x;
-    const int step = *step_counter;
-    if (b < batch && step < max_new) {
-        generated[(size_t)b * max_new + step] = ids[b];
-    }
-    __syncthreads();
-    if (b == 0) {
-        *step_counter = step + 1;
-    }
 }
 
 // pick the global arg-max out of tp (value, index) candidates per sequence
@@ -345,12 +321,19 @@ static int linear_fold_produce(tm_engine* e, LinearSlots& l, const half_t* x, in
 // Logits rows -> next ids for `n` sequences whose fp16 logits lie in d_logits at the batch slots [slot, slot + n): logits processors
 // (ids_in / cu_q (nullptr: one token per sequence) / ntok = the tokens this forward consumed for them, k_len = their context lengths),
 // then stochastic sampling or arg-max (tensor-parallel: over the gathered vocabulary shards).  Shared by every model family.
-int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_q, int ntok, const int* k_len, const int* active)
+// logits32: the rows are still fp32 ([n][vocab]) and become the fp16 ones here.  commit: what a decode step does with the tokens.
+int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_q, int ntok, const int* k_len, const int* active, const float* logits32,
+                const StepCommit* commit)
 {
     const tm_model_config& m      = e->cfg.model;
     hipStream_t            st     = e->stream;
     half_t*                logits = e->d_logits + (size_t)slot * e->vocab_local;
     int*                   ids    = e->d_next_ids + slot;
+    const bool             greedy = !e->use_comm && !e->sampling_on;
+    if (logits32 && !(greedy && !e->logits_on)) {
+        TM_TRY(launch_f32_to_f16_rows(logits, e->vocab_local, logits32, n, m.vocab, st));
+        logits32 = nullptr;
+    }
     if (e->logits_on) {
         // the tokens this forward consumed join the slots' seen masks, then penalty / bans on the (local) logits
         uint32_t* seen = e->d_seen + (size_t)slot * e->seen_words;
@@ -406,7 +389,9 @@ int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_
                                                e->d_topp + slot, e->d_minp + slot, e->d_u + slot, e->d_sample_ws, st, lpr ? &lp : nullptr)));
     }
     else if (!e->use_comm) {
-        TM_PROF(P_SAMPLE, TM_TRY(launch_argmax(ids, nullptr, logits, n, e->vocab_local, e->vocab_local, 0, st)));
+        TM_PROF(P_SAMPLE, TM_TRY(launch_greedy(ids, logits, e->vocab_local, logits32, logits32 ? m.vocab : e->vocab_local, n, e->d_greedy_ws,
+                                               e->greedy_ws_floats, e->d_greedy_tickets, e->cfg.max_batch_size + 1, commit ? *commit : StepCommit{}, st)));
+        return 0;
     }
     else {
         TM_TRY(launch_argmax(ids, e->d_argmax_val, logits, n, e->vocab_local, e->vocab_local, e->cfg.rank * e->vocab_local, st));
@@ -425,6 +410,16 @@ int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_
         pick_kernel<<<(n + 63) / 64, 64, 0, st>>>(ids, e->d_cand_all, e->cfg.tp, n);
         TM_HIP_CHECK(hipGetLastError());
     }
+    return commit ? launch_commit(ids, n, *commit, st) : 0;
+}
+
+int greedy_alloc(tm_engine* e)
+{
+    const int B         = e->cfg.max_batch_size;
+    e->greedy_ws_floats = greedy_workspace_floats(B, (e->vocab_local + 7) / 8 * 8);
+    TM_TRY(dmalloc(&e->d_greedy_ws, e->greedy_ws_floats));
+    TM_TRY(dmalloc(&e->d_greedy_tickets, (size_t)B + 1));
+    TM_HIP_CHECK(hipMemset(e->d_greedy_tickets, 0, ((size_t)B + 1) * 4));
     return 0;
 }
 
@@ -435,10 +430,11 @@ int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_
 // prefill tokens of `nseq` sequences described by e->d_cu_q / d_k_len / d_rows (d_rows already counts from row 0 of the
 // forward).  Every linear, norm and (MoE) FFN runs ONCE over all M rows -- one weight stream serves both.
 int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len,
-                   int kflat_stride, int slot0, const MixedDecode* md)
+                   int kflat_stride, int slot0, const MixedDecode* md, const StepEnds* ends)
 {
+    TM_REQUIRE(!ends || (decode && M == nseq), "internal: the ends of a decode step");
     if (e->lm) {  // layer-list model family (engine_layered.hip): same batch description, its own layer loop
-        return layered_forward(e, d_ids, M, nseq, decode, max_q_len, max_k_len, slot0, md);
+        return layered_forward(e, d_ids, M, nseq, decode, max_q_len, max_k_len, slot0, md, ends);
     }
     const tm_model_config& m = e->cfg.model;
     hipStream_t            st = e->stream;
@@ -446,8 +442,8 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
     TM_REQUIRE(!md || (!decode && nd > 0 && nd < M), "internal: mixed forward");
     half_t* const qkv_p  = e->d_qkv + (size_t)nd * e->qkv_n;            // first prefill row
     half_t* const attn_p = e->d_attn + (size_t)nd * e->q_heads * e->D;
-    TM_PROF(P_EMBED, TM_TRY(launch_embedding(e->d_resid, e->tok_embeddings, d_ids, M, e->hidden, m.vocab, st)));
-    TM_PROF(P_RES_NORM, TM_TRY(launch_rmsnorm(e->d_x, e->d_resid, e->layers[0].attn_norm, m.rms_eps, M, e->hidden, st)));
+    TM_PROF(P_EMBED, TM_TRY(launch_embedding_rmsnorm(e->d_x, e->d_resid, e->tok_embeddings, d_ids, m.vocab, e->layers[0].attn_norm, m.rms_eps, M, e->hidden,
+                                                     ends ? ends->begin : StepBegin{}, st)));
     const float scale_log2 = (1.0f / std::sqrt((float)e->D)) * 1.4426950408889634f;
     // tp > 1 prefill through RCCL: the row-wise part of every dense layer as two row halves, all-reduces on the side stream
     e->pipe_events_used = 0;
@@ -631,7 +627,7 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
                     const int* active = nullptr) -> int {
         half_t* logits = e->d_logits + (size_t)slot * e->vocab_local;
         TM_PROF(P_LM_HEAD, TM_TRY(linear_plain(e, e->output, hx, e->hidden, logits, e->vocab_local, n, false)));
-        return sample_rows(e, n, slot, ids_in, cu_q, ntok, k_len, active);
+        return sample_rows(e, n, slot, ids_in, cu_q, ntok, k_len, active, nullptr, ends ? &ends->commit : nullptr);
     };
     if (decode) {
         return head(e->d_x, nseq, slot0, d_ids, nullptr, M, e->d_k_len);
@@ -643,22 +639,15 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
     return head(e->d_last, nseq, slot0, d_ids + nd, e->d_cu_q, M - nd, e->d_k_len);
 }
 
-// next ids become the current ids and are appended to generated[b][step]
-static int commit_tokens(tm_engine* e)
+static StepCommit step_commit(tm_engine* e)
 {
-    TM_HIP_CHECK(hipMemcpyAsync(e->d_ids, e->d_next_ids, (size_t)e->batch * 4, hipMemcpyDeviceToDevice, e->stream));
-    record_kernel<<<1, std::max(64, ((e->batch + 63) / 64) * 64), 0, e->stream>>>(e->d_ids, e->d_generated, e->d_step,
-                                                                                  e->batch, e->max_new);
-    TM_HIP_CHECK(hipGetLastError());
-    return 0;
+    return StepCommit{e->d_ids, e->d_generated, e->d_step, e->max_new};
 }
 
 static int decode_step(tm_engine* e)
 {
-    advance_kernel<<<(e->batch + 63) / 64, 64, 0, e->stream>>>(e->d_k_len, e->batch);
-    TM_HIP_CHECK(hipGetLastError());
-    TM_TRY(forward(e, e->d_ids, e->batch, e->batch, true, 1, 0, 0, 0));
-    return commit_tokens(e);
+    const StepEnds ends{{e->d_k_len, nullptr}, step_commit(e)};
+    return forward(e, e->d_ids, e->batch, e->batch, true, 1, 0, 0, 0, nullptr, &ends);
 }
 
 }  // namespace tmk
@@ -1089,7 +1078,7 @@ int tm_engine_prefill(tm_engine* e, const int* host_ids, const int* host_lens, i
     TM_HIP_CHECK(hipMemcpyAsync(e->d_k_len, host_lens, batch * 4, hipMemcpyHostToDevice, e->stream));
     // generated[b][0] = first token; step counter = 1
     TM_HIP_CHECK(hipMemsetAsync(e->d_step, 0, 4, e->stream));
-    TM_TRY(commit_tokens(e));
+    TM_TRY(launch_commit(e->d_next_ids, e->batch, step_commit(e), e->stream));
     TM_HIP_CHECK(hipStreamSynchronize(e->stream));
     e->steps_done = 1;
 

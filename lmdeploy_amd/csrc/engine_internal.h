@@ -301,6 +301,9 @@ struct tm_engine {
     int *d_generated = nullptr, *d_step = nullptr;
     int *d_prefill_ids = nullptr;
     half_t* d_argmax_val = nullptr;
+    float*    d_greedy_ws      = nullptr;  // where the workgroups of a row's arg-max meet: [max_batch_size], and a ticket for each and for all
+    unsigned* d_greedy_tickets = nullptr;
+    size_t    greedy_ws_floats = 0;
     float*  d_cand = nullptr;
     float*  d_cand_all = nullptr;
 
@@ -322,7 +325,7 @@ struct tm_engine {
     std::vector<std::tuple<int, size_t, size_t>>    prof_spans;  // (category, start event, stop event)
     std::vector<float>                              h_ttft_ms;
     int            graph_batch = 0;
-    int            graph_max_new = 0;  // record_kernel's bound is a captured kernel argument
+    int            graph_max_new = 0;  // the record's bound is a captured kernel argument
 
     // continuous batching (tm_engine_submit / step / poll / cancel): slot-based, every decode step runs all
     // max_batch_size slots; free slots are parked on a scratch block with k_len = 1 and never advance
@@ -469,8 +472,13 @@ inline int dmalloc(T** p, size_t n)
     return 0;
 }
 
+// what a decode step's forward does besides: its first and its last launch
+struct StepEnds {
+    StepBegin  begin;
+    StepCommit commit;
+};
+
 // ---- shared between the engine translation units ----
-int launch_advance_active(int* k_len, const int* active, int n, hipStream_t st);
 size_t prof_event(tm_engine* e);
 void p2p_tables(tm_engine* e, half_t** data, uint32_t** flags);
 int reduce_residual_norm(tm_engine* e, int M, const half_t* norm_w);
@@ -478,9 +486,12 @@ bool prefill_pipe_ok(const tm_engine* e, int M);
 int allreduce_rows_side(tm_engine* e, int r0, int rows, hipEvent_t* done);
 int pipe_wait(tm_engine* e, hipEvent_t done);
 int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len, int kflat_stride, int slot0,
-            const MixedDecode* md = nullptr);
-int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_q, int ntok, const int* k_len, const int* active);
-int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len, int slot0, const MixedDecode* md);
+            const MixedDecode* md = nullptr, const StepEnds* ends = nullptr);
+int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_q, int ntok, const int* k_len, const int* active, const float* logits32,
+                const StepCommit* commit);
+int greedy_alloc(tm_engine* e);
+int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len, int slot0, const MixedDecode* md,
+                    const StepEnds* ends);
 int layered_process_weights(tm_engine* e);
 int layered_init_synthetic(tm_engine* e, uint64_t seed);
 int layered_start(tm_engine* e);

@@ -1103,6 +1103,7 @@ int layered_start(tm_engine* e)
     TM_TRY(lm_alloc(&e->d_step, (size_t)1, st));
     TM_TRY(lm_alloc(&e->d_prefill_ids, T, st));
     TM_TRY(lm_alloc(&e->d_argmax_val, (size_t)B, st));
+    TM_TRY(greedy_alloc(e));
     TM_TRY(lm_alloc(&e->d_cand, (size_t)B * 2, st));
     TM_TRY(lm_alloc(&e->d_cand_all, (size_t)B * 2, st));
     TM_TRY(lm_alloc(&e->d_block_ptrs, (size_t)B * e->max_blocks_per_seq, st));
@@ -1863,18 +1864,18 @@ static int both_layer(tm_engine* e, const LmLayer& L, const LmLayer* next, int M
 }
 
 // the layer loop over M rows described by `parts`; leaves the residual stream in lm.d_res
-static int layered_layers(tm_engine* e, const int* d_ids, int M, const LmPart* parts, int nparts)
+static int layered_layers(tm_engine* e, const int* d_ids, int M, const LmPart* parts, int nparts, const StepBegin& begin = {})
 {
     LayeredModel&            lm = *e->lm;
     const tm_layered_config& m  = lm.cfg;
     hipStream_t              st = e->stream;
     TM_REQUIRE(M >= 1 && M <= e->max_tokens, "forward: more rows than max_prefill_token_num");
-    for (int i = 0; i < nparts; ++i) {
+    for (int i = 0; i < nparts && !begin.k_len; ++i) {
         const LmPart& P = parts[i];
         TM_TRY(launch_rows_prepare(lm.d_row_seq + P.row0, lm.d_row_pos + P.row0, P.cu_q, P.k_len, P.nseq, P.rows, st));
     }
     TM_PROF(P_EMBED, TM_TRY(launch_embedding_f32(lm.d_res, lm.embed, lm.elem, d_ids, M, m.width, m.vocab, st, m.embed_scale != 0.f ? m.embed_scale : 1.f,
-                                                  m.loop_add ? lm.d_x0 : lm.d_hist)));
+                                                  m.loop_add ? lm.d_x0 : lm.d_hist, begin, lm.d_row_seq, lm.d_row_pos)));
     if (m.loop_times > 0) {  // the embedding output is read again where a loop pass begins
         TM_PROF(P_EMBED, TM_TRY(launch_embedding_f32(lm.d_x0, lm.embed, lm.elem, d_ids, M, m.width, m.vocab, st)));
     }
@@ -1963,20 +1964,25 @@ static int layered_logits(tm_engine* e, const int* rows, int n)
 
 // logits of `n` sequences -> the engine's fp16 logits rows at the batch slots [slot, slot + n) -> logits processors + sampling
 static int layered_head(tm_engine* e, const int* rows, int n, int slot, const int* ids_in, const int* cu_q, int ntok, const int* k_len,
-                        const int* active)
+                        const int* active, const StepCommit* commit = nullptr)
 {
     LayeredModel& lm = *e->lm;
+    if (n <= lm.max_logit_rows) {
+        TM_TRY(layered_logits(e, rows, n));
+        return sample_rows(e, n, slot, ids_in, cu_q, ntok, k_len, active, lm.d_logits_f32, commit);
+    }
     for (int r0 = 0; r0 < n; r0 += lm.max_logit_rows) {
         const int cnt = std::min(lm.max_logit_rows, n - r0);
         TM_TRY(layered_logits(e, rows + r0, cnt));
         TM_TRY(launch_f32_to_f16_rows(e->d_logits + (size_t)(slot + r0) * e->vocab_local, e->vocab_local, lm.d_logits_f32, cnt, lm.cfg.vocab,
                                       e->stream));
     }
-    return sample_rows(e, n, slot, ids_in, cu_q, ntok, k_len, active);
+    return sample_rows(e, n, slot, ids_in, cu_q, ntok, k_len, active, nullptr, commit);
 }
 
 // forward() of the engine for this family: the same batch description as every other model (engine_forward.hip)
-int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len, int slot0, const MixedDecode* md)
+int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len, int slot0, const MixedDecode* md,
+                    const StepEnds* ends)
 {
     LayeredModel& lm = *e->lm;
     const int     nd = md ? md->rows : 0;
@@ -1989,9 +1995,9 @@ int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode
     // (the decode step of continuous batching runs every slot: those without a running sequence are placeholders)
     parts[np++] = LmPart{nd, M - nd, nseq, e->d_cu_q, e->d_k_len, nullptr, e->d_block_ptrs, decode, decode ? 1 : max_q_len, slot0,
                          decode && e->sched ? e->d_active : nullptr};
-    TM_TRY(layered_layers(e, d_ids, M, parts, np));
+    TM_TRY(layered_layers(e, d_ids, M, parts, np, ends ? ends->begin : StepBegin{}));
     if (decode) {
-        return layered_head(e, lm.d_iota, nseq, slot0, d_ids, nullptr, M, e->d_k_len, nullptr);
+        return layered_head(e, lm.d_iota, nseq, slot0, d_ids, nullptr, M, e->d_k_len, nullptr, ends ? &ends->commit : nullptr);
     }
     if (md) {
         TM_TRY(layered_head(e, lm.d_iota, nd, 0, d_ids, nullptr, nd, md->k_len, md->active));

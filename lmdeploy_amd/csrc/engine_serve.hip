@@ -82,10 +82,8 @@ int cb_enter(tm_engine* e)
 static int decode_step_cb(tm_engine* e)
 {
     const int B = e->cfg.max_batch_size;
-    TM_TRY(launch_advance_active(e->d_k_len, e->d_active, B, e->stream));
-    TM_TRY(forward(e, e->d_ids, B, B, true, 1, 0, 0, 0));
-    TM_HIP_CHECK(hipMemcpyAsync(e->d_ids, e->d_next_ids, (size_t)B * 4, hipMemcpyDeviceToDevice, e->stream));
-    return 0;
+    const StepEnds ends{{e->d_k_len, e->d_active}, {e->d_ids}};
+    return forward(e, e->d_ids, B, B, true, 1, 0, 0, 0, nullptr, &ends);
 }
 
 // park a slot again after its sequence finished / was cancelled

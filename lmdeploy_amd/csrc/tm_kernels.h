@@ -40,8 +40,25 @@ struct KvCacheView {
     KvLayout        layout;
 };
 
+// ---- the two ends of a decode step ---------------------------------------------------------
+// its first launch, row t = sequence t: the context lengths grow by one (active != nullptr: where a sequence runs); k_len == nullptr: not a decode step
+struct StepBegin {
+    int*       k_len  = nullptr;
+    const int* active = nullptr;
+};
+// its last launch: the chosen tokens become the current ids and, with a step counter, generated[row][max_new]'s entry at the counter, which then grows by one
+struct StepCommit {
+    int* cur_ids   = nullptr;
+    int* generated = nullptr;
+    int* step      = nullptr;
+    int  max_new   = 0;
+};
+
 // ---- norm.hip ---------------------------------------------------------------------------
 int launch_rmsnorm(half_t* y, const half_t* x, const half_t* w, float eps, int M, int H, hipStream_t st);
+// resid = table[ids[row]] and its norm
+int launch_embedding_rmsnorm(half_t* y, half_t* resid, const half_t* table, const int* ids, int vocab, const half_t* w, float eps, int M, int H,
+                             const StepBegin& begin, hipStream_t st);
 int launch_residual_rmsnorm(half_t* y, half_t* resid, const half_t* hidden, const float* partial, int splits,
                             const half_t* bias, const half_t* w, float eps, int M, int H, hipStream_t st);
 
@@ -497,7 +514,7 @@ int launch_rmsnorm_f32(void* y0, void* y1, int ldy, int out_elem_bytes, const fl
 // out fp32 [T][H] = table[ids[t]] * scale (table bf16 | fp32 [vocab][H])
 // (out2 != nullptr: a second copy)
 int launch_embedding_f32(float* out, const void* table, int table_elem_bytes, const int* ids, int T, int H, int vocab, hipStream_t st, float scale = 1.f,
-                         float* out2 = nullptr);
+                         float* out2 = nullptr, const StepBegin& begin = {}, int* row_seq = nullptr, int* row_pos = nullptr);
 // row_seq / row_pos of the rows [0, cu_q[nseq]) of nseq sequences: position = k_len[s] - (cu_q[s + 1] - cu_q[s]) + offset in the sequence
 int launch_rows_prepare(int* row_seq, int* row_pos, const int* cu_q, const int* k_len, int nseq, int rows, hipStream_t st);
 // keys / values of the new rows -> paged cache.  qkv [rows][ld]: keys at column k_col ([kv_heads][dim]), values at v_col ([kv_heads][vdim])
@@ -698,6 +715,12 @@ int launch_embedding(half_t* out, const half_t* table, const int* ids, int T, in
 int launch_fill_uniform_f16(half_t* out, size_t n, float amp, uint32_t seed, hipStream_t st);  // tuner stand-in activations
 int launch_argmax(int* out_ids, half_t* out_val, const half_t* logits, int B, int V, int ld, int id_offset,
                   hipStream_t st);
+// greedy tokens of `rows` rows of fp16 logits [rows][ld] (logits32: made here of fp32 [rows][V]); ws, tickets (zero between launches; rows + 1 of them): where the
+// workgroups of a row meet
+size_t greedy_workspace_floats(int rows, int ld);
+int launch_greedy(int* out_ids, half_t* rows16, int ld, const float* logits32, int V, int rows, float* ws, size_t ws_floats, unsigned* tickets, int ticket_count,
+                  const StepCommit& cm, hipStream_t st);
+int launch_commit(const int* ids, int n, const StepCommit& cm, hipStream_t st);
 int launch_gather_rows(half_t* out, const half_t* in, const int* rows, int n, int H, hipStream_t st);
 int launch_silu_mul(half_t* out, const half_t* gate_up, int M, int inter, hipStream_t st);
 int launch_quantize_groupwise_u4(int32_t* qweight, half_t* scales, half_t* zeros, half_t* dequant, const half_t* w,
