@@ -168,6 +168,40 @@ __device__ __forceinline__ void static_for8(F&& f)
     }
 }
 
+// Grouped: the tile of this workgroup, e < 0: none.  One-dimensional grid over (expert, column tile, row block) with only the row blocks that hold rows, the
+// row blocks of a column tile on consecutive turns of one XCD (workgroups are dealt to the eight in turn): its second-level cache serves a weight unit to
+// all of them.  (Empty blocks in between would leave the shader engines they fall on idle: up to 1.9 times slower.)
+struct Fp8Tile {
+    int e, ct, m0, row0, Mloc;
+};
+template<int ROWS, int CG>
+__device__ __forceinline__ Fp8Tile fp8_tile_of(const Fp8Params& p)
+{
+    const int turn = blockIdx.x >> 3;
+    int       e, n_e = 1, in_e;
+    if (p.one_block) {  // decode: no expert has more rows than a block
+        e    = turn / p.ct8;
+        in_e = turn - e * p.ct8;
+    }
+    else {
+        const int ln = threadIdx.x & 63, nb = ln < p.experts ? (p.seg[ln + 1] - p.seg[ln] + ROWS - 1) / ROWS : 0;
+        int       upto = nb;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(upto, d);
+            upto += ln >= d ? o : 0;
+        }
+        e = __popcll(__ballot(upto * p.ct8 <= turn));  // experts whose workgroups come before this turn
+        if (e >= p.experts) {
+            return {-1, 0, 0, 0, 0};
+        }
+        n_e  = __builtin_amdgcn_readlane(nb, e);
+        in_e = turn - (__builtin_amdgcn_readlane(upto, e) - n_e) * p.ct8;
+    }
+    const int ct = in_e / n_e * 8 + (blockIdx.x & 7), m0 = in_e % n_e * ROWS, row0 = p.seg[e], Mloc = min(ROWS, p.seg[e + 1] - row0 - m0);
+    return {ct * CG >= p.ncg || Mloc <= 0 ? -1 : e, ct, m0, row0, Mloc};
+}
+
 template<int MH, int CG, int WK, int S, bool GRP>
 __global__ __launch_bounds__(CG* WK * 64) void gemm_fp8_kernel(Fp8Params p)
 {
@@ -197,41 +231,12 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_fp8_kernel(Fp8Params p)
     int         m0 = blockIdx.z * ROWS, row0 = 0, Mloc = min(ROWS, p.M - m0), ct = blockIdx.x;
     const void* wbase = p.wp;
     if constexpr (GRP) {
-        // One-dimensional grid over (expert, column tile, row block) with only the row blocks that hold rows, the row blocks of a column tile on
-        // consecutive turns of one XCD (workgroups are dealt to the eight in turn): its second-level cache serves a weight unit to all of them.  (Empty
-        // blocks in between would leave the shader engines they fall on idle: up to 1.9 times slower.)
-        const int turn = blockIdx.x >> 3;
-        int       e, n_e = 1, in_e;
-        if (p.one_block) {  // decode: no expert has more rows than a block
-            e    = turn / p.ct8;
-            in_e = turn - e * p.ct8;
+        const Fp8Tile tl = fp8_tile_of<ROWS, CG>(p);
+        if (tl.e < 0) {
+            return;  // whole workgroup, before any barrier
         }
-        else {
-            const int ln = threadIdx.x & 63, nb = ln < p.experts ? (p.seg[ln + 1] - p.seg[ln] + ROWS - 1) / ROWS : 0;
-            int       upto = nb;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int o = __shfl_up(upto, d);
-                upto += ln >= d ? o : 0;
-            }
-            e = __popcll(__ballot(upto * p.ct8 <= turn));  // experts whose workgroups come before this turn
-            if (e >= p.experts) {
-                return;  // whole workgroup, before any barrier
-            }
-            n_e  = __builtin_amdgcn_readlane(nb, e);
-            in_e = turn - (__builtin_amdgcn_readlane(upto, e) - n_e) * p.ct8;
-        }
-        ct = in_e / n_e * 8 + (blockIdx.x & 7);
-        if (ct * CG >= p.ncg) {
-            return;
-        }
-        m0   = in_e % n_e * ROWS;
-        row0 = p.seg[e];
-        Mloc        = min(ROWS, p.seg[e + 1] - row0 - m0);
-        if (Mloc <= 0) {
-            return;
-        }
-        wbase       = p.groups[e];
+        ct = tl.ct, m0 = tl.m0, row0 = tl.row0, Mloc = tl.Mloc;
+        wbase = p.groups[tl.e];
     }
     const int cg  = ct * CG + cgl;
     const int cgc = min(cg, p.ncg - 1);
@@ -442,6 +447,208 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_fp8_kernel(Fp8Params p)
     }
 }
 
+// ---- many rows: 256 x 256 tiles ---------------------------------------------------------------------------------------------------------------------
+// The kernel above gives a weight unit to 128 rows at most and runs at the 16-bit instructions' rate; here a k-block of 256 rows x 256 columns meets in LDS
+// (66 KB, two stages: the next one is on its way by LDS-DMA during this one's products), and one v_mfma_f32_16x16x128_f8f6f4 is a whole scale block of
+// 16 x 16 outputs at twice that rate.  Eight waves of 64 rows x 128 columns: the fp32 accumulators are vector operands of the scaling, which the
+// accumulation registers cannot be, so 128 a lane is the most there are.  Products and scaling take turns one by one (behind each other in groups of four
+// and sixteen the two hardly overlapped: matrix cores 36 % busy, now 46 %); the rest is the barrier a k-block and LDS (192 KB read, 66 KB written a k-block).
+// Expert block 4096 x 14336, 8 experts, top 2, 4000 tokens: 3104 -> 1765 us, 8000: 6170 -> 2985 (1.89 PFLOP/s with routing and quantisation).
+// Lane l of an A operand holds column l & 15 and 32 of the 128 channels, those of a P8 unit's vectors 2 (l >> 5), 2 (l >> 5) + 1 and half (l >> 4) & 1; B
+// takes the same channels of row l & 15, so the order the instruction gives them in does not matter.
+typedef int intx8 __attribute__((ext_vector_type(8)));
+
+// LDS-DMA of 16 or 4 bytes a lane to consecutive places from dst on
+__device__ __forceinline__ void fp8_dma16(const __amdgpu_buffer_rsrc_t rs, int off, int soff, unsigned dst)
+{
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "buffer_load_dwordx4 %1, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(off), "s"(dst), "s"(rs), "s"(soff)
+                 : "memory");
+}
+__device__ __forceinline__ void fp8_dma4(const __amdgpu_buffer_rsrc_t rs, int off, int soff, unsigned dst)
+{
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "buffer_load_dword %1, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(off), "s"(dst), "s"(rs), "s"(soff)
+                 : "memory");
+}
+
+constexpr int kFp8TileX     = 256 * 128;                       // codes of 256 rows
+constexpr int kFp8TileW     = 8 * kP8Unit + 128;               // eight units
+constexpr int kFp8TileStage = kFp8TileX + kFp8TileW + 256 * 4;  // and the rows' scales
+constexpr int kFp8TileOut   = 64 * 288;                        // a wave's results on their way out, 64 rows
+constexpr int kFp8TileLds   = 8 * kFp8TileOut > 2 * kFp8TileStage ? 8 * kFp8TileOut : 2 * kFp8TileStage;
+
+__global__ __launch_bounds__(512) void gemm_fp8_tile256_kernel(Fp8Params p)
+{
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int     tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Fp8Tile tl = fp8_tile_of<256, 8>(p);
+    if (tl.e < 0) {
+        return;  // whole workgroup, before any barrier
+    }
+    const auto rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.groups[tl.e], 0, (int)((size_t)p.KB * p.ncg * kP8Unit), 0x00020000);
+    const auto rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)p.xq, 0, (int)((size_t)p.x_rows * p.K), 0x00020000);
+    const auto rs_s = __builtin_amdgcn_make_buffer_rsrc((void*)p.sx, 0, (int)((size_t)p.KB * p.ldsx * 4), 0x00020000);
+    auto       xrow = [&](int m) {  // (clamped duplicates past Mloc only feed rows that are never stored)
+        const int f = tl.row0 + tl.m0 + min(m, tl.Mloc - 1);
+        return p.row_idx ? p.row_idx[f] : f;
+    };
+    // DMA of a k-block: wave w takes 32 rows of x (pieces of 8 rows x 128 bytes; 16-byte unit u of row r at u ^ ((r >> 1) & 7)), weight unit w (its last piece, 256
+    // bytes, runs into the next unit's head: the same bytes that land there anyway, or the room behind the eighth) and the scales of 64 rows (two waves the same)
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)smem);
+    int            xoff[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int row = (4 * wave + r) * 8 + (lane >> 3);
+        xoff[r]       = xrow(row) * p.K + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    }
+    const int soff = xrow((wave & 3) * 64 + lane) * 4, w0 = (tl.ct * 8 + wave) * kP8Unit, wstep = p.ncg * kP8Unit;
+    auto      fetch = [&](int kb, int buf, int n) {  // piece n = 0 .. 9 of this wave
+        const unsigned dst = lds0 + buf * kFp8TileStage;
+        if (n < 4) {
+            fp8_dma16(rs_x, xoff[n], kb * 128, dst + (4 * wave + n) * 1024);
+        }
+        else if (n < 8) {
+            fp8_dma16(rs_w, lane * 16 + (n - 4) * 1024, w0 + kb * wstep, dst + kFp8TileX + wave * kP8Unit + (n - 4) * 1024);
+        }
+        else if (n == 8) {
+            fp8_dma4(rs_w, lane * 4 + 4096, w0 + kb * wstep, dst + kFp8TileX + wave * kP8Unit + 4096);
+        }
+        else {
+            fp8_dma4(rs_s, soff, kb * p.ldsx * 4, dst + kFp8TileX + kFp8TileW + (wave & 3) * 256);
+        }
+    };
+    const int c = lane & 15, q = lane >> 4, wr = wave >> 1, wc = wave & 1;
+    int       xf[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        xf[j] = (wr * 64 + c) * 128 + (((4 * (q >> 1) + j) ^ (c >> 1)) << 4) + (q & 1) * 8;
+    }
+    const int wf = kFp8TileX + wc * 4 * kP8Unit + (q >> 1) * 2048 + (c + 32 * (q & 1)) * 16;
+    const int sf = kFp8TileX + kFp8TileW + (wr * 64 + c) * 4;
+
+    floatx4 acc[4][2][4];  // unit, column half, row tile
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                acc[u][h][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 10; ++n) {
+        fetch(0, 0, n);
+    }
+    for (int kb = 0; kb < p.KB; ++kb) {
+        // this wave's pieces of the k-block have landed and its reads of the other stage are over; then everybody's
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int   nxt = min(kb + 1, p.KB - 1), nbuf = (kb + 1) & 1;  // (behind the last block: again, into the stage that nobody reads)
+        const char* st  = smem + (kb & 1) * kFp8TileStage;
+        intx8       a[2], b[4];
+        auto        read_a = [&](int i) {  // column tile i = 0 .. 7
+            const u32x4 a0 = *(const u32x4*)(st + wf + (i >> 1) * kP8Unit + (i & 1) * 256);
+            const u32x4 a1 = *(const u32x4*)(st + wf + (i >> 1) * kP8Unit + (i & 1) * 256 + 1024);
+            a[i & 1]       = intx8{(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1[0], (int)a1[1], (int)a1[2], (int)a1[3]};
+        };
+        read_a(0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                int off = (int)(st - smem) + xf[j] + t * 2048;
+                asm("" : "+v"(off));  // (two tiles' rows in one instruction, as the compiler would have them, meet in the same banks)
+                const u32x2 v   = *(const u32x2*)(smem + off);
+                b[t][2 * j]     = (int)v[0];
+                b[t][2 * j + 1] = (int)v[1];
+            }
+        }
+        float sx[4], sw[4][2];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            sx[t]       = *(const float*)(st + sf + t * 64);
+            const u32x2 v = *(const u32x2*)(st + kFp8TileX + (wc * 4 + t) * kP8Unit + 4096);
+            sw[t][0] = bit_cast<float>(v[0]), sw[t][1] = bit_cast<float>(v[1]);
+        }
+        floatx4 tt[2][4];
+        auto    scale = [&](int i, int t) {  // the results of column tile i, row tile t join the sums
+            const float se = sx[t] * sw[i >> 1][0], so = sx[t] * sw[i >> 1][1];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                acc[i >> 1][i & 1][t][r] = __builtin_fmaf(tt[i & 1][t][r], (r & 1) ? so : se, acc[i >> 1][i & 1][t][r]);
+            }
+        };
+        // A product of column tile i, the scaling of one of tile i - 1 under it, in turn: 32 cycles of the matrix core, 24 of the vector unit; the next tile's
+        // operand and, first, the pieces of the next k-block with them
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            if (i < 7) {
+                read_a(i + 1);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {  // (formats 0: e4m3; both scales 0: the form without scales)
+                tt[i & 1][t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a[i & 1], b[t], floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0, 0, 0, 0);
+                if (i > 0) {
+                    scale(i - 1, t);
+                }
+                if (4 * i + t < 10) {
+                    fetch(nxt, nbuf, 4 * i + t);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            scale(7, t);
+        }
+    }
+    // A lane's results are four columns each of its rows; through the wave's own LDS they leave as whole runs of a row
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // every wave is through with the stages
+    asm volatile("" ::: "memory");
+    char* const out   = smem + wave * kFp8TileOut;
+    const bool  gated = p.epilogue == 1;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const floatx4 a   = acc[u][h][t];
+                char* const   row = out + (t * 16 + c) * 288;
+                if (gated) {
+                    const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
+                    const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+                    *(half2_t*)(row + u * 32 + h * 16 + q * 4) = half2_t{(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
+                }
+                else {
+                    *(half4_t*)(row + u * 64 + h * 32 + q * 8) = half4_t{(half_t)a[0], (half_t)a[1], (half_t)a[2], (half_t)a[3]};
+                }
+            }
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+    const int n0 = (tl.ct * 256 + wc * 128) >> (gated ? 1 : 0), N = p.N >> (gated ? 1 : 0), run = gated ? 8 : 16;  // 16-byte runs of a row
+    const int rr = gated ? lane >> 3 : lane >> 4, rc = lane & (run - 1), n = n0 + rc * 8;
+#pragma unroll 4
+    for (int r = rr; r < 64; r += 64 / run) {
+        const int m = wr * 64 + r;
+        if (m < tl.Mloc && n < N) {
+            *(half8_t*)(p.y + (size_t)(tl.row0 + tl.m0 + m) * p.ldy + n) = *(const half8_t*)(out + r * 288 + rc * 16);
+        }
+    }
+}
+
 template<int MH, int CG, int WK, bool GRP>
 static int launch_fp8_one(const Fp8Params& p, dim3 grid, hipStream_t st)
 {
@@ -542,11 +749,23 @@ int launch_linear_fp8_grouped(const LinearWeight& proto, const void* d_groups, i
     // Rows of a tile, by the expected rows of an expert: a weight unit costs a workgroup the same for 128 rows as for 32, but rows that are not there cost as
     // much as those that are.  Mixtral-sized experts (4096 x 14336, 8, top 2), us a layer with 32 / 64 / 128 rows: 16 expected 259 / 302 / 427, 48: 398 / 326
     // / 428, 64: 469 / 478 / 430, 100: 612 / 522 / 447, 128: 735 / 641 / 697, 256: 1304 / 1088 / 1013, 1024: 4915 / 3857 / 3264 (0.88 PFLOP/s; 64 rows with
-    // the row blocks of a column tile far apart: 4868)
-    const int rows = measured ? tv[0] : want <= 32 ? 32 : m_hint < 56 ? 64 : 128;
+    // the row blocks of a column tile far apart: 4868).  128 / 256 rows (the kernel of 256 x 256 tiles): 80 expected 489 / 544, 100: 452 / 499, 110: 561 / 489, 160: 773 / 506,
+    // 1000: 3104 / 1765; 32 experts of 4096 x 1536: 80: 283 / 293, 150: 509 / 351
+    const bool wide = ldy % 8 == 0 && (uintptr_t)y % 16 == 0;  // (rows leave in 16-byte runs)
+    int        rows = measured ? tv[0] : want <= 32 ? 32 : m_hint < 56 ? 64 : m_hint < 105 ? 128 : 256;
+    rows            = rows == 256 && !wide ? 128 : rows;
     p.experts      = E;
     p.ct8          = ((p.ncg + 3) / 4 + 7) / 8;
     p.one_block    = m_cap <= rows;
+    if (rows == 256) {
+        p.ct8 = ((p.ncg + 7) / 8 + 7) / 8;
+        if (const int rc = ensure_dynamic_lds((const void*)gemm_fp8_tile256_kernel, kFp8TileLds)) {
+            return rc;
+        }
+        gemm_fp8_tile256_kernel<<<p.ct8 * 8 * (p.one_block ? E : std::min(E * ((m_cap + rows - 1) / rows), total_rows / rows + E)), 512, kFp8TileLds, st>>>(p);
+        TM_HIP_CHECK(hipGetLastError());
+        return 0;
+    }
     const dim3 grid(p.ct8 * 8 * (p.one_block ? E : std::min(E * ((m_cap + rows - 1) / rows), total_rows / rows + E)));
     return rows == 32 ? launch_fp8_one<1, 4, 4, true>(p, grid, st) :
            rows == 64 ? launch_fp8_one<2, 4, 2, true>(p, grid, st) : launch_fp8_one<4, 4, 2, true>(p, grid, st);
