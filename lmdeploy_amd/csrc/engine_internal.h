@@ -152,7 +152,7 @@ struct LayeredModel {
     int                  ldproj = 0, ldq = 0, ldplain = 0, ldlat = 0, ldff = 0, ld2w = 0, max_top = 0;
     int                  max_logit_rows = 0;
     float*               d_res = nullptr;       // residual stream [max_tokens][width]
-    void *               d_h1 = nullptr, *d_h2 = nullptr, *d_qkv = nullptr, *d_cat = nullptr, *d_hn = nullptr;
+    void *               d_h1 = nullptr, *d_hh = nullptr, *d_qkv = nullptr, *d_cat = nullptr, *d_hn = nullptr;
     // wide blocks: fused projection (fp32), queries, unrotated query parts, latent attention output, activations
     float *              d_proj = nullptr, *d_x0 = nullptr, *d_moe_y = nullptr, *d_topk_w = nullptr;
     void *               d_q = nullptr, *d_plain = nullptr, *d_lat = nullptr, *d_ff = nullptr, *d_xx = nullptr, *d_moe_x = nullptr;

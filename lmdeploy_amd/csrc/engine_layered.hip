@@ -153,6 +153,12 @@ static int to_f32(tm_engine* e, const std::string& name, size_t n, float** out)
     return 0;
 }
 
+// first up column of a parallel block's fused [q | k | v | up] image
+static int plain_up_col(const LmLayer& L)
+{
+    return (L.n_q + L.n_k + L.n_v + 255) / 256 * 256;
+}
+
 static int place(tm_engine* e, DenseWeight& d, int row0, int col0, const std::string& name, int rows, int cols, size_t src_row = 0, int item = 0,
                  bool transpose = false, int half = 0)
 {
@@ -695,7 +701,8 @@ int layered_process_weights(tm_engine* e)
             TM_TRY(process_wide_layer(e, i, L, dt));
             continue;
         }
-        TM_TRY(dense_weight_alloc(L.qkv, W, L.n_q + L.n_k + L.n_v, dt, e->stream));
+        // [q | k | v | up] along N, the up rows from the first multiple of 256 on (whole tiles of every product kernel): one launch projects both sublayers, each from its own norm
+        TM_TRY(dense_weight_alloc(L.qkv, W, s.mlp ? plain_up_col(L) + s.ff : L.n_q + L.n_k + L.n_v, dt, e->stream));
         TM_TRY(place(e, L.qkv, 0, 0, lname(i, "mix.q"), L.n_q, W));
         TM_TRY(place(e, L.qkv, L.n_q, 0, lname(i, "mix.k"), L.n_k, W));
         TM_TRY(place(e, L.qkv, L.n_q + L.n_k, 0, lname(i, "mix.v"), L.n_v, W));
@@ -707,8 +714,7 @@ int layered_process_weights(tm_engine* e)
             TM_TRY(to_f32(e, lname(i, "mix.sink"), s.heads, &L.sink));
         }
         if (s.mlp) {
-            TM_TRY(dense_weight_alloc(L.up, W, s.ff, dt, e->stream));
-            TM_TRY(place(e, L.up, 0, 0, lname(i, "mlp.up"), s.ff, W));
+            TM_TRY(place(e, L.qkv, plain_up_col(L), 0, lname(i, "mlp.up"), s.ff, W));
             TM_TRY(place(e, L.out, 0, L.n_att, lname(i, "mlp.down"), W, s.ff));
             TM_TRY(to_f32(e, lname(i, "norm2"), W, &L.norm2));
         }
@@ -867,6 +873,7 @@ int layered_start(tm_engine* e)
     // cache block: every layer run has its keys [kv_heads][block_len][dim] and, behind them, its values transposed [kv_heads][vdim][block_len]
     lm.ldw      = (m.width + 31) / 32 * 32;
     int64_t off = 0;
+    bool    any_pair = false;
     int     max_qkv = 8, max_cat = 32, max_vdim = 0, max_heads = 0;
     int     max_proj = 0, max_q = 0, max_plain = 0, max_lat = 0, max_ff = 0;
     bool    any_moe = false;
@@ -946,8 +953,9 @@ int layered_start(tm_engine* e)
             continue;
         }
         if (!L.wide) {
-            max_qkv = std::max(max_qkv, L.qkv.N);
-            max_cat = std::max(max_cat, L.out.Kp);
+            max_qkv  = std::max(max_qkv, L.n_q + L.n_k + L.n_v);
+            max_cat  = std::max(max_cat, L.out.Kp);
+            any_pair = any_pair || L.spec.mlp;
             continue;
         }
         max_cat   = std::max(max_cat, L.wo.Kp);
@@ -1068,7 +1076,9 @@ int layered_start(tm_engine* e)
     lm.head.scratch = lm.loop_in.scratch = &lm.scratch;
     TM_TRY(lm_alloc(&lm.d_res, T * m.width, st));
     TM_TRY(lm_alloc((char**)&lm.d_h1, T * lm.ldw * lm.elem, st));
-    TM_TRY(lm_alloc((char**)&lm.d_h2, T * lm.ldw * lm.elem, st));
+    if (any_pair) {  // both norms of a parallel block, side by side
+        TM_TRY(lm_alloc((char**)&lm.d_hh, T * 2 * lm.ldw * lm.elem, st));
+    }
     TM_TRY(lm_alloc((char**)&lm.d_qkv, T * lm.ldqkv * lm.elem, st));
     TM_TRY(lm_alloc((char**)&lm.d_cat, T * lm.ldcat * lm.elem, st));
     TM_TRY(lm_alloc((char**)&lm.d_hn, (size_t)lm.max_logit_rows * lm.ldw * lm.elem, st));
@@ -1171,7 +1181,7 @@ void layered_free(tm_engine* e)
             (void)hipFree(p);
         }
     }
-    for (void* p : {(void*)lm.embed, (void*)lm.final_norm, (void*)lm.d_res, lm.d_h1, lm.d_h2, lm.d_qkv, lm.d_cat, lm.d_hn, (void*)lm.d_logits_f32,
+    for (void* p : {(void*)lm.embed, (void*)lm.final_norm, (void*)lm.d_res, lm.d_h1, lm.d_hh, lm.d_qkv, lm.d_cat, lm.d_hn, (void*)lm.d_logits_f32,
                     (void*)lm.d_row_seq, (void*)lm.d_row_pos, (void*)lm.d_iota, (void*)lm.d_want, (void*)lm.d_seq_slot, (void*)lm.d_step_ids,
                     (void*)lm.d_step_cu_q, (void*)lm.d_step_k_len, (void*)lm.d_attn_ws, (void*)lm.d_attn_tickets, (void*)lm.scratch.slabs, (void*)lm.scratch.tickets}) {
         if (p) {
@@ -1912,13 +1922,39 @@ static int layered_layers(tm_engine* e, const int* d_ids, int M, const LmPart* p
             TM_TRY(wide_layer(e, L, M, parts, nparts));
             continue;
         }
-        TM_PROF(P_RES_NORM, TM_TRY(launch_rmsnorm_f32(lm.d_h1, s.mlp ? lm.d_h2 : nullptr, lm.ldw, lm.elem, lm.d_res, nullptr, L.norm1, L.norm2,
-                                                      m.norm_offset, m.norm_eps, M, m.width, st)));
-        TM_PROF(P_GEMM_QKV, TM_TRY(launch_dense_linear(L.qkv, lm.d_h1, lm.ldw, lm.d_qkv, lm.ldqkv, M, kDenseStore, 1.f, st)));
+        // Both sublayers read the stream at once: their norms in one launch and their first products in another, [q | k | v] and relu(up)^2.  Apart, 32
+        // rows of 4096 -> 6144 and 21504 columns took 16.6 and 30.5 us, and the store of the keys and values, which few decode rows' product leaves in the cache
+        // itself, 4.7 us; together 45.4.
+        const bool sink = nparts == 1 && parts[0].decode && M <= kDenseSinkRows && s.mlp;
+        if (s.mlp) {
+            DenseCall c;
+            c.epi          = kDenseStoreRelu2;
+            c.first_n      = L.n_q + L.n_k + L.n_v;
+            c.split_n      = plain_up_col(L);
+            c.y2           = (char*)lm.d_cat + (size_t)L.n_att * lm.elem;
+            c.ldy2         = lm.ldcat;
+            c.n_seg        = 2;
+            c.seg_n0[1]    = c.split_n;
+            c.x_col_stride = lm.ldw;
+            if (sink) {
+                const GeneralAttnParams p = attn_params(e, L, parts[0]);
+                c.kv = DenseKvSink{p.row_seq, p.row_pos, p.seq_slot, p.block_ptrs, p.block_stride, p.block_len, p.dim, p.vdim, L.n_q, L.n_q + L.n_k, p.layer_offset, p.v_offset};
+            }
+            TM_PROF(P_RES_NORM, TM_TRY(launch_rmsnorm_f32(lm.d_hh, (char*)lm.d_hh + (size_t)lm.ldw * lm.elem, 2 * lm.ldw, lm.elem, lm.d_res, nullptr, L.norm1, L.norm2,
+                                                          m.norm_offset, m.norm_eps, M, m.width, st)));
+            TM_PROF(P_GEMM_QKV, TM_TRY(launch_dense_call(L.qkv, lm.d_hh, 2 * lm.ldw, lm.d_qkv, lm.ldqkv, M, c, st)));
+        }
+        else {
+            TM_PROF(P_RES_NORM, TM_TRY(launch_rmsnorm_f32(lm.d_h1, nullptr, lm.ldw, lm.elem, lm.d_res, nullptr, L.norm1, nullptr, m.norm_offset, m.norm_eps, M,
+                                                          m.width, st)));
+            TM_PROF(P_GEMM_QKV, TM_TRY(launch_dense_linear(L.qkv, lm.d_h1, lm.ldw, lm.d_qkv, lm.ldqkv, M, kDenseStore, 1.f, st)));
+        }
         for (int i = 0; i < nparts; ++i) {
             const LmPart&     P = parts[i];
             GeneralAttnParams p = attn_params(e, L, P);
-            TM_PROF(P_KV_STORE, TM_TRY(launch_kv_store_general(p.q, lm.ldqkv, L.n_q, L.n_q + L.n_k, p, st)));
+            if (!sink) {
+                TM_PROF(P_KV_STORE, TM_TRY(launch_kv_store_general(p.q, lm.ldqkv, L.n_q, L.n_q + L.n_k, p, st)));
+            }
             if (P.decode && lm.decode_splits > 1
                 && general_attention_workspace_bytes(P.rows, s.heads, s.vdim, lm.decode_splits) <= lm.attn_ws_bytes) {
                 p.splits     = lm.decode_splits;
@@ -1927,10 +1963,6 @@ static int layered_layers(tm_engine* e, const int* d_ids, int M, const LmPart* p
                 p.tickets    = lm.d_attn_tickets, p.ticket_count = lm.n_attn_tickets;
             }
             TM_PROF(P_ATTN, TM_TRY(launch_general_attention(p, !P.decode, st)));
-        }
-        if (s.mlp) {
-            TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_dense_linear(L.up, lm.d_h2, lm.ldw, (char*)lm.d_cat + (size_t)L.n_att * lm.elem, lm.ldcat, M,
-                                                               kDenseRelu2, 1.f, st)));
         }
         TM_PROF(P_GEMM_O, TM_TRY(launch_dense_linear(L.out, lm.d_cat, lm.ldcat, lm.d_res, m.width, M, kDenseResidAdd, m.residual_mult, st)));
     }

@@ -156,6 +156,49 @@ struct DenseEpi {
         if (left <= 0) {
             return;
         }
+        if (epi == kDenseStoreRelu2) {
+            float r[4];
+            if (n >= c.split_n) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float z = fmaxf(acc[e], 0.f);
+                    r[e]          = z * z;
+                }
+                store_run<T, 4>((T*)c.y2, (size_t)m * c.ldy2 + n - c.split_n, r, vec, left);
+                return;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                r[e] = acc[e];
+            }
+            if (EPI >= 0 || !c.kv.block_ptrs || n + 4 <= c.kv.k_col) {
+                if (n < c.first_n) {
+                    store_run<T, 4>((T*)a.y, (size_t)m * a.ldy + n, r, vec, c.first_n - n);
+                }
+                return;
+            }
+            const int s = c.kv.row_seq[m], pos = c.kv.row_pos[m], ti = pos % c.kv.block_len;
+            char* const base = (char*)c.kv.block_ptrs[(size_t)(c.kv.seq_slot ? c.kv.seq_slot[s] : s) * c.kv.block_stride + pos / c.kv.block_len] + c.kv.layer_offset;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int col = n + e;
+                if (col >= c.first_n) {
+                    break;
+                }
+                if (col < c.kv.k_col) {
+                    ((T*)a.y)[(size_t)m * a.ldy + col] = (T)r[e];
+                }
+                else if (col < c.kv.v_col) {
+                    const int g = (col - c.kv.k_col) / c.kv.dim, d = (col - c.kv.k_col) % c.kv.dim;
+                    ((T*)base)[((size_t)g * c.kv.block_len + ti) * c.kv.dim + d] = (T)r[e];
+                }
+                else {
+                    const int g = (col - c.kv.v_col) / c.kv.vdim, d = (col - c.kv.v_col) % c.kv.vdim;
+                    ((T*)(base + c.kv.v_offset))[((size_t)g * c.kv.vdim + d) * c.kv.block_len + ti] = (T)r[e];
+                }
+            }
+            return;
+        }
         const size_t i = (size_t)m * a.ldy + it.col_base + n;
         float        r[4];
         if (epi == kDenseStore || epi == kDenseRelu2 || epi == kDenseXielu || epi == kDenseActTable) {
@@ -432,6 +475,7 @@ int launch_dense_linear(const DenseWeight& d, const void* x, int ldx, void* y, i
         case kDenseGatedAct: LAUNCH(kDenseGatedAct); break;  \
         case kDenseXielu: LAUNCH(kDenseXielu); break;        \
         case kDenseActTable: LAUNCH(kDenseActTable); break;  \
+        case kDenseStoreRelu2: LAUNCH(kDenseStoreRelu2); break; \
     }
 
 template<class T, int MT, int NT, int CW, int KP>
@@ -508,6 +552,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
     }
     const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2,
                                      d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border);
+    TM_REQUIRE(p.skinny || !call.kv.block_ptrs, "dense linear: cache columns belong to products of few rows");
     if (p.skinny) {
         a.split_steps = p.split_steps;
         a.row_blocks  = p.row_blocks;
@@ -545,12 +590,18 @@ int launch_dense_call(const DenseWeight& d, const void* x, int ldx, void* y, int
 {
     const int epi = call.epi;
     TM_REQUIRE(d.w && x && y && M >= 0 && call.count >= 1 && call.count <= d.count, "dense linear: operands");
-    const int n_y = epi == kDenseGatedAct ? call.n_out : d.N;
+    const int n_y = epi == kDenseGatedAct ? call.n_out : epi == kDenseStoreRelu2 ? call.first_n : d.N;
     TM_REQUIRE(ldx >= d.Kp + (call.count - 1) * call.x_col_stride && ldy >= n_y + (call.count - 1) * call.y_col_stride, "dense linear: row lengths");
-    TM_REQUIRE(epi >= kDenseStore && epi <= kDenseActTable && (epi != kDenseXielu || call.act_par), "dense linear: epilogue");
+    TM_REQUIRE(epi >= kDenseStore && epi <= kDenseStoreRelu2 && (epi != kDenseXielu || call.act_par), "dense linear: epilogue");
     TM_REQUIRE(epi != kDenseGatedAct || (call.n_out >= 1 && dense_pair_rows(call.n_out) <= d.N), "dense linear: paired image");
     TM_REQUIRE(epi != kDenseBiasF32 || call.bias, "dense linear: bias");
-    TM_REQUIRE(!call.y2 || (epi == kDenseResidAdd && call.ldy2 >= d.N && call.count == 1), "dense linear: second output");
+    TM_REQUIRE(!call.y2 || epi == kDenseStoreRelu2 || (epi == kDenseResidAdd && call.ldy2 >= d.N && call.count == 1), "dense linear: second output");
+    TM_REQUIRE(epi != kDenseStoreRelu2 || (call.y2 && call.count == 1 && call.first_n >= 1 && call.first_n <= call.split_n && call.split_n % 4 == 0 && call.split_n < d.N
+                                           && call.ldy2 >= d.N - call.split_n),
+               "dense linear: two outputs");
+    TM_REQUIRE(!call.kv.block_ptrs || (epi == kDenseStoreRelu2 && M <= kDenseSinkRows && call.kv.row_seq && call.kv.row_pos && call.kv.dim >= 1 && call.kv.vdim >= 1
+                                       && call.kv.block_stride >= 1 && call.kv.k_col <= call.kv.v_col && call.kv.v_col <= call.first_n),
+               "dense linear: cache columns");
     TM_REQUIRE(epi != kDenseActTable || (call.table && call.ids && call.count == 1 && call.table_rows >= 1 && call.table_col >= 0
                                          && call.table_col + d.N <= call.ld_table),
                "dense linear: table");

@@ -376,6 +376,39 @@ __global__ void kv_store_general_kernel(const T* __restrict__ qkv, int ld, int k
     }
 }
 
+// The same for many rows: a workgroup takes 64 rows x 64 channels.  Keys: a lane copies 16 bytes of a row.  Values, which the cache holds channel by channel: a lane
+// is a row and stores eight channels one by one, so that the wave's rows are 128 consecutive bytes of each (element by element above, every store of a wave goes to
+// 64 lines).  8192 rows of 2 x 1024 channels: 90 -> 22 us.
+__global__ __launch_bounds__(256) void kv_store_rows_kernel(const uint16_t* __restrict__ qkv, int ld, int k_col, int v_col, int nk, int nv, GeneralAttnParams p)
+{
+    const int  nkb = (nk + 63) / 64;
+    const bool val = (int)blockIdx.y >= nkb;
+    const int  c0  = ((int)blockIdx.y - (val ? nkb : 0)) * 64, n = val ? nv : nk;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int it = threadIdx.x + i * 256, row = val ? it & 63 : it >> 3, c = c0 + (val ? it >> 6 : it & 7) * 8, t = blockIdx.x * 64 + row;
+        if (t >= p.rows || c >= n) {
+            continue;
+        }
+        const u32x4 v = *(const u32x4*)(qkv + (size_t)t * ld + (val ? v_col : k_col) + c);
+        const int   s = p.row_seq[t], pos = p.row_pos[t], ti = pos % p.block_len;
+        char* const base = (char*)p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len] + p.layer_offset;
+        if (!val) {
+            const int g = c / p.dim, d = c % p.dim;
+            *(u32x4*)((uint16_t*)base + ((size_t)g * p.block_len + ti) * p.dim + d) = v;
+        }
+        else {
+            const int g = c / p.vdim, d = c % p.vdim;
+            uint16_t* out = (uint16_t*)(base + p.v_offset) + ((size_t)g * p.vdim + d) * p.block_len + ti;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                out[(2 * e) * p.block_len]     = (uint16_t)(v[e] & 0xffff);
+                out[(2 * e + 1) * p.block_len] = (uint16_t)(v[e] >> 16);
+            }
+        }
+    }
+}
+
 int launch_kv_store_general(const void* qkv, int ld, int k_col, int v_col, const GeneralAttnParams& p, hipStream_t st)
 {
     TM_REQUIRE(qkv && p.row_seq && p.row_pos && p.block_ptrs && p.block_stride >= 1, "kv_store_general: operands");
@@ -384,7 +417,13 @@ int launch_kv_store_general(const void* qkv, int ld, int k_col, int v_col, const
     if (n == 0) {
         return 0;
     }
-    if (p.elem_bytes == 2) {
+    // (pieces of eight channels lie in one head, start at multiples of 16 bytes, and so do the cache's key rows)
+    const bool pieces = p.elem_bytes == 2 && (p.dim | p.vdim | ld | k_col | v_col) % 8 == 0 && (uintptr_t)qkv % 16 == 0 && p.layer_offset % 16 == 0;
+    if (pieces && p.rows >= 64) {
+        const int nk = kh * p.dim, nv = vh * p.vdim;
+        kv_store_rows_kernel<<<dim3((p.rows + 63) / 64, (nk + 63) / 64 + (nv + 63) / 64), 256, 0, st>>>((const uint16_t*)qkv, ld, k_col, v_col, nk, nv, p);
+    }
+    else if (p.elem_bytes == 2) {
         kv_store_general_kernel<uint16_t><<<(n + 255) / 256, 256, 0, st>>>((const uint16_t*)qkv, ld, k_col, v_col, p);
     }
     else {

@@ -376,7 +376,8 @@ enum { kDenseBf16 = 0, kDenseF32 = 1 };
 // so that both accumulators of an output element live in one thread: dense_weight_place with half = 1 / 2)
 // y = act(acc) * table[ids[m]][table_col + n] (activation type; one row of a bf16 table per output row, chosen by its token id)
 // y = xielu(acc) (activation type; act_par = {softplus(p), 1/2 + softplus(q)}: z > 0: a z^2 + z / 2, else b (e^z - 1 - z) + z / 2)
-enum { kDenseStore = 0, kDenseRelu2 = 1, kDenseResidAdd = 2, kDenseScaleF32 = 3, kDenseBiasF32 = 4, kDenseResidGate = 5, kDenseGatedAct = 6, kDenseXielu = 7, kDenseActTable = 8 };
+enum { kDenseStore = 0, kDenseRelu2 = 1, kDenseResidAdd = 2, kDenseScaleF32 = 3, kDenseBiasF32 = 4, kDenseResidGate = 5, kDenseGatedAct = 6, kDenseXielu = 7, kDenseActTable = 8,
+       kDenseStoreRelu2 = 9 };
 enum { kActRelu2 = 0, kActGeluTanh = 1, kActSilu = 2, kActXielu = 3, kActClamped = 5 };  // (= TM_ACT_*)
 __device__ __forceinline__ float act_apply(int act, float z)
 {
@@ -416,6 +417,15 @@ struct DenseWeight {
     size_t bytes = 0;
     const StreamScratch* scratch = nullptr;  // set by an engine for its own weights
 };
+// where the key and value columns of a product of few rows go instead of y: row t's entry of the paged cache in the general layout (keys [head][block_len][dim], v_offset
+// bytes on values [head][vdim][block_len]); the key columns begin at k_col, the value columns at v_col
+struct DenseKvSink {
+    const int *     row_seq = nullptr, *row_pos = nullptr, *seq_slot = nullptr;
+    const uint64_t* block_ptrs = nullptr;  // nullptr: no such columns
+    int             block_stride = 0, block_len = 64, dim = 0, vdim = 0, k_col = 0, v_col = 0;
+    int64_t         layer_offset = 0, v_offset = 0;
+};
+constexpr int kDenseSinkRows = 64;
 // one launch: the epilogue with its operands, and the items of a batched launch
 struct DenseCall {
     int          epi   = kDenseStore;
@@ -425,6 +435,8 @@ struct DenseCall {
     const float* gate_bias = nullptr;
     int          ldg   = 0;
     const float* act_par = nullptr;     // kDenseXielu: two fp32 numbers (device)
+    int          first_n = 0, split_n = 0;  // kDenseStoreRelu2: columns [0, first_n) go to y, relu(.)^2 of those from split_n on to y2 [M][ldy2]
+    DenseKvSink  kv;                    // ... and the key / value columns of the first part to the cache (at most kDenseSinkRows rows)
     void*        y2 = nullptr;          // kDenseResidAdd: the new stream element also leaves in the activation type, [M][ldy2] (nullptr: not)
     int          ldy2 = 0;
     const void*  table = nullptr;       // kDenseActTable: bf16 [table_rows][ld_table], and the token id of every row of y
