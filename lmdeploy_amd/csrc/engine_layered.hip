@@ -1924,7 +1924,7 @@ static int layered_layers(tm_engine* e, const int* d_ids, int M, const LmPart* p
         }
         // Both sublayers read the stream at once: their norms in one launch and their first products in another, [q | k | v] and relu(up)^2.  Apart, 32
         // rows of 4096 -> 6144 and 21504 columns took 16.6 and 30.5 us, and the store of the keys and values, which few decode rows' product leaves in the cache
-        // itself, 4.7 us; together 45.4.
+        // itself, 4.7 us; together 41.8.
         const bool sink = nparts == 1 && parts[0].decode && M <= kDenseSinkRows && s.mlp;
         if (s.mlp) {
             DenseCall c;
