@@ -1588,6 +1588,7 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
         c.epi         = kDenseRelu2;
         c.count       = E + (L.shared_fused ? 1 : 0);
         c.row_offsets = lm.d_offsets;
+        c.item_rows   = M;  // (the router never takes an expert of a token again)
         TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_dense_call(L.gu, lm.d_moe_x, lm.ldw, lm.d_ff, lm.ldff, rows, c, st)));
         c.epi = kDenseScaleF32;
         TM_PROF(P_GEMM_DOWN, TM_TRY(launch_dense_call(L.down, lm.d_ff, lm.ldff, lm.d_moe_y, W, rows, c, st)));

@@ -370,6 +370,8 @@ void dense_weight_free(DenseWeight& d)
 //     4096) 32 rows, one slice 95, four 36, eight 39; (4096, 6144) 32 rows, 96 columns four slices 14.8, 64 columns four 15.8, one 18.6; (2048, 2048) 8
 //     rows, narrow 5.1, four slices 6.3, one 7.9; (14336, 4096) 16 rows, narrow 27.3, four slices 21.6; fp32, 3 rows: (8448, 2048) narrow 19.9, eight slices
 //     15.3; (4096, 4096) narrow 13.8, four slices 16.2
+//   items with rows of their own: blocks of as many rows as an item has at most (the tokens of a routed mixture, not its rows in total).  Febivik width 2048, whole
+//     batches: 8 tokens 35.4 -> 35.0 ms, 16 tokens 32.5 -> 30.5 (48 rows, blocks of 64 before), 22 tokens 38.9 -> 37.5 (66 rows, tiles before), 32 the same
 //   items, pairs: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; nine items of (2048, 2816): one 21, three 31; pairs, four rows,
 //     (2048, 11264): one 17, two 23
 // us; cw: column tiles a workgroup (0: narrow kernel), ss: steps of one of sp slices
@@ -386,7 +388,7 @@ static double few_rows_cost(int steps, int cols, int rows, int elem, int cw, int
 }
 
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border,
-                       bool k_major)
+                       bool k_major, int item_rows)
 {
     struct Tile {
         int    rows, cols;
@@ -410,10 +412,11 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
             cost = c, best.tile = k;
         }
     }
-    if (own_rows ? rows > 64 : rows > 256) {  // (an item's rows are one block of the skinny kernel)
+    const int block = own_rows && item_rows > 0 ? std::min(rows, item_rows) : rows;  // rows that a workgroup may meet
+    if (own_rows ? block > 64 : rows > 256) {  // (an item's rows are one block of the skinny kernel)
         return best;
     }
-    const int mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, rb = (rows + 16 * mt - 1) / (16 * mt);
+    const int mt = block <= 16 ? 1 : block <= 32 ? 2 : 4, rb = (block + 16 * mt - 1) / (16 * mt);
     best.mt = mt, best.row_blocks = rb, best.cw = pairs ? 8 : 4, best.splits = 1, best.split_steps = (steps + 7) / 8 * 8;
     if (items == 1 && !pairs && rows <= 64) {
         // (the waves of a narrow workgroup read pieces of 4 KB that lie far apart in a k-major image: fp16 (2048, 16384) 8 rows, narrow 14.6, 64 columns 11.9,
@@ -439,7 +442,7 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
         return best;
     }
     const int    wg_cols = pairs ? 128 : 64, groups = (cols + wg_cols - 1) / wg_cols * items * rb;
-    const double step = 64.0 * (wg_cols + 0.7 * std::min(rows, 16 * mt)) / 25e3;
+    const double step = 64.0 * (wg_cols + 0.7 * std::min(block, 16 * mt)) / 25e3;
     int          sp   = groups >= (pairs ? 80 : 200) ? 1 : (256 + groups - 1) / groups;  // about one workgroup a CU
     sp          = std::max(1, std::min({sp, steps / 16, 16}));
     for (int more = sp; sp > 1 && more < 2 * sp && more <= 16; ++more) {  // slices of equal length
@@ -559,7 +562,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
         border = std::gcd(border, call.seg_n0[s]);
     }
     const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2,
-                                     d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border);
+                                     d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border, false, call.item_rows);
     TM_REQUIRE(p.skinny || !call.kv.block_ptrs, "dense linear: cache columns belong to products of few rows");
     if (p.skinny) {
         a.split_steps = p.split_steps;

@@ -792,9 +792,9 @@ struct StreamPlan {
 };
 // steps of k, image columns, rows, items (own_rows: each with rows of its own, `rows` in total), bytes of an element; pairs: a wave needs two
 // column tiles; ws_bytes / tickets: what slices of k may use (0: no slices); border: x is read elsewhere from multiples of this many columns on (a
-// multiple of 128; 0: nowhere); k_major: the image holds four steps of every column tile before the next four
+// multiple of 128; 0: nowhere); k_major: the image holds four steps of every column tile before the next four; item_rows: own_rows, the most an item has (0: rows)
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0,
-                       bool k_major = false);
+                       bool k_major = false, int item_rows = 0);
 constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
 constexpr int    kStreamTickets = 4096;
 

@@ -450,6 +450,7 @@ struct DenseCall {
     int          count = 1;             // items; item g uses image g, x column g * x_col_stride, y column g * y_col_stride ...
     int          x_col_stride = 0, y_col_stride = 0;
     const int*   row_offsets = nullptr; // ... and, when set, the rows [row_offsets[g], row_offsets[g + 1]) of x and y (device, [count + 1])
+    int          item_rows = 0;         // ... and how many of them an item has at most (0: not known)
     size_t       w_stride = 0;          // (set by the launcher)
     int          ldx = 0;               // (set by the launcher)
 };
