@@ -388,7 +388,7 @@ static double few_rows_cost(int steps, int cols, int rows, int elem, int cw, int
 }
 
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border,
-                       bool k_major, int item_rows)
+                       bool k_major, int item_rows, bool cut_ok)
 {
     struct Tile {
         int    rows, cols;
@@ -398,18 +398,39 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
                                   {64, 64, 0.125, 0.15, 0.24, 0.32, 1.0}};
     StreamPlan        best{};
     double            cost = 1e30;
+    auto rounds = [&](int k, int n_cols) {  // of tiles of shape k over n_cols columns, 256 tiles a round
+        const Tile&   t  = kTiles[k];
+        const int64_t rt = own_rows ? rows / t.rows + items : (int64_t)((rows + t.rows - 1) / t.rows) * items;
+        return (rt * ((n_cols + t.cols - 1) / t.cols) + 255) / 256;
+    };
+    auto tile_cost = [&](int k, int n_cols) {
+        const Tile&  t     = kTiles[k];
+        const double full  = elem == 4 ? t.full32 : t.full16, alone = elem == 4 ? t.alone32 : t.alone16;
+        const double fixed = k == 0 && pairs ? 22.0 : t.fixed;  // (an activation per output, and no other workgroup on the CU meanwhile)
+        return border % t.cols ? 1e30 : std::max(rounds(k, n_cols) * (full * steps + fixed), alone * steps + fixed);  // (a workgroup reads x at one place)
+    };
     for (int k = 0; k < 4; ++k) {
-        const Tile&   t     = kTiles[k];
-        if (border % t.cols) {  // a workgroup reads x at one place
-            continue;
-        }
-        const int64_t rt    = own_rows ? rows / t.rows + items : (int64_t)((rows + t.rows - 1) / t.rows) * items;
-        const int64_t n     = (rt * ((cols + t.cols - 1) / t.cols) + 255) / 256;
-        const double  full  = elem == 4 ? t.full32 : t.full16, alone = elem == 4 ? t.alone32 : t.alone16;
-        const double  fixed = k == 0 && pairs ? 22.0 : t.fixed;  // (an activation per output, and no other workgroup on the CU meanwhile)
-        const double  c     = std::max(n * (full * steps + fixed), alone * steps + fixed);
-        if (c < cost) {
+        if (const double c = tile_cost(k, cols); c < cost) {
             cost = c, best.tile = k;
+        }
+    }
+    // A last round that few tiles are left for: whole rounds of 256 x 256 tiles, and the columns behind them in smaller tiles of a launch of their own, if the
+    // model above sees 1 % in it after 4 us for the launch.  us, one launch / two: fp16 (14336, 4096) 4100 rows 591 / 449, (2048, 8448) 2040 rows 96 / 75, 8010 rows 283 /
+    // 262, (5120, 27648) gated 1030 rows 399 / 335, (4096, 6144) 5888 rows 303 / 262, least of 17 sizes (5120, 27648) 8010 rows 1873 / 1879; bf16 (4096, 27648) 8192
+    // rows 1469 / 1458
+    if (cut_ok && items == 1 && !own_rows && elem == 2 && border % 256 == 0) {
+        const int rt = (rows + 255) / 256;
+        for (int64_t full = rounds(0, cols) - 1; full >= 1 && full >= rounds(0, cols) - 2; --full) {
+            const int cut = (int)(full * 256 / rt) * 256;
+            if (cut <= 0 || cut >= cols) {
+                continue;
+            }
+            for (int k = 1; k < 4; ++k) {
+                const double c = tile_cost(0, cut) + tile_cost(k, cols - cut) + 4.0;
+                if (c < 0.99 * cost) {
+                    cost = c, best.tile = 0, best.cut = cut, best.tile2 = k;
+                }
+            }
         }
     }
     const int block = own_rows && item_rows > 0 ? std::min(rows, item_rows) : rows;  // rows that a workgroup may meet
@@ -513,7 +534,7 @@ static int launch_dense_narrow(const StreamArgs& a, const DenseCall& call, int v
 
 static dim3 stream_tile_grid(const StreamArgs& a, int bm, int bn, const DenseCall& call)
 {
-    const unsigned tns = (a.tiles * 16 + bn - 1) / bn;
+    const unsigned tns = ((a.col1 ? a.col1 : a.tiles * 16) - a.col0 + bn - 1) / bn;
     return call.row_offsets ? dim3((a.M / bm + call.count) * tns) : dim3((a.M + bm - 1) / bm * tns, call.count);
 }
 
@@ -544,6 +565,24 @@ static int launch_dense_tile256(const StreamArgs& a, const DenseCall& call, int 
 }
 
 template<class T>
+static int launch_dense_tiles(const StreamArgs& a, const DenseCall& call, int tile, int vec, hipStream_t st)
+{
+    const int epi = call.epi;
+#define TM_TILE(EPI_)                                                                    \
+    if constexpr (sizeof(T) == 2 && EPI_ != kDenseActTable) {                            \
+        if (tile == 0) {                                                                 \
+            return launch_dense_tile256<T, EPI_>(a, call, vec, st);                      \
+        }                                                                                \
+    }                                                                                    \
+    return tile <= 1 ? launch_dense_tile<T, EPI_, 256, 128, 2, 2>(a, call, vec, st) :    \
+           tile == 2 ? launch_dense_tile<T, EPI_, 128, 128, 2, 2>(a, call, vec, st) :    \
+                       launch_dense_tile<T, EPI_, 64, 64, 2, 2>(a, call, vec, st)
+    TM_EPI_SWITCH(TM_TILE)
+#undef TM_TILE
+    return 0;
+}
+
+template<class T>
 static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void* y, int ldy, int M, const DenseCall& call, hipStream_t st)
 {
     const int  epi = call.epi, G = call.count;
@@ -562,7 +601,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
         border = std::gcd(border, call.seg_n0[s]);
     }
     const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2,
-                                     d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border, false, call.item_rows);
+                                     d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border, false, call.item_rows, true);
     TM_REQUIRE(p.skinny || !call.kv.block_ptrs, "dense linear: cache columns belong to products of few rows");
     if (p.skinny) {
         a.split_steps = p.split_steps;
@@ -583,18 +622,16 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
         }
 #undef TM_SKINNY
     }
-#define TM_TILE(EPI_)                                                                    \
-    if constexpr (sizeof(T) == 2 && EPI_ != kDenseActTable) {                            \
-        if (p.tile == 0) {                                                               \
-            return launch_dense_tile256<T, EPI_>(a, call, vec, st);                      \
-        }                                                                                \
-    }                                                                                    \
-    return p.tile <= 1 ? launch_dense_tile<T, EPI_, 256, 128, 2, 2>(a, call, vec, st) :  \
-           p.tile == 2 ? launch_dense_tile<T, EPI_, 128, 128, 2, 2>(a, call, vec, st) :  \
-                         launch_dense_tile<T, EPI_, 64, 64, 2, 2>(a, call, vec, st)
-    TM_EPI_SWITCH(TM_TILE)
-#undef TM_TILE
-    return 0;
+    if (p.cut > 0) {
+        StreamArgs rest = a;
+        rest.col0       = p.cut;
+        a.col1          = p.cut;
+        if (const int rc = launch_dense_tiles<T>(a, call, p.tile, vec, st)) {
+            return rc;
+        }
+        return launch_dense_tiles<T>(rest, call, p.tile2, vec, st);
+    }
+    return launch_dense_tiles<T>(a, call, p.tile, vec, st);
 }
 
 int launch_dense_call(const DenseWeight& d, const void* x, int ldx, void* y, int ldy, int M, DenseCall call, hipStream_t st)

@@ -122,9 +122,17 @@ static int launch_tiles(K kernel, const StreamArgs& a, const F16Epi& epi, int bm
     if (const int rc = ensure_dynamic_lds((const void*)kernel, lds)) {
         return rc;
     }
-    kernel<<<dim3((unsigned)((a.M + bm - 1) / bm) * (unsigned)((a.tiles * 16 + bn - 1) / bn)), 256, lds, st>>>(a, epi);
+    kernel<<<dim3((unsigned)((a.M + bm - 1) / bm) * (unsigned)(((a.col1 ? a.col1 : a.tiles * 16) - a.col0 + bn - 1) / bn)), 256, lds, st>>>(a, epi);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
+}
+
+static int launch_tile_shape(const StreamArgs& a, const F16Epi& epi, int tile, hipStream_t st)
+{
+    return tile == 0 ? launch_tiles(stream_tile256_kernel<half_t, F16Epi>, a, epi, 256, 256, st) :
+           tile == 1 ? launch_tiles(stream_tile_kernel<half_t, F16Epi, 256, 128, 2, 2>, a, epi, 256, 128, st) :
+           tile == 2 ? launch_tiles(stream_tile_kernel<half_t, F16Epi, 128, 128, 2, 2>, a, epi, 128, 128, st) :
+                       launch_tiles(stream_tile_kernel<half_t, F16Epi, 64, 64, 2, 2>, a, epi, 64, 64, st);
 }
 
 // splits: slices of k the caller's workspace holds slabs for (1: none).  With slices, fp32 slabs [slices][M][N] are left in the workspace and *slabs says
@@ -134,7 +142,7 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
 {
     TM_REQUIRE(f16_stream_supported(w, M), "fp16 linear: image");
     const bool       slice = splits > 1 && workspace;
-    const StreamPlan p     = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, slice ? ~(size_t)0 : 0, slice ? 1 << 30 : 0, 0, true);
+    const StreamPlan p     = stream_plan(w.K / 32, w.N, M, 1, false, 2, false, slice ? ~(size_t)0 : 0, slice ? 1 << 30 : 0, 0, true, 0, true);
     StreamArgs       a{};
     a.x = (const char*)x, a.ldx = (int64_t)ldx * 2;
     a.w = (const char*)w.packed, a.tiles = w.N / 16, a.steps = w.K / 32;
@@ -153,10 +161,16 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
         }
         return p.mt == 1 ? launch_skinny<1>(a, epi, p, st) : p.mt == 2 ? launch_skinny<2>(a, epi, p, st) : launch_skinny<4>(a, epi, p, st);
     }
-    return p.tile == 0 ? launch_tiles(stream_tile256_kernel<half_t, F16Epi>, a, epi, 256, 256, st) :
-           p.tile == 1 ? launch_tiles(stream_tile_kernel<half_t, F16Epi, 256, 128, 2, 2>, a, epi, 256, 128, st) :
-           p.tile == 2 ? launch_tiles(stream_tile_kernel<half_t, F16Epi, 128, 128, 2, 2>, a, epi, 128, 128, st) :
-                         launch_tiles(stream_tile_kernel<half_t, F16Epi, 64, 64, 2, 2>, a, epi, 64, 64, st);
+    if (p.cut > 0) {
+        StreamArgs rest = a;
+        rest.col0       = p.cut;
+        a.col1          = p.cut;
+        if (const int rc = launch_tile_shape(a, epi, p.tile, st)) {
+            return rc;
+        }
+        return launch_tile_shape(rest, epi, p.tile2, st);
+    }
+    return launch_tile_shape(a, epi, p.tile, st);
 }
 
 }  // namespace tmk

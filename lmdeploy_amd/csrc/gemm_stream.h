@@ -54,6 +54,7 @@ struct StreamArgs {
     int         tiles;   // 16-column tiles the image holds
     int         steps;   // steps of k
     int         split_steps;  // skinny kernel: steps of one slice of k (grid z), a multiple of 8
+    int         col0, col1;   // tile kernels: the columns of the launch, multiples of its tile (col1 0: to the image's end)
     int         row_blocks;   // skinny kernel: blocks of 16 MT rows (grid y = item * row_blocks + block)
     void*       y;
     int         ldy, M, N;
@@ -438,7 +439,7 @@ struct StreamTile {
 template<int BM, int BN, int BAND>
 __device__ __forceinline__ StreamTile stream_tile_of(const StreamArgs& a, const int* row_offsets, int items)
 {
-    const int tms = row_offsets ? a.M / BM + items : (a.M + BM - 1) / BM, tns = (a.tiles * 16 + BN - 1) / BN, total = tms * tns;
+    const int tms = row_offsets ? a.M / BM + items : (a.M + BM - 1) / BM, tns = ((a.col1 ? a.col1 : a.tiles * 16) - a.col0 + BN - 1) / BN, total = tms * tns;
     const int i = blockIdx.x, q = total >> 3, rem = total & 7, xcd = i & 7;
     const int lin  = xcd * q + min(xcd, rem) + (i >> 3);
     const int band = lin / (BAND * tns), in = lin - band * BAND * tns, h = min(BAND, tms - band * BAND);
@@ -491,7 +492,7 @@ __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_k
     if (t.item < 0) {
         return;
     }
-    const int  m0 = t.tm * BM, n0 = t.tn * BN;
+    const int  m0 = t.tm * BM, n0 = a.col0 + t.tn * BN;
     const auto item = epi.item(t.item, a.M, n0);
     const int  Mloc = min(item.M - m0, BM);
     if (Mloc <= 0) {  // an item with fewer rows than the launch's largest
@@ -630,7 +631,7 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
     if (t.item < 0) {
         return;
     }
-    const int  m0 = t.tm * BM, n0 = t.tn * BN;
+    const int  m0 = t.tm * BM, n0 = a.col0 + t.tn * BN;
     const auto item = epi.item(t.item, a.M, n0);
     const int  Mloc = min(item.M - m0, BM);
     if (Mloc <= 0) {
@@ -789,12 +790,14 @@ struct StreamPlan {
     bool skinny, narrow;  // narrow: no slices across workgroups
     int  mt, cw, splits, split_steps, row_blocks;  // skinny kernel (cw: column tiles a workgroup)
     int  tile;                                 // 0: 256 x 256 (16-bit formats), 1: 256 x 128, 2: 128 x 128, 3: 64 x 64
+    int  cut, tile2;                           // > 0: columns [0, cut) in `tile`, the others in a launch of tile2
 };
 // steps of k, image columns, rows, items (own_rows: each with rows of its own, `rows` in total), bytes of an element; pairs: a wave needs two
 // column tiles; ws_bytes / tickets: what slices of k may use (0: no slices); border: x is read elsewhere from multiples of this many columns on (a
-// multiple of 128; 0: nowhere); k_major: the image holds four steps of every column tile before the next four; item_rows: own_rows, the most an item has (0: rows)
+// multiple of 128; 0: nowhere); k_major: the image holds four steps of every column tile before the next four; item_rows: own_rows, the most an item has (0: rows);
+// cut_ok: the columns may go to two launches
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0,
-                       bool k_major = false, int item_rows = 0);
+                       bool k_major = false, int item_rows = 0, bool cut_ok = false);
 constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
 constexpr int    kStreamTickets = 4096;
 
