@@ -1592,6 +1592,11 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
         TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_dense_call(L.gu, lm.d_moe_x, lm.ldw, lm.d_ff, lm.ldff, rows, c, st)));
         c.epi = kDenseScaleF32;
         TM_PROF(P_GEMM_DOWN, TM_TRY(launch_dense_call(L.down, lm.d_ff, lm.ldff, lm.d_moe_y, W, rows, c, st)));
+        const MoeRows mr{lm.d_moe_y, lm.d_topk_w, lm.d_en2f, k, L.shared_fused ? lm.d_moe_y + (size_t)M * k * W : nullptr};
+        if ((L.shared_fused || s.shared_ff <= 0) && layernorm_add_moe_ok(lm.d_res, lm.d_h1, lm.ldw, lm.elem, mr, L.norm2, L.norm2_b, W)) {
+            TM_PROF(P_RES_NORM, TM_TRY(launch_layernorm_add_moe_f32(lm.d_res, lm.d_h1, lm.ldw, lm.elem, mr, L.norm2, L.norm2_b, m.norm_eps, M, W, st)));
+            return 0;
+        }
         if (L.shared_fused) {
             TM_PROF(P_GEMM_DOWN, TM_TRY(launch_moe_combine_f32(lm.d_y, lm.d_moe_y, lm.d_topk_w, lm.d_en2f, nullptr, 0, nullptr, M, W, k, true, st, true,
                                                          lm.d_moe_y + (size_t)M * k * W)));

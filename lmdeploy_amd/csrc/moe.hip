@@ -384,11 +384,15 @@ int moe_prepare(MoeBlock& m, hipStream_t st)
     return 0;
 }
 
+// (rows: the sum is left to the caller, out is not written)
 // out[t] = sum_j w_j * W2_e( silu(W1_e x_t) * (W3_e x_t) ) over the top_k experts e of token t
 int moe_forward(const MoeBlock& m, half_t* out, int ldo, const half_t* x, int ldx, int tokens, void* workspace, int* topk_ids_out,
-                float* topk_w_out, hipStream_t st)
+                float* topk_w_out, hipStream_t st, MoeRows* rows)
 {
     TM_REQUIRE(m.groups13 && m.groups2, "moe: not prepared");
+    if (rows) {
+        *rows = MoeRows{};
+    }
     if (tokens == 0) {
         return 0;
     }
@@ -431,7 +435,12 @@ int moe_forward(const MoeBlock& m, half_t* out, int ldo, const half_t* x, int ld
         TM_TRY_RC(launch_linear_grouped(m.w2[0], m.groups2, m.experts, act, m.inter, (int)pairs, y2, m.hidden, tokens, hint, false, offs,
                                         nullptr, st));
     }
-    TM_TRY_RC(launch_moe_combine(out, ldo, y2, m.hidden, tw, en2f, tokens, m.hidden, m.top_k, st));
+    if (rows) {
+        *rows = MoeRows{y2, tw, en2f, m.top_k, nullptr};
+    }
+    else {
+        TM_TRY_RC(launch_moe_combine(out, ldo, y2, m.hidden, tw, en2f, tokens, m.hidden, m.top_k, st));
+    }
     if (topk_ids_out) {
         TM_HIP_CHECK(hipMemcpyAsync(topk_ids_out, ids, pairs * 4, hipMemcpyDeviceToDevice, st));
     }

@@ -102,6 +102,57 @@ int launch_embedding_rmsnorm(half_t* y, half_t* resid, const half_t* table, cons
     return 0;
 }
 
+// r += the sum of a mixture's rows (in fp32, in the order of the choices, one rounding), and its norm: 16 rows of 4096, two experts, 4.6 and 4.7 us apart, 4.6 together
+template<int NV>
+__global__ __launch_bounds__(kNormMaxThreads) void moe_rmsnorm_kernel(half_t* __restrict__ y, half_t* __restrict__ resid, MoeRows mr, const half_t* __restrict__ weight,
+                                                                      float eps, int M, int H)
+{
+    __shared__ float red[8];
+    const int        row = blockIdx.x, tid = threadIdx.x;
+    NormRowRegs<NV>  g;
+    norm_row_load<0, false, NV>(g, nullptr, resid, nullptr, weight, H, row, tid, blockDim.x);
+    float acc[NV][8] = {};
+    for (int j = 0; j < mr.k; ++j) {
+        const float   w  = mr.w[(size_t)row * mr.k + j];
+        const half_t* yr = (const half_t*)mr.y + (size_t)mr.en2f[(size_t)j * M + row] * H;
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const half8_t v = *(const half8_t*)(yr + (g.off[i] - (size_t)row * H));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                acc[i][e] = __builtin_fmaf(w, (float)v[e], acc[i][e]);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            g.hc[i][e] = (half_t)acc[i][e];
+        }
+    }
+    norm_row_finish<1, false, NV>(g, y, resid, nullptr, 0, eps, M, H, tid, blockDim.x, red);
+}
+
+int launch_moe_rmsnorm(half_t* y, half_t* resid, const MoeRows& mr, const half_t* w, float eps, int M, int H, hipStream_t st)
+{
+    TM_REQUIRE(H % 8 == 0 && H <= kNormMaxThreads * kNormMaxVec * 8, "rmsnorm: H must be a multiple of 8 and <= 8192");
+    TM_REQUIRE(mr.y && mr.w && mr.en2f && mr.k >= 1 && !mr.add, "moe rmsnorm: operands");
+    if (M == 0) {
+        return 0;
+    }
+    int threads, nv;
+    norm_geometry(H, &threads, &nv);
+    if (nv == 1) {
+        moe_rmsnorm_kernel<1><<<M, threads, 0, st>>>(y, resid, mr, w, eps, M, H);
+    }
+    else {
+        moe_rmsnorm_kernel<2><<<M, threads, 0, st>>>(y, resid, mr, w, eps, M, H);
+    }
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
 int launch_residual_rmsnorm(half_t*       y,
                             half_t*       resid,
                             const half_t* hidden,
@@ -345,10 +396,12 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(T* __restrict__ y, i
 
 // the same with everything it reads in registers ahead of the reductions (H <= 256 * NR), V floats at a time: V = 4 for multiples of four on 16-byte
 // aligned operands (8 rows of 2048 with ADD: 6.3 us a launch where weights and stream were read after the reductions, 5.2 now), V = 1 otherwise
-template<class T, bool ADD, int NR, int V>
+// MOE: the row is what a routed mixture's experts leave (and a shared expert's result), summed here as moe_combine_f32_kernel does: 8 rows of 2048, two experts, 4.6 and
+// 4.1 us apart, 4.7 together
+template<class T, bool ADD, int NR, int V, bool MOE = false>
 __global__ __launch_bounds__(256) void layernorm_f32_reg_kernel(T* __restrict__ y, int ldy, float* __restrict__ xs, const float* __restrict__ src,
                                                                 const int* __restrict__ rows, const float* __restrict__ w,
-                                                                const float* __restrict__ b, float eps, int H)
+                                                                const float* __restrict__ b, float eps, int H, MoeRows mr)
 {
     constexpr int NQ = NR / V;
     typedef float FV __attribute__((ext_vector_type(V)));
@@ -360,11 +413,39 @@ __global__ __launch_bounds__(256) void layernorm_f32_reg_kernel(T* __restrict__ 
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
         const int i = min((int)(threadIdx.x + q * 256) * V, H - V);
-        v[q]        = *(const FV*)(r + i);
+        if constexpr (MOE) {
+            v[q] = 0.f;
+        }
+        else {
+            v[q] = *(const FV*)(r + i);
+        }
         wv[q]       = *(const FV*)(w + i);
         bv[q]       = *(const FV*)(b + i);
         if constexpr (ADD) {
             xv[q] = *(const FV*)(xs + (size_t)m * H + i);
+        }
+    }
+    if constexpr (MOE) {
+        const int Tn = gridDim.x;
+        for (int j = 0; j < mr.k; j += 2) {  // two rows in flight
+            const int   j1 = min(j + 1, mr.k - 1);
+            const float w0 = mr.w[(size_t)m * mr.k + j], w1 = mr.w[(size_t)m * mr.k + j1];
+            const float *y0 = (const float*)mr.y + (size_t)mr.en2f[(size_t)j * Tn + m] * H, *y1 = (const float*)mr.y + (size_t)mr.en2f[(size_t)j1 * Tn + m] * H;
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                const int i  = min((int)(threadIdx.x + q * 256) * V, H - V);
+                const FV  v0 = *(const FV*)(y0 + i), v1 = *(const FV*)(y1 + i);
+                v[q] += w0 * v0;
+                if (j + 1 < mr.k) {
+                    v[q] += w1 * v1;
+                }
+            }
+        }
+        if (mr.add) {
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                v[q] = *(const FV*)(mr.add + (size_t)m * H + min((int)(threadIdx.x + q * 256) * V, H - V)) + v[q];
+            }
         }
     }
     float sm = 0.f;
@@ -410,21 +491,21 @@ __global__ __launch_bounds__(256) void layernorm_f32_reg_kernel(T* __restrict__ 
     }
 }
 
-template<class T, bool ADD, int V>
+template<class T, bool ADD, int V, bool MOE = false>
 static void launch_layernorm_reg(T* y, int ldy, float* xs, const float* src, const int* rows, const float* w, const float* b, float eps, int M, int H,
-                                 hipStream_t st)
+                                 hipStream_t st, const MoeRows& mr = {})
 {
     if (H <= 1024) {
-        layernorm_f32_reg_kernel<T, ADD, 4, V><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H);
+        layernorm_f32_reg_kernel<T, ADD, 4, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
     }
     else if (H <= 2048) {
-        layernorm_f32_reg_kernel<T, ADD, 8, V><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H);
+        layernorm_f32_reg_kernel<T, ADD, 8, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
     }
     else if (H <= 4096) {
-        layernorm_f32_reg_kernel<T, ADD, 16, V><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H);
+        layernorm_f32_reg_kernel<T, ADD, 16, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
     }
     else {
-        layernorm_f32_reg_kernel<T, ADD, 32, V><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H);
+        layernorm_f32_reg_kernel<T, ADD, 32, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
     }
 }
 
@@ -472,6 +553,29 @@ int launch_layernorm_add_f32(float* x, void* h, int ldh, int h_elem_bytes, const
     }
     else {
         launch_layernorm_any<float, true>((float*)h, ldh, x, r, nullptr, w, b, eps, M, H, st);
+    }
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// x += LN(the sum of a mixture's rows); false: not for these sizes (the caller sums first)
+bool layernorm_add_moe_ok(const float* x, const void* h, int ldh, int h_elem_bytes, const MoeRows& r, const float* w, const float* b, int H)
+{
+    return H <= 8192 && norm_by_four(H, ldh, h_elem_bytes, {x, (const float*)r.y, w, b, r.add}, {h});
+}
+int launch_layernorm_add_moe_f32(float* x, void* h, int ldh, int h_elem_bytes, const MoeRows& r, const float* w, const float* b, float eps, int M, int H,
+                                 hipStream_t st)
+{
+    TM_REQUIRE(x && h && r.y && r.w && r.en2f && r.k >= 1 && w && b && ldh >= H && (h_elem_bytes == 2 || h_elem_bytes == 4), "layernorm_add_moe_f32: operands");
+    TM_REQUIRE(layernorm_add_moe_ok(x, h, ldh, h_elem_bytes, r, w, b, H), "layernorm_add_moe_f32: widths of four channels on 16-byte aligned operands");
+    if (M == 0) {
+        return 0;
+    }
+    if (h_elem_bytes == 2) {
+        launch_layernorm_reg<__bf16, true, 4, true>((__bf16*)h, ldh, x, nullptr, nullptr, w, b, eps, M, H, st, r);
+    }
+    else {
+        launch_layernorm_reg<float, true, 4, true>((float*)h, ldh, x, nullptr, nullptr, w, b, eps, M, H, st, r);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;

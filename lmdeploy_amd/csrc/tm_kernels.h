@@ -54,7 +54,20 @@ struct StepCommit {
     int  max_new   = 0;
 };
 
+// what the experts of a routed mixture leave for M tokens: row en2f[j * M + t] of y is token t's j-th choice, with weight w[t * k + j]
+struct MoeRows {
+    const void*  y    = nullptr;  // fp16, or fp32 in the layer-list models: [rows][H]
+    const float* w    = nullptr;
+    const int*   en2f = nullptr;
+    int          k    = 0;
+    const float* add  = nullptr;  // a shared expert's rows, one a token, which come before the sum (fp32 models)
+};
+
 // ---- norm.hip ---------------------------------------------------------------------------
+int launch_moe_rmsnorm(half_t* y, half_t* resid, const MoeRows& mr, const half_t* w, float eps, int M, int H, hipStream_t st);
+bool layernorm_add_moe_ok(const float* x, const void* h, int ldh, int h_elem_bytes, const MoeRows& r, const float* w, const float* b, int H);
+int launch_layernorm_add_moe_f32(float* x, void* h, int ldh, int h_elem_bytes, const MoeRows& r, const float* w, const float* b, float eps, int M, int H,
+                                 hipStream_t st);
 int launch_rmsnorm(half_t* y, const half_t* x, const half_t* w, float eps, int M, int H, hipStream_t st);
 // resid = table[ids[row]] and its norm
 int launch_embedding_rmsnorm(half_t* y, half_t* resid, const half_t* table, const int* ids, int vocab, const half_t* w, float eps, int M, int H,
@@ -329,7 +342,7 @@ struct MoeBlock {
 size_t moe_workspace_bytes(const MoeBlock& m, int tokens);
 int    moe_prepare(MoeBlock& m, hipStream_t st);
 int    moe_forward(const MoeBlock& m, half_t* out, int ldo, const half_t* x, int ldx, int tokens, void* workspace, int* topk_ids_out,
-                   float* topk_w_out, hipStream_t st);
+                   float* topk_w_out, hipStream_t st, MoeRows* rows = nullptr);
 void   moe_free(MoeBlock& m);
 // mixture of experts (moe.hip, grouped GEMM in gemm_w4a16.hip)
 int moe_build_groups(void** d_groups, const LinearWeight* experts, int E, hipStream_t st);
