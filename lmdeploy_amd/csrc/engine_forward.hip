@@ -112,9 +112,12 @@ static int linear_residual_norm(tm_engine* e, LinearSlots& l, const half_t* x, i
     return reduce_residual_norm(e, M, norm_w);
 }
 
-static int linear_plain(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated)
+static int linear_plain(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, const F16KvSink* kv = nullptr,
+                        bool* kv_done = nullptr)
 {
     GemmConfig cfg = pick_config(e, l.w, M, gated);
+    cfg.kv         = kv;
+    cfg.kv_done    = kv_done;
     if (gemm_workspace_bytes(M, l.w.N, cfg.splits) > e->gemm_ws_bytes) {
         cfg.splits = 1;
     }
@@ -486,12 +489,17 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
                                                      e->d_gemm_ws, cfg.splits > 1, &qkv_slabs, st)));
         }
         else {
+            bool stored = false;
             if (!qkv_done) {
-                TM_PROF(P_GEMM_QKV, TM_TRY(linear_plain(e, L.qkv, e->d_x, e->hidden, e->d_qkv, e->qkv_n, M, false)));
+                const F16KvSink sink{e->d_k_len, e->d_rope, e->rope_max_pos, e->q_heads, cv};
+                TM_PROF(P_GEMM_QKV, TM_TRY(linear_plain(e, L.qkv, e->d_x, e->hidden, e->d_qkv, e->qkv_n, M, false,
+                                                        decode && cv.layout.bits == 16 && e->D == 128 ? &sink : nullptr, &stored)));
             }
             qkv_done = false;
-            TM_PROF(P_KV_STORE, TM_TRY(launch_kv_rope_store(qkv_p, e->q_heads, e->d_cu_q, e->d_k_len, nseq, M - nd, e->d_rope,
-                                                           e->rope_max_pos, cv, st)));
+            if (!stored) {
+                TM_PROF(P_KV_STORE, TM_TRY(launch_kv_rope_store(qkv_p, e->q_heads, e->d_cu_q, e->d_k_len, nseq, M - nd, e->d_rope,
+                                                               e->rope_max_pos, cv, st)));
+            }
         }
         if (md) {
             // decode rows: (fused prologue: RoPE + K/V quantise-store) + attention on the fp16 projection rows; they share

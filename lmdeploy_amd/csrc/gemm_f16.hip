@@ -72,6 +72,45 @@ struct F16Epi {
     }
 };
 
+// The same for a decode step's [q | k | v] product: queries and keys are rotated, keys and values go to the cache (kv_rope_store_kernel's arithmetic: the product's fp16
+// rounding first, then fp16 multiplications and additions on pairs), which a launch behind the product did.  8 sequences, 16 + 2 x 8 heads of 128, (2048, 4096): 5.4 +
+// 3.0 us, now 5.8
+struct F16EpiKv: F16Epi {
+    F16KvSink kv;
+
+    template<int NT>
+    __device__ __forceinline__ void rows(const StreamArgs& a, const F16Item&, int m, int n, const floatx4 (&acc)[NT]) const
+    {
+        const int      pos = kv.k_len[m] - 1;
+        const KvLayout L   = kv.cache.layout;
+        const int      blk = pos / L.block_len, ti = pos - blk * L.block_len;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int c = n + 16 * j, head = c >> 7, d = c & 127, kh = head - kv.q_heads;
+            if (c >= a.N) {
+                continue;
+            }
+            half4_t h = {(half_t)acc[j][0], (half_t)acc[j][1], (half_t)acc[j][2], (half_t)acc[j][3]};
+            if (kh < L.kv_heads && kv.cos_sin) {
+                const half4_t cs = *(const half4_t*)(kv.cos_sin + (size_t)min(pos, kv.max_pos - 1) * 64 + (d >> 1));
+#pragma unroll
+                for (int e = 0; e < 4; e += 2) {
+                    const half_t x0 = h[e], x1 = h[e + 1];
+                    const half_t a0 = cs[e] * x0, a1 = cs[e + 1] * x1, b0 = cs[e] * x1, b1 = cs[e + 1] * x0;
+                    h[e]     = a0 - a1;
+                    h[e + 1] = b0 + b1;
+                }
+            }
+            if (kh < 0) {
+                *(half4_t*)((half_t*)a.y + (size_t)m * a.ldy + c) = h;
+                continue;
+            }
+            char* block = (char*)kv.cache.block_ptrs[kv.cache.cu_block_nums[m] + blk] + kv.cache.layer_offset;
+            *(half4_t*)(block + (kh < L.kv_heads ? L.k_data(kh, ti) : L.v_data(kh - L.kv_heads, ti)) + d * 2) = h;
+        }
+    }
+};
+
 // Where gemm_kernel is still the better one: its workgroups of 64 rows x 128 columns take the weights straight into registers and read x half as often as 64
 // columns do, so it wins where about one round of them keeps the CUs busy.  us, gemm_kernel | here, weights from HBM:
 //   up to 64 rows, 193 ... 256 workgroups: (K, N) = (4096, 28672) gated 8 rows 35.4 | 34.7, 32 rows 35.5 | 38.5, 64 rows 40 | 44, (5120, 27648) gated 8 rows
@@ -93,23 +132,23 @@ int f16_stream_splits(const LinearWeight& w, int M)
     return p.skinny ? p.splits : 1;
 }
 
-template<int MT>
-static int launch_skinny(const StreamArgs& a, const F16Epi& epi, const StreamPlan& p, hipStream_t st)
+template<int MT, class Epi>
+static int launch_skinny(const StreamArgs& a, const Epi& epi, const StreamPlan& p, hipStream_t st)
 {
     const dim3 grid((a.tiles + p.cw - 1) / p.cw, a.row_blocks, p.splits);
     if (p.narrow) {
         if (MT <= 2 && stream_narrow_waves(a) == 16) {
-            stream_narrow_kernel<half_t, F16Epi, MT, 1, MT <= 2 ? 16 : 8><<<dim3(a.tiles, a.row_blocks), 1024, 0, st>>>(a, epi);
+            stream_narrow_kernel<half_t, Epi, MT, 1, MT <= 2 ? 16 : 8><<<dim3(a.tiles, a.row_blocks), 1024, 0, st>>>(a, epi);
         }
         else {
-            stream_narrow_kernel<half_t, F16Epi, MT, 1, 8><<<dim3(a.tiles, a.row_blocks), 512, 0, st>>>(a, epi);
+            stream_narrow_kernel<half_t, Epi, MT, 1, 8><<<dim3(a.tiles, a.row_blocks), 512, 0, st>>>(a, epi);
         }
     }
     else if (p.cw == 6) {
-        stream_skinny_kernel<half_t, F16Epi, MT, 1, 6, 1><<<grid, 384, 0, st>>>(a, epi);
+        stream_skinny_kernel<half_t, Epi, MT, 1, 6, 1><<<grid, 384, 0, st>>>(a, epi);
     }
     else {
-        stream_skinny_kernel<half_t, F16Epi, MT, 1, 4, 1><<<grid, 256, 0, st>>>(a, epi);
+        stream_skinny_kernel<half_t, Epi, MT, 1, 4, 1><<<grid, 256, 0, st>>>(a, epi);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
@@ -138,7 +177,7 @@ static int launch_tile_shape(const StreamArgs& a, const F16Epi& epi, int tile, h
 // splits: slices of k the caller's workspace holds slabs for (1: none).  With slices, fp32 slabs [slices][M][N] are left in the workspace and *slabs says
 // how many (defer, or no arrival counters), or they meet inside the launch (tickets)
 int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int splits, float* workspace,
-                      unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st)
+                      unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st, const F16KvSink* kv, bool* kv_done)
 {
     TM_REQUIRE(f16_stream_supported(w, M), "fp16 linear: image");
     const bool       slice = splits > 1 && workspace;
@@ -158,6 +197,12 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
             a.slabs   = workspace;
             a.tickets = defer || (a.tiles + p.cw - 1) / p.cw * p.row_blocks > ticket_count ? nullptr : tickets;
             *slabs    = a.tickets ? 1 : p.splits;
+        }
+        // (results that leave as slabs are rounded, rotated and stored by the launches behind this one)
+        if (kv && !gated && *slabs == 1 && ldy % 4 == 0 && (uintptr_t)y % 8 == 0) {
+            const F16EpiKv ek{epi, *kv};
+            *kv_done = true;
+            return p.mt == 1 ? launch_skinny<1>(a, ek, p, st) : p.mt == 2 ? launch_skinny<2>(a, ek, p, st) : launch_skinny<4>(a, ek, p, st);
         }
         return p.mt == 1 ? launch_skinny<1>(a, epi, p, st) : p.mt == 2 ? launch_skinny<2>(a, epi, p, st) : launch_skinny<4>(a, epi, p, st);
     }

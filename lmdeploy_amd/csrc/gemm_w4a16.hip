@@ -1192,7 +1192,7 @@ int launch_linear(const LinearWeight& w,
     TM_REQUIRE(w.packed != nullptr, "this linear holds only the decode kernels' image (prepared p32_only)");
     if (cfg.f16_stream) {
         int n = 1;
-        if (const int rc = launch_f16_stream(w, x, ldx, y, ldy, M, gated_silu, cfg.splits, workspace, cfg.tickets, cfg.ticket_count, defer_reduce, &n, st)) {
+        if (const int rc = launch_f16_stream(w, x, ldx, y, ldy, M, gated_silu, cfg.splits, workspace, cfg.tickets, cfg.ticket_count, defer_reduce, &n, st, cfg.kv, cfg.kv_done)) {
             return rc;
         }
         if (n > 1 && !defer_reduce) {

@@ -161,6 +161,13 @@ struct LinearWeight {
     // parameter of HBM next to the 0.53 the decode path streams: 14 GB for an 8 B model on a 288 GB device.
     half_t*   image16 = nullptr;
 };
+// What a decode step's [q | k | v] product (row t = sequence t's one token, heads of 128 channels, fp16 cache) needs to do launch_kv_rope_store's work on its results
+struct F16KvSink {
+    const int*     k_len;
+    const half2_t* cos_sin;  // nullptr: no rotation
+    int            max_pos, q_heads;
+    KvCacheView    cache;
+};
 struct GemmConfig {
     int nt;      // n-tiles (16 cols) per wave: 1,2,4
     int splits;  // split-K
@@ -171,6 +178,8 @@ struct GemmConfig {
     unsigned* tickets = nullptr;  // arrival counters (zero between launches) of the kShapeMerge shapes and of f16_stream: >= ceil(N / 64) * ceil(M / 32) words
     int       ticket_count = 0;   // (f16_stream: how many there are)
     bool      f16_stream = false; // the kernels of gemm_f16.hip
+    const F16KvSink* kv  = nullptr;  // a decode step's [q | k | v] product that may rotate and store its keys and values itself ...
+    bool*     kv_done    = nullptr;  // ... and whether it did
 };
 // (shape 10, once "dequantise + the vendor library's fp16 GEMM", does not exist -- no vendor GEMM on any path of this library)
 constexpr int kShapePre256     = 12;   // gemm_prefill.hip: 256 x 256 tiles, each weight dequantised once per workgroup tile (M > 64)
@@ -214,7 +223,7 @@ int launch_linear(const LinearWeight& w, const half_t* x, int ldx, half_t* y, in
 bool f16_stream_supported(const LinearWeight& w, int M);
 int  f16_stream_splits(const LinearWeight& w, int M);
 int  launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int splits, float* workspace,
-                       unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st);
+                       unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st, const F16KvSink* kv = nullptr, bool* kv_done = nullptr);
 
 // ---- gemm_decode.hip: W4A16 decode GEMM (M <= 64), 32x32x16 MFMA, 16 waves per CU ------------------------------
 size_t p32_bytes(int K, int N);
