@@ -621,13 +621,13 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
         if (L.is_moe) {
             if (!e->use_comm && !e->p2p_ready) {  // router + grouped expert FFNs; their rows meet in the residual + RMSNorm launch
                 MoeRows mr;
-                TM_PROF(P_GEMM_GATE_UP, TM_TRY(moe_forward(L.moe, nullptr, 0, e->d_x, e->hidden, M, e->d_moe_ws, nullptr, nullptr, st, &mr)));
+                TM_PROF(P_GEMM_GATE_UP, TM_TRY(moe_forward(L.moe, nullptr, 0, e->d_x, e->hidden, M, e->d_moe_ws, nullptr, nullptr, st, &mr, e->d_tickets)));
                 TM_PROF(P_RES_NORM, TM_TRY(launch_moe_rmsnorm(e->d_x, e->d_resid, mr, next_norm, m.rms_eps, M, e->hidden, st)));
                 continue;
             }
             // router + grouped expert FFNs + combine -> d_tmp, then (all-reduce +) residual + RMSNorm as for the dense FFN
             TM_PROF(P_GEMM_GATE_UP, TM_TRY(moe_forward(L.moe, e->d_tmp, e->hidden, e->d_x, e->hidden, M, e->d_moe_ws, nullptr,
-                                                       nullptr, st)));
+                                                       nullptr, st, nullptr, e->d_tickets)));
             TM_TRY(reduce_residual_norm(e, M, next_norm));
             continue;
         }

@@ -76,9 +76,10 @@ __device__ __forceinline__ int64_t stream_weight_bytes(const StreamArgs& a, int 
 // Weights run one chunk of eight steps ahead of the MFMAs in a second register buffer; all loads of a stage are unconditional (clamped).  Loads return in
 // order, so a stage's x is asked for ahead of its weights: the wait for x then leaves the weights in flight (the other way round every stage drained the
 // queue: 8 rows fp16 of (2048, 16384) 14.6 us, now 11.9 = 5.6 TB/s; bf16 of (2048, 8448) 12.0, 9.9; 3 rows fp32 of (2048, 8448) 19.9, 16.5).
-// 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 38 us = 5.5 TB/s, (4096, 21504) 39 us = 4.5 TB/s (with every wave reading x for itself, no
-// slices: 76 and 50).  The loop fetches without a branch: with one around the
-// loads the two above took 52 and 42.  Its last two stages stand behind it and fetch nothing beyond the slice: 8 rows bf16 of (8448, 2048) then took 15.1 -> 11.8.
+// 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 38 us = 5.5 TB/s, (4096, 21504) 30 us = 5.9 TB/s with 96 columns a workgroup, one for nearly every CU
+// (39 us with 64, of which some CUs get two; with every wave reading x for itself, no slices: 76 and 50).  The loop fetches without a branch: with one around the
+// loads, and 64 columns, the two took 52 and 42.  Its last two stages stand behind it and fetch nothing beyond the slice: 8 rows bf16 of (8448, 2048) then took
+// 15.1 -> 11.8.
 template<class T, class Epi, int MT, int NT, int CW, int KP>
 __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a, Epi epi)
 {

@@ -10,6 +10,7 @@
 //   route:  for every expert the tokens that selected it, in ascending token order:
 //           offsets[e] .. offsets[e+1] index the flat pair list; f2n[f] = token; en2f[j][t] = f.
 //   combine: out[t] = fp16( sum_j w[t][j] * float(y[en2f[j][t]]) ).
+#include "fp8_quant.h"
 #include "tm_common.h"
 #include "tm_kernels.h"
 
@@ -25,6 +26,7 @@ namespace tmk {
 
 constexpr int kMaxExperts = 64;
 constexpr int kMaxTopK    = 8;
+constexpr int kRouteTokens = 64, kRouteExperts = 256;  // what one workgroup's masks hold (moe_route_masks_kernel)
 
 // the largest v of a wave, the lower index on a tie (i = INT_MAX: no candidate); every lane ends up with lane 0's choice
 __device__ __forceinline__ void wave_argmax(float& v, int& i)
@@ -40,8 +42,11 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i)
 }
 
 // One 256-thread workgroup per token; Wg fp16 [H][E] (input-major like every other weight).  V experts share a pass over the token (V = 8: E a multiple of
-// eight, 16-byte loads of Wg), so the row is read E / V times and every load is independent of the last; one wave picks the experts.  Bound by that
-// chain: H = 4096, 8 experts: 24.6 us with a pass per expert and one thread picking, 8.5 us so.
+// eight, 16-byte loads of Wg), so the row is read E / V times and every load is independent of the last, sixteen rounds of them in flight; one wave picks the
+// experts.  Bound by that chain: H = 4096, 8 experts: 24.6 us with a pass per expert and one thread picking, 8.0 us with eight
+// rounds in flight, 7.0 with the tail beside it:
+// workgroups behind the tokens' quantise the rows, and of up to 64 tokens the last one's writes the routing tables.  16 tokens, fp8 experts: 8.0 + 4.7 (tables) + 4.8 us
+// (codes) -> 7.0.  More tokens keep the tables' own launch: their one workgroup walks the experts.
 template<int V>
 __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_ids,      // [T][k]
                                                        float* __restrict__ topk_w,      // [T][k]
@@ -53,10 +58,18 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_id
                                                        int E,
                                                        int k,
                                                        int norm_topk,
-                                                       float routed_scale)
+                                                       float routed_scale,
+                                                       int T,
+                                                       MoeGateTail tail)
 {
+    if ((int)blockIdx.x >= T) {
+        quant_fp8_groups(blockIdx.x - T, tail.xq, tail.sx, x, ldx, T, H, tail.ldsx);
+        return;
+    }
     typedef half_t HV __attribute__((ext_vector_type(V)));
-    __shared__ float part[4][kMaxExperts];
+    __shared__ float              part[4][kMaxExperts];
+    __shared__ unsigned long long mask[64];
+    __shared__ int                first[64];
     const int        t    = blockIdx.x;
     const int        lane = threadIdx.x & 63;
     const int        wave = threadIdx.x >> 6;
@@ -67,13 +80,23 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_id
         for (int i = 0; i < V; ++i) {
             acc[i] = 0.f;
         }
-#pragma unroll 8
-        for (int h = threadIdx.x; h < H; h += 256) {
-            const float xv = (float)xr[h];
-            const HV    wv = *(const HV*)(wg + (size_t)h * E + e);
+        for (int h0 = threadIdx.x; h0 < H; h0 += 256 * 16) {
+            half_t xv[16];
+            HV     wv[16];
 #pragma unroll
-            for (int i = 0; i < V; ++i) {
-                acc[i] = __builtin_fmaf(xv, (float)wv[i], acc[i]);
+            for (int r = 0; r < 16; ++r) {  // (the row's last channel again beyond its end)
+                const int h = min(h0 + r * 256, H - 1);
+                xv[r]       = xr[h];
+                wv[r]       = *(const HV*)(wg + (size_t)h * E + e);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const bool in = h0 + r * 256 < H;
+#pragma unroll
+                for (int i = 0; i < V; ++i) {
+                    acc[i] = in ? __builtin_fmaf((float)xv[r], (float)wv[r][i], acc[i]) : acc[i];
+                }
             }
         }
 #pragma unroll
@@ -112,8 +135,53 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_id
         denom = group_sum<64>(in ? __builtin_expf(logit - mx) : 0.f);
     }
     if (lane < k) {
-        topk_ids[(size_t)t * k + lane] = id;
-        topk_w[(size_t)t * k + lane]   = __builtin_expf(val - mx) * (1.0f / denom) * routed_scale;
+        topk_w[(size_t)t * k + lane] = __builtin_expf(val - mx) * (1.0f / denom) * routed_scale;
+        __hip_atomic_store(topk_ids + (size_t)t * k + lane, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!tail.ticket || !ticket_last_wave(tail.ticket, T)) {
+        return;
+    }
+    // The tables by one wave, as moe_route_masks_kernel builds them: at most 64 tokens and 64 experts, an expert on each lane
+    constexpr int kPairs = kRouteTokens * kMaxTopK / 64;
+    int           ids[kPairs];
+#pragma unroll
+    for (int r = 0; r < kPairs; ++r) {
+        if (r * 64 < T * k) {
+            ids[r] = __hip_atomic_load(topk_ids + min(r * 64 + lane, T * k - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    mask[lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+#pragma unroll
+    for (int r = 0; r < kPairs; ++r) {
+        if (r * 64 + lane < T * k) {
+            atomicOr(&mask[ids[r]], 1ull << ((r * 64 + lane) / k));
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    const int n = __popcll(mask[lane]);
+    int       f = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(f, d);
+        f += lane >= d ? y : 0;
+    }
+    first[lane] = f - n;
+    if (lane < E) {
+        tail.offsets[lane] = f - n;
+    }
+    if (lane == 0) {
+        tail.offsets[E] = T * k;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+#pragma unroll
+    for (int r = 0; r < kPairs; ++r) {
+        const int p = r * 64 + lane;
+        if (p < T * k) {
+            const int to = p / k, at = first[ids[r]] + __popcll(mask[ids[r]] & ((1ull << to) - 1));
+            tail.f2n[at]                               = to;
+            tail.en2f[(size_t)(p - to * k) * T + to] = at;
+        }
     }
 }
 
@@ -121,7 +189,6 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_id
 // expert's first row (a wave's scan over the experts) plus the tokens ahead of it in the mask -- no pass over the experts.  PICK: the experts are first
 // chosen here, one wave per token, as moe_topk_softmax_kernel does (expert e on lane e % 64).  A chain of latencies: 8 tokens, 8 experts, 2 a token take
 // 4.8 us, the two kernels for any size 5.7 + 9.5.
-constexpr int kRouteTokens = 64, kRouteExperts = 256;
 template<bool PICK>
 __global__ __launch_bounds__(1024) void moe_route_masks_kernel(int* __restrict__ offsets, int* __restrict__ f2n, int* __restrict__ en2f, int* topk_ids,
                                                                float* __restrict__ w, const float* __restrict__ logits, int ld, int T, int E, int k,
@@ -301,18 +368,17 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(half_t* __restrict__ o
 }
 
 int launch_moe_gate(int* topk_ids, float* topk_w, float* logits_out, const half_t* x, int ldx, const half_t* wg, int T, int H,
-                    int E, int k, bool norm_topk, float routed_scale, hipStream_t st)
+                    int E, int k, bool norm_topk, float routed_scale, hipStream_t st, const MoeGateTail& tail)
 {
     TM_REQUIRE(E >= 1 && E <= kMaxExperts && k >= 1 && k <= kMaxTopK && k <= E, "moe: 1 <= top_k <= experts <= 64, top_k <= 8");
+    TM_REQUIRE(!tail.ticket || T <= kRouteTokens, "moe gate: the tables of at most 64 tokens");
+    TM_REQUIRE(!tail.xq || (H % 128 == 0 && ldx % 8 == 0 && tail.ldsx >= T), "moe gate: fp8 rows of 128-channel groups, 16-byte aligned, ldsx >= T");
     if (T == 0) {
         return 0;
     }
-    if (E % 8 == 0 && (uintptr_t)wg % 16 == 0) {
-        moe_gate_kernel<8><<<T, 256, 0, st>>>(topk_ids, topk_w, logits_out, x, ldx, wg, H, E, k, norm_topk ? 1 : 0, routed_scale);
-    }
-    else {
-        moe_gate_kernel<1><<<T, 256, 0, st>>>(topk_ids, topk_w, logits_out, x, ldx, wg, H, E, k, norm_topk ? 1 : 0, routed_scale);
-    }
+    const int  grid = T + (tail.xq ? (T * (H / 128) + 15) / 16 : 0);
+    const auto gate = E % 8 == 0 && (uintptr_t)wg % 16 == 0 ? moe_gate_kernel<8> : moe_gate_kernel<1>;
+    gate<<<grid, 256, 0, st>>>(topk_ids, topk_w, logits_out, x, ldx, wg, H, E, k, norm_topk ? 1 : 0, routed_scale, T, tail);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }
@@ -384,10 +450,10 @@ int moe_prepare(MoeBlock& m, hipStream_t st)
     return 0;
 }
 
-// (rows: the sum is left to the caller, out is not written)
+// (rows: the sum is left to the caller, out is not written; ticket: a counter of the caller's stream, zero between launches, for one launch instead of two)
 // out[t] = sum_j w_j * W2_e( silu(W1_e x_t) * (W3_e x_t) ) over the top_k experts e of token t
 int moe_forward(const MoeBlock& m, half_t* out, int ldo, const half_t* x, int ldx, int tokens, void* workspace, int* topk_ids_out,
-                float* topk_w_out, hipStream_t st, MoeRows* rows)
+                float* topk_w_out, hipStream_t st, MoeRows* rows, unsigned* ticket)
 {
     TM_REQUIRE(m.groups13 && m.groups2, "moe: not prepared");
     if (rows) {
@@ -407,23 +473,31 @@ int moe_forward(const MoeBlock& m, half_t* out, int ldo, const half_t* x, int ld
     half_t*      act   = (half_t*)(w + o);
     o                  = (o + pairs * m.inter * 2 + 255) / 256 * 256;
     half_t*      y2    = (half_t*)(w + o);
-    TM_TRY_RC(launch_moe_gate(ids, tw, nullptr, x, ldx, m.gate, tokens, m.hidden, m.experts, m.top_k, m.norm_topk, m.routed_scale, st));
-    TM_TRY_RC(launch_moe_route(offs, f2n, en2f, ids, tokens, m.experts, m.top_k, st));
+    MoeGateTail tail;
+    if (ticket && tokens <= kRouteTokens) {
+        tail.ticket = ticket, tail.offsets = offs, tail.f2n = f2n, tail.en2f = en2f;
+    }
+    o                 = (o + pairs * m.hidden * 2 + 255) / 256 * 256;
+    uint8_t*  xq      = (uint8_t*)(w + o);
+    const int ldsx1   = (tokens + 3) / 4 * 4;
+    float*    sx1     = (float*)(xq + (size_t)tokens * m.hidden);
+    if (m.groups13_p8) {
+        TM_REQUIRE(ldx == m.hidden || tokens == 1, "moe fp8: x must be row-contiguous");
+        tail.xq = xq, tail.sx = sx1, tail.ldsx = ldsx1;
+    }
+    TM_TRY_RC(launch_moe_gate(ids, tw, nullptr, x, ldx, m.gate, tokens, m.hidden, m.experts, m.top_k, m.norm_topk, m.routed_scale, st, tail));
+    if (!tail.ticket) {
+        TM_TRY_RC(launch_moe_route(offs, f2n, en2f, ids, tokens, m.experts, m.top_k, st));
+    }
     // expert FFNs: gathered rows of x -> act (gated SiLU fused) -> y2, both grouped over the experts
     const int hint = (int)((pairs + m.experts - 1) / m.experts);  // expected rows per expert
     if (m.groups13_p8) {
         // e4m3 experts on the fp8 matrix cores (the reference's fp8 path: QuantizeSymm + fp8 GEMM, LlamaLinear.cu:67-127):
-        // x is quantised once per token, the gated-SiLU output once per (token, expert) row
-        o                  = (o + pairs * m.hidden * 2 + 255) / 256 * 256;
-        uint8_t*     xq    = (uint8_t*)(w + o);
-        const int    ldsx1 = (tokens + 3) / 4 * 4;
-        float*       sx1   = (float*)(xq + (size_t)tokens * m.hidden);
+        // x was quantised once per token beside the router, the gated-SiLU output once per (token, expert) row
         o                  = (o + fp8_act_workspace_bytes(tokens, m.hidden) + 255) / 256 * 256;
         uint8_t*     aq    = (uint8_t*)(w + o);
         const int    ldsx2 = ((int)pairs + 3) / 4 * 4;
         float*       sx2   = (float*)(aq + pairs * m.inter);
-        TM_REQUIRE(ldx == m.hidden || tokens == 1, "moe fp8: x must be row-contiguous");
-        TM_TRY_RC(launch_quant_fp8_rows(xq, sx1, x, ldx, tokens, m.hidden, ldsx1, st));
         TM_TRY_RC(launch_linear_fp8_grouped(m.w13[0], m.groups13_p8, m.experts, xq, sx1, ldsx1, tokens, act, m.inter, tokens, (int)pairs, hint, true,
                                             offs, f2n, st));
         TM_TRY_RC(launch_quant_fp8_rows(aq, sx2, act, m.inter, (int)pairs, m.inter, ldsx2, st));

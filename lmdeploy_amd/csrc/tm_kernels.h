@@ -63,6 +63,15 @@ struct MoeRows {
     const float* add  = nullptr;  // a shared expert's rows, one a token, which come before the sum (fp32 models)
 };
 
+// what the router's launch does besides, for T tokens
+struct MoeGateTail {
+    uint8_t*  xq      = nullptr;  // fp8 codes of the rows ([T][H], scales sx[g * ldsx + t]); nullptr: none
+    float*    sx      = nullptr;
+    int       ldsx    = 0;
+    unsigned* ticket  = nullptr;  // a counter, zero between launches: the last token's workgroup writes the routing tables (launch_moe_route); nullptr: nobody
+    int *     offsets = nullptr, *f2n = nullptr, *en2f = nullptr;
+};
+
 // ---- norm.hip ---------------------------------------------------------------------------
 int launch_moe_rmsnorm(half_t* y, half_t* resid, const MoeRows& mr, const half_t* w, float eps, int M, int H, hipStream_t st);
 bool layernorm_add_moe_ok(const float* x, const void* h, int ldh, int h_elem_bytes, const MoeRows& r, const float* w, const float* b, int H);
@@ -351,7 +360,7 @@ struct MoeBlock {
 size_t moe_workspace_bytes(const MoeBlock& m, int tokens);
 int    moe_prepare(MoeBlock& m, hipStream_t st);
 int    moe_forward(const MoeBlock& m, half_t* out, int ldo, const half_t* x, int ldx, int tokens, void* workspace, int* topk_ids_out,
-                   float* topk_w_out, hipStream_t st, MoeRows* rows = nullptr);
+                   float* topk_w_out, hipStream_t st, MoeRows* rows = nullptr, unsigned* ticket = nullptr);
 void   moe_free(MoeBlock& m);
 // mixture of experts (moe.hip, grouped GEMM in gemm_w4a16.hip)
 int moe_build_groups(void** d_groups, const LinearWeight* experts, int E, hipStream_t st);
@@ -359,7 +368,7 @@ int launch_linear_grouped(const LinearWeight& proto, const void* d_groups, int E
                           half_t* y, int ldy, int m_cap, int m_hint, bool gated_silu, const int* seg, const int* row_idx,
                           hipStream_t st);
 int launch_moe_gate(int* topk_ids, float* topk_w, float* logits_out, const half_t* x, int ldx, const half_t* wg, int T, int H,
-                    int E, int k, bool norm_topk, float routed_scale, hipStream_t st);
+                    int E, int k, bool norm_topk, float routed_scale, hipStream_t st, const MoeGateTail& tail = {});
 int launch_moe_route(int* offsets, int* f2n, int* en2f, const int* topk_ids, int T, int E, int k, hipStream_t st);
 int launch_moe_combine(half_t* out, int ldo, const half_t* y, int ldy, const float* topk_w, const int* en2f, int T, int H, int k,
                        hipStream_t st);
