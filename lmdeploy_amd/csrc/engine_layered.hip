@@ -1578,11 +1578,9 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
     else {
         const int k = s.top, E = s.experts;
         TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_dense_linear(L.router, lm.d_h1, lm.ldw, lm.d_proj, lm.ldproj, M, kDenseScaleF32, 1.f, st)));
-        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_softmax_route(lm.d_topk_ids, lm.d_topk_w, lm.d_offsets, lm.d_f2n, lm.d_en2f, lm.d_proj, lm.ldproj, M, E,
-                                                                k, s.router_scale, st)));
-        // the shared expert: item E of the batched products over a copy of all rows behind the routed ones
-        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_gather(lm.d_moe_x, lm.ldw, lm.d_h1, lm.ldw, lm.elem, lm.d_topk_w, lm.d_en2f, M, W, k, false, st,
-                                                         L.shared_fused ? lm.d_offsets : nullptr, E)));
+        // the rows in the experts' order; the shared expert: item E of the batched products over a copy of all rows behind the routed ones
+        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_softmax_route_gather(lm.d_topk_ids, lm.d_topk_w, lm.d_offsets, lm.d_f2n, lm.d_en2f, lm.d_proj, lm.ldproj, lm.d_moe_x,
+                                                                       lm.ldw, lm.d_h1, lm.ldw, lm.elem, M, W, E, k, s.router_scale, L.shared_fused, st)));
         const int rows = M * (k + (L.shared_fused ? 1 : 0));
         DenseCall c;
         c.epi         = kDenseRelu2;

@@ -26,7 +26,7 @@ namespace tmk {
 
 constexpr int kMaxExperts = 64;
 constexpr int kMaxTopK    = 8;
-constexpr int kRouteTokens = 64, kRouteExperts = 256;  // what one workgroup's masks hold (moe_route_masks_kernel)
+constexpr int kRouteTokens = 64, kRouteExperts = 256, kRoutePairs = 2048;  // what one workgroup's masks hold (moe_route_masks_kernel)
 
 // the largest v of a wave, the lower index on a tie (i = INT_MAX: no candidate); every lane ends up with lane 0's choice
 __device__ __forceinline__ void wave_argmax(float& v, int& i)
@@ -185,19 +185,43 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_id
     }
 }
 
+template<class X>
+struct MoeGather {  // rows of x, H channels, to xs in the experts' order; shared: and all of them behind
+    X*       xs     = nullptr;
+    int      lds    = 0;
+    const X* x      = nullptr;
+    int      ldx    = 0;
+    int      H      = 0;
+    int      shared = 0;
+};
+
 // Routing tables of up to kRouteTokens tokens and kRouteExperts experts in one workgroup: an expert's tokens are a 64-bit mask in LDS, a pair's place the
 // expert's first row (a wave's scan over the experts) plus the tokens ahead of it in the mask -- no pass over the experts.  PICK: the experts are first
 // chosen here, one wave per token, as moe_topk_softmax_kernel does (expert e on lane e % 64).  A chain of latencies: 8 tokens, 8 experts, 2 a token take
 // 4.8 us, the two kernels for any size 5.7 + 9.5.
-template<bool PICK>
+// V > 0: every workgroup makes the tables for itself, the first one writes them, and each copies four of the rows that moe_gather_kernel would (V channels a load, the
+// first of them asked for ahead of the routing).  8 tokens of 2048, three rows a token: 5.7 us, the two launches
+// 4.8 + 2.6.
+template<bool PICK, class X = __bf16, int V = 0>
 __global__ __launch_bounds__(1024) void moe_route_masks_kernel(int* __restrict__ offsets, int* __restrict__ f2n, int* __restrict__ en2f, int* topk_ids,
                                                                float* __restrict__ w, const float* __restrict__ logits, int ld, int T, int E, int k,
-                                                               float scale)
+                                                               float scale, MoeGather<X> g)
 {
     constexpr int NE = kRouteExperts / 64;
+    typedef X XV __attribute__((ext_vector_type(V ? V : 1)));
     __shared__ unsigned long long mask[kRouteExperts];
     __shared__ int                first[kRouteExperts];
+    __shared__ unsigned short     chosen[V ? kRoutePairs : 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int kk = k + g.shared, job = blockIdx.x * 4 + (tid >> 8), jt = min(job / kk, T - 1), jj = job % kk, c0 = (tid & 255) * V;
+    const X* const src = V ? g.x + (size_t)jt * g.ldx : nullptr;
+    XV             head{};
+    if constexpr (V > 0) {
+        if (c0 < g.H) {
+            head = *(const XV*)(src + c0);
+        }
+    }
+    const bool writes = blockIdx.x == 0;
     if (tid < kRouteExperts) {
         mask[tid] = 0;
     }
@@ -235,8 +259,13 @@ __global__ __launch_bounds__(1024) void moe_route_masks_kernel(int* __restrict__
                     taken[q] = taken[q] || q * 64 + lane == i;
                 }
                 if (lane == 0) {
-                    topk_ids[(size_t)t * k + j] = i;
-                    w[(size_t)t * k + j]        = scale * (expf(v - mx) / den);
+                    if (writes) {
+                        topk_ids[(size_t)t * k + j] = i;
+                        w[(size_t)t * k + j]        = scale * (expf(v - mx) / den);
+                    }
+                    if constexpr (V > 0) {
+                        chosen[t * k + j] = (unsigned short)i;
+                    }
                     atomicOr(&mask[i], 1ull << t);
                 }
             }
@@ -269,13 +298,34 @@ __global__ __launch_bounds__(1024) void moe_route_masks_kernel(int* __restrict__
         }
     }
     __syncthreads();
-    if (tid <= E) {
-        offsets[tid] = tid < E ? first[tid] : T * k;
+    if (writes) {
+        if (tid <= E) {
+            offsets[tid] = tid < E ? first[tid] : T * k;
+        }
+        if (V > 0 && tid == 0 && g.shared) {
+            offsets[E + 1] = T * kk;
+        }
+        for (int p = tid; p < T * k; p += 1024) {
+            const int t = p / k, e = V ? chosen[p] : topk_ids[p], f = first[e] + __popcll(mask[e] & ((1ull << t) - 1));
+            f2n[f]                          = t;
+            en2f[(size_t)(p - t * k) * T + t] = f;
+        }
     }
-    for (int p = tid; p < T * k; p += 1024) {
-        const int t = p / k, e = topk_ids[p], f = first[e] + __popcll(mask[e] & ((1ull << t) - 1));
-        f2n[f]                          = t;
-        en2f[(size_t)(p - t * k) * T + t] = f;
+    if constexpr (V > 0) {
+        if (job < T * kk) {
+            int f = T * k + jt;  // the copy behind the routed rows
+            if (jj < k) {
+                const int e = chosen[jt * k + jj];
+                f           = first[e] + __popcll(mask[e] & ((1ull << jt) - 1));
+            }
+            X* const dst = g.xs + (size_t)f * g.lds;
+            if (c0 < g.H) {
+                *(XV*)(dst + c0) = head;
+            }
+            for (int i = c0 + 256 * V; i < g.H; i += 256 * V) {
+                *(XV*)(dst + i) = *(const XV*)(src + i);
+            }
+        }
     }
 }
 
@@ -386,7 +436,7 @@ int launch_moe_gate(int* topk_ids, float* topk_w, float* logits_out, const half_
 int launch_moe_route(int* offsets, int* f2n, int* en2f, const int* topk_ids, int T, int E, int k, hipStream_t st)
 {
     if (T <= kRouteTokens && E <= kRouteExperts) {
-        moe_route_masks_kernel<false><<<1, 1024, 0, st>>>(offsets, f2n, en2f, (int*)topk_ids, nullptr, nullptr, 0, T, E, k, 0.f);
+        moe_route_masks_kernel<false><<<1, 1024, 0, st>>>(offsets, f2n, en2f, (int*)topk_ids, nullptr, nullptr, 0, T, E, k, 0.f, {});
     }
     else {
         moe_route_kernel<<<1, 1024, 0, st>>>(offsets, f2n, en2f, topk_ids, T, E, k);
@@ -623,7 +673,7 @@ int launch_moe_softmax_route(int* ids, float* w, int* offsets, int* f2n, int* en
         return launch_moe_route(offsets, f2n, en2f, ids, T, E, k, st);
     }
     if (T <= kRouteTokens && E <= kRouteExperts) {
-        moe_route_masks_kernel<true><<<1, 1024, 0, st>>>(offsets, f2n, en2f, ids, w, logits, ld, T, E, k, scale);
+        moe_route_masks_kernel<true><<<1, 1024, 0, st>>>(offsets, f2n, en2f, ids, w, logits, ld, T, E, k, scale, {});
         TM_HIP_CHECK(hipGetLastError());
         return 0;
     }
@@ -789,6 +839,40 @@ int launch_moe_gather(void* xs, int lds, const void* x, int ldx, int elem_bytes,
     }
     else {
         launch_moe_gather_t((float*)xs, lds, (const float*)x, ldx, w, en2f, T, H, k, scale, shared_offsets, E, st);
+    }
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+template<class T>
+static void launch_route_gather_t(int* ids, float* w, int* offsets, int* f2n, int* en2f, const float* logits, int ld, const MoeGather<T>& g, int Tn, int E, int k,
+                                  float scale, hipStream_t st)
+{
+    constexpr int V   = 16 / sizeof(T);
+    const int     wgs = (Tn * (k + g.shared) + 3) / 4;
+    if (g.H % V == 0 && g.lds % V == 0 && g.ldx % V == 0 && (uintptr_t)g.x % 16 == 0 && (uintptr_t)g.xs % 16 == 0) {
+        moe_route_masks_kernel<true, T, V><<<wgs, 1024, 0, st>>>(offsets, f2n, en2f, ids, w, logits, ld, Tn, E, k, scale, g);
+    }
+    else {
+        moe_route_masks_kernel<true, T, 1><<<wgs, 1024, 0, st>>>(offsets, f2n, en2f, ids, w, logits, ld, Tn, E, k, scale, g);
+    }
+}
+
+int launch_moe_softmax_route_gather(int* ids, float* w, int* offsets, int* f2n, int* en2f, const float* logits, int ld, void* xs, int lds, const void* x, int ldx,
+                                    int elem_bytes, int T, int H, int E, int k, float scale, bool shared, hipStream_t st)
+{
+    // (more tokens than a mask has bits, or more choices than its list: one workgroup's tables no longer cost less than a launch of their own)
+    if (T == 0 || T > kRouteTokens || E > kRouteExperts || T * k > kRoutePairs) {
+        TM_TRY_RC(launch_moe_softmax_route(ids, w, offsets, f2n, en2f, logits, ld, T, E, k, scale, st));
+        return launch_moe_gather(xs, lds, x, ldx, elem_bytes, w, en2f, T, H, k, false, st, shared ? offsets : nullptr, E);
+    }
+    TM_REQUIRE(ids && w && logits && E >= 1 && k >= 1 && k <= E && ld >= E, "moe top-k: operands");
+    TM_REQUIRE(xs && x && lds >= H && ldx >= H, "moe gather: operands");
+    if (elem_bytes == 2) {
+        launch_route_gather_t(ids, w, offsets, f2n, en2f, logits, ld, MoeGather<__bf16>{(__bf16*)xs, lds, (const __bf16*)x, ldx, H, shared ? 1 : 0}, T, E, k, scale, st);
+    }
+    else {
+        launch_route_gather_t(ids, w, offsets, f2n, en2f, logits, ld, MoeGather<float>{(float*)xs, lds, (const float*)x, ldx, H, shared ? 1 : 0}, T, E, k, scale, st);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;

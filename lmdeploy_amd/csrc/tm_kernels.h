@@ -625,6 +625,9 @@ int launch_moe_topk_grouped(int* ids, float* w, const float* logits, int ld, con
 // batched products), and shared_offsets[E + 1] = T (k + 1) is written
 int launch_moe_gather(void* xs, int lds, const void* x, int ldx, int elem_bytes, const float* w, const int* en2f, int T, int H, int k, bool scale,
                       hipStream_t st, int* shared_offsets = nullptr, int E = 0);
+// the soft-max router and the gather, in one launch where the tokens are few (shared: offsets[E + 1] too)
+int launch_moe_softmax_route_gather(int* ids, float* w, int* offsets, int* f2n, int* en2f, const float* logits, int ld, void* xs, int lds, const void* x, int ldx,
+                                    int elem_bytes, int T, int H, int E, int k, float scale, bool shared, hipStream_t st);
 int launch_moe_combine_f32(float* resid, const float* y, const float* w, const int* en2f, const float* gate, int ldg, const float* gate_bias, int T,
                            int H, int k, bool weighted, hipStream_t st, bool overwrite = false /* resid = sum instead of resid += sum */,
                            const float* add = nullptr /* overwrite: resid = add + sum ([T][H]) */,
