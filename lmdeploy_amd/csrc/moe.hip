@@ -46,7 +46,7 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i)
 // experts.  Bound by that chain: H = 4096, 8 experts: 24.6 us with a pass per expert and one thread picking, 8.0 us with eight
 // rounds in flight, 7.0 with the tail beside it:
 // workgroups behind the tokens' quantise the rows, and of up to 64 tokens the last one's writes the routing tables.  16 tokens, fp8 experts: 8.0 + 4.7 (tables) + 4.8 us
-// (codes) -> 7.0.  More tokens keep the tables' own launch: their one workgroup walks the experts.
+// (codes) -> 7.0.  More tokens keep the tables' own launch, which takes a workgroup an expert.
 template<int V>
 __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_ids,      // [T][k]
                                                        float* __restrict__ topk_w,      // [T][k]
@@ -329,63 +329,57 @@ __global__ __launch_bounds__(1024) void moe_route_masks_kernel(int* __restrict__
     }
 }
 
-// single workgroup: routing tables.  offsets [E+1], f2n [T*k], en2f [k][T]
+// Routing tables of any number of tokens: offsets [E+1], f2n [T*k], en2f [k][T].  A workgroup an expert: each reads all choices (they stay in L2), counts those of
+// lower experts, which is where its rows begin, and its own ahead of every thread's run of tokens; a second look at them writes its rows in token order.  Two
+// short passes over T k numbers instead of one workgroup's walk over the experts with barriers for each: 8 experts, 2 choices: 8000 tokens 70 -> 14 us, 4000
+// 36.7 -> 7.3.
 __global__ __launch_bounds__(1024) void moe_route_kernel(int* __restrict__ offsets, int* __restrict__ f2n, int* __restrict__ en2f,
                                                          const int* __restrict__ topk_ids, int T, int E, int k)
 {
-    __shared__ int s_scan[16];
-    __shared__ int s_base;
-    const int      tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) {
-        s_base     = 0;
-        offsets[0] = 0;
+    __shared__ int s_mine[16], s_lower[16];
+    const int      tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, e = blockIdx.x;
+    const int      run = (T + 1023) / 1024 * k;  // choices of a thread: whole tokens
+    const int      p0 = min(tid * run, T * k), p1 = min(p0 + run, T * k);
+    int            mine = 0, lower = 0;
+#pragma unroll 8
+    for (int p = p0; p < p1; ++p) {
+        const int id = topk_ids[p];
+        mine += id == e;
+        lower += (unsigned)id < (unsigned)e;
+    }
+    int x = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int y = __shfl_up(x, d);
+        x += lane >= d ? y : 0;
+        lower += __shfl_xor(lower, d);
+    }
+    if (lane == 63) {
+        s_mine[wave]  = x;
+        s_lower[wave] = lower;
     }
     __syncthreads();
-    for (int e = 0; e < E; ++e) {
-        int running = s_base;
-        for (int t0 = 0; t0 < T; t0 += 1024) {
-            const int t = t0 + tid;
-            int       j = -1;
-            if (t < T) {
-                for (int q = 0; q < k; ++q) {
-                    if (topk_ids[(size_t)t * k + q] == e) {
-                        j = q;
-                    }
-                }
-            }
-            const int flag = j >= 0;
-            int       x    = flag;
+    int f = x - mine;
 #pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int y = __shfl_up(x, d);
-                if (lane >= d) {
-                    x += y;
-                }
-            }
-            if (lane == 63) {
-                s_scan[wave] = x;
-            }
-            __syncthreads();
-            int before = 0, total = 0;
-            for (int w = 0; w < 16; ++w) {
-                if (w < wave) {
-                    before += s_scan[w];
-                }
-                total += s_scan[w];
-            }
-            if (flag) {
-                const int f             = running + before + x - 1;
-                f2n[f]                  = t;
-                en2f[(size_t)j * T + t] = f;
-            }
-            running += total;
-            __syncthreads();
+    for (int w = 0; w < 16; ++w) {
+        f += s_lower[w] + (w < wave ? s_mine[w] : 0);
+    }
+    if (tid == 0) {
+        offsets[e] = f;
+    }
+    if (tid == 1023 && e == E - 1) {
+        offsets[E] = f + mine;
+    }
+    if (mine == 0) {
+        return;
+    }
+    for (int p = p0; p < p1; ++p) {
+        if (topk_ids[p] == e) {
+            const int t                       = p / k;
+            f2n[f]                            = t;
+            en2f[(size_t)(p - t * k) * T + t] = f;
+            ++f;
         }
-        if (tid == 0) {
-            s_base         = running;
-            offsets[e + 1] = running;
-        }
-        __syncthreads();
     }
 }
 
@@ -439,7 +433,7 @@ int launch_moe_route(int* offsets, int* f2n, int* en2f, const int* topk_ids, int
         moe_route_masks_kernel<false><<<1, 1024, 0, st>>>(offsets, f2n, en2f, (int*)topk_ids, nullptr, nullptr, 0, T, E, k, 0.f, {});
     }
     else {
-        moe_route_kernel<<<1, 1024, 0, st>>>(offsets, f2n, en2f, topk_ids, T, E, k);
+        moe_route_kernel<<<E, 1024, 0, st>>>(offsets, f2n, en2f, topk_ids, T, E, k);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
