@@ -28,11 +28,27 @@ constexpr int kMaxExperts = 64;
 constexpr int kMaxTopK    = 8;
 constexpr int kRouteTokens = 64, kRouteExperts = 256, kRoutePairs = 2048;  // what one workgroup's masks hold (moe_route_masks_kernel)
 
-// the largest v of a wave, the lower index on a tie (i = INT_MAX: no candidate); every lane ends up with lane 0's choice
+// the largest v of a wave, the lower index on a tie (i = INT_MAX: no candidate, else i % 64 is the lane); every lane ends up with the choice
 __device__ __forceinline__ void wave_argmax(float& v, int& i)
 {
+    const bool in = i != 0x7fffffff;
+    if (__ballot(in && !(v == v)) == 0) {
+        // the maximum over DPP, then who has it: the twelve shuffles through LDS, one behind the other, cost 0.2 - 0.3 us a choice more
+        const float              mx  = group_max<64>(in ? v : -INFINITY);
+        const bool               has = in && v == mx;
+        const unsigned long long any = __ballot(has);
+        if (any) {
+            int low = 0;
+            while (!__ballot(has && i < (low + 1) * 64)) {  // (some lane has it: the loop ends)
+                ++low;
+            }
+            const int lane = __builtin_ctzll(__ballot(has && i < (low + 1) * 64));
+            v = mx, i = low * 64 + lane;
+        }
+        return;
+    }
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
+    for (int d = 1; d < 64; d <<= 1) {  // (with numbers that are none: as they compare)
         const float ov = __shfl_xor(v, d);
         const int   oi = __shfl_xor(i, d);
         if (oi != 0x7fffffff && (i == 0x7fffffff || ov > v || (ov == v && oi < i))) {
@@ -44,9 +60,9 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i)
 // One 256-thread workgroup per token; Wg fp16 [H][E] (input-major like every other weight).  V experts share a pass over the token (V = 8: E a multiple of
 // eight, 16-byte loads of Wg), so the row is read E / V times and every load is independent of the last, sixteen rounds of them in flight; one wave picks the
 // experts.  Bound by that chain: H = 4096, 8 experts: 24.6 us with a pass per expert and one thread picking, 8.0 us with eight
-// rounds in flight, 7.0 with the tail beside it:
+// rounds in flight, 6.4 with the tail beside it:
 // workgroups behind the tokens' quantise the rows, and of up to 64 tokens the last one's writes the routing tables.  16 tokens, fp8 experts: 8.0 + 4.7 (tables) + 4.8 us
-// (codes) -> 7.0.  More tokens keep the tables' own launch, which takes a workgroup an expert.
+// (codes) -> 6.4.  More tokens keep the tables' own launch, which takes a workgroup an expert.
 template<int V>
 __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_ids,      // [T][k]
                                                        float* __restrict__ topk_w,      // [T][k]
@@ -200,7 +216,7 @@ struct MoeGather {  // rows of x, H channels, to xs in the experts' order; share
 // chosen here, one wave per token, as moe_topk_softmax_kernel does (expert e on lane e % 64).  A chain of latencies: 8 tokens, 8 experts, 2 a token take
 // 4.8 us, the two kernels for any size 5.7 + 9.5.
 // V > 0: every workgroup makes the tables for itself, the first one writes them, and each copies four of the rows that moe_gather_kernel would (V channels a load, the
-// first of them asked for ahead of the routing).  8 tokens of 2048, three rows a token: 5.7 us, the two launches
+// first of them asked for ahead of the routing).  8 tokens of 2048, three rows a token: 5.0 us, the two launches
 // 4.8 + 2.6.
 template<bool PICK, class X = __bf16, int V = 0>
 __global__ __launch_bounds__(1024) void moe_route_masks_kernel(int* __restrict__ offsets, int* __restrict__ f2n, int* __restrict__ en2f, int* topk_ids,
