@@ -307,12 +307,14 @@ int64_t tm_debug_trace_records(char* host_out, int64_t cap);
 /* Host-only: the (workgroup shape, split-K) the decode GEMM dispatch picks for a W4A16 linear of K x N at M rows --
  * use_table bit 0: the measured table first (tm_engine_tune_gemm / tm_gemm_import), then the heuristic; clear: heuristic only;
  * bit 1: of a launch without a folded norm (tm_linear_forward, and the engine unless TM_FOLD_NORM asks for folded norms); clear: the heuristic of
- * the folded launches, which differs up to 32 rows of narrow and for 65 .. 256 rows of small projections;
+ * the folded launches, which differs up to 32 rows of narrow and for 65 .. 256 rows of small projections, and which beyond 128 rows, where no
+ * launch is folded, does not tell the two large prefill tiles apart (5 stands for both);
  * bits 8 .. 11: the linear's role -- 0 any, 1 w_qkv, 2 wo, 3 w1w3, 4 w2 (the table is keyed (role, K, N, M): the tuner times each
  * role with its own consumer kernel; an entry of role 0, e.g. an imported line without a role column, serves every role).
- * Shapes: 0..3 decode tiles (M <= 64), 4 / 5 the 128-row tiles (M > 64), 6..9 shapes 3, 0, 2, 1 on 32-row blocks
+ * Shapes: 0..3 decode tiles (M <= 64), 4 / 5 the 128-row tiles of 256 / 512 columns (M > 64), 6..9 shapes 3, 0, 2, 1 on 32-row blocks
  * (gemm_decode.hip), 11 the loader / consumer decode kernel (gemm_decode_lc.hip, M <= 64), 12 the 256 x 256 prefill tile with
- * the weights dequantised once per workgroup tile through LDS (gemm_prefill.hip, M > 64).  (10 was a vendor-library path: gone.) */
+ * each weight dequantised once per workgroup tile, in registers (gemm_prefill.hip, M > 64).  An explicit shape and a table line run exactly the
+ * tile they name.  (10 was a vendor-library path: gone.) */
 int tm_debug_pick_tiling(int K, int N, int M, int use_table, int* shape, int* splits);
 /* Host-only: the tiling of the general kernel (gemm_w4a16.hip: the fp16 lm_head, e4m3 weight-only linears, u4 with N % 32 != 0)
  * for a K x N linear of `weight_type` (TM_WEIGHT_*) and `role` (0 any, 1 w_qkv, 2 wo, 3 w1w3, 4 w2, 5 lm_head) at M rows:

@@ -1205,7 +1205,7 @@ static int launch_dec32_shape(const Dec32Params& p, dim3 grid, int shape, hipStr
     if constexpr (MH == 4) {
         // row blocks of 128 rows x 256 columns, 8 waves of 32 columns over the whole k slice (M > 64): every dequantised
         // weight fragment feeds 4 MFMAs, every x fragment read from LDS feeds 32 columns
-        if (shape == 5) {  // largest prefill tile, where 128 x 512 is the cheaper one (launch_linear_dec32): two weight fragments per x-fragment read
+        if (shape == 5) {  // 128 x 512 tile, two weight fragments per x-fragment read (gemm_pre64_kernel)
 #ifdef TM_EXPERIMENTS
             if (abl == 2) return launch_pre64_one<2>(p, grid, st);  // timing: no MFMA
             if (abl == 8) return launch_pre64_one<8>(p, grid, st);  // timing: raw codes on the matrix pipe
@@ -1569,8 +1569,8 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
         shape = 0;
     }
     if (M > 64) {
-        // M <= 256 (batch-128 decode, small admissions): 256-column tiles of 128 rows keep more workgroups alive; beyond that the largest prefill tile
-        // (shape 5) where its rounds cost less (TM_PRE64_MIN_M: first M that may take it).  With fewer tiles than CUs the 128 x 256 tile takes at most 4
+        // M <= 256 (batch-128 decode, small admissions): 256-column tiles of 128 rows keep more workgroups alive; beyond that a larger prefill tile
+        // where its rounds cost less (TM_PRE64_MIN_M: first M that may take it; shape 5, dec32_pick_plain says which of the two).  With fewer tiles than CUs the 128 x 256 tile takes at most 4
         // slices of k (measured by the tuner at the Llama-3-8B shapes, us per layer incl. the consumer -- M = 512: w_qkv 49.3 -> 36.5, wo 44.9 -> 28.5,
         // w2 74.2 -> 54.2; M = 1024: 66.8 -> 48.1, 61.4 -> 41.5, 105.5 -> 92.6)
         static const int pre64_from = env_int2("TM_PRE64_MIN_M", 257);
@@ -1629,7 +1629,7 @@ void dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out
 }
 
 // Tiling of a product without a folded norm: the measured table, then the lines below for few rows, then the rule above (which the folded launches keep:
-// their residual sums are formed in its slices' order)
+// their residual sums are formed in its slices' order) and, of prefill-sized products, the cheaper of the two large tiles
 void dec32_pick_plain(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table)
 {
     const int        ncg = w.N / 32, KB = w.K / 128;
@@ -1679,6 +1679,9 @@ void dec32_pick_plain(const LinearWeight& w, int M, int* shape_out, int* splits_
         }
     }
     dec32_pick_ex(w, M, shape_out, splits_out, false);
+    if (*shape_out == 5 && *splits_out == 1 && prefill_cost_256(ncg, M) <= prefill_cost_512(ncg, M)) {  // (slices of k: 128 x 512)
+        *shape_out = kShapePre256;
+    }
 }
 
 // y / slabs as launch_linear: *slabs_out = number of fp32 slabs written into `workspace` (1 = direct epilogue)
@@ -1727,9 +1730,6 @@ int launch_linear_dec32(const LinearWeight& w, const half_t* x, int ldx, half_t*
     TM_REQUIRE(w.packed32 != nullptr && w.N % 32 == 0, "decode GEMM: P32 layout missing");
     if (shape == kShapeF16 && (w.image16 == nullptr || M <= 64)) {
         shape = kShapePre256;  // a table entry for a linear without the fp16 image (operator-level handle, TM_PREFILL_F16_IMAGE=0): the fused 256 x 256 tile
-    }
-    if (shape == 5 && splits <= 1 && prefill_cost_256(w.N / 32, M) <= prefill_cost_512(w.N / 32, M)) {
-        shape = kShapePre256;
     }
     TM_REQUIRE(M >= 1 && shape >= 0 && (shape <= 9 || shape == kShapeWide2 || shape == kShapeLC || shape == kShapePre256 || shape == kShapeF16)
                    && (shape >= 6 || (M <= 64) == (shape < 4)) && (shape != kShapeLC || M <= 64) && (shape != kShapePre256 || M > 64)

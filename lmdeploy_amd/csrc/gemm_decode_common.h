@@ -99,7 +99,7 @@ __device__ __forceinline__ void static_for(F&& f)
 
 // gemm_decode_lc.hip: the loader / consumer decode kernel (shape kShapeLC), grid = (ceil(ncg / 4), splits)
 int launch_dec_lc(const Dec32Params& p, dim3 grid, hipStream_t st);
-// gemm_prefill.hip: 256 x 256 prefill tiles, each weight dequantised once per workgroup tile (shape kShapePre256; shape 5 where it costs less),
+// gemm_prefill.hip: 256 x 256 prefill tiles, each weight dequantised once per workgroup tile (shape kShapePre256),
 // grid = (ceil(ncg / 8), splits, ceil(M / 256))
 int launch_pre256(const Dec32Params& p, dim3 grid, hipStream_t st);
 // gemm_prefill_f16.hip: 256 x 256 tiles over the resident fp16 image (p.wp = LinearWeight::image16), both operands by LDS-DMA (shape kShapeF16),

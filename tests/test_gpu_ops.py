@@ -482,7 +482,7 @@ def test_w4a16_linear(tm, cuda, K, N, M):
 @pytest.mark.parametrize('M', [257, 300, 512, 1000, 2500])
 def test_w4a16_linear_prefill_tiles(tm, cuda, K, N, M, gated):
     """The prefill-shaped path (M > 256): 128-row x 512-column workgroup tiles with two weight fragments per x-fragment read
-    (0x205, the default from M = 257) and 128 x 256 tiles (0x204), the round-1 tile (explicit nt / waves), ragged last row
+    (0x205), 128 x 256 (0x204) and 256 x 256 tiles (0x20c), the general kernel's tile (explicit nt / waves), ragged last row
     block, column counts that do not fill the last workgroup, the automatic split-K of mid-size M (fewer than 256 workgroups otherwise) and explicit split counts, plain and gated-SiLU
     epilogues -- same oracle and tolerance as the decode shapes."""
     rng = np.random.default_rng(K + N + M + 11)
@@ -491,7 +491,7 @@ def test_w4a16_linear_prefill_tiles(tm, cuda, K, N, M, gated):
     ref = (o.w4a16_linear_gated_silu(x, q, s, z) if gated else x.astype(np.float32) @ _QCACHE[(K, N)][3]).astype(np.float32)
     ws = torch.zeros(max(1, tm.tm_linear_workspace(h, M)), dtype=torch.uint8, device='cuda')
     x_d = dev(x)
-    # 0x20c = shape 12 (gemm_prefill.hip): 256 x 256 tiles, weights dequantised once per workgroup tile through LDS
+    # 0x20c = shape 12 (gemm_prefill.hip): 256 x 256 tiles, each weight dequantised once per workgroup tile, in registers
     for nt, splits, waves in ((0, 0, 0), (0, 1, 0x204), (0, 2, 0x204), (0, 3, 0x204), (0, 1, 0x205), (0, 2, 0x205), (0, 5, 0x205),
                               (0, 1, 0x20c), (0, 2, 0x20c), (0, 3, 0x20c), (0, 1, 0x20d), (2, 1, 8), (2, 2, 8), (2, 4, 8), (4, 1, 4)):   # 0x20d = shape 13: the fp16 image
         if splits > K // 128:

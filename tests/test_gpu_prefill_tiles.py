@@ -53,3 +53,27 @@ def test_picked_prefill_tile(tm, cuda, K, N, M):
     ref = x.astype(np.float32) @ _QCACHE[(K, N)][3]
     assert (np.abs(host(y).astype(np.float32) - ref) <= 2e-3 + 2.0**-9 * np.abs(ref)).all()
     _ffi.check(tm.tm_linear_destroy(h))
+
+
+@pytest.mark.parametrize('K,N,M,shape', [(512, 8192, 2048, 12), (512, 6144, 2604, 5)])
+def test_reported_tile_runs(tm, cuda, K, N, M, shape):
+    """The tile that is reported for a size is the one that runs there, and an explicit shape runs that shape wherever the rule would take the other: the 256 x 256
+    tile adds the 32 channels of a step in another order than the 128 x 512 tile, so their results differ in single roundings."""
+    rng = np.random.default_rng(N)
+    h, _ = _make_linear(tm, rng, K, N)
+    sh, sp = _ffi.C.c_int(-1), _ffi.C.c_int(-1)
+    _ffi.check(tm.tm_debug_pick_tiling(K, N, M, 2, _ffi.C.byref(sh), _ffi.C.byref(sp)))
+    assert (sh.value, sp.value) == (shape, 1)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    ws = torch.zeros(max(1, tm.tm_linear_workspace(h, M)), dtype=torch.uint8, device='cuda')
+    x_d, ys = dev(x), []
+    for code in (0, 0x205, 0x20c):
+        y = torch.zeros((M, N), dtype=torch.float16, device='cuda')
+        _ffi.check(tm.tm_linear_forward(h, x_d.data_ptr(), K, y.data_ptr(), N, M, 0, 0, 1 if code else 0, code, ws.data_ptr(), st()))
+        ys.append(y)
+    ref = x.astype(np.float32) @ _QCACHE[(K, N)][3]
+    for y in ys:
+        assert (np.abs(host(y).astype(np.float32) - ref) <= 2e-3 + 2.0**-9 * np.abs(ref)).all()
+    assert not torch.equal(ys[1], ys[2])
+    assert torch.equal(ys[0], ys[1] if shape == 5 else ys[2])
+    _ffi.check(tm.tm_linear_destroy(h))

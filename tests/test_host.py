@@ -68,10 +68,23 @@ def test_reported_tiling_of_launches_without_a_folded_norm():
     lib = _ffi.load()
     assert _pick(lib, 4096, 6144, 8, 2)[0] == 3 and _pick(lib, 4096, 4096, 32, 2)[0] == 3 and _pick(lib, 14336, 4096, 1, 2)[0] == 3
     assert _pick(lib, 4096, 4096, 128, 2)[0] == 6 and _pick(lib, 4096, 4096, 256, 2)[0] == 6 and _pick(lib, 14336, 4096, 65, 2)[0] == 6
-    for K, N, M in ((4096, 6144, 33), (4096, 28672, 64), (4096, 28672, 8), (16384, 6144, 1), (13824, 5120, 128), (4096, 28672, 8192)):
+    for K, N, M in ((4096, 6144, 33), (4096, 28672, 64), (4096, 28672, 8), (16384, 6144, 1), (13824, 5120, 128), (4096, 28672, 640), (4096, 6144, 2604)):
         assert _pick(lib, K, N, M, 2) == _pick(lib, K, N, M, 0), (K, N, M)
     assert Engine.pick_tiling(4096, 6144, 8, use_table=False) == _pick(lib, 4096, 6144, 8, 2)
     assert Engine.pick_tiling(4096, 6144, 8, use_table=False, folded=True) == _pick(lib, 4096, 6144, 8, 0)
+
+
+def test_the_pick_decides_between_the_prefill_tiles(tmp_path):
+    """The dispatch of launches without a folded norm itself names the 128 x 512 (5) or the 256 x 256 tile (12), and a table line that names one of them is
+    what it answers where the rule would take the other."""
+    lib = _ffi.load()
+    for K, N, M, shape in ((4096, 28672, 8192, 12), (4096, 4096, 4096, 12), (14336, 4096, 2604, 12), (4096, 6144, 2604, 5), (4096, 28672, 640, 4)):
+        assert _pick(lib, K, N, M, 2) == (shape, 1), (K, N, M)
+    f = tmp_path / 't.txt'
+    f.write_text('2304 28672 8192 5 1\n2304 6144 4096 12 1\n')
+    assert lib.tm_gemm_import(str(f).encode()) == 0
+    assert _pick(lib, 2304, 28672, 8192, 2)[0] == 12 and _pick(lib, 2304, 28672, 8192, 3) == (5, 1)
+    assert _pick(lib, 2304, 6144, 2604, 2)[0] == 5 and _pick(lib, 2304, 6144, 2604, 3) == (12, 1)
 
 
 def test_decode_gemm_heuristic_equals_the_measured_winners(tmp_path):
