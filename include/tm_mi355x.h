@@ -321,7 +321,7 @@ int tm_debug_pick_tiling(int K, int N, int M, int use_table, int* shape, int* sp
  * config4 = {tiles per wave, split-K, waves, k-phases} -- the measured entry (tm_engine_tune_gemm / tm_gemm_import, `G` lines)
  * first, then the heuristic.  Reference: the same DispatchCache serves every GEMM of the model (gemm.cu:92-224). */
 int tm_debug_pick_general(int weight_type, int role, int K, int N, int M, int* config4);
-/* Host-only: the measured row-tile height of the grouped expert GEMMs (u4: 16 / 32 / 64, e4m3 on the fp8 matrix cores: 32 / 64 / 128)
+/* Host-only: the measured row-tile height of the grouped expert GEMMs (u4: 16 / 32 / 64, e4m3 on the fp8 matrix cores: 32 / 64 / 128 / 256)
  * for `tokens` rows per forward; *rows = 0: no entry, the launcher's own rule (by the expected rows per expert) applies. */
 int tm_debug_grouped_tile(int weight_type, int K, int N, int tokens, int* rows);
 /* Host-only: every (shape, splits) pair the start-up tuner (tm_engine_tune_gemm; gemm::Gemm::Run's dispatch candidates,

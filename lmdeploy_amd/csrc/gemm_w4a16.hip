@@ -869,7 +869,7 @@ static bool gen_entry_valid(int kind, int role, int K, int N, int M, const int v
         return (v[0] == 16 || v[0] == 32 || v[0] == 64) && M <= 64;
     }
     if (kind == kGenGrouped + 2) {  // e4m3 experts on the fp8 matrix cores
-        return v[0] == 32 || v[0] == 64 || v[0] == 128;
+        return v[0] == 32 || v[0] == 64 || v[0] == 128 || v[0] == 256;
     }
     return false;
 }
@@ -925,7 +925,7 @@ int gen_grouped_candidates(const LinearWeight& proto, int m_cap, int* rows_out, 
         }
     }
     else if (proto.type == 2) {
-        for (int r : {32, 64, 128}) {
+        for (int r : {32, 64, 128, 256}) {
             if (n < cap && (r == 32 || r / 2 < m_cap)) {
                 rows_out[n++] = r;
             }

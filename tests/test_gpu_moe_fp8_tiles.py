@@ -54,7 +54,7 @@ def test_row_tiles(tm, cuda, T, skew):
 
 
 def test_tiles_of_the_measured_dispatch(tm, cuda, tmp_path):
-    """a table line decides the tile: 32, 64 and 128 rows give the same result, whatever the rule would take for these 100 tokens"""
+    """a table line decides the tile: 32, 64, 128 and 256 rows give the same result, whatever the rule would take for these 100 tokens"""
     rng = np.random.default_rng(5)
     T, H, I, E, k = 100, 256, 384, 4, 2
     x = rng.standard_normal((T, H)).astype(f16)
@@ -69,7 +69,7 @@ def test_tiles_of_the_measured_dispatch(tm, cuda, tmp_path):
         _ffi.check(tm.tm_moe_set_expert(h, e, dev(q13).data_ptr(), dev(s13).data_ptr(), None, dev(q2).data_ptr(), dev(s2).data_ptr(), None, st()))
     ref = o.moe_ffn_fp8(x, gate, experts, k)[0].astype(np.float32)
     ws, table = torch.zeros(tm.tm_moe_workspace(h, T), dtype=torch.uint8, device='cuda'), tmp_path / 't.txt'
-    for rows in (32, 64, 128):
+    for rows in (32, 64, 128, 256):
         table.write_text(f'G 34 0 {H} {2 * I} {T} {rows} 0 0 0\nG 34 0 {I} {H} {T} {rows} 0 0 0\n')
         _ffi.check(tm.tm_gemm_import(str(table).encode()))
         out = torch.zeros((T, H), dtype=torch.float16, device='cuda')

@@ -617,7 +617,7 @@ def test_general_kernel_dispatch_table(tmp_path):
                  f'G 34 0 5120 20480 64 64 0 0 0\n'                   # fp8 experts: 64-row tiles for 64-token forwards
                  f'G 32 0 5120 20480 64 16 0 0 0\n'                   # u4 experts: 16-row tiles
                  f'G 17 5 {K} {N} 64 3 1 4 1\n'                       # invalid: nt = 3
-                 f'G 34 0 5120 20480 64 16 0 0 0\n'                   # invalid: the fp8 grouped kernel has 32-, 64- and 128-row tiles
+                 f'G 34 0 5120 20480 64 16 0 0 0\n'                   # invalid: the fp8 grouped kernel has 32-, 64-, 128- and 256-row tiles
                  f'G 32 0 5120 20480 128 32 0 0 0\n'                  # invalid: u4 grouped tiles are a decode-batch choice
                  f'G 18 0 {K} 6144 300 1 1 8 1\n'                     # invalid: 300 is not a table key (257 .. 512 -> 512)
                  f'{K} 6144 64 6 2 1\n')                              # a P32 line in the same file
@@ -635,16 +635,16 @@ def test_general_kernel_dispatch_table(tmp_path):
 
 
 def test_grouped_fp8_tiles_of_the_measured_dispatch(tmp_path):
-    """table lines of the grouped fp8 products name any tile the launcher has (32, 64, 128 rows) and no other"""
+    """table lines of the grouped fp8 products name any tile the launcher has (32, 64, 128, 256 rows) and no other"""
     lib = _ffi.load()
     f = tmp_path / 't.txt'
-    for rows in (32, 64, 128):
+    for rows in (32, 64, 128, 256):
         f.write_text(f'G 34 0 1280 4352 512 {rows} 0 0 0\n')
         assert lib.tm_gemm_import(str(f).encode()) == 0
         r = _ffi.C.c_int(-1)
         _ffi.check(lib.tm_debug_grouped_tile(2, 1280, 4352, 500, _ffi.C.byref(r)))
         assert r.value == rows
-    for rows in (0, 16, 96, 256):
+    for rows in (0, 16, 96, 512):
         f.write_text(f'G 34 0 1280 4352 512 {rows} 0 0 0\n')
         assert lib.tm_gemm_import(str(f).encode()) == 1
 
