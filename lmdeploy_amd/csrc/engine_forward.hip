@@ -321,6 +321,28 @@ static int linear_fold_produce(tm_engine* e, LinearSlots& l, const half_t* x, in
     return 0;
 }
 
+// the greedy tokens of the rows at slots [slot, slot + n), of a vocabulary that is not cut over ranks
+int greedy_rows(tm_engine* e, int n, int slot, const float* logits32, const StepCommit& commit)
+{
+    return launch_greedy(e->d_next_ids + slot, e->d_logits + (size_t)slot * e->vocab_local, e->vocab_local, logits32,
+                         logits32 ? e->cfg.model.vocab : e->vocab_local, n, e->d_greedy_ws, e->greedy_ws_floats, e->d_greedy_tickets,
+                         e->cfg.max_batch_size + 1, commit, e->stream);
+}
+
+// A mixture's router, experts and sum over the M rows of x.  Without ranks to reduce over, the residual + RMSNorm launch sums the experts' rows itself (y: the
+// normed rows); otherwise the sums are left in d_tmp for reduce_residual_norm.
+int moe_rows(tm_engine* e, const MoeBlock& moe, half_t* y, const half_t* x, int M, const half_t* norm_w)
+{
+    MoeRows    mr;
+    const bool sum_in_norm = !e->use_comm && !e->p2p_ready;
+    TM_PROF(P_GEMM_GATE_UP, TM_TRY(moe_forward(moe, sum_in_norm ? nullptr : e->d_tmp, e->hidden, x, e->hidden, M, e->d_moe_ws, nullptr, nullptr, e->stream,
+                                               sum_in_norm ? &mr : nullptr, e->d_tickets)));
+    if (sum_in_norm) {
+        TM_PROF(P_RES_NORM, TM_TRY(launch_moe_rmsnorm(y, e->d_resid, mr, norm_w, e->cfg.model.rms_eps, M, e->hidden, e->stream)));
+    }
+    return 0;
+}
+
 // Logits rows -> next ids for `n` sequences whose fp16 logits lie in d_logits at the batch slots [slot, slot + n): logits processors
 // (ids_in / cu_q (nullptr: one token per sequence) / ntok = the tokens this forward consumed for them, k_len = their context lengths),
 // then stochastic sampling or arg-max (tensor-parallel: over the gathered vocabulary shards).  Shared by every model family.
@@ -392,8 +414,7 @@ int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_
                                                e->d_topp + slot, e->d_minp + slot, e->d_u + slot, e->d_sample_ws, st, lpr ? &lp : nullptr)));
     }
     else if (!e->use_comm) {
-        TM_PROF(P_SAMPLE, TM_TRY(launch_greedy(ids, logits, e->vocab_local, logits32, logits32 ? m.vocab : e->vocab_local, n, e->d_greedy_ws,
-                                               e->greedy_ws_floats, e->d_greedy_tickets, e->cfg.max_batch_size + 1, commit ? *commit : StepCommit{}, st)));
+        TM_PROF(P_SAMPLE, TM_TRY(greedy_rows(e, n, slot, logits32, commit ? *commit : StepCommit{})));
         return 0;
     }
     else {
@@ -619,16 +640,10 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
         }
         TM_TRY(linear_residual_norm(e, L.wo, e->d_attn, e->q_heads * e->D, M, L.ffn_norm, P_GEMM_O));
         if (L.is_moe) {
-            if (!e->use_comm && !e->p2p_ready) {  // router + grouped expert FFNs; their rows meet in the residual + RMSNorm launch
-                MoeRows mr;
-                TM_PROF(P_GEMM_GATE_UP, TM_TRY(moe_forward(L.moe, nullptr, 0, e->d_x, e->hidden, M, e->d_moe_ws, nullptr, nullptr, st, &mr, e->d_tickets)));
-                TM_PROF(P_RES_NORM, TM_TRY(launch_moe_rmsnorm(e->d_x, e->d_resid, mr, next_norm, m.rms_eps, M, e->hidden, st)));
-                continue;
+            TM_TRY(moe_rows(e, L.moe, e->d_x, e->d_x, M, next_norm));
+            if (e->use_comm || e->p2p_ready) {  // (all-reduce +) residual + RMSNorm as for the dense FFN
+                TM_TRY(reduce_residual_norm(e, M, next_norm));
             }
-            // router + grouped expert FFNs + combine -> d_tmp, then (all-reduce +) residual + RMSNorm as for the dense FFN
-            TM_PROF(P_GEMM_GATE_UP, TM_TRY(moe_forward(L.moe, e->d_tmp, e->hidden, e->d_x, e->hidden, M, e->d_moe_ws, nullptr,
-                                                       nullptr, st, nullptr, e->d_tickets)));
-            TM_TRY(reduce_residual_norm(e, M, next_norm));
             continue;
         }
         TM_PROF(P_GEMM_GATE_UP, TM_TRY(linear_plain(e, L.w13, e->d_x, e->hidden, e->d_act, e->inter, M, true)));

@@ -490,6 +490,8 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
 int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_q, int ntok, const int* k_len, const int* active, const float* logits32,
                 const StepCommit* commit);
 int greedy_alloc(tm_engine* e);
+int greedy_rows(tm_engine* e, int n, int slot, const float* logits32, const StepCommit& commit);
+int moe_rows(tm_engine* e, const MoeBlock& moe, half_t* y, const half_t* x, int M, const half_t* norm_w);
 int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len, int slot0, const MixedDecode* md,
                     const StepEnds* ends);
 int layered_process_weights(tm_engine* e);

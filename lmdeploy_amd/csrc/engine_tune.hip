@@ -1,6 +1,7 @@
 // Measured GEMM dispatch of the engine (reference: the warm-up tuning of turbomind.cc:363-487 -> gemm::Gemm::Run's DispatchCache,
 // kernels/gemm/gemm.cu:92-224; TM_GEMM_TUNE / TM_GEMM_EXPORT / TM_GEMM_IMPORT).
 #include "engine_internal.h"
+#include <numeric>
 
 namespace tmk {
 
@@ -282,6 +283,38 @@ static int time_graph_us(tm_engine* e, const std::function<int()>& chain, float*
     return rc;
 }
 
+// M sequences of one token each, all at the first place of the pool's first block
+struct KvRows {
+    int *       k_len = nullptr, *cu = nullptr;
+    uint64_t*   blocks = nullptr;
+    KvCacheView view{};
+
+    int init(tm_engine* e, int M)
+    {
+        std::vector<int>      ones(M, 1), iota(M + 1);
+        std::vector<uint64_t> ptrs(M, (uint64_t)e->pool);
+        std::iota(iota.begin(), iota.end(), 0);
+        TM_TRY(dmalloc(&cu, (size_t)M + 1));
+        TM_TRY(dmalloc(&blocks, (size_t)M));
+        TM_TRY(dmalloc(&k_len, (size_t)M));
+        TM_HIP_CHECK(hipMemcpy(cu, iota.data(), ((size_t)M + 1) * 4, hipMemcpyHostToDevice));
+        TM_HIP_CHECK(hipMemcpy(blocks, ptrs.data(), (size_t)M * 8, hipMemcpyHostToDevice));
+        TM_HIP_CHECK(hipMemcpy(k_len, ones.data(), (size_t)M * 4, hipMemcpyHostToDevice));
+        view.block_ptrs    = blocks;
+        view.cu_block_nums = cu;
+        view.layout        = e->layout;
+        return 0;
+    }
+    ~KvRows()
+    {
+        for (void* p : {(void*)k_len, (void*)cu, (void*)blocks}) {
+            if (p) {
+                (void)hipFree(p);  // (waits for what the device still does with it)
+            }
+        }
+    }
+};
+
 static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
 {
     hipStream_t st = e->stream;
@@ -349,23 +382,40 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
             cand[nc++] = heur;
         }
         const bool norm_consumer = (r.which == 1 || r.which == 3) && !e->use_comm;
+        // a decode step's [q | k | v] over a 16-bit cache: the rotation and the store, in the product's epilogue or behind it; every row at the first place of the
+        // pool's first block
+        KvRows kv;
+        if (r.which == 0 && M <= e->cfg.max_batch_size && e->layout.bits == 16 && e->D == 128) {
+            TM_TRY(kv.init(e, M));
+        }
         float      best = 1e30f, t_heur = 1e30f;
         GemmConfig bc = heur;
         for (int i = 0; i < nc; ++i) {
-            const GemmConfig cfg = cand[i];
+            GemmConfig cfg = cand[i];
             if (gemm_workspace_bytes(M, w0.N, cfg.splits) > e->gemm_ws_bytes) {
                 continue;
             }
+            const F16KvSink sink{kv.k_len, e->d_rope, e->rope_max_pos, e->q_heads, kv.view};
+            bool            stored = false;
+            cfg.kv                 = kv.k_len ? &sink : nullptr;
+            cfg.kv_done            = &stored;
             auto chain = [&]() -> int {
                 for (const LinearWeight* w : ws) {
                     int slabs = 1;
+                    stored    = false;
                     TM_TRY(launch_linear(*w, r.x, r.ldx, r.y, r.ldy, M, r.gated, cfg, e->d_gemm_ws, norm_consumer && cfg.splits > 1, &slabs, st));
                     if (norm_consumer) {
                         TM_TRY(launch_residual_rmsnorm(norm_out, e->d_resid, slabs > 1 ? nullptr : e->d_tmp, slabs > 1 ? e->d_gemm_ws : nullptr,
                                                        slabs, nullptr, e->final_norm, e->cfg.model.rms_eps, M, e->hidden, st));
                     }
-                    else if (r.which == 4) {  // the head's consumer
-                        TM_TRY(launch_argmax(e->d_next_ids, nullptr, e->d_logits, M, e->vocab_local, e->vocab_local, 0, st));
+                    else if (kv.k_len && !stored) {
+                        TM_TRY(launch_kv_rope_store(r.y, e->q_heads, kv.cu, kv.k_len, M, M, e->d_rope, e->rope_max_pos, kv.view, st));
+                    }
+                    else if (r.which == 4 && !e->use_comm) {  // the head's consumer
+                        TM_TRY(greedy_rows(e, M, 0, nullptr, StepCommit{}));
+                    }
+                    else if (r.which == 4) {
+                        TM_TRY(launch_argmax(e->d_next_ids, e->d_argmax_val, e->d_logits, M, e->vocab_local, e->vocab_local, 0, st));
                     }
                 }
                 return 0;
@@ -391,6 +441,9 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
         if (!(best < 0.93f * t_heur)) {
             bc = heur;
         }
+        if (kv.k_len) {
+            TM_HIP_CHECK(hipMemsetAsync(e->pool, 0, e->block_bytes, st));
+        }
         // (fp16: gemm_kernel has one k-phase; an entry with two says that the dispatch's own kernels, gemm_f16.hip, were the fastest)
         const int v[4] = {bc.nt, bc.f16_stream ? 1 : bc.splits, bc.waves, bc.f16_stream ? 2 : w0.type == 1 || bc.kphases < 1 ? 1 : bc.kphases};
         gen_table_set(kGenDense + w0.type, w0.role, w0.K, w0.N, Mb, v);
@@ -407,11 +460,16 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
         }
     }
     if (moe.size() >= 2 && e->d_moe_ws) {
+        // (the stream grows by the experts' sums from one replay to the next: each timing starts from zero, and its few replays add small numbers)
         auto chain = [&]() -> int {
             for (Layer* L : moe) {
-                TM_TRY(moe_forward(L->moe, e->d_tmp, e->hidden, e->d_x, e->hidden, M, e->d_moe_ws, nullptr, nullptr, st));
+                TM_TRY(moe_rows(e, L->moe, norm_out, e->d_x, M, e->final_norm));
             }
             return 0;
+        };
+        auto time_chain = [&](float* us) -> int {
+            TM_HIP_CHECK(hipMemsetAsync(e->d_resid, 0, (size_t)M * e->hidden * 2, st));
+            return time_graph_us(e, chain, us);
         };
         for (int which = 0; which < 2; ++which) {
             const LinearWeight& proto = which == 0 ? moe[0]->moe.w13[0] : moe[0]->moe.w2[0];
@@ -426,11 +484,11 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
             }
             float t_heur = 1e30f, best = 1e30f;
             int   br = 0;
-            TM_TRY(time_graph_us(e, chain, &t_heur));  // no entry: the launchers' own rule
+            TM_TRY(time_chain(&t_heur));  // no entry: the launchers' own rule
             for (int i = 0; i < nc; ++i) {
                 gen_grouped_rows_override(rows[i]);  // this thread's launches only: nothing transient enters the shared table
                 float     us = 1e30f;
-                const int rc = time_graph_us(e, chain, &us);
+                const int rc = time_chain(&us);
                 gen_grouped_rows_override(0);
                 if (rc) {
                     return rc;
