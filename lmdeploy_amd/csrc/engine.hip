@@ -672,11 +672,7 @@ int tm_engine_stats(tm_engine* e, int64_t* weight_bytes, int64_t* kv_bytes_per_t
     }
     wb += (int64_t)e->output.w.packed_bytes;
     if (e->lm) {
-        for (size_t i = 0; i < e->lm->layers.size(); ++i) {
-            const LmLayer& L = e->lm->layers[i];
-            wb += L.src == (int)i ? (int64_t)(L.qkv.bytes + L.up.bytes + L.out.bytes) : 0;
-        }
-        wb += (int64_t)e->lm->head.bytes;
+        wb += layered_weight_bytes(e);
     }
     if (weight_bytes) *weight_bytes = wb;
     if (kv_bytes_per_token) *kv_bytes_per_token = e->started ? e->block_bytes / 64 : 0;

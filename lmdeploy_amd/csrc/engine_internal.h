@@ -496,6 +496,7 @@ int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode
                     const StepEnds* ends);
 int layered_process_weights(tm_engine* e);
 int layered_init_synthetic(tm_engine* e, uint64_t seed);
+int64_t layered_weight_bytes(const tm_engine* e);
 int layered_start(tm_engine* e);
 void layered_free(tm_engine* e);
 int device_marks_fetch(tm_engine* e, bool async);

@@ -159,6 +159,24 @@ static int plain_up_col(const LmLayer& L)
     return (L.n_q + L.n_k + L.n_v + 255) / 256 * 256;
 }
 
+// Bytes of the projections and the head, each as an image of its own (columns rounded up to 128): neither what lies between tiles that stand apart in memory nor the
+// columns between the two parts of a fused image
+int64_t layered_weight_bytes(const tm_engine* e)
+{
+    auto bytes = [](const DenseWeight& d, int gap) { return (int64_t)d.Kp * (d.Np - gap) * d.count * (d.dtype == kDenseF32 ? 4 : 2); };
+    int64_t n  = bytes(e->lm->head, 0);
+    for (size_t i = 0; i < e->lm->layers.size(); ++i) {
+        const LmLayer& L = e->lm->layers[i];
+        if (L.src != (int)i) {
+            continue;
+        }
+        const bool fused = !L.both && !L.pre && !L.post && !L.wide && L.spec.mlp;
+        const int  n_qkv = L.n_q + L.n_k + L.n_v;
+        n += bytes(L.qkv, fused ? plain_up_col(L) - (n_qkv + 127) / 128 * 128 : 0) + bytes(L.up, 0) + bytes(L.out, 0);
+    }
+    return n;
+}
+
 static int place(tm_engine* e, DenseWeight& d, int row0, int col0, const std::string& name, int rows, int cols, size_t src_row = 0, int item = 0,
                  bool transpose = false, int half = 0)
 {

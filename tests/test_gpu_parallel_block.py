@@ -7,7 +7,7 @@ import pytest
 from tests import layered_oracle as lo
 from tests.gpu_helpers import host, release_all
 from tests.test_gpu_febivik import Paged, attend
-from tests.test_gpu_layered import TOL, engine_for, rel_err, small_model
+from tests.test_gpu_layered import TOL, _layer, engine_for, rel_err, small_model
 
 pytestmark = pytest.mark.gpu
 
@@ -59,4 +59,14 @@ def test_decode_rows_around_the_line(cuda, n, dtype):
     got = np.concatenate(got, axis=1)
     for r in (0, 1, n // 2, n - 1):
         assert rel_err(got[r], lo.forward(cfg, w, reqs[r])[0]) <= TOL[dtype], r
+    eng.close()
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+def test_weight_bytes(cuda, dtype):
+    """the reported bytes are those of the weights (columns in whole groups of 128), not of the memory between tiles or between the parts of the fused product"""
+    cfg = lo.make_config(2048, 203, [_layer(dim=8, vdim=8, ff=24)])
+    eng = engine_for(cfg, lo.make_weights(cfg, 0), dtype)
+    # [q | k | v], up: 2048 to 64 and 24 columns; [o | down]: 32 + 24 to 2048; head
+    assert eng.stats()['weight_bytes'] == (2 if dtype == 'bfloat16' else 4) * (2048 * (128 + 128) + 64 * 2048 + 2048 * 256)
     eng.close()
