@@ -58,7 +58,8 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i)
 }
 
 // One 256-thread workgroup per token; Wg fp16 [H][E] (input-major like every other weight).  V experts share a pass over the token (V = 8: E a multiple of
-// eight, 16-byte loads of Wg), so the row is read E / V times and every load is independent of the last, sixteen rounds of them in flight; one wave picks the
+// eight, 16-byte loads of Wg), so the row is read E / V times and every load is independent of the last, sixteen rounds of them in flight (V = 1: a short pass an expert,
+// which loads beyond the row's end would only lengthen: eight; 60 experts of H = 2048, one token, a whole expert block 87 us, with sixteen 107); one wave picks the
 // experts.  Bound by that chain: H = 4096, 8 experts: 24.6 us with a pass per expert and one thread picking, 8.0 us with eight
 // rounds in flight, 6.4 with the tail beside it:
 // workgroups behind the tokens' quantise the rows, and of up to 64 tokens the last one's writes the routing tables.  16 tokens, fp8 experts: 8.0 + 4.7 (tables) + 4.8 us
@@ -96,7 +97,13 @@ __global__ __launch_bounds__(256) void moe_gate_kernel(int* __restrict__ topk_id
         for (int i = 0; i < V; ++i) {
             acc[i] = 0.f;
         }
-        for (int h0 = threadIdx.x; h0 < H; h0 += 256 * 16) {
+        if constexpr (V == 1) {
+#pragma unroll 8
+            for (int h = threadIdx.x; h < H; h += 256) {
+                acc[0] = __builtin_fmaf((float)xr[h], (float)wg[(size_t)h * E + e], acc[0]);
+            }
+        }
+        for (int h0 = threadIdx.x; V > 1 && h0 < H; h0 += 256 * 16) {
             half_t xv[16];
             HV     wv[16];
 #pragma unroll
