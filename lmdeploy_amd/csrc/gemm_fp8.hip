@@ -29,6 +29,7 @@
 #include "tm_common.h"
 #include "tm_kernels.h"
 #include <algorithm>
+#include <cmath>
 #include <stdlib.h>
 #include <type_traits>
 
@@ -720,9 +721,14 @@ int launch_linear_fp8_grouped(const LinearWeight& proto, const void* d_groups, i
     // much as those that are.  Mixtral-sized experts (4096 x 14336, 8, top 2), us a layer with 32 / 64 / 128 rows: 16 expected 259 / 302 / 427, 48: 398 / 326
     // / 428, 64: 469 / 478 / 430, 100: 612 / 522 / 447, 128: 735 / 641 / 697, 256: 1304 / 1088 / 1013, 1024: 4915 / 3857 / 3264 (0.88 PFLOP/s; 64 rows with
     // the row blocks of a column tile far apart: 4868).  128 / 256 rows (the kernel of 256 x 256 tiles): 80 expected 489 / 544, 100: 452 / 499, 110: 561 / 489, 160: 773 / 506,
-    // 1000: 3104 / 1765; 32 experts of 4096 x 1536: 80: 283 / 293, 150: 509 / 351
+    // 1000: 3104 / 1765; 32 experts of 4096 x 1536: 80: 283 / 293, 150: 509 / 351.  What the larger tile saves is a second round of the smaller ones: while those (of
+    // the rows that an expert has with the spread of a random choice) are about a round, the chip is emptier with a quarter as many.  One product, 128 rows and
+    // the difference of 256: (1024, 1024) 4 experts, 500 rows 128 tiles 48 us + 6; (14336, 4096) 8 experts, 110 rows 256 tiles + 62 of 439, 160 rows 512 tiles
+    // - 23 of 770; (4096, 4096) 4 experts, 160 rows 256 tiles + 14 of 132, 250 rows 384 tiles - 15 of 194; (6144, 2048) 2 experts, 1000 rows 288 tiles + 24 of 132
+    // (2000: - 66 of 299); (3584, 1024) 8 experts, 300 rows 192 tiles + 17 of 139, 500 rows 320 tiles - 9 of 208
     const bool wide = ldy % 8 == 0 && (uintptr_t)y % 16 == 0;  // (rows leave in 16-byte runs)
-    int        rows = measured ? tv[0] : want <= 32 ? 32 : m_hint < 56 ? 64 : m_hint < 105 ? 128 : 256;
+    const int  t128 = E * (int)std::ceil((m_hint + std::sqrt((double)m_hint)) / 128.0) * ((p.ncg + 3) / 4);
+    int        rows = measured ? tv[0] : want <= 32 ? 32 : m_hint < 56 ? 64 : m_hint < 105 || t128 <= 288 ? 128 : 256;
     rows            = rows == 256 && !wide ? 128 : rows;
     p.experts      = E;
     p.ct8          = ((p.ncg + 3) / 4 + 7) / 8;
