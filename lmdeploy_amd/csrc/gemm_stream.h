@@ -308,7 +308,8 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
 template<class T, class Epi, int MT, int NT, int W>
 __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi epi)
 {
-    constexpr int kChunk = MT * NT > 1 ? 4 : 8;
+    constexpr bool kAhead = MT == 1 || (MT == 2 && sizeof(T) == 2);
+    constexpr int  kChunk = MT * NT > 1 && kAhead ? 4 : 8 / NT;
     __shared__ __attribute__((aligned(16))) floatx4 red[W][MT * NT][64];
     const int  lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int  mb   = blockIdx.y % a.row_blocks * (MT * 16), tile0 = blockIdx.x * NT;
@@ -336,19 +337,23 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
             acc[t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    // x of a chunk leaves with its weights, ahead of them: loads return in order, and a load of x where it is used would wait for the next
-    // chunk's weights (fp16, 8 rows: (2048, 4096) 5.9 -> 5.4 us, (2048, 2048) 5.1 -> 4.8; fp32, 3 rows, (2048, 2048) 8.5 -> 8.0)
+    // Up to 16 rows, and up to 32 of a 16-bit format, x of a chunk leaves with its weights, ahead of them: loads return in order, and a load of x where it is used would
+    // wait for the next chunk's weights (fp16, 8 rows: (2048, 4096) 5.9 -> 5.4 us, (2048, 2048) 5.1 -> 4.8; fp32, 3 rows, (2048, 2048) 8.5 -> 8.0; bf16, 17
+    // rows, (4096, 4096) 11.9 -> 10.8).  More rows take more registers for it than they leave for weights: x there | where it is used, 64 rows: bf16 (2048, 2048)
+    // 11.8 | 11.4 us, fp32 (8448, 2048) 80.5 | 71.9, (2048, 2048) 23.0 | 21.0; fp32, 32 rows: 13.8 | 13.0
     u32x4 wa[kChunk][NT], wb[kChunk][NT], xa[kChunk][MT], xb[kChunk][MT];
     auto  fetch = [&](u32x4(&buf)[kChunk][NT], u32x4(&xbuf)[kChunk][MT], int base) {
+        if constexpr (kAhead) {
 #pragma unroll
-        for (int kk = 0; kk < kChunk; ++kk) {
-            const int s = min(base + kk, a.steps - 1);
+            for (int kk = 0; kk < kChunk; ++kk) {
+                const int s = min(base + kk, a.steps - 1);
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                xbuf[kk][t] = *(const u32x4*)(xp[t] + (int64_t)s * 64);
+                for (int t = 0; t < MT; ++t) {
+                    xbuf[kk][t] = *(const u32x4*)(xp[t] + (int64_t)s * 64);
+                }
             }
+            asm volatile("" ::: "memory");
         }
-        asm volatile("" ::: "memory");
 #pragma unroll
         for (int kk = 0; kk < kChunk; ++kk) {
             const int s = min(base + kk, a.steps - 1);
@@ -357,7 +362,9 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
                 buf[kk][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + (s >> 2) * a.w_quad + (s & 3) * 1024));
             }
         }
-        asm volatile("" ::: "memory");
+        if constexpr (kAhead) {
+            asm volatile("" ::: "memory");
+        }
     };
     auto compute = [&](const u32x4(&buf)[kChunk][NT], const u32x4(&xbuf)[kChunk][MT], int base) {
 #pragma unroll
@@ -365,9 +372,16 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
             if (base + kk < a.steps) {
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
+                    u32x4 b;
+                    if constexpr (kAhead) {
+                        b = xbuf[kk][t];
+                    }
+                    else {
+                        b = *(const u32x4*)(xp[t] + (int64_t)(base + kk) * 64);
+                    }
 #pragma unroll
                     for (int j = 0; j < NT; ++j) {
-                        acc[t][j] = StreamOp<T>::mma(buf[kk][j], xbuf[kk][t], acc[t][j]);
+                        acc[t][j] = StreamOp<T>::mma(buf[kk][j], b, acc[t][j]);
                     }
                 }
             }
