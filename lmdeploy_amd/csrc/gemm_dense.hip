@@ -93,6 +93,7 @@ struct DenseEpi {
     int       vec;  // rows of y (and of the operands read beside it) start at multiples of 16 bytes
 
     static constexpr bool kPairs = EPI == kDenseGatedAct && sizeof(T) == 2;
+    static constexpr bool kTileRuns = true;
     __device__ __forceinline__ const int* row_offsets() const
     {
         return c.row_offsets;
@@ -284,23 +285,17 @@ struct DenseEpi {
 // Images are stored in FRAGMENT ORDER: the 16 rows x 64 bytes block (n / 16, k / step) is one contiguous KB laid out as the 64 lanes of
 // its MFMA fragment (16 bytes each: lane = piece * 16 + n % 16), blocks of one 16-row tile consecutive along k -- a wave's fragment
 // load is one contiguous KB and a workgroup streams whole contiguous runs of HBM instead of 64-byte pieces of 16 rows
-//
-// Steps from one tile to the next in the image.  A launch reads a thousand tiles at about the same step: with distances that are multiples of 64 KB those places
-// fall on a part of the memory channels, so such tiles are 4 KB apart (2, 4, 8, 12 and 20 KB the same within 2 %, 1 KB no help).  bf16, 32 rows, weights from HBM:
-// (4096, 27648) 45.4 -> 41.8 us, (4096, 32000) 47.2 -> 43.4; nine items of (2048, 2816) 20.6 -> 19.5; fp32 tiles of (2048, 2048) 98 -> 95.6; elsewhere the same.
-static int dense_tile_steps(int steps)
-{
-    return steps % 64 == 0 ? steps + 4 : steps;
-}
+// (from stream_turn's step on)
 template<class T>
-__host__ __device__ inline size_t dense_frag_index(int n, int k, int tile_steps)
+__host__ __device__ inline size_t dense_frag_index(int n, int k, int steps)
 {
     constexpr int E = 16 / sizeof(T), S = 4 * E;  // elements of a 16-byte piece, of a step
-    return (((size_t)(n >> 4) * tile_steps + k / S) * 64 + (k % S) / E * 16 + (n & 15)) * E + k % E;
+    const int     at = k / S + stream_turn(n >> 4, steps);
+    return (((size_t)(n >> 4) * steps + (at < steps ? at : at - steps)) * 64 + (k % S) / E * 16 + (n & 15)) * E + k % E;
 }
 
 template<class T>
-__global__ void dense_place_kernel(T* __restrict__ dst, int tile_steps, int row0, int col0, const __bf16* __restrict__ src, int rows, int cols,
+__global__ void dense_place_kernel(T* __restrict__ dst, int steps, int row0, int col0, const __bf16* __restrict__ src, int rows, int cols,
                                    int transpose, int half)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -311,7 +306,7 @@ __global__ void dense_place_kernel(T* __restrict__ dst, int tile_steps, int row0
         if (half) {
             n = dense_pair_row(n, half - 1, sizeof(T) == 4);
         }
-        dst[dense_frag_index<T>(n, k, tile_steps)] = (T)(float)src[i];
+        dst[dense_frag_index<T>(n, k, steps)] = (T)(float)src[i];
     }
 }
 
@@ -324,7 +319,7 @@ int dense_weight_alloc(DenseWeight& d, int K, int N, int dtype, hipStream_t st, 
     d.Np    = (N + 127) / 128 * 128;
     d.dtype = dtype;
     d.count = count;
-    d.bytes = (size_t)dense_tile_steps(d.Kp / (dtype == kDenseF32 ? 16 : 32)) * 1024 * (d.Np / 16) * count;
+    d.bytes = (size_t)d.Kp * d.Np * count * (dtype == kDenseF32 ? 4 : 2);
     TM_HIP_CHECK(hipMalloc(&d.w, d.bytes));
     TM_HIP_CHECK(hipMemsetAsync(d.w, 0, d.bytes, st));
     return 0;
@@ -337,15 +332,15 @@ int dense_weight_place(DenseWeight& d, int row0, int col0, const void* src_bf16,
     TM_REQUIRE((half ? dense_pair_rows(row0 + (transpose ? cols : rows)) : row0 + (transpose ? cols : rows)) <= d.N
                    && col0 + (transpose ? rows : cols) <= d.K,
                "dense weight: part outside the image");
-    const size_t n = (size_t)rows * cols, at = d.bytes / d.count * item / (d.dtype == kDenseF32 ? 4 : 2);
+    const size_t n = (size_t)rows * cols, at = (size_t)item * d.Np * d.Kp;
     if (n == 0) {
         return 0;
     }
     if (d.dtype == kDenseF32) {
-        dense_place_kernel<float><<<(n + 255) / 256, 256, 0, st>>>((float*)d.w + at, dense_tile_steps(d.Kp / 16), row0, col0, (const __bf16*)src_bf16, rows, cols, transpose, half);
+        dense_place_kernel<float><<<(n + 255) / 256, 256, 0, st>>>((float*)d.w + at, d.Kp / 16, row0, col0, (const __bf16*)src_bf16, rows, cols, transpose, half);
     }
     else {
-        dense_place_kernel<__bf16><<<(n + 255) / 256, 256, 0, st>>>((__bf16*)d.w + at, dense_tile_steps(d.Kp / 32), row0, col0, (const __bf16*)src_bf16, rows, cols, transpose, half);
+        dense_place_kernel<__bf16><<<(n + 255) / 256, 256, 0, st>>>((__bf16*)d.w + at, d.Kp / 32, row0, col0, (const __bf16*)src_bf16, rows, cols, transpose, half);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
@@ -589,7 +584,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
     StreamArgs a{};
     a.x = (const char*)x, a.ldx = (int64_t)ldx * sizeof(T);
     a.w = (const char*)d.w, a.steps = (int)(d.Kp * sizeof(T) / 64), a.tiles = d.Np / 16;
-    a.w_tile = (int64_t)dense_tile_steps(a.steps) * 1024, a.w_quad = 4096;
+    a.w_tile = (int64_t)a.steps * 1024, a.w_quad = 4096;
     a.y = y, a.ldy = ldy, a.M = M, a.N = d.N;
     const bool f32_out = epi == kDenseResidAdd || epi == kDenseScaleF32 || epi == kDenseBiasF32 || epi == kDenseResidGate;
     const int  align   = f32_out || sizeof(T) == 4 ? 4 : 8;  // elements of 16 bytes
@@ -663,7 +658,7 @@ int launch_dense_call(const DenseWeight& d, const void* x, int ldx, void* y, int
     if (M == 0) {
         return 0;
     }
-    call.w_stride = d.bytes / d.count / (d.dtype == kDenseF32 ? 4 : 2);
+    call.w_stride = (size_t)d.Np * d.Kp;
     call.ldx      = ldx;
     if (d.dtype == kDenseF32) {
         TM_REQUIRE(ldx % 4 == 0, "dense linear (fp32): rows must be 16-byte aligned");

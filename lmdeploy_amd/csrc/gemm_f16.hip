@@ -22,7 +22,7 @@ struct F16Epi {
     int gated;  // columns alternate (gate_j, up_j): out[m][j] = silu(acc[m][2 j]) * acc[m][2 j + 1]
     int vec;    // rows of y start on 8 bytes
 
-    static constexpr bool kPairs = false;
+    static constexpr bool kPairs = false, kTileRuns = false;
     __device__ __forceinline__ const int* row_offsets() const
     {
         return nullptr;

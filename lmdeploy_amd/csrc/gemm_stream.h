@@ -61,6 +61,26 @@ struct StreamArgs {
     float*      slabs;        // skinny kernel, several slices: their partial sums, [item][slice][M][16 tiles]
     unsigned*   tickets;      // ... and an arrival counter per (column group, row block, item), zero between launches (nullptr: the slabs are the result)
 };
+// The step that stands first in a tile of an image whose tiles are one behind the other (Epi::kTileRuns).  A launch reads a thousand tiles at about the same step.
+// Where tiles are a multiple of 64 KB long those places fall on a part of the memory channels, so tiles of 128 KB and more are turned: they begin with another step,
+// 4 KB further in some order for every 16 tiles, and end with the steps ahead of it.  bf16, weights from HBM, plain / turned / tiles 4 KB apart (which reach over one
+// page more): (4096, 27648) 8 rows 41.1 / 38.1 / 37.0 us, 32 rows 44.6 / 41.3 / 41.5, 200 rows 78 / 80 / 81; (4096, 4096) 32 rows 14.7 / 14.1 / 13.8, 640 rows 43.9 / 43.5
+// / 45.9; (8192, 2048) 32 rows 23.1 / 21.7 / 21.9, 4096 rows 135 / 132 / 144.  Tiles of 64 KB gain nothing: (2048, 12288) 8 rows 11.5 / 12.7 / 11.6, 65 rows 17.9 /
+// 18.1 / 20.8; (2048, 8448) 65 rows 16.1 / 17.7 / 17.9 (and with the number of the sixteen alone, or three, five or seven times it, (2048, 32000) 32 rows 25 / 28).
+__host__ __device__ inline int stream_turn(int tile, int steps)
+{
+    return steps % 64 == 0 && steps >= 128 ? (((tile >> 4) ^ (tile >> 8)) * 11 & 15) * 4 : 0;
+}
+// where step s is in a tile (turn: the step that stands first)
+template<class Epi>
+__device__ __forceinline__ int64_t stream_step_at(const StreamArgs& a, int s, int turn)
+{
+    if constexpr (Epi::kTileRuns) {
+        const int at = s + turn;
+        return (at < a.steps ? at : at - a.steps) * 1024;
+    }
+    return (s >> 2) * a.w_quad + (s & 3) * 1024;
+}
 // from the first block of a column tile to the end of the image's last block
 __device__ __forceinline__ int64_t stream_weight_bytes(const StreamArgs& a, int tile)
 {
@@ -107,14 +127,15 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
     for (int j = 0; j < NT; ++j) {
         wp[j] = w + (int64_t)min(tile0 + j, a.tiles - 1) * a.w_tile;
     }
-    u32x4 wa[kChunk][NT], wb[kChunk][NT], xr[kXPer];
+    const int turn = stream_turn(tile0, a.steps);
+    u32x4     wa[kChunk][NT], wb[kChunk][NT], xr[kXPer];
     auto  fetch = [&](u32x4(&buf)[kChunk][NT], int base) {
 #pragma unroll
         for (int kk = 0; kk < kChunk; ++kk) {
             const int s = min(base + kk, a.steps - 1);
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                buf[kk][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + (s >> 2) * a.w_quad + (s & 3) * 1024));
+                buf[kk][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + stream_step_at<Epi>(a, s, turn)));
             }
         }
     };
@@ -341,7 +362,8 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
     // wait for the next chunk's weights (fp16, 8 rows: (2048, 4096) 5.9 -> 5.4 us, (2048, 2048) 5.1 -> 4.8; fp32, 3 rows, (2048, 2048) 8.5 -> 8.0; bf16, 17
     // rows, (4096, 4096) 11.9 -> 10.8).  More rows take more registers for it than they leave for weights: x there | where it is used, 64 rows: bf16 (2048, 2048)
     // 11.8 | 11.4 us, fp32 (8448, 2048) 80.5 | 71.9, (2048, 2048) 23.0 | 21.0; fp32, 32 rows: 13.8 | 13.0
-    u32x4 wa[kChunk][NT], wb[kChunk][NT], xa[kChunk][MT], xb[kChunk][MT];
+    const int turn = stream_turn(tile0, a.steps);
+    u32x4     wa[kChunk][NT], wb[kChunk][NT], xa[kChunk][MT], xb[kChunk][MT];
     auto  fetch = [&](u32x4(&buf)[kChunk][NT], u32x4(&xbuf)[kChunk][MT], int base) {
         if constexpr (kAhead) {
 #pragma unroll
@@ -355,11 +377,15 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
             asm volatile("" ::: "memory");
         }
 #pragma unroll
-        for (int kk = 0; kk < kChunk; ++kk) {
-            const int s = min(base + kk, a.steps - 1);
+        for (int kk = 0; kk < kChunk; kk += 4) {
+            const int64_t at   = stream_step_at<Epi>(a, min(base + kk, a.steps - 1) & ~3, turn);  // (four steps are contiguous)
+            const int     last = a.steps - 1 - (min(base + kk, a.steps - 1) & ~3);
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                buf[kk][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + (s >> 2) * a.w_quad + (s & 3) * 1024));
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    buf[kk + e][j] = __builtin_nontemporal_load((const u32x4*)(wp[j] + at + min(e, last) * 1024));
+                }
             }
         }
         if constexpr (kAhead) {
@@ -528,8 +554,9 @@ __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_k
     for (int r = 0; r < kWP; ++r) {
         woff[r] = (int)(min(kWP * wave + r, a.tiles - 1 - (n0 >> 4)) * a.w_tile) + lane * 16;
     }
-    auto dma = [&](int s, int buf) {
-        const int      ws  = (int)((s >> 2) * a.w_quad) + (s & 3) * 1024;
+    const int turn = stream_turn(n0 >> 4, a.steps);
+    auto      dma  = [&](int s, int buf) {
+        const int      ws  = (int)stream_step_at<Epi>(a, s, turn);
         const unsigned dst = lds0 + buf * kStage;
 #pragma unroll
         for (int r = 0; r < kXP; ++r) {
@@ -663,13 +690,14 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
         xoff[r]       = (int)(min(row, Mloc - 1) * a.ldx) + ((lane & 3) ^ ((row >> 1) & 3)) * 16;
         woff[r]       = (int)(min(kWP * wave + r, a.tiles - 1 - (n0 >> 4)) * a.w_tile) + lane * 16;
     }
-    auto dma_piece = [&](int s, int buf, int n) {
+    const int turn      = stream_turn(n0 >> 4, a.steps);
+    auto      dma_piece = [&](int s, int buf, int n) {
         const unsigned dst = lds0 + buf * kStage + (4 * wave + (n & 3)) * 1024;
         if (n < 4) {
             stream_dma16(rs_x, xoff[n], s * 64, dst);
         }
         else {
-            stream_dma16(rs_w, woff[n - 4], (int)((s >> 2) * a.w_quad) + (s & 3) * 1024, dst + kXB);
+            stream_dma16(rs_w, woff[n - 4], (int)stream_step_at<Epi>(a, s, turn), dst + kXB);
         }
     };
     floatx4 acc[8][8];

@@ -17,7 +17,7 @@ from tests.test_gpu_bedenex import engine as bedenex_engine
 from tests.test_gpu_bedenex import model_folder as bedenex_folder
 from tests.test_gpu_febivik import engine, model_folder
 from tests.test_gpu_febivik import rel_err as rel_err_febivik
-from tests.test_gpu_layered import _layer, engine_for, rel_err
+from tests.test_gpu_layered import TOL, _layer, engine_for, rel_err
 from tests.test_gpu_roravik import engine as roravik_engine
 from tests.test_gpu_roravik import model_folder as roravik_folder
 
@@ -214,3 +214,43 @@ def test_epilogues_of_256_column_tiles(cuda, tmp_path, name):
     eng.close()
     # roundings to bf16 (2^-9) of the normed rows, heads, activations and their products' inputs; a column from a wrong place is off by its own size
     assert errs.max() <= 4e-2, np.sort(errs)[-5:]
+
+
+@pytest.mark.parametrize('dtype,K', [(0, 4096), (0, 8192), (1, 2048), (0, 2048), (0, 4128)])
+def test_turned_tiles(tm, cuda, dtype, K):
+    """tiles of 128 KB and more (multiples of 64 KB) begin at a step of their own, shorter ones and those of other lengths do not: more than sixteen times 256 columns,
+    the last not full, in every kernel"""
+    N = 4500
+    g = torch.Generator('cuda').manual_seed(K)
+    w = torch.randn(N, K, generator=g, device='cuda').bfloat16()
+    h = C.c_void_p()
+    _ffi.check(tm.tm_dense_create(C.byref(h), K, N, dtype, w.data_ptr(), st()))
+    T = torch.bfloat16 if dtype == 0 else torch.float32
+    for M in (1, 20, 40, 65, 200, 300, 1100, 2100):
+        x = torch.randn(M, K, generator=g, device='cuda').to(T)
+        ref, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+        y = torch.full((M + 1, N), -3.0, device='cuda', dtype=T)
+        _ffi.check(tm.tm_dense_forward(h, x.data_ptr(), K, y.data_ptr(), N, M, 0, 1.0, st()))
+        check(y[:M], ref, size, K, dtype == 0)
+        assert bool((y[M] == -3.0).all())
+    _ffi.check(tm.tm_dense_destroy(h))
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+def test_turned_tiles_in_slices(cuda, dtype):
+    """the same in an engine's decode steps, whose products may be cut along k, and in its prompts"""
+    cfg = lo.make_config(4096, 203, [_layer(heads=8, kv_heads=2, dim=32, vdim=32, ff=4160)], mult=0.4)
+    w = lo.make_weights(cfg, 5)
+    eng = engine_for(cfg, w, dtype, max_batch_size=20, cache_blocks=24)
+    rng = np.random.default_rng(3)
+    for rows in (3, 20):
+        toks = rng.integers(0, cfg['vocab'], (rows, 6))
+        sess = [eng.open_session() for _ in range(rows)]
+        got = [eng.step_tokens([(s, t[:4], [0, 1, 2, 3]) for s, t in zip(sess, toks)]).reshape(rows, 4, -1)]
+        got += [eng.step_tokens([(s, t[i:i + 1], [0]) for s, t in zip(sess, toks)]).reshape(rows, 1, -1) for i in (4, 5)]
+        got = np.concatenate(got, axis=1)
+        for r in (0, rows - 1):
+            assert rel_err(got[r], lo.forward(cfg, w, toks[r].tolist())[0]) <= TOL[dtype]
+        for s in sess:
+            eng.close_session(s)
+    eng.close()
