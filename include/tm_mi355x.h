@@ -324,6 +324,11 @@ int tm_debug_pick_general(int weight_type, int role, int K, int N, int M, int* c
 /* Host-only: the measured row-tile height of the grouped expert GEMMs (u4: 16 / 32 / 64, e4m3 on the fp8 matrix cores: 32 / 64 / 128 / 256)
  * for `tokens` rows per forward; *rows = 0: no entry, the launcher's own rule (by the expected rows per expert) applies. */
 int tm_debug_grouped_tile(int weight_type, int K, int N, int tokens, int* rows);
+/* Host-only: what a plain product x [M][K] . W of N columns runs.  kind 0: bf16, 1: fp32 (tm_dense_forward and the layer-list engines), 2: fp16 (TM_WEIGHT_F16
+ * linears); scratch: 1 with slabs and arrival counters for slices of k (an engine), 0 without (tm_dense_forward).  plan5 = {kernel, column tiles a workgroup,
+ * row tiles of 16, slices of k, columns of a first launch of 256 x 256 tiles (0: one launch)}; kernel 0: the general kernel (kind 2 only), 1: narrow, 2: the
+ * weight stream with rows in LDS, 3 .. 6: tiles of 256 x 256, 256 x 128, 128 x 128, 64 x 64. */
+int tm_debug_stream_plan(int kind, int K, int N, int M, int scratch, int* plan5);
 /* Host-only: every (shape, splits) pair the start-up tuner (tm_engine_tune_gemm; gemm::Gemm::Run's dispatch candidates,
  * src/turbomind/kernels/gemm/gemm.cu:92-224) may pick for a K x N linear at M rows; *count = how many exist (<= 128), the first
  * min(cap, *count) are written.  The full-size parity tests sweep exactly this list. */

@@ -116,13 +116,15 @@ struct F16EpiKv: F16Epi {
 //   up to 64 rows, 193 ... 256 workgroups: (K, N) = (4096, 28672) gated 8 rows 35.4 | 34.7, 32 rows 35.5 | 38.5, 64 rows 40 | 44, (5120, 27648) gated 8 rows
 //     43.6 | 44.1, 64 rows 48 | 55, (4096, 32000) 64 rows 42 | 47; not (4096, 24576) 32 rows 34 | 32, (4096, 20480) 64 rows 37 | 31, (2048, 16384) gated 21 | 15,
 //     nor (4096, 36864) 32 rows 65 | 55, (4096, 8192) gated 27 | 16
-//   41 ... 64 rows of very wide outputs: (4096, 128256) 64 rows 186 | 197, 48 rows 179 | 183, (2048, 92544) 64 rows 72 | 74; not 32 rows 171 | 167
+//   41 ... 64 rows of wider outputs, where their last round is at least three quarters full or one of many: K = 4096, 64 rows, 256 workgroups 42.6 | 46.1, 448 77 | 87, 512
+//     84 | 93, 723 127 | 137, 1002 179 | 192, 1188 218 | 232; not 288 68 | 58, 384 73 | 68, 576 113 | 111, nor K = 2048 640 63 | 61; nor 32 rows, 384 71 | 62, 1002 170 | 166
 //   more rows, one round of them where 64 x 64 tiles take two: (2048, 16384) gated, 128 rows 20.9 | 26, (4096, 6144) 192 rows 30 | 42, (4096, 4096) 320 rows 29 |
 //     39, (14336, 4096) 320 rows 92 | 130; not where one round of tiles is enough, (4096, 4096) 256 rows 29 | 23, nor where it takes two, 640 rows 58 | 45
 bool f16_stream_supported(const LinearWeight& w, int M)
 {
     const int  rb = (M + 63) / 64, t64 = (w.N + 63) / 64 * rb, t128 = (w.N + 127) / 128 * rb;
-    const bool general = M <= 64 ? (t128 > 192 && t128 <= 256) || (M > 40 && t128 > 448) : t64 > 256 && t128 <= 256;
+    const bool full    = t128 % 256 == 0 || t128 % 256 >= 192 || t128 > 1024;
+    const bool general = M <= 64 ? t128 > 192 && (M > 40 ? full : t128 <= 256) : t64 > 256 && t128 <= 256;
     return w.type == 1 && w.packed && (size_t)w.K * w.N * 2 < ((size_t)1 << 31) && !general;  // (byte offsets inside the image are 32 bits)
 }
 
@@ -216,6 +218,22 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
         return launch_tile_shape(rest, epi, p.tile2, st);
     }
     return launch_tile_shape(a, epi, p.tile, st);
+}
+
+void stream_plan_report(int kind, int K, int N, int M, bool scratch, int* plan)
+{
+    LinearWeight w{};
+    w.type = 1, w.K = K, w.N = N, w.packed = &w;  // (as loaded)
+    if (kind == 2 && !f16_stream_supported(w, M)) {
+        std::fill(plan, plan + 5, 0);
+        return;
+    }
+    const size_t     ws = scratch ? (kind == 2 ? ~(size_t)0 : kStreamWsBytes) : 0;
+    const int        tickets = scratch ? (kind == 2 ? 1 << 30 : kStreamTickets) : 0;
+    const StreamPlan p = kind == 2 ? stream_plan(K / 32, N, M, 1, false, 2, false, ws, tickets, 0, true, 0, true) :
+                                     stream_plan((K + 31) / 32 * (kind == 1 ? 2 : 1), (N + 127) / 128 * 128, M, 1, false, kind == 1 ? 4 : 2, false, ws, tickets, 0, false, 0, true);
+    const int out[5] = {p.skinny ? (p.narrow ? 1 : 2) : 3 + p.tile, p.skinny ? (p.narrow ? 1 : p.cw) : 0, p.skinny ? p.mt : 0, p.skinny ? p.splits : 1, p.skinny ? 0 : p.cut};
+    std::copy(out, out + 5, plan);
 }
 
 }  // namespace tmk

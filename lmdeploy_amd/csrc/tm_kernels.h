@@ -231,6 +231,7 @@ int launch_linear(const LinearWeight& w, const half_t* x, int ldx, half_t* y, in
 // ---- gemm_f16.hip: fp16 linears on the kernels of gemm_stream.h ---------------------------------------------------
 bool f16_stream_supported(const LinearWeight& w, int M);
 int  f16_stream_splits(const LinearWeight& w, int M);
+void stream_plan_report(int kind, int K, int N, int M, bool scratch, int* plan);  // (tm_debug_stream_plan)
 int  launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int splits, float* workspace,
                        unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st, const F16KvSink* kv = nullptr, bool* kv_done = nullptr);
 

@@ -682,3 +682,17 @@ def test_bench_gemm_family_roofline_arithmetic():
     # one rank of TP = 8: every linear is an eighth (column- / row-parallel), the family with it
     per8, tot8 = bench.gemm_family_bytes(bench.LLAMA3_8B, 8)
     assert abs(tot8 * 8 - tot) < 1 and per8['w_qkv'] * 8 == per['w_qkv']
+
+
+def stream_plan(kind, K, N, M, scratch=1):
+    """(kernel, column tiles a workgroup, row tiles, slices of k, columns of a first launch) of a plain product: tm_debug_stream_plan"""
+    v = (_ffi.C.c_int * 5)()
+    _ffi.check(_ffi.load().tm_debug_stream_plan(kind, K, N, M, scratch, v))
+    return tuple(v)
+
+
+def test_line_between_the_kernels_of_fp16_products():
+    """the general kernel where a round of its 64 x 128 workgroups, or beyond 40 rows the last of several, is at least three quarters full; the weight stream elsewhere"""
+    for wgs, few, many in ((192, 2, 2), (216, 0, 0), (256, 0, 0), (288, 2, 2), (384, 2, 2), (448, 2, 0), (512, 2, 0), (576, 2, 2), (640, 2, 2), (723, 2, 0), (1002, 2, 0), (1188, 2, 0)):
+        for rows, kernel in ((17, few), (40, few), (41, many), (64, many)):
+            assert stream_plan(2, 4096, 128 * wgs, rows)[0] == kernel, (wgs, rows)
