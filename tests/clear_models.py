@@ -29,7 +29,8 @@ def weights(cfg, seed, quantized=True, attention=False):
             g = np.linalg.qr(rng.standard_normal((cfg.hidden, cfg.moe_experts)))[0].astype(f32)
             L['moe_gate'] = g.astype(f16)
             choice = np.argsort(rng.random((cfg.vocab, cfg.moe_experts)), axis=1)[:, :cfg.moe_top_k]
-            emb += 0.3 * g.T[choice].sum(axis=1) / np.sqrt(cfg.layers)
+            share = 0.3 * (1 + 0.08 * np.arange(cfg.moe_top_k) / cfg.moe_top_k)   # clear of the experts not chosen, and none the same
+            emb += np.einsum('k,vkh->vh', share, g.T[choice]).astype(f32) / np.sqrt(cfg.layers)
     w['tok_embeddings'] = emb.astype(f16)
     return w
 

@@ -9,6 +9,7 @@ import torch
 from lmdeploy_amd import _ffi
 from oracle import tm_oracle as o
 from tests.gpu_helpers import dev, host, release_all, st
+from tests.test_gpu_moe_fp8_wide_tiles import near
 
 pytestmark = pytest.mark.gpu
 f16 = np.float16
@@ -32,8 +33,8 @@ def test_row_tiles(tm, cuda, T, skew):
     _ffi.check(tm.tm_moe_create(_ffi.C.byref(h), H, I, E, k, 2, 1, 1.0))
     _ffi.check(tm.tm_moe_set_gate(h, dev(gate).data_ptr(), st()))
     for e in range(E):
-        w1, w3 = ((rng.standard_normal((H, I)) * (0.1 / math.sqrt(H))).astype(f16) for _ in range(2))
-        w2 = (rng.standard_normal((I, H)) * (0.1 / math.sqrt(I))).astype(f16)
+        w1, w3 = ((rng.standard_normal((H, I)) / math.sqrt(H)).astype(f16) for _ in range(2))
+        w2 = (2 * rng.standard_normal((I, H)) / math.sqrt(I)).astype(f16)
         (q1, s1), (q3, s3), (q2, s2) = (o.fp8_quantize_blockwise(w) for w in (w1, w3, w2))
         q13, s13 = o.interleave_w1w3(q1, q3), np.concatenate([s1, s3], axis=1)
         experts.append(((q13, s13), (q2, s2)))
@@ -47,9 +48,10 @@ def test_row_tiles(tm, cuda, T, skew):
     ref, ref_ids, ref_w = o.moe_ffn_fp8(x, gate, experts, k)
     assert np.array_equal(host(ids), ref_ids)
     assert np.abs(host(wts) - ref_w).max() <= 1e-5
-    # an fp32 sum in another order can move an fp16 unit of a gated row and with it an e4m3 code (2^-3 relative) of one of 640 channels
-    err, ref = np.abs(host(out).astype(np.float32) - ref.astype(np.float32)), np.abs(ref.astype(np.float32))
-    assert (err <= 4e-3 + 2.0**-6 * ref).all(), err.max()
+    # (as near says; results of order one, so that nothing, a row's neighbour and a 32-column group's neighbour lie outside)
+    ref = ref.astype(np.float32)
+    assert np.abs(ref).max() > 1 and not near(0 * ref, ref) and not near(np.roll(ref, 32, axis=1), ref) and (T == 1 or not near(np.roll(ref, 1, axis=0), ref))
+    assert near(host(out).astype(np.float32), ref)
     _ffi.check(tm.tm_moe_destroy(h))
 
 
@@ -62,8 +64,8 @@ def test_tiles_of_the_measured_dispatch(tm, cuda, tmp_path):
     _ffi.check(tm.tm_moe_create(_ffi.C.byref(h), H, I, E, k, 2, 1, 1.0))
     _ffi.check(tm.tm_moe_set_gate(h, dev(gate).data_ptr(), st()))
     for e in range(E):
-        w1, w3 = ((rng.standard_normal((H, I)) * (0.1 / math.sqrt(H))).astype(f16) for _ in range(2))
-        (q1, s1), (q3, s3), (q2, s2) = (o.fp8_quantize_blockwise(w) for w in (w1, w3, (rng.standard_normal((I, H)) * (0.1 / math.sqrt(I))).astype(f16)))
+        w1, w3 = ((rng.standard_normal((H, I)) / math.sqrt(H)).astype(f16) for _ in range(2))
+        (q1, s1), (q3, s3), (q2, s2) = (o.fp8_quantize_blockwise(w) for w in (w1, w3, (2 * rng.standard_normal((I, H)) / math.sqrt(I)).astype(f16)))
         q13, s13 = o.interleave_w1w3(q1, q3), np.concatenate([s1, s3], axis=1)
         experts.append(((q13, s13), (q2, s2)))
         _ffi.check(tm.tm_moe_set_expert(h, e, dev(q13).data_ptr(), dev(s13).data_ptr(), None, dev(q2).data_ptr(), dev(s2).data_ptr(), None, st()))
@@ -74,5 +76,5 @@ def test_tiles_of_the_measured_dispatch(tm, cuda, tmp_path):
         _ffi.check(tm.tm_gemm_import(str(table).encode()))
         out = torch.zeros((T, H), dtype=torch.float16, device='cuda')
         _ffi.check(tm.tm_moe_forward(h, out.data_ptr(), dev(x).data_ptr(), T, ws.data_ptr(), None, None, st()))
-        assert (np.abs(host(out).astype(np.float32) - ref) <= 4e-3 + 2.0**-6 * np.abs(ref)).all()
+        assert near(host(out).astype(np.float32), ref), rows
     _ffi.check(tm.tm_moe_destroy(h))

@@ -7,6 +7,7 @@ import pytest
 from lmdeploy_amd.turbomind.engine import Engine
 from lmdeploy_amd.turbomind.loader import export_weights
 from oracle import tm_oracle as o
+from tests import clear_models
 from tests import febivik_oracle as fo
 from tests.test_gpu_febivik import TOL, engine
 
@@ -30,12 +31,13 @@ def test_layer_norm(tmp_path, cuda, width, top, shared):
     eng.close()
 
 
-@pytest.mark.parametrize('hidden', [256, 4352])
-def test_rms_norm(cuda, hidden):
+@pytest.mark.parametrize('hidden,top', [(256, 2), (4352, 2), (256, 3), (384, 1)])
+def test_rms_norm(cuda, hidden, top):
+    """two layers, every expert chosen (the second layer's choices cannot turn): the sum with weights, the stream it joins and its norm for the next layer"""
     cfg = o.ModelConfig(hidden=hidden, layers=2, q_heads=2, kv_heads=1, head_dim=128, inter=128, vocab=256, kv_bits=8, rope=o.RopeParam(128, 10000.0),
-                        moe_experts=4, moe_top_k=2, weight_format='fp8', moe_fp8_act=True)
-    w = o.make_synthetic_weights(cfg, seed=hidden)
-    eng = Engine.from_model_config(cfg, weight_type=2, max_batch_size=2, session_len=128, quant_policy=8, max_prefill_token_num=128)
+                        moe_experts=top, moe_top_k=top, weight_format='u4')
+    w = clear_models.weights(cfg, hidden)
+    eng = Engine.from_model_config(cfg, weight_type=0, max_batch_size=2, session_len=128, quant_policy=8, max_prefill_token_num=128)
     eng.load_weights(export_weights(cfg, w))
     eng.start()
     rng = np.random.default_rng(hidden)
@@ -46,8 +48,17 @@ def test_rms_norm(cuda, hidden):
         eng.decode(1)
         got.append(eng.fetch_logits())
     toks = eng.fetch()
-    model = o.OracleModel(cfg, w, batch=2, max_ctx=128)
-    ref = [model.forward(prompts)[1]] + [model.forward([[int(t)] for t in toks[:, s]])[1] for s in range(2)]
-    # the bound of the engine's other fp8 models: an fp32 sum in another order turns single e4m3 codes of the activations
-    assert max(np.abs(a.astype(np.float32) - b.astype(np.float32)).max() for a, b in zip(got, ref)) <= 3e-2
     eng.close()
+    ref = clear_models.forced(cfg, w, prompts, toks, 2)
+    bound = 2.0**-7   # a dozen roundings to fp16
+    ffn, pick = o.moe_ffn, o.moe_gate
+    try:   # no sum; its channels moved by one; another token's rows; equal weights
+        for wrong in (lambda d: 0 * d, lambda d: np.roll(d, 1, axis=1), lambda d: np.roll(d, 1, axis=0)):
+            o.moe_ffn = lambda *a: (lambda d, i, t: (wrong(d), i, t))(*ffn(*a))
+            assert clear_models.differ(clear_models.forced(cfg, w, prompts, toks, 2), ref) > 2 * bound
+        if top > 1:
+            o.moe_ffn, o.moe_gate = ffn, lambda *a: (lambda z, i, t: (z, i, 0 * t + 1 / top))(*pick(*a))
+            assert clear_models.differ(clear_models.forced(cfg, w, prompts, toks, 2), ref) > 2 * bound
+    finally:
+        o.moe_ffn, o.moe_gate = ffn, pick
+    assert clear_models.differ(got, ref) <= bound
