@@ -14,7 +14,7 @@
 //   * rows AND raw weight units come by LDS-DMA (a unit goes to the wave that owns its columns): one counted queue, nothing staged in registers.
 // A step is 32 k: 64 MFMAs a wave, 16 row fragments read a whole step ahead, the next step's four weight fragments dequantised three or four operations per four
 // MFMAs; four row stages of 16 KB, two slots of weight units; one barrier a step.
-// 8192 rows, MI355X: (K, N) = (4096, 28672) gated 1508 us = 1.28 PFLOP/s, (14336, 4096) 700 = 1.37, (4096, 6144) 319, (4096, 4096) 218; tiles of 128 x 512 on
+// 8192 rows, MI355X, one launch after another: (K, N) = (4096, 28672) gated 1508 us = 1.28 PFLOP/s (between a model's other kernels 1530 - 1670), (14336, 4096) 700 = 1.37, (4096, 6144) 319, (4096, 4096) 218; tiles of 128 x 512 on
 // 32x32x16 1638, 779, 366 and 247 on the same box; 256 x 256 tiles that dequantised through LDS for 32x32x16 were no faster than those.
 // fp16 results leave in 16-byte pieces (eight and four bytes a lane: (2048, 16384) gated, 4096 rows 272 us against 258).
 // grid = (ceil(N / 256), splits, ceil(M / 256)); epilogue straight from the accumulators (fp16, gated SiLU, fp32 slabs).
