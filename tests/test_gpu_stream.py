@@ -254,3 +254,27 @@ def test_turned_tiles_in_slices(cuda, dtype):
         for s in sess:
             eng.close_session(s)
     eng.close()
+
+
+@pytest.mark.parametrize('dtype,width', [('float32', 2048), ('bfloat16', 4096)])
+def test_turned_items(tmp_path, cuda, dtype, width):
+    """the same in the first product of a mixture's experts: each item's tiles begin where their own columns say, whatever item it is; prompts and decode steps"""
+    cfg = fo.make_config(width, 97, [fo.lightning_layer(2, 8, 8, [0.9, 0.9], fo.moe(3, 2 if dtype == 'float32' else 3, 600, 1.0, 0))])
+    w = fo.random_weights(cfg, 11)
+    folder = str(tmp_path / 'm')
+    fo.write_checkpoint(folder, cfg, w)
+    rng = np.random.default_rng(2)
+    reqs = [rng.integers(0, 97, 132).tolist() for _ in range(2)]
+    eng = engine(folder, dtype)
+    sess = [eng.open_session() for _ in reqs]
+    got = [eng.step_tokens([(s, r[:130], [63, 129]) for s, r in zip(sess, reqs)]).reshape(2, 2, -1)]
+    got += [eng.step_tokens([(s, r[i:i + 1], [0]) for s, r in zip(sess, reqs)]).reshape(2, 1, -1) for i in (130, 131)]
+    ref = np.stack([fo.forward(cfg, w, r)[[63, 129, 130, 131]] for r in reqs])
+    assert rel_err_febivik(np.concatenate(got, axis=1), ref) <= TOL[dtype]
+    bad = dict(w)                    # one group of columns that takes its steps from another place than its rows do
+    for e in range(3):
+        bad[f'l0.mlp.e{e}.up'] = m = np.array(w[f'l0.mlp.e{e}.up'])
+        m[256:512] = np.roll(m[256:512], 128, axis=1)
+    wrong = np.stack([fo.forward(cfg, bad, r)[[63, 129, 130, 131]] for r in reqs])
+    assert rel_err_febivik(wrong, ref) > 2 * TOL[dtype]
+    eng.close()
