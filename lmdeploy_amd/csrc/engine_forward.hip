@@ -126,6 +126,35 @@ static int linear_plain(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, 
     return launch_linear(l.w, x, ldx, y, ldy, M, gated, cfg, e->d_gemm_ws, false, nullptr, e->stream);
 }
 
+// A decode step of a few rows, dense fp16 layers: a product that closes a residual block adds to the residual stream itself, and the product behind it makes the norm
+// of its rows (gemm_rows.h): no norm launch between them.  The first has to have whole sums: one slice of k, or slices that meet inside its launch.  8 sequences of
+// InternLM2-1.8B's layer: output product 4.6 -> 4.8 us, norm 3.1 -> 0, gate / up 12.2 -> 12.1; down product, whose seven slices now meet, 7.4 -> 10.4, norm 4.4 -> 0,
+// [q | k | v] 6.0 -> 5.5.  A linear that a measured table gives to gemm_kernel keeps its launches.
+static bool adds_to_resid(const tm_engine* e, const LinearWeight& w, int M)
+{
+    if (M > 16 || e->hidden % 4 || !f16_stream_supported(w, M)) {
+        return false;
+    }
+    const GemmConfig cfg = gemm_pick_config(w, M);
+    return cfg.f16_stream && (cfg.splits <= 1 || gemm_workspace_bytes(M, w.N, cfg.splits) > e->gemm_ws_bytes || (w.N + 63) / 64 <= e->n_tickets);
+}
+
+static bool norm_in_product(const tm_engine* e, const LinearSlots& first, const LinearSlots& second, int M)
+{
+    return !e->use_comm && !e->p2p_ready && f16_norm_rows_supported(second.w, M) && gemm_pick_config(second.w, M).f16_stream && adds_to_resid(e, first.w, M);
+}
+
+static int linear_residual(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, int M)
+{
+    GemmConfig cfg = gemm_pick_config(l.w, M);
+    int        slabs;
+    if (gemm_workspace_bytes(M, l.w.N, cfg.splits) > e->gemm_ws_bytes) {
+        cfg.splits = 1;
+    }
+    return launch_f16_stream(l.w, x, ldx, e->d_resid, e->hidden, M, false, cfg.splits, e->d_gemm_ws, e->d_tickets, e->n_tickets, false, &slabs, e->stream, nullptr, nullptr,
+                             true);
+}
+
 // Tensor-parallel prefill forward, dense layer, from the attention output to the next layer's QKV projection, as two row halves
 // A = [0, Ma), B = [Ma, M): every operator here is row-wise, so a half's all-reduce (RCCL on the side stream, engine_comm.hip) runs
 // under the other half's GEMMs on the engine stream --
@@ -483,6 +512,7 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
         TM_TRY(forward_layers_two_microbatches(e, M, nseq, max_q_len, max_k_len, kflat_stride, scale_log2));
     }
     bool        qkv_done = false;  // the previous layer's two-halves tail already projected this layer's QKV
+    bool        norm_in_qkv = false;  // the residual stream is complete, its norm is this layer's QKV product's
     int         ss_tiles   = 0;  // > 0: d_x holds r . g of a folded producer, d_ss its sums of squares (the next GEMM applies the row factor)
     for (int li = 0; li < (two_mb ? 0 : m.layers); ++li) {
         Layer& L = e->layers[li];
@@ -493,7 +523,15 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
         // applies RoPE and quantises/stores the new K/V itself -> no splitk_reduce, no kv_rope_store launch
         const bool fuse_qkv = decode && e->fuse_qkv;
         int        qkv_slabs = 1;
-        if (fold) {
+        if (norm_in_qkv) {
+            const F16KvSink sink{e->d_k_len, e->d_rope, e->rope_max_pos, e->q_heads, cv};
+            const bool      store = !fuse_qkv && cv.layout.bits == 16 && e->D == 128;
+            TM_PROF(P_GEMM_QKV, TM_TRY(launch_f16_norm_rows(L.qkv.w, e->d_resid, L.attn_norm, m.rms_eps, e->d_qkv, e->qkv_n, M, false, st, store ? &sink : nullptr)));
+            if (!fuse_qkv && !store) {
+                TM_PROF(P_KV_STORE, TM_TRY(launch_kv_rope_store(qkv_p, e->q_heads, e->d_cu_q, e->d_k_len, nseq, M, e->d_rope, e->rope_max_pos, cv, st)));
+            }
+        }
+        else if (fold) {
             TM_PROF(P_GEMM_QKV, TM_TRY(linear_fold_consume(e, L.qkv, e->d_x, e->hidden, e->d_qkv, e->qkv_n, M, false, ss_tiles, fuse_qkv, &qkv_slabs)));
             ss_tiles = 0;
             if (!fuse_qkv) {
@@ -638,7 +676,14 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
             }
             continue;
         }
-        TM_TRY(linear_residual_norm(e, L.wo, e->d_attn, e->q_heads * e->D, M, L.ffn_norm, P_GEMM_O));
+        const bool norm_in = decode && !L.is_moe && norm_in_product(e, L.wo, L.w13, M);
+        if (norm_in) {
+            TM_PROF(P_GEMM_O, TM_TRY(linear_residual(e, L.wo, e->d_attn, e->q_heads * e->D, M)));
+            TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_f16_norm_rows(L.w13.w, e->d_resid, L.ffn_norm, m.rms_eps, e->d_act, e->inter, M, true, st)));
+        }
+        else {
+            TM_TRY(linear_residual_norm(e, L.wo, e->d_attn, e->q_heads * e->D, M, L.ffn_norm, P_GEMM_O));
+        }
         if (L.is_moe) {
             TM_TRY(moe_rows(e, L.moe, e->d_x, e->d_x, M, next_norm));
             if (e->use_comm || e->p2p_ready) {  // (all-reduce +) residual + RMSNorm as for the dense FFN
@@ -646,8 +691,16 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
             }
             continue;
         }
-        TM_PROF(P_GEMM_GATE_UP, TM_TRY(linear_plain(e, L.w13, e->d_x, e->hidden, e->d_act, e->inter, M, true)));
-        TM_TRY(linear_residual_norm(e, L.w2, e->d_act, e->inter, M, next_norm, P_GEMM_DOWN));
+        if (!norm_in) {
+            TM_PROF(P_GEMM_GATE_UP, TM_TRY(linear_plain(e, L.w13, e->d_x, e->hidden, e->d_act, e->inter, M, true)));
+        }
+        norm_in_qkv = decode && li + 1 < m.layers && norm_in_product(e, L.w2, e->layers[li + 1].qkv, M);
+        if (norm_in_qkv) {
+            TM_PROF(P_GEMM_DOWN, TM_TRY(linear_residual(e, L.w2, e->d_act, e->inter, M)));
+        }
+        else {
+            TM_TRY(linear_residual_norm(e, L.w2, e->d_act, e->inter, M, next_norm, P_GEMM_DOWN));
+        }
     }
     // last-token hidden states -> logits -> next ids, for `n` sequences whose logits / next ids land in the batch slots
     // [slot, slot + n): hx = their hidden rows, ids / cu_q (nullptr: one token per sequence) / ntok = the tokens this forward

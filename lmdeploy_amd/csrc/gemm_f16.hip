@@ -7,7 +7,7 @@
 //
 // Weights from HBM, MI355X, here | gemm_kernel: 8 rows (2048, 4096) 7.2 | 13.0 us, (8192, 2048) 14.1 | 43.7, (2048, 16384) gated 15.7 | 17.2; 64 rows (14336,
 // 4096) 33 | 101; 2664 rows (2048, 16384) gated 215 | 501; 8192 rows (4096, 28672) gated 1702 | 5390 us (1.13 PFLOP/s), (14336, 4096) 810 | 2159 (1.19).
-#include "gemm_stream.h"
+#include "gemm_rows.h"
 #include "tm_kernels.h"
 #include <algorithm>
 
@@ -111,6 +111,22 @@ struct F16EpiKv: F16Epi {
     }
 };
 
+// The same for a product that closes a residual block: y += h(acc), in fp16 (residual_rmsnorm's addition)
+struct F16EpiAdd: F16Epi {
+    template<int NT>
+    __device__ __forceinline__ void rows(const StreamArgs& a, const F16Item&, int m, int n, const floatx4 (&acc)[NT]) const
+    {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int c = n + 16 * j;
+            if (c < a.N) {
+                half4_t* y = (half4_t*)((half_t*)a.y + (size_t)m * a.ldy + c);
+                *y         = *y + half4_t{(half_t)acc[j][0], (half_t)acc[j][1], (half_t)acc[j][2], (half_t)acc[j][3]};
+            }
+        }
+    }
+};
+
 // Where gemm_kernel is still the better one: its workgroups of 64 rows x 128 columns take the weights straight into registers and read x half as often as 64
 // columns do, so it wins where about one round of them keeps the CUs busy.  us, gemm_kernel | here, weights from HBM:
 //   up to 64 rows, 193 ... 256 workgroups: (K, N) = (4096, 28672) gated 8 rows 35.4 | 34.7, 32 rows 35.5 | 38.5, 64 rows 40 | 44, (5120, 27648) gated 8 rows
@@ -179,7 +195,8 @@ static int launch_tile_shape(const StreamArgs& a, const F16Epi& epi, int tile, h
 // splits: slices of k the caller's workspace holds slabs for (1: none).  With slices, fp32 slabs [slices][M][N] are left in the workspace and *slabs says
 // how many (defer, or no arrival counters), or they meet inside the launch (tickets)
 int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int splits, float* workspace,
-                      unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st, const F16KvSink* kv, bool* kv_done)
+                      unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st, const F16KvSink* kv, bool* kv_done,
+                      bool add)
 {
     TM_REQUIRE(f16_stream_supported(w, M), "fp16 linear: image");
     const bool       slice = splits > 1 && workspace;
@@ -206,8 +223,14 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
             *kv_done = true;
             return p.mt == 1 ? launch_skinny<1>(a, ek, p, st) : p.mt == 2 ? launch_skinny<2>(a, ek, p, st) : launch_skinny<4>(a, ek, p, st);
         }
+        if (add) {
+            TM_REQUIRE(*slabs == 1 && !gated && ldy % 4 == 0 && (uintptr_t)y % 8 == 0, "fp16 linear: a residual addition");
+            const F16EpiAdd ea{epi};
+            return p.mt == 1 ? launch_skinny<1>(a, ea, p, st) : p.mt == 2 ? launch_skinny<2>(a, ea, p, st) : launch_skinny<4>(a, ea, p, st);
+        }
         return p.mt == 1 ? launch_skinny<1>(a, epi, p, st) : p.mt == 2 ? launch_skinny<2>(a, epi, p, st) : launch_skinny<4>(a, epi, p, st);
     }
+    TM_REQUIRE(!add, "fp16 linear: a residual addition");
     if (p.cut > 0) {
         StreamArgs rest = a;
         rest.col0       = p.cut;
@@ -218,6 +241,72 @@ int launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y
         return launch_tile_shape(rest, epi, p.tile2, st);
     }
     return launch_tile_shape(a, epi, p.tile, st);
+}
+
+// ---- few rows that come with their norm ------------------------------------------------------------------------------------------------
+template<int RPW, int P, int CW, int KP, int R, class Epi>
+static int launch_rows(const StreamArgs& a, const Epi& epi, const half_t* resid, const half_t* norm_w, float eps, int team, hipStream_t st)
+{
+    const auto kernel = stream_rows_kernel<half_t, Epi, NormRows<RPW, P>, CW, KP, R>;
+    const int  lds    = stream_rows_lds(a.M, a.steps, CW, KP);
+    if (const int rc = ensure_dynamic_lds((const void*)kernel, lds)) {
+        return rc;
+    }
+    kernel<<<dim3((a.tiles + CW - 1) / CW), CW * KP * 64, lds, st>>>(a, epi, NormRows<RPW, P>{resid, norm_w, eps, team});
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+bool f16_norm_rows_supported(const LinearWeight& w, int M)
+{
+    return w.type == 1 && w.packed && (size_t)w.K * w.N * 2 < ((size_t)1 << 31) && w.K % 512 == 0 && M >= 1 && (M <= 8 ? w.K <= 4096 : M <= 16 && w.K <= 2048);
+}
+
+template<int CW, int KP, int R, class Epi>
+static int launch_rows_of(const StreamArgs& a, const Epi& epi, const half_t* resid, const half_t* norm_w, float eps, hipStream_t st)
+{
+    const int waves = CW * KP;
+    int       teams = 1;
+    while (teams < waves && teams < a.M) {
+        teams *= 2;
+    }
+    const int team = waves / teams, p = (a.steps / 16 + team - 1) / team, rpw = (a.M + teams - 1) / teams;
+    TM_REQUIRE(rpw == 1 ? p <= 8 : rpw == 2 && p <= 4, "fp16 linear with its norm: rows");
+    return rpw == 2 ? launch_rows<2, 4, CW, KP, R>(a, epi, resid, norm_w, eps, team, st) :
+           p <= 1   ? launch_rows<1, 1, CW, KP, R>(a, epi, resid, norm_w, eps, team, st) :
+           p <= 2   ? launch_rows<1, 2, CW, KP, R>(a, epi, resid, norm_w, eps, team, st) :
+           p <= 4   ? launch_rows<1, 4, CW, KP, R>(a, epi, resid, norm_w, eps, team, st) :
+                      launch_rows<1, 8, CW, KP, R>(a, epi, resid, norm_w, eps, team, st);
+}
+
+// us with the norm in the product | as a launch of its own ahead of the better of the other kernels (graph replays, weights from HBM): K = 2048, 8 rows, N = 2048 6.4 |
+// 8.5, 4096 7.0 | 9.1, 6144 8.6 | 11.2, 10240 11.3 | 12.7, 16384 13.7 | 15.5, 28672 21.3 | 22.8; one row, 16384 13.1 | 14.8; 16 rows, 4096 8.1 | 9.8, 16384 14.8 | 15.7;
+// K = 1024, 8 rows, 4096 6.2 | 7.7; K = 4096, 8 rows, 4096 10.5 | 11.4, 16384 24.1 | 24.3; one row 22.5 | 24.4.  One column tile a workgroup is best while one round of them
+// fills the CUs (8 rows, K = 2048, N = 4096: 7.0, two tiles 8.2), two up to 512 tiles (N = 8192: 10.1 and 9.3, four 10.8); beyond, four waves that
+// take a column tile each where their rows leave them time for it (one row, N = 16384: 13.1, eight waves 13.6; 16 rows: 15.6 and 14.8)
+template<class Epi>
+static int launch_norm_rows(const StreamArgs& a, const Epi& epi, const half_t* resid, const half_t* norm_w, float eps, hipStream_t st)
+{
+    if (a.tiles <= 256) {
+        return launch_rows_of<1, 8, 8>(a, epi, resid, norm_w, eps, st);
+    }
+    if (a.tiles <= 512) {
+        return launch_rows_of<2, 4, 8>(a, epi, resid, norm_w, eps, st);
+    }
+    return a.M <= 4 ? launch_rows_of<4, 1, 16>(a, epi, resid, norm_w, eps, st) : launch_rows_of<4, 2, 8>(a, epi, resid, norm_w, eps, st);
+}
+
+int launch_f16_norm_rows(const LinearWeight& w, const half_t* resid, const half_t* norm_w, float eps, half_t* y, int ldy, int M, bool gated, hipStream_t st,
+                         const F16KvSink* kv)
+{
+    TM_REQUIRE(f16_norm_rows_supported(w, M) && resid && norm_w && y, "fp16 linear with its norm");
+    TM_REQUIRE(!kv || (!gated && ldy % 4 == 0 && (uintptr_t)y % 8 == 0), "fp16 linear with its norm: cache store");
+    StreamArgs a{};
+    a.w = (const char*)w.packed, a.tiles = w.N / 16, a.steps = w.K / 32;
+    a.w_tile = 4096, a.w_quad = (int64_t)a.tiles * 4096;
+    a.y = y, a.ldy = ldy, a.M = M, a.N = w.N;
+    const F16Epi epi{gated ? 1 : 0, gated ? (ldy % 2 == 0 && (uintptr_t)y % 4 == 0) : (ldy % 4 == 0 && (uintptr_t)y % 8 == 0)};
+    return kv ? launch_norm_rows(a, F16EpiKv{epi, *kv}, resid, norm_w, eps, st) : launch_norm_rows(a, epi, resid, norm_w, eps, st);
 }
 
 void stream_plan_report(int kind, int K, int N, int M, bool scratch, int* plan)

@@ -233,7 +233,12 @@ bool f16_stream_supported(const LinearWeight& w, int M);
 int  f16_stream_splits(const LinearWeight& w, int M);
 void stream_plan_report(int kind, int K, int N, int M, bool scratch, int* plan);  // (tm_debug_stream_plan)
 int  launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int splits, float* workspace,
-                       unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st, const F16KvSink* kv = nullptr, bool* kv_done = nullptr);
+                       unsigned* tickets, int ticket_count, bool defer, int* slabs, hipStream_t st, const F16KvSink* kv = nullptr, bool* kv_done = nullptr,
+                       bool add = false /* y += x . W, rounded to fp16 first (few rows, one slab) */);
+// few rows with their norm: y = rmsnorm(resid) . W
+bool f16_norm_rows_supported(const LinearWeight& w, int M);
+int  launch_f16_norm_rows(const LinearWeight& w, const half_t* resid, const half_t* norm_w, float eps, half_t* y, int ldy, int M, bool gated, hipStream_t st,
+                          const F16KvSink* kv = nullptr);
 
 // ---- gemm_decode.hip: W4A16 decode GEMM (M <= 64), 32x32x16 MFMA, 16 waves per CU ------------------------------
 size_t p32_bytes(int K, int N);
