@@ -316,10 +316,10 @@ int tm_linear_forward(const tm_linear* w, const void* x, int ldx, void* y, int l
         TM_REQUIRE(dec32_supported(w->w, M), "decode kernel: u4 weights, N % 32 == 0");
         cfg.d32_shape = waves & 0xff;
         TM_REQUIRE((cfg.d32_shape >= 6 && cfg.d32_shape <= 9) || (cfg.d32_shape <= 5 && (cfg.d32_shape >= 4) == (M > 64))
-                       || (cfg.d32_shape == kShapeWide2 && M <= 64)
+                       || (cfg.d32_shape == kShapeWide2 && M <= 64) || (cfg.d32_shape == kShapeRows && M <= 16)
                        || (cfg.d32_shape == kShapeLC && M <= 64) || ((cfg.d32_shape == kShapePre256 || cfg.d32_shape == kShapeF16) && M > 64)
                        || (dec32_is_merge_shape(cfg.d32_shape) && M <= 64),
-                   "P32 kernel shape 0..3 / 11 (M <= 64), 4 / 5 / 12 (M > 64), 6..9 (32-row blocks, any M) or 16 + (0..3 | 6..9) "
+                   "P32 kernel shape 0..3 / 11 (M <= 64), 14 (M <= 16), 4 / 5 / 12 (M > 64), 6..9 (32-row blocks, any M) or 16 + (0..3 | 6..9) "
                    "(M <= 64: split-K merged inside the launch)");
         waves = 0;
     }
@@ -349,6 +349,9 @@ int tm_linear_residual_norm(const tm_linear* w, const void* x, int ldx, void* y,
     TM_REQUIRE(w && x && y && resid && norm_w && workspace, "null pointer");
     const int N = w->w.N;
     GemmConfig cfg = gemm_pick_config(w->w, M);
+    if (cfg.d32_shape == kShapeRows) {  // (its residual stream is tm_linear_fold_produce's, to the bit: the tiles that both have)
+        dec32_pick_plain(w->w, M, &cfg.d32_shape, &cfg.splits, true);
+    }
     if (shape >= 0) {
         TM_REQUIRE(dec32_supported(w->w, M) && (shape <= 3 || (shape >= 6 && shape <= 10) || shape == kShapeLC)
                        && (M <= 64 || (M <= kFoldMaxRows && shape >= 6 && shape <= 9)),
@@ -980,7 +983,7 @@ int tm_debug_pick_tiling(int K, int N, int M, int use_table, int* shape, int* sp
     w.N    = N;
     w.role = (use_table >> 8) & 0xf;  // 0 any, 1 w_qkv, 2 wo, 3 w1w3, 4 w2: the measured table is keyed (role, K, N, M)
     TM_REQUIRE(w.role <= 4, "role 0 .. 4 in bits 8 .. 11 of use_table");
-    (use_table & 2 ? dec32_pick_plain : dec32_pick_ex)(w, M, shape, splits, (use_table & 1) != 0);
+    (use_table & 4 ? dec32_pick_launch : use_table & 2 ? dec32_pick_plain : dec32_pick_ex)(w, M, shape, splits, (use_table & 1) != 0);
     return 0;
 }
 

@@ -73,7 +73,7 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
             dec32_pick_ex(w0, M, &hs, &hp, false);
         }
         else {
-            dec32_pick_plain(w0, M, &hs, &hp, false);
+            dec32_pick_launch(w0, M, &hs, &hp, false);
         }
         int       cand[96][2];
         int       nc = dec32_candidates(w0, M, cand, 95);

@@ -1410,7 +1410,7 @@ int dec32_table_import(const char* path)
         const bool lc  = shape == kShapeLC && M <= 64;
         const bool p256 = (shape == kShapePre256 || (shape == kShapeF16 && splits == 1)) && M > 64;  // what launch_linear_dec32 accepts (the tuner only proposes them for M, N >= 256)
         const bool mrg = dec32_is_merge_shape(shape) && M <= 64 && splits >= 2;  // in-launch merged split-K (decode batches only)
-        const bool w2k = shape == kShapeWide2 && M <= 64;
+        const bool w2k = (shape == kShapeWide2 && M <= 64) || (shape == kShapeRows && M <= 16);
         if (K > 0 && N > 0 && M > 0 && M == dec32_m_bucket(M) && shape >= 0 && (shape <= 9 || lc || p256 || mrg || w2k) && splits >= 1 && splits <= 16
             && (big ? shape >= 4 : (shape != 4 && shape != 5)) && !(shape == 5 && N < 512) && K % 128 == 0 && N % 32 == 0) {
             dec32_table_set(K, N, M, shape, splits, role);
@@ -1503,6 +1503,13 @@ int dec32_candidates(const LinearWeight& w, int M, int (*out)[2], int cap)
                 out[n][1] = s;
                 ++n;
             }
+        }
+    }
+    for (const int s : {1, 2, 4, 8}) {  // gemm_w4_rows.hip
+        if (M <= 16 && (s == 1 || KB / s >= 8) && w4_rows_supported(w, M, s) && n < cap) {
+            out[n][0] = kShapeRows;
+            out[n][1] = s;
+            ++n;
         }
     }
     if (M >= 1024 && M <= 8192 && w.N >= 256 && w.image16 != nullptr && n < cap) {  // gemm_prefill_f16.hip: the resident fp16 image, no split-K
@@ -1684,6 +1691,20 @@ void dec32_pick_plain(const LinearWeight& w, int M, int* shape_out, int* splits_
     }
 }
 
+// What a launch takes: a measured line, or the row kernel of up to 16 rows (gemm_w4_rows.hip; a tiling forced from outside keeps the tiles above), or dec32_pick_plain's tiling
+void dec32_pick_launch(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table)
+{
+    static const bool forced = env_int2("TM_D32_SHAPE", -1) >= 0 || env_int2("TM_D32_SPLITS", 0) > 0;
+    if (use_table && dec32_table_get(w.K, w.N, dec32_m_bucket(M), shape_out, splits_out, w.role)) {
+        return;
+    }
+    if (!forced && w4_rows_plan(w, M, splits_out)) {
+        *shape_out = kShapeRows;
+        return;
+    }
+    dec32_pick_plain(w, M, shape_out, splits_out, false);
+}
+
 // y / slabs as launch_linear: *slabs_out = number of fp32 slabs written into `workspace` (1 = direct epilogue)
 // (shape, M) pairs a folded launch can run: see launch_linear_dec32
 bool dec32_fold_shape_m(int shape, int M, bool producer)
@@ -1714,6 +1735,14 @@ int launch_linear_dec32(const LinearWeight& w, const half_t* x, int ldx, half_t*
     const bool produce = nf && nf->resid != nullptr;
     const bool consume = nf && nf->ss_in != nullptr;
     bool       merge   = false;
+    if (shape == kShapeRows) {
+        TM_REQUIRE(!produce && !consume && M <= 16, "decode GEMM: shape 14 takes M <= 16 and no folded norm");
+        if (w4_rows_supported(w, M, splits)) {
+            return launch_w4_rows(w, x, ldx, y, ldy, M, gated_silu, splits, workspace, slabs_out, st);
+        }
+        int own;  // (without room for slabs its rows need not fit in LDS)
+        dec32_pick_plain(w, M, &shape, &own, false);
+    }
     if (dec32_is_merge_shape(shape)) {  // split-K merged in the launch (fp16 / gated epilogues); a producer does that anyway
         shape -= kShapeMerge;
         merge = !produce && splits > 1;

@@ -938,7 +938,7 @@ GemmConfig gemm_pick_config(const LinearWeight& w, int M)
 {
     if (dec32_supported(w, M)) {  // decode batch: the weight-streaming kernel of gemm_decode.hip
         GemmConfig cfg{};
-        dec32_pick_plain(w, M, &cfg.d32_shape, &cfg.splits, true);
+        dec32_pick_launch(w, M, &cfg.d32_shape, &cfg.splits, true);
         cfg.nt      = 2;
         cfg.waves   = 16;
         cfg.kphases = 1;

@@ -202,6 +202,8 @@ constexpr int kShapeMerge      = 16;
 // 256 columns x 2 k-phases x 16 waves on 2-k-block stages (gemm_dec32_kernel<MH, 8, 2, 2, 2>): the 256-column decode tile that does not
 // spill (shape 1 = the same wave layout on 4-k-block stages with a 4-deep ring: 60 B / lane of scratch at the 128-register cap)
 constexpr int kShapeWide2      = 10;
+// gemm_w4_rows.hip: up to 16 rows, all of them in LDS (its workgroup shape follows from sizes and slices)
+constexpr int kShapeRows = 14;
 inline bool dec32_is_merge_shape(int shape)
 {
     const int b = shape - kShapeMerge;
@@ -247,6 +249,10 @@ bool   dec32_supported(const LinearWeight& w, int M);
 void   dec32_pick(const LinearWeight& w, int M, int* shape_out, int* splits_out);  // measured table first, then the heuristic
 void   dec32_pick_ex(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table);
 void   dec32_pick_plain(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table);  // ... of a product without a folded norm
+void   dec32_pick_launch(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table);  // ... with up to 16 rows on gemm_w4_rows.hip (kShapeRows)
+bool   w4_rows_supported(const LinearWeight& w, int M, int slices);
+bool   w4_rows_plan(const LinearWeight& w, int M, int* slices);
+int    launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int slices, float* workspace, int* slabs, hipStream_t st);
 // measured dispatch table of the decode linears: key (K, N, M <= 64) -> (shape, splits)
 void   dec32_table_set(int K, int N, int M, int shape, int splits, int role = 0);
 bool   dec32_table_get(int K, int N, int M, int* shape, int* splits, int role = 0);  // the role's entry, else the role-0 entry

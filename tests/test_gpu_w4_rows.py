@@ -1,0 +1,62 @@
+"""GPU test of the W4 products of up to 16 rows that keep their rows in LDS and apply scales and zero points to sums (gemm_w4_rows.hip): its four workgroup shapes, column
+groups and k-blocks that leave waves without work, slices of unequal length, the two ways the row sums are made, plain and gated results, rows with strides -- against
+64-bit results, which it has to be as close to as the kernel that rounds its weights, and the rule that takes it."""
+import numpy as np
+import pytest
+import torch
+
+from lmdeploy_amd import _ffi
+from oracle import tm_oracle as o
+from tests.gpu_helpers import dev, host, release_all, st
+from tests.test_gpu_ops import _QCACHE, _make_linear
+
+pytestmark = pytest.mark.gpu
+ROWS = 14
+
+
+@pytest.fixture(autouse=True)
+def _release():
+    yield
+    release_all()
+
+
+def _run(tm, h, x, N, M, shape, splits, gated=0):
+    cols = N // 2 if gated else N
+    y = torch.full((M + 1, cols + 4), 7.0, dtype=torch.float16, device='cuda')
+    ws = torch.zeros(max(1, tm.tm_linear_workspace(h, M)), dtype=torch.uint8, device='cuda')
+    _ffi.check(tm.tm_linear_forward(h, dev(x).data_ptr(), x.shape[1], y.data_ptr(), cols + 4, M, gated, 0, splits, 0x200 | shape, ws.data_ptr(), st()))
+    y = host(y)
+    assert (y[M] == 7.0).all() and (y[:M, cols:] == 7.0).all()
+    return y[:M, :cols].astype(np.float64)
+
+
+# sizes whose shapes are 1 x 8, 2 x 4, 2 x 8 and 4 x 4 waves (column groups of 32 x k-phases) and their neighbours
+@pytest.mark.parametrize('K,N,splits,gated', [
+    (128, 32, 1, 0), (384, 96, 1, 1), (2048, 4096, 1, 0), (2304, 4128, 2, 0), (2048, 10272, 1, 1), (2048, 2048, 4, 0), (4096, 10240, 1, 1), (4096, 4096, 4, 0),
+    (4224, 5152, 4, 0), (2048, 28704, 1, 1), (8192, 2048, 8, 0), (8320, 608, 8, 0), (14336, 512, 4, 0)])
+@pytest.mark.parametrize('M', [1, 3, 8, 9, 16])
+def test_against_64_bits(tm, cuda, K, N, splits, gated, M):
+    rng = np.random.default_rng(K + N + M)
+    h, _ = _make_linear(tm, rng, K, N)
+    q, s, z = _QCACHE[(K, N)][:3]
+    x = rng.standard_normal((M, K + 8)).astype(np.float16)
+    x[:, ::7] *= 30
+    w = q * np.repeat(s.astype(np.float64), 128, 0) + np.repeat((-z * s).astype(np.float16).astype(np.float64), 128, 0)
+    ref = x[:, :K].astype(np.float64) @ w
+    if gated:
+        ref = ref[:, ::2] / (1 + np.exp(-ref[:, ::2])) * ref[:, 1::2]
+    got, other = _run(tm, h, x, N, M, ROWS, splits, gated), _run(tm, h, x, N, M, 0, splits, gated)
+    _ffi.check(tm.tm_linear_destroy(h))
+    rms = np.sqrt((ref**2).mean())
+    assert np.sqrt(((got - ref)**2).mean()) <= 1.02 * np.sqrt(((other - ref)**2).mean())
+    assert (np.abs(got - ref) <= 2.0**-11 * np.abs(ref) + 2.0**-9 * rms).all()    # one rounding to fp16; sums of 1039 |x| in fp32 beside results of about 52
+
+
+def test_what_a_launch_takes(tm, cuda):
+    def pick(K, N, M):
+        sh, sp = _ffi.C.c_int(), _ffi.C.c_int()
+        _ffi.check(tm.tm_debug_pick_tiling(K, N, M, 4, _ffi.C.byref(sh), _ffi.C.byref(sp)))
+        return sh.value, sp.value
+    for K, N, M, want in ((4096, 28672, 1, (ROWS, 1)), (4096, 6144, 8, (ROWS, 2)), (4096, 4096, 16, (ROWS, 4)), (14336, 4096, 8, None), (14336, 4096, 9, (3, 4)), (4096, 6144, 17, (3, 2)),
+                          (4096, 768, 4, (ROWS, 4))):
+        assert pick(K, N, M) == want if want else pick(K, N, M)[0] == ROWS, (K, N, M)
