@@ -51,7 +51,9 @@ struct NormRows {
             g.w[q] = *(const half8_t*)(weight + (size_t)piece(nv, wave, lane, q) * 8);
         }
     }
-    __device__ __forceinline__ void finish(Regs& g, int M, int n, int pitch, char* x, float* sums, int wave, int lane, int waves) const
+    // put(m, piece of eight channels, values): where they go; every wave comes here, and a barrier stands behind it
+    template<class Put>
+    __device__ __forceinline__ void finish(Regs& g, int M, int n, float* sums, int wave, int lane, int waves, Put put) const
     {
         const int nv = n * 4;
         float     ss[RPW];
@@ -92,7 +94,7 @@ struct NormRows {
                     for (int e = 0; e < 8; ++e) {
                         y[e] = (half_t)__builtin_fmaf((float)g.r[j][q][e], inv, -0.f);  // (a product: one instruction with both conversions)
                     }
-                    *(half8_t*)(x + m * pitch + piece(nv, wave, lane, q) * 16) = y * g.w[q];
+                    put(m, piece(nv, wave, lane, q), y * g.w[q]);
                 }
             }
         }
@@ -128,7 +130,7 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_rows_kernel(StreamArgs a, 
         ring[k] = load(k);
     }
     asm volatile("" ::: "memory");
-    rows.finish(g, M, n, pitch, smem, (float*)(smem + M * pitch), wave, lane, kWaves);
+    rows.finish(g, M, n, (float*)(smem + M * pitch), wave, lane, kWaves, [&](int m, int piece, half8_t y) { *(half8_t*)(smem + m * pitch + piece * 16) = y; });
 
     const int   fr = lane & 15, fc = lane >> 4;
     const char* xf  = smem + min(fr, M - 1) * pitch + fc * 16;

@@ -16,6 +16,7 @@
 // us, one launch and a tiny one ahead of it, (4096, 28672) gated / (4096, 6144) / (4096, 4096) / (14336, 4096), the last two with the norm behind them, gemm_dec32_kernel | here: one row
 // 17.9 | 14.8, 9.1 | 7.3, 10.6 | 9.4, 14.7 | 12.6; 8 rows 17.5 | 15.6, 9.2 | 7.8, 11.1 | 9.9, 15.2 | 14.3; 16 rows 18.5 | 17.8, 9.4 | 8.8, 11.3 | 10.2, 15.9 | 16.1 (not taken).
 #include "gemm_decode_common.h"
+#include "gemm_rows.h"
 #include "tm_kernels.h"
 #include <algorithm>
 
@@ -33,9 +34,11 @@ __device__ __forceinline__ half8_t w4_rows_codes(uint32_t w, uint32_t m1024, uin
 
 constexpr int kW4RowsPad = 16;
 
-// CW column groups (32 columns) x KP k-phases of waves, R units in flight a wave.  Grid (column groups / CW, slices of k)
-template<int CW, int KP, int R, int XB, bool MANY>
-__global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p)
+// CW column groups (32 columns) x KP k-phases of waves, R units in flight a wave.  Grid (column groups / CW, slices of k).  MANY: more than eight rows.  NP > 0: the rows
+// are made here, the norm of p.resid's (gemm_rows.h: as many waves a row as there are, NP pieces each; one slice of k): one row, gate / up of Llama-3-8B between a model's
+// other kernels 13.5 us, its norm and gemm_dec32_kernel 4.6 + 15.0
+template<int CW, int KP, int R, int XB, bool MANY, int NP>
+__global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p, int team)
 {
     constexpr int T = CW * KP * 64;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -51,9 +54,16 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
     const int per = nkb * 16, pieces = M * per;
     u32x4     xr[XB];
     auto      x_of = [&](int i) { const int m = i / per; return (const u32x4*)(p.x + (size_t)m * p.ldx + (size_t)kb0 * 128 + (i - m * per) * 8); };
+    const NormRows<1, NP ? NP : 1>           norm{p.resid, p.norm_w, p.ss_eps, team};
+    typename NormRows<1, NP ? NP : 1>::Regs g;
+    if constexpr (NP > 0) {
+        norm.load(g, M, nkb * 4, wave, lane, CW * KP);
+    }
+    else {
 #pragma unroll
-    for (int r = 0; r < XB; ++r) {
-        xr[r] = *x_of(min(tid + r * T, pieces - 1));
+        for (int r = 0; r < XB; ++r) {
+            xr[r] = *x_of(min(tid + r * T, pieces - 1));
+        }
     }
     asm volatile("" ::: "memory");
     const auto rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)p.wp, 0, (int)((size_t)p.KB * p.ncg * kP32Unit), 0x00020000);
@@ -71,29 +81,35 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
         load(s, min(s, max(n - 1, 0)));
     }
     asm volatile("" ::: "memory");
-    auto park = [&](int i, u32x4 v) {
+    // (in: the same for 16 neighbouring lanes)
+    auto park = [&](int m, int at, half8_t h, bool in) {
         float c, t;
         if constexpr (!MANY) {
-            const half8_t h = bit_cast<half8_t>(v);
-            const float   a = ((float)h[0] + (float)h[1]) + ((float)h[4] + (float)h[5]), b = ((float)h[2] + (float)h[3]) + ((float)h[6] + (float)h[7]);
+            const float a = ((float)h[0] + (float)h[1]) + ((float)h[4] + (float)h[5]), b = ((float)h[2] + (float)h[3]) + ((float)h[6] + (float)h[7]);
             c = group_sum<16>(-1024.f * a - 64.f * b), t = group_sum<16>(a + b);
         }
-        if (i < pieces) {
-            const int m = i / per, at = i - m * per;
-            *(u32x4*)(smem + m * pitch + at * 16) = v;
+        if (in) {
+            *(half8_t*)(smem + m * pitch + at * 16) = h;
             if (!MANY && fr == 0) {
                 sums[(at >> 4) * M + m] = float2{c, t};
             }
         }
     };
+    if constexpr (NP > 0) {
+        norm.finish(g, M, nkb * 4, (float*)(sums + M * nkb), wave, lane, CW * KP, [&](int m, int at, half8_t h) { park(m, at, h, true); });
+    }
+    else {
 #pragma unroll
-    for (int r = 0; r < XB; ++r) {
-        park(tid + r * T, xr[r]);
+        for (int r = 0; r < XB; ++r) {
+            const int i = tid + r * T, m = i / per;
+            park(m, i - m * per, bit_cast<half8_t>(xr[r]), i < pieces);
+        }
+        for (int i = tid + XB * T; i - tid < pieces; i += T) {
+            const int m = i / per;
+            park(m, i - m * per, bit_cast<half8_t>(*x_of(min(i, pieces - 1))), i < pieces);
+        }
+        __syncthreads();
     }
-    for (int i = tid + XB * T; i - tid < pieces; i += T) {
-        park(i, *x_of(min(i, pieces - 1)));
-    }
-    __syncthreads();
 
     uint32_t m1024 = 0x64006400u, m64 = 0x54005400u;
     asm volatile("" : "+v"(m1024), "+v"(m64));  // magic numbers in VGPRs: one v_and_or_b32 per pair
@@ -198,14 +214,19 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
             *(half2_t*)(p.y + (size_t)fr * p.ldy + (c >> 1)) = half2_t{(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
         }
         else {
-            *(half4_t*)(p.y + (size_t)fr * p.ldy + c) = half4_t{(half_t)a[0], (half_t)a[1], (half_t)a[2], (half_t)a[3]};
+            half4_t* y = (half4_t*)(p.y + (size_t)fr * p.ldy + c);
+            half4_t  h = {(half_t)a[0], (half_t)a[1], (half_t)a[2], (half_t)a[3]};
+            if (p.epilogue == 4) {  // the residual stream: the product's fp16 rounding, then an addition in fp16
+                h = *y + h;
+            }
+            *y = h;
         }
     }
 }
 
 static int w4_rows_lds(int M, int nkb, int cw, int kp)
 {
-    return std::max(M * (nkb * 256 + kW4RowsPad) + M * nkb * 8, (kp - 1) * cw * 2048);
+    return std::max(M * (nkb * 256 + kW4RowsPad) + M * nkb * 8 + cw * kp * 4, (kp - 1) * cw * 2048);
 }
 
 // ---- which shape, how many slices of k -------------------------------------------------------------------------------------------------
@@ -260,7 +281,7 @@ bool w4_rows_supported(const LinearWeight& w, int M, int slices)
 }
 
 // Products below what was timed stay with gemm_dec32_kernel (whose rows have the bits that they have in forwards of more rows), and so do more than eight rows of a long
-// k: (14336, 4096) 16 rows 16.1 here, 15.9 there.  A slice has eight k-blocks at least
+// k: (14336, 4096) 16 rows 16.1 here, 15.9 there.  A slice has eight k-blocks at least; a gate / up product's slabs are nobody's to sum but a launch's of its own (3.3 us)
 bool w4_rows_plan(const LinearWeight& w, int M, int* slices)
 {
     const int KB = w.K / 128, ncg = w.N / 32;
@@ -274,6 +295,7 @@ bool w4_rows_plan(const LinearWeight& w, int M, int* slices)
         if ((s > 1 && KB / s < 8) || !w4_rows_supported(w, M, s) || w4_rows_shape(ncg, KB, M, s, &cost) < 0) {
             continue;
         }
+        cost += s > 1 && w.role == 3 ? 3.3 : 0.0;
         if (*slices == 0 || cost < best) {
             *slices = s, best = cost;
         }
@@ -281,33 +303,41 @@ bool w4_rows_plan(const LinearWeight& w, int M, int* slices)
     return *slices > 0;
 }
 
-template<int CW, int KP, bool MANY>
-static int launch_w4_rows_shape(const Dec32Params& p, int slices, hipStream_t st)
+template<int CW, int KP, bool MANY, int NP>
+static int launch_w4_rows_shape(const Dec32Params& p, int slices, int team, hipStream_t st)
 {
-    const auto kernel = gemm_w4_rows_kernel<CW, KP, 2, CW * KP == 16 ? 2 : 4, MANY>;
+    const auto kernel = gemm_w4_rows_kernel<CW, KP, 2, CW * KP == 16 ? 2 : 4, MANY, NP>;
     const int  lds    = w4_rows_lds(p.M, p.kb_per_split, CW, KP);
     if (const int rc = ensure_dynamic_lds((const void*)kernel, lds)) {
         return rc;
     }
-    kernel<<<dim3((p.ncg + CW - 1) / CW, slices), CW * KP * 64, lds, st>>>(p);
+    kernel<<<dim3((p.ncg + CW - 1) / CW, slices), CW * KP * 64, lds, st>>>(p, team);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }
 
-// as launch_linear_dec32: several slices leave fp32 slabs [slice][M][N] in the workspace
-int launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int slices, float* workspace, int* slabs, hipStream_t st)
+static Dec32Params w4_rows_params(const LinearWeight& w, half_t* y, int ldy, int M, int slices)
 {
-    TM_REQUIRE(w.packed32 && w.N % 32 == 0 && w.K % 128 == 0 && ldx % 8 == 0 && w4_rows_supported(w, M, slices) && (slices == 1 || workspace), "W4 product of few rows");
     Dec32Params p{};
-    p.x = x, p.ldx = ldx, p.wp = w.packed32, p.y = y, p.ldy = ldy, p.partial = workspace;
+    p.wp = w.packed32, p.y = y, p.ldy = ldy;
     p.M = M, p.N = w.N, p.K = w.K, p.KB = w.K / 128, p.ncg = w.N / 32;
     p.kb_per_split = w4_rows_slice(p.KB, slices);
-    p.epilogue     = slices > 1 ? 2 : gated ? 1 : 0;
+    return p;
+}
+
+// as launch_linear_dec32: several slices leave fp32 slabs [slice][M][N] in the workspace; add (one slice): y += x . W, rounded to fp16 first
+int launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int slices, float* workspace, int* slabs, hipStream_t st, bool add)
+{
+    TM_REQUIRE(w.packed32 && w.N % 32 == 0 && w.K % 128 == 0 && ldx % 8 == 0 && w4_rows_supported(w, M, slices) && (slices == 1 || workspace), "W4 product of few rows");
+    TM_REQUIRE(!add || (slices == 1 && !gated), "W4 product of few rows: a residual addition");
+    Dec32Params p = w4_rows_params(w, y, ldy, M, slices);
+    p.x = x, p.ldx = ldx, p.partial = workspace;
+    p.epilogue = slices > 1 ? 2 : gated ? 1 : add ? 4 : 0;
     if (slabs) {
         *slabs = slices;
     }
     double cost;
-#define TM_W4_ROWS(CW, KP) return M > 8 ? launch_w4_rows_shape<CW, KP, true>(p, slices, st) : launch_w4_rows_shape<CW, KP, false>(p, slices, st)
+#define TM_W4_ROWS(CW, KP) return M > 8 ? launch_w4_rows_shape<CW, KP, true, 0>(p, slices, 0, st) : launch_w4_rows_shape<CW, KP, false, 0>(p, slices, 0, st)
     switch (w4_rows_shape(p.ncg, p.KB, M, slices, &cost)) {
         case 0: TM_W4_ROWS(1, 8);
         case 1: TM_W4_ROWS(2, 4);
@@ -315,6 +345,53 @@ int launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, i
         default: TM_W4_ROWS(4, 4);
     }
 #undef TM_W4_ROWS
+}
+
+// One slice of k, for a product that closes a residual block and leaves the norm to the next: it may cost little more than the plan's slices, less than the launch that it
+// spares (3.3 us of a model's step, of which the next product takes 0.4 back).  us, whole | slices and their norm: (4096, 4096) one row 9.4 | 9.4 (norm in both), 8 rows 11.7 | 9.9;
+// (14336, 4096) one row 14.8 | 12.6 (cost 1.2 apart, taken), two 16.1 | 13.3 (1.7, not taken)
+bool w4_rows_whole(const LinearWeight& w, int M)
+{
+    int    slices;
+    double one, best;
+    return w4_rows_plan(w, M, &slices) && w4_rows_supported(w, M, 1) && w4_rows_shape(w.N / 32, w.K / 128, M, 1, &one) >= 0
+           && w4_rows_shape(w.N / 32, w.K / 128, M, slices, &best) >= 0 && one <= best + 1.4;
+}
+
+bool w4_norm_rows_supported(const LinearWeight& w, int M)
+{
+    return M <= 8 && w.K % 512 == 0 && w.K <= 8192 && w4_rows_supported(w, M, 1);
+}
+
+template<int CW, int KP>
+static int launch_w4_norm_rows_shape(const Dec32Params& p, hipStream_t st)
+{
+    int teams = 1;
+    while (teams < p.M) {
+        teams *= 2;
+    }
+    const int team = CW * KP / teams, pieces = (p.K / 512 + team - 1) / team;
+    return pieces <= 1 ? launch_w4_rows_shape<CW, KP, false, 1>(p, 1, team, st) :
+           pieces <= 2 ? launch_w4_rows_shape<CW, KP, false, 2>(p, 1, team, st) :
+           pieces <= 4 ? launch_w4_rows_shape<CW, KP, false, 4>(p, 1, team, st) :
+           pieces <= 8 ? launch_w4_rows_shape<CW, KP, false, 8>(p, 1, team, st) :
+                         launch_w4_rows_shape<CW, KP, false, 16>(p, 1, team, st);
+}
+
+// y = rmsnorm(resid) . W
+int launch_w4_norm_rows(const LinearWeight& w, const half_t* resid, const half_t* norm_w, float eps, half_t* y, int ldy, int M, bool gated, hipStream_t st)
+{
+    TM_REQUIRE(w.packed32 && w4_norm_rows_supported(w, M) && resid && norm_w && y, "W4 product with its norm");
+    Dec32Params p = w4_rows_params(w, y, ldy, M, 1);
+    p.resid = const_cast<half_t*>(resid), p.norm_w = norm_w, p.ss_eps = eps;
+    p.epilogue = gated ? 1 : 0;
+    double cost;
+    switch (w4_rows_shape(p.ncg, p.KB, M, 1, &cost)) {
+        case 0: return launch_w4_norm_rows_shape<1, 8>(p, st);
+        case 1: return launch_w4_norm_rows_shape<2, 4>(p, st);
+        case 2: return launch_w4_norm_rows_shape<2, 8>(p, st);
+        default: return launch_w4_norm_rows_shape<4, 4>(p, st);
+    }
 }
 
 }  // namespace tmk

@@ -252,7 +252,11 @@ void   dec32_pick_plain(const LinearWeight& w, int M, int* shape_out, int* split
 void   dec32_pick_launch(const LinearWeight& w, int M, int* shape_out, int* splits_out, bool use_table);  // ... with up to 16 rows on gemm_w4_rows.hip (kShapeRows)
 bool   w4_rows_supported(const LinearWeight& w, int M, int slices);
 bool   w4_rows_plan(const LinearWeight& w, int M, int* slices);
-int    launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int slices, float* workspace, int* slabs, hipStream_t st);
+int    launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int slices, float* workspace, int* slabs, hipStream_t st,
+                      bool add = false);
+bool   w4_rows_whole(const LinearWeight& w, int M);
+bool   w4_norm_rows_supported(const LinearWeight& w, int M);
+int    launch_w4_norm_rows(const LinearWeight& w, const half_t* resid, const half_t* norm_w, float eps, half_t* y, int ldy, int M, bool gated, hipStream_t st);
 // measured dispatch table of the decode linears: key (K, N, M <= 64) -> (shape, splits)
 void   dec32_table_set(int K, int N, int M, int shape, int splits, int role = 0);
 bool   dec32_table_get(int K, int N, int M, int* shape, int* splits, int role = 0);  // the role's entry, else the role-0 entry

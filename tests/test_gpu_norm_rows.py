@@ -1,4 +1,4 @@
-"""GPU test of decode steps of a few rows of fp16 models whose products add to the residual stream and make the norm of their rows themselves: a row of one wave and of
+"""GPU test of decode steps of a few rows of fp16 and W4 models whose products add to the residual stream and make the norm of their rows themselves: a row of one wave and of
 several, two rows a wave, widths of one piece a wave to eight, the three shapes of the product, slices of the product ahead that meet in its launch, one row more than
 it takes -- engines whose logits the attention or the feed-forward makes, against the oracle's separate sequence."""
 import contextlib
@@ -46,14 +46,29 @@ def _times(result, factor):
     (2048, 4, 1, 4608, 4, False), (2048, 4, 1, 4608, 5, False), (2048, 4, 1, 256, 16, True), (2048, 2, 1, 8192, 8, False), (4096, 2, 1, 256, 8, True), (4096, 4, 1, 4608, 3, False),
     (4096, 2, 1, 256, 9, False), (512, 2, 1, 256, 17, False), (640, 2, 1, 256, 3, False)])
 def test_decode(cuda, hidden, heads, kv_heads, inter, batch, attention):
-    cfg = o.ModelConfig(hidden=hidden, layers=2, q_heads=heads, kv_heads=kv_heads, head_dim=128, inter=inter, vocab=256, kv_bits=16, rope=o.RopeParam(128, 10000.0))
-    w = clear_models.weights(cfg, batch, quantized=False, attention=attention)
+    taken = hidden % 512 == 0 and (batch <= 8 or batch <= 16 and hidden <= 2048)
+    _decode(o.ModelConfig(hidden=hidden, layers=2, q_heads=heads, kv_heads=kv_heads, head_dim=128, inter=inter, vocab=256, kv_bits=16, rope=o.RopeParam(128, 10000.0)),
+            batch, attention, False, 1 if taken else 4)
+
+
+# norms: launches of a step; up to eight rows one (the last), or two where the down product keeps its slices
+@pytest.mark.parametrize('hidden,heads,kv_heads,inter,batch,attention,norms', [
+    (2048, 16, 2, 2048, 1, False, 1), (2048, 16, 2, 2048, 2, True, 1), (2048, 16, 2, 2048, 5, False, 1), (2048, 16, 2, 2048, 8, True, 2), (2048, 16, 2, 2048, 9, False, 4),
+    (2560, 16, 2, 11264, 3, False, 2), (4096, 16, 2, 2048, 7, False, 2), (4096, 16, 1, 11008, 1, False, 1), (4096, 32, 8, 14336, 2, False, 2)])
+def test_decode_w4(cuda, hidden, heads, kv_heads, inter, batch, attention, norms):
+    _decode(o.ModelConfig(hidden=hidden, layers=2, q_heads=heads, kv_heads=kv_heads, head_dim=128, inter=inter, vocab=256, kv_bits=8, rope=o.RopeParam(128, 10000.0)),
+            batch, attention, True, norms)
+
+
+def _decode(cfg, batch, attention, quantized, launches):
+    hidden = cfg.hidden
+    w = clear_models.weights(cfg, batch, quantized=quantized, attention=attention)
     rng = np.random.default_rng(batch)
     w['tok_embeddings'] = (w['tok_embeddings'].astype(np.float32) * 2.0**rng.integers(0, 4, (cfg.vocab, 1))).astype(np.float16)    # (rows whose factors differ)
     for L in w['layers']:
         for n in ('attn_norm', 'ffn_norm'):
             L[n] = (L[n].astype(np.float32) * rng.choice([0.25, 0.5, 1], hidden)).astype(np.float16)
-    eng = Engine.from_model_config(cfg, weight_type=1, max_batch_size=batch, session_len=64, quant_policy=0, max_prefill_token_num=256)
+    eng = Engine.from_model_config(cfg, weight_type=0 if quantized else 1, max_batch_size=batch, session_len=64, quant_policy=cfg.kv_bits % 16, max_prefill_token_num=256)
     eng.load_weights(export_weights(cfg, w))
     eng.start()
     prompts = [rng.integers(0, cfg.vocab, 2 + i % 3).astype(np.int32) for i in range(batch)]
@@ -67,8 +82,7 @@ def test_decode(cuda, hidden, heads, kv_heads, inter, batch, attention):
     toks = eng.fetch()
     resid = eng.fetch_residual(batch)
     eng.close()
-    taken = hidden % 512 == 0 and (batch <= 8 or batch <= 16 and hidden <= 2048)
-    assert norms == (1 if taken else 4)
+    assert norms == launches
     model = []
 
     class Kept(o.OracleModel):
