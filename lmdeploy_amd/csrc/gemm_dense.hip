@@ -364,7 +364,8 @@ void dense_weight_free(DenseWeight& d)
 //     average 0.8 % and at most 10 % slower than the best.  us, bf16: (4096, 21504) 32 rows, 64 columns 38.9 (two workgroups on some CUs), 96 columns 30.1; (25600,
 //     4096) 32 rows, one slice 95, four 36, eight 39; (4096, 6144) 32 rows, 96 columns four slices 14.8, 64 columns four 15.8, one 18.6; (2048, 2048) 8
 //     rows, narrow 5.1, four slices 6.3, one 7.9; (14336, 4096) 16 rows, narrow 27.3, four slices 21.6; fp32, 3 rows: (8448, 2048) narrow 19.9, eight slices
-//     15.3; (4096, 4096) narrow 13.8, four slices 16.2
+//     15.3; (4096, 4096) narrow 13.8, four slices 16.2; 128 columns where nearly every CU gets one workgroup of them, of 64 two, and
+//     x is long: bf16 (4096, 27648) 32 rows 39.0 / 37.3, 64 rows 44.3 / 41.3, (4096, 32000) 64 rows 47.5 / 44.6; not (2048, 28160) 32 rows 22.0 / 22.4, (4096, 27648) 8 rows 36.7 / 36.6
 //   items with rows of their own: blocks of as many rows as an item has at most (the tokens of a routed mixture, not its rows in total).  Febivik width 2048, whole
 //     batches: 8 tokens 35.4 -> 35.0 ms, 16 tokens 32.5 -> 30.5 (48 rows, blocks of 64 before), 22 tokens 38.9 -> 37.5 (66 rows, tiles before), 32 the same
 //   items, pairs: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; nine items of (2048, 2816): one 21, three 31; pairs, four rows,
@@ -439,9 +440,9 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
         // (2048, 4096) 48 rows 10.2 and 9.4)
         double least = k_major && cols > (rows > 32 ? 2048 : 8192) ? 1e30 : few_rows_cost(steps, cols, rows, elem, 0, 1, 0);
         best.skinny = best.narrow = true;
-        for (int cw : {4, 6}) {
+        for (int cw : {4, 6, 8}) {
             const int groups = (cols / 16 + cw - 1) / cw;
-            if (border % (16 * cw)) {
+            if (border % (16 * cw) || (cw == 8 && (elem == 4 || k_major || rows <= 16 || steps < 128 || groups < 192 || groups > 256))) {
                 continue;
             }
             for (int sp = 1; sp <= 16 && (sp == 1 || steps / sp >= 16); ++sp) {
@@ -449,7 +450,7 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
                 if ((steps + ss - 1) / ss != sp || (sp > 1 && ((size_t)sp * rows * cols * 4 > ws_bytes || groups > tickets))) {
                     continue;
                 }
-                const double c = few_rows_cost(steps, cols, rows, elem, cw, sp, ss);
+                const double c = few_rows_cost(steps, cols, rows, elem, cw, sp, ss) * (cw == 8 ? 0.95 : 1.0);
                 if (c < least) {
                     least = c, best.narrow = false, best.cw = cw, best.splits = sp, best.split_steps = ss;
                 }
@@ -473,6 +474,14 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     }
     if (sp > 1 && ((size_t)items * sp * rows * cols * 4 > ws_bytes || groups > tickets)) {
         sp = 1, best.narrow = true;
+    }
+    // One slice: 96 columns a workgroup where the fullest CU then streams fewer.  Items with rows of their own count as often as rows dealt at random leave one
+    // any.  Nine items of (2816, 2048), 8 tokens, 288 workgroups of 64 columns 21.4 us, 198 of 96 17.9; but one token, three items with rows, whole steps 2.5 to 5 %
+    // slower with 66 workgroups than with 96
+    const int used = (own_rows ? (int)std::ceil(items * (1.0 - std::pow(1.0 - 1.0 / items, rows))) : items) * rb;
+    const int g64 = (cols + 63) / 64 * used, g96 = (cols + 95) / 96 * used;
+    if (sp == 1 && items > 1 && elem == 2 && !pairs && !best.narrow && border % 96 == 0 && g64 <= 1024 && (g96 + 255) / 256 * 6 < (g64 + 255) / 256 * 4) {
+        best.cw = 6;
     }
     const int    ss = ((steps + sp - 1) / sp + 7) / 8 * 8;
     const double c  = std::max(1.0, groups * sp / 256.0) * ss * step + 3.0;
@@ -604,8 +613,9 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
         a.slabs       = p.splits > 1 ? d.scratch->slabs : nullptr;
         a.tickets     = p.splits > 1 ? d.scratch->tickets : nullptr;
         const dim3 grid((unsigned)((a.tiles + p.cw - 1) / p.cw), G * p.row_blocks, p.splits);
+        const bool pairs = epi == kDenseGatedAct && sizeof(T) == 2;
 #define TM_SKINNY(MT_, NT_, CW_, KP_)                                                    \
-    if (p.mt == MT_ && p.cw == CW_ * NT_) {                                              \
+    if (p.mt == MT_ && p.cw == CW_ * NT_ && pairs == (NT_ == 2)) {                                              \
         if (p.narrow) {                                                                  \
             return launch_dense_narrow<T, MT_, NT_>(a, call, vec, G, st);                \
         }                                                                                \
