@@ -19,13 +19,14 @@
 // One launch serves every row of a forward, prefill portions and decoded tokens alike: row t belongs to sequence row_seq[t] at
 // position row_pos[t] and sees the cache entries 0 .. row_pos[t] of that sequence (its own key was stored before the launch).
 //   * row kernel : one wave per (row, query head, key split); lanes own keys for the scores and value channels for the output.
-//                  The decode path (few rows, long contexts: split keys + merge kernel) and the fp32 path.
+//                  What the others do not serve: odd sizes, keys of more than 256 channels, other block lengths.
 //   * tile kernel: bf16 prefill on the matrix cores -- 64 query rows of one sequence x one query head per workgroup, four waves of 16
 //                  rows; S^T = K Q^T and O^T += V^T P^T as v_mfma_f32_16x16x32_bf16 with every operand a 16-byte load straight from the
 //                  cache (keys [token][channel], values stored transposed [channel][token]); online soft-max in fp32; no LDS, no barrier.
 //   * staged kernel: the tile kernel's products over cache blocks that a workgroup brings into LDS once (head sizes of 64 ... 256).
 //   * decode kernel: the same products with the query HEADS of one key head as the 16 rows (one row per sequence): a workgroup per
 //                  (sequence, key head, key split), its four waves take every fourth cache block and merge at the end.
+//   * heads kernel : that in fp32, for decoded rows and for prompts; a wave takes sixteen keys of every block.
 // Cache block layout per layer: keys [kv_heads][64][dim], then values [kv_heads][vdim][64].
 #include "tm_kernels.h"
 #include "decode_merge.h"
@@ -680,6 +681,91 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(GeneralAttnParams p, in
     }
 }
 
+// The end of a kernel whose four waves hold, for the 16 heads from h0 on (nh of them exist) of row t, sums over different keys: lane (lr, lg) the channels
+// 16 v + 4 lg .. + 3 of head h0 + lr, maximum and sum in the e^x domain.  Common maximum, rescaled sums, then the row's output or a split's results; the
+// last split to arrive merges them
+template<class T, int VT>
+__device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t, int sp, int nsplit, int h0, int nh, float m, float l, floatx4 (&o)[VT],
+                                               float (&ml_s)[4][16][2], float (&o_s)[3][16][VT * 16 + 4], unsigned* last_s)
+{
+    const int  lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4, V = p.vdim;
+    const bool h_ok = lr < nh;
+    const int  h    = h0 + (h_ok ? lr : 0);
+    if (lg == 0) {
+        ml_s[wave][lr][0] = m;
+        ml_s[wave][lr][1] = l;
+    }
+    __syncthreads();
+    const float mf = fmaxf(fmaxf(ml_s[0][lr][0], ml_s[1][lr][0]), fmaxf(ml_s[2][lr][0], ml_s[3][lr][0]));
+    const float a  = __expf(m - mf);
+    if (wave > 0) {
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            *(floatx4*)&o_s[wave - 1][lr][v * 16 + lg * 4] = o[v] * a;
+        }
+    }
+    __syncthreads();
+    if (wave > 0) {
+        if (nsplit == 1 || !p.tickets) {
+            return;
+        }
+    }
+    else {
+        float lt = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            lt += ml_s[w][lr][1] * __expf(ml_s[w][lr][0] - mf);
+        }
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            const int c = v * 16 + lg * 4;
+            o[v]        = o[v] * a + ((*(const floatx4*)&o_s[0][lr][c] + *(const floatx4*)&o_s[1][lr][c]) + *(const floatx4*)&o_s[2][lr][c]);
+        }
+        if (nsplit == 1) {
+            float inv;
+            if (p.sink) {
+                const float sk = p.sink[h], m2 = fmaxf(mf, sk), a2 = __expf(mf - m2);
+                inv            = a2 / (lt * a2 + __expf(sk - m2));
+            }
+            else {
+                inv = 1.f / lt;
+            }
+            inv *= ga_out_gate(p, t, h);
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+                const int c = v * 16 + lg * 4;
+                if (h_ok && c < V) {
+                    ga_store4<T>(p, t, h, c, o[v] * inv);
+                }
+            }
+            return;
+        }
+        float* po = p.partial_o + (((size_t)t * p.q_heads + h) * p.splits + sp) * V;
+        float* pm = p.partial_ml + (((size_t)t * p.q_heads + h) * p.splits + sp) * 2;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            const int c = v * 16 + lg * 4;
+            if (h_ok && c < V) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    agent_store(po + c + r, o[v][r]);
+                }
+            }
+        }
+        if (h_ok && lg == 0) {
+            agent_store(pm, mf);
+            agent_store(pm + 1, lt);
+        }
+    }
+    if (p.tickets && ticket_last_workgroup(p.tickets + (size_t)t * p.q_heads + h0, nsplit, last_s)) {
+        const int pieces = V / 4;
+        for (int i = threadIdx.x; i < nh * pieces; i += 256) {
+            const int head = i / pieces, c0 = (i - head * pieces) * 4;
+            ga_merge<T, 4>(p, t, h0 + head, nsplit, [=](int c) { return c0 + c; });
+        }
+    }
+}
+
 // Decode: grid (sequences, kv_heads * head chunks, splits).  The 16 rows are query heads g * group + chunk * 16 + (lane % 16) of row t;
 // wave w takes the blocks b0 + w, b0 + w + 4, ... of the split; waves 1..3 hand their (m, l, O) to wave 0 through LDS.
 template<int DS, int VT>
@@ -734,83 +820,9 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
                                              (const __bf16*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V, D, V, limit, lower,
                                              keep - b * 64, qscale, cap, inv_cap, bias, r1, r2, m1, l1, o1, tab, p.dist_table_len);
     }
-    const float m = m1[0] * kLn2, l = l1[0];  // back from the log2 domain: the merge below and the split merge kernel use e^x
-    floatx4 (&o)[VT] = o1[0];
-    // ---- merge the four waves: common maximum, rescaled sums ----
-    if (lg == 0) {
-        ml_s[wave][lr][0] = m;
-        ml_s[wave][lr][1] = l;
-    }
-    __syncthreads();
-    const float mf = fmaxf(fmaxf(ml_s[0][lr][0], ml_s[1][lr][0]), fmaxf(ml_s[2][lr][0], ml_s[3][lr][0]));
-    const float a  = __expf(m - mf);
-    if (wave > 0) {
-#pragma unroll
-        for (int v = 0; v < VT; ++v) {
-            *(floatx4*)&o_s[wave - 1][lr][v * 16 + lg * 4] = o[v] * a;
-        }
-    }
-    __syncthreads();
-    const int nheads = min(16, group - chunk * 16);
-    if (wave > 0) {
-        if (nsplit == 1 || !p.tickets) {
-            return;
-        }
-    }
-    else {
-        float lt = 0.f;
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            lt += ml_s[w][lr][1] * __expf(ml_s[w][lr][0] - mf);
-        }
-#pragma unroll
-        for (int v = 0; v < VT; ++v) {
-            const int c = v * 16 + lg * 4;
-            o[v]        = o[v] * a + ((*(const floatx4*)&o_s[0][lr][c] + *(const floatx4*)&o_s[1][lr][c]) + *(const floatx4*)&o_s[2][lr][c]);
-        }
-        if (nsplit == 1) {
-            float inv;
-            if (p.sink) {
-                const float sk = p.sink[h], m2 = fmaxf(mf, sk), a2 = __expf(mf - m2);
-                inv            = a2 / (lt * a2 + __expf(sk - m2));
-            }
-            else {
-                inv = 1.f / lt;
-            }
-            inv *= ga_out_gate(p, t, h);
-#pragma unroll
-            for (int v = 0; v < VT; ++v) {
-                const int c = v * 16 + lg * 4;
-                if (h_ok && c < V) {
-                    ga_store4<__bf16>(p, t, h, c, o[v] * inv);
-                }
-            }
-            return;
-        }
-        float* po = p.partial_o + (((size_t)t * p.q_heads + h) * p.splits + sp) * V;
-        float* pm = p.partial_ml + (((size_t)t * p.q_heads + h) * p.splits + sp) * 2;
-#pragma unroll
-        for (int v = 0; v < VT; ++v) {
-            const int c = v * 16 + lg * 4;
-            if (h_ok && c < V) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    agent_store(po + c + r, o[v][r]);
-                }
-            }
-        }
-        if (h_ok && lg == 0) {
-            agent_store(pm, mf);
-            agent_store(pm + 1, lt);
-        }
-    }
-    if (p.tickets && ticket_last_workgroup(p.tickets + (size_t)t * p.q_heads + g * group + chunk * 16, nsplit, &last_s)) {
-        const int pieces = V / 4;
-        for (int i = threadIdx.x; i < nheads * pieces; i += 256) {
-            const int head = i / pieces, c0 = (i - head * pieces) * 4;
-            ga_merge<__bf16, 4>(p, t, g * group + chunk * 16 + head, nsplit, [=](int c) { return c0 + c; });
-        }
-    }
+    const int h0 = g * group + chunk * 16;
+    // (back from the log2 domain: the merges use e^x)
+    ga_close_heads<__bf16, VT>(p, t, sp, nsplit, h0, min(16, group - chunk * 16), m1[0] * kLn2, l1[0], o1[0], ml_s, o_s, &last_s);
 }
 
 bool general_attention_tiles_ok(const GeneralAttnParams& p)
@@ -1186,6 +1198,156 @@ int launch_general_attention_decode(const GeneralAttnParams& p, hipStream_t st)
     return 0;
 }
 
+// ---- fp32: the heads of a key head as a tile ------------------------------------------------------------------------------------------
+// attn_decode_kernel's arrangement for an fp32 cache, v_mfma_f32_16x16x4: workgroup per (row, 16 heads of a key head, key split), each wave 16 of a block's 64
+// keys.  S^T = K Q^T with the channels of a step dealt so that a lane's four are one load, and P^T then stands in the registers that O^T += V^T P^T reads.
+// What bounds it is a CU's load path -- the row kernel brings every key once per query head through it -- and at few rows the chain of dependent loads.
+// us, row kernel / this one: 16 / 1 heads of 256 / 192, 3 rows over ~180 tokens 20.7 / 15.6, 2 rows over 2000 62.8 / 29.4, 420 rows of three prompts 148 / 33, a
+// prompt of 2000 7810 / 670; 32 / 8 heads of 128 / 128 15.0 / 10.1, 46.5 / 20.3, 146 / 69, 8430 / 1960; and where a head has a key head of its own (the tile holds one
+// row of sixteen) 16 / 16 heads of 128 / 128 16.5 / 10.1, 56.8 / 22.1, 145 / 124, 10300 / 3850: nothing was slower, so it serves every size it can.
+template<int DS, int VT>
+__global__ __launch_bounds__(256) void attn_heads_f32_kernel(GeneralAttnParams p, int chunks)
+{
+    __shared__ float    ml_s[4][16][2];
+    __shared__ unsigned last_s;
+    __shared__ float    o_s[3][16][VT * 16 + 4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
+    const int t = blockIdx.x, g = blockIdx.y / chunks, chunk = blockIdx.y % chunks, sp = blockIdx.z;
+    const int D = p.dim, V = p.vdim, group = p.q_heads / p.kv_heads, h0 = g * group + chunk * 16, nh = min(16, group - chunk * 16);
+    const int h = h0 + min(lr, nh - 1), pos = p.row_pos[t], s = p.row_seq[t];
+    const uint64_t* table = p.block_ptrs + (size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride;
+    const int first = ga_first_key(p, pos), bf = first / 64;
+    const int keep = ga_keep(p), nk = ga_keep_blocks(p, first, bf, 64);
+    const int nvis = nk + pos / 64 + 1 - bf, per = ga_split_len(p, nvis), nsplit = ga_split_count(p, nvis);
+    const int i0 = sp * per, i1 = min(nvis, i0 + per);
+    if (sp >= nsplit) {
+        return;
+    }
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    floatx4       q[DS], o[VT];
+#pragma unroll
+    for (int i = 0; i < DS; ++i) {
+        const int d = i * 16 + lg * 4;
+        q[i]        = *(const ga_floatx4_any*)((const float*)p.q + (size_t)t * p.ldq + (size_t)h * D + min(d, D - 4));
+        if (d >= D) {
+            q[i] = zero;
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+        o[v] = zero;
+    }
+    const float  qscale = p.scale * ga_query_temp(p, pos);
+    const bool   bias   = p.dist_r1 != nullptr;
+    const float  r1 = bias ? p.dist_r1[h] : 0.f, r2 = bias ? p.dist_r2[h] : 0.f;
+    const float* tab = p.dist_table ? p.dist_table + (size_t)h * p.dist_table_len : nullptr;
+    float        m = -1e30f, l = 0.f;
+    const int    j0 = wave * 16;
+    for (int bi = i0; bi < i1; ++bi) {
+        const int b = ga_block_at(bi, nk, bf), limit = pos - b * 64, lower = first - b * 64, klo = keep - b * 64;
+        if (j0 > limit || (j0 + 15 < lower && j0 >= klo)) {  // none of the wave's keys is seen
+            continue;
+        }
+        const char*  base = (const char*)table[b] + p.layer_offset;
+        const float* kb   = (const float*)base + ((size_t)ga_key_head(p, g) * 64 + j0 + lr) * D;
+        const float* vb   = (const float*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V + j0 + lg * 4;
+        floatx4      k[DS], v4[VT];
+#pragma unroll
+        for (int i = 0; i < DS; ++i) {
+            k[i] = *(const ga_floatx4_any*)(kb + min(i * 16 + lg * 4, D - 4));
+        }
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            v4[v] = *(const ga_floatx4_any*)(vb + (size_t)min(v * 16 + lr, V - 1) * 64);
+        }
+        floatx4 sc = zero;
+#pragma unroll
+        for (int i = 0; i < DS; ++i) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                sc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][c], q[i][c], sc, 0, 0, 0);
+            }
+        }
+        bool  seen[4];
+        float mx = -1e30f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = j0 + lg * 4 + r;
+            seen[r]     = j <= limit && (j >= lower || j < klo);
+            float x     = ga_modify(p, sc[r], qscale);
+            if (bias) {
+                x -= r1 * log1pf(r2 * (float)(limit - j));
+            }
+            if (tab && seen[r]) {
+                x += tab[min(limit - j, p.dist_table_len - 1)];
+            }
+            sc[r] = seen[r] ? x : -1e30f;
+            mx    = fmaxf(mx, sc[r]);
+        }
+        const float m_new = fmaxf(m, ga_max_groups(mx)), alpha = __expf(m - m_new);
+        m = m_new;
+        l *= alpha;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            sc[r] = seen[r] ? __expf(sc[r] - m_new) : 0.f;
+            l += sc[r];
+        }
+        const bool whole = j0 + 15 <= limit;  // (entries behind a row's own may hold anything: a weight of zero does not take them out)
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+            o[v] *= alpha;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float x = whole || j0 + lg * 4 + r <= limit ? v4[v][r] : 0.f;
+                o[v]          = __builtin_amdgcn_mfma_f32_16x16x4f32(x, sc[r], o[v], 0, 0, 0);
+            }
+        }
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    ga_close_heads<float, VT>(p, t, sp, nsplit, h0, nh, m, l, o, ml_s, o_s, &last_s);
+}
+
+bool general_attention_heads_f32_ok(const GeneralAttnParams& p)
+{
+    return p.elem_bytes == 4 && p.block_len == 64 && p.dim % 4 == 0 && p.vdim % 4 == 0 && p.dim >= 4 && p.dim <= 256 && p.vdim >= 4 && p.vdim <= 256 && p.kv_heads >= 1
+           && p.q_heads % p.kv_heads == 0 && p.splits >= 1 && (p.splits == 1 || (p.partial_o && p.partial_ml));
+}
+
+int launch_general_attention_heads_f32(const GeneralAttnParams& p, hipStream_t st)
+{
+    TM_REQUIRE(general_attention_heads_f32_ok(p), "attention over heads: fp32, 64-token blocks, dim and vdim multiples of 4 up to 256");
+    TM_REQUIRE(p.rows >= 0 && p.chunk >= 0 && (!p.dist_r1 || p.dist_r2) && (!p.out_gate || p.ld_gate >= p.q_heads), "attention: chunk / distance penalty / gate");
+    TM_REQUIRE(p.window >= 0 && p.keep_first >= 0, "attention: window / kept first tokens");
+    TM_REQUIRE(p.k_heads >= 0 && p.v_heads >= 0 && (!p.dist_table || p.dist_table_len >= 1), "attention: key / value head counts, distance table");
+    TM_REQUIRE(p.qtemp_coef == 0.f || p.qtemp_every > 0.f, "attention: query temperature period");
+    if (p.rows == 0) {
+        return 0;
+    }
+    const int         chunks = (p.q_heads / p.kv_heads + 15) / 16;
+    GeneralAttnParams a      = p;
+    a.tickets                = ga_tickets(p);
+    a.split_blocks           = std::min(4, std::max(1, p.rows * p.kv_heads * chunks / 64));  // (as in the decode kernel)
+    const dim3 grid(p.rows, p.kv_heads * chunks, p.splits);
+    const int  ds = (p.dim + 15) / 16, vt = (p.vdim + 15) / 16;
+#define TM_HEADS(DS_, VT_)                                            \
+    if (ds <= DS_ && vt <= VT_) {                                     \
+        attn_heads_f32_kernel<DS_, VT_><<<grid, 256, 0, st>>>(a, chunks); \
+    }                                                                 \
+    else
+    TM_HEADS(4, 4) TM_HEADS(4, 8) TM_HEADS(8, 8) TM_HEADS(16, 8) TM_HEADS(16, 12)
+    {
+        attn_heads_f32_kernel<16, 16><<<grid, 256, 0, st>>>(a, chunks);
+    }
+#undef TM_HEADS
+    TM_HIP_CHECK(hipGetLastError());
+    if (p.splits > 1 && !a.tickets) {
+        launch_rows_merge<float>(a, st);
+        TM_HIP_CHECK(hipGetLastError());
+    }
+    return 0;
+}
+
 int launch_general_attention_tiles(const GeneralAttnParams& p, hipStream_t st)
 {
     TM_REQUIRE(general_attention_tiles_ok(p), "attention tile kernel: bf16, 64-token blocks, dim and vdim multiples of 8 up to 256, sequence description");
@@ -1215,6 +1377,9 @@ int launch_general_attention(const GeneralAttnParams& p, bool prefill, hipStream
     }
     if (!prefill && tiles_on && general_attention_decode_ok(p)) {
         return launch_general_attention_decode(p, st);
+    }
+    if (tiles_on && general_attention_heads_f32_ok(p)) {
+        return launch_general_attention_heads_f32(p, st);
     }
     return launch_general_attention_rows(p, st);
 }
