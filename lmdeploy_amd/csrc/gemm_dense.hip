@@ -394,10 +394,13 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
                                   {64, 64, 0.125, 0.15, 0.24, 0.32, 1.0}};
     StreamPlan        best{};
     double            cost = 1e30;
+    // row tiles: items with rows of their own fill half of their last one on average, and each that has rows needs one
+    auto row_tiles = [&](int bm) -> int64_t {
+        return own_rows ? std::max(rows / bm + (items + 1) / 2 + (bm == 256), std::min(rows, items)) : (int64_t)((rows + bm - 1) / bm) * items;
+    };
     auto rounds = [&](int k, int n_cols) {  // of tiles of shape k over n_cols columns, 256 tiles a round
-        const Tile&   t  = kTiles[k];
-        const int64_t rt = own_rows ? rows / t.rows + items : (int64_t)((rows + t.rows - 1) / t.rows) * items;
-        return (rt * ((n_cols + t.cols - 1) / t.cols) + 255) / 256;
+        const Tile& t = kTiles[k];
+        return (row_tiles(t.rows) * ((n_cols + t.cols - 1) / t.cols) + 255) / 256;
     };
     auto tile_cost = [&](int k, int n_cols) {
         const Tile&  t     = kTiles[k];
@@ -414,8 +417,10 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     // model above sees 1 % in it after 4 us for the launch.  us, one launch / two: fp16 (14336, 4096) 4100 rows 591 / 449, (2048, 8448) 2040 rows 96 / 75, 8010 rows 283 /
     // 262, (5120, 27648) gated 1030 rows 399 / 335, (4096, 6144) 5888 rows 303 / 262, least of 17 sizes (5120, 27648) 8010 rows 1873 / 1879; bf16 (4096, 27648) 8192
     // rows 1469 / 1458
-    if (cut_ok && items == 1 && !own_rows && elem == 2 && border % 256 == 0) {
-        const int rt = (rows + 255) / 256;
+    // Items with rows of their own, nine of (2048, 2816) and (2816, 2048), one launch / two: 23800 rows 314 / 302 and 344 / 306, 12400 rows the first 174 / 166, 16500 rows
+    // the second 232 / 237 (the line is drawn wider for them: their last tiles are not known here)
+    if (cut_ok && (items == 1 || own_rows) && elem == 2 && border % 256 == 0) {
+        const int64_t rt = row_tiles(256);
         for (int64_t full = rounds(0, cols) - 1; full >= 1 && full >= rounds(0, cols) - 2; --full) {
             const int cut = (int)(full * 256 / rt) * 256;
             if (cut <= 0 || cut >= cols) {
@@ -423,7 +428,7 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
             }
             for (int k = 1; k < 4; ++k) {
                 const double c = tile_cost(0, cut) + tile_cost(k, cols - cut) + 4.0;
-                if (c < 0.99 * cost) {
+                if (c < (own_rows ? 0.97 : 0.99) * cost) {
                     cost = c, best.tile = 0, best.cut = cut, best.tile2 = k;
                 }
             }
