@@ -179,7 +179,7 @@ struct LayeredModel {
     int                  ldcq = 0, ldside = 0;
     float*               d_hist = nullptr;
     size_t               hist_stride = 0;
-    float*               d_blocks = nullptr;    // scratch of the forget-gate mixer's chunks
+    float*               d_blocks = nullptr;    // scratch of the state mixers' chunks
     size_t               blocks_floats = 0;
     float*               d_logits_f32 = nullptr;  // [max_logit_rows][vocab]
     int *                d_row_seq = nullptr, *d_row_pos = nullptr, *d_iota = nullptr, *d_want = nullptr, *d_seq_slot = nullptr;

@@ -948,16 +948,19 @@ int layered_start(tm_engine* e)
             max_ff    = std::max(max_ff, L.down.Kp);
             lm.ldside = std::max(lm.ldside, L.side_proj.Kp);
             if (L.spec.mixer == TM_MIXER_FORGET) {
-                lm.blocks_floats = std::max(lm.blocks_floats, decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim));
+                lm.blocks_floats = std::max(lm.blocks_floats, decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim, false));
             }
             continue;
         }
         if (L.both) {
-            lm.blocks_floats = std::max(lm.blocks_floats, parallel ? decay_workspace_floats((int)T, B, L.spec.r_heads, L.spec.r_dim)
-                                                                   : decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim));
+            lm.blocks_floats = std::max(lm.blocks_floats, parallel ? decay_workspace_floats((int)T, B, L.spec.r_heads, L.spec.r_dim, false)
+                                                                   : decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim, false));
         }
-        if (L.post && L.spec.mixer == TM_MIXER_LIGHTNING) {
-            lm.blocks_floats = std::max(lm.blocks_floats, decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim));
+        if (L.post && (L.spec.mixer == TM_MIXER_LIGHTNING || L.spec.mixer == TM_MIXER_DELTA)) {
+            lm.blocks_floats = std::max(lm.blocks_floats, decay_workspace_floats((int)T, B, L.spec.heads, L.spec.dim, L.spec.mixer == TM_MIXER_DELTA));
+        }
+        if (L.post && parallel) {  // its right mixer is the gated delta rule
+            lm.blocks_floats = std::max(lm.blocks_floats, decay_workspace_floats((int)T, B, L.spec.r_heads, L.spec.r_dim, true));
         }
         if (L.post || L.both) {
             max_cat  = std::max(max_cat, L.wo.Kp);
@@ -1489,6 +1492,7 @@ static int group_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* part
             sp.decay_w = lm.d_wdec + (size_t)P.row0 * lm.ldmix, sp.ld_w = lm.ldmix;
             sp.unit    = lm.d_aux + (size_t)P.row0 * lm.ldmix, sp.ld_u = lm.ldmix;
             sp.out     = lm.d_mixo + (size_t)P.row0 * lm.ldmix, sp.ldo = lm.ldmix;
+            sp.rows = P.rows, sp.blocks = lm.d_blocks, sp.blocks_floats = lm.blocks_floats;
             TM_PROF(P_ATTN, TM_TRY(launch_state_mix(sp, kStateDelta, st)));
         }
         TM_PROF(P_ATTN, TM_TRY(launch_gated_group_norm(lm.d_cat, lm.ldcat, lm.elem, lm.d_mixo, lm.ldmix, L.r_norm, lm.d_gate2, lm.ldmix, M, Hr, dvr,

@@ -24,11 +24,12 @@
 // vectors (q, k, and w, a u, u for the delta rule), loaded TB tokens at a time: the next stage's global loads are issued before the
 // current stage's tokens are walked and land in the other LDS buffer afterwards, so their latency hides under the recurrence.  A slab is
 // stored as the wave holds it, [ii][column of the pair][lane]: loading and storing it are fully coalesced.
-// The delta rule walks its tokens one by one (two dependent reductions per token); the other mixers take this kernel for decoded tokens, their prompt
-// portions run in chunks on the matrix cores (below).
+// The delta rule walks portions of up to 32 tokens one by one (two dependent reductions per token); longer ones, and every portion of the other mixers, run
+// in chunks on the matrix cores (below).
 // One kernel serves prompt portions (many rows per sequence) and decoded tokens (one row, TB = 1): the state traffic of a decode step,
 // 2 * dim * vdim * 4 bytes per head, is what bounds it.
 #include "tm_kernels.h"
+#include "gemm_stream.h"  // stream_dma16
 
 namespace tmk {
 
@@ -323,7 +324,7 @@ static void launch_state_dq(const StateMixParams& p, dim3 grid, hipStream_t st)
 // ---- linear attention with decays over prompt portions: chunks of 16 tokens on the fp32 matrix cores -------------------------------------
 // Serves the forget-gate mixer (k = 1 - f), lightning attention (f = the head's decay; silu on q, k and v as they are loaded), retention (f = the head's
 // decay, q and k rotated as they are loaded) and the bonus recurrence.
-// 8 prompts of ~1000 tokens, 16 heads of 128 / 128, lightning: 84 + 190 us a layer; on the vector units (16 tokens at a time in LDS) 790.
+// 8 prompts of ~1000 tokens, 16 heads of 128 / 128, lightning: 84 + 143 us a layer; on the vector units (16 tokens at a time in LDS) 790.
 // Per chunk, head and key channel d, with t, j counting tokens of the chunk and P(a..b) = prod of f_s[d] for a <= s <= b:
 //   o_t = sum_d q_t P(0..t) S0[d] + sum_{j <= t} A[t][j] v_j,    A[t][j] = sum_d q_t k_j P(j+1..t)
 //   S   = P(0..15) S0 + sum_j k_j P(j+1..15) v_j^T
@@ -343,10 +344,13 @@ __host__ __device__ inline int decay_tiles(int dim)  // row tiles of an instanti
     const int n = (dim + 15) / 16;
     return n <= 2 ? 2 : n <= 4 ? 4 : n <= 8 ? 8 : 16;
 }
-__host__ __device__ inline size_t decay_block_floats(int dim)
+__host__ __device__ constexpr int decay_block_floats_of(int dr, bool delta)  // whole pieces of 1 KB, as the DMA brings them
 {
-    const int dr = decay_tiles(dim);
-    return (size_t)dr * 64 * 4 * 2 + 256 + dr * 16;
+    return ((delta ? 4 : 2) * dr * 256 + (delta ? 3 : 1) * 256 + dr * 16 + 255) / 256 * 256;
+}
+__host__ __device__ inline size_t decay_block_floats(int dim, bool delta)
+{
+    return decay_block_floats_of(decay_tiles(dim), delta);
 }
 // chunk c of sequence s, whose first row is row0 of the launch: sequences take (rows before) / 16 + s onwards, which never overlaps
 __device__ __forceinline__ size_t decay_chunk_index(int s, int row0, int c)
@@ -354,9 +358,9 @@ __device__ __forceinline__ size_t decay_chunk_index(int s, int row0, int c)
     return (size_t)(row0 / kChunkT + s + c);
 }
 
-size_t decay_workspace_floats(int rows, int nseq, int heads, int dim)
+size_t decay_workspace_floats(int rows, int nseq, int heads, int dim, bool delta)
 {
-    return ((size_t)rows / kChunkT + nseq + 1) * heads * decay_block_floats(dim);
+    return ((size_t)rows / kChunkT + nseq + 1) * heads * decay_block_floats(dim, delta);
 }
 
 // grid (nseq * chunks, heads), 256 threads
@@ -372,7 +376,7 @@ __global__ __launch_bounds__(256) void decay_blocks_kernel(StateMixParams p, int
     if (nt <= 0) {
         return;
     }
-    float* out = p.blocks + (decay_chunk_index(s, row0, c) * p.heads + h) * decay_block_floats(D);
+    float* out = p.blocks + (decay_chunk_index(s, row0, c) * p.heads + h) * decay_block_floats_of(DR, false);
     for (int i = tid; i < kChunkT * DP; i += 256) {
         const int  t = i / DP, d = i % DP;
         float      q = 0.f, k = 0.f, f = 1.f;  // tokens behind the portion and channels behind dim: nothing read, nothing written, nothing forgotten
@@ -483,23 +487,191 @@ __global__ __launch_bounds__(256) void decay_blocks_kernel(StateMixParams p, int
     }
 }
 
-// grid (nseq, heads, ceil(vdim / 64)), 256 threads: wave -> 16 value columns; SILU: on the values
-template<int DR, bool SILU>
-__global__ __launch_bounds__(256) void decay_chunks_kernel(StateMixParams p)
+// The delta rule, S_t = diag(w_t) S - b_t e_t + k_t v_t^T with b = a u and e_t = S^T u_t (S as the token finds it).  With
+//   U0[t] = u_t P(0..t-1),   Auk[t][j < t] = sum_d u_t k_j P(j+1..t-1),   Aub likewise,   Aqk[t][j <= t] = sum_d q_t k_j P(j+1..t),   Aqb likewise
+// the e of a chunk solve (I + Aub) E = U0 S0 + Auk V, and
+//   o = Q0 S0 + Aqk V - Aqb E,   S = P(0..15) S0 + K1^T V - B1^T E      (Q0, K1 and B1 with their running products as above).
+// Aub is strictly lower triangular: (I + Aub)^-1 is applied to the columns of U0 and Auk by forward substitution here, a column a thread, so that the walk
+// over the chunks has E by products alone.  u has norm one, a and w lie in [0, 1]: every factor diag(w) - b u^T is a contraction, and what the substitution
+// forms stays as small as its right sides.
+// Block: as above, then U [DR][64][4], B1 [DR][64][4], Aqb [64][4], W = (I + Aub)^-1 Auk [64][4].  Dynamic LDS: delta_blocks_lds(DR)
+constexpr int delta_blocks_lds(int dr)
 {
-    constexpr int NC = kStateNC, WV = kStateCW * kStateNC;
-    const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, cb = blockIdx.z * 4 + (threadIdx.x >> 6);
-    const int D = p.dim, V = p.vdim, dq = (D + 7) / 8, ncb = (V + WV - 1) / WV;
-    if (cb >= ncb) {
+    return (5 * kChunkT * (dr * 16 + 4) + 2 * kChunkT * kChunkT) * 4;
+}
+template<int DR>
+__global__ __launch_bounds__(256) void delta_blocks_kernel(StateMixParams p, int chunks)
+{
+    constexpr int DP = DR * 16, LD = DP + 4, NM = (DP + 63) / 64;
+    extern __shared__ __attribute__((aligned(16))) float delta_lds[];
+    float *sq = delta_lds, *sk = sq + kChunkT * LD, *sf = sk + kChunkT * LD, *sb = sf + kChunkT * LD, *su = sb + kChunkT * LD;
+    float *ab = su + kChunkT * LD, *wk = ab + kChunkT * kChunkT;  // Aub, Auk [t][j]
+    const int s = blockIdx.x / chunks, c = blockIdx.x % chunks, h = blockIdx.y, D = p.dim, tid = threadIdx.x;
+    const int row0 = p.cu_q[s] - p.cu_q[0], q_len = p.cu_q[s + 1] - p.cu_q[s];
+    const int t0 = c * kChunkT, nt = min(kChunkT, q_len - t0);
+    if (nt <= 0) {
         return;
     }
+    float* out = p.blocks + (decay_chunk_index(s, row0, c) * p.heads + h) * decay_block_floats_of(DR, true);
+    float *oA = out + DR * 512, *oF = oA + 256, *oU = oF + DP, *oB = oU + DR * 256, *oAb = oB + DR * 256, *oW = oAb + 256;
+    for (int i = tid; i < kChunkT * DP; i += 256) {
+        const int  t = i / DP, d = i % DP;
+        const bool ok = t < nt && d < D;  // tokens behind the portion and channels behind dim read, write and forget nothing
+        const size_t row = (size_t)(row0 + t0 + (ok ? t : 0));
+        const float* pr  = p.proj + row * p.ld + h * D + (ok ? d : 0);
+        sq[t * LD + d] = ok ? pr[p.c_q] : 0.f;
+        sk[t * LD + d] = ok ? pr[p.c_k] : 0.f;
+        sb[t * LD + d] = ok ? pr[p.c_a] : 0.f;
+        sf[t * LD + d] = ok ? p.decay_w[row * p.ld_w + h * D + d] : 1.f;
+        su[t * LD + d] = ok ? p.unit[row * p.ld_u + h * D + d] : 0.f;
+    }
+    __syncthreads();
+    {   // the four A: 16 lanes share a key j, each with its channels; the key and b decay as t moves on
+        const int j = tid >> 4, sl = tid & 15;
+        floatx4   k[NM], b[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) {
+            const int d = m * 64 + sl * 4;
+            k[m]        = d < DP ? *(const floatx4*)(sk + j * LD + d) : floatx4{0.f, 0.f, 0.f, 0.f};
+            b[m]        = d < DP ? *(const floatx4*)(sb + j * LD + d) : floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll 4
+        for (int t = 0; t < kChunkT; ++t) {
+            float uk = 0.f, ub = 0.f, qk = 0.f, qb = 0.f;
+#pragma unroll
+            for (int m = 0; m < NM; ++m) {
+                const int d = m * 64 + sl * 4;
+                if (d < DP) {
+                    const floatx4 q = *(const floatx4*)(sq + t * LD + d), f = *(const floatx4*)(sf + t * LD + d), u = *(const floatx4*)(su + t * LD + d);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        uk = fmaf(u[i], k[m][i], uk);
+                        ub = fmaf(u[i], b[m][i], ub);
+                        const float w = t > j ? f[i] : 1.f;
+                        k[m][i] *= w;
+                        b[m][i] *= w;
+                        qk = fmaf(q[i], k[m][i], qk);
+                        qb = fmaf(q[i], b[m][i], qb);
+                    }
+                }
+            }
+            uk = group_sum<16>(uk), ub = group_sum<16>(ub), qk = group_sum<16>(qk), qb = group_sum<16>(qb);
+            if (sl == t) {
+                const int at = ((j >> 2) * 16 + t) * 4 + (j & 3);  // operand order: lane = (j / 4) * 16 + t, element j % 4
+                oA[at]              = t >= j ? qk : 0.f;
+                oAb[at]             = t >= j ? qb : 0.f;
+                wk[t * kChunkT + j] = t > j ? uk : 0.f;
+                ab[t * kChunkT + j] = t > j ? ub : 0.f;
+            }
+        }
+    }
+    __syncthreads();
+    auto substitute = [&](float (&x)[kChunkT]) {  // (I + Aub) x = right side, in place
+#pragma unroll
+        for (int t = 1; t < kChunkT; ++t) {
+            float r = x[t];
+#pragma unroll
+            for (int j = 0; j < t; ++j) {
+                r = fmaf(-ab[t * kChunkT + j], x[j], r);
+            }
+            x[t] = r;
+        }
+    };
+    for (int i = tid; i < 2 * DP; i += 256) {  // running products down the tokens (queries, u) and up (keys, b); the solution's columns
+        const int d = i % DP;
+        float     run = 1.f, x[kChunkT];
+        if (i < DP) {
+#pragma unroll
+            for (int t = 0; t < kChunkT; ++t) {
+                x[t] = su[t * LD + d] * run;
+                run *= sf[t * LD + d];
+                sq[t * LD + d] *= run;
+            }
+            oF[d] = run;
+            substitute(x);
+#pragma unroll
+            for (int t = 0; t < kChunkT; ++t) {
+                su[t * LD + d] = x[t];
+            }
+        }
+        else {
+#pragma unroll
+            for (int t = kChunkT - 1; t >= 0; --t) {
+                sk[t * LD + d] *= run;
+                sb[t * LD + d] *= run;
+                run *= sf[t * LD + d];
+            }
+            if (d < kChunkT) {
+#pragma unroll
+                for (int t = 0; t < kChunkT; ++t) {
+                    x[t] = wk[t * kChunkT + d];
+                }
+                substitute(x);
+#pragma unroll
+                for (int t = 0; t < kChunkT; ++t) {
+                    wk[t * kChunkT + d] = x[t];
+                }
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < DR * 64; i += 256) {
+        const int r = i >> 6, l = i & 63, row = (l & 15) * LD + r * 16 + (l >> 4) * 4;
+        *(floatx4*)(out + (size_t)i * 4) = *(const floatx4*)(sq + row);
+        *(floatx4*)(oU + (size_t)i * 4)  = *(const floatx4*)(su + row);
+        floatx4 k, b;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            k[e] = sk[((l >> 4) * 4 + e) * LD + r * 16 + (l & 15)];
+            b[e] = sb[((l >> 4) * 4 + e) * LD + r * 16 + (l & 15)];
+        }
+        *(floatx4*)(out + (size_t)(DR * 64 + i) * 4) = k;
+        *(floatx4*)(oB + (size_t)i * 4)              = b;
+    }
+    if (tid < 64) {
+        *(floatx4*)(oW + tid * 4) = *(const floatx4*)(wk + (tid & 15) * kChunkT + (tid >> 4) * 4);
+    }
+}
+
+// grid (nseq, heads, ceil(vdim / 64)), 384 threads: waves 0 - 3 -> 16 value columns each, waves 4 and 5 bring blocks and values into LDS by DMA, a ring of stages
+// deep.  SILU: on the values; DELTA: blocks of delta_blocks_kernel.  The walk is as long as the longest prompt, with one wave a SIMD for the products: what
+// bounds it is that wave's issue slots, so the products' waves do nothing else (with their own share of the DMA, about sixty instructions a chunk for addresses,
+// lightning took 180 us and the delta rule 287).  8 prompts of ~1000 tokens, 16 heads of 128 / 128: lightning 190 us -> 143, the delta rule 226 (with its
+// blocks 458; a token at a time on the vector units 1090)
+constexpr int kValueStage = kChunkT * 64;  // floats of the workgroup's 64 value columns
+constexpr int decay_chunk_stages(int dr, bool delta)
+{
+    return dr > 8 && delta ? 2 : 3;
+}
+constexpr int decay_chunks_lds(int dr, bool delta)
+{
+    return decay_chunk_stages(dr, delta) * (decay_block_floats_of(dr, delta) + kValueStage) * 4;
+}
+// 64 consecutive words of LDS from 64 addresses
+__device__ __forceinline__ void chunk_dma4(__amdgpu_buffer_rsrc_t rs, int voff, unsigned lds)
+{
+    unsigned keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %2\n\ts_nop 0\n\t"
+                 "buffer_load_dword %1, %3, 0 offen lds\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep)
+                 : "v"(voff), "s"(lds), "s"(rs)
+                 : "memory");
+}
+template<int DR, bool SILU, bool DELTA>
+__global__ __launch_bounds__(384) void decay_chunks_kernel(StateMixParams p)
+{
+    constexpr int NC = kStateNC, WV = kStateCW * kStateNC, BF = decay_block_floats_of(DR, DELTA), DP = DR * 16, NB = decay_chunk_stages(DR, DELTA);
+    extern __shared__ __attribute__((aligned(16))) char chunk_lds[];
+    const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int D = p.dim, V = p.vdim, dq = (D + 7) / 8, ncb = (V + WV - 1) / WV, cb = blockIdx.z * 4 + wave;
+    const bool wave_on = wave < 4 && cb < ncb;
     const int row0 = p.cu_q[s] - p.cu_q[0], q_len = p.cu_q[s + 1] - p.cu_q[s];
     const int pos0 = p.k_len[s] - q_len, g = lane >> 4, col = cb * 16 + (lane & 15);
     int       slot = p.seq_slot ? p.seq_slot[s] : p.slot0 + s;
     if (p.active && !p.active[s]) {
         slot = p.park_slot;
     }
-    float* slab = p.state + (size_t)slot * p.slot_stride + p.layer_offset + ((size_t)h * ncb + cb) * dq * 64 * NC;
+    float* slab = p.state + (size_t)slot * p.slot_stride + p.layer_offset + ((size_t)h * ncb + (wave_on ? cb : 0)) * dq * 64 * NC;
     // element (d, column) of the slab as state_mix_kernel keeps it
     auto at = [&](int d) { return ((d % dq) * NC + (lane & 15) % NC) * 64 + d / dq * kStateCW + (lane & 15) / NC; };
     floatx4 S[DR];
@@ -508,96 +680,164 @@ __global__ __launch_bounds__(256) void decay_chunks_kernel(StateMixParams p)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int d = r * 16 + g * 4 + i;
-            S[r][i]     = pos0 > 0 && d < D ? slab[at(d)] : 0.f;
+            S[r][i]     = wave_on && pos0 > 0 && d < D ? slab[at(d)] : 0.f;
         }
     }
-    const size_t bf  = decay_block_floats(D);
-    const float* blk = p.blocks + (decay_chunk_index(s, row0, 0) * p.heads + h) * bf;
-    struct Operands {
-        floatx4 q[DR], k[DR], f[DR], a, v;
-    };
-    auto fetch = [&](Operands& o, int t0, const float* b) {
+    const int    chunks = (q_len + kChunkT - 1) / kChunkT;
+    const float* blk    = p.blocks + (decay_chunk_index(s, row0, 0) * p.heads + h) * BF;
+    const size_t next   = (size_t)p.heads * BF;
+    const float* val    = p.proj + (size_t)row0 * p.ld + p.c_v + h * V;
+    const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)chunk_lds);
+    const int      vcol = min((int)blockIdx.z * 64 + lane, V - 1) * 4;
+    constexpr int  kStage = (BF + kValueStage) * 4, kPieces = BF / 256, kOps = kPieces / 2 + kChunkT / 2;  // bytes; pieces of 1 KB; the fewest operations of a wave
+    auto dma = [&](int c) {  // waves 4, 5: every other piece, every other token
+        const unsigned dst = lds0 + __builtin_amdgcn_readfirstlane(c % NB * kStage);
+        const auto     rs  = __builtin_amdgcn_make_buffer_rsrc((void*)(blk + (size_t)c * next), 0, BF * 4, 0x00020000);
 #pragma unroll
-        for (int r = 0; r < DR; ++r) {
-            o.q[r] = *(const floatx4*)(b + (size_t)(r * 64 + lane) * 4);
-            o.k[r] = *(const floatx4*)(b + (size_t)((DR + r) * 64 + lane) * 4);
-            o.f[r] = *(const floatx4*)(b + DR * 64 * 4 * 2 + 256 + r * 16 + g * 4);
-        }
-        o.a = *(const floatx4*)(b + DR * 64 * 4 * 2 + lane * 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int t = min(t0 + g * 4 + e, q_len - 1);  // (keys behind the portion are zero: any finite value will do)
-            o.v[e]      = p.proj[(size_t)(row0 + t) * p.ld + p.c_v + h * V + min(col, V - 1)];
-        }
-    };
-    auto step = [&](Operands& o, int t0) {
-        if constexpr (SILU) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                o.v[e] = sm_silu(o.v[e]);
+        for (int i = 0; i < kPieces; i += 2) {
+            const int at = __builtin_amdgcn_readfirstlane((i + wave - 4) * 1024);
+            if (at < BF * 4) {
+                stream_dma16(rs, lane * 16, at, dst + at);
             }
         }
-        floatx4 y[4], ya = {0.f, 0.f, 0.f, 0.f};  // short chains of sums: independent products for the matrix core and less rounding
+        const int  last = min(kChunkT, q_len - c * kChunkT) - 1;  // (keys behind the portion are zero: any finite value will do)
+        const auto rv   = __builtin_amdgcn_make_buffer_rsrc((void*)(val + (size_t)c * kChunkT * p.ld), 0, (last * p.ld + V) * 4, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            y[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < kChunkT; i += 2) {
+            const int t = __builtin_amdgcn_readfirstlane(i + wave - 4);
+            chunk_dma4(rv, min(t, last) * p.ld * 4 + vcol, dst + BF * 4 + t * 256);
         }
-#pragma unroll
-        for (int r = 0; r < DR; ++r) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[r][i], S[r][i], y[i], 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            ya = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[e], o.v[e], ya, 0, 0, 0);
-        }
-#pragma unroll
-        for (int r = 0; r < DR; ++r) {
-            S[r] *= o.f[r];
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
+    };
+    float* out  = p.out + (size_t)(row0 + g * 4) * p.ldo + h * V + col;
+    auto   step = [&](const float* b, floatx4 vv, int t0) {
+        auto    lane4 = [&](int at) { return *(const floatx4*)(b + at + lane * 4); };
+        const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+        floatx4       add[DR], y[4], z[4], ya[2], yb[2];  // short chains of sums: independent products for the matrix core and less rounding
+        auto outer = [&](int at, const floatx4& x) {  // add += (scaled keys at `at`)^T x: neighbouring products meet different sums
+            floatx4 k[DR];
 #pragma unroll
             for (int r = 0; r < DR; ++r) {
-                S[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[r][e], o.v[e], S[r], 0, 0, 0);
+                k[r] = lane4(at + r * 256);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int r = 0; r < DR; ++r) {
+                    add[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[r][e], x[e], add[r], 0, 0, 0);
+                }
+            }
+        };
+        auto inner = [&](floatx4 (&o)[2], int at, const floatx4& x) {  // o += (triangle at `at`) x
+            const floatx4 a = lane4(at);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o[e & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], x[e], o[e & 1], 0, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            y[i] = z[i] = ya[i & 1] = yb[i & 1] = zero;
+        }
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {
+            add[r] = zero;
+        }
+        constexpr int oA = DR * 512, oF = oA + 256, oU = oF + DP, oB = oU + DR * 256, oAb = oB + DR * 256, oW = oAb + 256;
+        if constexpr (DELTA) {
+            const floatx4 w = lane4(oW);
+#pragma unroll
+            for (int r = 0; r < DR; ++r) {
+                const floatx4 u = lane4(oU + r * 256);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    z[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(u[i], S[r][i], z[i], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                z[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], vv[e], z[e], 0, 0, 0);
             }
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int t = t0 + g * 4 + i;
-            if (t < q_len && col < V) {
-                p.out[(size_t)(row0 + t) * p.ldo + h * V + col] = ((y[0][i] + y[1][i]) + (y[2][i] + y[3][i])) + ya[i];
+        for (int r = 0; r < DR; ++r) {  // (vector work between the products, which take 32 cycles each)
+            const floatx4 q = lane4(r * 256);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[i], S[r][i], y[i], 0, 0, 0);
+            }
+            if constexpr (SILU) {
+#pragma unroll
+                for (int e = r * 4 / DR; e < (r + 1) * 4 / DR; ++e) {
+                    vv[e] = sm_silu(vv[e]);
+                }
+            }
+        }
+        inner(ya, oA, vv);
+        outer(DR * 256, vv);
+        if constexpr (DELTA) {
+            const floatx4 e = -((z[0] + z[1]) + (z[2] + z[3]));
+            inner(yb, oAb, e);
+            outer(oB, e);
+        }
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {  // (one rounding of the state a chunk)
+            const floatx4 f = *(const floatx4*)(b + oF + r * 16 + g * 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                S[r][i] = fmaf(S[r][i], f[i], add[r][i]);
+            }
+        }
+        const floatx4 sum = ((y[0] + y[1]) + (y[2] + y[3])) + ((ya[0] + ya[1]) + (yb[0] + yb[1]));
+        float* o = out + (size_t)t0 * p.ldo;
+        if (col < V) {
+            if (t0 + kChunkT <= q_len) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    o[i * p.ldo] = sum[i];
+                }
+            }
+            else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (t0 + g * 4 + i < q_len) {
+                        o[i * p.ldo] = sum[i];
+                    }
+                }
             }
         }
     };
-    const size_t next = (size_t)p.heads * bf;
-    if constexpr (DR <= 8) {  // the next chunk's operands are in flight under this chunk's products
-        Operands a, b;
-        if (q_len > 0) {
-            fetch(a, 0, blk);
+    if (wave >= 4) {
+        for (int c = 0; c < NB - 1 && c < chunks; ++c) {
+            dma(c);
         }
-        for (int t0 = 0; t0 < q_len; t0 += 2 * kChunkT, blk += 2 * next) {
-            const bool more = t0 + kChunkT < q_len;
-            if (more) {
-                fetch(b, t0 + kChunkT, blk + next);
+        for (int c = 0; c < chunks; ++c) {
+            if (NB > 2 && c + NB - 2 < chunks) {  // the stages behind this one may still be on their way
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * kOps) : "memory");
             }
-            step(a, t0);
-            if (t0 + 2 * kChunkT < q_len) {
-                fetch(a, t0 + 2 * kChunkT, blk + 2 * next);
+            else {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
-            if (more) {
-                step(b, t0 + kChunkT);
+            __syncthreads();  // stage c has landed, and nobody reads the stage before it any more
+            if (c + NB - 1 < chunks) {
+                dma(c + NB - 1);
             }
+        }
+        return;
+    }
+    for (int c = 0; c < chunks; ++c) {
+        __syncthreads();
+        if (wave_on) {
+            const float* b = (const float*)chunk_lds + c % NB * (kStage / 4);
+            floatx4      v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = b[BF + (g * 4 + e) * 64 + wave * 16 + (lane & 15)];
+            }
+            step(b, v, c * kChunkT);
         }
     }
-    else {
-        Operands a;
-        for (int t0 = 0; t0 < q_len; t0 += kChunkT, blk += next) {
-            fetch(a, t0, blk);
-            step(a, t0);
-        }
+    if (!wave_on) {
+        return;
     }
 #pragma unroll
     for (int r = 0; r < DR; ++r) {
@@ -611,26 +851,41 @@ __global__ __launch_bounds__(256) void decay_chunks_kernel(StateMixParams p)
     }
 }
 
+template<int DR, int KIND>
+static int launch_decay_chunks_dr(const StateMixParams& p, hipStream_t st)
+{
+    constexpr bool DELTA = KIND == kStateDelta;
+    constexpr int  lds    = decay_chunks_lds(DR, DELTA);
+    const int      chunks = (p.max_q_len + kChunkT - 1) / kChunkT;
+    const dim3     gb(p.nseq * chunks, p.heads), gc(p.nseq, p.heads, (p.vdim + 63) / 64);
+    if constexpr (DELTA) {
+        if (const int rc = ensure_dynamic_lds((const void*)delta_blocks_kernel<DR>, delta_blocks_lds(DR))) {
+            return rc;
+        }
+        delta_blocks_kernel<DR><<<gb, 256, delta_blocks_lds(DR), st>>>(p, chunks);
+    }
+    else {
+        decay_blocks_kernel<DR, KIND><<<gb, 256, 0, st>>>(p, chunks);
+    }
+    const auto k = decay_chunks_kernel<DR, KIND == kStateLinear, DELTA>;
+    if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {
+        return rc;
+    }
+    k<<<gc, 384, lds, st>>>(p);
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
 template<int KIND>
 static int launch_decay_chunks(const StateMixParams& p, hipStream_t st)
 {
-    TM_REQUIRE(p.blocks && p.blocks_floats >= decay_workspace_floats(p.rows, p.nseq, p.heads, p.dim), "state mixer: chunk workspace");
-    const int  chunks = (p.max_q_len + kChunkT - 1) / kChunkT;
-    const dim3 gb(p.nseq * chunks, p.heads), gc(p.nseq, p.heads, (p.vdim + 63) / 64);
-#define TM_CHUNKS(DR_)                                                  \
-    case DR_:                                                           \
-        decay_blocks_kernel<DR_, KIND><<<gb, 256, 0, st>>>(p, chunks); \
-        decay_chunks_kernel<DR_, KIND == kStateLinear><<<gc, 256, 0, st>>>(p); \
-        break;
+    TM_REQUIRE(p.blocks && p.blocks_floats >= decay_workspace_floats(p.rows, p.nseq, p.heads, p.dim, KIND == kStateDelta), "state mixer: chunk workspace");
     switch (decay_tiles(p.dim)) {
-        TM_CHUNKS(2)
-        TM_CHUNKS(4)
-        TM_CHUNKS(8)
-        TM_CHUNKS(16)
+        case 2: return launch_decay_chunks_dr<2, KIND>(p, st);
+        case 4: return launch_decay_chunks_dr<4, KIND>(p, st);
+        case 8: return launch_decay_chunks_dr<8, KIND>(p, st);
+        default: return launch_decay_chunks_dr<16, KIND>(p, st);
     }
-#undef TM_CHUNKS
-    TM_HIP_CHECK(hipGetLastError());
-    return 0;
 }
 
 int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
@@ -657,6 +912,10 @@ int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
     }
     if (p.max_q_len > 1 && kind == kStateBonus) {
         return launch_decay_chunks<kStateBonus>(p, st);
+    }
+    // (the walk costs 0.9 us a token, the blocks and a chunk or two 34: 8 x 16 tokens 19.5, 8 x 17 in chunks 34, 1 x 16 17, 1 x 32 in chunks 31)
+    if (p.max_q_len > 2 * kChunkT && kind == kStateDelta) {
+        return launch_decay_chunks<kStateDelta>(p, st);
     }
     const int  wcols = 4 * kStateCW * kStateNC;  // value columns of a workgroup
     const dim3 grid(p.nseq, p.heads, (p.vdim + wcols - 1) / wcols);
