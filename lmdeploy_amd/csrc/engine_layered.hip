@@ -1586,7 +1586,14 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
                                                        delta ? H : 1, delta ? s.dim : L.n_att, m.norm_eps, st)));
     }
     TM_PROF(P_GEMM_O, TM_TRY(launch_dense_linear(L.wo, lm.d_cat, lm.ldcat, lm.d_y, W, M, kDenseScaleF32, 1.f, st)));
-    TM_PROF(P_RES_NORM, TM_TRY(launch_layernorm_add_f32(lm.d_res, lm.d_h1, lm.ldw, lm.elem, lm.d_y, L.norm1, L.norm1_b, m.norm_eps, M, W, st)));
+    const bool router = s.mlp == TM_MLP_MOE && layernorm_add_router_ok(lm.d_res, lm.d_h1, lm.ldw, lm.elem, lm.d_y, L.norm1, L.norm1_b, M, W, L.router);
+    if (router) {
+        TM_PROF(P_RES_NORM, TM_TRY(launch_layernorm_add_router_f32(lm.d_res, lm.d_h1, lm.ldw, lm.elem, lm.d_y, L.norm1, L.norm1_b, m.norm_eps, M, W, L.router, lm.d_proj,
+                                                                   lm.ldproj, st)));
+    }
+    else {
+        TM_PROF(P_RES_NORM, TM_TRY(launch_layernorm_add_f32(lm.d_res, lm.d_h1, lm.ldw, lm.elem, lm.d_y, L.norm1, L.norm1_b, m.norm_eps, M, W, st)));
+    }
     if (s.mlp == TM_MLP_NONE) {
         return 0;
     }
@@ -1599,7 +1606,9 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
     }
     else {
         const int k = s.top, E = s.experts;
-        TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_dense_linear(L.router, lm.d_h1, lm.ldw, lm.d_proj, lm.ldproj, M, kDenseScaleF32, 1.f, st)));
+        if (!router) {
+            TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_dense_linear(L.router, lm.d_h1, lm.ldw, lm.d_proj, lm.ldproj, M, kDenseScaleF32, 1.f, st)));
+        }
         // the rows in the experts' order; the shared expert: item E of the batched products over a copy of all rows behind the routed ones
         TM_PROF(P_GEMM_GATE_UP, TM_TRY(launch_moe_softmax_route_gather(lm.d_topk_ids, lm.d_topk_w, lm.d_offsets, lm.d_f2n, lm.d_en2f, lm.d_proj, lm.ldproj, lm.d_moe_x,
                                                                        lm.ldw, lm.d_h1, lm.ldw, lm.elem, M, W, E, k, s.router_scale, L.shared_fused, st)));

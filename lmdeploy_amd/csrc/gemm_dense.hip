@@ -281,19 +281,7 @@ struct DenseEpi {
 };
 
 // ---- weight images ----------------------------------------------------------------------------------------------------------------
-// src: bf16 [rows][cols] (checkpoint bytes) -> dst[(row0 + r) * Kp + col0 + c], T = bf16 (copy) or float (exact widening)
-// Images are stored in FRAGMENT ORDER: the 16 rows x 64 bytes block (n / 16, k / step) is one contiguous KB laid out as the 64 lanes of
-// its MFMA fragment (16 bytes each: lane = piece * 16 + n % 16), blocks of one 16-row tile consecutive along k -- a wave's fragment
-// load is one contiguous KB and a workgroup streams whole contiguous runs of HBM instead of 64-byte pieces of 16 rows
-// (from stream_turn's step on)
-template<class T>
-__host__ __device__ inline size_t dense_frag_index(int n, int k, int steps)
-{
-    constexpr int E = 16 / sizeof(T), S = 4 * E;  // elements of a 16-byte piece, of a step
-    const int     at = k / S + stream_turn(n >> 4, steps);
-    return (((size_t)(n >> 4) * steps + (at < steps ? at : at - steps)) * 64 + (k % S) / E * 16 + (n & 15)) * E + k % E;
-}
-
+// src: bf16 [rows][cols] (checkpoint bytes) -> dst at dense_frag_index of (row0 + r, col0 + c), T = bf16 (copy) or float (exact widening)
 template<class T>
 __global__ void dense_place_kernel(T* __restrict__ dst, int steps, int row0, int col0, const __bf16* __restrict__ src, int rows, int cols,
                                    int transpose, int half)

@@ -833,6 +833,19 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
     }
 }
 
+// ---- weight images of bf16 and fp32 linears ----------------------------------------------------------------------------------------
+// Images are stored in FRAGMENT ORDER: the 16 rows x 64 bytes block (n / 16, k / step) is one contiguous KB laid out as the 64 lanes of
+// its MFMA fragment (16 bytes each: lane = piece * 16 + n % 16), blocks of one 16-row tile consecutive along k -- a wave's fragment
+// load is one contiguous KB and a workgroup streams whole contiguous runs of HBM instead of 64-byte pieces of 16 rows
+// (from stream_turn's step on)
+template<class T>
+__host__ __device__ inline size_t dense_frag_index(int n, int k, int steps)
+{
+    constexpr int E = 16 / sizeof(T), S = 4 * E;  // elements of a 16-byte piece, of a step
+    const int     at = k / S + stream_turn(n >> 4, steps);
+    return (((size_t)(n >> 4) * steps + (at < steps ? at : at - steps)) * 64 + (k % S) / E * 16 + (n & 15)) * E + k % E;
+}
+
 // ---- which kernel, which shape -------------------------------------------------------------------------------------------------------
 // (row tiles, column tiles a wave, column waves, k-phases) of the skinny kernels that exist: 64 columns a workgroup of four waves, 96 of six and 128 of eight where those
 // fill the CUs more evenly or read x less often, and 128 columns where a wave needs a pair of column tiles.  k-phases gave nothing at 184 sizes.

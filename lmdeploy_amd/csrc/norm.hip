@@ -10,6 +10,7 @@
 #include "tm_common.h"
 #include "tm_kernels.h"
 #include "norm_row.h"
+#include "gemm_stream.h"  // dense_frag_index
 #include <initializer_list>
 
 namespace tmk {
@@ -394,19 +395,30 @@ __global__ __launch_bounds__(256) void layernorm_f32_kernel(T* __restrict__ y, i
     }
 }
 
+struct RouterRows {  // a router's bf16 image and where its logits go
+    const void* w       = nullptr;
+    int         steps   = 0;
+    float*      logits  = nullptr;
+    int         ld      = 0, experts = 0;
+};
+
 // the same with everything it reads in registers ahead of the reductions (H <= 256 * NR), V floats at a time: V = 4 for multiples of four on 16-byte
 // aligned operands (8 rows of 2048 with ADD: 6.3 us a launch where weights and stream were read after the reductions, 5.2 now), V = 1 otherwise
 // MOE: the row is what a routed mixture's experts leave (and a shared expert's result), summed here as moe_combine_f32_kernel does: 8 rows of 2048, two experts, 4.6 and
 // 4.1 us apart, 4.7 together
-template<class T, bool ADD, int NR, int V, bool MOE = false>
+// RE > 0: the new row also meets a router of up to RE experts (bf16 products, fp32 sums, as the product's own launch), whose weights are asked for with the row.  8 rows of
+// 2048, 8 experts: 4.2 and 4.6 us apart, 4.3 together
+template<class T, bool ADD, int NR, int V, bool MOE = false, int RE = 0>
 __global__ __launch_bounds__(256) void layernorm_f32_reg_kernel(T* __restrict__ y, int ldy, float* __restrict__ xs, const float* __restrict__ src,
                                                                 const int* __restrict__ rows, const float* __restrict__ w,
-                                                                const float* __restrict__ b, float eps, int H, MoeRows mr)
+                                                                const float* __restrict__ b, float eps, int H, MoeRows mr, RouterRows rt)
 {
     constexpr int NQ = NR / V;
     typedef float FV __attribute__((ext_vector_type(V)));
     typedef T     TV __attribute__((ext_vector_type(V)));
-    __shared__ float red[4];
+    __shared__ float red[4], part[4][RE > 0 ? RE : 1];
+    TV           rw[NQ][RE > 0 ? RE : 1];
+    float        dot[RE > 0 ? RE : 1];
     const int    m = blockIdx.x;
     const float* r = src + (size_t)(rows ? rows[m] : m) * H;
     FV           v[NQ], wv[NQ], bv[NQ], xv[NQ];
@@ -423,6 +435,19 @@ __global__ __launch_bounds__(256) void layernorm_f32_reg_kernel(T* __restrict__ 
         bv[q]       = *(const FV*)(b + i);
         if constexpr (ADD) {
             xv[q] = *(const FV*)(xs + (size_t)m * H + i);
+        }
+        if constexpr (RE > 0) {
+            const T* at = (const T*)rt.w + dense_frag_index<T>(0, i, rt.steps);  // (experts of a tile lie side by side)
+#pragma unroll
+            for (int e = 0; e < RE; ++e) {
+                rw[q][e] = *(const TV*)(at + e * 8);
+            }
+        }
+    }
+    if constexpr (RE > 0) {
+#pragma unroll
+        for (int e = 0; e < RE; ++e) {
+            dot[e] = 0.f;
         }
     }
     if constexpr (MOE) {
@@ -487,25 +512,50 @@ __global__ __launch_bounds__(256) void layernorm_f32_reg_kernel(T* __restrict__ 
                 *(FV*)(xs + (size_t)m * H + i) = o;
             }
             *(TV*)(y + (size_t)m * ldy + i) = t;
+            if constexpr (RE > 0) {
+#pragma unroll
+                for (int e = 0; e < RE; ++e) {
+#pragma unroll
+                    for (int c = 0; c < V; ++c) {
+                        dot[e] = fmaf((float)t[c], (float)rw[q][e][c], dot[e]);
+                    }
+                }
+            }
+        }
+    }
+    if constexpr (RE > 0) {
+#pragma unroll
+        for (int e = 0; e < RE; ++e) {
+            dot[e] = group_sum<64>(dot[e]);
+        }
+        if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+            for (int e = 0; e < RE; ++e) {
+                part[threadIdx.x >> 6][e] = dot[e];
+            }
+        }
+        __syncthreads();
+        if ((int)threadIdx.x < rt.experts) {
+            rt.logits[(size_t)m * rt.ld + threadIdx.x] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
         }
     }
 }
 
-template<class T, bool ADD, int V, bool MOE = false>
+template<class T, bool ADD, int V, bool MOE = false, int RE = 0>
 static void launch_layernorm_reg(T* y, int ldy, float* xs, const float* src, const int* rows, const float* w, const float* b, float eps, int M, int H,
-                                 hipStream_t st, const MoeRows& mr = {})
+                                 hipStream_t st, const MoeRows& mr = {}, const RouterRows& rt = {})
 {
     if (H <= 1024) {
-        layernorm_f32_reg_kernel<T, ADD, 4, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
+        layernorm_f32_reg_kernel<T, ADD, 4, V, MOE, RE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr, rt);
     }
     else if (H <= 2048) {
-        layernorm_f32_reg_kernel<T, ADD, 8, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
+        layernorm_f32_reg_kernel<T, ADD, 8, V, MOE, RE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr, rt);
     }
     else if (H <= 4096) {
-        layernorm_f32_reg_kernel<T, ADD, 16, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
+        layernorm_f32_reg_kernel<T, ADD, 16, V, MOE, RE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr, rt);
     }
-    else {
-        layernorm_f32_reg_kernel<T, ADD, 32, V, MOE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr);
+    else if constexpr (RE == 0) {
+        layernorm_f32_reg_kernel<T, ADD, 32, V, MOE, RE><<<M, 256, 0, st>>>(y, ldy, xs, src, rows, w, b, eps, H, mr, rt);
     }
 }
 
@@ -553,6 +603,30 @@ int launch_layernorm_add_f32(float* x, void* h, int ldh, int h_elem_bytes, const
     }
     else {
         launch_layernorm_any<float, true>((float*)h, ldh, x, r, nullptr, w, b, eps, M, H, st);
+    }
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
+// few rows: a workgroup a row brings the router's weights once a row, which more rows than CUs would wait for
+bool layernorm_add_router_ok(const float* x, const void* h, int ldh, int h_elem_bytes, const float* r, const float* w, const float* b, int M, int H, const DenseWeight& router)
+{
+    return M <= 256 && h_elem_bytes == 2 && H <= 4096 && router.N <= 16 && router.K == H && router.count == 1 && norm_by_four(H, ldh, h_elem_bytes, {x, r, w, b}, {h});
+}
+int launch_layernorm_add_router_f32(float* x, void* h, int ldh, int h_elem_bytes, const float* r, const float* w, const float* b, float eps, int M, int H,
+                                    const DenseWeight& router, float* logits, int ld, hipStream_t st)
+{
+    TM_REQUIRE(x && h && r && w && b && ldh >= H && logits && ld >= router.N, "layernorm_add_router_f32: operands");
+    TM_REQUIRE(layernorm_add_router_ok(x, h, ldh, h_elem_bytes, r, w, b, M, H, router), "layernorm_add_router_f32: sizes");
+    if (M == 0) {
+        return 0;
+    }
+    const RouterRows rt{router.w, router.Kp / 32, logits, ld, router.N};
+    if (router.N <= 8) {
+        launch_layernorm_reg<__bf16, true, 4, false, 8>((__bf16*)h, ldh, x, r, nullptr, w, b, eps, M, H, st, {}, rt);
+    }
+    else {
+        launch_layernorm_reg<__bf16, true, 4, false, 16>((__bf16*)h, ldh, x, r, nullptr, w, b, eps, M, H, st, {}, rt);
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;

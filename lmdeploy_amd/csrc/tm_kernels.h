@@ -659,6 +659,10 @@ int launch_layernorm_f32(void* y, int ldy, int out_elem_bytes, const float* x, c
                          int H, hipStream_t st);
 int launch_layernorm_add_f32(float* x, void* h, int ldh, int h_elem_bytes, const float* r, const float* w, const float* b, float eps, int M, int H,
                              hipStream_t st);
+// ... and the updated row's router logits [M][ld], fp32: one launch instead of two at few rows (layernorm_add_router_ok: bf16, up to 16 experts)
+bool layernorm_add_router_ok(const float* x, const void* h, int ldh, int h_elem_bytes, const float* r, const float* w, const float* b, int M, int H, const DenseWeight& router);
+int  launch_layernorm_add_router_f32(float* x, void* h, int ldh, int h_elem_bytes, const float* r, const float* w, const float* b, float eps, int M, int H,
+                                     const DenseWeight& router, float* logits, int ld, hipStream_t st);
 // RMS norm in groups on the fp32 stream: the row is split into `groups` equal consecutive parts, each divided by its own
 // sqrt(mean(part^2) + eps), the whole times w.  launch_group_rmsnorm_f32: y[m] = GN(x[rows ? rows[m] : m]);
 // launch_group_rmsnorm_add_f32: x[m] += GN(r[m]) and the updated row also goes to h in the activation type.  r2 != nullptr: the normed
