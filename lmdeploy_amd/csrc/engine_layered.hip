@@ -1556,18 +1556,22 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
     }
     else {
         const bool delta = s.mixer == TM_MIXER_DELTA;
-        if (delta) {  // decay logits = w2 tanh(w1 h) + w0; then unit keys, removal rates and decays as the recurrence reads them
+        if (delta) {  // decay logits = w2 tanh(w1 h) + w0
             TM_PROF(P_KV_STORE, TM_TRY(launch_act_cast_f32(lm.d_lora, lm.ldlora, lm.elem, lm.d_proj + L.c_w1, lm.ldproj, M, s.decay_rank, 1, st)));
             DenseCall c;
             c.epi  = kDenseBiasF32;
             c.bias = L.w0;
             TM_PROF(P_GEMM_QKV, TM_TRY(launch_dense_call(L.w2, lm.d_lora, lm.ldlora, lm.d_wdec, lm.ldmix, M, c, st)));
-            TM_PROF(P_KV_STORE, TM_TRY(launch_delta_prep(lm.d_proj, lm.ldproj, L.c_k, L.c_a, lm.d_wdec, lm.ldmix, lm.d_aux, lm.ldmix, M, H, s.dim, st)));
         }
         for (int i = 0; i < nparts; ++i) {
             const LmPart&  P = parts[i];
             StateMixParams sp;
             sp.max_q_len = P.decode ? 1 : std::max(1, P.max_q_len);
+            sp.raw       = delta && state_mix_chunks(sp.max_q_len);
+            if (delta && !sp.raw) {  // unit keys, removal rates and decays as the walk reads them
+                TM_PROF(P_KV_STORE, TM_TRY(launch_delta_prep(lm.d_proj + (size_t)P.row0 * lm.ldproj, lm.ldproj, L.c_k, L.c_a, lm.d_wdec + (size_t)P.row0 * lm.ldmix, lm.ldmix,
+                                                             lm.d_aux + (size_t)P.row0 * lm.ldmix, lm.ldmix, P.rows, H, s.dim, st)));
+            }
             sp.nseq = P.nseq, sp.cu_q = P.cu_q, sp.k_len = P.k_len, sp.seq_slot = P.seq_slot, sp.slot0 = P.slot0, sp.active = P.active;
             sp.park_slot   = e->cfg.max_batch_size;
             sp.state       = lm.d_state;

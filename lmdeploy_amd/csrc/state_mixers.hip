@@ -41,6 +41,16 @@ __device__ __forceinline__ float sm_silu(float z)
     return z / (1.f + expf(-z));
 }
 
+// the delta rule's removal vector a u and decay from their logits
+__device__ __forceinline__ float delta_rate(float u, float logit)
+{
+    return u / (1.f + expf(-logit));
+}
+__device__ __forceinline__ float delta_decay(float logit)
+{
+    return expf(-0.60653065971263342f / (1.f + expf(-logit)));
+}
+
 // staged vectors per token: q, k; the delta rule's decays, a u and u; the forget gates; the bonus recurrence's decays and u k
 __host__ __device__ constexpr int state_vectors(int kind)
 {
@@ -499,7 +509,9 @@ constexpr int delta_blocks_lds(int dr)
 {
     return (5 * kChunkT * (dr * 16 + 4) + 2 * kChunkT * kChunkT) * 4;
 }
-template<int DR>
+// RAW: key, removal-rate logits and decay logits come as the projections left them and are turned here as delta_prep_kernel turns them (8 x ~970 tokens, 16 heads of
+// 128: 94 us of that launch and 236 of this one, 261 together)
+template<int DR, bool RAW>
 __global__ __launch_bounds__(256) void delta_blocks_kernel(StateMixParams p, int chunks)
 {
     constexpr int DP = DR * 16, LD = DP + 4, NM = (DP + 63) / 64;
@@ -523,9 +535,26 @@ __global__ __launch_bounds__(256) void delta_blocks_kernel(StateMixParams p, int
         sk[t * LD + d] = ok ? pr[p.c_k] : 0.f;
         sb[t * LD + d] = ok ? pr[p.c_a] : 0.f;
         sf[t * LD + d] = ok ? p.decay_w[row * p.ld_w + h * D + d] : 1.f;
-        su[t * LD + d] = ok ? p.unit[row * p.ld_u + h * D + d] : 0.f;
+        if constexpr (!RAW) {
+            su[t * LD + d] = ok ? p.unit[row * p.ld_u + h * D + d] : 0.f;
+        }
     }
     __syncthreads();
+    if constexpr (RAW) {
+        const int t = tid >> 4, sl = tid & 15;  // 16 lanes a token
+        float     ss = 0.f;
+        for (int d = sl; d < DP; d += 16) {
+            ss = fmaf(sk[t * LD + d], sk[t * LD + d], ss);
+        }
+        const float inv = 1.0f / sqrtf(group_sum<16>(ss) + 1e-6f);
+        for (int d = sl; d < DP; d += 16) {
+            const float u  = sk[t * LD + d] * inv;
+            su[t * LD + d] = u;
+            sb[t * LD + d] = delta_rate(u, sb[t * LD + d]);
+            sf[t * LD + d] = t < nt && d < D ? delta_decay(sf[t * LD + d]) : 1.f;
+        }
+        __syncthreads();
+    }
     {   // the four A: 16 lanes share a key j, each with its channels; the key and b decay as t moves on
         const int j = tid >> 4, sl = tid & 15;
         floatx4   k[NM], b[NM];
@@ -637,7 +666,7 @@ __global__ __launch_bounds__(256) void delta_blocks_kernel(StateMixParams p, int
 // deep.  SILU: on the values; DELTA: blocks of delta_blocks_kernel.  The walk is as long as the longest prompt, with one wave a SIMD for the products: what
 // bounds it is that wave's issue slots, so the products' waves do nothing else (with their own share of the DMA, about sixty instructions a chunk for addresses,
 // lightning took 180 us and the delta rule 287).  8 prompts of ~1000 tokens, 16 heads of 128 / 128: lightning 190 us -> 143, the delta rule 226 (with its
-// blocks 458; a token at a time on the vector units 1090)
+// blocks and what prepares them 487; a token at a time on the vector units 1184)
 constexpr int kValueStage = kChunkT * 64;  // floats of the workgroup's 64 value columns
 constexpr int decay_chunk_stages(int dr, bool delta)
 {
@@ -859,10 +888,11 @@ static int launch_decay_chunks_dr(const StateMixParams& p, hipStream_t st)
     const int      chunks = (p.max_q_len + kChunkT - 1) / kChunkT;
     const dim3     gb(p.nseq * chunks, p.heads), gc(p.nseq, p.heads, (p.vdim + 63) / 64);
     if constexpr (DELTA) {
-        if (const int rc = ensure_dynamic_lds((const void*)delta_blocks_kernel<DR>, delta_blocks_lds(DR))) {
+        const auto blocks = p.raw ? delta_blocks_kernel<DR, true> : delta_blocks_kernel<DR, false>;
+        if (const int rc = ensure_dynamic_lds((const void*)blocks, delta_blocks_lds(DR))) {
             return rc;
         }
-        delta_blocks_kernel<DR><<<gb, 256, delta_blocks_lds(DR), st>>>(p, chunks);
+        blocks<<<gb, 256, delta_blocks_lds(DR), st>>>(p, chunks);
     }
     else {
         decay_blocks_kernel<DR, KIND><<<gb, 256, 0, st>>>(p, chunks);
@@ -888,11 +918,17 @@ static int launch_decay_chunks(const StateMixParams& p, hipStream_t st)
     }
 }
 
+// the delta rule: the walk costs 0.9 us a token, the blocks and a chunk or two 34: 8 x 16 tokens 19.5, 8 x 17 in chunks 34, 1 x 16 17, 1 x 32 in chunks 31
+bool state_mix_chunks(int max_q_len)
+{
+    return max_q_len > 2 * kChunkT;
+}
+
 int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
 {
     TM_REQUIRE(p.nseq >= 0 && p.heads >= 1 && p.dim >= 1 && p.dim <= 256 && p.vdim >= 1 && p.max_q_len >= 1, "state mixer: sizes (dim <= 256)");
     TM_REQUIRE(p.cu_q && p.k_len && p.state && p.proj && p.out && p.ld >= 1 && p.ldo >= p.heads * p.vdim, "state mixer: operands");
-    TM_REQUIRE(kind == kStateDelta ? (p.decay_w && p.unit && p.ld_w >= p.heads * p.dim && p.ld_u >= p.heads * p.dim) :
+    TM_REQUIRE(kind == kStateDelta ? (p.decay_w && p.ld_w >= p.heads * p.dim && (p.raw || (p.unit && p.ld_u >= p.heads * p.dim))) :
                kind == kStateForget ? (p.f_bias && p.f_low) :
                kind == kStateBonus ? (p.decay_w && p.bonus && p.ld_w >= p.heads * p.dim) : ((kind == kStateLinear || kind == kStateRetention) && p.decay_h),
                "state mixer: decay operands");
@@ -913,8 +949,8 @@ int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
     if (p.max_q_len > 1 && kind == kStateBonus) {
         return launch_decay_chunks<kStateBonus>(p, st);
     }
-    // (the walk costs 0.9 us a token, the blocks and a chunk or two 34: 8 x 16 tokens 19.5, 8 x 17 in chunks 34, 1 x 16 17, 1 x 32 in chunks 31)
-    if (p.max_q_len > 2 * kChunkT && kind == kStateDelta) {
+    TM_REQUIRE(!p.raw || (kind == kStateDelta && state_mix_chunks(p.max_q_len)), "state mixer: logits only for chunks of the delta rule");
+    if (kind == kStateDelta && state_mix_chunks(p.max_q_len)) {
         return launch_decay_chunks<kStateDelta>(p, st);
     }
     const int  wcols = 4 * kStateCW * kStateNC;  // value columns of a workgroup
@@ -960,8 +996,8 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(float* __restrict__ pro
         const float u  = k[i] * inv;
         float&      a  = pr[c_a + h * D + i];
         float&      w  = decay[(size_t)t * ld_w + h * D + i];
-        a              = u / (1.f + expf(-a));
-        w              = expf(-0.60653065971263342f / (1.f + expf(-w)));
+        a              = delta_rate(u, a);
+        w              = delta_decay(w);
         unit[(size_t)t * ld_u + h * D + i] = u;
     }
 }

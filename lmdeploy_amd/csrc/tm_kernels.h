@@ -709,6 +709,7 @@ struct StateMixParams {
     const float* decay_h = nullptr;   // lightning: [heads]
     const float* decay_w = nullptr;   // delta: [rows][ld_w] decay per key channel
     const float* unit = nullptr;      // delta: [rows][ld_u] unit keys
+    int          raw = 0;             // delta in chunks: c_a and decay_w hold the logits that launch_delta_prep would turn, and unit is not read
     int          ld_w = 0, ld_u = 0;
     const float* inv_freq = nullptr;  // retention: queries and keys turn in their first rot_dims channels (channel i with i + rot_dims / 2) by
     int          rot_dims = 0;        // position * inv_freq[i]; keys are then multiplied by k_mult
@@ -752,6 +753,7 @@ int    launch_block_close(const BlockClose& c, hipStream_t st);
 size_t state_mix_floats(int heads, int dim, int vdim);  // floats of one layer's state in one slot
 size_t decay_workspace_floats(int rows, int nseq, int heads, int dim, bool delta);
 enum { kStateLinear = 0, kStateDelta = 1, kStateForget = 2, kStateRetention = 3, kStateBonus = 4 };
+bool   state_mix_chunks(int max_q_len);  // the delta rule runs portions of this length in chunks (and takes logits: StateMixParams::raw)
 int    launch_state_mix(const StateMixParams& p, int kind, hipStream_t st);
 int    launch_delta_prep(float* proj, int ld, int c_k, int c_a, float* decay, int ld_w, float* unit, int ld_u, int rows, int heads, int dim,
                          hipStream_t st);
