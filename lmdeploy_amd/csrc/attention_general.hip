@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256) void attn_rows_kernel(GeneralAttnParams p)
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     for (int bi = i0; bi < i1; ++bi) {
         const int   b    = ga_block_at(bi, nk, bf);
-        const char* base = (const char*)table[b] + p.layer_offset;
+        const char* base = global_ptr(table[b]) + p.layer_offset;
         const T*    kb   = (const T*)base + (size_t)ga_key_head(p, g) * p.block_len * D;
         const T*    vb   = (const T*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * p.block_len * V;  // [V][block_len]
         const int   n    = min(p.block_len, nkeys - b * p.block_len);
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(GeneralAttnParams p, in
     const int keep = ga_keep(p), bf = first_lo / 64, nk = ga_keep_blocks(p, first_lo, bf, 64);
     for (int bi = 0; bi < nk + nblk - bf; ++bi) {
         const int   b    = ga_block_at(bi, nk, bf);
-        const char* base = (const char*)table[b] + p.layer_offset;
+        const char* base = global_ptr(table[b]) + p.layer_offset;
         int         limit[RT], lower[RT];
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
@@ -814,7 +814,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, i
     }
     for (int bi = i0 + wave; bi < i1; bi += 4) {
         const int   b    = ga_block_at(bi, nk, bf);
-        const char* base = (const char*)table[b] + p.layer_offset;
+        const char* base = global_ptr(table[b]) + p.layer_offset;
         const int limit[1] = {pos - b * 64}, lower[1] = {first - b * 64};
         ga_block_step<DS, VT, 1, true, true>(qf, (const __bf16*)base + (size_t)ga_key_head(p, g) * 64 * D,
                                              (const __bf16*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V, D, V, limit, lower,
@@ -1202,8 +1202,8 @@ int launch_general_attention_decode(const GeneralAttnParams& p, hipStream_t st)
 // attn_decode_kernel's arrangement for an fp32 cache, v_mfma_f32_16x16x4: workgroup per (row, 16 heads of a key head, key split), each wave 16 of a block's 64
 // keys.  S^T = K Q^T with the channels of a step dealt so that a lane's four are one load, and P^T then stands in the registers that O^T += V^T P^T reads.
 // What bounds it is a CU's load path -- the row kernel brings every key once per query head through it -- and at few rows the chain of dependent loads.
-// us, row kernel / this one: 16 / 1 heads of 256 / 192, 3 rows over ~180 tokens 20.7 / 15.6, 2 rows over 2000 62.8 / 29.4, 420 rows of three prompts 148 / 33, a
-// prompt of 2000 7810 / 670; 32 / 8 heads of 128 / 128 15.0 / 10.1, 46.5 / 20.3, 146 / 69, 8430 / 1960; and where a head has a key head of its own (the tile holds one
+// us, row kernel / this one: 16 / 1 heads of 256 / 192, 3 rows over ~180 tokens 21.0 / 15.1, 2 rows over 2000 61.3 / 27.4, 420 rows of three prompts 148 / 31, a
+// prompt of 2000 7165 / 597; 32 / 8 heads of 128 / 128 14.9 / 9.9, 44.2 / 19.3, 147 / 66, 7690 / 1915; and where a head has a key head of its own (the tile holds one
 // row of sixteen) 16 / 16 heads of 128 / 128 16.5 / 10.1, 56.8 / 22.1, 145 / 124, 10300 / 3850: nothing was slower, so it serves every size it can.
 template<int DS, int VT>
 __global__ __launch_bounds__(256) void attn_heads_f32_kernel(GeneralAttnParams p, int chunks)
@@ -1248,7 +1248,7 @@ __global__ __launch_bounds__(256) void attn_heads_f32_kernel(GeneralAttnParams p
         if (j0 > limit || (j0 + 15 < lower && j0 >= klo)) {  // none of the wave's keys is seen
             continue;
         }
-        const char*  base = (const char*)table[b] + p.layer_offset;
+        const char*  base = global_ptr(table[b]) + p.layer_offset;
         const float* kb   = (const float*)base + ((size_t)ga_key_head(p, g) * 64 + j0 + lr) * D;
         const float* vb   = (const float*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V + j0 + lg * 4;
         floatx4      k[DS], v4[VT];

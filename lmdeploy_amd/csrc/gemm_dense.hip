@@ -179,7 +179,7 @@ struct DenseEpi {
                 return;
             }
             const int s = c.kv.row_seq[m], pos = c.kv.row_pos[m], ti = pos % c.kv.block_len;
-            char* const base = (char*)c.kv.block_ptrs[(size_t)(c.kv.seq_slot ? c.kv.seq_slot[s] : s) * c.kv.block_stride + pos / c.kv.block_len] + c.kv.layer_offset;
+            char* const base = global_ptr(c.kv.block_ptrs[(size_t)(c.kv.seq_slot ? c.kv.seq_slot[s] : s) * c.kv.block_stride + pos / c.kv.block_len]) + c.kv.layer_offset;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int col = n + e;

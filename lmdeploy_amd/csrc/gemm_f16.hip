@@ -105,7 +105,7 @@ struct F16EpiKv: F16Epi {
                 *(half4_t*)((half_t*)a.y + (size_t)m * a.ldy + c) = h;
                 continue;
             }
-            char* block = (char*)kv.cache.block_ptrs[kv.cache.cu_block_nums[m] + blk] + kv.cache.layer_offset;
+            char* block = global_ptr(kv.cache.block_ptrs[kv.cache.cu_block_nums[m] + blk]) + kv.cache.layer_offset;
             *(half4_t*)(block + (kh < L.kv_heads ? L.k_data(kh, ti) : L.v_data(kh - L.kv_heads, ti)) + d * 2) = h;
         }
     }

@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void kv_rope_store_kernel(half_t* __restrict__
     const int kv_head = is_k ? head - q_heads : head - q_heads - kv_heads;
     const int blk     = pos / L.block_len;
     const int ti      = pos - blk * L.block_len;
-    char*     block   = (char*)cache.block_ptrs[cache.cu_block_nums[b] + blk] + cache.layer_offset;
+    char*     block   = global_ptr(cache.block_ptrs[cache.cu_block_nums[b] + blk]) + cache.layer_offset;
     const int doff    = is_k ? L.k_data(kv_head, ti) : L.v_data(kv_head, ti);
 
     if constexpr (BITS == 16) {
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(256) void flatten_kv_kernel(half_t* __restrict__ k_
 
     const int    lane16 = threadIdx.x & 15;
     const int    row    = threadIdx.x >> 4;  // 16 token rows per pass
-    const char*  block  = (const char*)cache.block_ptrs[cache.cu_block_nums[b] + blockIdx.x] + cache.layer_offset;
+    const char*  block  = global_ptr(cache.block_ptrs[cache.cu_block_nums[b] + blockIdx.x]) + cache.layer_offset;
     const size_t obase  = (size_t)hd * k_stride + cu_k_off[b];
 
 #pragma unroll
@@ -363,7 +363,7 @@ __global__ void kv_store_general_kernel(const T* __restrict__ qkv, int ld, int k
     }
     const int t = (int)(i / per), c = (int)(i % per);
     const int s = p.row_seq[t], pos = p.row_pos[t];
-    char* base = (char*)p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len] + p.layer_offset;
+    char* base = global_ptr(p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len]) + p.layer_offset;
     const int ti = pos % p.block_len;
     const int nk = kh * p.dim;
     if (c < nk) {
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256) void kv_store_rows_kernel(const uint16_t* __re
         }
         const u32x4 v = *(const u32x4*)(qkv + (size_t)t * ld + (val ? v_col : k_col) + c);
         const int   s = p.row_seq[t], pos = p.row_pos[t], ti = pos % p.block_len;
-        char* const base = (char*)p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len] + p.layer_offset;
+        char* const base = global_ptr(p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len]) + p.layer_offset;
         if (!val) {
             const int g = c / p.dim, d = c % p.dim;
             *(u32x4*)((uint16_t*)base + ((size_t)g * p.block_len + ti) * p.dim + d) = v;
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const float* __restrict_
         }
         return;
     }
-    char* base = (char*)p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len] + p.layer_offset;
+    char* base = global_ptr(p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len]) + p.layer_offset;
     if (kind == 1) {
         T* k = (T*)base + ((size_t)head * p.block_len + ti) * n;
         for (int i = lane; i < n; i += 64) {
@@ -604,7 +604,7 @@ __global__ __launch_bounds__(256) void talk_prep_kernel(const float* __restrict_
         return;
     }
     const int s = p.row_seq[t], pos = p.row_pos[t], ti = pos % p.block_len;
-    char*     base = (char*)p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len] + p.layer_offset;
+    char*     base = global_ptr(p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len]) + p.layer_offset;
     T*        kc   = (T*)base + (size_t)ti * (G * D);   // one key head of size G D
     T*        vc   = (T*)(base + p.v_offset) + ti;      // G value heads [D][block_len]: channel c D + d of the row at (c D + d) * block_len
     for (int i = threadIdx.x; i < G * D; i += 256) {
@@ -704,7 +704,7 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* __restric
     if (a.dkv_col < 0) {
         return;
     }
-    char*        base = (char*)p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len] + p.layer_offset;
+    char*        base = global_ptr(p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len]) + p.layer_offset;
     T*           k    = (T*)base + (size_t)ti * (C + R);
     T*           vt   = (T*)(base + p.v_offset) + ti;
     const float* kv   = x + a.dkv_col;
