@@ -1292,13 +1292,14 @@ __global__ __launch_bounds__(256) void attn_heads_f32_kernel(GeneralAttnParams p
             sc[r] = seen[r] ? __expf(sc[r] - m_new) : 0.f;
             l += sc[r];
         }
-        const bool whole = j0 + 15 <= limit;  // (entries behind a row's own may hold anything: a weight of zero does not take them out)
+        // entries that the row does not see -- behind its own, and before its window or chunk -- may hold anything: a weight of zero does not take them out
+        const bool whole = j0 + 15 <= limit && (j0 >= lower || j0 + 15 < klo);
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
             o[v] *= alpha;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float x = whole || j0 + lg * 4 + r <= limit ? v4[v][r] : 0.f;
+                const float x = whole || seen[r] ? v4[v][r] : 0.f;
                 o[v]          = __builtin_amdgcn_mfma_f32_16x16x4f32(x, sc[r], o[v], 0, 0, 0);
             }
         }

@@ -27,7 +27,7 @@ PORTIONS = [[(1, 1), (3, 17), (66, 130)], [(1, 16), (1, 64), (1, 65), (1, 700), 
 
 
 def run(tm, D, V, portions, H, G, kernel=0, splits=1, cap=0.0, sink=False, window=0, keep=0, chunk=0, bias=False, table=0, gate=False, space=0, k_heads=0, v_heads=0,
-        temp=0.0):
+        temp=0.0, unseen=False):
     g = torch.Generator('cuda').manual_seed(D + H)
     kh, vh = k_heads or G, v_heads or G
     n = len(portions)
@@ -42,6 +42,13 @@ def run(tm, D, V, portions, H, G, kernel=0, splits=1, cap=0.0, sink=False, windo
         behind = (portions[s][1] - 1) % 64 + 1      # entries behind a sequence's own hold what they may
         last[:kh * 64 * D].view(kh, 64, D)[:, behind:] = float('nan')
         last[kh * 64 * D:].view(vh, V, 64)[:, :, behind:] = float('nan')
+        if unseen:                                  # and so do those that no row of the portion sees any more
+            lo = portions[s][1] - portions[s][0]
+            lo = lo // chunk * chunk if chunk else max(0, lo - window + 1)
+            for i in range(keep, lo):
+                e = pool[int(order[at + i // 64])]
+                e[:kh * 64 * D].view(kh, 64, D)[:, i % 64] = float('nan')
+                e[kh * 64 * D:].view(vh, V, 64)[:, :, i % 64] = float('inf')
         at += b
     lens = [q for q, _ in portions]
     rows, ldq, hs = sum(lens), H * D + 3, V + space
@@ -76,6 +83,8 @@ def run(tm, D, V, portions, H, G, kernel=0, splits=1, cap=0.0, sink=False, windo
     for s, (m, k) in enumerate(portions):
         blk = pool[torch.from_numpy(order[at:at + blocks[s]].copy()).cuda()].double()
         at += blocks[s]
+        if unseen:
+            blk = blk.nan_to_num(0.0, 0.0, 0.0)
         p, j = torch.arange(k - m, k, device='cuda'), torch.arange(k, device='cuda')
         d = p[:, None] - j[None, :]
         hide = d < 0
@@ -136,3 +145,10 @@ FORMS = [dict(cap=3.0), dict(sink=True), dict(window=20), dict(window=70, keep=5
 def test_modifiers(tm, cuda, form):
     for rows, splits in ((0, 1), (1, 1), (1, 3)):
         check(tm, 96, 80, PORTIONS[rows], 8, 2, splits=splits, **form)
+
+
+@pytest.mark.parametrize('form', [dict(window=20), dict(window=70, keep=5), dict(window=17, keep=40), dict(chunk=48)], ids=lambda f: '-'.join(f))
+def test_entries_that_are_not_seen(tm, cuda, form):
+    """entries before a window or a chunk that no row of a launch sees hold what they may, as those behind a sequence's own do"""
+    for portions, splits in (([(1, 1), (3, 170), (20, 130)], 1), ([(1, 64), (1, 65), (1, 700), (1, 129)], 3)):
+        check(tm, 96, 80, portions, 8, 2, splits=splits, unseen=True, **form)
