@@ -133,13 +133,16 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
     }
     const float2* sf = sums + row;
     floatx4       out[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    float         odd    = 0.f;  // NaN once a sum of x is not finite
     auto          compute = [&](int s, int i) {
         const int    kb = ph + i * KP;
         const float2 cs  = sf[kb * M];
-        floatx4      acc[2] = {{cs.x, cs.x, cs.x, cs.x}, {cs.x, cs.x, cs.x, cs.x}};
+        half8_t      x  = *(const half8_t*)(xf + kb * 256);
+        __builtin_amdgcn_sched_barrier(0);  // (asked for ahead of the wait for the weights)
+        floatx4 acc[2] = {{cs.x, cs.x, cs.x, cs.x}, {cs.x, cs.x, cs.x, cs.x}};
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const half8_t x = *(const half8_t*)(xf + kb * 256 + t * 64);
+            x = t == 0 ? x : *(const half8_t*)(xf + kb * 256 + t * 64);
             const auto    d = __builtin_amdgcn_permlane16_swap(w[s][t >> 1][2 * t & 3], w[s][t >> 1][(2 * t & 3) + 1], false, false);
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -154,6 +157,7 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
                 out[u][e]        = __builtin_fmaf((float)pr[0], acc[u][e], __builtin_fmaf((float)pr[1], cs.y, out[u][e]));
             }
         }
+        odd = __builtin_fmaf(cs.x, 0.f, odd);
     };
     int i = 0;
     for (; i + 2 * R <= n; i += R) {
@@ -175,6 +179,37 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
     for (int s = 0; s < R; ++s) {
         if (i + s < n) {
             compute(s, i + s);
+        }
+    }
+    // A row that holds an infinity: with the codes' exponent bits on every sum of it is infinity less infinity.  Its results are then made from weights.
+    if (__ballot(odd != odd) != 0) {
+        floatx4 alt[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        for (int j = 0; j < n; ++j) {
+            const int   kb   = ph + j * KP;
+            const char* unit = (const char*)p.wp + ((size_t)(kb0 + kb) * p.ncg + cgc) * kP32Unit;
+            half2_t     s2[2], z2[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const half2_t pr = *(const half2_t*)(unit + 2048 + (u * 16 + fr) * 4);
+                s2[u] = half2_t{pr[0], pr[0]}, z2[u] = half2_t{pr[1], pr[1]};
+            }
+#pragma unroll 1
+            for (int t = 0; t < 4; ++t) {
+                const half8_t   x = *(const half8_t*)(xf + kb * 256 + t * 64);
+                const uint32_t* q = (const uint32_t*)(unit + (t >> 1) * 1024 + lane * 16) + (2 * t & 3);
+                const auto      d = __builtin_amdgcn_permlane16_swap(q[0], q[1], false, false);
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    alt[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8_p32(d[u], s2[u], z2[u], m1024, m64), x, alt[u], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                out[u][e] = odd != odd ? alt[u][e] : out[u][e];
+            }
         }
     }
     if constexpr (KP > 1) {

@@ -52,6 +52,28 @@ def test_against_64_bits(tm, cuda, K, N, splits, gated, M):
     assert (np.abs(got - ref) <= 2.0**-11 * np.abs(ref) + 2.0**-9 * rms).all()    # one rounding to fp16; sums of 1039 |x| in fp32 beside results of about 52
 
 
+@pytest.mark.parametrize('K,N,splits,gated', [(2048, 4096, 1, 0), (2304, 4128, 2, 0), (2048, 2048, 4, 1), (4096, 10240, 1, 1), (2048, 28704, 1, 0)])
+@pytest.mark.parametrize('M', [1, 4, 16])
+def test_infinities(tm, cuda, K, N, splits, gated, M):
+    """a row with infinities has the infinities and NaN that its weights give it, as in the kernel that makes them; the other rows keep their bits"""
+    rng = np.random.default_rng(K + N + M)
+    h, _ = _make_linear(tm, rng, K, N)
+    x = rng.standard_normal((M, K + 8)).astype(np.float16)
+    plain = _run(tm, h, x, N, M, ROWS, splits, gated)
+    rows = [0] if M == 1 else [1, M - 1]
+    x[rows[0], [5, 131]] = np.inf, -np.inf
+    for r in rows[1:]:
+        x[r, K - 3] = -np.inf
+    got, other = _run(tm, h, x, N, M, ROWS, splits, gated), _run(tm, h, x, N, M, 0, splits, gated)
+    _ffi.check(tm.tm_linear_destroy(h))
+    left = np.setdiff1d(np.arange(M), rows)
+    assert np.array_equal(got[left], plain[left]) and not np.isfinite(got[rows]).any()
+    if not gated:
+        assert np.isinf(got[rows]).any()
+    same = np.where(np.isnan(got[rows]), 0, got[rows]) == np.where(np.isnan(other[rows]), 0, other[rows])
+    assert same.all()
+
+
 def test_what_a_launch_takes(tm, cuda):
     def pick(K, N, M):
         sh, sp = _ffi.C.c_int(), _ffi.C.c_int()
