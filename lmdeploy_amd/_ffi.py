@@ -178,6 +178,7 @@ _SIGNATURES = {
     'tm_debug_pick_tiling': (c_int, [c_int, c_int, c_int, c_int, POINTER(c_int), POINTER(c_int)]),
     'tm_debug_pick_general': (c_int, [c_int, c_int, c_int, c_int, c_int, c_void_p]),
     'tm_debug_grouped_tile': (c_int, [c_int, c_int, c_int, c_int, POINTER(c_int)]),
+    'tm_debug_mixer_kernel': (c_int, [c_int, POINTER(c_int), c_int, POINTER(c_int)]),
     'tm_debug_stream_plan': (c_int, [c_int, c_int, c_int, c_int, c_int, POINTER(c_int)]),
     'tm_engine_comm_drop_rccl': (c_int, [c_void_p]),
     'tm_engine_comm_info': (c_int, [c_void_p, POINTER(c_int), POINTER(c_int), POINTER(c_int)]),

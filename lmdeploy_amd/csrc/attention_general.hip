@@ -19,7 +19,7 @@
 // One launch serves every row of a forward, prefill portions and decoded tokens alike: row t belongs to sequence row_seq[t] at
 // position row_pos[t] and sees the cache entries 0 .. row_pos[t] of that sequence (its own key was stored before the launch).
 //   * row kernel : one wave per (row, query head, key split); lanes own keys for the scores and value channels for the output.
-//                  What the others do not serve: odd sizes, keys of more than 256 channels, other block lengths.
+//                  What the others do not serve: odd sizes, keys of more than 256 channels, other block lengths; in fp32 many rows of few keys and few heads a key head.
 //   * tile kernel: bf16 prefill on the matrix cores -- 64 query rows of one sequence x one query head per workgroup, four waves of 16
 //                  rows; S^T = K Q^T and O^T += V^T P^T as v_mfma_f32_16x16x32_bf16 with every operand a 16-byte load straight from the
 //                  cache (keys [token][channel], values stored transposed [channel][token]); online soft-max in fp32; no LDS, no barrier.
@@ -1202,9 +1202,9 @@ int launch_general_attention_decode(const GeneralAttnParams& p, hipStream_t st)
 // attn_decode_kernel's arrangement for an fp32 cache, v_mfma_f32_16x16x4: workgroup per (row, 16 heads of a key head, key split), each wave 16 of a block's 64
 // keys.  S^T = K Q^T with the channels of a step dealt so that a lane's four are one load, and P^T then stands in the registers that O^T += V^T P^T reads.
 // What bounds it is a CU's load path -- the row kernel brings every key once per query head through it -- and at few rows the chain of dependent loads.
-// us, row kernel / this one: 16 / 1 heads of 256 / 192, 3 rows over ~180 tokens 21.0 / 15.1, 2 rows over 2000 61.3 / 27.4, 420 rows of three prompts 148 / 31, a
-// prompt of 2000 7165 / 597; 32 / 8 heads of 128 / 128 14.9 / 9.9, 44.2 / 19.3, 147 / 66, 7690 / 1915; and where a head has a key head of its own (the tile holds one
-// row of sixteen) 16 / 16 heads of 128 / 128 16.5 / 10.1, 56.8 / 22.1, 145 / 124, 10300 / 3850: nothing was slower, so it serves every size it can.
+// us, row kernel / this one: 16 / 1 heads of 256 / 192, 3 rows over ~180 tokens alone 21.0 / 15.1 (in a model, latency and all, 22.0 / 21.5), 2 rows over 2000 61.3 / 27.4, 420 rows
+// of three prompts 148 / 31, a prompt of 2000 7165 / 597; 32 / 8 heads of 128 / 128 14.9 / 9.9, 44.2 / 19.3, 147 / 66, 7690 / 1915; 16 / 16 heads of 128 / 128, where
+// the tile holds one row of sixteen, 16.5 / 10.1, 56.8 / 22.1, 145 / 124, 10300 / 3850.  Where it loses: general_attention_heads_f32_pays.
 template<int DS, int VT>
 __global__ __launch_bounds__(256) void attn_heads_f32_kernel(GeneralAttnParams p, int chunks)
 {
@@ -1315,6 +1315,30 @@ bool general_attention_heads_f32_ok(const GeneralAttnParams& p)
            && p.q_heads % p.kv_heads == 0 && p.splits >= 1 && (p.splits == 1 || (p.partial_o && p.partial_ml));
 }
 
+// The heads kernel or the row kernel.  Up to about two workgroups a CU latency counts, which the heads kernel has less of.  Beyond, a workgroup of it costs what a tile of sixteen
+// heads costs however many of them exist, and the merge of its four waves: with a few heads a key head and few keys a row the row kernel's waves, each of them one head, do less.
+// ns a tile or head where the chip is full, fitted to 1950 sizes (16 ... 256 channels, 1 ... 8 heads a key head, 1 ... 2000 rows, 17 ... 1000 keys).  us, row kernel / heads kernel:
+// 32 / 32 heads of 12, 420 prompt rows 35 / 100; 32 / 32 of 128, 60 prompts of 33 267 / 736, a prompt of 1000 2631 / 2015; 32 / 8 of 64, 60 prompts of 33 125 / 96;
+// 8 / 8 of 256, 128 decoded rows over 20 keys 19 / 47, three rows over 180 25 / 14.  What a row sees besides its own portion is not known here: a prompt counts as its own
+// keys, a decoded row as half a block (4 heads of 256 a key head, 128 rows over 20 keys lose by it, 31 / 47; over 60 keys they gain)
+bool general_attention_heads_f32_pays(const GeneralAttnParams& p, bool prefill)
+{
+    const int     group = p.q_heads / p.kv_heads, chunks = (group + 15) / 16, ds = (p.dim + 15) / 16, vt = (p.vdim + 15) / 16;
+    const int     steps = ds <= 4 && vt <= 8 ? 4 + (vt <= 4 ? 4 : 8) : ds <= 8 && vt <= 8 ? 16 : 16 + (vt <= 8 ? 8 : vt <= 12 ? 12 : 16);  // channel steps of the instantiation
+    const int64_t tiles = (int64_t)p.rows * p.kv_heads * chunks;
+    if (tiles <= (steps > 16 ? 256 : 512)) {
+        return true;
+    }
+    prefill     = prefill && p.max_q_len > 1;
+    double keys = prefill ? p.max_q_len / 2.0 : 32.0;
+    keys        = std::min(keys, p.chunk > 0 ? p.chunk / 2.0 : keys);
+    keys        = std::min(keys, p.window > 0 ? (double)p.window + p.keep_first : keys);
+    const double blocks = prefill ? keys / 64 + 0.5 : 1.0;
+    const double tile   = steps > 16 ? steps * (0.6 + 0.62 * blocks) : steps * (0.3 + 0.6 * blocks);
+    const double head   = 0.84 + 0.0035 * (p.dim + p.vdim) + (0.56 + 0.041 * (p.dim + p.vdim)) * keys / 64;
+    return tile < head * group / chunks;
+}
+
 int launch_general_attention_heads_f32(const GeneralAttnParams& p, hipStream_t st)
 {
     TM_REQUIRE(general_attention_heads_f32_ok(p), "attention over heads: fp32, 64-token blocks, dim and vdim multiples of 4 up to 256");
@@ -1379,7 +1403,7 @@ int launch_general_attention(const GeneralAttnParams& p, bool prefill, hipStream
     if (!prefill && tiles_on && general_attention_decode_ok(p)) {
         return launch_general_attention_decode(p, st);
     }
-    if (tiles_on && general_attention_heads_f32_ok(p)) {
+    if (tiles_on && general_attention_heads_f32_ok(p) && general_attention_heads_f32_pays(p, prefill)) {
         return launch_general_attention_heads_f32(p, st);
     }
     return launch_general_attention_rows(p, st);

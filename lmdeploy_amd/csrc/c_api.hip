@@ -1016,6 +1016,19 @@ int tm_debug_stream_plan(int kind, int K, int N, int M, int scratch, int* plan5)
     return 0;
 }
 
+int tm_debug_mixer_kernel(int what, const int* v, int n, int* kernel)
+{
+    TM_REQUIRE(v && kernel && what == 0 && n == 9, "arguments");
+    for (int i = 0; i < n; ++i) {
+        TM_REQUIRE(v[i] >= (i < 5 ? 1 : 0), "sizes");
+    }
+    GeneralAttnParams p;
+    p.elem_bytes = 4, p.block_len = 64, p.splits = 1;
+    p.rows = v[0], p.q_heads = v[1], p.kv_heads = v[2], p.dim = v[3], p.vdim = v[4], p.max_q_len = v[6], p.window = v[7], p.chunk = v[8];
+    *kernel = general_attention_heads_f32_ok(p) && general_attention_heads_f32_pays(p, v[5] != 0);
+    return 0;
+}
+
 int tm_debug_tiling_candidates(int K, int N, int M, int* shapes, int* splits, int cap, int* count)
 {
     TM_REQUIRE(shapes && splits && count && cap >= 0 && K > 0 && N > 0 && M > 0, "arguments");

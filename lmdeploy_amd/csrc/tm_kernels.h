@@ -562,12 +562,13 @@ bool   general_attention_decode_ok(const GeneralAttnParams& p);
 int    launch_general_attention_decode(const GeneralAttnParams& p, hipStream_t st);
 // the same for an fp32 cache, and for the rows of a prompt too: one row a workgroup
 bool   general_attention_heads_f32_ok(const GeneralAttnParams& p);
+bool   general_attention_heads_f32_pays(const GeneralAttnParams& p, bool prefill);  // where it is faster than the row kernel
 int    launch_general_attention_heads_f32(const GeneralAttnParams& p, hipStream_t st);
 // bf16 tile kernel; TM_INVALID when the sizes are outside what it serves (general_attention_tiles_ok)
 bool   general_attention_tiles_ok(const GeneralAttnParams& p);
 int    launch_general_attention_tiles(const GeneralAttnParams& p, hipStream_t st);
-// dispatch: prefill portions in bf16 -> the tile kernel on the matrix cores where it serves the sizes, decoded rows in bf16 and all rows in
-// fp32 -> theirs, everything else -> the row kernel
+// dispatch: prefill portions in bf16 -> the tile kernel on the matrix cores where it serves the sizes, decoded rows in bf16 and rows in
+// fp32 -> theirs, the latter where it pays, everything else -> the row kernel
 int    launch_general_attention(const GeneralAttnParams& p, bool prefill, hipStream_t st);
 
 // ---- norm.hip / kv_cache.hip / misc.hip: the fp32 residual stream ------------------------------------------------------------------

@@ -696,3 +696,26 @@ def test_line_between_the_kernels_of_fp16_products():
     for wgs, few, many in ((192, 2, 2), (216, 0, 0), (256, 0, 0), (288, 2, 2), (384, 2, 2), (448, 2, 0), (512, 2, 0), (576, 2, 2), (640, 2, 2), (723, 2, 0), (1002, 2, 0), (1188, 2, 0)):
         for rows, kernel in ((17, few), (40, few), (41, many), (64, many)):
             assert stream_plan(2, 4096, 128 * wgs, rows)[0] == kernel, (wgs, rows)
+
+
+def _mixer(what, *sizes):
+    k = _ffi.C.c_int(-1)
+    _ffi.check(_ffi.load().tm_debug_mixer_kernel(what, (_ffi.C.c_int * len(sizes))(*sizes), len(sizes), _ffi.C.byref(k)))
+    return k.value
+
+
+@pytest.mark.parametrize('sizes,heads', [
+    # rows, query heads, key heads, dim, vdim, prompts, longest, window, chunk (us, row kernel / heads kernel)
+    ((3, 16, 1, 256, 192, 0, 1, 0, 0), 1), ((420, 16, 1, 256, 192, 1, 140, 0, 0), 1), ((128, 16, 1, 256, 192, 0, 1, 0, 0), 1), ((1980, 32, 4, 128, 128, 1, 33, 0, 0), 1),
+    ((1980, 32, 8, 64, 64, 1, 33, 0, 0), 1), ((128, 32, 8, 128, 128, 1, 1, 0, 0), 1), ((1000, 32, 32, 128, 128, 1, 1000, 0, 0), 1), ((24, 8, 8, 256, 256, 0, 1, 0, 0), 1), ((1, 64, 64, 64, 64, 0, 1, 0, 0), 1),
+    ((420, 32, 32, 12, 12, 1, 140, 0, 0), 0),           # 35 / 100
+    ((1980, 32, 32, 128, 128, 1, 33, 0, 0), 0),         # 267 / 736
+    ((1980, 8, 8, 256, 256, 1, 33, 0, 0), 0),           # 194 / 659
+    ((1000, 8, 8, 256, 256, 1, 1000, 0, 64), 0),        # 203 / 352 (chunks of 64)
+    ((128, 8, 8, 256, 256, 0, 1, 0, 0), 0),             # 19 / 47 over 20 keys
+    ((128, 32, 32, 12, 12, 0, 1, 0, 0), 0),             # 11 / 28 over 60 keys
+    ((1000, 4, 4, 32, 32, 1, 1000, 100, 0), 0),         # 37 / 48 (windows of 100)
+])
+def test_fp32_attention_takes_the_faster_kernel(sizes, heads):
+    """measured where the two kernels of fp32 attention differ most: many rows of few keys with few heads a key head are the row kernel's"""
+    assert _mixer(0, *sizes) == heads
