@@ -316,7 +316,10 @@ bool w4_rows_supported(const LinearWeight& w, int M, int slices)
 }
 
 // Products below what was timed stay with gemm_dec32_kernel (whose rows have the bits that they have in forwards of more rows), and so do more than eight rows of a long
-// k: (14336, 4096) 16 rows 16.1 here, 15.9 there.  A slice has eight k-blocks at least; a gate / up product's slabs are nobody's to sum but a launch's of its own (3.3 us)
+// k: (14336, 4096) 16 rows 16.1 here, 15.9 there.  A slice has eight k-blocks at least; a gate / up product's slabs are nobody's to sum but a launch's of its own (3.3 us).
+// Wide products whose rows do not fit in LDS whole would have slices only for that, and slabs of all columns: where gemm_dec32_kernel needs none, it keeps them, unless more than a
+// quarter of its last round of 128-column workgroups stays empty.  us, there | here in two slices: (5120, 20480) 16 rows 16.9 | 22.5, (6144, 28672) 14 rows 22.5 | 26.7, (8192, 57344)
+// 12 rows 54.6 | 59.6, (16384, 20480) 8 rows 42.7 | 47.6, 4 rows 45.1 | 40.8; (8192, 40960), 1.25 rounds, 12 rows 50.8 | 44.9
 bool w4_rows_plan(const LinearWeight& w, int M, int* slices)
 {
     const int KB = w.K / 128, ncg = w.N / 32;
@@ -333,6 +336,14 @@ bool w4_rows_plan(const LinearWeight& w, int M, int* slices)
         cost += s > 1 && w.role == 3 ? 3.3 : 0.0;
         if (*slices == 0 || cost < best) {
             *slices = s, best = cost;
+        }
+    }
+    if (*slices > 1 && M > 4 && w.N >= 16384) {
+        int shape, splits;
+        dec32_pick_plain(w, M, &shape, &splits, false);
+        const int wgs = (w.N + 127) / 128, rounds = (wgs + 255) / 256;
+        if (splits == 1 && (rounds == 1 || wgs > 192 * rounds)) {
+            return false;
         }
     }
     return *slices > 0;

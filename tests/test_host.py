@@ -698,6 +698,14 @@ def test_line_between_the_kernels_of_fp16_products():
             assert stream_plan(2, 4096, 128 * wgs, rows)[0] == kernel, (wgs, rows)
 
 
+@pytest.mark.parametrize('K,N,M,rows', [(5120, 20480, 14, True), (5120, 20480, 16, False), (5120, 27648, 16, False), (6144, 28672, 14, False), (8192, 28672, 9, True), (8192, 28672, 10, False),
+                                        (8192, 57344, 12, False), (8192, 40960, 12, True), (8192, 14336, 16, True), (8192, 57344, 8, True), (16384, 20480, 8, False),
+                                        (16384, 20480, 4, True), (16384, 20480, 1, True)])
+def test_wide_few_row_products_without_slabs(K, N, M, rows):
+    """W4 products of up to 16 rows whose rows do not fit in LDS in one slice of k: wide ones stay on the tile that needs no slabs (measured: 4 to 25 % faster)"""
+    assert (_pick(_ffi.load(), K, N, M, 4)[0] == 14) == rows
+
+
 def _mixer(what, *sizes):
     k = _ffi.C.c_int(-1)
     _ffi.check(_ffi.load().tm_debug_mixer_kernel(what, (_ffi.C.c_int * len(sizes))(*sizes), len(sizes), _ffi.C.byref(k)))
