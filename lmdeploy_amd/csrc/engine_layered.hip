@@ -1563,27 +1563,39 @@ static int post_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
             c.bias = L.w0;
             TM_PROF(P_GEMM_QKV, TM_TRY(launch_dense_call(L.w2, lm.d_lora, lm.ldlora, lm.d_wdec, lm.ldmix, M, c, st)));
         }
+        // unit keys, removal rates and decays as the walk reads them; portions in chunks take the logits
+        auto prep = [&](int row0, int rows) {
+            return launch_delta_prep(lm.d_proj + (size_t)row0 * lm.ldproj, lm.ldproj, L.c_k, L.c_a, lm.d_wdec + (size_t)row0 * lm.ldmix, lm.ldmix,
+                                     lm.d_aux + (size_t)row0 * lm.ldmix, lm.ldmix, rows, H, s.dim, st);
+        };
+        auto seqs = [&](const LmPart& P) {
+            StateMixParams sp = state_seqs(e, P);
+            sp.rows = P.rows, sp.heads = H, sp.dim = s.dim, sp.vdim = s.vdim;
+            sp.raw = 1;
+            sp.raw = delta && state_mix_chunks(sp);
+            return sp;
+        };
+        bool walk = delta;
         for (int i = 0; i < nparts; ++i) {
-            const LmPart&  P = parts[i];
-            StateMixParams sp;
-            sp.max_q_len = P.decode ? 1 : std::max(1, P.max_q_len);
-            sp.raw       = delta && state_mix_chunks(sp.max_q_len);
-            if (delta && !sp.raw) {  // unit keys, removal rates and decays as the walk reads them
-                TM_PROF(P_KV_STORE, TM_TRY(launch_delta_prep(lm.d_proj + (size_t)P.row0 * lm.ldproj, lm.ldproj, L.c_k, L.c_a, lm.d_wdec + (size_t)P.row0 * lm.ldmix, lm.ldmix,
-                                                             lm.d_aux + (size_t)P.row0 * lm.ldmix, lm.ldmix, P.rows, H, s.dim, st)));
+            walk = walk && !seqs(parts[i]).raw;
+        }
+        if (walk) {
+            TM_PROF(P_KV_STORE, TM_TRY(prep(0, M)));
+        }
+        for (int i = 0; i < nparts; ++i) {
+            const LmPart&  P  = parts[i];
+            StateMixParams sp = seqs(P);
+            if (delta && !walk && !sp.raw) {
+                TM_PROF(P_KV_STORE, TM_TRY(prep(P.row0, P.rows)));
             }
-            sp.nseq = P.nseq, sp.cu_q = P.cu_q, sp.k_len = P.k_len, sp.seq_slot = P.seq_slot, sp.slot0 = P.slot0, sp.active = P.active;
-            sp.park_slot   = e->cfg.max_batch_size;
-            sp.state       = lm.d_state;
-            sp.slot_stride = lm.state_slot_floats, sp.layer_offset = L.state_offset;
-            sp.heads = H, sp.dim = s.dim, sp.vdim = s.vdim;
+            sp.layer_offset = L.state_offset;
             sp.proj = lm.d_proj + (size_t)P.row0 * lm.ldproj, sp.ld = lm.ldproj;
             sp.c_q = 0, sp.c_k = L.c_k, sp.c_v = L.c_v, sp.c_a = L.c_a;
             sp.decay_h = L.decay_d;
             sp.decay_w = lm.d_wdec + (size_t)P.row0 * lm.ldmix, sp.ld_w = lm.ldmix;
             sp.unit    = lm.d_aux + (size_t)P.row0 * lm.ldmix, sp.ld_u = lm.ldmix;
             sp.out     = lm.d_mixo + (size_t)P.row0 * lm.ldmix, sp.ldo = lm.ldmix;
-            sp.rows = P.rows, sp.blocks = lm.d_blocks, sp.blocks_floats = lm.blocks_floats;
+            sp.blocks = lm.d_blocks, sp.blocks_floats = lm.blocks_floats;
             TM_PROF(P_ATTN, TM_TRY(launch_state_mix(sp, delta ? kStateDelta : kStateLinear, st)));
         }
         TM_PROF(P_ATTN, TM_TRY(launch_gated_group_norm(lm.d_cat, lm.ldcat, lm.elem, lm.d_mixo, lm.ldmix, L.mix_norm, lm.d_proj + L.c_g, lm.ldproj, M,

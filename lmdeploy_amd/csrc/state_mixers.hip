@@ -24,12 +24,13 @@
 // vectors (q, k, and w, a u, u for the delta rule), loaded TB tokens at a time: the next stage's global loads are issued before the
 // current stage's tokens are walked and land in the other LDS buffer afterwards, so their latency hides under the recurrence.  A slab is
 // stored as the wave holds it, [ii][column of the pair][lane]: loading and storing it are fully coalesced.
-// The delta rule walks portions of up to 32 tokens one by one (two dependent reductions per token); longer ones, and every portion of the other mixers, run
-// in chunks on the matrix cores (below).
+// The delta rule walks short portions, and portions of many heads x sequences, one token after the other (two dependent reductions per token; state_mix_chunks); the
+// others, and every portion of the other mixers, run in chunks on the matrix cores (below).
 // One kernel serves prompt portions (many rows per sequence) and decoded tokens (one row, TB = 1): the state traffic of a decode step,
 // 2 * dim * vdim * 4 bytes per head, is what bounds it.
 #include "tm_kernels.h"
 #include "gemm_stream.h"  // stream_dma16
+#include <algorithm>
 
 namespace tmk {
 
@@ -918,10 +919,23 @@ static int launch_decay_chunks(const StateMixParams& p, hipStream_t st)
     }
 }
 
-// the delta rule: the walk costs 0.9 us a token, the blocks and a chunk or two 34: 8 x 16 tokens 19.5, 8 x 17 in chunks 34, 1 x 16 17, 1 x 32 in chunks 31
-bool state_mix_chunks(int max_q_len)
+// Portions of the delta rule in chunks, or walked token by token.  A few heads x sequences leave the walk a chain of tokens, which chunks shorten; where there are enough of
+// them to fill the chip the walk is bound by its work, and chunks do about as much of it and more for the last, part-filled one.  A model of both in microseconds, fitted
+// to 800 sizes (32 ... 256 channels, 2 ... 2048 heads x sequences, 33 ... 1000 tokens): what it takes is 0.9 % slower than the better one on average.  us, walk with the launch
+// that prepares its operands / chunks: 128 channels, 16 heads, one prompt of 33 tokens 35 / 31, 8 of 1000 974 / 411, 32 of 33 85 / 111, 32 of 64 146 / 137; 256 channels, 32 heads, 32 of
+// 33 530 / 881, of 64 1005 / 1136, of 256 3890 / 3855.  Up to 32 tokens it was never chunks (one prompt of 32 29 / 31).  Without logits (raw: 0) the operands are prepared either way.
+bool state_mix_chunks(const StateMixParams& p)
 {
-    return max_q_len > 2 * kChunkT;
+    if (p.max_q_len <= 2 * kChunkT) {
+        return false;
+    }
+    const double rows = p.rows > 0 ? p.rows : (double)p.nseq * p.max_q_len, state = (double)p.dim * p.vdim;
+    const double walk = 5 + std::max((0.31 + 0.005 * p.dim) * p.max_q_len, (0.00055 + 2.1e-7 * state) * p.heads * rows)
+                        - (p.raw ? 0.0 : 2 + 5e-6 * p.heads * rows * p.dim);
+    const int    chunks = (p.max_q_len + kChunkT - 1) / kChunkT, dp = decay_tiles(p.dim) * 16;
+    const double whole = std::min((double)p.nseq * chunks * kChunkT, rows + (kChunkT - 1.0) * p.nseq), tile = (double)dp * std::max(p.vdim, dp / 2);
+    const double blocks = 9.9 + 0.081 * dp + std::max((0.035 + 0.0013 * dp) * chunks * kChunkT, (0.00038 + 1.6e-7 * tile) * p.heads * whole) + 3.3e-6 * p.heads * p.nseq * tile;
+    return 1.05 * blocks < walk;
 }
 
 int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
@@ -949,8 +963,8 @@ int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
     if (p.max_q_len > 1 && kind == kStateBonus) {
         return launch_decay_chunks<kStateBonus>(p, st);
     }
-    TM_REQUIRE(!p.raw || (kind == kStateDelta && state_mix_chunks(p.max_q_len)), "state mixer: logits only for chunks of the delta rule");
-    if (kind == kStateDelta && state_mix_chunks(p.max_q_len)) {
+    TM_REQUIRE(!p.raw || (kind == kStateDelta && state_mix_chunks(p)), "state mixer: logits only for chunks of the delta rule");
+    if (kind == kStateDelta && state_mix_chunks(p)) {
         return launch_decay_chunks<kStateDelta>(p, st);
     }
     const int  wcols = 4 * kStateCW * kStateNC;  // value columns of a workgroup

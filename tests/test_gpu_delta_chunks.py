@@ -53,3 +53,24 @@ def test_sequences_of_all_lengths_in_a_launch(cuda, tmp_path, dtype):
     eng.step_tokens([(s, r, []) for s, r in zip(sess, reqs)])
     assert np.abs(eng.fetch_residual(sum(lens)) - ref).max() <= TOL[dtype] * 3 * np.abs(ref).max()
     eng.close()
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+def test_many_heads_are_walked(cuda, tmp_path, dtype):
+    """heads x sequences that fill the chip: portions beyond 32 tokens one token after the other, and in chunks again for a single sequence"""
+    cfg = fo.make_config(48, 61, [fo.delta_layer(32, 256, 8)])
+    rng = np.random.default_rng(4)
+    folder, w = model_folder(tmp_path, cfg, 11)
+    reqs = [rng.integers(0, 61, n).tolist() for n in (33, 40, 35, 36)]
+    eng = engine(folder, dtype, max_batch_size=len(reqs), cache_blocks=20)
+    eng.stop_after(1)
+    tol = TOL[dtype] * 3
+
+    def check(sess, toks, ref):
+        eng.step_tokens([(s, t, []) for s, t in zip(sess, toks)])
+        assert np.abs(eng.fetch_residual(len(ref)) - ref).max() <= tol * np.abs(ref).max()
+    refs = [fo.forward(cfg, w, r + r[:34], True)[1][0] for r in reqs]
+    sess = [eng.open_session() for _ in reqs]
+    check(sess, reqs, np.concatenate([f[:len(r)] for f, r in zip(refs, reqs)]))
+    check(sess[:1], [reqs[0][:34]], refs[0][33:67])
+    eng.close()

@@ -727,3 +727,18 @@ def _mixer(what, *sizes):
 def test_fp32_attention_takes_the_faster_kernel(sizes, heads):
     """measured where the two kernels of fp32 attention differ most: many rows of few keys with few heads a key head are the row kernel's"""
     assert _mixer(0, *sizes) == heads
+
+
+@pytest.mark.parametrize('sizes,chunks', [
+    # sequences, longest, rows, heads, dim, vdim, logits (us, walk / chunks)
+    ((1, 32, 32, 16, 128, 128, 1), 0), ((1, 33, 33, 16, 128, 128, 1), 1), ((8, 1000, 7900, 16, 128, 128, 1), 1), ((1, 1000, 1000, 32, 256, 256, 1), 1), ((4, 48, 192, 8, 64, 64, 0), 1),
+    ((32, 33, 1056, 16, 128, 128, 1), 0),      # 85 / 111
+    ((32, 33, 1056, 32, 32, 32, 1), 0),        # 35 / 52
+    ((4, 33, 132, 32, 256, 256, 1), 0),        # 76 / 117
+    ((32, 64, 2048, 32, 256, 256, 1), 0),      # 1005 / 1136
+    ((32, 96, 3072, 32, 128, 128, 0), 0),      # operands made either way: 378 / 376
+    ((32, 96, 3072, 32, 128, 128, 1), 1),      # 441 / 388
+])
+def test_delta_rule_takes_the_faster_kernel(sizes, chunks):
+    """portions of the delta rule run in chunks where that was measured to be faster: not where heads x sequences fill the chip and the portions are short"""
+    assert _mixer(1, *sizes) == chunks
