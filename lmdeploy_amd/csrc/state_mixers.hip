@@ -921,7 +921,7 @@ static int launch_decay_chunks(const StateMixParams& p, hipStream_t st)
 
 // Portions of the delta rule in chunks, or walked token by token.  A few heads x sequences leave the walk a chain of tokens, which chunks shorten; where there are enough of
 // them to fill the chip the walk is bound by its work, and chunks do about as much of it and more for the last, part-filled one.  A model of both in microseconds, fitted
-// to 800 sizes (32 ... 256 channels, 2 ... 2048 heads x sequences, 33 ... 1000 tokens): what it takes is 0.9 % slower than the better one on average.  us, walk with the launch
+// to 800 sizes (32 ... 256 channels, 2 ... 2048 heads x sequences, 33 ... 1000 tokens): what it takes is at most 6 % slower than the walk and 1.4 % slower than the better one on average.  us, walk with the launch
 // that prepares its operands / chunks: 128 channels, 16 heads, one prompt of 33 tokens 35 / 31, 8 of 1000 974 / 411, 32 of 33 85 / 111, 32 of 64 146 / 137; 256 channels, 32 heads, 32 of
 // 33 530 / 881, of 64 1005 / 1136, of 256 3890 / 3855.  Up to 32 tokens it was never chunks (one prompt of 32 29 / 31).  Without logits (raw: 0) the operands are prepared either way.
 bool state_mix_chunks(const StateMixParams& p)
@@ -935,7 +935,7 @@ bool state_mix_chunks(const StateMixParams& p)
     const int    chunks = (p.max_q_len + kChunkT - 1) / kChunkT, dp = decay_tiles(p.dim) * 16;
     const double whole = std::min((double)p.nseq * chunks * kChunkT, rows + (kChunkT - 1.0) * p.nseq), tile = (double)dp * std::max(p.vdim, dp / 2);
     const double blocks = 9.9 + 0.081 * dp + std::max((0.035 + 0.0013 * dp) * chunks * kChunkT, (0.00038 + 1.6e-7 * tile) * p.heads * whole) + 3.3e-6 * p.heads * p.nseq * tile;
-    return 1.05 * blocks < walk;
+    return 1.12 * blocks < walk;
 }
 
 int launch_state_mix(const StateMixParams& p, int kind, hipStream_t st)
