@@ -333,7 +333,7 @@ int tm_debug_stream_plan(int kind, int K, int N, int M, int scratch, int* plan5)
 /* Host-only: which kernel a mixer's launch of these sizes runs.  what 0: fp32 attention over a paged cache with 64-token blocks, sizes[9] = {rows, query heads, key heads,
  * dim, vdim, 1 for portions of prompts, rows of the longest portion, window, chunk}; *kernel = 1: the heads of a key head as a tile, 0: a wave a row and head.
  * what 1: the delta rule, sizes[7] = {sequences, rows of the longest portion, rows, heads, dim, vdim, 1 if its operands are still logits}; *kernel = 1: in chunks, 0: token by
- * token. */
+ * token.  what 2: the chunks of the other mixers with a state, the same sizes; *kernel = 1: the walk of short portions, 0: the one that is fed through LDS. */
 int tm_debug_mixer_kernel(int what, const int* sizes, int n, int* kernel);
 /* Host-only: every (shape, splits) pair the start-up tuner (tm_engine_tune_gemm; gemm::Gemm::Run's dispatch candidates,
  * src/turbomind/kernels/gemm/gemm.cu:92-224) may pick for a K x N linear at M rows; *count = how many exist (<= 128), the first

@@ -1018,15 +1018,15 @@ int tm_debug_stream_plan(int kind, int K, int N, int M, int scratch, int* plan5)
 
 int tm_debug_mixer_kernel(int what, const int* v, int n, int* kernel)
 {
-    TM_REQUIRE(v && kernel && (what == 0 ? n == 9 : what == 1 && n == 7), "arguments");
+    TM_REQUIRE(v && kernel && (what == 0 ? n == 9 : (what == 1 || what == 2) && n == 7), "arguments");
     for (int i = 0; i < n; ++i) {
         TM_REQUIRE(v[i] >= (i < 5 ? 1 : 0), "sizes");
     }
-    if (what == 1) {
+    if (what > 0) {
         StateMixParams m;
         m.nseq = v[0], m.max_q_len = v[1], m.rows = v[2], m.heads = v[3], m.dim = v[4], m.vdim = v[5], m.raw = v[6];
         TM_REQUIRE(m.dim <= 256 && m.vdim >= 1, "sizes");
-        *kernel = state_mix_chunks(m);
+        *kernel = what == 1 ? state_mix_chunks(m) : state_mix_short(m);
         return 0;
     }
     GeneralAttnParams p;

@@ -881,6 +881,134 @@ __global__ __launch_bounds__(384) void decay_chunks_kernel(StateMixParams p)
     }
 }
 
+// The walk of short portions (at most 128 channels; not the delta rule): as above, without LDS.  Each wave fetches its own operands, the next chunk's under this chunk's products:
+// nothing has to come through two barriers first, and more workgroups fit on a CU.  us with the blocks, this / the one above, forget gate, 16 heads of 128: one portion of 20
+// tokens 18.7 / 20.5, of 33 21.0 / 21.9, of 64 23.1 / 23.2, of 1000 156 / 108; 32 portions of 20 53 / 62; 32 heads of 32, 32 portions of 64 30 / 35, of 256 85 / 90.
+// grid (nseq, heads, ceil(vdim / 64)), 256 threads: wave -> 16 value columns; SILU: on the values
+template<int DR, bool SILU>
+__global__ __launch_bounds__(256) void decay_chunks_short_kernel(StateMixParams p)
+{
+    constexpr int NC = kStateNC, WV = kStateCW * kStateNC;
+    const int s = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, cb = blockIdx.z * 4 + (threadIdx.x >> 6);
+    const int D = p.dim, V = p.vdim, dq = (D + 7) / 8, ncb = (V + WV - 1) / WV;
+    if (cb >= ncb) {
+        return;
+    }
+    const int row0 = p.cu_q[s] - p.cu_q[0], q_len = p.cu_q[s + 1] - p.cu_q[s];
+    const int pos0 = p.k_len[s] - q_len, g = lane >> 4, col = cb * 16 + (lane & 15);
+    int       slot = p.seq_slot ? p.seq_slot[s] : p.slot0 + s;
+    if (p.active && !p.active[s]) {
+        slot = p.park_slot;
+    }
+    float* slab = p.state + (size_t)slot * p.slot_stride + p.layer_offset + ((size_t)h * ncb + cb) * dq * 64 * NC;
+    // element (d, column) of the slab as state_mix_kernel keeps it
+    auto at = [&](int d) { return ((d % dq) * NC + (lane & 15) % NC) * 64 + d / dq * kStateCW + (lane & 15) / NC; };
+    floatx4 S[DR];
+#pragma unroll
+    for (int r = 0; r < DR; ++r) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int d = r * 16 + g * 4 + i;
+            S[r][i]     = pos0 > 0 && d < D ? slab[at(d)] : 0.f;
+        }
+    }
+    constexpr size_t bf = decay_block_floats_of(DR, false);
+    const float* blk = p.blocks + (decay_chunk_index(s, row0, 0) * p.heads + h) * bf;
+    struct Operands {
+        floatx4 q[DR], k[DR], f[DR], a, v;
+    };
+    auto fetch = [&](Operands& o, int t0, const float* b) {
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {
+            o.q[r] = *(const floatx4*)(b + (size_t)(r * 64 + lane) * 4);
+            o.k[r] = *(const floatx4*)(b + (size_t)((DR + r) * 64 + lane) * 4);
+            o.f[r] = *(const floatx4*)(b + DR * 64 * 4 * 2 + 256 + r * 16 + g * 4);
+        }
+        o.a = *(const floatx4*)(b + DR * 64 * 4 * 2 + lane * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = min(t0 + g * 4 + e, q_len - 1);  // (keys behind the portion are zero: any finite value will do)
+            o.v[e]      = p.proj[(size_t)(row0 + t) * p.ld + p.c_v + h * V + min(col, V - 1)];
+        }
+    };
+    auto step = [&](Operands& o, int t0) {
+        if constexpr (SILU) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o.v[e] = sm_silu(o.v[e]);
+            }
+        }
+        floatx4 y[4], ya = {0.f, 0.f, 0.f, 0.f};  // short chains of sums: independent products for the matrix core and less rounding
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            y[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                y[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[r][i], S[r][i], y[i], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            ya = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[e], o.v[e], ya, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < DR; ++r) {
+            S[r] *= o.f[r];
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int r = 0; r < DR; ++r) {
+                S[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[r][e], o.v[e], S[r], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int t = t0 + g * 4 + i;
+            if (t < q_len && col < V) {
+                p.out[(size_t)(row0 + t) * p.ldo + h * V + col] = ((y[0][i] + y[1][i]) + (y[2][i] + y[3][i])) + ya[i];
+            }
+        }
+    };
+    const size_t next = (size_t)p.heads * bf;
+    Operands a, b;
+    if (q_len > 0) {
+        fetch(a, 0, blk);
+    }
+    for (int t0 = 0; t0 < q_len; t0 += 2 * kChunkT, blk += 2 * next) {
+        const bool more = t0 + kChunkT < q_len;
+        if (more) {
+            fetch(b, t0 + kChunkT, blk + next);
+        }
+        step(a, t0);
+        if (t0 + 2 * kChunkT < q_len) {
+            fetch(a, t0 + 2 * kChunkT, blk + 2 * next);
+        }
+        if (more) {
+            step(b, t0 + kChunkT);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < DR; ++r) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int d = r * 16 + g * 4 + i;
+            if (d < dq * 8) {  // (the slab's padding rows are stored as the zeros they are)
+                slab[at(d)] = S[r][i];
+            }
+        }
+    }
+}
+
+// Up to three chunks, and heads of few channels that fill the chip several times over, whose blocks are small against what the other walk's stages take of a CU
+bool state_mix_short(const StateMixParams& p)
+{
+    return decay_tiles(p.dim) <= 8 && (p.max_q_len <= 3 * kChunkT || (decay_tiles(p.dim) == 2 && (int64_t)p.nseq * p.heads * ((p.vdim + 63) / 64) >= 1024));
+}
+
 template<int DR, int KIND>
 static int launch_decay_chunks_dr(const StateMixParams& p, hipStream_t st)
 {
@@ -897,6 +1025,13 @@ static int launch_decay_chunks_dr(const StateMixParams& p, hipStream_t st)
     }
     else {
         decay_blocks_kernel<DR, KIND><<<gb, 256, 0, st>>>(p, chunks);
+        if constexpr (DR <= 8) {
+            if (state_mix_short(p)) {
+                decay_chunks_short_kernel<DR, KIND == kStateLinear><<<gc, 256, 0, st>>>(p);
+                TM_HIP_CHECK(hipGetLastError());
+                return 0;
+            }
+        }
     }
     const auto k = decay_chunks_kernel<DR, KIND == kStateLinear, DELTA>;
     if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {

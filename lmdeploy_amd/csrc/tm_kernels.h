@@ -755,6 +755,7 @@ size_t state_mix_floats(int heads, int dim, int vdim);  // floats of one layer's
 size_t decay_workspace_floats(int rows, int nseq, int heads, int dim, bool delta);
 enum { kStateLinear = 0, kStateDelta = 1, kStateForget = 2, kStateRetention = 3, kStateBonus = 4 };
 bool   state_mix_chunks(const StateMixParams& p);  // the delta rule runs this launch in chunks (sizes and `raw` only: whether logits are what it would take)
+bool   state_mix_short(const StateMixParams& p);  // the other mixers' portions are short: their chunks are walked without LDS
 int    launch_state_mix(const StateMixParams& p, int kind, hipStream_t st);
 int    launch_delta_prep(float* proj, int ld, int c_k, int c_a, float* decay, int ld_w, float* unit, int ld_u, int rows, int heads, int dim,
                          hipStream_t st);

@@ -742,3 +742,14 @@ def test_fp32_attention_takes_the_faster_kernel(sizes, heads):
 def test_delta_rule_takes_the_faster_kernel(sizes, chunks):
     """portions of the delta rule run in chunks where that was measured to be faster: not where heads x sequences fill the chip and the portions are short"""
     assert _mixer(1, *sizes) == chunks
+
+
+@pytest.mark.parametrize('sizes,short', [
+    # sequences, longest, rows, heads, dim, vdim (us, short walk / the other)
+    ((1, 20, 20, 16, 128, 128, 0), 1), ((32, 20, 640, 16, 128, 128, 0), 1), ((1, 48, 48, 16, 64, 64, 0), 1),     # 19 / 21, 53 / 61
+    ((1, 49, 49, 16, 128, 128, 0), 0), ((8, 1000, 7900, 16, 128, 128, 0), 0), ((1, 20, 20, 16, 129, 129, 0), 0), ((1, 20, 20, 16, 256, 256, 0), 0),
+    ((32, 256, 8192, 32, 32, 32, 0), 1), ((32, 256, 8192, 16, 32, 32, 0), 0), ((16, 256, 4096, 32, 20, 65, 0), 1),   # 85 / 90
+])
+def test_short_portions_of_states_take_the_faster_walk(sizes, short):
+    """portions of up to three chunks of 16 tokens, and heads of few channels that fill the chip, take the walk that needs no LDS"""
+    assert _mixer(2, *sizes) == short
