@@ -130,48 +130,52 @@ static int linear_plain(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, 
 // of its rows (gemm_rows.h): no norm launch between them.  The first has to have whole sums: one slice of k, or slices that meet inside its launch.  8 sequences of
 // InternLM2-1.8B's layer: output product 4.6 -> 4.8 us, norm 3.1 -> 0, gate / up 12.2 -> 12.1; down product, whose seven slices now meet, 7.4 -> 10.4, norm 4.4 -> 0,
 // [q | k | v] 6.0 -> 5.5.  W4: up to eight rows, where the first product is about as fast in one slice (output products; of a long k, one row).  Linears that a measured table gives to other kernels keep their launches.
-static bool adds_to_resid(const tm_engine* e, const LinearWeight& w, int M)
+static bool adds_to_resid(const tm_engine* e, const LinearWeight& w, const GemmConfig& cfg, int M)
 {
     if (M > 16 || e->hidden % 4) {
         return false;
     }
-    const GemmConfig cfg = gemm_pick_config(w, M);
     if (w.type == 0) {
         return cfg.d32_shape == kShapeRows && w4_rows_whole(w, M);
     }
     return cfg.f16_stream && (cfg.splits <= 1 || gemm_workspace_bytes(M, w.N, cfg.splits) > e->gemm_ws_bytes || (w.N + 63) / 64 <= e->n_tickets);
 }
 
-static bool norm_in_product(const tm_engine* e, const LinearSlots& first, const LinearSlots& second, int M)
+bool norm_in_product(const tm_engine* e, const LinearWeight& first, const GemmConfig& c1, const LinearWeight& second, const GemmConfig& c2, int M)
 {
     if (e->use_comm || e->p2p_ready || M > 16) {
         return false;
     }
-    const GemmConfig cfg = gemm_pick_config(second.w, M);
-    const bool       ok  = second.w.type == 0 ? cfg.d32_shape == kShapeRows && cfg.splits == 1 && w4_norm_rows_supported(second.w, M) :
-                                                cfg.f16_stream && f16_norm_rows_supported(second.w, M);
-    return ok && adds_to_resid(e, first.w, M);
+    const bool ok = second.type == 0 ? c2.d32_shape == kShapeRows && c2.splits == 1 && w4_norm_rows_supported(second, M) : c2.f16_stream && f16_norm_rows_supported(second, M);
+    return ok && adds_to_resid(e, first, c1, M);
+}
+
+static bool norm_in_product(const tm_engine* e, const LinearSlots& first, const LinearSlots& second, int M)
+{
+    return M <= 16 && norm_in_product(e, first.w, gemm_pick_config(first.w, M), second.w, gemm_pick_config(second.w, M), M);
+}
+
+int linear_residual(tm_engine* e, const LinearWeight& w, GemmConfig cfg, const half_t* x, int ldx, int M)
+{
+    if (w.type == 0) {
+        return launch_w4_rows(w, x, ldx, e->d_resid, e->hidden, M, false, 1, nullptr, nullptr, e->stream, true);
+    }
+    int slabs;
+    if (gemm_workspace_bytes(M, w.N, cfg.splits) > e->gemm_ws_bytes) {
+        cfg.splits = 1;
+    }
+    return launch_f16_stream(w, x, ldx, e->d_resid, e->hidden, M, false, cfg.splits, e->d_gemm_ws, e->d_tickets, e->n_tickets, false, &slabs, e->stream, nullptr, nullptr, true);
 }
 
 static int linear_residual(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, int M)
 {
-    if (l.w.type == 0) {
-        return launch_w4_rows(l.w, x, ldx, e->d_resid, e->hidden, M, false, 1, nullptr, nullptr, e->stream, true);
-    }
-    GemmConfig cfg = gemm_pick_config(l.w, M);
-    int        slabs;
-    if (gemm_workspace_bytes(M, l.w.N, cfg.splits) > e->gemm_ws_bytes) {
-        cfg.splits = 1;
-    }
-    return launch_f16_stream(l.w, x, ldx, e->d_resid, e->hidden, M, false, cfg.splits, e->d_gemm_ws, e->d_tickets, e->n_tickets, false, &slabs, e->stream, nullptr, nullptr,
-                             true);
+    return linear_residual(e, l.w, gemm_pick_config(l.w, M), x, ldx, M);
 }
 
-// y = rmsnorm(residual stream) . W
-static int linear_norm_rows(tm_engine* e, LinearSlots& l, const half_t* norm_w, half_t* y, int ldy, int M, bool gated, const F16KvSink* kv = nullptr)
+int linear_norm_rows(tm_engine* e, const LinearWeight& w, const half_t* norm_w, half_t* y, int ldy, int M, bool gated, const F16KvSink* kv)
 {
-    return l.w.type == 0 ? launch_w4_norm_rows(l.w, e->d_resid, norm_w, e->cfg.model.rms_eps, y, ldy, M, gated, e->stream) :
-                           launch_f16_norm_rows(l.w, e->d_resid, norm_w, e->cfg.model.rms_eps, y, ldy, M, gated, e->stream, kv);
+    return w.type == 0 ? launch_w4_norm_rows(w, e->d_resid, norm_w, e->cfg.model.rms_eps, y, ldy, M, gated, e->stream) :
+                         launch_f16_norm_rows(w, e->d_resid, norm_w, e->cfg.model.rms_eps, y, ldy, M, gated, e->stream, kv);
 }
 
 // Tensor-parallel prefill forward, dense layer, from the attention output to the next layer's QKV projection, as two row halves
@@ -545,7 +549,7 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
         if (norm_in_qkv) {
             const F16KvSink sink{e->d_k_len, e->d_rope, e->rope_max_pos, e->q_heads, cv};
             const bool      store = L.qkv.w.type == 1 && !fuse_qkv && cv.layout.bits == 16 && e->D == 128;
-            TM_PROF(P_GEMM_QKV, TM_TRY(linear_norm_rows(e, L.qkv, L.attn_norm, e->d_qkv, e->qkv_n, M, false, store ? &sink : nullptr)));
+            TM_PROF(P_GEMM_QKV, TM_TRY(linear_norm_rows(e, L.qkv.w, L.attn_norm, e->d_qkv, e->qkv_n, M, false, store ? &sink : nullptr)));
             if (!fuse_qkv && !store) {
                 TM_PROF(P_KV_STORE, TM_TRY(launch_kv_rope_store(qkv_p, e->q_heads, e->d_cu_q, e->d_k_len, nseq, M, e->d_rope, e->rope_max_pos, cv, st)));
             }
@@ -698,7 +702,7 @@ int forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int ma
         const bool norm_in = decode && !L.is_moe && norm_in_product(e, L.wo, L.w13, M);
         if (norm_in) {
             TM_PROF(P_GEMM_O, TM_TRY(linear_residual(e, L.wo, e->d_attn, e->q_heads * e->D, M)));
-            TM_PROF(P_GEMM_GATE_UP, TM_TRY(linear_norm_rows(e, L.w13, L.ffn_norm, e->d_act, e->inter, M, true)));
+            TM_PROF(P_GEMM_GATE_UP, TM_TRY(linear_norm_rows(e, L.w13.w, L.ffn_norm, e->d_act, e->inter, M, true, nullptr)));
         }
         else {
             TM_TRY(linear_residual_norm(e, L.wo, e->d_attn, e->q_heads * e->D, M, L.ffn_norm, P_GEMM_O));

@@ -491,6 +491,10 @@ int sample_rows(tm_engine* e, int n, int slot, const int* ids_in, const int* cu_
                 const StepCommit* commit);
 int greedy_alloc(tm_engine* e);
 int greedy_rows(tm_engine* e, int n, int slot, const float* logits32, const StepCommit& commit);
+// few rows of a decode step: `first` adds to the residual stream itself and `second` makes the norm of its rows (with these configurations), no launch between them ...
+bool norm_in_product(const tm_engine* e, const LinearWeight& first, const GemmConfig& c1, const LinearWeight& second, const GemmConfig& c2, int M);
+int  linear_residual(tm_engine* e, const LinearWeight& w, GemmConfig cfg, const half_t* x, int ldx, int M);  // ... residual stream += x . w
+int  linear_norm_rows(tm_engine* e, const LinearWeight& w, const half_t* norm_w, half_t* y, int ldy, int M, bool gated, const F16KvSink* kv);  // ... y = rmsnorm(residual stream) . w
 int moe_rows(tm_engine* e, const MoeBlock& moe, half_t* y, const half_t* x, int M, const half_t* norm_w);
 int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode, int max_q_len, int max_k_len, int slot0, const MixedDecode* md,
                     const StepEnds* ends);

@@ -5,6 +5,65 @@
 
 namespace tmk {
 
+// ------------------------------------------------------------------------------------------------------------------
+// wo and w1w3, w2 and the next layer's w_qkv at a few rows of a decode step: the norm between them is a launch of its own or made by the second product
+// (norm_in_product), as both configurations allow, so a candidate of either is timed with the other, on its measured or own choice, and whatever stands between them.
+// ------------------------------------------------------------------------------------------------------------------
+struct NormPair {
+    const LinearWeight *first, *second;
+    const half_t*       norm_w;
+};
+
+static bool norm_pairs(const tm_engine* e, int M, int type)
+{
+    return M <= (type == 0 ? 8 : 16) && !e->use_comm && !e->p2p_ready && e->layers.size() >= 2 && !e->layers[0].is_moe && !(e->fold_norm != 0 && M <= e->fold_max_rows);
+}
+
+// the pairs of role `which` (0 qkv, 1 wo, 2 w13, 3 w2), one a layer
+static std::vector<NormPair> pairs_of(tm_engine* e, int which)
+{
+    std::vector<NormPair> out;
+    for (size_t i = 0; i < e->layers.size(); ++i) {
+        Layer& L = e->layers[i];
+        Layer& n = e->layers[(i + 1) % e->layers.size()];
+        out.push_back(which == 1 || which == 2 ? NormPair{&L.wo.w, &L.w13.w, L.ffn_norm} : NormPair{&L.w2.w, &n.qkv.w, n.attn_norm});
+    }
+    return out;
+}
+
+static int run_pair(tm_engine* e, const NormPair& p, int which, GemmConfig c1, GemmConfig c2, half_t* normed, int M)
+{
+    const bool          ffn = which == 1 || which == 2;
+    hipStream_t         st  = e->stream;
+    half_t* const       y   = ffn ? e->d_act : e->d_qkv;
+    const half_t* const x   = ffn ? e->d_attn : e->d_act;
+    const int           ldy = ffn ? e->inter : e->qkv_n, ldx = ffn ? e->q_heads * e->D : e->inter;
+    for (GemmConfig* c : {&c1, &c2}) {
+        c->splits       = gemm_workspace_bytes(M, (c == &c1 ? p.first : p.second)->N, c->splits) > e->gemm_ws_bytes ? 1 : c->splits;
+        c->tickets      = e->d_tickets;
+        c->ticket_count = e->n_tickets;
+    }
+    if (norm_in_product(e, *p.first, c1, *p.second, c2, M)) {
+        TM_TRY(linear_residual(e, *p.first, c1, x, ldx, M));
+        return linear_norm_rows(e, *p.second, p.norm_w, y, ldy, M, ffn, c2.kv);
+    }
+    int slabs = 1;
+    TM_TRY(launch_linear(*p.first, x, ldx, e->d_tmp, e->hidden, M, false, c1, e->d_gemm_ws, c1.splits > 1, &slabs, st));
+    TM_TRY(launch_residual_rmsnorm(normed, e->d_resid, slabs > 1 ? nullptr : e->d_tmp, slabs > 1 ? e->d_gemm_ws : nullptr, slabs, nullptr, p.norm_w,
+                                   e->cfg.model.rms_eps, M, e->hidden, st));
+    return launch_linear(*p.second, normed, e->hidden, y, ldy, M, ffn, c2, e->d_gemm_ws, false, nullptr, st);
+}
+
+// what a role's winner has to be faster by: 7 % of the role (see below), of a pair the part that its weights are, but not less than the spread between runs
+static float tune_bar(const NormPair* p, int which)
+{
+    if (!p) {
+        return 0.07f;
+    }
+    const double a = (double)p->first->K * p->first->N, b = (double)p->second->K * p->second->N, own = which == 1 || which == 3 ? a : b;
+    return 0.07f * (float)std::max(0.6, own / (a + b));
+}
+
 }  // namespace tmk
 
 extern "C" {
@@ -17,7 +76,7 @@ extern "C" {
 // Cache holds, as in a decode step -- and each node is followed by the kernel that consumes its result (the fused split-K
 // reduce + residual + RMSNorm for wo / w2, the slab reduce standing in for the attention prologue for w_qkv): a split-K
 // GEMM looks cheap in isolation and pays at the kernel boundary (profiles/r02_gemm_boundary_gap.txt).  The winner enters
-// the (K, N, M) table that dec32_pick consults first; it replaces the heuristic only when it is >= 7 % faster.
+// the (K, N, M) table that dec32_pick consults first; it replaces the heuristic only when it is >= 7 % faster.  (Few rows: pairs of roles, NormPair above.)
 // ------------------------------------------------------------------------------------------------------------------
 int tune_decode_gemms(tm_engine* e, int M, bool verbose)
 {
@@ -65,6 +124,7 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
             continue;
         }
         const LinearWeight& w0 = *ws[0];
+        const std::vector<NormPair> pairs = norm_pairs(e, M, 0) ? pairs_of(e, r.which) : std::vector<NormPair>{};
         int                 hs, hp;
         if (dec32_table_get(w0.K, w0.N, M, &hs, &hp, r.which + 1)) {
             continue;  // imported / tuned already
@@ -114,7 +174,17 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
                 continue;
             }
             cfg.tickets = e->d_tickets;
+            bool together = false;
             auto chain = [&]() -> int {
+                for (const NormPair& p : pairs) {
+                    const bool       one = r.which == 1 || r.which == 3;  // the role is the pair's first product
+                    const GemmConfig c1 = one ? cfg : gemm_pick_config(*p.first, M), c2 = one ? gemm_pick_config(*p.second, M) : cfg;
+                    together            = norm_in_product(e, *p.first, c1, *p.second, c2, M);
+                    TM_TRY(run_pair(e, p, r.which, c1, c2, norm_out, M));
+                }
+                if (!pairs.empty()) {
+                    return 0;
+                }
                 if (folded) {
                     const int tiles = e->hidden / 64;
                     for (const LinearWeight* w : ws) {
@@ -145,7 +215,7 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
                 }
                 return 0;
             };
-            if (norm_consumer) {  // the chain accumulates into the residual stream: every candidate starts from zero
+            if (norm_consumer || !pairs.empty()) {  // the chain accumulates into the residual stream: every candidate starts from zero
                 TM_HIP_CHECK(hipMemsetAsync(e->d_resid, 0, (size_t)M * e->hidden * 2, st));
             }
             if ((rc = chain())) {  // eager once: lazy module loading, function attributes
@@ -198,8 +268,9 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
                 bp   = cand[i][1];
             }
             if (verbose) {
-                fprintf(stderr, "[tm tune] %-5s K=%d N=%d M=%d shape %d splits %2d: %7.2f us / layer%s\n", r.name, w0.K, w0.N, M, cand[i][0],
-                        cand[i][1], us, (cand[i][0] == hs && cand[i][1] == hp) ? "  <- heuristic" : "");
+                fprintf(stderr, "[tm tune] %-5s K=%d N=%d M=%d shape %d splits %2d: %7.2f us / layer%s%s\n", r.name, w0.K, w0.N, M, cand[i][0],
+                        cand[i][1], us, pairs.empty() ? "" : together ? " (norm in its product)" : " (norm between products)",
+                        (cand[i][0] == hs && cand[i][1] == hp) ? "  <- heuristic" : "");
             }
         }
         if (rc) {
@@ -209,7 +280,7 @@ int tune_decode_gemms(tm_engine* e, int M, bool verbose)
         // measured 18.35 / 18.72 / 19.13 us in three starts on one box), and the chain here is not the model (the same kernel back
         // to back, its activations hot in L2): with a 3 % bar w2 of Llama-3-8B once flipped from (3, 4) to (6, 2) -- 12 % slower in
         // the model (0.61 vs 0.54 ms per step)
-        if (!(best < 0.93f * heur)) {
+        if (!(best < (1.f - tune_bar(pairs.empty() ? nullptr : &pairs[0], r.which)) * heur)) {
             bs = hs;
             bp = hp;
         }
@@ -362,6 +433,7 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
             continue;
         }
         const LinearWeight& w0 = *ws[0];
+        const std::vector<NormPair> pairs = r.which < 4 && w0.type == 1 && norm_pairs(e, M, 1) ? pairs_of(e, r.which) : std::vector<NormPair>{};
         if (gen_table_get(kGenDense + w0.type, w0.role, w0.K, w0.N, Mb, tv)) {
             continue;  // imported / tuned already
         }
@@ -399,8 +471,20 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
             bool            stored = false;
             cfg.kv                 = kv.k_len ? &sink : nullptr;
             cfg.kv_done            = &stored;
+            bool together          = false;
             auto chain = [&]() -> int {
-                for (const LinearWeight* w : ws) {
+                for (const NormPair& p : pairs) {
+                    const bool one = r.which == 1 || r.which == 3;
+                    GemmConfig c1 = one ? cfg : gemm_pick_config(*p.first, M), c2 = one ? gemm_pick_config(*p.second, M) : cfg;
+                    c1.kv    = nullptr;
+                    together = norm_in_product(e, *p.first, c1, *p.second, c2, M);
+                    stored   = together && c2.kv;
+                    TM_TRY(run_pair(e, p, r.which, c1, c2, norm_out, M));
+                    if (kv.k_len && !stored) {
+                        TM_TRY(launch_kv_rope_store(r.y, e->q_heads, kv.cu, kv.k_len, M, M, e->d_rope, e->rope_max_pos, kv.view, st));
+                    }
+                }
+                for (const LinearWeight* w : pairs.empty() ? ws : std::vector<const LinearWeight*>{}) {
                     int slabs = 1;
                     stored    = false;
                     TM_TRY(launch_linear(*w, r.x, r.ldx, r.y, r.ldy, M, r.gated, cfg, e->d_gemm_ws, norm_consumer && cfg.splits > 1, &slabs, st));
@@ -420,7 +504,7 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
                 }
                 return 0;
             };
-            if (norm_consumer) {
+            if (norm_consumer || !pairs.empty()) {
                 TM_HIP_CHECK(hipMemsetAsync(e->d_resid, 0, (size_t)M * e->hidden * 2, st));
             }
             float us = 1e30f;
@@ -434,11 +518,11 @@ static int tune_aux_gemms(tm_engine* e, int M, bool verbose)
                 bc   = cfg;
             }
             if (verbose) {
-                fprintf(stderr, "[tm tune] %-7s K=%d N=%d M=%d general nt %d splits %d: %8.2f us%s\n", r.name, w0.K, w0.N, M, cfg.nt, cfg.splits, us,
-                        same(cfg, heur) ? "  <- heuristic" : "");
+                fprintf(stderr, "[tm tune] %-7s K=%d N=%d M=%d general nt %d splits %d: %8.2f us%s%s\n", r.name, w0.K, w0.N, M, cfg.nt, cfg.splits, us,
+                        pairs.empty() ? "" : together ? " (norm in its product)" : " (norm between products)", same(cfg, heur) ? "  <- heuristic" : "");
             }
         }
-        if (!(best < 0.93f * t_heur)) {
+        if (!(best < (1.f - tune_bar(pairs.empty() ? nullptr : &pairs[0], r.which)) * t_heur)) {
             bc = heur;
         }
         if (kv.k_len) {
