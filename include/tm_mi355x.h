@@ -314,8 +314,9 @@ int64_t tm_debug_trace_records(char* host_out, int64_t cap);
  * role with its own consumer kernel; an entry of role 0, e.g. an imported line without a role column, serves every role).
  * Shapes: 0..3 decode tiles (M <= 64), 4 / 5 the 128-row tiles of 256 / 512 columns (M > 64), 6..9 shapes 3, 0, 2, 1 on 32-row blocks
  * (gemm_decode.hip), 11 the loader / consumer decode kernel (gemm_decode_lc.hip, M <= 64), 12 the 256 x 256 prefill tile with
- * each weight dequantised once per workgroup tile, in registers (gemm_prefill.hip, M > 64), 14 the row kernel (gemm_w4_rows.hip, M <= 16).  An explicit shape and a table line run exactly the
- * tile they name.  (10 was a vendor-library path: gone.) */
+ * each weight dequantised once per workgroup tile, in registers (gemm_prefill.hip, M > 64), 14 the row kernel (gemm_w4_rows.hip, M <= 16, where the rows of a
+ * slice of k fit in LDS).  An explicit shape and a table line run exactly the tile they name, or are refused; of 14, up to eight rows of a decode step may run in one slice and leave
+ * their norm to the next product.  (10 was a vendor-library path: gone.) */
 int tm_debug_pick_tiling(int K, int N, int M, int use_table, int* shape, int* splits);
 /* Host-only: the tiling of the general kernel (gemm_w4a16.hip: the fp16 lm_head, e4m3 weight-only linears, u4 with N % 32 != 0)
  * for a K x N linear of `weight_type` (TM_WEIGHT_*) and `role` (0 any, 1 w_qkv, 2 wo, 3 w1w3, 4 w2, 5 lm_head) at M rows:

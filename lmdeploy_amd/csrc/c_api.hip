@@ -311,6 +311,7 @@ int tm_linear_forward(const tm_linear* w, const void* x, int ldx, void* y, int l
         // operator level: the fp16 image is built on first use (the engine builds it at load)
         TM_TRY_RC(linear_weight_build_f16_image(const_cast<tm_linear*>(w)->w, (hipStream_t)st));
     }
+    const bool rows_named = waves > 0 && (waves & 0x200) && (waves & 0xff) == kShapeRows;
     if (waves > 0 && (waves & 0x200)) {
         // 0x200 + shape: the decode kernel (gemm_decode.hip) with an explicit workgroup shape; M <= 64, u4, N % 32 == 0
         TM_REQUIRE(dec32_supported(w->w, M), "decode kernel: u4 weights, N % 32 == 0");
@@ -339,6 +340,7 @@ int tm_linear_forward(const tm_linear* w, const void* x, int ldx, void* y, int l
     if (!workspace) {
         cfg.splits = 1;
     }
+    TM_REQUIRE(!rows_named || w4_rows_supported(w->w, M, cfg.splits), "shape 14: the rows of a slice of k fit in LDS, every slice has k-blocks");
     return launch_linear(w->w, (const half_t*)x, ldx, (half_t*)y, ldy, M, gated_silu != 0, cfg, (float*)workspace, false,
                          nullptr, (hipStream_t)st);
 }

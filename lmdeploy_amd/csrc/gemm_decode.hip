@@ -1410,7 +1410,9 @@ int dec32_table_import(const char* path)
         const bool lc  = shape == kShapeLC && M <= 64;
         const bool p256 = (shape == kShapePre256 || (shape == kShapeF16 && splits == 1)) && M > 64;  // what launch_linear_dec32 accepts (the tuner only proposes them for M, N >= 256)
         const bool mrg = dec32_is_merge_shape(shape) && M <= 64 && splits >= 2;  // in-launch merged split-K (decode batches only)
-        const bool w2k = (shape == kShapeWide2 && M <= 64) || (shape == kShapeRows && M <= 16);
+        LinearWeight w{};
+        w.K = K, w.N = N;
+        const bool w2k = (shape == kShapeWide2 && M <= 64) || (shape == kShapeRows && K > 0 && N > 0 && K % 128 == 0 && N % 32 == 0 && w4_rows_supported(w, M, splits));
         if (K > 0 && N > 0 && M > 0 && M == dec32_m_bucket(M) && shape >= 0 && (shape <= 9 || lc || p256 || mrg || w2k) && splits >= 1 && splits <= 16
             && (big ? shape >= 4 : (shape != 4 && shape != 5)) && !(shape == 5 && N < 512) && K % 128 == 0 && N % 32 == 0) {
             dec32_table_set(K, N, M, shape, splits, role);
@@ -1740,7 +1742,7 @@ int launch_linear_dec32(const LinearWeight& w, const half_t* x, int ldx, half_t*
         if (w4_rows_supported(w, M, splits)) {
             return launch_w4_rows(w, x, ldx, y, ldy, M, gated_silu, splits, workspace, slabs_out, st);
         }
-        int own;  // (without room for slabs its rows need not fit in LDS)
+        int own;  // (a plan's slices were dropped for want of a workspace, or others were asked for: its rows need not fit in LDS)
         dec32_pick_plain(w, M, &shape, &own, false);
     }
     if (dec32_is_merge_shape(shape)) {  // split-K merged in the launch (fp16 / gated epilogues); a producer does that anyway

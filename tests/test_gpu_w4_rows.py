@@ -74,6 +74,19 @@ def test_infinities(tm, cuda, K, N, splits, gated, M):
     assert same.all()
 
 
+def test_a_named_shape_runs_or_is_refused(tm, cuda):
+    """rows beyond LDS, slices without k-blocks, and a launch whose slices would be dropped for want of a workspace"""
+    rng = np.random.default_rng(1)
+    for K, M, splits, ws, ok in ((14336, 16, 1, True, False), (14336, 16, 4, True, True), (14336, 16, 4, False, False), (14336, 4, 4, False, True), (2304, 8, 8, True, False)):
+        h, _ = _make_linear(tm, rng, K, 64)
+        x, y = dev(rng.standard_normal((M, K)).astype(np.float16)), torch.full((M, 64), 7.0, dtype=torch.float16, device='cuda')
+        buf = torch.zeros(tm.tm_linear_workspace(h, M), dtype=torch.uint8, device='cuda')
+        rc = tm.tm_linear_forward(h, x.data_ptr(), K, y.data_ptr(), 64, M, 0, 0, splits, 0x200 | ROWS, buf.data_ptr() if ws else None, st())
+        assert (rc == 0) == ok and (ok or (host(y) == 7.0).all()), (K, M, splits, ws)
+        assert tm.tm_linear_forward(h, x.data_ptr(), K, y.data_ptr(), 64, M, 0, 0, splits, 0, buf.data_ptr() if ws else None, st()) == 0    # (no shape named)
+        _ffi.check(tm.tm_linear_destroy(h))
+
+
 def test_what_a_launch_takes(tm, cuda):
     def pick(K, N, M):
         sh, sp = _ffi.C.c_int(), _ffi.C.c_int()

@@ -706,6 +706,18 @@ def test_wide_few_row_products_without_slabs(K, N, M, rows):
     assert (_pick(_ffi.load(), K, N, M, 4)[0] == 14) == rows
 
 
+def test_lines_that_the_row_kernel_cannot_run_are_skipped(tmp_path):
+    """shape 14 keeps the rows of a slice of k in LDS and gives every slice k-blocks: a line that asks for more is not filed, one that asks for as much is"""
+    lib = _ffi.load()
+    f = tmp_path / 't.txt'
+    for line, ok in (('14336 2080 16 14 1', False), ('2304 2080 8 14 8', False), ('14336 2080 16 14 4', True), ('2304 2080 8 14 6', True)):
+        K, N, M, _, sp = map(int, line.split())
+        before = _pick(lib, K, N, M, 5)
+        f.write_text(line + '\n')
+        assert (lib.tm_gemm_import(str(f).encode()) == 0) == ok
+        assert _pick(lib, K, N, M, 5) == ((14, sp) if ok else before)
+
+
 def _mixer(what, *sizes):
     k = _ffi.C.c_int(-1)
     _ffi.check(_ffi.load().tm_debug_mixer_kernel(what, (_ffi.C.c_int * len(sizes))(*sizes), len(sizes), _ffi.C.byref(k)))
