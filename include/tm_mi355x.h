@@ -191,7 +191,7 @@ int    tm_linear_dequant_f16(const tm_linear* w, void* out_nk, tm_stream_t st);
  * followed by invokeResidualBiasRMSNorm (src/turbomind/models/llama/unified_decoder.cc:149,226; kernels/norm/rms_norm.cu:286-362):
  *   resid += fp16(x . W);  y = RMSNorm(resid) * norm_w.
  * The GEMM (fp32 split-K slabs when it splits), then the reduce-norm kernel.
- * shape: decode tile 0..3 / 6..9 / 11, -1 = dispatch; splits: 0 = dispatch.  workspace >= tm_linear_workspace(w, M) + M * N * 2 bytes. */
+ * shape: decode tile 0..3 / 6..9 / 11, or 14 (the row kernel, M <= 16), -1 = dispatch (of the tiles); splits: 0 = dispatch.  workspace >= tm_linear_workspace(w, M) + M * N * 2 bytes. */
 int    tm_linear_residual_norm(const tm_linear* w, const void* x, int ldx, void* y, void* resid, const void* norm_w, float eps, int M,
                                int shape, int splits, void* workspace, tm_stream_t st);
 /* The same pair of operators with the RMSNorm FOLDED into the two GEMMs around it (the engine's decode step at tp = 1):

@@ -351,13 +351,13 @@ int tm_linear_residual_norm(const tm_linear* w, const void* x, int ldx, void* y,
     TM_REQUIRE(w && x && y && resid && norm_w && workspace, "null pointer");
     const int N = w->w.N;
     GemmConfig cfg = gemm_pick_config(w->w, M);
-    if (cfg.d32_shape == kShapeRows) {  // (its residual stream is tm_linear_fold_produce's, to the bit: the tiles that both have)
-        dec32_pick_plain(w->w, M, &cfg.d32_shape, &cfg.splits, true);
+    if (cfg.d32_shape == kShapeRows) {  // (the tiles that tm_linear_fold_produce has too, also where a measured line names the row kernel)
+        dec32_pick_plain(w->w, M, &cfg.d32_shape, &cfg.splits, false);
     }
     if (shape >= 0) {
-        TM_REQUIRE(dec32_supported(w->w, M) && (shape <= 3 || (shape >= 6 && shape <= 10) || shape == kShapeLC)
+        TM_REQUIRE(dec32_supported(w->w, M) && (shape <= 3 || (shape >= 6 && shape <= 10) || shape == kShapeLC || (shape == kShapeRows && M <= 16))
                        && (M <= 64 || (M <= kFoldMaxRows && shape >= 6 && shape <= 9)),
-                   "decode tile 0..3 / 6..10 / 11 at M <= 64; the 32-row-block tiles 6..9 up to 128 rows");
+                   "decode tile 0..3 / 6..10 / 11 at M <= 64; the row kernel 14 at M <= 16; the 32-row-block tiles 6..9 up to 128 rows");
         cfg.d32_shape = shape;
     }
     if (splits > 0) {
@@ -365,6 +365,7 @@ int tm_linear_residual_norm(const tm_linear* w, const void* x, int ldx, void* y,
         cfg.f16_stream = false;  // (its slices are its own)
     }
     TM_REQUIRE(cfg.splits <= 16, "splits <= 16");
+    TM_REQUIRE(shape != kShapeRows || w4_rows_supported(w->w, M, cfg.splits), "shape 14: the rows of a slice of k fit in LDS, every slice has k-blocks");
     // slabs (or, with one slice, the fp16 product parked at the end of the workspace) + the reduce-norm kernel
     int     slabs = 1;
     half_t* tmp   = (half_t*)((char*)workspace + gemm_workspace_bytes(M, N, 16));

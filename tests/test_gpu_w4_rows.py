@@ -87,6 +87,47 @@ def test_a_named_shape_runs_or_is_refused(tm, cuda):
         _ffi.check(tm.tm_linear_destroy(h))
 
 
+def _residual(tm, h, x, N, M, shape, splits):
+    rng = np.random.default_rng(M)
+    r, g = dev(rng.standard_normal((M, N)).astype(np.float16)), dev(rng.choice([0.5, 1, 2], N).astype(np.float16))
+    y, before = torch.zeros((M, N), dtype=torch.float16, device='cuda'), host(r).astype(np.float64)
+    ws = torch.zeros(tm.tm_linear_workspace(h, M) + 2 * M * N, dtype=torch.uint8, device='cuda')
+    _ffi.check(tm.tm_linear_residual_norm(h, dev(x).data_ptr(), x.shape[1], y.data_ptr(), r.data_ptr(), g.data_ptr(), 1e-5, M, shape, splits, ws.data_ptr(), st()))
+    return host(r).astype(np.float64), host(y).astype(np.float64), before, host(g).astype(np.float64)
+
+
+@pytest.mark.parametrize('K,N,M,splits', [(2304, 2144, 8, 1), (2304, 2144, 8, 2), (2304, 2144, 13, 4), (4096, 512, 1, 4)])
+def test_slabs_and_the_norm_behind_them(tm, cuda, K, N, M, splits):
+    """the row kernel's slabs through the launch that adds them to the residual stream and makes its norm, as an engine runs them"""
+    rng = np.random.default_rng(K + N + M)
+    h, _ = _make_linear(tm, rng, K, N)
+    q, s, z = _QCACHE[(K, N)][:3]
+    x = (3 * rng.standard_normal((M, K))).astype(np.float16)
+    r, y, before, g = _residual(tm, h, x, N, M, ROWS, splits)
+    _ffi.check(tm.tm_linear_destroy(h))
+    ref = before + x.astype(np.float64) @ (q * np.repeat(s.astype(np.float64), 128, 0) + np.repeat((-z * s).astype(np.float16).astype(np.float64), 128, 0))
+    rms = np.sqrt((ref**2).mean(1, keepdims=True))
+    assert (np.abs(r - ref) <= 2.0**-10 * np.abs(ref) + 2.0**-9 * rms).all()            # the product's rounding to fp16 and the sum's
+    norm = r / np.sqrt((r**2).mean(1, keepdims=True) + 1e-5) * g
+    assert (np.abs(y - norm) <= 2.0**-9 * np.abs(norm) + 2.0**-14).all()                # two roundings to fp16, a row sum in fp32
+
+
+def test_the_residual_stream_keeps_its_tile_with_a_line(tm, cuda, tmp_path):
+    """a measured line that names the row kernel is the engine's: tm_linear_residual_norm has the bits that it has without one"""
+    K, N, M = 2432, 2208, 8
+    rng = np.random.default_rng(2)
+    h, _ = _make_linear(tm, rng, K, N)
+    x = rng.standard_normal((M, K)).astype(np.float16)
+    first = _residual(tm, h, x, N, M, -1, 0)
+    assert not np.array_equal(first[0], _residual(tm, h, x, N, M, ROWS, 2)[0])          # (or this would show nothing)
+    f = tmp_path / 't.txt'
+    f.write_text(f'{K} {N} {M} {ROWS} 2\n')
+    assert tm.tm_gemm_import(str(f).encode()) == 0
+    again = _residual(tm, h, x, N, M, -1, 0)
+    _ffi.check(tm.tm_linear_destroy(h))
+    assert np.array_equal(first[0], again[0]) and np.array_equal(first[1], again[1])
+
+
 def test_what_a_launch_takes(tm, cuda):
     def pick(K, N, M):
         sh, sp = _ffi.C.c_int(), _ffi.C.c_int()
