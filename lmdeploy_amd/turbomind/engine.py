@@ -132,10 +132,10 @@ class Engine:
     @staticmethod
     def pick_tiling(K: int, N: int, M: int, use_table: bool = True, role: int = 0, folded: bool = False):
         """(shape, split-K) the decode GEMM dispatch runs a K x N W4A16 linear with at M rows (measured table first); role: 0 any,
-        1 w_qkv, 2 wo, 3 w1w3, 4 w2 -- the measured table is keyed (role, K, N, M); folded: in a launch with a folded norm.  (Up to 16 rows without a
-        measured line a launch runs the row kernel in place of the tile: tm_debug_pick_tiling, bit 2)"""
+        1 w_qkv, 2 wo, 3 w1w3, 4 w2 -- the measured table is keyed (role, K, N, M); folded: in a launch with a folded norm.  use_table=False: the tile of the
+        rule alone, without measured lines and without the row kernel that launches of up to 16 rows take in place of a tile"""
         sh, sp = C.c_int(), C.c_int()
-        flags = (1 if use_table else 0) | (0 if folded else 2) | (role << 8)
+        flags = (1 if use_table else 0) | (0 if folded else 6 if use_table else 2) | (role << 8)
         _ffi.check(_ffi.load().tm_debug_pick_tiling(K, N, M, flags, C.byref(sh), C.byref(sp)))
         return sh.value, sp.value
 

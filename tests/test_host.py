@@ -74,6 +74,20 @@ def test_reported_tiling_of_launches_without_a_folded_norm():
     assert Engine.pick_tiling(4096, 6144, 8, use_table=False, folded=True) == _pick(lib, 4096, 6144, 8, 0)
 
 
+def test_reported_tiling_of_up_to_16_rows(tmp_path):
+    """Engine.pick_tiling says what a launch runs: the row kernel up to 16 rows, the tile beyond and in folded launches, a measured line wherever there is one"""
+    from lmdeploy_amd.turbomind.engine import Engine
+    lib = _ffi.load()
+    for K, N, M, role in ((4096, 28672, 1, 3), (4096, 6144, 8, 1), (4096, 4096, 16, 2)):
+        assert Engine.pick_tiling(K, N, M, role=role) == _pick(lib, K, N, M, 5, role) and Engine.pick_tiling(K, N, M, role=role)[0] == 14
+        assert Engine.pick_tiling(K, N, M, role=role, folded=True) == _pick(lib, K, N, M, 1, role) != _pick(lib, K, N, M, 5, role)
+    assert Engine.pick_tiling(4096, 6144, 17) == _pick(lib, 4096, 6144, 17, 3)
+    f = tmp_path / 't.txt'
+    f.write_text('2176 6144 8 3 2\n')
+    assert Engine.pick_tiling(2176, 6144, 8)[0] == 14 and lib.tm_gemm_import(str(f).encode()) == 0
+    assert Engine.pick_tiling(2176, 6144, 8) == (3, 2)
+
+
 def test_the_pick_decides_between_the_prefill_tiles(tmp_path):
     """The dispatch of launches without a folded norm itself names the 128 x 512 (5) or the 256 x 256 tile (12), and a table line that names one of them is
     what it answers where the rule would take the other."""
