@@ -608,7 +608,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
         const dim3 grid((unsigned)((a.tiles + p.cw - 1) / p.cw), G * p.row_blocks, p.splits);
         const bool pairs = epi == kDenseGatedAct && sizeof(T) == 2;
 #define TM_SKINNY(MT_, NT_, CW_, KP_)                                                    \
-    if (p.mt == MT_ && p.cw == CW_ * NT_ && pairs == (NT_ == 2)) {                                              \
+    if (p.mt == MT_ && p.cw == CW_ * NT_ && pairs == (NT_ == 2)) {                       \
         if (p.narrow) {                                                                  \
             return launch_dense_narrow<T, MT_, NT_>(a, call, vec, G, st);                \
         }                                                                                \
@@ -616,7 +616,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
     }
         TM_STREAM_SHAPES(TM_SKINNY)
         if constexpr (sizeof(T) == 2) {
-            TM_STREAM_SHAPES_PAIRS(TM_SKINNY)
+            TM_STREAM_SHAPES_WIDE(TM_SKINNY) TM_STREAM_SHAPES_PAIRS(TM_SKINNY)
         }
 #undef TM_SKINNY
     }

@@ -847,9 +847,10 @@ __host__ __device__ inline size_t dense_frag_index(int n, int k, int steps)
 }
 
 // ---- which kernel, which shape -------------------------------------------------------------------------------------------------------
-// (row tiles, column tiles a wave, column waves, k-phases) of the skinny kernels that exist: 64 columns a workgroup of four waves, 96 of six and 128 of eight where those
-// fill the CUs more evenly or read x less often, and 128 columns where a wave needs a pair of column tiles.  k-phases gave nothing at 184 sizes.
-#define TM_STREAM_SHAPES(X) X(1, 1, 4, 1) X(2, 1, 4, 1) X(4, 1, 4, 1) X(1, 1, 6, 1) X(2, 1, 6, 1) X(4, 1, 6, 1) X(1, 1, 8, 1) X(2, 1, 8, 1) X(4, 1, 8, 1)
+// (row tiles, column tiles a wave, column waves, k-phases) of the skinny kernels that exist: 64 columns a workgroup of four waves, 96 of six where those
+// fill the CUs more evenly; bf16 beyond 16 rows also 128 of eight, which read x less often; and 128 columns where a wave needs a pair of column tiles.  k-phases gave nothing at 184 sizes.
+#define TM_STREAM_SHAPES(X) X(1, 1, 4, 1) X(2, 1, 4, 1) X(4, 1, 4, 1) X(1, 1, 6, 1) X(2, 1, 6, 1) X(4, 1, 6, 1)
+#define TM_STREAM_SHAPES_WIDE(X) X(2, 1, 8, 1) X(4, 1, 8, 1)
 #define TM_STREAM_SHAPES_PAIRS(X) X(1, 2, 4, 2) X(2, 2, 4, 2) X(4, 2, 4, 1)
 
 // waves of the narrow kernel (row tiles x column tiles <= 2): eight where sixteen would have nothing to do, or would keep a second workgroup off the CU
