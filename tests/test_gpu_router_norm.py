@@ -17,12 +17,15 @@ def test_router_behind_the_norm(tmp_path, cuda, monkeypatch, width, experts, row
     w = fo.random_weights(cfg, experts + width)
     folder = str(tmp_path / 'm')
     fo.write_checkpoint(folder, cfg, w)
-    toks = np.random.default_rng(rows).integers(0, 97, rows).tolist()
+    gaps, seed = [], rows
+    monkeypatch.setattr(fo, 'moe_ff', lambda *a: _moe_ff(*a, gaps))
+    while not (gaps and (np.concatenate(gaps) > 0.05).any()):        # (one row alone may have no clear choice, and would show nothing)
+        gaps.clear()
+        toks = np.random.default_rng(seed).integers(0, 97, rows).tolist()
+        ref = fo.forward(cfg, w, toks)
+        seed += 1000
     eng = engine(folder, 'bfloat16', max_batch_size=2, cache_blocks=12, session_len=512, max_prefill_token_num=512)
     got = eng.step_tokens([(eng.open_session(), toks, list(range(rows)))]).reshape(rows, -1)
-    gaps = []
-    monkeypatch.setattr(fo, 'moe_ff', lambda *a: _moe_ff(*a, gaps))
-    ref = fo.forward(cfg, w, toks)
     clear = np.concatenate(gaps) > 0.05
-    assert (rows < 20 or clear.mean() > 0.5) and np.abs(got - ref)[clear].max(initial=0) <= TOL['bfloat16'] * np.abs(ref).max()
+    assert clear.any() and (rows < 20 or clear.mean() > 0.5) and np.abs(got - ref)[clear].max() <= TOL['bfloat16'] * np.abs(ref).max()
     eng.close()
