@@ -130,9 +130,6 @@ __device__ __forceinline__ float fast_exp2(float x)
     return __builtin_amdgcn_exp2f(x);  // v_exp_f32 (no denormal range handling needed here)
 }
 
-// ---- results of several workgroups met in one launch ----
-// Partial results are written through to the device's memory (agent_store), drained, and counted in a ticket that is zero between launches; who arrives last
-// reads them past its caches (agent_load) and finishes.  No workgroup waits for another.
 // A pointer that a table holds as a number.  Cast to a plain pointer its loads are flat ones, which count as LDS traffic too and return in no order that a
 // wait could use: whatever is in flight has to arrive before the first of them is used (fp32 attention, 16 / 1 heads of 256 / 192, a prompt
 // of 2000: 667 -> 597 us, row kernel 7810 -> 7165; 2 decoded rows over 2000 29.4 -> 27.4)
@@ -141,6 +138,9 @@ __device__ __forceinline__ char* global_ptr(uint64_t address)
     return (char*)(__attribute__((address_space(1))) char*)address;
 }
 
+// ---- results of several workgroups met in one launch ----
+// Partial results are written through to the device's memory (agent_store), drained, and counted in a ticket that is zero between launches; who arrives last
+// reads them past its caches (agent_load) and finishes.  No workgroup waits for another.
 __device__ __forceinline__ void agent_store(float* p, float v)
 {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
