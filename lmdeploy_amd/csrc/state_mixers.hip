@@ -503,7 +503,7 @@ __global__ __launch_bounds__(256) void decay_blocks_kernel(StateMixParams p, int
 // the e of a chunk solve (I + Aub) E = U0 S0 + Auk V, and
 //   o = Q0 S0 + Aqk V - Aqb E,   S = P(0..15) S0 + K1^T V - B1^T E      (Q0, K1 and B1 with their running products as above).
 // Aub is strictly lower triangular: (I + Aub)^-1 is applied to the columns of U0 and Auk by forward substitution here, a column a thread, so that the walk
-// over the chunks has E by products alone.  The substitution is the recurrence itself on those columns, token after token, and grows as that does: with |u| = 1 and rates and
+// over the chunks has E by products alone.  The substitution is the recurrence itself on those columns, token after token, and grows as that does: with |u| <= 1 and rates and
 // decays in [0, 1] a factor diag(w) - b u^T may lengthen a vector where the rates differ from channel to channel, by 2 / sqrt 3 at most, and does not where they are alike.
 // Block: as above, then U [DR][64][4], B1 [DR][64][4], Aqb [64][4], W = (I + Aub)^-1 Auk [64][4].  Dynamic LDS: delta_blocks_lds(DR)
 constexpr int delta_blocks_lds(int dr)
