@@ -316,7 +316,9 @@ bool w4_rows_supported(const LinearWeight& w, int M, int slices)
 }
 
 // Products below what was timed stay with gemm_dec32_kernel (whose rows have the bits that they have in forwards of more rows), and so do more than eight rows of a long
-// k: (14336, 4096) 16 rows 16.1 here, 15.9 there.  A slice has eight k-blocks at least; a gate / up product's slabs are nobody's to sum but a launch's of its own (3.3 us).
+// k: (14336, 4096) 16 rows 16.1 here, 15.9 there.  A slice has eight k-blocks at least; a gate / up product's slabs are nobody's to sum but a launch's of its own: in
+// a model's step 1 us of the model above's, also against one slice that makes its norm (176 sizes, K 4096 ... 8192, N 3584 ... 14336: on average 0.05 us a layer from the best).  us a
+// layer, gemm_dec32_kernel | one slice | four: (8192, 3584) 9 rows 48.8 | 53.6 | 48.0, 8 rows 48.8 | 51.4 | 47.5, (7168, 4096) 9 rows 45.3 | 48.1 | 44.0, (8192, 7168) 4 rows 51.4 | 48.0 | 48.9.
 // Wide products whose rows do not fit in LDS whole would have slices only for that, and slabs of all columns: where gemm_dec32_kernel needs none, it keeps them, unless more than a
 // quarter of its last round of 128-column workgroups stays empty.  us, there | here in two slices: (5120, 20480) 16 rows 16.9 | 22.5, (6144, 28672) 14 rows 22.5 | 26.7, (8192, 57344)
 // 12 rows 54.6 | 59.6, (16384, 20480) 8 rows 42.7 | 47.6, 4 rows 45.1 | 40.8; (8192, 40960), 1.25 rounds, 12 rows 50.8 | 44.9
@@ -333,7 +335,7 @@ bool w4_rows_plan(const LinearWeight& w, int M, int* slices)
         if ((s > 1 && KB / s < 8) || !w4_rows_supported(w, M, s) || w4_rows_shape(ncg, KB, M, s, &cost) < 0) {
             continue;
         }
-        cost += s > 1 && w.role == 3 ? 3.3 : 0.0;
+        cost += s > 1 && w.role == 3 ? 1.0 : 0.0;
         if (*slices == 0 || cost < best) {
             *slices = s, best = cost;
         }

@@ -720,6 +720,15 @@ def test_wide_few_row_products_without_slabs(K, N, M, rows):
     assert (_pick(_ffi.load(), K, N, M, 4)[0] == 14) == rows
 
 
+@pytest.mark.parametrize('K,N,M,slices', [
+    # us a layer in a model's step, one slice / four
+    (8192, 3584, 9, 4), (7168, 4096, 9, 4), (8192, 7168, 8, 4), (6144, 8192, 12, 4),    # 53.6 / 48.0, 48.1 / 44.0, 53.0 / 50.4, 49.8 / 48.4
+    (7168, 4096, 1, 1), (8192, 7168, 4, 1), (4096, 7168, 8, 1), (5120, 9216, 14, 1)])   # 39.9 / 41.3, 48.0 / 48.9, 40.6 / 42.4, 49.0 / 52.0
+def test_slices_of_gate_up_products(K, N, M, slices):
+    """gate / up products of up to 16 rows take slices of k, whose slabs need a launch of their own, where a model's step gains by them"""
+    assert _pick(_ffi.load(), K, N, M, 4 | 3 << 8) == (14, slices)
+
+
 def test_lines_that_the_row_kernel_cannot_run_are_skipped(tmp_path):
     """shape 14 keeps the rows of a slice of k in LDS and gives every slice k-blocks: a line that asks for more is not filed, one that asks for as much is"""
     lib = _ffi.load()
