@@ -129,14 +129,14 @@ static int linear_plain(tm_engine* e, LinearSlots& l, const half_t* x, int ldx, 
 // A decode step of a few rows, dense layers: a product that closes a residual block adds to the residual stream itself, and the product behind it makes the norm
 // of its rows (gemm_rows.h): no norm launch between them.  The first has to have whole sums: one slice of k, or slices that meet inside its launch.  8 sequences of
 // InternLM2-1.8B's layer: output product 4.6 -> 4.8 us, norm 3.1 -> 0, gate / up 12.2 -> 12.1; down product, whose seven slices now meet, 7.4 -> 10.4, norm 4.4 -> 0,
-// [q | k | v] 6.0 -> 5.5.  W4: up to eight rows, where the first product is about as fast in one slice (output products; of a long k, one row).  Linears that a measured table gives to other kernels keep their launches.
-static bool adds_to_resid(const tm_engine* e, const LinearWeight& w, const GemmConfig& cfg, int M)
+// [q | k | v] 6.0 -> 5.5.  W4: up to eight rows, where it pays (w4_norm_pays).  Linears that a measured table gives to other kernels keep their launches.
+static bool adds_to_resid(const tm_engine* e, const LinearWeight& w, const GemmConfig& cfg, const LinearWeight& next, int M)
 {
     if (M > 16 || e->hidden % 4) {
         return false;
     }
     if (w.type == 0) {
-        return cfg.d32_shape == kShapeRows && w4_rows_whole(w, M);
+        return cfg.d32_shape == kShapeRows && w4_norm_pays(w, next, M);
     }
     return cfg.f16_stream && (cfg.splits <= 1 || gemm_workspace_bytes(M, w.N, cfg.splits) > e->gemm_ws_bytes || (w.N + 63) / 64 <= e->n_tickets);
 }
@@ -147,7 +147,7 @@ bool norm_in_product(const tm_engine* e, const LinearWeight& first, const GemmCo
         return false;
     }
     const bool ok = second.type == 0 ? c2.d32_shape == kShapeRows && c2.splits == 1 && w4_norm_rows_supported(second, M) : c2.f16_stream && f16_norm_rows_supported(second, M);
-    return ok && adds_to_resid(e, first, c1, M);
+    return ok && adds_to_resid(e, first, c1, second, M);
 }
 
 static bool norm_in_product(const tm_engine* e, const LinearSlots& first, const LinearSlots& second, int M)

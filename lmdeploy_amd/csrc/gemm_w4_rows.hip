@@ -395,15 +395,16 @@ int launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, i
 #undef TM_W4_ROWS
 }
 
-// One slice of k, for a product that closes a residual block and leaves the norm to the next: it may cost little more than the plan's slices, less than the launch that it
-// spares (3.3 us of a model's step, of which the next product takes 0.4 back).  us, whole | slices and their norm: (4096, 4096) one row 9.4 | 9.4 (norm in both), 8 rows 11.7 | 9.9;
-// (14336, 4096) one row 14.8 | 12.6 (cost 1.2 apart, taken), two 16.1 | 13.3 (1.7, not taken)
-bool w4_rows_whole(const LinearWeight& w, int M)
+// `first` in one slice of k, adding to the residual stream, and the norm made by `next`, instead of the plan's slices and a norm launch that sums them: it spares a launch, costs what
+// one slice is slower by, and every workgroup of the next product norms all rows once more.  Fitted to 180 pairs in the steps of 19 models (hidden 2048 ... 8192, 1 ... 8
+// rows): on average 0.04 us a layer from the better side, 0.9 at most.  us a layer, launch | pair: (4096, 4096) and (4096, 28672) one row 50.1 | 49.1, 8 rows 53.3 | 55.5; (5120, 5120)
+// and (5120, 55296) one row 80.5 | 78.8, 4 rows 80.5 | 83.4, 8 rows 85.6 | 92.1; (2048, 2048) and (2048, 16384) 8 rows 37.3 | 36.1; (8192, 2048) and (2048, 4096) one row 35.6 | 34.6, 4 rows 36.8 | 37.9
+bool w4_norm_pays(const LinearWeight& first, const LinearWeight& next, int M)
 {
     int    slices;
     double one, best;
-    return w4_rows_plan(w, M, &slices) && w4_rows_supported(w, M, 1) && w4_rows_shape(w.N / 32, w.K / 128, M, 1, &one) >= 0
-           && w4_rows_shape(w.N / 32, w.K / 128, M, slices, &best) >= 0 && one <= best + 1.4;
+    return w4_rows_plan(first, M, &slices) && w4_rows_supported(first, M, 1) && w4_rows_shape(first.N / 32, first.K / 128, M, 1, &one) >= 0
+           && w4_rows_shape(first.N / 32, first.K / 128, M, slices, &best) >= 0 && one - best + 0.6 * M * (next.K / 8192.0) * (next.N / 28672.0) <= 1.25;
 }
 
 bool w4_norm_rows_supported(const LinearWeight& w, int M)

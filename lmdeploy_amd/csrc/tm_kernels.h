@@ -254,7 +254,7 @@ bool   w4_rows_supported(const LinearWeight& w, int M, int slices);
 bool   w4_rows_plan(const LinearWeight& w, int M, int* slices);
 int    launch_w4_rows(const LinearWeight& w, const half_t* x, int ldx, half_t* y, int ldy, int M, bool gated, int slices, float* workspace, int* slabs, hipStream_t st,
                       bool add = false);
-bool   w4_rows_whole(const LinearWeight& w, int M);
+bool   w4_norm_pays(const LinearWeight& first, const LinearWeight& next, int M);
 bool   w4_norm_rows_supported(const LinearWeight& w, int M);
 int    launch_w4_norm_rows(const LinearWeight& w, const half_t* resid, const half_t* norm_w, float eps, half_t* y, int ldy, int M, bool gated, hipStream_t st);
 // measured dispatch table of the decode linears: key (K, N, M <= 64) -> (shape, splits)
