@@ -146,7 +146,7 @@ bool norm_in_product(const tm_engine* e, const LinearWeight& first, const GemmCo
     if (e->use_comm || e->p2p_ready || M > 16) {
         return false;
     }
-    const bool ok = second.type == 0 ? c2.d32_shape == kShapeRows && c2.splits == 1 && w4_norm_rows_supported(second, M) : c2.f16_stream && f16_norm_rows_supported(second, M);
+    const bool ok = second.type == 0 ? c2.d32_shape == kShapeRows && c2.splits == 1 && w4_norm_rows_supported(second, M) : c2.f16_stream && f16_norm_rows_supported(second, M) && f16_norm_rows_pays(second);
     return ok && adds_to_resid(e, first, c1, second, M);
 }
 

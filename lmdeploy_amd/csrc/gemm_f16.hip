@@ -262,6 +262,16 @@ bool f16_norm_rows_supported(const LinearWeight& w, int M)
     return w.type == 1 && w.packed && (size_t)w.K * w.N * 2 < ((size_t)1 << 31) && w.K % 512 == 0 && M >= 1 && (M <= 8 ? w.K <= 4096 : M <= 16 && w.K <= 2048);
 }
 
+// Beyond 512 column tiles a workgroup takes four, whatever their number: where the fullest CU then streams longer than memory takes for all of them, and than a plan of four or six
+// tiles would leave it, by more than a norm launch is worth, the launch stays.  us a layer, launch | norm in the product, 8 rows (12 and 16 alike): (2048, 16896) 44.8 | 47.3, (2048, 22016)
+// 48.7 | 49.6, (2560, 19456) 53.2 | 56.8, (1536, 17920) 41.4 | 43.2, (4096, 19456) 76.3 | 82.0; (2048, 24576) 50.9 | 50.8, one row 50.5 | 48.3; (2048, 16384) 43.6 | 42.2
+bool f16_norm_rows_pays(const LinearWeight& w)
+{
+    const int tiles = w.N / 16;
+    auto      us    = [&](int cw) { return ((tiles + cw - 1) / cw + 255) / 256 * cw * (w.K * 32 / 33e3); };  // a CU's load path: 33 KB a microsecond
+    return tiles <= 512 || us(4) <= std::max(tiles * (w.K * 32 / 6e6), std::min(us(4), us(6))) + 0.75;
+}
+
 template<int CW, int KP, int R, class Epi>
 static int launch_rows_of(const StreamArgs& a, const Epi& epi, const half_t* resid, const half_t* norm_w, float eps, hipStream_t st)
 {

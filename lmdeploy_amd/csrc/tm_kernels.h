@@ -239,6 +239,7 @@ int  launch_f16_stream(const LinearWeight& w, const half_t* x, int ldx, half_t* 
                        bool add = false /* y += x . W, rounded to fp16 first (few rows, one slab) */);
 // few rows with their norm: y = rmsnorm(resid) . W
 bool f16_norm_rows_supported(const LinearWeight& w, int M);
+bool f16_norm_rows_pays(const LinearWeight& w);
 int  launch_f16_norm_rows(const LinearWeight& w, const half_t* resid, const half_t* norm_w, float eps, half_t* y, int ldy, int M, bool gated, hipStream_t st,
                           const F16KvSink* kv = nullptr);
 

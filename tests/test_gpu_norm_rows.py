@@ -60,9 +60,9 @@ def test_decode_w4(cuda, hidden, heads, kv_heads, inter, batch, attention, norms
             batch, attention, True, norms)
 
 
-# gate / up products that are faster behind a norm launch: W4 whose many workgroups would norm many rows each
+# gate / up products that are faster behind a norm launch: fp16 whose last round of four-tile workgroups is nearly empty, W4 whose many workgroups would norm many rows each
 @pytest.mark.parametrize('hidden,heads,kv_heads,inter,batch,quantized,norms', [
-    (4096, 16, 2, 11008, 8, True, 4), (2048, 16, 2, 8192, 8, True, 2)])
+    (2048, 4, 1, 8448, 3, False, 3), (1536, 4, 1, 8960, 12, False, 3), (4096, 16, 2, 11008, 8, True, 4), (2048, 16, 2, 8192, 8, True, 2)])
 def test_norm_launches_that_stay(cuda, hidden, heads, kv_heads, inter, batch, quantized, norms):
     _decode(o.ModelConfig(hidden=hidden, layers=2, q_heads=heads, kv_heads=kv_heads, head_dim=128, inter=inter, vocab=256, kv_bits=8 if quantized else 16,
                           rope=o.RopeParam(128, 10000.0)), batch, False, quantized, norms)
