@@ -329,7 +329,8 @@ int tm_debug_grouped_tile(int weight_type, int K, int N, int tokens, int* rows);
 /* Host-only: what a plain product x [M][K] . W of N columns runs.  kind 0: bf16, 1: fp32 (tm_dense_forward and the layer-list engines), 2: fp16 (TM_WEIGHT_F16
  * linears); scratch: 1 with slabs and arrival counters for slices of k (an engine), 0 without (tm_dense_forward).  plan5 = {kernel, column tiles a workgroup,
  * row tiles of 16, slices of k, columns of a first launch of 256 x 256 tiles (0: one launch)}; kernel 0: the general kernel (kind 2 only), 1: narrow, 2: the
- * weight stream with rows in LDS, 3 .. 6: tiles of 256 x 256, 256 x 128, 128 x 128, 64 x 64. */
+ * weight stream with rows in LDS, 3 .. 6: tiles of 256 x 256, 256 x 128, 128 x 128, 64 x 64.  kind 0 and 1: items with rows of their own, M in total, in bits 8 .. 19 of kind (0: one
+ * plain product), the most rows that one of them has in bits 20 .. 30. */
 int tm_debug_stream_plan(int kind, int K, int N, int M, int scratch, int* plan5);
 /* Host-only: which kernel a mixer's launch of these sizes runs.  what 0: fp32 attention over a paged cache with 64-token blocks, sizes[9] = {rows, query heads, key heads,
  * dim, vdim, 1 for portions of prompts, rows of the longest portion, window, chunk}; *kernel = 1: the heads of a key head as a tile, 0: a wave a row and head.

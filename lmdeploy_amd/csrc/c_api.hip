@@ -1014,7 +1014,7 @@ int tm_debug_grouped_tile(int weight_type, int K, int N, int tokens, int* rows)
 
 int tm_debug_stream_plan(int kind, int K, int N, int M, int scratch, int* plan5)
 {
-    TM_REQUIRE(plan5 && kind >= 0 && kind <= 2 && K > 0 && N > 0 && M > 0 && (kind != 2 || (K % 128 == 0 && N % 16 == 0)), "arguments");
+    TM_REQUIRE(plan5 && kind >= 0 && ((kind & 0xff) <= 1 || kind == 2) && K > 0 && N > 0 && M > 0 && (kind != 2 || (K % 128 == 0 && N % 16 == 0)), "arguments");
     stream_plan_report(kind, K, N, M, scratch != 0, plan5);
     return 0;
 }

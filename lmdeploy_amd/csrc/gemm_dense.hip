@@ -468,12 +468,13 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
     if (sp > 1 && ((size_t)items * sp * rows * cols * 4 > ws_bytes || groups > tickets)) {
         sp = 1, best.narrow = true;
     }
-    // One slice: 96 columns a workgroup where the fullest CU then streams fewer.  Items with rows of their own count as often as rows dealt at random leave one
-    // any.  Nine items of (2816, 2048), 8 tokens, 288 workgroups of 64 columns 21.4 us, 198 of 96 17.9; but one token, three items with rows, whole steps 2.5 to 5 %
-    // slower with 66 workgroups than with 96
-    const int used = (own_rows ? (int)std::ceil(items * (1.0 - std::pow(1.0 - 1.0 / items, rows))) : items) * rb;
-    const int g64 = (cols + 63) / 64 * used, g96 = (cols + 95) / 96 * used;
-    if (sp == 1 && items > 1 && elem == 2 && !pairs && !best.narrow && border % 96 == 0 && g64 <= 1024 && (g96 + 255) / 256 * 6 < (g64 + 255) / 256 * 4) {
+    // One slice: 96 columns a workgroup where the fullest CU then streams fewer, if of items with rows of their own nearly all have some (less than one is expected to have none,
+    // rows dealt at random).  Where fewer have rows the CUs that get a second workgroup of 64 columns wait less for it than six waves of one CU for their loads.  us a routed layer in
+    // a step, 64 | 96 columns: nine items, top 2, (4096, 2048) 8 rows 102.6 | 96.0, 16 rows 114.2 | 106.5; seventeen, top 2, (4096, 2048) 4 rows 123.6 | 129.2, (1408, 2048) 4 rows
+    // 66.2 | 69.6; nine, (2048, 2816) 4 rows 73.3 | 75.6; seventeen, top 4, (2048, 1536) 6 rows 82.8 | 85.3, (2048, 1024) 12 rows 73.4 | 69.5
+    const bool all = !own_rows || items * std::pow(1.0 - 1.0 / items, rows) < 0.85;
+    const int  g64 = (cols + 63) / 64 * items * rb, g96 = (cols + 95) / 96 * items * rb;
+    if (sp == 1 && items > 1 && elem == 2 && !pairs && !best.narrow && border % 96 == 0 && all && g64 <= 1024 && (g96 + 255) / 256 * 6 < (g64 + 255) / 256 * 4) {
         best.cw = 6;
     }
     const int    ss = ((steps + sp - 1) / sp + 7) / 8 * 8;

@@ -712,6 +712,16 @@ def test_line_between_the_kernels_of_fp16_products():
             assert stream_plan(2, 4096, 128 * wgs, rows)[0] == kernel, (wgs, rows)
 
 
+@pytest.mark.parametrize('items,top,K,N,tokens,tiles', [
+    # us a routed layer in a step, 64 / 96 columns a workgroup
+    (9, 2, 4096, 2048, 8, 6), (9, 2, 2816, 2048, 16, 6), (17, 4, 2048, 1024, 12, 6),                             # 102.6 / 96.0, 94.1 / 90.0, 73.4 / 69.5
+    (17, 2, 4096, 2048, 4, 4), (17, 2, 3072, 2048, 5, 4), (17, 2, 1408, 2048, 4, 4),                             # 123.6 / 129.2, 104.1 / 108.3, 66.2 / 69.6
+    (9, 2, 2048, 2816, 4, 4), (9, 2, 2048, 2816, 16, 4), (17, 4, 2048, 1536, 6, 4), (33, 4, 2048, 1024, 5, 4)])  # 73.3 / 75.6, 94.1 / 98.5, 82.8 / 85.3, 79.1 / 82.1
+def test_columns_of_experts_workgroups(items, top, K, N, tokens, tiles):
+    """experts (one of them shared) of a few tokens: 96 columns a workgroup only where that was measured to be faster, with rows for nearly every expert"""
+    assert stream_plan(items << 8 | tokens << 20, K, N, tokens * (top + 1))[1] == tiles
+
+
 @pytest.mark.parametrize('K,N,M,rows', [(5120, 20480, 14, True), (5120, 20480, 16, False), (5120, 27648, 16, False), (6144, 28672, 14, False), (8192, 28672, 9, True), (8192, 28672, 10, False),
                                         (8192, 57344, 12, False), (8192, 40960, 12, True), (8192, 14336, 16, True), (8192, 57344, 8, True), (16384, 20480, 8, False),
                                         (16384, 20480, 4, True), (16384, 20480, 1, True)])
