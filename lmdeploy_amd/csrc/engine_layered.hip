@@ -160,7 +160,7 @@ static int plain_up_col(const LmLayer& L)
 }
 
 // Bytes of the projections and the head, each as an image of its own (columns rounded up to 128): neither what lies between tiles that stand apart in memory nor the
-// columns between the two parts of a fused image
+// columns between the two parts of a fused image.  fp32 engines count their parameters in fp32, though the images hold the bf16 numbers that they are
 int64_t layered_weight_bytes(const tm_engine* e)
 {
     auto bytes = [](const DenseWeight& d, int gap) { return (int64_t)d.Kp * (d.Np - gap) * d.count * (d.dtype == kDenseF32 ? 4 : 2); };

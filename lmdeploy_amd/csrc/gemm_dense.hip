@@ -1,7 +1,8 @@
 // Dense linears with unquantised weights: y = x . W^T for W stored [N][K] (the checkpoint's own orientation), in two number formats.
 //
 //   bf16 : weights and activations bfloat16, fp32 accumulation on the matrix cores (v_mfma_f32_16x16x32_bf16).
-//   fp32 : weights and activations fp32, multiplied and added in 32 bits (v_mfma_f32_16x16x4_f32).
+//   fp32 : activations fp32, weights as they come (bf16, every one an fp32 number), multiplied and added in 32 bits: a row's numbers are split
+//          into three of bf16 on the way to the matrix cores (StreamOp).
 //
 // The kernels are gemm_stream.h's: the weight stream for up to 64 rows (a decode step), tiles staged in LDS for more (prompts).
 // Weights are kept as zero-padded images of Np x Kp elements in fragment order (Np % 128 == 0, Kp % 32 == 0; dense_frag_index): no bounds
@@ -114,7 +115,7 @@ struct DenseEpi {
             it.x_off += (int64_t)it.row_base * c.ldx;
             it.M = c.row_offsets[g + 1] - it.row_base;
         }
-        it.x_off *= sizeof(T), it.w_off *= sizeof(T);
+        it.x_off *= sizeof(T), it.w_off *= 2;
         return it;
     }
     // acc[j]: columns n + 16 j .. + 3
@@ -281,10 +282,9 @@ struct DenseEpi {
 };
 
 // ---- weight images ----------------------------------------------------------------------------------------------------------------
-// src: bf16 [rows][cols] (checkpoint bytes) -> dst at dense_frag_index of (row0 + r, col0 + c), T = bf16 (copy) or float (exact widening)
-template<class T>
-__global__ void dense_place_kernel(T* __restrict__ dst, int steps, int row0, int col0, const __bf16* __restrict__ src, int rows, int cols,
-                                   int transpose, int half)
+// src: bf16 [rows][cols] (checkpoint bytes) -> dst at dense_frag_index of (row0 + r, col0 + c); half (1, 2): rows of a paired image, in the order of fp32 outputs or not
+__global__ void dense_place_kernel(__bf16* __restrict__ dst, int steps, int row0, int col0, const __bf16* __restrict__ src, int rows, int cols,
+                                   int transpose, int half, int f32)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < (size_t)rows * cols) {
@@ -292,9 +292,9 @@ __global__ void dense_place_kernel(T* __restrict__ dst, int steps, int row0, int
         int       n = row0 + (transpose ? c : r);  // transposed: the block's columns become output rows
         const int k = col0 + (transpose ? r : c);
         if (half) {
-            n = dense_pair_row(n, half - 1, sizeof(T) == 4);
+            n = dense_pair_row(n, half - 1, f32);
         }
-        dst[dense_frag_index<T>(n, k, steps)] = (T)(float)src[i];
+        dst[dense_frag_index(n, k, steps)] = src[i];
     }
 }
 
@@ -307,7 +307,7 @@ int dense_weight_alloc(DenseWeight& d, int K, int N, int dtype, hipStream_t st, 
     d.Np    = (N + 127) / 128 * 128;
     d.dtype = dtype;
     d.count = count;
-    d.bytes = (size_t)d.Kp * d.Np * count * (dtype == kDenseF32 ? 4 : 2);
+    d.bytes = (size_t)d.Kp * d.Np * count * 2;
     TM_HIP_CHECK(hipMalloc(&d.w, d.bytes));
     TM_HIP_CHECK(hipMemsetAsync(d.w, 0, d.bytes, st));
     return 0;
@@ -324,12 +324,7 @@ int dense_weight_place(DenseWeight& d, int row0, int col0, const void* src_bf16,
     if (n == 0) {
         return 0;
     }
-    if (d.dtype == kDenseF32) {
-        dense_place_kernel<float><<<(n + 255) / 256, 256, 0, st>>>((float*)d.w + at, d.Kp / 16, row0, col0, (const __bf16*)src_bf16, rows, cols, transpose, half);
-    }
-    else {
-        dense_place_kernel<__bf16><<<(n + 255) / 256, 256, 0, st>>>((__bf16*)d.w + at, d.Kp / 32, row0, col0, (const __bf16*)src_bf16, rows, cols, transpose, half);
-    }
+    dense_place_kernel<<<(n + 255) / 256, 256, 0, st>>>((__bf16*)d.w + at, d.Kp / 32, row0, col0, (const __bf16*)src_bf16, rows, cols, transpose, half, d.dtype == kDenseF32);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
 }
@@ -348,18 +343,17 @@ void dense_weight_free(DenseWeight& d)
 //     33, 23, 20 us; (2048, 2048) with 2600 rows: 50, 36, 35, 48 us; fp16 (5120, 5120) with 400 rows: -, 74, 44, 57, (4096, 4096) with 200: -, 69, 38, 20
 //   few rows of one item (few_rows_cost): what the workgroups of the fullest CU stream, at 32 - 33 GB/s of weights a CU with a line of x (from L2) at a fraction
 //     of the price of a line of weights; 6.1 TB/s for all of them; a workgroup's chain of steps; for slices the way through memory.  Of 184 sizes
-//     (K 768 ... 25600, N 768 ... 32000, 1 ... 64 rows, bf16 and fp32, 64 and 96 columns a workgroup, 1 ... 16 slices and the narrow kernel) what it takes is on
+//     (K 768 ... 25600, N 768 ... 32000, 1 ... 64 rows, 64 and 96 columns a workgroup, 1 ... 16 slices and the narrow kernel) what it takes is on
 //     average 0.8 % and at most 10 % slower than the best.  us, bf16: (4096, 21504) 32 rows, 64 columns 38.9 (two workgroups on some CUs), 96 columns 30.1; (25600,
 //     4096) 32 rows, one slice 95, four 36, eight 39; (4096, 6144) 32 rows, 96 columns four slices 14.8, 64 columns four 15.8, one 18.6; (2048, 2048) 8
-//     rows, narrow 5.1, four slices 6.3, one 7.9; (14336, 4096) 16 rows, narrow 27.3, four slices 21.6; fp32, 3 rows: (8448, 2048) narrow 19.9, eight slices
-//     15.3; (4096, 4096) narrow 13.8, four slices 16.2; 128 columns where nearly every CU gets one workgroup of them, of 64 two, and
+//     rows, narrow 5.1, four slices 6.3, one 7.9; (14336, 4096) 16 rows, narrow 27.3, four slices 21.6; 128 columns where nearly every CU gets one workgroup of them, of 64 two, and
 //     x is long: bf16 (4096, 27648) 32 rows 39.0 / 37.3, 64 rows 44.3 / 41.3, (4096, 32000) 64 rows 47.5 / 44.6; not (2048, 28160) 32 rows 22.0 / 22.4, (4096, 27648) 8 rows 36.7 / 36.6
 //   items with rows of their own: blocks of as many rows as an item has at most (the tokens of a routed mixture, not its rows in total).  Febivik width 2048, whole
 //     batches: 8 tokens 35.4 -> 35.0 ms, 16 tokens 32.5 -> 30.5 (48 rows, blocks of 64 before), 22 tokens 38.9 -> 37.5 (66 rows, tiles before), 32 the same
 //   items, pairs: as many slices of k as give every CU a workgroup, none of fewer than 16 steps; nine items of (2048, 2816): one 21, three 31; pairs, four rows,
 //     (2048, 11264): one 17, two 23
 // us; cw: column tiles a workgroup (0: narrow kernel), ss: steps of one of sp slices
-static double few_rows_cost(int steps, int cols, int rows, int elem, int cw, int sp, int ss)
+static double few_rows_cost(int steps, int cols, int rows, int cw, int sp, int ss)
 {
     const int    mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, wgs = cw ? (cols / 16 + cw - 1) / cw * sp : cols / 16;
     const double per_cu = wgs <= 1024 ? (wgs + 255) / 256 : wgs / 256.0;
@@ -367,19 +361,35 @@ static double few_rows_cost(int steps, int cols, int rows, int elem, int cw, int
     if (cw == 0) {
         return 2.4 + std::max(all, per_cu * steps * 64 * (16 + 0.82 * rows) / 33e3);
     }
-    const double chain = ss * (0.018 + 0.037 * mt * (elem == 4 ? 2.6 : 1.0)), mfma = elem == 4 ? per_cu * ss * cw * mt * 0.026 : 0.0;  // (fp32: the matrix unit too)
-    return 2.6 + std::max({all, per_cu * ss * 64 * (cw * 16 + 0.26 * rows) / 32e3, chain, mfma}) + (sp > 1 ? 2.4 + 0.66 * sp * rows * cols * 4e-6 : 0.0);
+    return 2.6 + std::max({all, per_cu * ss * 64 * (cw * 16 + 0.26 * rows) / 32e3, ss * (0.018 + 0.037 * mt)}) + (sp > 1 ? 2.4 + 0.66 * sp * rows * cols * 4e-6 : 0.0);
+}
+
+// The same for fp32 rows, whose lines are twice as many: blocks of 64 rows side by side up to 256, and (cw < 0) 64 x 64 tiles.  Of 486 sizes (K 64 ... 14336, N 256 ... 32000, 1 ...
+// 256 rows) what it takes is on average 1.6 % slower than the best, at most 45 % ((256, 24500) 129 rows).  us: (2048, 2048) 3 rows, narrow 5.3, four slices 7.0; (8448, 2048) 3
+// rows, narrow 14.9, six slices 12.5; (2048, 8448) 32 rows, 96 columns two slices 16.1, 64 columns one 18.3, narrow 28.9; (2048, 1024) 90 rows, eight slices 15.9, tiles 17.2; (2048,
+// 32000) 48 rows, slices 62, tiles 35 (up to 64 rows tiles are taken where the model sees 15 % in them)
+static double few_rows_cost_f32(int steps, int cols, int rows, int cw, int sp, int ss)
+{
+    const int    mt = rows <= 16 ? 1 : rows <= 32 ? 2 : 4, rb = (rows + 63) / 64, wgs = (cw < 0 ? (cols + 63) / 64 : cw ? (cols / 16 + cw - 1) / cw * sp : cols / 16) * rb;
+    const double per_cu = cw < 0 || wgs <= 1024 ? (wgs + 255) / 256 : wgs / 256.0, all = cols * 64e-6 * steps / 5.9, lines = per_cu * ss * 64e-3;
+    if (cw < 0) {
+        return std::max(per_cu * (0.143 * steps + 1.49), 0.168 * steps + 2.41);
+    }
+    if (cw == 0) {
+        return 2.95 + 0.124 * ((steps + 31) / 32) * mt + std::max(all, lines * (16 + 1.36 * std::min(rows, 64)) / 31.1);
+    }
+    return 2.19 + 0.07 * mt + std::max({all, lines * (cw * 16 + 1.48 * std::min(rows, 64)) / 35.5, ss * 0.18}) + (sp > 1 ? 3.62 + 0.378 * sp * rows * cols * 4e-6 : 0.0);
 }
 
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border,
-                       bool k_major, int item_rows, bool cut_ok)
+                       bool k_major, int item_rows, bool cut_ok, bool few_only)
 {
     struct Tile {
         int    rows, cols;
         double full16, alone16, full32, alone32, fixed;
     };
-    static const Tile kTiles[] = {{256, 256, 0.83, 0.83, 1e9, 1e9, 8.0}, {256, 128, 0.46, 0.55, 1.75, 1.75, 5.0}, {128, 128, 0.283, 0.30, 0.90, 0.95, 3.0},
-                                  {64, 64, 0.125, 0.15, 0.24, 0.32, 1.0}};
+    static const Tile kTiles[] = {{256, 256, 0.83, 0.83, 1e9, 1e9, 8.0}, {256, 128, 0.46, 0.55, 1e9, 1e9, 5.0}, {128, 128, 0.283, 0.30, 0.61, 0.73, 3.0},
+                                  {64, 64, 0.125, 0.15, 0.20, 0.30, 1.0}};
     StreamPlan        best{};
     double            cost = 1e30;
     // row tiles: items with rows of their own fill half of their last one on average, and each that has rows needs one
@@ -423,36 +433,40 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
         }
     }
     const int block = own_rows && item_rows > 0 ? std::min(rows, item_rows) : rows;  // rows that a workgroup may meet
-    if (own_rows ? block > 64 : rows > 256) {  // (an item's rows are one block of the skinny kernel)
+    if (own_rows ? block > 64 : rows > 256 || (elem == 4 && rows > 64 && items > 1)) {  // (an item's rows are one block of the skinny kernel)
         return best;
     }
     const int mt = block <= 16 ? 1 : block <= 32 ? 2 : 4, rb = (block + 16 * mt - 1) / (16 * mt);
     best.mt = mt, best.row_blocks = rb, best.cw = pairs ? 8 : 4, best.splits = 1, best.split_steps = (steps + 7) / 8 * 8;
-    if (items == 1 && !pairs && rows <= 64) {
+    if (items == 1 && !pairs && rows <= (elem == 4 && !own_rows ? 256 : 64)) {
+        auto few = [&](int cw, int sp, int ss) { return elem == 4 ? few_rows_cost_f32(steps, cols, rows, cw, sp, ss) : few_rows_cost(steps, cols, rows, cw, sp, ss); };
         // (the waves of a narrow workgroup read pieces of 4 KB that lie far apart in a k-major image: fp16 (2048, 16384) 8 rows, narrow 14.6, 64 columns 11.9,
         // (2048, 4096) 48 rows 10.2 and 9.4)
-        double least = k_major && cols > (rows > 32 ? 2048 : 8192) ? 1e30 : few_rows_cost(steps, cols, rows, elem, 0, 1, 0);
+        double least = k_major && cols > (rows > 32 ? 2048 : 8192) ? 1e30 : few(0, 1, steps);
         best.skinny = best.narrow = true;
         for (int cw : {4, 6, 8}) {
             const int groups = (cols / 16 + cw - 1) / cw;
             if (border % (16 * cw) || (cw == 8 && (elem == 4 || k_major || rows <= 16 || steps < 128 || groups < 192 || groups > 256))) {
                 continue;
             }
-            for (int sp = 1; sp <= 16 && (sp == 1 || steps / sp >= 16); ++sp) {
+            for (int sp = 1; sp <= 16 && (sp == 1 || steps / sp >= (elem == 4 ? 8 : 16)); ++sp) {
                 const int ss = ((steps + sp - 1) / sp + 7) / 8 * 8;
-                if ((steps + ss - 1) / ss != sp || (sp > 1 && ((size_t)sp * rows * cols * 4 > ws_bytes || groups > tickets))) {
+                if ((steps + ss - 1) / ss != sp || (sp > 1 && ((size_t)sp * rows * cols * 4 > ws_bytes || groups * rb > tickets))) {
                     continue;
                 }
-                const double c = few_rows_cost(steps, cols, rows, elem, cw, sp, ss) * (cw == 8 ? 0.95 : 1.0);
+                const double c = few(cw, sp, ss) * (cw == 8 ? 0.95 : 1.0);
                 if (c < least) {
                     least = c, best.narrow = false, best.cw = cw, best.splits = sp, best.split_steps = ss;
                 }
             }
         }
+        if (elem == 4 && !few_only && border % 64 == 0 && few(-1, 1, steps) < (rows <= 64 ? 0.85 : 1.0) * least) {
+            best.skinny = false, best.tile = 3;
+        }
         return best;
     }
     const int    wg_cols = pairs ? 128 : 64, groups = (cols + wg_cols - 1) / wg_cols * items * rb;
-    const double step = 64.0 * (wg_cols + 0.7 * std::min(block, 16 * mt)) / 25e3;
+    const double step = 64.0 * (wg_cols + (elem == 4 ? 1.4 : 0.7) * std::min(block, 16 * mt)) / 25e3;
     int          sp   = groups >= (pairs ? 80 : 200) ? 1 : (256 + groups - 1) / groups;  // about one workgroup a CU
     sp          = std::max(1, std::min({sp, steps / 16, 16}));
     for (int more = sp; sp > 1 && more < 2 * sp && more <= 16; ++more) {  // slices of equal length
@@ -549,6 +563,19 @@ static int launch_dense_tile(const StreamArgs& a, const DenseCall& call, int vec
     return 0;
 }
 
+template<int EPI, int BM, int BN, int KP>
+static int launch_dense_tile_split(const StreamArgs& a, const DenseCall& call, int vec, hipStream_t st)
+{
+    constexpr int lds = KP * stream_split_bufs(BM, KP) * (BM * 2 + BN) * 64;
+    const auto    k   = stream_tile_split_kernel<DenseEpi<float, EPI>, BM, BN, KP>;
+    if (const int rc = ensure_dynamic_lds((const void*)k, lds)) {
+        return rc;
+    }
+    k<<<stream_tile_grid(a, BM, BN, call), 256 * KP, lds, st>>>(a, DenseEpi<float, EPI>{call, vec});
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
+}
+
 template<class T, int EPI>
 static int launch_dense_tile256(const StreamArgs& a, const DenseCall& call, int vec, hipStream_t st)
 {
@@ -565,16 +592,25 @@ static int launch_dense_tile256(const StreamArgs& a, const DenseCall& call, int 
 template<class T>
 static int launch_dense_tiles(const StreamArgs& a, const DenseCall& call, int tile, int vec, hipStream_t st)
 {
-    const int epi = call.epi;
-#define TM_TILE(EPI_)                                                                    \
-    if constexpr (sizeof(T) == 2 && EPI_ != kDenseActTable) {                            \
-        if (tile == 0) {                                                                 \
-            return launch_dense_tile256<T, EPI_>(a, call, vec, st);                      \
-        }                                                                                \
-    }                                                                                    \
-    return tile <= 1 ? launch_dense_tile<T, EPI_, 256, 128, 2, 2>(a, call, vec, st) :    \
-           tile == 2 ? launch_dense_tile<T, EPI_, 128, 128, 2, 2>(a, call, vec, st) :    \
-                       launch_dense_tile<T, EPI_, 64, 64, 2, 2>(a, call, vec, st)
+    const int  epi   = call.epi;
+    const dim3 grid  = stream_tile_grid(a, 64, 64, call);
+    const bool alone = a.steps >= 32 && grid.x * grid.y <= 256;  // (fp32: four groups of waves a tile, see stream_tile_split_kernel; at 24 steps it is a tie)
+#define TM_TILE(EPI_)                                                                        \
+    if constexpr (sizeof(T) == 4) {                                                          \
+        return tile == 2 ? launch_dense_tile_split<EPI_, 128, 128, 1>(a, call, vec, st) :    \
+               alone     ? launch_dense_tile_split<EPI_, 64, 64, 4>(a, call, vec, st) :      \
+                           launch_dense_tile_split<EPI_, 64, 64, 1>(a, call, vec, st);       \
+    }                                                                                        \
+    else {                                                                                   \
+        if constexpr (EPI_ != kDenseActTable) {                                              \
+            if (tile == 0) {                                                                 \
+                return launch_dense_tile256<T, EPI_>(a, call, vec, st);                      \
+            }                                                                                \
+        }                                                                                    \
+        return tile <= 1 ? launch_dense_tile<T, EPI_, 256, 128, 2, 2>(a, call, vec, st) :    \
+               tile == 2 ? launch_dense_tile<T, EPI_, 128, 128, 2, 2>(a, call, vec, st) :    \
+                           launch_dense_tile<T, EPI_, 64, 64, 2, 2>(a, call, vec, st);       \
+    }
     TM_EPI_SWITCH(TM_TILE)
 #undef TM_TILE
     return 0;
@@ -586,7 +622,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
     const int  epi = call.epi, G = call.count;
     StreamArgs a{};
     a.x = (const char*)x, a.ldx = (int64_t)ldx * sizeof(T);
-    a.w = (const char*)d.w, a.steps = (int)(d.Kp * sizeof(T) / 64), a.tiles = d.Np / 16;
+    a.w = (const char*)d.w, a.steps = d.Kp / 32, a.tiles = d.Np / 16;
     a.w_tile = (int64_t)a.steps * 1024, a.w_quad = 4096;
     a.y = y, a.ldy = ldy, a.M = M, a.N = d.N;
     const bool f32_out = epi == kDenseResidAdd || epi == kDenseScaleF32 || epi == kDenseBiasF32 || epi == kDenseResidGate;
@@ -599,7 +635,7 @@ static int launch_dense_typed(const DenseWeight& d, const void* x, int ldx, void
         border = std::gcd(border, call.seg_n0[s]);
     }
     const StreamPlan p = stream_plan(a.steps, d.Np, M, G, call.row_offsets != nullptr, sizeof(T), epi == kDenseGatedAct && sizeof(T) == 2,
-                                     d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border, false, call.item_rows, true);
+                                     d.scratch ? d.scratch->bytes : 0, d.scratch ? d.scratch->count : 0, border, false, call.item_rows, true, call.kv.block_ptrs != nullptr);
     TM_REQUIRE(p.skinny || !call.kv.block_ptrs, "dense linear: cache columns belong to products of few rows");
     if (p.skinny) {
         a.split_steps = p.split_steps;

@@ -332,7 +332,7 @@ void stream_plan_report(int kind, int K, int N, int M, bool scratch, int* plan)
     const size_t     ws = scratch ? (kind == 2 ? ~(size_t)0 : kStreamWsBytes) : 0;
     const int        tickets = scratch ? (kind == 2 ? 1 << 30 : kStreamTickets) : 0;
     const StreamPlan p = kind == 2 ? stream_plan(K / 32, N, M, 1, false, 2, false, ws, tickets, 0, true, 0, true) :
-                                     stream_plan((K + 31) / 32 * (kind == 1 ? 2 : 1), (N + 127) / 128 * 128, M, std::max(items, 1), items > 0, kind == 1 ? 4 : 2, false, ws, tickets, 0, false,
+                                     stream_plan((K + 31) / 32, (N + 127) / 128 * 128, M, std::max(items, 1), items > 0, kind == 1 ? 4 : 2, false, ws, tickets, 0, false,
                                                  item_rows, true);
     const int out[5] = {p.skinny ? (p.narrow ? 1 : 2) : 3 + p.tile, p.skinny ? (p.narrow ? 1 : p.cw) : 0, p.skinny ? p.mt : 0, p.skinny ? p.splits : 1, p.skinny ? 0 : p.cut};
     std::copy(out, out + 5, plan);

@@ -1,10 +1,9 @@
 // Building blocks of the unquantised products y = x . W^T (gemm_dense.hip: bf16 and fp32 checkpoint weights; gemm_f16.hip: the fp16
 // linears of the Llama family), one set for the three number formats.
 //
-// Weight image: 16 output columns x 64 bytes of k are one contiguous KB in MFMA fragment order, lane l holds column l % 16 and the 16 bytes at
-// (l / 16) * 16 of that column's 64 -- eight k of a 16-bit format (v_mfma_f32_16x16x32), four of fp32 (four v_mfma_f32_16x16x4, which
-// multiply and add in full 32 bits).  A "step" below is such a 64-byte range of k.  Rows of x are read in the same 64 bytes a step, so
-// everything that moves data counts in bytes and is the same code for every format.
+// Weight image: 16 output columns x 32 k of a 16-bit format are one contiguous KB in MFMA fragment order, lane l holds column l % 16 and its eight k at
+// (l / 16) * 8 (v_mfma_f32_16x16x32).  A "step" below is such a range of 32 k: 64 bytes of a weight column, and 64 of a row of x in 16 bits, 128 in fp32.
+// fp32 products have bf16 weights (as every checkpoint of these models) and fp32 rows: a row's number is the sum of three bf16 numbers, exactly (StreamOp).
 //
 // The weight is the MFMA's A operand: a lane's four results are four CONSECUTIVE output columns of one row of x, so results leave in
 // 8- or 16-byte stores, and a gate / up pair of a feed-forward is in one lane.
@@ -32,18 +31,43 @@ struct StreamOp<half_t> {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(bit_cast<half8_t>(a), bit_cast<half8_t>(b), c, 0, 0, 0);
     }
 };
+// fp32 rows: 24 bits of significand are three times the eight of bf16, so x = high + middle + low exactly (each part the rest's leading bits, cut off; a part that
+// underflows is below 2^-126), and a product of two bf16 numbers is exact in fp32: three bf16 matrix instructions multiply as exactly as fp32 ones do, in 48
+// cycles instead of 256.  They cut the sum off where v_mfma_f32_16x16x4 rounds it, so sums of one sign would drift: every kSplitSteps steps begin at zero and are
+// added to the others in fp32, and few rows sum the low and middle parts apart from the high ones.  What remains of an infinity after its leading part is zero, not a NaN.
+struct SplitRow {
+    u32x4 part[3];  // low, middle, high
+};
+__device__ __forceinline__ SplitRow stream_split(u32x4 a, u32x4 b)
+{
+    SplitRow o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float r[2] = {bit_cast<float>(i < 2 ? a[2 * i] : b[2 * i - 4]), bit_cast<float>(i < 2 ? a[2 * i + 1] : b[2 * i - 3])};
+#pragma unroll
+        for (int p = 2; p >= 0; --p) {
+            o.part[p][i] = __builtin_amdgcn_perm(bit_cast<uint32_t>(r[1]), bit_cast<uint32_t>(r[0]), 0x07060302);  // both leading halves
+#pragma unroll
+            for (int e = 0; p > 0 && e < 2; ++e) {
+                const float rest = r[e] - bit_cast<float>(bit_cast<uint32_t>(r[e]) & 0xffff0000u);
+                r[e]             = p == 2 ? __builtin_amdgcn_fmed3f(rest, rest, 0.f) : rest;  // (the median with a NaN is the smallest of the others)
+            }
+        }
+    }
+    return o;
+}
 template<>
 struct StreamOp<float> {
     static __device__ __forceinline__ floatx4 mma(u32x4 a, u32x4 b, floatx4 c)
     {
-        const floatx4 fa = bit_cast<floatx4>(a), fb = bit_cast<floatx4>(b);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            c = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], c, 0, 0, 0);
-        }
-        return c;
+        return StreamOp<__bf16>::mma(a, b, c);
     }
 };
+template<class T>
+constexpr int kStreamParts = sizeof(T) == 4 ? 3 : 1;  // matrix instructions a fragment of x takes
+template<class T>
+constexpr int kStreamXStep = 32 * sizeof(T);          // bytes of a row of x in a step
+constexpr int kSplitSteps = 8;                        // most steps of fp32 rows that the matrix cores add up by themselves
 
 struct StreamArgs {
     const char* x;       // rows of ldx bytes, 16-byte aligned
@@ -95,7 +119,7 @@ __device__ __forceinline__ int64_t stream_weight_bytes(const StreamArgs& a, int 
 // slices in slice order (the sum never depends on the order of arrival; no workgroup waits for another).
 // Weights run one chunk of eight steps ahead of the MFMAs in a second register buffer; all loads of a stage are unconditional (clamped).  Loads return in
 // order, so a stage's x is asked for ahead of its weights: the wait for x then leaves the weights in flight (the other way round every stage drained the
-// queue: 8 rows fp16 of (2048, 16384) 14.6 us, now 11.9 = 5.6 TB/s; bf16 of (2048, 8448) 12.0, 9.9; 3 rows fp32 of (2048, 8448) 19.9, 16.5).
+// queue: 8 rows fp16 of (2048, 16384) 14.6 us, now 11.9 = 5.6 TB/s; bf16 of (2048, 8448) 12.0, 9.9).
 // 32 rows bf16, weights from HBM: (K, N) = (25600, 4096) 38 us = 5.5 TB/s, (4096, 21504) 30 us = 5.9 TB/s with 96 columns a workgroup, one for nearly every CU
 // (39 us with 64, of which some CUs get two; with every wave reading x for itself, no slices: 76 and 50).  The loop fetches without a branch: with one around the
 // loads, and 64 columns, the two took 52 and 42.  Its last two stages stand behind it and fetch nothing beyond the slice: 8 rows bf16 of (8448, 2048) then took
@@ -103,11 +127,13 @@ __device__ __forceinline__ int64_t stream_weight_bytes(const StreamArgs& a, int 
 template<class T, class Epi, int MT, int NT, int CW, int KP>
 __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a, Epi epi)
 {
-    constexpr int kThreads = CW * KP * 64, kChunk = 8;
-    constexpr int kXVecs  = KP * MT * kChunk * 64;                          // 16-byte pieces of one x stage
+    constexpr int kParts = kStreamParts<T>, kXS = kStreamXStep<T>;
+    constexpr int kThreads = CW * KP * 64, kChunk = kParts > 1 && MT == 4 ? 4 : 8;
+    constexpr int kXVecs  = KP * MT * kChunk * 64;                          // fragments' pieces of eight k of one x stage
     constexpr int kXPer   = (kXVecs + kThreads - 1) / kThreads;             // ... per thread (kXVecs is a multiple of kThreads or of 64)
+    constexpr int kRaw    = kXS / 64;                                       // 16-byte loads of a piece
     constexpr int kRed    = KP > 1 ? (KP - 1) * CW * MT * NT * 64 * 16 : 0;  // the other k-phases' sums
-    constexpr int kXBytes = 2 * kXVecs * 16;
+    constexpr int kStage  = kParts * kXVecs * 16, kXBytes = 2 * kStage;
     __shared__ __attribute__((aligned(16))) char smem[kXBytes > kRed ? kXBytes : kRed];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -128,7 +154,7 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
         wp[j] = w + (int64_t)min(tile0 + j, a.tiles - 1) * a.w_tile;
     }
     const int turn = stream_turn(tile0, a.steps);
-    u32x4     wa[kChunk][NT], wb[kChunk][NT], xr[kXPer];
+    u32x4     wa[kChunk][NT], wb[kChunk][NT], xr[kXPer][kRaw];
     auto  fetch = [&](u32x4(&buf)[kChunk][NT], int base) {
 #pragma unroll
         for (int kk = 0; kk < kChunk; ++kk) {
@@ -140,16 +166,19 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
         }
     };
     // x stage: [phase][row tile][pair of steps] blocks of 16 rows x 128 bytes, 16-byte piece c of row r at r * 128 + ((c ^ (r & 7)) * 16): a
-    // fragment read meets every bank once, a row's 128 bytes are one line of memory
+    // fragment read meets every bank once, a row's 128 bytes (256 in fp32) are whole lines of memory.  fp32 rows are split once, by who stores them: a stage for each part
     auto fetch_x = [&](int base) {
 #pragma unroll
         for (int i = 0; i < kXPer; ++i) {
             const int v = tid + i * kThreads;
             const int c = v & 7, r = (v >> 3) & 15, blk = v >> 7;
-            const int pair = blk & 3, rt = (blk >> 2) % MT, p = (blk >> 2) / MT;
+            const int pair = blk % (kChunk / 2), rt = blk / (kChunk / 2) % MT, p = blk / (kChunk / 2) / MT;
             const int row = min(rt * 16 + r, M - 1);
-            const int64_t col = min((int64_t)(base + p * kChunk + pair * 2) * 64 + c * 16, (int64_t)a.steps * 64 - 16);
-            xr[i] = *(const u32x4*)(x + row * a.ldx + col);
+            const int64_t col = min((int64_t)(base + p * kChunk + pair * 2) * kXS + c * 16 * kRaw, (int64_t)a.steps * kXS - 16 * kRaw);
+#pragma unroll
+            for (int h = 0; h < kRaw; ++h) {
+                xr[i][h] = *(const u32x4*)(x + row * a.ldx + col + 16 * h);
+            }
         }
     };
     auto stash_x = [&](int buf) {
@@ -157,8 +186,18 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
         for (int i = 0; i < kXPer; ++i) {
             const int v = tid + i * kThreads;
             if (kXVecs % kThreads == 0 || v < kXVecs) {
-                const int c = v & 7, r = (v >> 3) & 15, blk = v >> 7;
-                *(u32x4*)(smem + buf * kXVecs * 16 + blk * 2048 + r * 128 + ((c ^ (r & 7)) << 4)) = xr[i];
+                const int   c = v & 7, r = (v >> 3) & 15, blk = v >> 7;
+                char* const at = smem + buf * kStage + blk * 2048 + r * 128 + ((c ^ (r & 7)) << 4);
+                if constexpr (kParts > 1) {
+                    const SplitRow f = stream_split(xr[i][0], xr[i][1]);
+#pragma unroll
+                    for (int p = 0; p < kParts; ++p) {
+                        *(u32x4*)(at + p * kXVecs * 16) = f.part[p];
+                    }
+                }
+                else {
+                    *(u32x4*)at = xr[i][0];
+                }
             }
         }
     };
@@ -171,18 +210,33 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
         }
     }
     const int   fr = lane & 15, fc = lane >> 4;
-    const char* xf = smem + ph * (MT * 4 * 2048) + fr * 128;
+    const char* xf = smem + ph * (MT * (kChunk / 2) * 2048) + fr * 128;
+    floatx4     sum[2][MT][NT];  // (fp32: of the chunk, the low and middle parts' and the high parts')
     auto        one = [&](const u32x4(&buf)[kChunk][NT], int xbuf, int kk) {
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            const u32x4 b = *(const u32x4*)(xf + xbuf * kXVecs * 16 + (t * 4 + (kk >> 1)) * 2048 + ((((kk & 1) * 4 + fc) ^ (fr & 7)) << 4));
+        for (int p = 0; p < kParts; ++p) {
+            floatx4(&to)[MT][NT] = kParts > 1 ? sum[p / 2] : acc;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                acc[t][j] = StreamOp<T>::mma(buf[kk][j], b, acc[t][j]);
+            for (int t = 0; t < MT; ++t) {
+                const u32x4 b = *(const u32x4*)(xf + xbuf * kStage + p * kXVecs * 16 + (t * (kChunk / 2) + (kk >> 1)) * 2048 + ((((kk & 1) * 4 + fc) ^ (fr & 7)) << 4));
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    to[t][j] = StreamOp<T>::mma(buf[kk][j], b, to[t][j]);
+                }
             }
         }
     };
     auto compute = [&](const u32x4(&buf)[kChunk][NT], int xbuf, int base) {
+        static_assert(kParts == 1 || kChunk <= kSplitSteps, "sums of fp32 rows");
+        if constexpr (kParts > 1) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    sum[0][t][j] = sum[1][t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+        }
         if (base + kChunk <= s1) {
 #pragma unroll
             for (int kk = 0; kk < kChunk; ++kk) {
@@ -194,6 +248,15 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
             for (int kk = 0; kk < kChunk; ++kk) {
                 if (base + kk < s1) {
                     one(buf, xbuf, kk);
+                }
+            }
+        }
+        if constexpr (kParts > 1) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    acc[t][j] += sum[0][t][j] + sum[1][t][j];
                 }
             }
         }
@@ -329,8 +392,9 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
 template<class T, class Epi, int MT, int NT, int W>
 __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi epi)
 {
-    constexpr bool kAhead = MT == 1 || (MT == 2 && sizeof(T) == 2);
-    constexpr int  kChunk = MT * NT > 1 && kAhead ? 4 : 8 / NT;
+    constexpr int  kParts = kStreamParts<T>, kXS = kStreamXStep<T>, kRaw = kXS / 64;
+    constexpr bool kAhead = MT == 1 || (MT == 2 && kParts == 1);
+    constexpr int  kChunk = (MT * NT > 1 || kParts > 1) && kAhead ? 4 : 8 / NT;
     __shared__ __attribute__((aligned(16))) floatx4 red[W][MT * NT][64];
     const int  lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int  mb   = blockIdx.y % a.row_blocks * (MT * 16), tile0 = blockIdx.x * NT;
@@ -344,7 +408,7 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
     const char* wp[NT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-        xp[t] = a.x + item.x_off + (int64_t)(mb + min(t * 16 + fr, M - 1)) * a.ldx + fc * 16;
+        xp[t] = a.x + item.x_off + (int64_t)(mb + min(t * 16 + fr, M - 1)) * a.ldx + fc * 16 * kRaw;
     }
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
@@ -359,19 +423,31 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
         }
     }
     // Up to 16 rows, and up to 32 of a 16-bit format, x of a chunk leaves with its weights, ahead of them: loads return in order, and a load of x where it is used would
-    // wait for the next chunk's weights (fp16, 8 rows: (2048, 4096) 5.9 -> 5.4 us, (2048, 2048) 5.1 -> 4.8; fp32, 3 rows, (2048, 2048) 8.5 -> 8.0; bf16, 17
+    // wait for the next chunk's weights (fp16, 8 rows: (2048, 4096) 5.9 -> 5.4 us, (2048, 2048) 5.1 -> 4.8; bf16, 17
     // rows, (4096, 4096) 11.9 -> 10.8).  More rows take more registers for it than they leave for weights: x there | where it is used, 64 rows: bf16 (2048, 2048)
-    // 11.8 | 11.4 us, fp32 (8448, 2048) 80.5 | 71.9, (2048, 2048) 23.0 | 21.0; fp32, 32 rows: 13.8 | 13.0
+    // 11.8 | 11.4 us
     const int turn = stream_turn(tile0, a.steps);
-    u32x4     wa[kChunk][NT], wb[kChunk][NT], xa[kChunk][MT], xb[kChunk][MT];
-    auto  fetch = [&](u32x4(&buf)[kChunk][NT], u32x4(&xbuf)[kChunk][MT], int base) {
+    struct Raw {
+        u32x4 h[kRaw];
+    };
+    auto load_x = [&](int t, int s) {
+        Raw r;
+#pragma unroll
+        for (int h = 0; h < kRaw; ++h) {
+            r.h[h] = *(const u32x4*)(xp[t] + (int64_t)s * kXS + 16 * h);
+        }
+        return r;
+    };
+    u32x4     wa[kChunk][NT], wb[kChunk][NT];
+    Raw       xa[kChunk][MT], xb[kChunk][MT];
+    auto  fetch = [&](u32x4(&buf)[kChunk][NT], Raw(&xbuf)[kChunk][MT], int base) {
         if constexpr (kAhead) {
 #pragma unroll
             for (int kk = 0; kk < kChunk; ++kk) {
                 const int s = min(base + kk, a.steps - 1);
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
-                    xbuf[kk][t] = *(const u32x4*)(xp[t] + (int64_t)s * 64);
+                    xbuf[kk][t] = load_x(t, s);
                 }
             }
             asm volatile("" ::: "memory");
@@ -392,23 +468,54 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
             asm volatile("" ::: "memory");
         }
     };
-    auto compute = [&](const u32x4(&buf)[kChunk][NT], const u32x4(&xbuf)[kChunk][MT], int base) {
+    floatx4 sum[2][MT][NT];  // (fp32: of the chunk, the low and middle parts' and the high parts')
+    auto    compute = [&](const u32x4(&buf)[kChunk][NT], const Raw(&xbuf)[kChunk][MT], int base) {
+        static_assert(kParts == 1 || kChunk <= kSplitSteps, "sums of fp32 rows");
+        if constexpr (kParts > 1) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    sum[0][t][j] = sum[1][t][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+        }
 #pragma unroll
         for (int kk = 0; kk < kChunk; ++kk) {
             if (base + kk < a.steps) {
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
-                    u32x4 b;
+                    Raw b;
                     if constexpr (kAhead) {
                         b = xbuf[kk][t];
                     }
                     else {
-                        b = *(const u32x4*)(xp[t] + (int64_t)(base + kk) * 64);
+                        b = load_x(t, base + kk);
+                    }
+                    SplitRow f;
+                    if constexpr (kParts > 1) {
+                        f = stream_split(b.h[0], b.h[1]);
+                    }
+                    else {
+                        f.part[0] = b.h[0];
                     }
 #pragma unroll
-                    for (int j = 0; j < NT; ++j) {
-                        acc[t][j] = StreamOp<T>::mma(buf[kk][j], b, acc[t][j]);
+                    for (int p = 0; p < kParts; ++p) {
+                        floatx4(&to)[MT][NT] = kParts > 1 ? sum[p / 2] : acc;
+#pragma unroll
+                        for (int j = 0; j < NT; ++j) {
+                            to[t][j] = StreamOp<T>::mma(buf[kk][j], f.part[p], to[t][j]);
+                        }
                     }
+                }
+            }
+        }
+        if constexpr (kParts > 1) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    acc[t][j] += sum[0][t][j] + sum[1][t][j];
                 }
             }
         }
@@ -536,6 +643,11 @@ constexpr int stream_tile_bufs(int bm, int bn)
     return bm == 64 && bn == 64 ? 6 : bm == 128 && bn == 128 || bm == 256 && bn == 256 ? 4 : 3;
 }
 
+constexpr int stream_split_bufs(int bm, int kp)  // ... of a group of waves of a tile whose rows are fp32
+{
+    return bm == 64 && kp == 1 ? 4 : 3;
+}
+
 template<class T, class Epi, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_kernel(StreamArgs a, Epi epi)
 {
@@ -638,7 +750,7 @@ __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_k
         }
 #pragma unroll
         for (int g = 0; g < MI + NI; ++g) {  // the next step's fragment reads go between the MFMAs
-            __builtin_amdgcn_sched_group_barrier(0x008, MI * NI / (MI + NI) * (sizeof(T) == 4 ? 4 : 1), 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, MI * NI / (MI + NI), 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
         buf = nxt;
@@ -655,6 +767,181 @@ __global__ __launch_bounds__(256, BM* BN > 256 * 128 ? 1 : 2) void stream_tile_k
         const int m = m0 + wm * (BM / WM) + i * 16 + fr;
         if (m < item.M) {
             epi.template rows<NI>(a, item, m, n0 + wn * NI * 16 + fc * 4, acc[i]);
+        }
+    }
+}
+
+// ---- many rows in fp32: tiles whose rows are split on the way to the matrix cores ---------------------------------------------------------
+// As above with rows of 128 bytes a step in LDS, piece c of row r at c ^ ((r >> 1) & 7); the waves share out the rows and each has all columns of the tile, since a
+// fragment of x takes 52 vector instructions to split and 48 cycles of matrix work for every 16 columns.  us, fp32 weights and matrix instructions before / now:
+// (2048, 8448) 450 rows 153 / 69, 6000 rows 1506 / 524 (128 x 128 tiles, 1.2 PFLOP/s of bf16 products); (2048, 2048) 450 rows 38 / 24: one tile a CU, whose 12 KB a step
+// come at 36 GB/s, what a CU's lines in flight give over the way to memory.  Relative error against 64 bits (2-norm), before / now: normal rows, K 2048 8.1e-7 / 1.7e-7;
+// sums of one sign 6.3e-7 / 6.3e-8 (in one run of all steps 9.8e-7: see kSplitSteps)
+// KP groups of four waves share out k, each with stages of its own, and meet in LDS in their order: where every tile has a CU to itself, four groups have more on their way
+// (one / four, us: (2048, 2048) 200 rows 21.9 / 17.8, 450 rows 23.3 / 21.8; (8448, 2048) 300 rows 81 / 59; (768, 2048) 200 rows 10.4 / 10.6).
+template<class Epi, int BM, int BN, int KP>
+__global__ __launch_bounds__(256 * KP, KP == 1 ? 2 : 4) void stream_tile_split_kernel(StreamArgs a, Epi epi)
+{
+    constexpr int MI = BM / 64, NI = BN / 16;
+    constexpr int kXB = BM * 128, kWB = BN * 64, kStage = kXB + kWB, kBufs = stream_split_bufs(BM, KP);
+    constexpr int kXP = BM / 32, kWP = BN / 64;  // DMA pieces of one KB per wave and stage
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, ph = __builtin_amdgcn_readfirstlane(tid >> 8);
+    const StreamTile t = stream_tile_of<BM, BN, 8>(a, epi.row_offsets(), epi.items());
+    if (t.item < 0) {
+        return;
+    }
+    const int  m0 = t.tm * BM, n0 = a.col0 + t.tn * BN;
+    const auto item = epi.item(t.item, a.M, n0);
+    const int  Mloc = min(item.M - m0, BM);
+    if (Mloc <= 0) {  // an item with fewer rows than the launch's largest
+        return;
+    }
+    const auto rs_x = __builtin_amdgcn_make_buffer_rsrc((void*)(a.x + item.x_off + m0 * a.ldx), 0, (int)((Mloc - 1) * a.ldx + (int64_t)a.steps * 128), 0x00020000);
+    const int64_t w_left = stream_weight_bytes(a, n0 >> 4);
+    const auto rs_w = __builtin_amdgcn_make_buffer_rsrc((void*)(a.w + item.w_off + (int64_t)(n0 >> 4) * a.w_tile), 0, (int)min(w_left, (int64_t)0xffffffff), 0x00020000);
+    char* const    stages = smem + ph * (kBufs * kStage);
+    const unsigned lds0   = __builtin_amdgcn_readfirstlane((unsigned)(size_t)stages);
+    int            xoff[kXP], woff[kWP];
+#pragma unroll
+    for (int r = 0; r < kXP; ++r) {
+        const int row = 8 * (kXP * wave + r) + (lane >> 3);
+        xoff[r]       = (int)(min(row, Mloc - 1) * a.ldx) + ((lane & 7) ^ ((row >> 1) & 7)) * 16;
+    }
+#pragma unroll
+    for (int r = 0; r < kWP; ++r) {
+        woff[r] = (int)(min(kWP * wave + r, a.tiles - 1 - (n0 >> 4)) * a.w_tile) + lane * 16;
+    }
+    const int turn = stream_turn(n0 >> 4, a.steps);
+    auto      dma  = [&](int s, int buf) {
+        const int      ws  = (int)stream_step_at<Epi>(a, s, turn);
+        const unsigned dst = lds0 + buf * kStage;
+#pragma unroll
+        for (int r = 0; r < kXP; ++r) {
+            stream_dma16(rs_x, xoff[r], s * 128, dst + (kXP * wave + r) * 1024);
+        }
+#pragma unroll
+        for (int r = 0; r < kWP; ++r) {
+            stream_dma16(rs_w, woff[r], ws, dst + kXB + (kWP * wave + r) * 1024);
+        }
+    };
+    floatx4 acc[MI][NI], sum[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    const int fr = lane & 15, fc = lane >> 4;
+    const int xrow = (wave * (BM / 4) + fr) * 128, sw = (fr >> 1) & 7;
+    const int wf = kXB + lane * 16;
+    // a group's steps begin at s0; all groups walk as many as the first has, for the barriers, the last ones some without products
+    const int run = ((a.steps + KP - 1) / KP + kSplitSteps - 1) / kSplitSteps * kSplitSteps, s0 = min(ph * run, a.steps - 1);
+    const int steps = min(a.steps - ph * run, run), walk = min(run, a.steps);
+    u32x4     fx[2][MI][2], fw[2][NI];
+    auto      read = [&](int q, int buf) {
+        const char* st = stages + buf * kStage;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                fx[q][i][h] = *(const u32x4*)(st + xrow + i * 2048 + (((2 * fc + h) ^ sw) << 4));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+            fw[q][j] = *(const u32x4*)(st + wf + j * 1024);
+        }
+    };
+    constexpr int kPieces = kXP + kWP;
+#pragma unroll
+    for (int b = 0; b < kBufs; ++b) {
+        dma(s0 + max(min(b, steps - 1), 0), b);
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kBufs - 1) * kPieces) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0);
+    int  buf  = 0;  // stage of step s
+    auto step = [&](auto Nth, int s) {  // step N of a run of kSplitSteps
+        constexpr int n = decltype(Nth)::value, q = n & 1;
+        const int     nxt = buf == kBufs - 1 ? 0 : buf + 1;
+        // this wave's fragments of step s are in registers and its pieces of stage s + 1 have landed; then everybody's
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((kBufs - 2) * kPieces) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        dma(s0 + max(min(s + kBufs, steps - 1), 0), buf);
+        read(q ^ 1, nxt);
+        buf = nxt;
+        if (KP > 1 && s >= steps) {
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            const SplitRow f = stream_split(fx[q][i][0], fx[q][i][1]);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    sum[i][j] = StreamOp<float>::mma(fw[q][j], f.part[p], n == 0 && p == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : sum[i][j]);
+                }
+            }
+        }
+    };
+    for (int s = 0; s < walk; s += kSplitSteps) {
+        static_assert(kSplitSteps == 8, "the steps below");
+        step(std::integral_constant<int, 0>{}, s);
+#define TM_STEP(N)                                           \
+    if (s + N < walk) {                                       \
+        step(std::integral_constant<int, N>{}, s + N);       \
+    }
+        TM_STEP(1) TM_STEP(2) TM_STEP(3) TM_STEP(4) TM_STEP(5) TM_STEP(6) TM_STEP(7)
+#undef TM_STEP
+        if (KP == 1 || s < steps) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    acc[i][j] += sum[i][j];
+                }
+            }
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the DMA writes this workgroup's LDS)
+    if constexpr (KP > 1) {
+        static_assert(kBufs * kStage * KP >= (KP - 1) * BM * BN * 4, "the groups' sums lie where their stages were");
+        __syncthreads();
+        floatx4* const red = (floatx4*)smem;
+        if (ph > 0) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    red[(((ph - 1) * 4 + wave) * MI * NI + i * NI + j) * 64 + lane] = acc[i][j];
+                }
+            }
+        }
+        __syncthreads();
+        if (ph > 0) {
+            return;
+        }
+#pragma unroll
+        for (int p = 0; p < KP - 1; ++p) {  // fixed order
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+#pragma unroll
+                for (int j = 0; j < NI; ++j) {
+                    acc[i][j] += red[((p * 4 + wave) * MI * NI + i * NI + j) * 64 + lane];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int m = m0 + wave * (BM / 4) + i * 16 + fr;
+        if (m < item.M) {
+            epi.template rows<NI>(a, item, m, n0 + fc * 4, acc[i]);
         }
     }
 }
@@ -838,10 +1125,9 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
 // its MFMA fragment (16 bytes each: lane = piece * 16 + n % 16), blocks of one 16-row tile consecutive along k -- a wave's fragment
 // load is one contiguous KB and a workgroup streams whole contiguous runs of HBM instead of 64-byte pieces of 16 rows
 // (from stream_turn's step on)
-template<class T>
 __host__ __device__ inline size_t dense_frag_index(int n, int k, int steps)
 {
-    constexpr int E = 16 / sizeof(T), S = 4 * E;  // elements of a 16-byte piece, of a step
+    constexpr int E = 8, S = 4 * E;  // elements of a 16-byte piece, of a step
     const int     at = k / S + stream_turn(n >> 4, steps);
     return (((size_t)(n >> 4) * steps + (at < steps ? at : at - steps)) * 64 + (k % S) / E * 16 + (n & 15)) * E + k % E;
 }
@@ -868,9 +1154,9 @@ struct StreamPlan {
 // steps of k, image columns, rows, items (own_rows: each with rows of its own, `rows` in total), bytes of an element; pairs: a wave needs two
 // column tiles; ws_bytes / tickets: what slices of k may use (0: no slices); border: x is read elsewhere from multiples of this many columns on (a
 // multiple of 128; 0: nowhere); k_major: the image holds four steps of every column tile before the next four; item_rows: own_rows, the most an item has (0: rows);
-// cut_ok: the columns may go to two launches
+// cut_ok: the columns may go to two launches; few_only: up to 64 rows no tiles (their epilogues store no cache columns)
 StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, int elem, bool pairs, size_t ws_bytes, int tickets, int border = 0,
-                       bool k_major = false, int item_rows = 0, bool cut_ok = false);
+                       bool k_major = false, int item_rows = 0, bool cut_ok = false, bool few_only = false);
 constexpr size_t kStreamWsBytes = (size_t)16 << 20;  // scratch and arrival counters that serve every plan
 constexpr int    kStreamTickets = 4096;
 

@@ -437,7 +437,7 @@ __global__ __launch_bounds__(256) void layernorm_f32_reg_kernel(T* __restrict__ 
             xv[q] = *(const FV*)(xs + (size_t)m * H + i);
         }
         if constexpr (RE > 0) {
-            const T* at = (const T*)rt.w + dense_frag_index<T>(0, i, rt.steps);  // (experts of a tile lie side by side)
+            const T* at = (const T*)rt.w + dense_frag_index(0, i, rt.steps);  // (experts of a tile lie side by side)
 #pragma unroll
             for (int e = 0; e < RE; ++e) {
                 rw[q][e] = *(const TV*)(at + e * 8);
