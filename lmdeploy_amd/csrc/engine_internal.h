@@ -184,6 +184,15 @@ struct LayeredModel {
     float*               d_logits_f32 = nullptr;  // [max_logit_rows][vocab]
     int *                d_row_seq = nullptr, *d_row_pos = nullptr, *d_iota = nullptr, *d_want = nullptr, *d_seq_slot = nullptr;
     int *                d_step_ids = nullptr, *d_step_cu_q = nullptr, *d_step_k_len = nullptr;
+    // a recorded step's description, [cu_q][k_len][slots][ids] in one allocation, and where the host writes it (pinned)
+    int *                d_step = nullptr, *h_step = nullptr;
+    // recorded steps of one token a session, as graphs: one for a number of rows (and whether their logits are wanted), from its second step on
+    struct RecordedStep {
+        int            rows = 0, want = 0, seen = 0;
+        hipGraphExec_t graph = nullptr;
+    };
+    std::vector<RecordedStep> recorded;
+    const RecordedStep*       recording = nullptr;  // what recorded_step() captures
     float*               d_attn_ws = nullptr;
     unsigned*            d_attn_tickets = nullptr;  // [max rows][max heads], zero between launches
     int                  n_attn_tickets = 0;

@@ -1,0 +1,67 @@
+"""GPU tests of recorded steps (step_tokens) of one token a session, which run as graphs from the second step of as many rows on: the same bits as launch by launch, over prompts,
+other numbers of rows, sessions that close and open, and steps that want other rows in between; contexts grow over the ends of cache blocks."""
+import numpy as np
+import pytest
+
+from tests.gpu_helpers import release_all
+from tests.test_gpu_febivik import engine as febivik_engine
+from tests.test_gpu_febivik import full_model as febivik_model
+from tests.test_gpu_febivik import model_folder as febivik_folder
+from tests.test_gpu_sanozen import engine as sanozen_engine
+from tests.test_gpu_sanozen import full_model as sanozen_model
+from tests.test_gpu_sanozen import model_folder as sanozen_folder
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _release():
+    yield
+    release_all()
+
+
+def _walk(eng, vocab):
+    """every logits row that a fixed course of sessions gives"""
+    rng, out = np.random.default_rng(3), []
+
+    def step(entries):
+        out.append(eng.step_tokens(entries).copy())
+
+    def one(sessions, want=True):
+        step([(s, rng.integers(0, vocab, 1), [0] if want else []) for s in sessions])
+    a, b, c = (eng.open_session() for _ in range(3))
+    step([(a, rng.integers(0, vocab, 60), [59]), (b, rng.integers(0, vocab, 61), [3, 60]), (c, rng.integers(0, vocab, 7), [])])
+    for i in range(8):
+        one((a, b, c))
+        if i == 4:
+            d = eng.open_session()
+            step([(d, rng.integers(0, vocab, 30), [29]), (a, rng.integers(0, vocab, 1), [0])])      # a portion beside a decoded token
+    for i in range(5):
+        one((b, d) if i % 2 else (d, a, b, c), i != 2)
+    step([(a, rng.integers(0, vocab, 1), [0]), (c, rng.integers(0, vocab, 1), [])])                     # one of two rows wanted
+    eng.close_session(b)
+    e = eng.open_session()
+    step([(e, rng.integers(0, vocab, 5), [4])])
+    for _ in range(4):
+        one((e, c, a))
+        one((a, ))
+    for s in (a, c, d, e):
+        eng.close_session(s)
+    return out
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('family', ['sanozen', 'febivik'])
+def test_graphs_give_the_bits_of_launches(tmp_path, cuda, family, dtype):
+    cfg = sanozen_model() if family == 'sanozen' else febivik_model(dtype)
+    folder, _ = (sanozen_folder if family == 'sanozen' else febivik_folder)(tmp_path, cfg, 2)
+    build = sanozen_engine if family == 'sanozen' else febivik_engine
+    rows = []
+    for graphs in (0, 1):
+        eng = build(folder, dtype, use_graph=graphs)
+        rows.append(_walk(eng, cfg['vocab']))
+        rows.append(_walk(eng, cfg['vocab']))      # with the graphs of the first course
+        eng.close()
+    for other in rows[1:]:
+        assert len(other) == len(rows[0]) and all(np.array_equal(x.view(np.uint32), y.view(np.uint32)) for x, y in zip(rows[0], other))
+    assert all(np.isfinite(x).all() for x in rows[0]) and not np.array_equal(rows[0][1], rows[0][2])
