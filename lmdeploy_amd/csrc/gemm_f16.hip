@@ -46,8 +46,8 @@ struct F16Epi {
             }
             const floatx4 v = acc[j];
             if (gated) {
-                const float s0 = v[0] / (1.0f + __builtin_expf(-v[0]));
-                const float s1 = v[2] / (1.0f + __builtin_expf(-v[2]));
+                const float s0 = silu_f32(v[0]);
+                const float s1 = silu_f32(v[2]);
                 half_t*     y  = (half_t*)a.y + (size_t)m * a.ldy + (c >> 1);
                 if (vec) {
                     *(half2_t*)y = half2_t{(half_t)(s0 * v[1]), (half_t)(s1 * v[3])};

@@ -405,8 +405,8 @@ __global__ __launch_bounds__(CG* WK * 64) void gemm_fp8_kernel(Fp8Params p)
                 *(floatx4*)(p.partial + ((size_t)blockIdx.y * p.M + mg) * p.N + n) = a;
             }
             else if (p.epilogue == 1) {
-                const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-                const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+                const float s0 = silu_f32(a[0]);
+                const float s1 = silu_f32(a[2]);
                 half2_t     o  = {(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
                 *(half2_t*)(p.y + mg * p.ldy + (n >> 1)) = o;
             }
@@ -598,8 +598,8 @@ __global__ __launch_bounds__(512) void gemm_fp8_tile256_kernel(Fp8Params p)
                 const floatx4 a   = acc[u][h][t];
                 char* const   row = out + (t * 16 + c) * 288;
                 if (gated) {
-                    const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-                    const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+                    const float s0 = silu_f32(a[0]);
+                    const float s1 = silu_f32(a[2]);
                     *(half2_t*)(row + u * 32 + h * 16 + q * 4) = half2_t{(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
                 }
                 else {

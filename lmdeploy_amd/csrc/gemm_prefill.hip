@@ -287,10 +287,8 @@ __global__ __launch_bounds__(256, 1) void gemm_pre256_kernel(Dec32Params p)
             uint32_t o[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const floatx4 a  = acc[i][j];
-                const float   s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-                const float   s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
-                o[j]             = bit_cast<uint32_t>(half2_t{(half_t)(s0 * a[1]), (half_t)(s1 * a[3])});
+                const floatx4 a = acc[i][j];
+                o[j]            = bit_cast<uint32_t>(half2_t{(half_t)(silu_f32(a[0]) * a[1]), (half_t)(silu_f32(a[2]) * a[3])});
             }
             if (wide) {
                 pre256_transpose(o);

@@ -244,8 +244,8 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
             store_wt((floatx4*)(p.partial + ((size_t)blockIdx.y * M + fr) * p.N + c), a);
         }
         else if (p.epilogue == 1) {
-            const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-            const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+            const float s0 = silu_f32(a[0]);
+            const float s1 = silu_f32(a[2]);
             *(half2_t*)(p.y + (size_t)fr * p.ldy + (c >> 1)) = half2_t{(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
         }
         else {

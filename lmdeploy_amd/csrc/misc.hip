@@ -372,7 +372,7 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(half_t* __restrict__ out,
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const float gf = (float)g[e];
-        o[e]           = (half_t)((gf / (1.0f + __builtin_expf(-gf))) * (float)u[e]);
+        o[e]           = (half_t)(silu_f32(gf) * (float)u[e]);
     }
     *(half8_t*)(out + (size_t)m * inter + c) = o;
 }

@@ -433,7 +433,7 @@ __device__ __forceinline__ float act_apply(int act, float z)
         return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
     }
     if (act == kActSilu) {
-        return z / (1.f + expf(-z));
+        return silu_f32(z);
     }
     const float r = fmaxf(z, 0.f);
     return r * r;
