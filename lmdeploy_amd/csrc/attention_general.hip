@@ -667,15 +667,12 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(GeneralAttnParams p, in
             inv = 1.f / l[rt];
         }
         inv *= ga_out_gate(p, row_base + row0 + rt * 16 + lr, h);
-        // lane holds O[row lr][channel t * 16 + lg * 4 + r]
+        // lane holds O[row lr][channels t * 16 + lg * 4 .. + 3] (V is a multiple of 8)
 #pragma unroll
         for (int t = 0; t < VT; ++t) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int v = t * 16 + lg * 4 + r;
-                if (v < V) {
-                    ga_store<__bf16>(p, row_base + row0 + rt * 16 + lr, h, v, o[rt][t][r] * inv);
-                }
+            const int v = t * 16 + lg * 4;
+            if (v < V) {
+                ga_store4<__bf16>(p, row_base + row0 + rt * 16 + lr, h, v, o[rt][t] * inv);
             }
         }
     }
@@ -837,9 +834,11 @@ bool general_attention_tiles_ok(const GeneralAttnParams& p)
 // arithmetic (per score three transcendentals with a cap, one without, at quarter rate) beside about as many cycles of MFMA, so what matters is that two waves
 // share a SIMD and run out of phase: under 256 registers a wave, 64 KB of LDS for 128 / 128 heads (two workgroups of four waves), one workgroup of eight
 // waves for key size 256, one row tile a wave there (two spill: 640 us where one takes 271).
-// MI355X, 4 x 2048 rows: 32 / 8 heads of 128 / 128 273 us = 0.50 PFLOP/s (8000 rows: 0.72; attn_tiles_kernel, which reads fragments straight from the
-// cache with one wave a SIMD: 1126 us), 16 / 1 heads of 256 / 192 271 us (1055), 16 / 8 heads of 64 / 128 with a cap 139 us (465), 40 x 100 rows of 32 / 8
-// heads of 128 / 128 61 us (136).
+// A score's form is a template parameter: a plain score's scale and a cap's outer product go into the exponent (three and seven vector instructions a score beside the
+// transcendentals, five and nine before).  A lane's four channels of an output row leave in one store: one by one they were 64 stores of two bytes a lane, as long as
+// the products of four blocks.
+// MI355X, us, before both / now: 4 x 2048 rows, 32 / 8 heads of 128 / 128 264 / 204 = 0.67 PFLOP/s (with a cap 298 / 246; 8000 rows 717 / 606 = 0.87), 16 / 1 heads of 256 / 192 236 / 194;
+// 2 x 3000 rows, 16 / 8 heads of 64 / 128 with a cap 155 / 129; 40 x 100 rows, 16 / 1 heads of 256 / 192 58 / 38.
 // Serves the sizes of staged_shape(); attn_tiles_kernel serves the rest (sizes that do not fill the pieces of a DMA or the 16-channel tiles).
 typedef unsigned ga_u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float ga_max_groups(float v)  // over the four lane groups (lanes l ^ 16, l ^ 32)
@@ -859,7 +858,10 @@ __device__ __forceinline__ int ga_key_swizzle(int row)
     return DS == 2 ? (row & 2) | ((row & 8) >> 1) : (row & 8) | ((row & 3) << 1);
 }
 
-template<int DS, int VT, int RT, bool MASK>
+// What a launch does with its scores, where the compiler knows it: nothing (the scale goes into the exponent), a soft cap, or any of the modifiers
+enum { kScorePlain = 0, kScoreCap = 1, kScoreAny = 2 };
+
+template<int DS, int VT, int RT, bool MASK, int MOD>
 __device__ __forceinline__ void ga_staged_step(const bf16x8 (&qf)[RT][DS], const char* __restrict__ kt_lds, const char* __restrict__ vt_lds, const int (&limit)[RT],
                                                const int (&lower)[RT], int keep_rel, const float (&qscale)[RT], float cap, float inv_cap, bool bias, float r1,
                                                float r2, float (&m)[RT], float (&l)[RT], floatx4 (&o)[RT][VT], const float* __restrict__ tab, int tab_len)
@@ -888,7 +890,10 @@ __device__ __forceinline__ void ga_staged_step(const bf16x8 (&qf)[RT][DS], const
     const float cap2 = cap * kLog2e;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
-        const float k1 = cap > 0.f ? qscale[rt] * inv_cap * (2.f * kLog2e) : qscale[rt] * kLog2e;
+        // the exponent of a weight is base * (what each() leaves) + shift - maximum
+        const bool  capped = MOD == kScoreCap || (MOD == kScoreAny && cap > 0.f);
+        const float k1     = capped ? qscale[rt] * inv_cap * (2.f * kLog2e) : qscale[rt] * kLog2e;
+        const float base = MOD == kScorePlain ? k1 : MOD == kScoreCap ? -2.f * cap2 : 1.f, shift = MOD == kScoreCap ? cap2 : 0.f;
         // (one loop per modifier, the branch outside: a branch per score would leave every score in a block of its own)
         auto each = [&](auto f) {
 #pragma unroll
@@ -899,34 +904,43 @@ __device__ __forceinline__ void ga_staged_step(const bf16x8 (&qf)[RT][DS], const
                 }
             }
         };
-        if (cap > 0.f) {
-            each([&](float v, int) { return fmaf(__builtin_amdgcn_rcpf(fast_exp2(v * k1) + 1.f), -2.f * cap2, cap2); });
+        if constexpr (MOD == kScoreCap) {  // cap tanh(x) = cap - 2 cap w with w = 1 / (e^2x + 1): the largest score has the smallest w
+            each([&](float v, int) { return __builtin_amdgcn_rcpf(fast_exp2(v * k1) + 1.f); });
         }
-        else {
-            each([&](float v, int) { return v * k1; });
+        if constexpr (MOD == kScoreAny) {
+            if (cap > 0.f) {
+                each([&](float v, int) { return fmaf(__builtin_amdgcn_rcpf(fast_exp2(v * k1) + 1.f), -2.f * cap2, cap2); });
+            }
+            else {
+                each([&](float v, int) { return v * k1; });
+            }
+            if (bias) {  // (a key ahead of the row gives the logarithm of a number that may be negative: the mask below discards it)
+                each([&](float v, int key) { return fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, (float)(limit[rt] - key), 1.f)), v); });
+            }
+            if (tab) {  // (a key ahead of the row reads entry 0 and is masked below)
+                each([&](float v, int key) { return fmaf(tab[min(max(limit[rt] - key, 0), tab_len - 1)], kLog2e, v); });
+            }
         }
-        if (bias) {  // (a key ahead of the row gives the logarithm of a number that may be negative: the mask below discards it)
-            each([&](float v, int key) { return fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, (float)(limit[rt] - key), 1.f)), v); });
-        }
-        if (tab) {  // (a key ahead of the row reads entry 0 and is masked below)
-            each([&](float v, int key) { return fmaf(tab[min(max(limit[rt] - key, 0), tab_len - 1)], kLog2e, v); });
-        }
+        constexpr float kUnseen = MOD == kScorePlain ? -INFINITY : MOD == kScoreCap ? INFINITY : -1e30f;  // (scaled scores below the maximum that stands in for none)
         if (MASK) {
-            each([&](float v, int key) { return (key <= limit[rt] && (key >= lower[rt] || key < keep_rel)) ? v : -1e30f; });
+            each([&](float v, int key) { return (key <= limit[rt] && (key >= lower[rt] || key < keep_rel)) ? v : kUnseen; });
         }
-        float bmax = -1e30f;
+        float best = kUnseen;
         each([&](float v, int) {
-            bmax = fmaxf(bmax, v);
+            best = MOD == kScoreCap ? fminf(best, v) : fmaxf(best, v);
             return v;
         });
-        const float m_new = fmaxf(m[rt], ga_max_groups(bmax));
+        // (a plain score's scale is not negative: plain_scores())
+        const float m_new = fmaxf(m[rt], ga_max_groups(fmaf(best, base, shift)));
         const float m_ref = fmaxf(m_new, -1e29f);  // a row that has seen no key yet (its chunk starts behind this block): every weight is 0
+        const float bend  = shift - m_ref;
         float       sum   = 0.f;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float e = fast_exp2(sc[rt][kt][r] - m_ref);  // a masked score is -1e30: 2^(-1e30 - m) = 0
+                // (an unseen key's exponent is below -1e29, or -inf)
+                const float e = fast_exp2(MOD == kScoreAny ? sc[rt][kt][r] - m_ref : fmaf(sc[rt][kt][r], base, bend));
                 sum += e;
                 pf[rt][kt >> 1][(kt & 1) * 4 + r] = (__bf16)e;
             }
@@ -956,7 +970,7 @@ __device__ __forceinline__ void ga_staged_step(const bf16x8 (&qf)[RT][DS], const
     }
 }
 
-template<int DS, int VT, int RT, int W>
+template<int DS, int VT, int RT, int W, int MOD>
 __global__ __launch_bounds__(W * 64, 2) void attn_staged_kernel(GeneralAttnParams p, int tiles_per_seq)
 {
     constexpr int kKeyBytes = 64 * DS * 64, kBytes = kKeyBytes + VT * 16 * 128, kPieces = DS * 4 + VT * 2;  // of one block; DMA pieces of 1 KB
@@ -1063,7 +1077,7 @@ __global__ __launch_bounds__(W * 64, 2) void attn_staged_kernel(GeneralAttnParam
             }
             const bool whole = b * 64 + 63 <= pos0 + row0 && b * 64 >= hi_w;  // every row of the wave sees the whole block
 #define TM_STAGED(MASK_) \
-    ga_staged_step<DS, VT, RT, MASK_>(qf, kt, vt, limit, lower, MASK_ ? keep - b * 64 : 0, qscale, cap, inv_cap, bias, r1, r2, m, l, o, tab, p.dist_table_len)
+    ga_staged_step<DS, VT, RT, MASK_, MOD>(qf, kt, vt, limit, lower, MASK_ ? keep - b * 64 : 0, qscale, cap, inv_cap, bias, r1, r2, m, l, o, tab, p.dist_table_len)
             if (whole) {
                 TM_STAGED(false);
             }
@@ -1094,25 +1108,31 @@ __global__ __launch_bounds__(W * 64, 2) void attn_staged_kernel(GeneralAttnParam
         const int t0 = row_base + row0 + rt * 16 + lr;
         inv *= ga_out_gate(p, t0, h);
 #pragma unroll
-        for (int t = 0; t < VT; ++t) {  // lane holds O[row lr][channel t * 16 + lg * 4 + r]
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                ga_store<__bf16>(p, t0, h, t * 16 + lg * 4 + r, o[rt][t][r] * inv);
-            }
+        for (int t = 0; t < VT; ++t) {  // lane holds O[row lr][channels t * 16 + lg * 4 .. + 3]
+            ga_store4<__bf16>(p, t0, h, t * 16 + lg * 4, o[rt][t] * inv);
         }
     }
 }
 
-template<int DS, int VT, int RT, int W>
-static int launch_staged(const GeneralAttnParams& p, hipStream_t st)
+template<int DS, int VT, int RT, int W, int MOD>
+static int launch_staged_mod(const GeneralAttnParams& p, hipStream_t st)
 {
     constexpr int lds = 2 * (64 * DS * 64 + VT * 16 * 128);
-    const auto    k   = attn_staged_kernel<DS, VT, RT, W>;
+    const auto    k   = attn_staged_kernel<DS, VT, RT, W, MOD>;
     TM_TRY_RC(ensure_dynamic_lds((const void*)k, lds));
     const int tiles = (p.max_q_len + W * RT * 16 - 1) / (W * RT * 16);
     k<<<(unsigned)(p.nseq * tiles) * (unsigned)p.q_heads, W * 64, lds, st>>>(p, tiles);
     TM_HIP_CHECK(hipGetLastError());
     return 0;
+}
+
+template<int DS, int VT, int RT, int W>
+static int launch_staged(const GeneralAttnParams& p, hipStream_t st)
+{
+    const bool more = p.dist_r1 || p.dist_table || !(p.scale > 0.f) || !(p.qtemp_coef >= 0.f);  // (a plain score's largest has the largest weight)
+    return more             ? launch_staged_mod<DS, VT, RT, W, kScoreAny>(p, st) :
+           p.softcap > 0.f  ? launch_staged_mod<DS, VT, RT, W, kScoreCap>(p, st) :
+                              launch_staged_mod<DS, VT, RT, W, kScorePlain>(p, st);
 }
 
 // key / value sizes of the staged kernel (0: none)
