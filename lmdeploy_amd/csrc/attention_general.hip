@@ -462,7 +462,7 @@ __device__ __forceinline__ float ga_tanh_fast(float x)
 // (the kept first tokens, block-relative; <= 0: none); r1 / r2: the distance penalty of the lane's rows' head
 // (r1 * log2(1 + r2 * (limit - key)) leaves the score, which lives in the log2 domain; bias = false: none); tab: the distance table's row
 // of the lane's rows' head (nullptr: none)
-template<int DS, int VT, int RT, bool MASK, bool EAGER>
+template<int DS, int VT, int RT, bool MASK>
 __device__ __forceinline__ void ga_block_step(const bf16x8 (&qf)[RT][DS], const __bf16* __restrict__ kb, const __bf16* __restrict__ vb, int D,
                                               int V, const int (&limit)[RT], const int (&lower)[RT], int keep_rel, const float (&qscale)[RT], float cap,
                                               float inv_cap, bool bias, float r1, float r2, float (&m)[RT], float (&l)[RT],
@@ -480,18 +480,8 @@ __device__ __forceinline__ void ga_block_step(const bf16x8 (&qf)[RT][DS], const 
         const __bf16* kr = kb + (size_t)((kt >> 1) * 32 + (lr >> 2) * 8 + (kt & 1) * 4 + (lr & 3)) * D;
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) {
-            // EAGER (decode: a wave has one or two blocks, latency is everything): every load is unconditional -- clamped address, value
-            // selected afterwards -- so that all of them are in flight at once; a guarded load is waited for at the join of its branch.
-            // The prefill kernel keeps the guarded form: with four row tiles per wave the eager form costs registers it does not have.
-            const int d = ds * 32 + lg * 8;
-            bf16x8    kf;
-            if constexpr (EAGER) {
-                const bf16x8 kl = *(const bf16x8*)(kr + min(d, D - 8));
-                kf              = d < D ? kl : zero8;
-            }
-            else {
-                kf = d < D ? *(const bf16x8*)(kr + d) : zero8;
-            }
+            const int    d  = ds * 32 + lg * 8;
+            const bf16x8 kf = d < D ? *(const bf16x8*)(kr + d) : zero8;
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 sc[rt][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[rt][ds], sc[rt][kt], 0, 0, 0);
@@ -502,17 +492,9 @@ __device__ __forceinline__ void ga_block_step(const bf16x8 (&qf)[RT][DS], const 
 #pragma unroll
     for (int t = 0; t < VT; ++t) {
         const int v = t * 16 + lr;
-        if constexpr (EAGER) {
-            const __bf16* vr = vb + (size_t)min(v, V - 1) * 64 + lg * 8;
-            const bf16x8  v0 = *(const bf16x8*)(vr), v1 = *(const bf16x8*)(vr + 32);
-            vf[t][0]         = v < V ? v0 : zero8;
-            vf[t][1]         = v < V ? v1 : zero8;
-        }
-        else {
-            const __bf16* vr = vb + (size_t)v * 64 + lg * 8;
-            vf[t][0]         = v < V ? *(const bf16x8*)(vr) : zero8;
-            vf[t][1]         = v < V ? *(const bf16x8*)(vr + 32) : zero8;
-        }
+        const __bf16* vr = vb + (size_t)v * 64 + lg * 8;
+        vf[t][0]         = v < V ? *(const bf16x8*)(vr) : zero8;
+        vf[t][1]         = v < V ? *(const bf16x8*)(vr + 32) : zero8;
     }
     // lane holds S[row lr of tile rt][key (kt / 2) * 32 + lg * 8 + (kt % 2) * 4 + r].  From here on scores live in the log2 domain
     // (multiplied by log2 e) so that every exponential is one v_exp_f32: the capped score is
@@ -646,10 +628,10 @@ __global__ __launch_bounds__(256) void attn_tiles_kernel(GeneralAttnParams p, in
         const __bf16 *vb = (const __bf16*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V;
         // every row of the wave sees the whole block (rows beyond the portion are discarded anyway)
         if (b * 64 + 63 <= pos0 + row0 && b * 64 >= first_hi) {
-            ga_block_step<DS, VT, RT, false, false>(qf, kb, vb, D, V, limit, lower, 0, qscale, cap, inv_cap, bias, r1, r2, m, l, o, tab, p.dist_table_len);
+            ga_block_step<DS, VT, RT, false>(qf, kb, vb, D, V, limit, lower, 0, qscale, cap, inv_cap, bias, r1, r2, m, l, o, tab, p.dist_table_len);
         }
         else {
-            ga_block_step<DS, VT, RT, true, false>(qf, kb, vb, D, V, limit, lower, keep - b * 64, qscale, cap, inv_cap, bias, r1, r2, m, l, o, tab,
+            ga_block_step<DS, VT, RT, true>(qf, kb, vb, D, V, limit, lower, keep - b * 64, qscale, cap, inv_cap, bias, r1, r2, m, l, o, tab,
                                                    p.dist_table_len);
         }
     }
@@ -743,10 +725,7 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
         for (int v = 0; v < VT; ++v) {
             const int c = v * 16 + lg * 4;
             if (h_ok && c < V) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    agent_store(po + c + r, o[v][r]);
-                }
+                agent_store4(po + c, o[v]);
             }
         }
         if (h_ok && lg == 0) {
@@ -755,10 +734,64 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
         }
     }
     if (p.tickets && ticket_last_workgroup(p.tickets + (size_t)t * p.q_heads + h0, nsplit, last_s)) {
-        const int pieces = V / 4;
-        for (int i = threadIdx.x; i < nh * pieces; i += 256) {
-            const int head = i / pieces, c0 = (i - head * pieces) * 4;
-            ga_merge<T, 4>(p, t, h0 + head, nsplit, [=](int c) { return c0 + c; });
+        // The join of the splits (ga_merge), four channels a piece: everything that several splits have for all of a thread's pieces is asked for together.  Piece
+        // by piece, and a channel at a time, 16 heads of 192 took three trips to memory: three fp32 rows over ~180 entries, 21.0 us then, 14.7 now
+        constexpr int kPieces = (VT * 64 + 255) / 256, kSplits = kPieces <= 2 ? 8 : 4;
+        const int     pieces = V / 4, n = nh * pieces;
+        if ((int)threadIdx.x >= n) {
+            return;
+        }
+        int     head[kPieces], c0[kPieces];
+        float   mm[kPieces], ll[kPieces];
+        floatx4 oo[kPieces];
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            const int at = min((int)threadIdx.x + i * 256, n - 1);
+            head[i] = h0 + at / pieces, c0[i] = at % pieces * 4;
+            mm[i] = p.sink ? p.sink[head[i]] : -1e30f, ll[i] = p.sink ? 1.f : 0.f;
+            oo[i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        for (int s0 = 0; s0 < nsplit; s0 += kSplits) {
+            floatx2 ml[kPieces][kSplits], ov[kPieces][kSplits][2];
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) {
+                if (i * 256 < n) {
+#pragma unroll
+                    for (int k = 0; k < kSplits; ++k) {
+                        const size_t slot = ((size_t)t * p.q_heads + head[i]) * p.splits + min(s0 + k, nsplit - 1);
+                        ml[i][k]          = agent_load2(p.partial_ml + slot * 2);
+                        ov[i][k][0]       = agent_load2(p.partial_o + slot * V + c0[i]);
+                        ov[i][k][1]       = agent_load2(p.partial_o + slot * V + c0[i] + 2);
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) {
+                if (i * 256 < n) {
+                    float mn = mm[i];
+#pragma unroll
+                    for (int k = 0; k < kSplits; ++k) {
+                        mn = fmaxf(mn, ml[i][k][0]);
+                    }
+                    const float a0 = fast_exp2((mm[i] - mn) * kLog2e);
+                    ll[i] *= a0;
+                    oo[i] *= a0;
+#pragma unroll
+                    for (int k = 0; k < kSplits; ++k) {
+                        const float ak = s0 + k < nsplit ? fast_exp2((ml[i][k][0] - mn) * kLog2e) : 0.f;
+                        ll[i]          = fmaf(ak, ml[i][k][1], ll[i]);
+                        oo[i][0] = fmaf(ak, ov[i][k][0][0], oo[i][0]), oo[i][1] = fmaf(ak, ov[i][k][0][1], oo[i][1]);
+                        oo[i][2] = fmaf(ak, ov[i][k][1][0], oo[i][2]), oo[i][3] = fmaf(ak, ov[i][k][1][1], oo[i][3]);
+                    }
+                    mm[i] = mn;
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            if ((int)threadIdx.x + i * 256 < n) {
+                ga_store4<T>(p, t, head[i], c0[i], oo[i] * (ga_out_gate(p, t, head[i]) / ll[i]));
+            }
         }
     }
 }
@@ -766,60 +799,176 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
 // Decode: grid (sequences, kv_heads * head chunks, splits).  The 16 rows are query heads g * group + chunk * 16 + (lane % 16) of row t;
 // wave w takes the blocks b0 + w, b0 + w + 4, ... of the split; waves 1..3 hand their (m, l, O) to wave 0 through LDS.
 template<int DS, int VT>
-__global__ __launch_bounds__(256) void attn_decode_kernel(GeneralAttnParams p, int chunks)
+__global__ __launch_bounds__(256, VT <= 8 && DS * 16 + VT * 8 <= 128 ? 2 : 1) void attn_decode_kernel(GeneralAttnParams p, int chunks)
 {
     __shared__ float    ml_s[4][16][2];
     __shared__ unsigned last_s;
     __shared__ float o_s[3][16][VT * 16 + 4];  // + 4: the sixteen rows start in different banks
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lg = lane >> 4;
     const int t = blockIdx.x, g = blockIdx.y / chunks, chunk = blockIdx.y % chunks, sp = blockIdx.z;
-    const int D = p.dim, V = p.vdim, group = p.q_heads / p.kv_heads;
-    const int lr = lane & 15, lg = lane >> 4;
-    const int hg = chunk * 16 + lr;           // head inside the group
-    const bool h_ok = hg < group;
-    const int  h    = g * group + (h_ok ? hg : 0);
-    const int  s = p.row_seq[t], pos = p.row_pos[t];
+    const int D = p.dim, V = p.vdim, group = p.q_heads / p.kv_heads, h0 = g * group + chunk * 16, nh = min(16, group - chunk * 16);
+    const int h = h0 + min(lr, nh - 1);  // (rows without a head repeat the last one's; they are not stored)
+    const int s = p.row_seq[t], pos = p.row_pos[t];
     const uint64_t* table = p.block_ptrs + (size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride;
-    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    bf16x8 qf[1][DS];
-    {
-        const __bf16* q = (const __bf16*)p.q + (size_t)t * p.ldq + (size_t)h * D;
-#pragma unroll
-        for (int ds = 0; ds < DS; ++ds) {
-            const int    d  = ds * 32 + lg * 8;
-            const bf16x8 ql = *(const bf16x8*)(q + min(d, D - 8));
-            qf[0][ds]       = (h_ok && d < D) ? ql : zero8;
-        }
-    }
-    const float qscale[1] = {p.scale * ga_query_temp(p, pos)};
-    const float cap = p.softcap, inv_cap = cap > 0.f ? 1.f / cap : 0.f;
-    float   m1[1] = {-1e30f}, l1[1] = {0.f};
-    floatx4 o1[1][VT];
-#pragma unroll
-    for (int v = 0; v < VT; ++v) {
-        o1[0][v] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-    const bool  bias = p.dist_r1 != nullptr;
-    const float r1 = bias ? p.dist_r1[h] : 0.f, r2 = bias ? p.dist_r2[h] : 0.f;  // of the lane's head
-    const float* tab = p.dist_table ? p.dist_table + (size_t)h * p.dist_table_len : nullptr;
     const int first = ga_first_key(p, pos), bf = first / 64;
     const int keep = ga_keep(p), nk = ga_keep_blocks(p, first, bf, 64);
     const int nvis = nk + pos / 64 + 1 - bf, per = ga_split_len(p, nvis), nsplit = ga_split_count(p, nvis);
-    const int i0 = sp * per, i1 = min(nvis, i0 + per);
+    const int i1 = min(nvis, sp * per + per);
     if (sp >= nsplit) {
         return;
     }
-    for (int bi = i0 + wave; bi < i1; bi += 4) {
-        const int   b    = ga_block_at(bi, nk, bf);
-        const char* base = global_ptr(table[b]) + p.layer_offset;
-        const int limit[1] = {pos - b * 64}, lower[1] = {first - b * 64};
-        ga_block_step<DS, VT, 1, true, true>(qf, (const __bf16*)base + (size_t)ga_key_head(p, g) * 64 * D,
-                                             (const __bf16*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V, D, V, limit, lower,
-                                             keep - b * 64, qscale, cap, inv_cap, bias, r1, r2, m1, l1, o1, tab, p.dist_table_len);
+    // A wave has one or two blocks, so latency is everything: all keys of a block are asked for at once, then all values, with unconditional addresses.  Left to
+    // itself the compiler waits for each key fragment of 256 channels before it asks for the next, 32 trips to memory in a row; hence the barriers to its
+    // scheduling and, for sizes that keys and values together do not fit in the registers, values that follow the first half of the products.  us, before / with it:
+    // 4 rows of 16 / 1 heads of 256 / 192 over ~2040 entries 34.6 / 26.2, 32 rows of 32 / 8 heads of 128 over ~150 10.1 / 9.2
+    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    const bool   tail  = D < DS * 32;  // channels that do not exist: zero on both sides
+    const __bf16* const q = (const __bf16*)p.q + (size_t)t * p.ldq + (size_t)h * D;
+    bf16x8       qf[DS], kf[4][DS], vf[VT][2];
+    floatx4      o[VT];
+    const __bf16 *kb = nullptr, *vb = nullptr;
+    auto         load_keys = [&](int bi) {
+        const char* base = global_ptr(table[ga_block_at(bi, nk, bf)]) + p.layer_offset;
+        kb               = (const __bf16*)base + (size_t)ga_key_head(p, g) * 64 * D;
+        vb               = (const __bf16*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            const uint32_t row = ((kt >> 1) * 32 + (lr >> 2) * 8 + (kt & 1) * 4 + (lr & 3)) * D;
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) {
+                kf[kt][ds] = *(const bf16x8*)(kb + row + (uint32_t)min(ds * 32 + lg * 8, D - 8));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_values = [&](int t0, int t1) {
+#pragma unroll
+        for (int v = t0; v < t1; ++v) {
+            const uint32_t row = min(v * 16 + lr, V - 1) * 64 + lg * 8;  // (channels behind the last are not stored)
+            vf[v][0]           = *(const bf16x8*)(vb + row);
+            vf[v][1]           = *(const bf16x8*)(vb + row + 32);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds) {
+        qf[ds] = *(const bf16x8*)(q + min(ds * 32 + lg * 8, D - 8));
     }
-    const int h0 = g * group + chunk * 16;
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+        o[v] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    float m = -1e30f, l = 0.f;
+    int   bi = sp * per + wave;
+    if (bi < i1) {
+        load_keys(bi);
+        const float qscale = p.scale * ga_query_temp(p, pos), cap = p.softcap, cap2 = cap * kLog2e;
+        const float k1     = cap > 0.f ? qscale / cap * (2.f * kLog2e) : qscale * kLog2e;  // (scores in the log2 domain, as in ga_block_step)
+        const bool  bias   = p.dist_r1 != nullptr;
+        const float r1 = bias ? p.dist_r1[h] : 0.f, r2 = bias ? p.dist_r2[h] : 0.f;  // of the lane's head
+        const float* tab = p.dist_table + (size_t)h * p.dist_table_len;
+        if (tail) {
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) {
+                qf[ds] = ds * 32 + lg * 8 < D ? qf[ds] : zero8;
+            }
+        }
+        for (;;) {
+            const int b = ga_block_at(bi, nk, bf), limit = pos - b * 64, lower = first - b * 64, klo = keep - b * 64;
+            floatx4   sc[4];
+            constexpr int kEarly = DS * 16 + VT * 8 <= 128 ? VT : VT / 2;  // value tiles beside all keys
+            if constexpr (DS * 16 + VT * 8 <= 128) {
+                load_values(0, VT);
+            }
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                if (tail) {
+#pragma unroll
+                    for (int ds = 0; ds < DS; ++ds) {
+                        kf[kt][ds] = ds * 32 + lg * 8 < D ? kf[kt][ds] : zero8;
+                    }
+                }
+                sc[kt] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int ds = 0; ds < DS; ++ds) {
+                    sc[kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[kt][ds], qf[ds], sc[kt], 0, 0, 0);
+                }
+                if constexpr (DS * 16 + VT * 8 > 128) {
+                    if (kt == 1) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        load_values(0, kEarly);
+                    }
+                    if (kt == 3) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        load_values(kEarly, VT);
+                    }
+                }
+            }
+            // lane: head lr, keys (kt / 2) * 32 + lg * 8 + (kt % 2) * 4 + r
+            float add[4][4] = {};
+            if (p.dist_table) {  // the lane's head's row of the distance table (a key ahead of the row reads entry 0 and is masked below)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int key      = (i >> 3) * 32 + lg * 8 + (i & 7);
+                    add[i >> 2][i & 3] = tab[min(max(limit - key, 0), p.dist_table_len - 1)];
+                }
+            }
+            float bmax = -1e30f;
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float v = sc[kt][r] * k1;
+                    if (cap > 0.f) {
+                        v = fmaf(__builtin_amdgcn_rcpf(fast_exp2(v) + 1.f), -2.f * cap2, cap2);
+                    }
+                    const int key = (kt >> 1) * 32 + lg * 8 + (kt & 1) * 4 + r;
+                    if (bias) {  // (a key ahead of the row gives the logarithm of a number that may be negative: the mask below discards it)
+                        v = fmaf(-r1, __builtin_amdgcn_logf(fmaf(r2, (float)(limit - key), 1.f)), v);
+                    }
+                    if (p.dist_table) {
+                        v = fmaf(add[kt][r], kLog2e, v);
+                    }
+                    sc[kt][r] = key <= limit && (key >= lower || key < klo) ? v : -1e30f;
+                    bmax      = fmaxf(bmax, sc[kt][r]);
+                }
+            }
+            bmax              = fmaxf(bmax, __shfl_xor(bmax, 16));
+            bmax              = fmaxf(bmax, __shfl_xor(bmax, 32));
+            const float m_new = fmaxf(m, bmax), alpha = fast_exp2(m - m_new);
+            const float m_ref = fmaxf(m_new, -1e29f);  // no key seen yet: every weight is 0
+            float       bsum  = 0.f;
+            bf16x8      pf[2];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float e = fast_exp2(sc[kt][r] - m_ref);  // a masked score is -1e30: 2^(-1e30 - m) = 0
+                    bsum += e;
+                    pf[kt >> 1][(kt & 1) * 4 + r] = (__bf16)e;
+                }
+            }
+            bsum += __shfl_xor(bsum, 16);
+            bsum += __shfl_xor(bsum, 32);
+            l = l * alpha + bsum;
+            m = m_new;
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+                o[v] *= alpha;
+#pragma unroll
+                for (int ks = 0; ks < 2; ++ks) {
+                    o[v] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[v][ks], pf[ks], o[v], 0, 0, 0);
+                }
+            }
+            bi += 4;
+            if (bi >= i1) {
+                break;
+            }
+            load_keys(bi);
+        }
+    }
     // (back from the log2 domain: the merges use e^x)
-    ga_close_heads<__bf16, VT>(p, t, sp, nsplit, h0, min(16, group - chunk * 16), m1[0] * kLn2, l1[0], o1[0], ml_s, o_s, &last_s);
+    ga_close_heads<__bf16, VT>(p, t, sp, nsplit, h0, nh, m * kLn2, l, o, ml_s, o_s, &last_s);
 }
 
 bool general_attention_tiles_ok(const GeneralAttnParams& p)
@@ -1231,7 +1380,7 @@ __global__ __launch_bounds__(256) void attn_heads_f32_kernel(GeneralAttnParams p
     __shared__ float    ml_s[4][16][2];
     __shared__ unsigned last_s;
     __shared__ float    o_s[3][16][VT * 16 + 4];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lr = lane & 15, lg = lane >> 4;
     const int t = blockIdx.x, g = blockIdx.y / chunks, chunk = blockIdx.y % chunks, sp = blockIdx.z;
     const int D = p.dim, V = p.vdim, group = p.q_heads / p.kv_heads, h0 = g * group + chunk * 16, nh = min(16, group - chunk * 16);
     const int h = h0 + min(lr, nh - 1), pos = p.row_pos[t], s = p.row_seq[t];
@@ -1243,85 +1392,127 @@ __global__ __launch_bounds__(256) void attn_heads_f32_kernel(GeneralAttnParams p
     if (sp >= nsplit) {
         return;
     }
+    // Keys and values of a block are asked for all at once, before the queries are waited for; the barrier keeps the compiler from asking for them two at a time (420 rows of three prompts, 16 / 1 heads of 256 / 192: 36.6 -> 31.6 us)
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-    floatx4       q[DS], o[VT];
+    const bool    tail = D < DS * 16;
+    floatx4       q[DS], o[VT], k[DS], v4[VT];
 #pragma unroll
     for (int i = 0; i < DS; ++i) {
-        const int d = i * 16 + lg * 4;
-        q[i]        = *(const ga_floatx4_any*)((const float*)p.q + (size_t)t * p.ldq + (size_t)h * D + min(d, D - 4));
-        if (d >= D) {
-            q[i] = zero;
-        }
+        q[i] = *(const ga_floatx4_any*)((const float*)p.q + (size_t)t * p.ldq + (size_t)h * D + min(i * 16 + lg * 4, D - 4));
     }
 #pragma unroll
     for (int v = 0; v < VT; ++v) {
         o[v] = zero;
     }
-    const float  qscale = p.scale * ga_query_temp(p, pos);
-    const bool   bias   = p.dist_r1 != nullptr;
-    const float  r1 = bias ? p.dist_r1[h] : 0.f, r2 = bias ? p.dist_r2[h] : 0.f;
-    const float* tab = p.dist_table ? p.dist_table + (size_t)h * p.dist_table_len : nullptr;
-    float        m = -1e30f, l = 0.f;
-    const int    j0 = wave * 16;
-    for (int bi = i0; bi < i1; ++bi) {
+    float     m = -1e30f, l = 0.f;
+    const int j0 = wave * 16;
+    auto      unseen = [&](int bi) {  // none of the wave's keys of the block is seen
         const int b = ga_block_at(bi, nk, bf), limit = pos - b * 64, lower = first - b * 64, klo = keep - b * 64;
-        if (j0 > limit || (j0 + 15 < lower && j0 >= klo)) {  // none of the wave's keys is seen
-            continue;
-        }
-        const char*  base = global_ptr(table[b]) + p.layer_offset;
-        const float* kb   = (const float*)base + ((size_t)ga_key_head(p, g) * 64 + j0 + lr) * D;
-        const float* vb   = (const float*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V + j0 + lg * 4;
-        floatx4      k[DS], v4[VT];
+        return j0 > limit || (j0 + 15 < lower && j0 >= klo);
+    };
+    auto load = [&](int bi) {
+        const char*  base = global_ptr(table[ga_block_at(bi, nk, bf)]) + p.layer_offset;
+        const float* kb   = (const float*)base + (size_t)ga_key_head(p, g) * 64 * D;
+        const float* vb   = (const float*)(base + p.v_offset) + (size_t)ga_value_head(p, g) * 64 * V;
 #pragma unroll
         for (int i = 0; i < DS; ++i) {
-            k[i] = *(const ga_floatx4_any*)(kb + min(i * 16 + lg * 4, D - 4));
+            k[i] = *(const ga_floatx4_any*)(kb + (uint32_t)((j0 + lr) * D + min(i * 16 + lg * 4, D - 4)));
         }
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
-            v4[v] = *(const ga_floatx4_any*)(vb + (size_t)min(v * 16 + lr, V - 1) * 64);
+            v4[v] = *(const ga_floatx4_any*)(vb + (uint32_t)(min(v * 16 + lr, V - 1) * 64 + j0 + lg * 4));
         }
-        floatx4 sc = zero;
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int bi = i0;
+    while (bi < i1 && unseen(bi)) {
+        ++bi;
+    }
+    if (bi < i1) {
+        load(bi);
+        const float  qscale = p.scale * ga_query_temp(p, pos);
+        const bool   bias   = p.dist_r1 != nullptr;
+        const float  r1 = bias ? p.dist_r1[h] : 0.f, r2 = bias ? p.dist_r2[h] : 0.f;
+        const float* tab = p.dist_table + (size_t)h * p.dist_table_len;
+        if (tail) {
 #pragma unroll
-        for (int i = 0; i < DS; ++i) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                sc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][c], q[i][c], sc, 0, 0, 0);
+            for (int i = 0; i < DS; ++i) {
+                q[i] = i * 16 + lg * 4 < D ? q[i] : zero;
             }
         }
-        bool  seen[4];
-        float mx = -1e30f;
+        for (;;) {
+            const int b = ga_block_at(bi, nk, bf), limit = pos - b * 64, lower = first - b * 64, klo = keep - b * 64;
+            // two chains: a product that waits for the one before it takes longer than the matrix core needs
+            floatx4 sc = zero, sc2 = zero;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int j = j0 + lg * 4 + r;
-            seen[r]     = j <= limit && (j >= lower || j < klo);
-            float x     = ga_modify(p, sc[r], qscale);
-            if (bias) {
-                x -= r1 * log1pf(r2 * (float)(limit - j));
+            for (int i = 0; i < DS; i += 2) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    sc = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][c], q[i][c], sc, 0, 0, 0);
+                    if (i + 1 < DS) {
+                        sc2 = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i + 1][c], q[i + 1][c], sc2, 0, 0, 0);
+                    }
+                }
             }
-            if (tab && seen[r]) {
-                x += tab[min(limit - j, p.dist_table_len - 1)];
+            sc += sc2;
+            float add[4] = {};
+            if (p.dist_table) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    add[r] = tab[min(max(limit - (j0 + lg * 4 + r), 0), p.dist_table_len - 1)];
+                }
             }
-            sc[r] = seen[r] ? x : -1e30f;
-            mx    = fmaxf(mx, sc[r]);
-        }
-        const float m_new = fmaxf(m, ga_max_groups(mx)), alpha = __expf(m - m_new);
-        m = m_new;
-        l *= alpha;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            sc[r] = seen[r] ? __expf(sc[r] - m_new) : 0.f;
-            l += sc[r];
-        }
-        // entries that the row does not see -- behind its own, and before its window or chunk -- may hold anything: a weight of zero does not take them out
-        const bool whole = j0 + 15 <= limit && (j0 >= lower || j0 + 15 < klo);
-#pragma unroll
-        for (int v = 0; v < VT; ++v) {
-            o[v] *= alpha;
+            bool  seen[4];
+            float mx = -1e30f;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float x = whole || seen[r] ? v4[v][r] : 0.f;
-                o[v]          = __builtin_amdgcn_mfma_f32_16x16x4f32(x, sc[r], o[v], 0, 0, 0);
+                const int j = j0 + lg * 4 + r;
+                seen[r]     = j <= limit && (j >= lower || j < klo);
+                float x     = ga_modify(p, sc[r], qscale);
+                if (bias) {
+                    x -= r1 * log1pf(r2 * (float)(limit - j));
+                }
+                x += add[r];
+                sc[r] = seen[r] ? x : -1e30f;
+                mx    = fmaxf(mx, sc[r]);
             }
+            const float m_new = fmaxf(m, ga_max_groups(mx)), alpha = __expf(m - m_new);
+            m = m_new;
+            l *= alpha;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                sc[r] = seen[r] ? __expf(sc[r] - m_new) : 0.f;
+                l += sc[r];
+            }
+            // entries that the row does not see -- behind its own, and before its window or chunk -- may hold anything: a weight of zero does not take them out
+            const bool whole = j0 + 15 <= limit && (j0 >= lower || j0 + 15 < klo);
+            if (!whole) {
+#pragma unroll
+                for (int v = 0; v < VT; ++v) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        v4[v][r] = seen[r] ? v4[v][r] : 0.f;
+                    }
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < VT; ++v) {
+                o[v] *= alpha;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                for (int v = 0; v < VT; ++v) {
+                    o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[v][r], sc[r], o[v], 0, 0, 0);
+                }
+            }
+            do {
+                ++bi;
+            } while (bi < i1 && unseen(bi));
+            if (bi >= i1) {
+                break;
+            }
+            load(bi);
         }
     }
     l += __shfl_xor(l, 16);

@@ -12,6 +12,7 @@ typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef float    floatx4 __attribute__((ext_vector_type(4)));
+typedef float    floatx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -160,6 +161,16 @@ __device__ __forceinline__ void agent_store(float* p, float v)
 __device__ __forceinline__ float agent_load(const float* p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// four neighbours, two at a time
+__device__ __forceinline__ void agent_store4(float* p, floatx4 v)
+{
+    __hip_atomic_store((uint64_t*)p, bit_cast<uint64_t>(floatx2{v[0], v[1]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store((uint64_t*)p + 1, bit_cast<uint64_t>(floatx2{v[2], v[3]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ floatx2 agent_load2(const float* p)
+{
+    return bit_cast<floatx2>(__hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 // of n arrivals: is this the last one (which also clears the ticket)?  One lane calls it after the stores are drained
 __device__ __forceinline__ bool ticket_last(unsigned* ticket, int n)

@@ -42,3 +42,30 @@ def test_rows_of_one_and_of_many_splits(tm, cuda, seqs, heads, kv_heads, D, V, w
             ref = row_oracle(spec, q[s], K[s][:n + 1], W[s][:n + 1], n)
             # weights and results are rounded to bf16, 2^-9 of each: 3e-2 of the largest value leaves the same room as the kernels' other tests
             assert np.abs(got[s] - ref).max() <= 3e-2 * max(1.0, np.abs(ref).max()), (kernel, s, n)
+
+
+@pytest.mark.parametrize('splits', [1, 3])
+@pytest.mark.parametrize('D,V', [(8, 8), (128, 128), (128, 136), (120, 128), (192, 64), (192, 72), (256, 16), (256, 192), (248, 192), (136, 256), (256, 256)])
+def test_sizes_of_either_load_order(tm, cuda, D, V, splits):
+    """sizes whose keys and values are asked for at once and sizes whose values follow, with and without channels short of the instantiation's; waves with
+    no block, one and two; three heads a key head: rows of the tile without a head"""
+    rng = np.random.default_rng(D + V)
+    lens = [0, 62, 63, 64, 255, 256, 700]
+    spec = dict(heads=6, kv_heads=2, dim=D, vdim=V, scale=D ** -0.5, window=0, keep=0)
+    cache = Paged(0, 2, D, V, [n + 1 for n in lens], rng)
+    K = [_rounded(rng.normal(0, 1, (n + 1, 2, D)), 0) for n in lens]
+    W = [_rounded(rng.normal(0, 1, (n + 1, 2, V)), 0) for n in lens]
+
+    def call(lo, hi, kernel, prefill, n):
+        rs = np.repeat(np.arange(len(lens)), np.subtract(hi, lo))
+        rp = np.concatenate([np.arange(a, b) for a, b in zip(lo, hi)]).astype(int)
+        q = _rounded(rng.normal(0, 1, (len(rs), 6 * D)), 0)
+        kn, vn = (np.stack([c[s][p].reshape(-1) for s, p in zip(rs, rp)]) for c in (K, W))
+        return q, attend(tm, 0, spec, cache, q, kn, vn, rs, rp, np.concatenate([[0], np.cumsum(np.subtract(hi, lo))]), hi, kernel, n, prefill)
+
+    call([0] * len(lens), lens, 1, 1, 1)                      # fills the cache
+    q, got = call(lens, [n + 1 for n in lens], 3, 0, splits)
+    for s, n in enumerate(lens):
+        ref = row_oracle(spec, q[s], K[s][:n + 1], W[s][:n + 1], n)
+        # a weight and a result are rounded to bf16, 2^-9 of each; scores are sums of exact products of bf16 numbers in fp32, off by D 2^-24 of some 10
+        assert np.abs(got[s] - ref).max() <= (2 ** -8 + D * 2 ** -19) * max(1.0, np.abs(W[s][:n + 1]).max()), (s, n)
