@@ -23,6 +23,7 @@ struct F16Epi {
     int vec;    // rows of y start on 8 bytes
 
     static constexpr bool kPairs = false, kTileRuns = false;
+    static constexpr int  kReads = 0;
     __device__ __forceinline__ const int* row_offsets() const
     {
         return nullptr;

@@ -1106,6 +1106,22 @@ __global__ __launch_bounds__(256, 1) void stream_tile256_kernel(StreamArgs a, Ep
                 }
             }
         }
+        else if constexpr (Epi::kReads > 0) {  // what kReads outputs need is on its way together (DenseEpi)
+            constexpr int kOps = Epi::kReads;
+#pragma unroll 1
+            for (int n0 = 0; n0 < 16; n0 += kOps) {
+                typename Epi::Operand op[kOps];
+                epi.template operands<kOps>(a, item, [&](int n) { return int2{min(mb + (n0 + n) * 2 + half, item.M - 1), nb + l31 * 4}; }, op);
+#pragma unroll
+                for (int n = 0; n < kOps; ++n) {
+                    const int     r = (n0 + n) * 2 + half;
+                    const floatx4 v = sw[r * 32 + (l31 ^ r)];
+                    if (mb + r < item.M) {
+                        epi.join(a, item, mb + r, nb + l31 * 4, v, op[n]);
+                    }
+                }
+            }
+        }
         else {
 #pragma unroll
             for (int n = 0; n < 16; ++n) {
