@@ -231,6 +231,12 @@ struct DenseEpi {
         it.x_off *= sizeof(T), it.w_off *= 2;
         return it;
     }
+    // asks early for what an output is added to (its first element brings the line); whoever calls it keeps the result until rows()
+    __device__ __forceinline__ unsigned touch(const StreamArgs& a, const DenseItem& it, int m, int n) const
+    {
+        const int epi = EPI >= 0 ? EPI : c.epi;
+        return epi == kDenseResidAdd || epi == kDenseResidGate ? ((const unsigned*)a.y)[(size_t)(m + it.row_base) * a.ldy + it.col_base + n] : 0u;
+    }
     // acc[j]: columns n + 16 j .. + 3
     template<int NT>
     __device__ __forceinline__ void rows(const StreamArgs& a, const DenseItem& it, int m, int n, const floatx4 (&acc)[NT]) const

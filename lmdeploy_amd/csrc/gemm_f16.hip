@@ -36,6 +36,10 @@ struct F16Epi {
     {
         return {0, 0, M};
     }
+    __device__ __forceinline__ unsigned touch(const StreamArgs&, const F16Item&, int, int) const  // (nothing is read)
+    {
+        return 0;
+    }
     template<int NT>
     __device__ __forceinline__ void rows(const StreamArgs& a, const F16Item&, int m, int n, const floatx4 (&acc)[NT]) const
     {
@@ -114,6 +118,10 @@ struct F16EpiKv: F16Epi {
 
 // The same for a product that closes a residual block: y += h(acc), in fp16 (residual_rmsnorm's addition)
 struct F16EpiAdd: F16Epi {
+    __device__ __forceinline__ unsigned touch(const StreamArgs& a, const F16Item&, int m, int n) const
+    {
+        return ((const unsigned short*)a.y)[(size_t)m * a.ldy + n];
+    }
     template<int NT>
     __device__ __forceinline__ void rows(const StreamArgs& a, const F16Item&, int m, int n, const floatx4 (&acc)[NT]) const
     {

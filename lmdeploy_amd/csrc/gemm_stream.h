@@ -359,18 +359,49 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
         if (ph > 0) {
             return;
         }
+        // in the order of the slices, several of them and what the outputs are added to asked for at once: the seven slices of (8192, 2048) were four trips to memory in a
+        // row, and the outputs a fifth (fp16, 8 rows 10.3 -> 9.8 us in a model)
+        constexpr int kZ = MT * NT >= 4 ? 2 : 8 / (MT * NT);
+        unsigned      warm[MT][NT];
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            if (t * 16 < M) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                acc[t][j]  = floatx4{0.f, 0.f, 0.f, 0.f};
+                warm[t][j] = epi.touch(a, item, mb + min(t * 16 + fr, M - 1), min(n + 16 * j, a.N - 1));
+            }
+        }
+        for (int z0 = 0; z0 < (int)gridDim.z; z0 += kZ) {
+            u32x4 part[MT][NT][kZ];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
 #pragma unroll
                 for (int j = 0; j < NT; ++j) {
                     const int at = ((mb + min(t * 16 + fr, M - 1)) * ld + min(n + 16 * j, ld - 4)) * 4;
-                    acc[t][j]    = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-                    for (int z = 0; z < (int)gridDim.z; ++z) {
-                        acc[t][j] += bit_cast<floatx4>(__builtin_amdgcn_raw_buffer_load_b128(rs, at, (int)(z * rows), /*sc1*/ 16));
+#pragma unroll
+                    for (int z = 0; z < kZ; ++z) {
+                        part[t][j][z] = __builtin_amdgcn_raw_buffer_load_b128(rs, at, (int)(min(z0 + z, (int)gridDim.z - 1) * rows), /*sc1*/ 16);
                     }
                 }
+            }
+#pragma unroll
+            for (int z = 0; z < kZ; ++z) {
+                if (z0 + z < (int)gridDim.z) {
+#pragma unroll
+                    for (int t = 0; t < MT; ++t) {
+#pragma unroll
+                        for (int j = 0; j < NT; ++j) {
+                            acc[t][j] += bit_cast<floatx4>(part[t][j][z]);
+                        }
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                asm volatile("" ::"v"(warm[t][j]));
             }
         }
     }
@@ -539,6 +570,10 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
             compute(wa, xa, base);
         }
     }
+    unsigned warm = 0;  // (what the outputs are added to is on its way while the waves meet; two tiles of columns have no register for it)
+    if (NT == 1 && wave < MT) {
+        warm = epi.touch(a, item, mb + min(wave * 16 + fr, M - 1), min(tile0 * 16 + fc * 4, a.N - 1));
+    }
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
 #pragma unroll
@@ -555,6 +590,9 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
                 s += red[v][wave * NT + j][lane];
             }
             acc[0][j] = s;
+        }
+        if constexpr (NT == 1) {
+            asm volatile("" ::"v"(warm));
         }
         const int m = wave * 16 + fr;
         if (m < M) {
