@@ -852,9 +852,177 @@ __global__ __launch_bounds__(NT) void layer_close_kernel(LayerClose c)
     }
 }
 
+// The same by fours (H % 4 = 0, H <= NT * 4 * NQ, every row at a multiple of four elements): memory bounds it with many rows -- a layer reads the stream, the side's
+// result and all layers before it -- and a chain of trips to memory with few, so whatever needs no statistic is asked for first: the first U layers of the depth, the
+// norm's weights.  us, a channel at a time / this: 8010 rows of 2048 with one to eight layers before 115 / 101 (5.3 TB/s), 420 rows 15.1 / 9.0, three rows 6.4 / 4.2.
+// Other widths and rows that are not aligned, and more than 8192 channels, take the kernel above
+template<class T, int NT, int NQ, int U>
+__global__ __launch_bounds__(NT) void layer_close4_kernel(LayerClose c)
+{
+    __shared__ float red[NT / 64];
+    const int     m = blockIdx.x, H = c.H, depth = c.depth;
+    const size_t  r0 = (size_t)m * H;
+    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+    int           at[NQ];  // (threads behind the row's end read its last four channels)
+    bool          in[NQ];
+    floatx4       v[NQ], y[NQ], sw[NQ], lw[NQ], lb[NQ], past[U][NQ];
+    float         w[U], wv = 0.f;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int i = (threadIdx.x + q * NT) * 4;
+        in[q]       = i < H;
+        at[q]       = min(i, H - 4);
+        v[q]        = *(const floatx4*)(c.x + r0 + at[q]);
+    }
+    if (c.y) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            y[q]  = *(const floatx4*)(c.y + r0 + at[q]);
+            sw[q] = *(const floatx4*)(c.side_w + at[q]);
+        }
+    }
+    auto load_past = [&](int j0) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int j = min(j0 + u, depth - 1);
+            w[u]        = c.dwa[j];
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) {
+                past[u][q] = *(const floatx4*)(c.history + (size_t)j * c.stride + r0 + at[q]);
+            }
+        }
+    };
+    if (depth > 0) {
+        wv = c.dwa[depth];
+        load_past(0);
+    }
+    if (c.ln_w) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            lw[q] = *(const floatx4*)(c.ln_w + at[q]);
+            lb[q] = *(const floatx4*)(c.ln_b + at[q]);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (c.y) {
+        float ss = 0.f;
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            y[q] = in[q] ? y[q] : zero;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                ss = fmaf(y[q][e], y[q][e], ss);
+            }
+        }
+        const float inv = 1.0f / sqrtf(block_sum<NT>(ss, red) / (float)H + c.eps);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[q][e] = fmaf(y[q][e] * inv, sw[q][e], v[q][e]);
+            }
+        }
+    }
+    if (depth > 0) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            if (in[q] && !c.last) {
+                *(floatx4*)(c.history + (size_t)depth * c.stride + r0 + at[q]) = v[q];
+            }
+            v[q] *= wv;
+        }
+        for (int j0 = 0;;) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (j0 + u < depth) {
+#pragma unroll
+                    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            v[q][e] = fmaf(w[u], past[u][q][e], v[q][e]);
+                        }
+                    }
+                }
+            }
+            j0 += U;
+            if (j0 >= depth) {
+                break;
+            }
+            load_past(j0);
+        }
+    }
+    float sm = 0.f;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        if (in[q]) {
+            *(floatx4*)(c.x + r0 + at[q]) = v[q];
+            sm += (v[q][0] + v[q][1]) + (v[q][2] + v[q][3]);
+        }
+    }
+    if (!c.ln_w) {
+        return;
+    }
+    const float mean = block_sum<NT>(sm, red) / (float)H;
+    float       ss   = 0.f;
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float d = in[q] ? v[q][e] - mean : 0.f;
+            ss            = fmaf(d, d, ss);
+        }
+    }
+    const float inv = 1.0f / sqrtf(block_sum<NT>(ss, red) / (float)H + c.eps);
+    typedef T   T4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        if (in[q]) {
+            T4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                o[e] = (T)fmaf((v[q][e] - mean) * inv, lw[q][e], lb[q][e]);
+            }
+            *(T4*)((T*)c.h + (size_t)m * c.ldh + at[q]) = o;
+        }
+    }
+}
+
+template<class T>
+static bool launch_layer_close4(const LayerClose& c, hipStream_t st)
+{
+    auto aligned = [](const void* p, size_t n) { return (uintptr_t)p % n == 0; };
+    if (c.H % 4 || c.H < 4 || c.H > 8192 || !aligned(c.x, 16) || (c.y && (!aligned(c.y, 16) || !aligned(c.side_w, 16))) || (c.depth > 0 && (!aligned(c.history, 16) || c.stride % 4))
+        || (c.ln_w && (!aligned(c.ln_w, 16) || !aligned(c.ln_b, 16) || !aligned(c.h, 4 * sizeof(T)) || c.ldh % 4))) {
+        return false;
+    }
+    const bool few = c.M <= 256;  // latency counts: every wave the row can fill
+    if (c.H <= 1024) {
+        layer_close4_kernel<T, 256, 1, 4><<<c.M, 256, 0, st>>>(c);
+    }
+    else if (c.H <= 2048 && few) {
+        layer_close4_kernel<T, 512, 1, 8><<<c.M, 512, 0, st>>>(c);
+    }
+    else if (c.H <= 2048) {
+        layer_close4_kernel<T, 256, 2, 4><<<c.M, 256, 0, st>>>(c);
+    }
+    else if (c.H <= 4096 && !few) {
+        layer_close4_kernel<T, 256, 4, 2><<<c.M, 256, 0, st>>>(c);
+    }
+    else if (c.H <= 4096) {
+        layer_close4_kernel<T, 1024, 1, 8><<<c.M, 1024, 0, st>>>(c);
+    }
+    else {
+        layer_close4_kernel<T, 1024, 2, 4><<<c.M, 1024, 0, st>>>(c);
+    }
+    return true;
+}
+
 template<class T>
 static void launch_layer_close_t(const LayerClose& c, hipStream_t st)
 {
+    if (launch_layer_close4<T>(c, st)) {
+        return;
+    }
     if (c.M <= 256 && c.H > 1024 && c.H <= 8192) {  // few rows: latency counts, every wave the row can fill
         if (c.H <= 4096) {
             layer_close_kernel<T, 1024, 4><<<c.M, 1024, 0, st>>>(c);
