@@ -175,6 +175,16 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
         }
         i += R;
     }
+    half4_t stream[2] = {};  // what the results are added to, asked for ahead of the last products: behind them it was two trips to memory in a row
+    // (one sequence, 8 layers of Llama-3-8B's shapes: 8.62 -> 8.54 ms for 37 tokens and 16 more)
+    if constexpr (NP == 0) {
+        if (p.epilogue == 4 && ph == 0) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                stream[u] = *(const half4_t*)(p.y + (size_t)min(fr, M - 1) * p.ldy + cgc * 32 + u * 16 + fc * 4);
+            }
+        }
+    }
 #pragma unroll
     for (int s = 0; s < R; ++s) {
         if (i + s < n) {
@@ -252,7 +262,7 @@ __global__ __launch_bounds__(CW* KP * 64) void gemm_w4_rows_kernel(Dec32Params p
             half4_t* y = (half4_t*)(p.y + (size_t)fr * p.ldy + c);
             half4_t  h = {(half_t)a[0], (half_t)a[1], (half_t)a[2], (half_t)a[3]};
             if (p.epilogue == 4) {  // the residual stream: the product's fp16 rounding, then an addition in fp16
-                h = *y + h;
+                h = stream[u] + h;
             }
             *y = h;
         }
