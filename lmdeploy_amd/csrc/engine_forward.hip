@@ -993,8 +993,10 @@ int prefill_slots(tm_engine* e, const int* const* seq_ids, const int* host_lens,
         e->d_block_ptrs += (size_t)(slot0 + b0) * e->max_blocks_per_seq;
         const MixedDecode md{nd, merge ? mix->k_len : nullptr, merge ? mix->block_ptrs : nullptr, merge ? mix->cu_q : nullptr,
                              merge ? mix->active : nullptr};
-        const int rc    = forward(e, e->d_prefill_ids, nd + tokens, nseq, false, max_q, max_k, e->kflat_stride, slot0 + b0,
-                                  merge ? &md : nullptr);
+        e->prompts_whole = klen[0] == cu_q[1];  // (only the first sequence of a portion may have been begun before)
+        const int rc     = forward(e, e->d_prefill_ids, nd + tokens, nseq, false, max_q, max_k, e->kflat_stride, slot0 + b0,
+                                   merge ? &md : nullptr);
+        e->prompts_whole = false;
         e->d_block_ptrs = saved_ptrs;
         e->mb           = {};
         if (rc) {

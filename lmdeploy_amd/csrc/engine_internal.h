@@ -85,6 +85,7 @@ struct LmLayer {
     int           c_k = 0, c_v = 0, c_g = 0, c_rg1 = 0, c_rg2 = 0, c_router = 0;  // columns of the fused projection
     int           plain_stride = 0, lat_stride = 0;      // latent: head strides of the unrotated query parts / of the latent attention output
     DenseWeight   wo, gu, down;      // output projection; [gate | up] along N; down (experts: one image per expert in gu / down)
+    DenseWeight   ukv;               // latent, where prompts expand it: [keys' own channels of every head | values of every head], K kv_rank
     DenseWeight   uk, uv;            // latent: key expansion transposed [kv_rank][dim] and value expansion [vdim][kv_rank], one image per head
     float *       r1 = nullptr, *r2 = nullptr, *rg1_b = nullptr, *rg2_b = nullptr, *c_norm = nullptr, *inv_freq = nullptr;
     // post-norm blocks (spec.post_norm): x += LN1(mixer(x)); x += LN2(ff(x)).  `qkv` holds every projection of the mixer's input side by
@@ -155,6 +156,11 @@ struct LayeredModel {
     void *               d_h1 = nullptr, *d_hh = nullptr, *d_qkv = nullptr, *d_cat = nullptr, *d_hn = nullptr;
     // wide blocks: fused projection (fp32), queries, unrotated query parts, latent attention output, activations
     float *              d_proj = nullptr, *d_x0 = nullptr, *d_moe_y = nullptr, *d_topk_w = nullptr;
+    // latent attention over whole prompts: their entries as rows, what every head makes of them, blocks and table of the attention
+    void *               d_entries = nullptr, *d_up = nullptr;
+    char*                d_xblocks = nullptr;
+    uint64_t*            d_xtable = nullptr;
+    int                  lde = 0, ldup = 0, xstride = 0, entries_of = -1;  // entries_of: the layer whose entries d_entries holds in this forward
     void *               d_q = nullptr, *d_plain = nullptr, *d_lat = nullptr, *d_ff = nullptr, *d_xx = nullptr, *d_moe_x = nullptr;
     int *                d_topk_ids = nullptr, *d_offsets = nullptr, *d_f2n = nullptr, *d_en2f = nullptr;
     // post-norm blocks: a sublayer's fp32 result, state mixers' fp32 output and per-row vectors, the decay's inner activations
@@ -214,6 +220,7 @@ struct LmPart {
     int             max_q_len;
     int             slot0  = 0;         // seq_slot == nullptr: sequence i lives in batch slot slot0 + i (the recurrent states are per slot)
     const int*      active = nullptr;   // [nseq] or nullptr; 0: a placeholder row of a slot without a running sequence
+    bool            whole  = false;     // prompts from their first token on: no sequence of the part has earlier keys
 };
 
 }  // namespace tmk
@@ -221,6 +228,7 @@ struct LmPart {
 using namespace tmk;
 
 struct tm_engine {
+    bool prompts_whole = false;  // the prompt rows of the forward being issued begin their sequences
     tm_engine_config cfg{};
     // local (per-rank) dims
     int q_heads = 0, kv_heads = 0, inter = 0, vocab_local = 0, hidden = 0, D = 128;

@@ -221,6 +221,16 @@ static int upload_f32(tm_engine* e, const std::vector<float>& v, float** out)
     return 0;
 }
 
+// Whether attention over whole prompts may run on keys and values that every head makes of the latent entries, instead of on the entries: a product of the attention then has
+// dim + rot_dim and vdim channels instead of kv_rank + rot_dim and kv_rank.  bf16, the sizes of the staged tile kernel
+static bool latent_can_expand(const tm_engine* e, const LmLayer& L)
+{
+    const tm_layer_spec& s = L.spec;
+    const int            K = s.dim + s.rot_dim, V = s.vdim;
+    return e->lm->elem == 2 && e->cfg.cache_block_seq_len == 64 && ((K == 64 && V == 64) || (K == 64 && V == 128) || (K == 128 && V == 128)) && s.dim % 8 == 0 && s.dim >= 8 && s.rot_dim % 8 == 0
+           && s.kv_rank % 8 == 0 && 2 * s.kv_rank + s.rot_dim > K + V;
+}
+
 // latent attention: the per-head expansions of the latent vector, and the rotation's frequencies
 static int process_latent_expansion(tm_engine* e, int i, LmLayer& L, int dt)
 {
@@ -236,6 +246,11 @@ static int process_latent_expansion(tm_engine* e, int i, LmLayer& L, int dt)
     std::vector<float> f(rd / 2);
     for (int j = 0; j < rd / 2; ++j) {
         f[j] = (float)std::pow((double)s.rot_base, -2.0 * j / rd);
+    }
+    if (latent_can_expand(e, L)) {
+        TM_TRY(dense_weight_alloc(L.ukv, C, H * (s.dim + s.vdim), dt, e->stream));
+        TM_TRY(place(e, L.ukv, 0, 0, lname(i, "mix.uk"), H * s.dim, C));
+        TM_TRY(place(e, L.ukv, H * s.dim, 0, lname(i, "mix.uv"), H * s.vdim, C));
     }
     return upload_f32(e, f, &L.inv_freq);
 }
@@ -747,7 +762,7 @@ int layered_process_weights(tm_engine* e)
         else if (L.src != i) {
             const LmLayer& S = lm.layers[L.src];
             L.qkv = S.qkv, L.up = S.up, L.out = S.out, L.norm1 = S.norm1, L.norm2 = S.norm2, L.sink = S.sink;
-            L.wo = S.wo, L.gu = S.gu, L.down = S.down, L.uk = S.uk, L.uv = S.uv;
+            L.wo = S.wo, L.gu = S.gu, L.down = S.down, L.uk = S.uk, L.uv = S.uv, L.ukv = S.ukv;
             L.r1 = S.r1, L.r2 = S.r2, L.rg1_b = S.rg1_b, L.rg2_b = S.rg2_b, L.c_norm = S.c_norm, L.inv_freq = S.inv_freq;
             L.w2 = S.w2, L.router = S.router, L.sh_up = S.sh_up, L.sh_down = S.sh_down, L.norm1_b = S.norm1_b, L.norm2_b = S.norm2_b;
             L.proj_bias = S.proj_bias, L.q_w = S.q_w, L.k_w = S.k_w, L.mix_norm = S.mix_norm, L.w0 = S.w0, L.act_par = S.act_par;
@@ -865,7 +880,7 @@ int layered_init_synthetic(tm_engine* e, uint64_t seed)
 static std::vector<DenseWeight*> dense_weights(LmLayer& L)
 {
     return {&L.qkv, &L.up, &L.out, &L.wo, &L.gu, &L.down, &L.uk, &L.uv, &L.w2, &L.router, &L.sh_up, &L.sh_down, &L.wo_r, &L.a2, &L.g2, &L.uq,
-            &L.side_gate, &L.side_proj, &L.sh_gu};
+            &L.side_gate, &L.side_proj, &L.sh_gu, &L.ukv};
 }
 
 template<class T>
@@ -1007,6 +1022,22 @@ int layered_start(tm_engine* e)
         TM_TRY(lm_alloc((char**)&lm.d_q, T * lm.ldq * lm.elem, st));
         TM_TRY(lm_alloc((char**)&lm.d_plain, T * lm.ldplain * lm.elem, st));
         TM_TRY(lm_alloc((char**)&lm.d_lat, T * lm.ldlat * lm.elem, st));
+        size_t entry = 0, up = 0, block = 0;
+        for (const LmLayer& L : lm.layers) {
+            const tm_layer_spec& s = L.spec;
+            if (s.mixer == TM_MIXER_LATENT && latent_can_expand(e, L)) {
+                entry = std::max(entry, (size_t)s.kv_rank + s.rot_dim);
+                up    = std::max(up, (size_t)s.heads * (s.dim + s.vdim));
+                block = std::max(block, (size_t)s.heads * 64 * (s.dim + s.rot_dim + s.vdim) * 2);
+            }
+        }
+        if (up > 0) {
+            lm.lde = ((int)entry + 31) / 32 * 32, lm.ldup = ((int)up + 31) / 32 * 32, lm.xstride = (int)(T / 64) + 1;
+            TM_TRY(lm_alloc((char**)&lm.d_entries, T * lm.lde * 2, st));
+            TM_TRY(lm_alloc((char**)&lm.d_up, T * lm.ldup * 2, st));
+            TM_TRY(lm_alloc(&lm.d_xblocks, (T / 64 + B) * block, st));
+            TM_TRY(lm_alloc(&lm.d_xtable, (size_t)B * lm.xstride, st));
+        }
         TM_TRY(lm_alloc((char**)&lm.d_ff, TT * lm.ldff * lm.elem, st));
         if (any_moe) {
             TM_TRY(lm_alloc((char**)&lm.d_moe_x, TT * lm.ldw * lm.elem, st));
@@ -1209,7 +1240,7 @@ void layered_free(tm_engine* e)
             (void)hipFree(p);
         }
     }
-    for (void* p : {(void*)lm.loop_step, (void*)lm.d_proj, (void*)lm.d_x0, (void*)lm.d_moe_y, (void*)lm.d_topk_w, lm.d_q, lm.d_plain, lm.d_lat,
+    for (void* p : {(void*)lm.loop_step, (void*)lm.d_proj, (void*)lm.d_x0, (void*)lm.d_moe_y, (void*)lm.d_topk_w, lm.d_q, lm.d_plain, lm.d_lat, lm.d_entries, lm.d_up, (void*)lm.d_xblocks, (void*)lm.d_xtable,
                     lm.d_ff, lm.d_xx, lm.d_moe_x, (void*)lm.d_topk_ids, (void*)lm.d_offsets, (void*)lm.d_f2n, (void*)lm.d_en2f}) {
         if (p) {
             (void)hipFree(p);
@@ -1329,12 +1360,59 @@ static LatentPrep latent_prep_args(tm_engine* e, const LmLayer& L, const LmPart&
     return a;
 }
 
+// Whether a latent layer's attention over this forward runs on expanded keys and values: whole prompts alone, with entries at hand that this layer or the one whose
+// entries it reads has left.  Against attention on the entries it costs the launch that lays keys and values out and saves as many multiply-adds a row in products as it takes; it is the
+// faster one from the shortest prompts on.  Eight layers of Sanozen, 2048 wide, 16 heads of 64 + 64 / 128 over entries of 192 + 64, ms, entries | expanded: 32 prompts of 33
+// 2.69 | 2.66, 8 of 128 2.47 | 2.44, 2 of 256 1.84 | 1.81, 8 of 512 5.66 | 5.56, 8 of 1024 9.70 | 9.28, 4 of 2040 10.18 | 9.62.  Later portions would have to expand all they follow
+static bool latent_expands(const tm_engine* e, const LmLayer& L, const LmPart* parts, int nparts)
+{
+    const LayeredModel& lm = *e->lm;
+    const int           li = (int)(&L - lm.layers.data()), from = L.pre && L.spec.kv_from >= 0 ? L.spec.kv_from : li;
+    return nparts == 1 && parts[0].whole && !parts[0].decode && L.ukv.w && lm.d_up && parts[0].nseq <= e->cfg.max_batch_size
+           && (from == li || lm.entries_of == from);
+}
+
+// queries [head][dim | rot_dim] side by side, and the entries as rows, for such a forward
+static void latent_prep_expanded(tm_engine* e, const LmLayer& L, LatentPrep& a)
+{
+    LayeredModel&        lm = *e->lm;
+    const tm_layer_spec& s  = L.spec;
+    a.q_plain = lm.d_q, a.ldp = lm.ldq, a.plain_stride = s.dim + s.rot_dim;
+    a.q_full = lm.d_q, a.full_stride = s.dim + s.rot_dim, a.full_off = s.dim;
+    if (a.dkv_col >= 0) {
+        a.entries = lm.d_entries, a.lde = lm.lde;
+        lm.entries_of = (int)(&L - lm.layers.data());
+    }
+}
+
+static int expanded_attention(tm_engine* e, const LmLayer& L, int M, const LmPart& P)
+{
+    LayeredModel&        lm = *e->lm;
+    const tm_layer_spec& s  = L.spec;
+    const int            K  = s.dim + s.rot_dim;
+    TM_PROF(P_GEMM_QKV, TM_TRY(launch_dense_call(L.ukv, lm.d_entries, lm.lde, lm.d_up, lm.ldup, M, DenseCall{}, e->stream)));
+    LatentExpand x;
+    x.up = lm.d_up, x.ldu = lm.ldup, x.entries = lm.d_entries, x.lde = lm.lde;
+    x.C = s.kv_rank, x.D = s.dim, x.R = s.rot_dim, x.V = s.vdim, x.heads = s.heads;
+    x.cu_q = P.cu_q, x.nseq = P.nseq, x.rows = P.rows, x.stride = lm.xstride, x.blocks = lm.d_xblocks, x.table = lm.d_xtable;
+    TM_PROF(P_KV_STORE, TM_TRY(launch_latent_expand(x, e->stream)));
+    GeneralAttnParams p = attn_params(e, L, P);
+    p.q = lm.d_q, p.out = lm.d_cat, p.ldo = lm.ldcat, p.out_head_stride = s.vdim;
+    p.seq_slot = nullptr, p.block_ptrs = lm.d_xtable, p.block_stride = lm.xstride, p.layer_offset = 0, p.v_offset = (int64_t)s.heads * 64 * K * 2;
+    p.q_heads = p.kv_heads = s.heads, p.k_heads = p.v_heads = 0, p.dim = K, p.vdim = s.vdim;
+    TM_PROF(P_ATTN, TM_TRY(launch_general_attention(p, true, e->stream)));
+    return 0;
+}
+
 // attention in the latent space once the prepare launch has split the queries: the key expansion carried to the queries, attention over
 // the cached latents, the value expansion of its output -> d_cat
 static int latent_attention(tm_engine* e, const LmLayer& L, int M, const LmPart* parts, int nparts)
 {
     LayeredModel&        lm = *e->lm;
     const tm_layer_spec& s  = L.spec;
+    if (latent_expands(e, L, parts, nparts)) {
+        return expanded_attention(e, L, M, parts[0]);
+    }
     DenseCall            c;
     c.count        = s.heads;
     c.x_col_stride = L.plain_stride;
@@ -1366,6 +1444,9 @@ static int wide_layer(tm_engine* e, const LmLayer& L, int M, const LmPart* parts
         if (latent) {
             LatentPrep a = latent_prep_args(e, L, P);
             a.dkv_col    = L.c_k;
+            if (latent_expands(e, L, parts, nparts)) {
+                latent_prep_expanded(e, L, a);
+            }
             TM_PROF(P_KV_STORE, TM_TRY(launch_latent_prep(proj, lm.ldproj, a, p, st)));
         }
         else {
@@ -1689,6 +1770,9 @@ static int pre_layer(tm_engine* e, int li, const LmLayer& L, const LmLayer* next
             LatentPrep              a = latent_prep_args(e, L, P);
             a.q_col   = uq ? -1 : 0;
             a.dkv_col = s.kv_from >= 0 ? -1 : L.c_k;
+            if (latent_expands(e, L, parts, nparts)) {
+                latent_prep_expanded(e, L, a);
+            }
             if (uq) {
                 a.q_rank = s.q_rank;
                 a.cq     = (char*)lm.d_cq + (size_t)P.row0 * lm.ldcq * lm.elem, a.ldcq = lm.ldcq;
@@ -1702,6 +1786,9 @@ static int pre_layer(tm_engine* e, int li, const LmLayer& L, const LmLayer* next
                 const GeneralAttnParams p = attn_params(e, L, P);
                 LatentPrep              a = latent_prep_args(e, L, P);
                 a.dkv_col = -1;
+                if (latent_expands(e, L, parts, nparts)) {
+                    latent_prep_expanded(e, L, a);
+                }
                 TM_PROF(P_KV_STORE, TM_TRY(launch_latent_prep(lm.d_proj + (size_t)P.row0 * lm.ldproj, lm.ldproj, a, p, st)));
             }
         }
@@ -1943,6 +2030,7 @@ static int layered_layers(tm_engine* e, const int* d_ids, int M, const LmPart* p
     const tm_layered_config& m  = lm.cfg;
     hipStream_t              st = e->stream;
     TM_REQUIRE(M >= 1 && M <= e->max_tokens, "forward: more rows than max_prefill_token_num");
+    lm.entries_of = -1;
     for (int i = 0; i < nparts && !begin.k_len; ++i) {
         const LmPart& P = parts[i];
         TM_TRY(launch_rows_prepare(lm.d_row_seq + P.row0, lm.d_row_pos + P.row0, P.cu_q, P.k_len, P.nseq, P.rows, st));
@@ -2089,7 +2177,7 @@ int layered_forward(tm_engine* e, const int* d_ids, int M, int nseq, bool decode
     }
     // (the decode step of continuous batching runs every slot: those without a running sequence are placeholders)
     parts[np++] = LmPart{nd, M - nd, nseq, e->d_cu_q, e->d_k_len, nullptr, e->d_block_ptrs, decode, decode ? 1 : max_q_len, slot0,
-                         decode && e->sched ? e->d_active : nullptr};
+                         decode && e->sched ? e->d_active : nullptr, !decode && e->prompts_whole};
     TM_TRY(layered_layers(e, d_ids, M, parts, np, ends ? ends->begin : StepBegin{}));
     if (decode) {
         return layered_head(e, lm.d_iota, nseq, slot0, d_ids, nullptr, M, e->d_k_len, nullptr, ends ? &ends->commit : nullptr);
@@ -2901,6 +2989,7 @@ int tm_engine_step_tokens(tm_engine* e, const tm_step_entry* entries, int n_entr
     }
     LmPart parts[2];
     int    np = 0;
+    bool   whole = true;
     if (n_dec > 0) {
         parts[np++] = LmPart{0, n_dec, n_dec, lm.d_step_cu_q, lm.d_step_k_len, lm.d_seq_slot, e->d_block_ptrs, true, 1};
     }
@@ -2908,6 +2997,10 @@ int tm_engine_step_tokens(tm_engine* e, const tm_step_entry* entries, int n_entr
         // the portions' description starts at entry n_dec: cu_q values count from row 0 of the forward, the part's rows from n_dec
         parts[np++] = LmPart{n_dec, total - n_dec, n_entries - n_dec, lm.d_step_cu_q + n_dec, lm.d_step_k_len + n_dec, lm.d_seq_slot + n_dec,
                              e->d_block_ptrs, false, max_q};
+        for (int i = n_dec; i < n_entries; ++i) {
+            whole = whole && k_len[i] == cu_q[i + 1] - cu_q[i];
+        }
+        parts[np - 1].whole = whole;
     }
     int rc = layered_layers(e, lm.d_step_ids, total, parts, np);
     for (size_t r0 = 0; rc == 0 && r0 < want.size(); r0 += lm.max_logit_rows) {

@@ -661,6 +661,7 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* __restric
     // the two channels of rotation i
     auto first  = [&](int i) { return a.rot_pairs ? 2 * i : i; };
     auto second = [&](int i) { return a.rot_pairs ? 2 * i + 1 : i + half; };
+    const int fs = a.full_stride > 0 ? a.full_stride : C + R, fo = a.full_stride > 0 ? a.full_off : C;
     // 1 / root mean square of x[col .. col + n) (every thread calls it)
     auto inv_rms = [&](int col, int n) {
         float ss = 0.f;
@@ -686,13 +687,13 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* __restric
             const float u = q[h * (D + R) + D + f0], v = q[h * (D + R) + D + f1];
             float       sn, cs;
             sincosf((float)pos * a.inv_freq[f], &sn, &cs);
-            T* o  = (T*)a.q_full + (size_t)t * a.ldq + (size_t)h * (C + R) + C;
+            T* o  = (T*)a.q_full + (size_t)t * a.ldq + (size_t)h * fs + fo;
             o[f0] = (T)(u * cs - v * sn);
             o[f1] = (T)(v * cs + u * sn);
         }
         for (int i = threadIdx.x; i < H * still; i += 256) {  // channels of the rotated part that do not turn
             const int h = i / still, f = rd + i % still;
-            ((T*)a.q_full)[(size_t)t * a.ldq + (size_t)h * (C + R) + C + f] = (T)q[h * (D + R) + D + f];
+            ((T*)a.q_full)[(size_t)t * a.ldq + (size_t)h * fs + fo + f] = (T)q[h * (D + R) + D + f];
         }
     }
     if (a.cq) {
@@ -707,12 +708,16 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* __restric
     char*        base = global_ptr(p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len]) + p.layer_offset;
     T*           k    = (T*)base + (size_t)ti * (C + R);
     T*           vt   = (T*)(base + p.v_offset) + ti;
+    T*           row  = a.entries ? (T*)a.entries + (size_t)t * a.lde : nullptr;
     const float* kv   = x + a.dkv_col;
     const float  inv  = inv_rms(a.dkv_col, C);
     for (int i = threadIdx.x; i < C; i += 256) {
         const T c = (T)(kv[i] * inv * a.c_norm_w[i]);
         k[i]                        = c;
         vt[(size_t)i * p.block_len] = c;
+        if (row) {
+            row[i] = c;
+        }
     }
     for (int f = threadIdx.x; f < half; f += 256) {
         const int   f0 = first(f), f1 = second(f);
@@ -721,10 +726,93 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* __restric
         sincosf((float)pos * a.inv_freq[f], &sn, &cs);
         k[C + f0] = (T)(u * cs - v * sn);
         k[C + f1] = (T)(v * cs + u * sn);
+        if (row) {
+            row[C + f0] = k[C + f0], row[C + f1] = k[C + f1];
+        }
     }
     for (int f = rd + threadIdx.x; f < R; f += 256) {
         k[C + f] = (T)kv[C + f];
+        if (row) {
+            row[C + f] = k[C + f];
+        }
     }
+}
+
+// grid (blocks, heads), 256 threads.  A prompt's blocks start at (its first row) / 64 + its number, which leaves room for every one before it.  Memory
+// bounds it: 8010 rows of 16 heads, 50 MB read and 67 written, 27 us
+template<int V>
+__global__ __launch_bounds__(256) void latent_expand_kernel(LatentExpand a)
+{
+    constexpr int kLd = V + 8;
+    __shared__ __attribute__((aligned(16))) __bf16 tile[64 * kLd];
+    typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+    const int        blk = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, row0 = a.cu_q[0];
+    int              lo = 0, hi = a.nseq - 1;  // the last prompt whose blocks start at or before this one
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if ((a.cu_q[mid] - row0) / 64 + mid <= blk) {
+            lo = mid;
+        }
+        else {
+            hi = mid - 1;
+        }
+    }
+    const int start = a.cu_q[lo] - row0, len = a.cu_q[lo + 1] - row0 - start, at = blk - (start / 64 + lo), n = min(64, len - at * 64);
+    if (n <= 0) {
+        return;
+    }
+    const int     K    = a.D + a.R;
+    const size_t  size = (size_t)a.heads * 64 * (K + V) * 2;
+    char* const   base = a.blocks + (size_t)blk * size;
+    __bf16* const keys = (__bf16*)base + (size_t)h * 64 * K;
+    __bf16* const vals = (__bf16*)base + (size_t)a.heads * 64 * K + (size_t)h * V * 64;
+    const __bf16* up   = (const __bf16*)a.up + (size_t)(start + at * 64) * a.ldu;
+    const __bf16* ent  = (const __bf16*)a.entries + (size_t)(start + at * 64) * a.lde + a.C;
+    if (h == 0 && tid == 0) {
+        a.table[(size_t)lo * a.stride + at] = (uint64_t)base;
+    }
+    const v4u zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = tid; i < 64 * V / 8; i += 256) {
+        const int t = i / (V / 8), c = i % (V / 8) * 8;
+        const v4u v = *(const v4u*)(up + (size_t)min(t, n - 1) * a.ldu + (size_t)a.heads * a.D + (size_t)h * V + c);
+        *(v4u*)(tile + t * kLd + c) = t < n ? v : zero;
+    }
+    const int pieces = K / 8, own = a.D / 8;
+    for (int i = tid; i < 64 * pieces; i += 256) {
+        const int t = i / pieces, c = i % pieces, tc = min(t, n - 1);
+        const v4u v = c < own ? *(const v4u*)(up + (size_t)tc * a.ldu + (size_t)h * a.D + c * 8) : *(const v4u*)(ent + (size_t)tc * a.lde + (c - own) * 8);
+        *(v4u*)(keys + (size_t)t * K + c * 8) = t < n ? v : zero;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = tid; i < V * 8; i += 256) {  // eight tokens of a channel
+        const int v = i % V, t0 = i / V * 8;
+        __bf16 __attribute__((aligned(16))) o[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            o[e] = tile[(t0 + e) * kLd + v];
+        }
+        *(v4u*)(vals + (size_t)v * 64 + t0) = *(const v4u*)o;
+    }
+}
+
+int launch_latent_expand(const LatentExpand& a, hipStream_t st)
+{
+    auto aligned = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+    TM_REQUIRE(a.up && a.entries && a.blocks && a.table && a.cu_q && a.nseq >= 1 && a.heads >= 1 && (a.V == 64 || a.V == 128), "latent_expand: operands");
+    TM_REQUIRE(a.C % 8 == 0 && a.D % 8 == 0 && a.R % 8 == 0 && a.D >= 8 && a.ldu % 8 == 0 && a.lde % 8 == 0 && a.ldu >= a.heads * (a.D + a.V) && a.lde >= a.C + a.R && aligned(a.up)
+                   && aligned(a.entries) && aligned(a.blocks),
+               "latent_expand: sizes");
+    const dim3 grid(a.rows / 64 + a.nseq, a.heads);
+    if (a.V == 64) {
+        latent_expand_kernel<64><<<grid, 256, 0, st>>>(a);
+    }
+    else {
+        latent_expand_kernel<128><<<grid, 256, 0, st>>>(a);
+    }
+    TM_HIP_CHECK(hipGetLastError());
+    return 0;
 }
 
 int launch_latent_prep(const float* proj, int ld, const LatentPrep& a, const GeneralAttnParams& p, hipStream_t st)

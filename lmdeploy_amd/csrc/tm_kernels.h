@@ -629,9 +629,24 @@ struct LatentPrep {
     const float *c_norm_w = nullptr, *inv_freq = nullptr, *cq_norm_w = nullptr;
     void *       q_plain = nullptr, *q_full = nullptr, *cq = nullptr;
     int          ldp = 0, plain_stride = 0, ldq = 0, ldcq = 0;
+    int          full_stride = 0, full_off = 0;  // head h's rotated channels start at h * full_stride + full_off of a q_full row (full_stride 0: C + R, C)
+    void*        entries = nullptr;              // != nullptr: the cache entries [C | R] as rows, too
+    int          lde = 0;
     float        eps = 0.f;
 };
 int launch_latent_prep(const float* proj, int ld, const LatentPrep& a, const GeneralAttnParams& layout, hipStream_t st);
+// Keys and values of every head, made from the latent entries of whole prompts, into blocks of 64 tokens laid out as a cache: keys [heads][64][D + R] (own channels from
+// `up`, the shared rotated ones from the entries), values transposed [heads][V][64], zero behind a prompt's end; and the block table [nseq][stride].
+// up [rows][ldu], bf16: head h's own channels at h * D, its values at heads * D + h * V.  blocks: rows / 64 + nseq of them
+struct LatentExpand {
+    const void *    up = nullptr, *entries = nullptr;
+    int             ldu = 0, lde = 0, C = 0, D = 0, R = 0, V = 0, heads = 0;
+    const int*      cu_q = nullptr;
+    int             nseq = 0, rows = 0, stride = 0;
+    char*           blocks = nullptr;
+    uint64_t*       table = nullptr;
+};
+int launch_latent_expand(const LatentExpand& a, hipStream_t st);
 // out[m] = [a[m] | b[m]] (a, b fp32 [M][H]) in bf16 | fp32
 int launch_concat2(void* out, int ldo, int out_elem_bytes, const float* a, const float* b, int M, int H, hipStream_t st);
 // mixture of experts on the fp32 stream: sigmoid router top-k from fp32 logits; gather (optionally scaled) rows in expert order; gated sum

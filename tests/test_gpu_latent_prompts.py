@@ -1,0 +1,46 @@
+"""GPU test of latent attention over whole prompts, whose keys and values every head makes of the latent entries: prompts around the blocks' borders side by side, layers that
+read another layer's entries, later portions and decoded tokens over the same cache (attention on the entries), and batches in which only some prompts are whole -- against the
+float64 oracle, the same bound as the other tests of the model."""
+import numpy as np
+import pytest
+
+from tests import sanozen_oracle as so
+from tests.test_gpu_sanozen import TOL, engine, model_folder, row_errs
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(3, 64, 64, 128, 192), (2, 32, 32, 64, 72), (5, 48, 16, 128, 96), (2, 120, 8, 128, 264)]  # heads, dim, rot_dim, vdim, kv_rank
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('H,D,R,V,C', SIZES)
+def test_whole_prompts_and_what_follows(cuda, tmp_path, H, D, R, V, C, dtype):
+    layers = [so.attention_layer(H, D, R, V, C, 40), so.hgrn2_layer(1, 8, 8), so.attention_layer(H + 1, D, R, V, C, 24, kv_from=0), so.attention_layer(H, D, R, V, C, 40),
+              so.attention_layer(1, D, R, V, C, 16, kv_from=0)]  # (the last reads entries that another layer has replaced)
+    cfg = so.make_config(56, 83, layers, side=4)
+    folder, w = model_folder(tmp_path, cfg, 5)
+    rng = np.random.default_rng(D)
+    eng = engine(folder, dtype, max_batch_size=8, max_prefill_token_num=1024, cache_blocks=40)
+    seqs = [rng.integers(0, 83, n).tolist() for n in (300, 2, 63, 64, 65, 320, 129)]
+    refs = [so.forward(cfg, w, s) for s in seqs]
+    cut = [300, 2, 63, 64, 65, 190, 0]                            # whole prompts; the last two go on
+    sess = [eng.open_session() for _ in seqs]
+    errs = []
+
+    def step(which, lo, hi):
+        got = eng.step_tokens([(sess[i], seqs[i][lo[i]:hi[i]], list(range(hi[i] - lo[i]))) for i in which])
+        at = 0
+        for i in which:
+            n = hi[i] - lo[i]
+            errs.append(row_errs(got[at:at + n], refs[i][lo[i]:hi[i]]))
+            at += n
+    step(range(6), [0] * 7, cut)
+    step([5, 6], cut, [0, 0, 0, 0, 0, 260, 129])                  # a later portion beside a whole prompt
+    for t in range(260, 264):
+        step([5], [t] * 7, [t + 1] * 7)
+    for s in sess:
+        eng.close_session(s)
+    eng.close()
+    errs = np.concatenate(errs)
+    # (as in the model's tests: a side vector next to zero, scaled up by the norm behind it, puts a row here and there off in bf16)
+    assert (errs > TOL[dtype]).sum() <= (len(errs) // 100 if dtype == 'bfloat16' else 0) and np.median(errs) <= TOL[dtype] / 4, np.sort(errs)[-8:]
