@@ -735,7 +735,7 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
     }
     if (p.tickets && ticket_last_workgroup(p.tickets + (size_t)t * p.q_heads + h0, nsplit, last_s)) {
         // The join of the splits (ga_merge), four channels a piece: everything that several splits have for all of a thread's pieces is asked for together.  Piece
-        // by piece, and a channel at a time, 16 heads of 192 took three trips to memory: three fp32 rows over ~180 entries, 21.0 us then, 14.7 now
+        // by piece, and a channel at a time, 16 heads of 192 took three trips to memory: three fp32 rows over ~180 entries, 21.0 us then, 14.1 now
         constexpr int kPieces = (VT * 64 + 255) / 256, kSplits = kPieces <= 2 ? 8 : 4;
         const int     pieces = V / 4, n = nh * pieces;
         if ((int)threadIdx.x >= n) {
@@ -1371,7 +1371,7 @@ int launch_general_attention_decode(const GeneralAttnParams& p, hipStream_t st)
 // attn_decode_kernel's arrangement for an fp32 cache, v_mfma_f32_16x16x4: workgroup per (row, 16 heads of a key head, key split), each wave 16 of a block's 64
 // keys.  S^T = K Q^T with the channels of a step dealt so that a lane's four are one load, and P^T then stands in the registers that O^T += V^T P^T reads.
 // What bounds it is a CU's load path -- the row kernel brings every key once per query head through it -- and at few rows the chain of dependent loads.
-// us, row kernel / this one: 16 / 1 heads of 256 / 192, 3 rows over ~180 tokens alone 21.0 / 15.1 (in a model, latency and all, 22.0 / 21.5), 2 rows over 2000 61.3 / 27.4, 420 rows
+// us, row kernel / this one: 16 / 1 heads of 256 / 192, 3 rows over ~180 tokens in a model 22.0 / 14.1; before this kernel's loads were in flight together, alone: 3 rows 21.0 / 15.1, 2 rows over 2000 61.3 / 27.4, 420 rows
 // of three prompts 148 / 31, a prompt of 2000 7165 / 597; 32 / 8 heads of 128 / 128 14.9 / 9.9, 44.2 / 19.3, 147 / 66, 7690 / 1915; 16 / 16 heads of 128 / 128, where
 // the tile holds one row of sixteen, 16.5 / 10.1, 56.8 / 22.1, 145 / 124, 10300 / 3850.  Where it loses: general_attention_heads_f32_pays.
 template<int DS, int VT>

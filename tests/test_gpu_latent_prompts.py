@@ -4,7 +4,9 @@ float64 oracle, the same bound as the other tests of the model."""
 import numpy as np
 import pytest
 
+from tests import bedenex_oracle as bo
 from tests import sanozen_oracle as so
+from tests import test_gpu_bedenex
 from tests.test_gpu_sanozen import TOL, engine, model_folder, row_errs
 
 pytestmark = pytest.mark.gpu
@@ -44,3 +46,19 @@ def test_whole_prompts_and_what_follows(cuda, tmp_path, H, D, R, V, C, dtype):
     errs = np.concatenate(errs)
     # (as in the model's tests: a side vector next to zero, scaled up by the norm behind it, puts a row here and there off in bf16)
     assert (errs > TOL[dtype]).sum() <= (len(errs) // 100 if dtype == 'bfloat16' else 0) and np.median(errs) <= TOL[dtype] / 4, np.sort(errs)[-8:]
+
+
+@pytest.mark.parametrize('kw', [{}, dict(loop=(0, 1, 2))])
+@pytest.mark.parametrize('D,R,V,C', [(64, 64, 128, 192), (32, 32, 64, 104), (48, 80, 128, 136)])
+def test_wide_blocks_and_runs_that_borrow_weights(cuda, tmp_path, D, R, V, C, kw):
+    cfg = bo.make_config(64, 97, [bo.latent_layer(3, D, R, V, C, (D + R) ** -0.5)], **kw)
+    folder, w = test_gpu_bedenex.model_folder(tmp_path, cfg, 3)
+    rng = np.random.default_rng(C)
+    eng = test_gpu_bedenex.engine(folder, 'bfloat16', max_batch_size=4, max_prefill_token_num=512, cache_blocks=24)
+    seqs = [rng.integers(0, 97, n).tolist() for n in (130, 64, 191)]
+    sess = [eng.open_session() for _ in seqs]
+    got = eng.step_tokens([(s, t, list(range(len(t)))) for s, t in zip(sess, seqs)])
+    for s in sess:
+        eng.close_session(s)
+    eng.close()
+    assert test_gpu_bedenex.rel_err(got, np.concatenate([bo.forward(cfg, w, t) for t in seqs])) <= test_gpu_bedenex.TOL['bfloat16']
