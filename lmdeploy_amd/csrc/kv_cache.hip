@@ -439,10 +439,10 @@ int launch_kv_store_general(const void* qkv, int ld, int k_col, int v_col, const
 // ([kv_heads][vdim]).  Queries go to q_out [rows][ldq] (head h at h * dim), keys / values into the cache in the general layout.
 template<class T>
 __global__ __launch_bounds__(256) void attn_prep_kernel(const float* __restrict__ proj, int ld, int q_col, int k_col, int v_col, T* __restrict__ q_out,
-                                                        int ldq, int qk_norm, int v_norm, float eps, GeneralAttnParams p, AttnPrepExtra ex)
+                                                        int ldq, int qk_norm, int v_norm, float eps, GeneralAttnParams p, AttnPrepExtra ex, int GV)
 {
     const int lane = threadIdx.x & 63, t = blockIdx.x, u = blockIdx.y * 4 + (threadIdx.x >> 6);
-    const int H = p.q_heads, G = p.k_heads > 0 ? p.k_heads : p.kv_heads, GV = p.v_heads > 0 ? p.v_heads : p.kv_heads;
+    const int H = p.q_heads, G = p.k_heads > 0 ? p.k_heads : p.kv_heads;
     if (u >= H + G + GV) {
         return;
     }
@@ -530,6 +530,30 @@ __global__ __launch_bounds__(256) void attn_prep_kernel(const float* __restrict_
     }
 }
 
+// Its values for many rows, which the cache holds channel by channel: a workgroup takes 64 rows x 64 channels, a lane is a row, so that a wave's stores of a channel are one
+// line (as kv_store_rows_kernel; by head vectors every two bytes of them are a line of their own).  7748 rows of 16 + 8 + 8 heads of 128: 184 us by head vectors, now 90 and 17
+template<class T>
+__global__ __launch_bounds__(256) void value_rows_kernel(const float* __restrict__ proj, int ld, int v_col, int nv, float mult, GeneralAttnParams p)
+{
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int it = threadIdx.x + i * 256, t = blockIdx.x * 64 + (it & 63), c = blockIdx.y * 64 + (it >> 6) * 8;
+        if (t >= p.rows || c >= nv) {
+            continue;
+        }
+        const float*  x = proj + (size_t)t * ld + v_col + c;
+        const floatx4 a = *(const floatx4*)x, b = *(const floatx4*)(x + 4);
+        const int     s = p.row_seq[t], pos = p.row_pos[t], g = c / p.vdim, d = c % p.vdim;
+        char* const   base = global_ptr(p.block_ptrs[(size_t)(p.seq_slot ? p.seq_slot[s] : s) * p.block_stride + pos / p.block_len]) + p.layer_offset;
+        T*            out  = (T*)(base + p.v_offset) + ((size_t)g * p.vdim + d) * p.block_len + pos % p.block_len;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            out[e * p.block_len]       = (T)(a[e] * mult);
+            out[(4 + e) * p.block_len] = (T)(b[e] * mult);
+        }
+    }
+}
+
 int launch_attn_prep(const float* proj, int ld, int q_col, int k_col, int v_col, void* q_out, int ldq, bool qk_norm, bool v_norm, float eps,
                      const GeneralAttnParams& p, hipStream_t st, AttnPrepExtra ex)
 {
@@ -542,12 +566,22 @@ int launch_attn_prep(const float* proj, int ld, int q_col, int k_col, int v_col,
     if (p.rows == 0) {
         return 0;
     }
-    const dim3 grid(p.rows, (p.q_heads + kh + vh + 3) / 4);
+    // prompts: neighbouring rows are neighbouring entries of a channel; decoded rows and prompts of a few tokens are not, and a launch more costs them some 4 us
+    // (pieces of eight channels lie in one head and start at multiples of 16 bytes; scaled values need their head's sum)
+    const bool apart = p.rows >= 64 && p.max_q_len >= 16 && !v_norm && !ex.conv_w && p.vdim % 8 == 0 && ld % 4 == 0 && v_col % 4 == 0 && (uintptr_t)proj % 16 == 0;
+    const int  own   = apart ? 0 : vh;  // value heads of the launch by head vectors
+    const dim3 grid(p.rows, (p.q_heads + kh + own + 3) / 4), rows((p.rows + 63) / 64, (vh * p.vdim + 63) / 64);
     if (p.elem_bytes == 2) {
-        attn_prep_kernel<__bf16><<<grid, 256, 0, st>>>(proj, ld, q_col, k_col, v_col, (__bf16*)q_out, ldq, qk_norm, v_norm, eps, p, ex);
+        attn_prep_kernel<__bf16><<<grid, 256, 0, st>>>(proj, ld, q_col, k_col, v_col, (__bf16*)q_out, ldq, qk_norm, v_norm, eps, p, ex, own);
+        if (apart) {
+            value_rows_kernel<__bf16><<<rows, 256, 0, st>>>(proj, ld, v_col, vh * p.vdim, ex.v_mult, p);
+        }
     }
     else {
-        attn_prep_kernel<float><<<grid, 256, 0, st>>>(proj, ld, q_col, k_col, v_col, (float*)q_out, ldq, qk_norm, v_norm, eps, p, ex);
+        attn_prep_kernel<float><<<grid, 256, 0, st>>>(proj, ld, q_col, k_col, v_col, (float*)q_out, ldq, qk_norm, v_norm, eps, p, ex, own);
+        if (apart) {
+            value_rows_kernel<float><<<rows, 256, 0, st>>>(proj, ld, v_col, vh * p.vdim, ex.v_mult, p);
+        }
     }
     TM_HIP_CHECK(hipGetLastError());
     return 0;
