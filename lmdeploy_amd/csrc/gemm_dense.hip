@@ -110,7 +110,7 @@ struct DenseEpi {
 
     static constexpr bool kPairs = EPI == kDenseGatedAct && sizeof(T) == 2;
     static constexpr bool kTileRuns = true;
-    // What an output needs besides its product: the stream's element, its bias, its gate, its row of a table.  Where a lane has many outputs their operands are
+    // What an output needs besides its product: the stream's element, its bias, its row of a table.  Where a lane has many outputs their operands are
     // asked for together (read), before the first of them is stored (join): a load that follows a store which may have written there waits in line, and a tile's 64
     // outputs a lane paid 64 trips to memory one after the other.  us, one by one / sixteen together: 8010 rows of bf16 into the stream, (2048, 2048) 104 / 85,
     // (8448, 2048) 275 / 253
