@@ -376,8 +376,8 @@ __global__ __launch_bounds__(768) void gemm_dec_lc_kernel(Dec32Params p)
                 }
             }
             else if (p.epilogue == 1) {
-                const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-                const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+                const float s0 = silu_f32(a[0]);
+                const float s1 = silu_f32(a[2]);
                 half2_t     o  = {(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
                 half2_t*    dst = (half2_t*)(p.y + (size_t)m * p.ldy + (n >> 1));
                 if (p.wt & 2) {

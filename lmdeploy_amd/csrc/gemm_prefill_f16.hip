@@ -239,8 +239,8 @@ __global__ __launch_bounds__(512) void gemm_f16_256_kernel(Dec32Params p)
                 const floatx4 a  = {acc[c][h][4 * g4], acc[c][h][4 * g4 + 1], acc[c][h][4 * g4 + 2], acc[c][h][4 * g4 + 3]};
                 const size_t  mg = (size_t)m0 + m;
                 if (p.epilogue == 1) {
-                    const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-                    const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+                    const float s0 = silu_f32(a[0]);
+                    const float s1 = silu_f32(a[2]);
                     half2_t     o  = {(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
                     *(half2_t*)(p.y + mg * p.ldy + (n >> 1)) = o;
                 }

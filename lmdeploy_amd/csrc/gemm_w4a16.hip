@@ -676,8 +676,8 @@ __global__ __launch_bounds__(WN * WK * 64) void gemm_kernel(GemmParams p)
                 *(floatx4*)(p.partial + ((size_t)blockIdx.y * p.M + m) * p.N + n) = a;
             }
             else if (p.epilogue == 1) {
-                const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-                const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+                const float s0 = silu_f32(a[0]);
+                const float s1 = silu_f32(a[2]);
                 half2_t     o  = {(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
                 *(half2_t*)(p.y + (size_t)m * p.ldy + (n >> 1)) = o;
             }
@@ -714,8 +714,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(half_t* __restrict__
         a += *(const floatx4*)(partial + ((size_t)s * M + m) * N + n);
     }
     if (gated) {
-        const float s0 = a[0] / (1.0f + __builtin_expf(-a[0]));
-        const float s1 = a[2] / (1.0f + __builtin_expf(-a[2]));
+        const float s0 = silu_f32(a[0]);
+        const float s1 = silu_f32(a[2]);
         half2_t     o  = {(half_t)(s0 * a[1]), (half_t)(s1 * a[3])};
         *(half2_t*)(y + (size_t)m * ldy + (n >> 1)) = o;
     }

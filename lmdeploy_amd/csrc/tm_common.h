@@ -50,16 +50,10 @@ __device__ __forceinline__ To bit_cast(const From& f)
     return __builtin_bit_cast(To, f);
 }
 
-// z / (1 + e^-z) in fp32, about 2 units in the last place: e^-z as 2^t with t's rounding error multiplied back in, the quotient by a reciprocal and one Newton step (a division
-// and a call of expf take 24 instructions and are most of a gated tile's epilogue)
+// z / (1 + e^-z) in fp32, the one silu of every product's epilogue: a call's numbers do not depend on which tile makes them
 __device__ __forceinline__ float silu_f32(float z)
 {
-    const float c = __builtin_amdgcn_fmed3f(z, -87.f, 104.f), t = c * -1.44269504f;  // (2^t stays finite; beyond, the quotient is z or less than 1e-35)
-    const float rest = __builtin_fmaf(c, -1.925963033e-8f, __builtin_fmaf(c, -1.44269504f, -t)) * 0.69314718f;
-    float       e    = __builtin_amdgcn_exp2f(t);
-    e                = __builtin_fmaf(e, rest, e);
-    const float d = 1.f + e, r = __builtin_amdgcn_rcpf(d);
-    return z * __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
+    return z / (1.0f + __builtin_expf(-z));
 }
 
 __device__ __forceinline__ half2_t h2_fma(half2_t a, half2_t b, half2_t c)

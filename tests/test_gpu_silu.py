@@ -1,10 +1,13 @@
-"""GPU test of silu(gate) * up as the gated products' epilogues make it (tm_silu_mul runs the same function): every fp16 gate against 64 bits"""
+"""GPU tests of silu(gate) * up as the gated products' epilogues make it (tm_silu_mul runs the same function): every fp16 gate against 64 bits, and in fp32 and bf16 gates
+that are far below zero, whose silu is zero whatever it is multiplied by"""
 import numpy as np
 import pytest
 import torch
 
 from lmdeploy_amd import _ffi
+from tests import bedenex_oracle as bo
 from tests.gpu_helpers import release_all, st
+from tests.test_gpu_bedenex import TOL, engine, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +37,25 @@ def test_every_gate(tm, cuda, up):
     unit = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(ref[ok]), 2.0 ** -14))) - 10)
     assert (np.abs(y[ok] - ref[ok]) <= (0.5 + 2.0 ** -9) * unit).all()
     assert y[np.isposinf(z)] == np.sign(up) * np.inf and not np.isfinite(y[np.isneginf(z)])
+
+
+@pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
+@pytest.mark.parametrize('rows', [2, 90])                   # products of few rows and tiles
+def test_gates_far_below_zero(cuda, tmp_path, dtype, rows):
+    """a gate of -64 ... -2^126 times an `up` of some 2^60 stays below 2^-20 of the stream; the model's other gates are ordinary"""
+    cfg = bo.make_config(64, 97, [bo.attention_layer(4, 1, 16, 32, 0.5, 33, bo.moe(1, 1, 96))])
+    w = bo.make_weights(cfg, 3)
+    w['embed'][:, 0], w['l0.norm1'][0], w['l0.mlp.router'][0] = 1.0, 1.0, 0.0     # every row's first channel is positive, its score 1/2
+    w['l0.mlp.e0.gate'][32:], w['l0.mlp.e0.up'][32:] = 0.0, w['l0.mlp.e0.up'][32:] * 2.0 ** 60
+    w['l0.mlp.e0.gate'][32:, 0] = -2.0 ** np.linspace(8, 127, 64).round()
+    folder = str(tmp_path / 'm')
+    bo.write_checkpoint(folder, cfg, w)
+    toks = np.random.default_rng(rows).integers(0, 97, rows)
+    with np.errstate(over='ignore'):
+        ref = bo.forward(cfg, w, toks)
+    eng = engine(folder, dtype)
+    s = eng.open_session()
+    got = eng.step_tokens([(s, toks, list(range(rows)))])
+    eng.close_session(s)
+    eng.close()
+    assert rel_err(got, ref) <= TOL[dtype]
