@@ -2922,6 +2922,7 @@ int tm_engine_step_tokens(tm_engine* e, const tm_step_entry* entries, int n_entr
         need += nb;
         total += en.n_tokens;
         n_dec += en.n_tokens == 1;
+        TM_REQUIRE(host_logits || en.n_want <= 0, "host_logits is null but logits are wanted");  // (nothing is refused once the sessions below have grown)
         for (int w = 0; w < en.n_want; ++w) {
             TM_REQUIRE(en.want && en.want[w] >= 0 && en.want[w] < en.n_tokens, "want: index outside the entry's tokens");
         }
@@ -2963,7 +2964,6 @@ int tm_engine_step_tokens(tm_engine* e, const tm_step_entry* entries, int n_entr
     for (int i = 0; i < n_entries; ++i) {
         want.insert(want.end(), want_rows[i].begin(), want_rows[i].end());
     }
-    TM_REQUIRE(host_logits || want.empty(), "host_logits is null but logits are wanted");
     hipStream_t st = e->stream;
     const int   B  = e->cfg.max_batch_size;
     std::copy(cu_q.begin(), cu_q.end(), lm.h_step);

@@ -1,8 +1,10 @@
 """GPU tests of recorded steps (step_tokens) of one token a session, which run as graphs from the second step of as many rows on: the same bits as launch by launch, over prompts,
-other numbers of rows, sessions that close and open, and steps that want other rows in between; contexts grow over the ends of cache blocks."""
+other numbers of rows, sessions that close and open, and steps that want other rows in between; contexts grow over the ends of cache blocks.  A step that is refused leaves no
+trace."""
 import numpy as np
 import pytest
 
+from lmdeploy_amd import _ffi
 from tests.gpu_helpers import release_all
 from tests.test_gpu_febivik import engine as febivik_engine
 from tests.test_gpu_febivik import full_model as febivik_model
@@ -65,3 +67,28 @@ def test_graphs_give_the_bits_of_launches(tmp_path, cuda, family, dtype):
     for other in rows[1:]:
         assert len(other) == len(rows[0]) and all(np.array_equal(x.view(np.uint32), y.view(np.uint32)) for x, y in zip(rows[0], other))
     assert all(np.isfinite(x).all() for x in rows[0]) and not np.array_equal(rows[0][1], rows[0][2])
+
+
+@pytest.mark.parametrize('graphs', [0, 1])
+@pytest.mark.parametrize('n', [1, 2, 70])
+def test_a_refused_step_leaves_its_sessions_as_they_were(tmp_path, cuda, n, graphs):
+    """logits are wanted and there is no place for them: the next step has the logits of a session that never saw the refusal (keys, values and states included)"""
+    cfg = sanozen_model()
+    folder, _ = sanozen_folder(tmp_path, cfg, 4)
+    eng = sanozen_engine(folder, 'float32', use_graph=graphs)
+    rng = np.random.default_rng(n)
+    first, other = rng.integers(0, cfg['vocab'], (2, 20)).astype(np.int32)
+    refused, then = rng.integers(0, cfg['vocab'], (2, n)).astype(np.int32)
+    want = np.array([n - 1], np.int32)
+    out = []
+    for refuse in (False, True, False, True):
+        a, b = eng.open_session(), eng.open_session()
+        eng.step_tokens([(a, first, []), (b, other, [])])
+        if refuse:
+            entries = (_ffi.StepEntry * 2)(_ffi.StepEntry(b, other.ctypes.data, 1, None, 0), _ffi.StepEntry(a, refused.ctypes.data, n, want.ctypes.data, 1))
+            assert eng._lib.tm_engine_step_tokens(eng._h, entries, 2, None) == 1      # TM_INVALID
+        out.append(np.concatenate([eng.step_tokens([(a, then, [n - 1]), (b, other[:1], [0])]) for _ in range(3)]))
+        eng.close_session(a)
+        eng.close_session(b)
+    eng.close()
+    assert all(np.array_equal(out[0].view(np.uint32), o.view(np.uint32)) for o in out[1:])
