@@ -4,6 +4,7 @@
 #pragma once
 #include "../../include/tm_mi355x.h"
 #include "scheduler.h"
+#include "step_graphs.h"
 #include "tm_common.h"
 #include "tm_kernels.h"
 #include <algorithm>
@@ -192,13 +193,9 @@ struct LayeredModel {
     int *                d_step_ids = nullptr, *d_step_cu_q = nullptr, *d_step_k_len = nullptr;
     // a recorded step's description, [cu_q][k_len][slots][ids] in one allocation, and where the host writes it (pinned)
     int *                d_step = nullptr, *h_step = nullptr;
-    // recorded steps of one token a session, as graphs: one for a number of rows (and whether their logits are wanted), from its second step on
-    struct RecordedStep {
-        int            rows = 0, want = 0, seen = 0;
-        hipGraphExec_t graph = nullptr;
-    };
-    std::vector<RecordedStep> recorded;
-    const RecordedStep*       recording = nullptr;  // what recorded_step() captures
+    // recorded steps of one token a session, as graphs
+    StepGraphs<hipGraphExec_t> recorded{32};
+    int                        recorded_rows = 0, recorded_want = 0;  // what recorded_step() runs
     float*               d_attn_ws = nullptr;
     unsigned*            d_attn_tickets = nullptr;  // [max rows][max heads], zero between launches
     int                  n_attn_tickets = 0;

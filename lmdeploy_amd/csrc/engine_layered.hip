@@ -1196,23 +1196,13 @@ int layered_start(tm_engine* e)
     return 0;
 }
 
-static void recorded_free(LayeredModel& lm)
-{
-    for (auto& r : lm.recorded) {
-        if (r.graph) {
-            (void)hipGraphExecDestroy(r.graph);
-        }
-    }
-    lm.recorded.clear();
-}
-
 void layered_free(tm_engine* e)
 {
     if (!e->lm) {
         return;
     }
     LayeredModel& lm = *e->lm;
-    recorded_free(lm);
+    lm.recorded.clear([](hipGraphExec_t g) { (void)hipGraphExecDestroy(g); });
     if (lm.h_step) {
         (void)hipHostFree(lm.h_step);
     }
@@ -2237,42 +2227,32 @@ static int validate_both_layer(const tm_layered_config* m, int i)
 static int recorded_step(tm_engine* e)
 {
     LayeredModel& lm = *e->lm;
-    const int     n  = lm.recording->rows;
+    const int     n  = lm.recorded_rows;
     const LmPart  part{0, n, n, lm.d_step_cu_q, lm.d_step_k_len, lm.d_seq_slot, e->d_block_ptrs, true, 1};
     TM_TRY(layered_layers(e, lm.d_step_ids, n, &part, 1));
-    return lm.recording->want ? layered_logits(e, lm.d_iota, n) : 0;
+    return lm.recorded_want ? layered_logits(e, lm.d_iota, n) : 0;
 }
 
-// Runs such a step: some 120 launches, which leave the host more slowly than small models run them, so from its second time on a step of as many rows is a graph.
-// What it reads -- tokens, positions, slots, the block table -- lies where every step writes it.  Three rows of Sanozen in fp32, 2048 wide, a
-// prompt and 12 steps: 13.4 -> 12.6 ms
+// Runs such a step, as a graph where it can.  What it reads -- tokens, positions, slots, the block table -- lies where every step writes it.  Three rows of Sanozen in fp32,
+// 2048 wide, a prompt and 12 steps: 13.4 -> 12.6 ms
 static int run_recorded_step(tm_engine* e, int rows, int want)
 {
     LayeredModel& lm = *e->lm;
-    size_t        i  = 0;
-    while (i < lm.recorded.size() && (lm.recorded[i].rows != rows || lm.recorded[i].want != want)) {
-        ++i;
-    }
-    if (i == lm.recorded.size()) {
-        if (i >= 32) {  // (every step ends with a synchronisation: none of them is running)
-            recorded_free(lm);
-            i = 0;
-        }
-        LayeredModel::RecordedStep r;
-        r.rows = rows, r.want = want;
-        lm.recorded.push_back(r);
-    }
-    LayeredModel::RecordedStep& r = lm.recorded[i];
-    lm.recording                  = &r;
-    const bool graphs = graph_enabled(e) && lm.debug_layers < 0 && !e->prof_on;
-    if (graphs && ++r.seen == 2) {  // (the first, launch by launch, has loaded every kernel)
-        TM_TRY(capture_step(e, recorded_step, &r.graph));
-    }
-    if (graphs && r.graph) {
-        TM_HIP_CHECK(hipGraphLaunch(r.graph, e->stream));
-        return 0;
-    }
-    return recorded_step(e);
+    lm.recorded_rows = rows, lm.recorded_want = want;
+    return lm.recorded.run(
+        rows, want, graph_enabled(e) && lm.debug_layers < 0 && !e->prof_on, [&] { return recorded_step(e); },
+        [&](hipGraphExec_t* g) {
+            const int rc = capture_step(e, recorded_step, g);
+            if (rc) {  // (the sessions have advanced: the step has to run all the same)
+                (void)hipGetLastError();
+            }
+            return rc;
+        },
+        [&](hipGraphExec_t g) {
+            TM_HIP_CHECK(hipGraphLaunch(g, e->stream));
+            return 0;
+        },
+        [](hipGraphExec_t g) { (void)hipGraphExecDestroy(g); });
 }
 
 }  // namespace tmk

@@ -1,0 +1,70 @@
+// CPU-only harness for lmdeploy_amd/csrc/step_graphs.h: which steps run as graphs, counted with a stand-in for a graph.  Built and run by
+// tests/test_step_graphs.py.
+#include "../../lmdeploy_amd/csrc/step_graphs.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <set>
+
+using namespace tmk;
+
+#define CHECK(c)                                                                     \
+    do {                                                                             \
+        if (!(c)) {                                                                  \
+            std::fprintf(stderr, "%s:%d: CHECK(%s) failed\n", __FILE__, __LINE__, #c); \
+            std::exit(1);                                                            \
+        }                                                                            \
+    } while (0)
+
+struct Counts {
+    int           launches = 0, captures = 0, replays = 0, made = 0;
+    bool          fails = false;
+    std::set<int> live;
+};
+
+static int step(StepGraphs<int>& g, Counts& c, int rows, int want = 1, bool on = true)
+{
+    return g.run(
+        rows, want, on, [&] { return ++c.launches, 0; },
+        [&](int* graph) {
+            ++c.captures;
+            if (c.fails) {
+                *graph = 99;  // (whatever a failed call leaves)
+                return 3;
+            }
+            c.live.insert(*graph = ++c.made);
+            return 0;
+        },
+        [&](int graph) {
+            CHECK(c.live.count(graph));
+            return ++c.replays, 0;
+        },
+        [&](int graph) { CHECK(c.live.erase(graph) == 1); });
+}
+
+int main()
+{
+    {  // the first by launches, the others as a graph; logits wanted or not are steps of their own
+        StepGraphs<int> g(4);
+        Counts          c;
+        for (int i = 0; i < 5; ++i) {
+            CHECK(step(g, c, 3) == 0 && step(g, c, 3, 0) == 0);
+        }
+        CHECK(c.launches == 2 && c.captures == 2 && c.replays == 8 && c.live.size() == 2);
+        CHECK(step(g, c, 3, 1, false) == 0 && c.launches == 3);  // not in use: by launches
+        g.clear([&](int graph) { CHECK(c.live.erase(graph) == 1); });
+        CHECK(c.live.empty() && g.size() == 0);
+    }
+    {  // a step that cannot be captured runs, and is not tried again
+        StepGraphs<int> g(4);
+        Counts          c;
+        c.fails = true;
+        for (int i = 0; i < 5; ++i) {
+            CHECK(step(g, c, 7) == 0);
+        }
+        CHECK(c.launches == 5 && c.captures == 1 && c.replays == 0);
+        g.clear([&](int) { CHECK(false); });
+    }
+    std::puts("ok");
+    return 0;
+}
