@@ -194,7 +194,7 @@ struct LayeredModel {
     // a recorded step's description, [cu_q][k_len][slots][ids] in one allocation, and where the host writes it (pinned)
     int *                d_step = nullptr, *h_step = nullptr;
     // recorded steps of one token a session, as graphs
-    StepGraphs<hipGraphExec_t> recorded{32};
+    StepGraphs<hipGraphExec_t> recorded;
     int                        recorded_rows = 0, recorded_want = 0;  // what recorded_step() runs
     float*               d_attn_ws = nullptr;
     unsigned*            d_attn_tickets = nullptr;  // [max rows][max heads], zero between launches

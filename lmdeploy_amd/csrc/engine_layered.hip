@@ -1142,6 +1142,7 @@ int layered_start(tm_engine* e)
     TM_TRY(lm_alloc(&lm.d_step, 3 * (size_t)B + 1 + T, st));
     TM_HIP_CHECK(hipHostMalloc((void**)&lm.h_step, (3 * (size_t)B + 1 + T) * 4, hipHostMallocDefault));
     lm.d_step_cu_q = lm.d_step, lm.d_step_k_len = lm.d_step + B + 1, lm.d_seq_slot = lm.d_step_k_len + B, lm.d_step_ids = lm.d_seq_slot + B;
+    lm.recorded.set_slots(B);
     iota_kernel<<<(T + 255) / 256, 256, 0, st>>>(lm.d_iota, (int)T);
     TM_HIP_CHECK(hipGetLastError());
     // decode rows split their keys so that a few long sequences still fill the device: >= 4 cache blocks per split at full length

@@ -1,8 +1,10 @@
 // Which recorded steps run as graphs (host only, no device code, so that it can be driven from a CPU test).
 //
 // A step of one token a session is some 120 launches, which leave the host more slowly than small models run them: from its second time on a step of as many rows is one
-// graph launch.  The first, launch by launch, has loaded every kernel.
+// graph launch.  The first, launch by launch, has loaded every kernel.  Where all places are taken the step that has not come for the longest time gives up its own: emptied as a
+// whole, the places of a course that goes round among more numbers of rows than there are places never came to be used.
 #pragma once
+#include <algorithm>
 #include <cstddef>
 #include <vector>
 
@@ -11,14 +13,19 @@ namespace tmk {
 template<class Graph>
 class StepGraphs {
     struct Step {
-        int   rows, want, seen;
-        Graph graph;
+        int    rows, want, seen;
+        size_t used;
+        Graph  graph;
     };
     std::vector<Step> steps_;
-    size_t            most_;
+    size_t            most_ = 32, now_ = 0;
 
 public:
-    explicit StepGraphs(size_t most): most_(most) {}
+    // places for `slots` sessions: every number of rows with and without logits, up to 256 (a graph of 120 launches takes some 15 KB of host memory and 0.2 ms to make)
+    void set_slots(int slots)
+    {
+        most_ = std::min<size_t>(2 * (size_t)std::max(slots, 1), 256);
+    }
     size_t size() const
     {
         return steps_.size();
@@ -36,13 +43,19 @@ public:
             ++i;
         }
         if (i == steps_.size()) {
-            if (i >= most_) {
-                clear(destroy);
-                i = 0;
+            if (i < most_) {
+                steps_.push_back(Step{});
             }
-            steps_.push_back(Step{rows, want, 0, Graph{}});
+            else {
+                i = std::min_element(steps_.begin(), steps_.end(), [](const Step& a, const Step& b) { return a.used < b.used; }) - steps_.begin();
+                if (steps_[i].graph) {
+                    destroy(steps_[i].graph);
+                }
+            }
+            steps_[i] = Step{rows, want, 0, 0, Graph{}};
         }
         Step& s = steps_[i];
+        s.used  = ++now_;
         if (s.seen < 2 && ++s.seen == 2 && capture(&s.graph) != 0) {
             s.graph = Graph{};
         }

@@ -69,6 +69,25 @@ def test_graphs_give_the_bits_of_launches(tmp_path, cuda, family, dtype):
     assert all(np.isfinite(x).all() for x in rows[0]) and not np.array_equal(rows[0][1], rows[0][2])
 
 
+def test_as_many_graphs_as_numbers_of_rows(tmp_path, cuda):
+    """sessions that pause and go on: 20 numbers of rows, with and without logits, three times round, against launch by launch"""
+    cfg = sanozen_model()
+    folder, _ = sanozen_folder(tmp_path, cfg, 6)
+    rows = []
+    for graphs in (0, 1):
+        eng = sanozen_engine(folder, 'float32', use_graph=graphs, max_batch_size=20, cache_blocks=60)
+        rng = np.random.default_rng(8)
+        sess, out = [eng.open_session() for _ in range(20)], []
+        eng.step_tokens([(s, rng.integers(0, cfg['vocab'], 3 + i), []) for i, s in enumerate(sess)])
+        for _ in range(3):
+            for n in range(20, 0, -1):
+                for want in ([0], []):
+                    out.append(eng.step_tokens([(s, rng.integers(0, cfg['vocab'], 1), want) for s in sess[:n]]).copy())
+        rows.append(np.concatenate(out))
+        eng.close()
+    assert np.array_equal(rows[0].view(np.uint32), rows[1].view(np.uint32)) and np.isfinite(rows[0]).all()
+
+
 @pytest.mark.parametrize('graphs', [0, 1])
 @pytest.mark.parametrize('n', [1, 2, 70])
 def test_a_refused_step_leaves_its_sessions_as_they_were(tmp_path, cuda, n, graphs):
