@@ -160,10 +160,10 @@ static int plain_up_col(const LmLayer& L)
 }
 
 // Bytes of the projections and the head, each as an image of its own (columns rounded up to 128): neither what lies between tiles that stand apart in memory nor the
-// columns between the two parts of a fused image.  fp32 engines count their parameters in fp32, though the images hold the bf16 numbers that they are
+// columns between the two parts of a fused image.  Two bytes an element in either type: fp32 engines hold the bf16 numbers of their checkpoint
 int64_t layered_weight_bytes(const tm_engine* e)
 {
-    auto bytes = [](const DenseWeight& d, int gap) { return (int64_t)d.Kp * (d.Np - gap) * d.count * (d.dtype == kDenseF32 ? 4 : 2); };
+    auto bytes = [](const DenseWeight& d, int gap) { return (int64_t)d.Kp * (d.Np - gap) * d.count * 2; };
     int64_t n  = bytes(e->lm->head, 0);
     for (size_t i = 0; i < e->lm->layers.size(); ++i) {
         const LmLayer& L = e->lm->layers[i];

@@ -64,9 +64,9 @@ def test_decode_rows_around_the_line(cuda, n, dtype):
 
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
 def test_weight_bytes(cuda, dtype):
-    """the reported bytes are those of the weights (columns in whole groups of 128), not of the memory between tiles or between the parts of the fused product"""
+    """the reported bytes are those of the weights (columns in whole groups of 128, bf16 in either type), not of the memory between tiles or between the parts of the fused product"""
     cfg = lo.make_config(2048, 203, [_layer(dim=8, vdim=8, ff=24)])
     eng = engine_for(cfg, lo.make_weights(cfg, 0), dtype)
     # [q | k | v], up: 2048 to 64 and 24 columns; [o | down]: 32 + 24 to 2048; head
-    assert eng.stats()['weight_bytes'] == (2 if dtype == 'bfloat16' else 4) * (2048 * (128 + 128) + 64 * 2048 + 2048 * 256)
+    assert eng.stats()['weight_bytes'] == 2 * (2048 * (128 + 128) + 64 * 2048 + 2048 * 256)
     eng.close()
