@@ -670,6 +670,9 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
     const int  lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4, V = p.vdim;
     const bool h_ok = lr < nh;
     const int  h    = h0 + (h_ok ? lr : 0);
+    const size_t slots  = (size_t)p.q_heads * p.splits;  // of row t
+    const auto   row_o  = agent_base(p.partial_o + t * slots * V, slots * V * 4);
+    const auto   row_ml = agent_base(p.partial_ml + t * slots * 2, slots * 8);
     if (lg == 0) {
         ml_s[wave][lr][0] = m;
         ml_s[wave][lr][1] = l;
@@ -719,13 +722,12 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
             }
             return;
         }
-        float* po = p.partial_o + (((size_t)t * p.q_heads + h) * p.splits + sp) * V;
         float* pm = p.partial_ml + (((size_t)t * p.q_heads + h) * p.splits + sp) * 2;
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
             const int c = v * 16 + lg * 4;
             if (h_ok && c < V) {
-                agent_store4(po + c, o[v]);
+                agent_store4(row_o, ((h * p.splits + sp) * V + c) * 4, o[v]);
             }
         }
         if (h_ok && lg == 0) {
@@ -752,16 +754,16 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
             oo[i] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
         for (int s0 = 0; s0 < nsplit; s0 += kSplits) {
-            floatx2 ml[kPieces][kSplits], ov[kPieces][kSplits][2];
+            floatx2 ml[kPieces][kSplits];
+            floatx4 ov[kPieces][kSplits];
 #pragma unroll
             for (int i = 0; i < kPieces; ++i) {
                 if (i * 256 < n) {
 #pragma unroll
                     for (int k = 0; k < kSplits; ++k) {
-                        const size_t slot = ((size_t)t * p.q_heads + head[i]) * p.splits + min(s0 + k, nsplit - 1);
-                        ml[i][k]          = agent_load2(p.partial_ml + slot * 2);
-                        ov[i][k][0]       = agent_load2(p.partial_o + slot * V + c0[i]);
-                        ov[i][k][1]       = agent_load2(p.partial_o + slot * V + c0[i] + 2);
+                        const int slot = head[i] * p.splits + min(s0 + k, nsplit - 1);
+                        ml[i][k]       = agent_load2(row_ml, slot * 8);
+                        ov[i][k]       = agent_load4(row_o, (slot * V + c0[i]) * 4);
                     }
                 }
             }
@@ -780,8 +782,10 @@ __device__ __forceinline__ void ga_close_heads(const GeneralAttnParams& p, int t
                     for (int k = 0; k < kSplits; ++k) {
                         const float ak = s0 + k < nsplit ? fast_exp2((ml[i][k][0] - mn) * kLog2e) : 0.f;
                         ll[i]          = fmaf(ak, ml[i][k][1], ll[i]);
-                        oo[i][0] = fmaf(ak, ov[i][k][0][0], oo[i][0]), oo[i][1] = fmaf(ak, ov[i][k][0][1], oo[i][1]);
-                        oo[i][2] = fmaf(ak, ov[i][k][1][0], oo[i][2]), oo[i][3] = fmaf(ak, ov[i][k][1][1], oo[i][3]);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            oo[i][c] = fmaf(ak, ov[i][k][c], oo[i][c]);
+                        }
                     }
                     mm[i] = mn;
                 }

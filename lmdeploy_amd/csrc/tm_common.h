@@ -156,15 +156,26 @@ __device__ __forceinline__ float agent_load(const float* p)
 {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// four neighbours, two at a time
-__device__ __forceinline__ void agent_store4(float* p, floatx4 v)
+// The same for several neighbours, at `at` bytes behind a base that all lanes share (agent_base: its first `bytes` bytes): buffer instructions with the agent's scope (sc1),
+// which need no more than the four-byte alignment of a float
+__device__ __forceinline__ auto agent_base(const float* base, size_t bytes)
 {
-    __hip_atomic_store((uint64_t*)p, bit_cast<uint64_t>(floatx2{v[0], v[1]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store((uint64_t*)p + 1, bit_cast<uint64_t>(floatx2{v[2], v[3]}), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ floatx2 agent_load2(const float* p)
+template<class Base>
+__device__ __forceinline__ void agent_store4(Base base, int at, floatx4 v)
 {
-    return bit_cast<floatx2>(__hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    __builtin_amdgcn_raw_buffer_store_b128(bit_cast<u32x4>(v), base, at, 0, /*sc1*/ 16);
+}
+template<class Base>
+__device__ __forceinline__ floatx4 agent_load4(Base base, int at)
+{
+    return bit_cast<floatx4>(__builtin_amdgcn_raw_buffer_load_b128(base, at, 0, /*sc1*/ 16));
+}
+template<class Base>
+__device__ __forceinline__ floatx2 agent_load2(Base base, int at)
+{
+    return bit_cast<floatx2>(__builtin_amdgcn_raw_buffer_load_b64(base, at, 0, /*sc1*/ 16));
 }
 // of n arrivals: is this the last one (which also clears the ticket)?  One lane calls it after the stores are drained
 __device__ __forceinline__ bool ticket_last(unsigned* ticket, int n)
