@@ -34,11 +34,19 @@ struct StreamOp<half_t> {
 // fp32 rows: 24 bits of significand are three times the eight of bf16, so x = high + middle + low exactly (each part the rest's leading bits, cut off; a part that
 // underflows is below 2^-126), and a product of two bf16 numbers is exact in fp32: three bf16 matrix instructions multiply as exactly as fp32 ones do, in 48
 // cycles instead of 256.  They cut the sum off where v_mfma_f32_16x16x4 rounds it, so sums of one sign would drift: every kSplitSteps steps begin at zero and are
-// added to the others in fp32, and few rows sum the low and middle parts apart from the high ones.  What remains of an infinity after its leading part is zero, not a NaN.
+// added to the others in fp32, and few rows sum the low and middle parts apart from the high ones.  What remains of an infinity after its leading part is what remains of the
+// largest number, and a NaN whose leading half is that of an infinity (its payload in the lower one) is a NaN in the middle part: the median of three numbers is the least of
+// them where one is a NaN, and a signalling NaN where that comes last.
 struct SplitRow {
     u32x4 part[3];  // low, middle, high
 };
-__device__ __forceinline__ SplitRow stream_split(u32x4 a, u32x4 b)
+__device__ __forceinline__ float stream_most()
+{
+    float most = 3.402823466e38f;
+    asm("" : "+s"(most));  // (the compiler may not know the value: it puts constants last.  Once a kernel: once a split, it moved the splits of the 128 x 128 tile behind their barrier, 7 %)
+    return most;
+}
+__device__ __forceinline__ SplitRow stream_split(u32x4 a, u32x4 b, float most)
 {
     SplitRow o;
 #pragma unroll
@@ -49,8 +57,10 @@ __device__ __forceinline__ SplitRow stream_split(u32x4 a, u32x4 b)
             o.part[p][i] = __builtin_amdgcn_perm(bit_cast<uint32_t>(r[1]), bit_cast<uint32_t>(r[0]), 0x07060302);  // both leading halves
 #pragma unroll
             for (int e = 0; p > 0 && e < 2; ++e) {
-                const float rest = r[e] - bit_cast<float>(bit_cast<uint32_t>(r[e]) & 0xffff0000u);
-                r[e]             = p == 2 ? __builtin_amdgcn_fmed3f(rest, rest, 0.f) : rest;  // (the median with a NaN is the smallest of the others)
+                if (p == 2) {
+                    r[e] = __builtin_amdgcn_fmed3f(most, -most, r[e]);
+                }
+                r[e] -= bit_cast<float>(bit_cast<uint32_t>(r[e]) & 0xffff0000u);
             }
         }
     }
@@ -153,6 +163,7 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
     for (int j = 0; j < NT; ++j) {
         wp[j] = w + (int64_t)min(tile0 + j, a.tiles - 1) * a.w_tile;
     }
+    const float most = stream_most();
     const int turn = stream_turn(tile0, a.steps);
     u32x4     wa[kChunk][NT], wb[kChunk][NT], xr[kXPer][kRaw];
     auto  fetch = [&](u32x4(&buf)[kChunk][NT], int base) {
@@ -189,7 +200,7 @@ __global__ __launch_bounds__(CW* KP * 64) void stream_skinny_kernel(StreamArgs a
                 const int   c = v & 7, r = (v >> 3) & 15, blk = v >> 7;
                 char* const at = smem + buf * kStage + blk * 2048 + r * 128 + ((c ^ (r & 7)) << 4);
                 if constexpr (kParts > 1) {
-                    const SplitRow f = stream_split(xr[i][0], xr[i][1]);
+                    const SplitRow f = stream_split(xr[i][0], xr[i][1], most);
 #pragma unroll
                     for (int p = 0; p < kParts; ++p) {
                         *(u32x4*)(at + p * kXVecs * 16) = f.part[p];
@@ -457,6 +468,7 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
     // wait for the next chunk's weights (fp16, 8 rows: (2048, 4096) 5.9 -> 5.4 us, (2048, 2048) 5.1 -> 4.8; bf16, 17
     // rows, (4096, 4096) 11.9 -> 10.8).  More rows take more registers for it than they leave for weights: x there | where it is used, 64 rows: bf16 (2048, 2048)
     // 11.8 | 11.4 us
+    const float most = stream_most();
     const int turn = stream_turn(tile0, a.steps);
     struct Raw {
         u32x4 h[kRaw];
@@ -525,7 +537,7 @@ __global__ __launch_bounds__(W * 64) void stream_narrow_kernel(StreamArgs a, Epi
                     }
                     SplitRow f;
                     if constexpr (kParts > 1) {
-                        f = stream_split(b.h[0], b.h[1]);
+                        f = stream_split(b.h[0], b.h[1], most);
                     }
                     else {
                         f.part[0] = b.h[0];
@@ -863,6 +875,7 @@ __global__ __launch_bounds__(256 * KP, KP == 1 ? 2 : 4) void stream_tile_split_k
             stream_dma16(rs_w, woff[r], ws, dst + kXB + (kWP * wave + r) * 1024);
         }
     };
+    const float most = stream_most();
     floatx4 acc[MI][NI], sum[MI][NI];
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
@@ -917,7 +930,7 @@ __global__ __launch_bounds__(256 * KP, KP == 1 ? 2 : 4) void stream_tile_split_k
         }
 #pragma unroll
         for (int i = 0; i < MI; ++i) {
-            const SplitRow f = stream_split(fx[q][i][0], fx[q][i][1]);
+            const SplitRow f = stream_split(fx[q][i][0], fx[q][i][1], most);
 #pragma unroll
             for (int p = 0; p < 3; ++p) {
 #pragma unroll

@@ -77,6 +77,22 @@ def test_rows_that_are_not_finite(tm, cuda, K, N, M):
     assert float((product(tm, w, x).double() / ref - 1).abs().max()) <= (72 + K / 256) * 2.0 ** -24
 
 
+@pytest.mark.parametrize('K,N,M', [(96, 200, 3), (520, 260, 20), (520, 260, 40), (520, 1000, 300), (1024, 4100, 2500)])
+@pytest.mark.parametrize('bits', [0x7F800001, -0x7FFFFF, 0x7F80FFFF, 0x7FC00000])
+def test_every_nan_is_one(tm, cuda, K, N, M, bits):
+    """also those whose payload the leading bf16 part does not hold"""
+    g = torch.Generator('cuda').manual_seed(M)
+    w = torch.randn(N, K, generator=g, device='cuda').bfloat16()
+    x = torch.zeros(M, (K + 31) // 32 * 32, device='cuda')
+    x[:, :K] = torch.randn(M, K, generator=g, device='cuda')
+    plain = product(tm, w, x)
+    x.view(torch.int32)[M // 3, 7] = bits
+    y = product(tm, w, x)
+    assert bool(torch.isnan(y[M // 3]).all())
+    keep = [m for m in range(M) if m != M // 3]
+    assert torch.equal(y[keep], plain[keep])
+
+
 def test_kernels_of_the_sizes_above():
     """what the sizes of the first test run: the narrow kernel, the weight stream with one and several blocks of rows, both tiles"""
     for K, N, M, plan in ((264, 2052, 3, 1), (1024, 4100, 5, 1), (8448, 260, 40, 1), (2080, 1030, 90, 6), (264, 2052, 257, 6), (1024, 4100, 2500, 5)):
