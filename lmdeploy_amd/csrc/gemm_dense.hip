@@ -479,7 +479,7 @@ static double few_rows_cost(int steps, int cols, int rows, int cw, int sp, int s
 }
 
 // The same for fp32 rows, whose lines are twice as many: blocks of 64 rows side by side up to 256, and (cw < 0) 64 x 64 tiles.  Of 486 sizes (K 64 ... 14336, N 256 ... 32000, 1 ...
-// 256 rows) what it takes is on average 1.6 % slower than the best, at most 45 % ((256, 24500) 129 rows).  us: (2048, 2048) 3 rows, narrow 5.3, four slices 7.0; (8448, 2048) 3
+// 256 rows) what it took without the two terms at the line to tiles (stream_plan) was on average 1.6 % slower than the best, at most 45 % ((256, 24500) 129 rows).  us: (2048, 2048) 3 rows, narrow 5.3, four slices 7.0; (8448, 2048) 3
 // rows, narrow 14.9, six slices 12.5; (2048, 8448) 32 rows, 96 columns two slices 16.1, 64 columns one 18.3, narrow 28.9; (2048, 1024) 90 rows, eight slices 15.9, tiles 17.2; (2048,
 // 32000) 48 rows, slices 62, tiles 35 (up to 64 rows tiles are taken where the model sees 15 % in them)
 static double few_rows_cost_f32(int steps, int cols, int rows, int cw, int sp, int ss)
@@ -574,8 +574,15 @@ StreamPlan stream_plan(int steps, int cols, int rows, int items, bool own_rows, 
                 }
             }
         }
-        if (elem == 4 && !few_only && border % 64 == 0 && few(-1, 1, steps) < (rows <= 64 ? 0.85 : 1.0) * least) {
-            best.skinny = false, best.tile = 3;
+        if (elem == 4 && !few_only && border % 64 == 0) {
+            // what a workgroup of the weight stream stages and splits of the rows are whole tiles of 16, and four of them take its stages twice as often, which weighs where the
+            // model's other terms are short (1320 sizes without slices, both timed: this line is 0.9 % over the better one in the mean, 23 % at most; without these two terms
+            // 2.5 % and 93 %.  us, stream / tile: (256, 32000) 256 rows 44 / 23, (1536, 8448) 33 rows 26 / 16, (256, 2048) 33 rows 7.6 / 5.8)
+            const bool   one  = best.splits == 1;
+            const double held = one && !best.narrow ? few_rows_cost_f32(steps, cols, rows <= 64 ? 16 * mt : rows, best.cw, 1, best.split_steps) + (mt < 4 ? 0.0 : rows <= 64 ? 0.7 : 2.5) : least;
+            if (few(-1, 1, steps) < (rows <= 64 ? 0.85 : one ? 1.1 : 1.0) * held) {
+                best.skinny = false, best.tile = 3;
+            }
         }
         return best;
     }

@@ -705,6 +705,14 @@ def stream_plan(kind, K, N, M, scratch=1):
     return tuple(v)
 
 
+def test_line_between_the_kernels_of_fp32_products():
+    """64 x 64 tiles where the weight stream splits whole tiles of rows for little, the stream elsewhere (both timed at these sizes)"""
+    for K, N, M in ((256, 2048, 33), (256, 32000, 40), (1536, 8448, 33), (256, 24500, 129), (256, 32000, 256), (2048, 8448, 200)):
+        assert stream_plan(1, K, N, M, 0)[0] == 6, (K, N, M)
+    for K, N, M in ((256, 2048, 32), (768, 768, 40), (4096, 4096, 33), (2048, 2048, 40), (1024, 24500, 24)):
+        assert stream_plan(1, K, N, M, 0)[0] < 3, (K, N, M)
+
+
 def test_line_between_the_kernels_of_fp16_products():
     """the general kernel where a round of its 64 x 128 workgroups, or beyond 40 rows the last of several, is at least three quarters full; the weight stream elsewhere"""
     for wgs, few, many in ((192, 2, 2), (216, 0, 0), (256, 0, 0), (288, 2, 2), (384, 2, 2), (448, 2, 0), (512, 2, 0), (576, 2, 2), (640, 2, 2), (723, 2, 0), (1002, 2, 0), (1188, 2, 0)):
