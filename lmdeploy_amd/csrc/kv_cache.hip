@@ -566,9 +566,11 @@ int launch_attn_prep(const float* proj, int ld, int q_col, int k_col, int v_col,
     if (p.rows == 0) {
         return 0;
     }
-    // prompts: neighbouring rows are neighbouring entries of a channel; decoded rows and prompts of a few tokens are not, and a launch more costs them some 4 us
+    // prompts: neighbouring rows are neighbouring entries of a channel; decoded rows and prompts of a few tokens are not, and a launch more costs some 4 us, which a million values
+    // are worth: us, by head vectors / apart, 16 + 8 + 8 heads of 128, 64 rows 4.3 / 7.9, 256 rows 6.1 / 9.0, 512 10.7 / 10.7, 1000 17.9 / 16.7, 4000 57.9 / 45.1; 32 + 4 + 4 of 128, 1000 rows 19.4 /
+    // 21.7, 4000 65.3 / 60.1; 8 + 2 + 2 of 64, 4000 rows 18.6 / 20.3
     // (pieces of eight channels lie in one head and start at multiples of 16 bytes; scaled values need their head's sum)
-    const bool apart = p.rows >= 64 && p.max_q_len >= 16 && !v_norm && !ex.conv_w && p.vdim % 8 == 0 && ld % 4 == 0 && v_col % 4 == 0 && (uintptr_t)proj % 16 == 0;
+    const bool apart = (int64_t)p.rows * vh * p.vdim >= 1000000 && p.max_q_len >= 16 && !v_norm && !ex.conv_w && p.vdim % 8 == 0 && ld % 4 == 0 && v_col % 4 == 0 && (uintptr_t)proj % 16 == 0;
     const int  own   = apart ? 0 : vh;  // value heads of the launch by head vectors
     const dim3 grid(p.rows, (p.q_heads + kh + own + 3) / 4), rows((p.rows + 63) / 64, (vh * p.vdim + 63) / 64);
     if (p.elem_bytes == 2) {
