@@ -2,11 +2,14 @@
 their edges, with a bound that needs every part and the short runs of steps; rows with infinities, NaN and numbers near the largest."""
 import ctypes as C
 
+import numpy as np
 import pytest
 import torch
 
 from lmdeploy_amd import _ffi
+from tests import layered_oracle as lo
 from tests.gpu_helpers import release_all, st
+from tests.test_gpu_layered import _layer, engine_for
 from tests.test_host import stream_plan
 
 pytestmark = pytest.mark.gpu
@@ -54,6 +57,40 @@ def test_every_part_counts(tm, cuda, K, N, rows, sign):
         assert bool((err <= (72 + K / 256) * 2.0 ** -24 * size).all()), (M, float((err / size).max()) * 2 ** 24)
         if sign == 'one' and K >= 1024:      # ... and the mean shows no drift of long sums: each run's cuts are 24 of at most 2^-23, half of that each on average
             assert float((err / size).mean()) <= (24 + K / 256) * 2.0 ** -24, M
+
+
+SLICED = {   # (K, N): rows and the plan they have in an engine: weight stream, column tiles a workgroup, row tiles, slices
+    (2048, 250): {16: (2, 4, 1, 8), 17: (2, 4, 2, 8), 40: (2, 4, 4, 8), 65: (2, 4, 4, 8), 129: (2, 4, 4, 8), 256: (2, 4, 4, 8)},
+    (2048, 770): {40: (2, 4, 4, 8), 90: (2, 4, 4, 8), 129: (2, 6, 4, 8), 200: (2, 4, 4, 4)},
+    (8192, 2050): {3: (2, 6, 1, 8), 16: (2, 6, 1, 11), 24: (2, 6, 2, 11), 64: (2, 6, 4, 11), 90: (2, 6, 4, 11), 129: (2, 6, 4, 11), 200: (2, 6, 4, 8)}}
+
+
+@pytest.mark.parametrize('sign', ['both', 'one'])
+@pytest.mark.parametrize('K,N', SLICED)
+def test_every_part_counts_in_slices(cuda, K, N, sign):
+    """The head's product of an engine, which has scratch for slices of k: the logits of rows that are their embedding's norm.  As above, and the norm's own errors: its mean of squares within
+    K / 256 + 8 roundings, half of that in its root, and four of each number"""
+    cfg = lo.make_config(K, N, [_layer(heads=1, kv_heads=1, dim=8, vdim=8, ff=0)], logit_scale=1.0)
+    w = lo.make_weights(cfg, K + N)
+    w['l0.mix.o'][:] = 0
+    if sign == 'one':
+        w['embed'], w['head'], w['final.norm'] = (np.abs(w[k]) for k in ('embed', 'head', 'final.norm'))
+    eng = engine_for(cfg, w, 'float32', max_batch_size=2)
+    rng = np.random.default_rng(K)
+    for M, plan in SLICED[K, N].items():
+        assert stream_plan(1, K, N, M)[:4] == plan, (M, stream_plan(1, K, N, M))
+        toks, got = rng.integers(0, N, M), []
+        for _ in range(2):      # (arrival counters are back at zero)
+            s = eng.open_session()
+            got.append(eng.step_tokens([(s, toks, list(range(M)))]))
+            eng.close_session(s)
+        assert np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+        x = lo.rms_norm(w['embed'][toks], w['final.norm'], cfg['eps'], cfg['offset'])
+        err, size = np.abs(got[0] - x @ w['head'].T), np.abs(x) @ np.abs(w['head']).T
+        assert (err <= (80 + K / 128) * 2.0 ** -24 * size).all(), (M, (err / size).max() * 2 ** 24)
+        if sign == 'one':
+            assert (err / size).mean() <= (24 + K / 128) * 2.0 ** -24, (M, (err / size).mean() * 2 ** 24)
+    eng.close()
 
 
 @pytest.mark.parametrize('K,N,M', [(96, 200, 3), (520, 260, 20), (520, 260, 40), (520, 1000, 300), (1024, 4100, 2500)])
