@@ -6,9 +6,7 @@ import pytest
 
 from lmdeploy_amd import _ffi
 from tests.gpu_helpers import release_all
-from tests.test_gpu_febivik import engine as febivik_engine
-from tests.test_gpu_febivik import full_model as febivik_model
-from tests.test_gpu_febivik import model_folder as febivik_folder
+from tests import test_gpu_bedenex, test_gpu_febivik, test_gpu_layered, test_gpu_mededra, test_gpu_roravik
 from tests.test_gpu_sanozen import engine as sanozen_engine
 from tests.test_gpu_sanozen import full_model as sanozen_model
 from tests.test_gpu_sanozen import model_folder as sanozen_folder
@@ -52,17 +50,38 @@ def _walk(eng, vocab):
     return out
 
 
+def _fokonex(tmp_path, dtype):
+    cfg, w = test_gpu_layered.small_model(2)
+    return cfg['vocab'], lambda **kw: test_gpu_layered.engine_for(cfg, w, dtype, **kw)
+
+
+def _of(module, cfg):
+    def build(tmp_path, dtype):
+        c = cfg(dtype)
+        folder = module.model_folder(tmp_path, c, 2)[0]
+        return c['vocab'], lambda **kw: module.engine(folder, dtype, **kw)
+    return build
+
+
+def _sanozen(tmp_path, dtype):
+    folder, _ = sanozen_folder(tmp_path, sanozen_model(), 2)
+    return sanozen_model()['vocab'], lambda **kw: sanozen_engine(folder, dtype, **kw)
+
+
+FAMILIES = {'fokonex': _fokonex, 'bedenex': _of(test_gpu_bedenex, test_gpu_bedenex.looped_model), 'febivik': _of(test_gpu_febivik, test_gpu_febivik.full_model),
+            'mededra': _of(test_gpu_mededra, lambda dtype: test_gpu_mededra.full_model()), 'sanozen': _sanozen,
+            'roravik': _of(test_gpu_roravik, lambda dtype: test_gpu_roravik.full_model())}
+
+
 @pytest.mark.parametrize('dtype', ['float32', 'bfloat16'])
-@pytest.mark.parametrize('family', ['sanozen', 'febivik'])
+@pytest.mark.parametrize('family', FAMILIES)
 def test_graphs_give_the_bits_of_launches(tmp_path, cuda, family, dtype):
-    cfg = sanozen_model() if family == 'sanozen' else febivik_model(dtype)
-    folder, _ = (sanozen_folder if family == 'sanozen' else febivik_folder)(tmp_path, cfg, 2)
-    build = sanozen_engine if family == 'sanozen' else febivik_engine
+    vocab, build = FAMILIES[family](tmp_path, dtype)
     rows = []
     for graphs in (0, 1):
-        eng = build(folder, dtype, use_graph=graphs)
-        rows.append(_walk(eng, cfg['vocab']))
-        rows.append(_walk(eng, cfg['vocab']))      # with the graphs of the first course
+        eng = build(use_graph=graphs)
+        rows.append(_walk(eng, vocab))
+        rows.append(_walk(eng, vocab))      # with the graphs of the first course
         eng.close()
     for other in rows[1:]:
         assert len(other) == len(rows[0]) and all(np.array_equal(x.view(np.uint32), y.view(np.uint32)) for x, y in zip(rows[0], other))
