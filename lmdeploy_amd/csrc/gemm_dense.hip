@@ -95,58 +95,37 @@ struct DenseEpi {
 
     static constexpr bool kPairs = EPI == kDenseGatedAct && sizeof(T) == 2;
     static constexpr bool kTileRuns = true;
-    // What an output needs besides its product: the stream's element, its bias, its row of a table.  Where a lane has many outputs their operands are
+    // What an output needs besides its product: the stream's element or its bias.  Where a lane of a 256 x 256 tile has its outputs, their operands are
     // asked for together (read), before the first of them is stored (join): a load that follows a store which may have written there waits in line, and a tile's 64
     // outputs a lane paid 64 trips to memory one after the other.  us, one by one / sixteen together: 8010 rows of bf16 into the stream, (2048, 2048) 104 / 85,
-    // (8448, 2048) 275 / 253
-    static constexpr int kReads = EPI == kDenseResidAdd || EPI == kDenseBiasF32 ? 16 : EPI == kDenseActTable ? 4 : 0;  // so many at a time
+    // (8448, 2048) 275 / 253; 8000 rows of (2048, 2050) 97 / 92.  Not in the smaller tiles, whose other workgroup on the CU covers the trips: 128 x 128 and 256 x 128
+    // took 1 - 7 % longer with it ((2048, 2048) 2500 rows 39.7 / 41.4), a ragged edge 16 % ((1000, 3000) 2500 rows 32.2 / 37.4)
+    static constexpr int kReads = EPI == kDenseResidAdd || EPI == kDenseBiasF32 ? 16 : 0;  // so many at a time
     struct Operand {
         floatx4 v;
     };
-    template<bool VEC>
+    template<bool WHOLE>
     __device__ __forceinline__ Operand read(const StreamArgs& a, const DenseItem& it, int m, int n) const
     {
-        typedef float  float4_any __attribute__((ext_vector_type(4), aligned(4)));
-        typedef __bf16 bf16x4_any __attribute__((ext_vector_type(4), aligned(2)));
-        m += it.row_base;
-        if constexpr (EPI == kDenseActTable) {
-            const int     id = min(max(c.ids[m], 0), c.table_rows - 1);
-            const __bf16* t  = (const __bf16*)c.table + (size_t)id * c.ld_table + c.table_col + n;
-            if constexpr (VEC) {
-                const bf16x4_any v = *(const bf16x4_any*)t;
-                return {floatx4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]}};
-            }
-            else {
-                return {some(t, a.N - n)};
-            }
+        typedef float float4_any __attribute__((ext_vector_type(4), aligned(4)));
+        const float*  at = EPI == kDenseBiasF32 ? c.bias + n : (const float*)a.y + (size_t)(m + it.row_base) * a.ldy + it.col_base + n;
+        if constexpr (WHOLE) {
+            return {*(const float4_any*)at};
         }
-        else {
-            const float* at = EPI == kDenseBiasF32 ? c.bias + n : (const float*)a.y + (size_t)m * a.ldy + it.col_base + n;
-            if constexpr (VEC) {
-                return {*(const float4_any*)at};
-            }
-            else {
-                return {some(at, a.N - n)};
-            }
-        }
-    }
-    template<class O>
-    __device__ __forceinline__ static floatx4 some(const O* p, int left)
-    {
-        floatx4 v = {0.f, 0.f, 0.f, 0.f};
+        Operand o = {{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            if (e < left) {
-                v[e] = (float)p[e];
+            if (n + e < a.N) {
+                o.v[e] = at[e];
             }
         }
-        return v;
+        return o;
     }
     // the operands of N outputs: output j is row at(j).x of the item, columns at(j).y .. + 3
     template<int N, class At>
     __device__ __forceinline__ void operands(const StreamArgs& a, const DenseItem& it, At&& at, Operand (&op)[N]) const
     {
-        bool whole = vec != 0;
+        bool whole = true;  // (the loads need no alignment but their elements')
 #pragma unroll
         for (int j = 0; j < N; ++j) {
             whole = whole && at(j).y + 4 <= a.N;
@@ -175,22 +154,11 @@ struct DenseEpi {
         float        r[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float z = acc[e];
-            if constexpr (EPI == kDenseActTable) {
-                r[e] = act_apply(c.act, z) * op.v[e];
-            }
-            else {
-                r[e] = EPI == kDenseBiasF32 ? z + op.v[e] : op.v[e] + c.alpha * z;
-            }
+            r[e] = EPI == kDenseBiasF32 ? acc[e] + op.v[e] : op.v[e] + c.alpha * acc[e];
         }
-        if constexpr (EPI == kDenseActTable) {
-            store_run<T, 4>((T*)a.y, i, r, vec, left);
-        }
-        else {
-            store_run<float, 4>((float*)a.y, i, r, vec, left);
-            if (EPI == kDenseResidAdd && c.y2) {
-                store_run<T, 4>((T*)c.y2, (size_t)m * c.ldy2 + n, r, vec, left);
-            }
+        store_run<float, 4>((float*)a.y, i, r, vec, left);
+        if (EPI == kDenseResidAdd && c.y2) {
+            store_run<T, 4>((T*)c.y2, (size_t)m * c.ldy2 + n, r, vec, left);
         }
     }
     __device__ __forceinline__ const int* row_offsets() const
@@ -248,16 +216,6 @@ struct DenseEpi {
                     dense_gated(c, g, u, r);
                     store_run<T, 4>((T*)a.y, (size_t)m * a.ldy + it.col_base + o, r, vec, c.n_out - o);
                 }
-            }
-            return;
-        }
-        if constexpr (kReads > 0) {
-            m -= it.row_base;
-            Operand op[NT];
-            operands<NT>(a, it, [=](int j) { return int2{m, n + 16 * j}; }, op);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                join(a, it, m, n + 16 * j, acc[j], op[j]);
             }
             return;
         }

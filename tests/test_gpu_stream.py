@@ -20,6 +20,7 @@ from tests.test_gpu_febivik import rel_err as rel_err_febivik
 from tests.test_gpu_layered import TOL, _layer, engine_for, rel_err
 from tests.test_gpu_roravik import engine as roravik_engine
 from tests.test_gpu_roravik import model_folder as roravik_folder
+from tests.test_host import stream_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -278,3 +279,23 @@ def test_turned_items(tmp_path, cuda, dtype, width):
     wrong = np.stack([fo.forward(cfg, bad, r)[[63, 129, 130, 131]] for r in reqs])
     assert rel_err_febivik(wrong, ref) > 2 * TOL[dtype]
     eng.close()
+
+
+@pytest.mark.parametrize('K,N,M,tile', [(264, 2049, 7990, 3), (264, 2052, 8001, 3), (264, 2299, 4000, 3), (1000, 3000, 2500, 4), (264, 1027, 900, 6)])
+@pytest.mark.parametrize('more', [0, 1, 2, 3])              # rows of the stream on and off multiples of 16 bytes, a ragged last column tile
+def test_sums_into_the_stream(tm, cuda, K, N, M, tile, more):
+    """y += alpha x w, whose old values a 256 x 256 tile reads sixteen together and the smaller ones one by one"""
+    assert stream_plan(0, K, N, M, 0)[0] == tile
+    g = torch.Generator('cuda').manual_seed(N + more)
+    w, x = torch.randn(N, K, generator=g, device='cuda').bfloat16(), torch.zeros(M, (K + 31) // 32 * 32, device='cuda').bfloat16()
+    x[:, :K] = torch.randn(M, K, generator=g, device='cuda').bfloat16()
+    ldy = N + more
+    y = torch.randn(M + 1, ldy, generator=g, device='cuda')
+    old = y.double()
+    h = C.c_void_p()
+    _ffi.check(tm.tm_dense_create(C.byref(h), K, N, 0, w.data_ptr(), st()))
+    _ffi.check(tm.tm_dense_forward(h, x.data_ptr(), x.shape[1], y.data_ptr(), ldy, M, 2, 0.5, st()))
+    _ffi.check(tm.tm_dense_destroy(h))
+    ref, size = old[:M, :N] + 0.5 * (x[:, :K].double() @ w.double().t()), x[:, :K].double().abs() @ w.double().abs().t()
+    assert bool(((y[:M, :N].double() - ref).abs() <= K * 2.0 ** -24 * size + 2.0 ** -23 * ref.abs() + 1e-30).all())
+    assert torch.equal(y[:M, N:].double(), old[:M, N:]) and torch.equal(y[M].double(), old[M])
