@@ -690,8 +690,9 @@ int tm_engine_debug_stop_after(tm_engine* e, int layers);
  * tm_rmsnorm_f32: y_i = x / sqrt(mean(x^2) + eps) * (w_offset + w_i) for one or two weight vectors (y1 / w1 may be NULL) from ONE
  *   statistic; x fp32 [M][H] (rows != NULL: row m is x[rows[m]]), w fp32 [H], y bf16 (out_elem_bytes 2) or fp32 (4) [M][ldy].
  * tm_dense_*: unquantised linear, weight given in checkpoint orientation [N][K] as bf16 bits; dtype TM_DTYPE_BF16 runs on the bf16
- *   matrix cores with fp32 accumulation, TM_DTYPE_F32 widens the weight and computes in fp32.  epilogue: 0 y = acc, 1 y = relu(acc)^2
- *   (x's type), 2 y_f32 += alpha * acc, 3 y_f32 = alpha * acc.  ldx >= K rounded up to 32 (pad columns finite).
+ *   matrix cores with fp32 accumulation, TM_DTYPE_F32 keeps the bf16 weight and splits each fp32 row into three bf16 parts, whose products are
+ *   exact and whose sums are fp32 (weights have to be finite: an infinite one times a number with a part of zero is a NaN).  epilogue: 0 y = acc,
+ *   1 y = relu(acc)^2 (x's type), 2 y_f32 += alpha * acc, 3 y_f32 = alpha * acc.  ldx >= K rounded up to 32 (pad columns finite).
  * tm_general_attention: causal attention of `rows` query rows over a paged cache with arbitrary key / value sizes; the layout of a block
  *   is [kv_heads][64][dim] keys at layer_offset, values TRANSPOSED [kv_heads][vdim][64] at layer_offset + v_offset, elements bf16 or fp32.  With
  *   store_kv != 0 the keys / values of the rows (kv, [rows][ldkv]: keys at column k_col, values at v_col) are written to the cache first.
@@ -700,7 +701,7 @@ int tm_engine_debug_stop_after(tm_engine* e, int layers);
  *   kernel: 0 dispatch (prefill != 0: the tile kernel where it serves the sizes), 1 row kernel, 3 decode kernel (bf16, one row per sequence:
  *   row t = sequence t), 2 tile kernel (needs cu_q / k_len / nseq:
  *   rows grouped by sequence, cu_q[nseq + 1], k_len[nseq] context lengths including the rows).  splits > 1 needs workspace of
- *   tm_general_attention_workspace() bytes. */
+ *   tm_general_attention_workspace() bytes, aligned as a float is. */
 int tm_rmsnorm_f32(void* y0, void* y1, int ldy, int out_elem_bytes, const float* x, const int* rows, const float* w0, const float* w1,
                    float w_offset, float eps, int M, int H, tm_stream_t st);
 typedef struct tm_dense tm_dense;
